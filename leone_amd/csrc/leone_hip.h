@@ -96,7 +96,8 @@ int leone_attention_prefill(const void* q, void* out, const void* k_pool, const 
                             float* part_ml, int splits, hipStream_t stream);
 
 // C[M,N] = A[M,K] . B[N,K]^T in float.
-int leone_gemm_f32(const float* a, const float* b, float* c, int m, int n, int k, hipStream_t stream);
+int leone_gemm_f32_planes(int m, int n, int k);      // planes [m, n] of floats that leone_gemm_f32 needs beside C, 0 for none
+int leone_gemm_f32(const float* a, const float* b, float* c, float* planes, int m, int n, int k, hipStream_t stream);
 
 // Tiled weights.  The two weight-streaming products below read W either row by row ([N,K]) or, with w_tiled, from
 // a copy laid out in the order in which their waves ask for it, for K a multiple of 64: rows in tiles of 16

@@ -702,9 +702,12 @@ def gemm_f32(a: torch.Tensor, b: torch.Tensor, out: Optional[torch.Tensor] = Non
         raise KernelError(f"gemm_f32: inner sizes {k} and {k2} differ")
     if out is None:
         out = torch.empty((m, n), dtype=torch.float32, device=a.device)
+    # where the kernel cuts K into parts, it needs room for their results
+    parts = library().leone_gemm_f32_planes(m, n, k)
+    planes = torch.empty((parts, m, n), dtype=torch.float32, device=a.device) if parts else None
     with profile.span("gemm f32", b):
         call("leone_gemm_f32", _dev(a, "gemm a", torch.float32), _dev(b, "gemm b", torch.float32),
-             _dev(out, "gemm out", torch.float32, (m, n)), m, n, k, _stream())
+             _dev(out, "gemm out", torch.float32, (m, n)), _dev(planes, "gemm planes"), m, n, k, _stream())
     return out
 
 

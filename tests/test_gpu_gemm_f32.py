@@ -1,0 +1,52 @@
+"""The single-precision product: both kernels, their tiles' edges, the cut of the inner size, operands off 16 bytes."""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def worst(m, n, k, shift=0, seed=1):
+    """The largest error of the product over what its sums can be off by (``shift``: elements the operands are moved by)."""
+    from leone_amd import ops
+    gen = torch.Generator(device=DEV).manual_seed(seed)
+    a = torch.randn(m * k + shift, generator=gen, device=DEV)[shift:].view(m, k)
+    b = torch.randn(n * k + shift, generator=gen, device=DEV)[shift:].view(n, k)
+    got = ops.gemm_f32(a, b)
+    want = a.double() @ b.double().T
+    # every product and every addition of a chain of k is off by at most 2^-24 of the running sum's size, whose root mean
+    # square is sqrt(k); the errors add up like a random walk, and none of so many is beyond eight times its deviation
+    bound = 8.0 * 2.0 ** -24 * math.sqrt(k) * math.sqrt(k + math.log2(k + 1))
+    return float((got.double() - want).abs().max()) / bound
+
+
+# rows: every number of row tiles of the streaming kernel and its edges, then the tiled kernel with both tiles; columns off 16
+# and 64; inner sizes below a run, off a run, off 4, and long enough to be cut
+@pytest.mark.parametrize("m", [1, 2, 15, 16, 17, 32, 33, 63, 64, 65, 127, 130, 777])
+@pytest.mark.parametrize("n,k", [(16, 8), (17, 60), (96, 64), (130, 333), (2048, 512), (520, 2052), (1536, 6144)])
+def test_sizes(m, n, k):
+    assert worst(m, n, k) < 1.0
+
+
+def test_many_tiles():
+    assert worst(1500, 6144, 256) < 1.0 and worst(1025, 8200, 100) < 1.0
+
+
+@pytest.mark.parametrize("m", [3, 40, 200])
+def test_operands_off_sixteen_bytes(m):
+    assert worst(m, 100, 512, shift=1) < 1.0 and worst(m, 100, 512, shift=3) < 1.0
+
+
+def test_rows_do_not_depend_on_their_neighbours():
+    """A row that holds infinities and NaN spoils its own results only."""
+    from leone_amd import ops
+    for m, n, k in ((5, 70, 96), (130, 70, 1000)):
+        a, b = torch.randn(m, k, device=DEV), torch.randn(n, k, device=DEV)
+        clean = ops.gemm_f32(a, b)
+        a[1, 3], a[2, k - 1] = math.inf, math.nan
+        spoilt = ops.gemm_f32(a, b)
+        keep = [i for i in range(m) if i not in (1, 2)]
+        assert torch.equal(clean[keep], spoilt[keep])
+        assert bool(torch.isinf(spoilt[1]).all()) and bool(torch.isnan(spoilt[2]).all())
