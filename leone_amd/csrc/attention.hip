@@ -13,6 +13,7 @@
 // Cache layout of one layer: [page][kv head] blocks of page_tokens * head_dim
 // elements, packed inside as key_offset() and value_offset() say.
 #include "common.h"
+#include "attention_f32.h"
 #include "leone_hip.h"
 #include "score_shape.h"
 
@@ -290,6 +291,14 @@ extern "C" int leone_attention_rows_shaped(const void* q, void* out, const void*
     LEONE_REQUIRE(head_dim % 8 == 0 && page_tokens % 8 == 0,
                   "attention_rows: head_dim %d and page_tokens %d must be multiples of 8", head_dim, page_tokens);
     LEONE_REQUIRE(window >= 0, "attention_rows: window %d must not be negative", window);
+    if (dtype == kF32 && attention_f32_takes(q, out, k_pool, v_pool, q_heads, kv_heads, head_dim, v_dim, page_tokens)) {
+        launch_attention_f32(static_cast<const float*>(q), static_cast<float*>(out), static_cast<const float*>(k_pool),
+                             static_cast<const float*>(v_pool), positions, row_entry, block_table, max_blocks, rows, q_heads, kv_heads,
+                             head_dim, page_tokens, scale, window, gate, gate_stride, keep_first, gate_each, slopes, temp_coef,
+                             temp_every, shape, chunk, stream);
+        LEONE_LAUNCH_CHECK("attention_rows");
+        return 0;
+    }
     dim3 grid(rows, q_heads);
     if (dtype == kF32)
         attention_rows_kernel<float><<<grid, kRowThreads, 0, stream>>>(

@@ -1,0 +1,291 @@
+// Attention over the paged cache in single precision, on the float matrix instructions: the function of
+// attention_rows_kernel (attention.hip; scores, softmax and sums in float) for heads of 64 or 128 elements.
+//
+// A query row alone reads every key for itself, which bounds a row by the walk along its keys (one dot product and one
+// step of the softmax a key).  Here a workgroup takes up to 16 queries that read the same keys - the query heads of one
+// kv head, of a few neighbouring rows of one request - and its waves share out the keys, 16 at a time, each wave with a
+// running softmax of its own; the waves' results are merged through shared memory in a fixed order.  What bounds it is
+// the matrix instructions: 64 of 32 cycles for 16 keys of 128 elements, whose loads (16 KB a wave) are in flight meanwhile.
+//
+// Lane l of a wave holds, of a product, row or column l % 16, and inner elements 4 (l / 16) .. + 3 of every 16: with the
+// cache's runs of 8 a 16-byte load a lane brings 16 keys x 16 elements, or 16 value elements x 16 tokens.  Scores are made
+// as keys x queries, so that a lane's four scores belong to its own query and to the four keys it holds values of: they
+// are the operand of the second product as they stand.
+//
+// Measured (us; the row kernel of attention.hip before): 16 heads over 4 of 128 elements, one row at 780 keys 29 (314), a prompt
+// of 777 rows 81 (1375).
+#include "common.h"
+#include "leone_hip.h"
+#include "score_shape.h"
+
+#include <math.h>
+
+namespace leone {
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int kQueries = 16;
+constexpr int kKeys = 16;
+
+struct AttentionF32Args {
+    const float* q;
+    float* out;
+    const float* k_pool;
+    const float* v_pool;
+    const int* positions;
+    const int* row_entry;
+    const int* block_table;
+    int max_blocks, rows, q_heads, kv_heads, page_tokens;
+    float scale;
+    int window;
+    const float* gate;
+    long gate_stride;
+    int keep_first, gate_each;
+    const float* slopes;
+    float temp_coef;
+    int temp_every;
+    ScoreShape shape;
+    int chunk;
+};
+
+template <int kDim, int kWaves>
+__global__ void __launch_bounds__(kWaves * kWave) attention_f32_kernel(const AttentionF32Args g) {
+    constexpr int kRuns = kDim / 16;
+    __shared__ float sm_m[kWaves][kQueries], sm_l[kWaves][kQueries];
+    __shared__ f32x4 sm_acc[kWaves / 2][kRuns][kWave];
+
+    // The rows of this workgroup: from this one on, those of the same request up to the next multiple of `most`; the
+    // workgroups of the rows that another one takes have nothing to do.
+    const int group = g.q_heads / g.kv_heads, most = kQueries / group;
+    const int first_row = blockIdx.x, kvh = blockIdx.y;
+    const int entry = g.row_entry[first_row];
+    if (first_row % most != 0 && g.row_entry[first_row - 1] == entry) return;
+    int count = 1;
+    while ((first_row + count) % most != 0 && first_row + count < g.rows && g.row_entry[first_row + count] == entry) ++count;
+
+    const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+    const int mine = lane % 16, h = (lane / 16) * 4;
+    // this lane's query: lanes past the last one repeat it and write nothing
+    const bool real = mine < count * group;
+    const int query = real ? mine : count * group - 1;
+    const int row = first_row + query / group, head = kvh * group + query % group;
+    const int pos = g.positions[row];
+    float scale = g.scale;
+    if (g.temp_every > 0) scale *= 1.0f + g.temp_coef * logf(static_cast<float>((pos + 1) / g.temp_every + 1));
+    const float slope = g.slopes ? g.slopes[head] : 0.f;
+    const int first = first_key(pos, g.window, g.chunk);
+
+    f32x4 q[kRuns];
+    const float* qr = g.q + (static_cast<long>(row) * g.q_heads + head) * kDim;
+#pragma unroll
+    for (int i = 0; i < kRuns; ++i) q[i] = *reinterpret_cast<const f32x4*>(qr + i * 16 + h);
+
+    // what the rows together see: tiles of 16 keys from the earliest row's first one on, and those of the kept first keys
+    int low = first, high = pos;
+#pragma unroll
+    for (int off = 8; off > 0; off >>= 1) {
+        low = min(low, __shfl_xor(low, off, kWave));
+        high = max(high, __shfl_xor(high, off, kWave));
+    }
+    const int low_tile = low / kKeys;
+    const int kept_tiles = min((g.keep_first + kKeys - 1) / kKeys, low_tile);
+    const int tiles = kept_tiles + high / kKeys + 1 - low_tile;
+    const int* table = g.block_table + static_cast<long>(entry) * g.max_blocks;
+    const long page_floats = static_cast<long>(g.page_tokens) * kDim;
+
+    f32x4 kf[kRuns], vf[kRuns], acc[kRuns] = {};
+    float m = -INFINITY, l = 0.f;
+    bool mapped = true, mapped_next = true;
+    const auto start_of = [&](int t) { return (t < kept_tiles ? t : low_tile + t - kept_tiles) * kKeys; };
+    const auto block_of = [&](int start, bool& there) {
+        const int page = table[start / g.page_tokens];
+        there = page >= 0;
+        return (static_cast<long>(there ? page : 0) * g.kv_heads + kvh) * page_floats;
+    };
+    const auto fetch_keys = [&](int start, long block) {
+        const float* at = g.k_pool + block + (static_cast<long>(h / 8) * g.page_tokens + start % g.page_tokens + mine) * 8 + h % 8;
+#pragma unroll
+        for (int i = 0; i < kRuns; ++i) kf[i] = *reinterpret_cast<const f32x4*>(at + static_cast<long>(2 * i) * g.page_tokens * 8);
+    };
+    const auto fetch_values = [&](int start, long block) {
+        const float* at = g.v_pool + block + (static_cast<long>((start % g.page_tokens + h) / 8) * kDim + mine) * 8 + h % 8;
+#pragma unroll
+        for (int i = 0; i < kRuns; ++i) vf[i] = *reinterpret_cast<const f32x4*>(at + i * 128);
+    };
+    int t = wave;
+    long block = 0;
+    if (t < tiles) {
+        block = block_of(start_of(t), mapped);
+        fetch_keys(start_of(t), block);
+    }
+    for (; t < tiles; t += kWaves) {
+        const int start = start_of(t);
+        fetch_values(start, block);
+        f32x4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < kRuns; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) s = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[i][j], q[i][j], s, 0, 0, 0);
+        if (t + kWaves < tiles) {             // the keys' registers are free: the next tile's are on their way from here on
+            const int next = start_of(t + kWaves);
+            block = block_of(next, mapped_next);
+            fetch_keys(next, block);
+        }
+        float top = -INFINITY;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int key = start + h + r;
+            const bool seen = key <= pos && (key >= first || key < g.keep_first);
+            float v = s[r] * scale;
+            if (g.shape.cap > 0.f) v = g.shape.cap * tanhf(v / g.shape.cap);
+            v -= slope * static_cast<float>(pos - key);
+            // an unmapped block poisons the result of every row that sees it
+            s[r] = seen ? (mapped ? v : __builtin_nanf("")) : -INFINITY;
+            top = fmaxf(top, s[r]);
+        }
+        top = fmaxf(top, __shfl_xor(top, 16, kWave));
+        top = fmaxf(top, __shfl_xor(top, 32, kWave));
+        const float m_new = fmaxf(m, top);
+        const float reference = m_new == -INFINITY ? 0.f : m_new;      // nothing seen yet: every weight is 0
+        const float alpha = expf(m - reference);
+        float sum = 0.f;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            s[r] = expf(s[r] - reference);
+            sum += s[r];
+        }
+        sum += __shfl_xor(sum, 16, kWave);
+        sum += __shfl_xor(sum, 32, kWave);
+        l = l * alpha + sum;
+        m = m_new;
+        if (!mapped || start + kKeys > high + 1) {       // places nobody has written: their weight is 0, but not what they may hold
+#pragma unroll
+            for (int i = 0; i < kRuns; ++i)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (!mapped || start + h + r > high) vf[i][r] = 0.f;
+        }
+        f32x4 odd = {0.f, 0.f, 0.f, 0.f};                // stays 0 unless a value is infinite or NaN
+#pragma unroll
+        for (int i = 0; i < kRuns; ++i) {
+            acc[i] *= alpha;
+            odd += vf[i] * 0.f;
+        }
+        if (__any(!(odd[0] + odd[1] + odd[2] + odd[3] == 0.f))) {
+            // such a value is for the rows that see it, and no weight of 0 keeps it from the others: one key after the other
+            for (int from = 0; from < 4; ++from)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const int key = start + 4 * from + j;
+                    const bool seen = key <= pos && (key >= first || key < g.keep_first);
+                    const float p = __shfl(s[j], from * 16 + mine, kWave);
+#pragma unroll
+                    for (int i = 0; i < kRuns; ++i)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            const float v = __shfl(vf[i][j], from * 16 + h + r, kWave);
+                            if (seen) acc[i][r] = fmaf(p, v, acc[i][r]);
+                        }
+                }
+        } else {
+#pragma unroll
+            for (int i = 0; i < kRuns; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[i][j], s[j], acc[i], 0, 0, 0);
+        }
+        mapped = mapped_next;
+    }
+
+    // ---- the waves' results, merged -------------------------------------------------------------------------------
+    if (lane < kQueries) {
+        sm_m[wave][lane] = m;
+        sm_l[wave][lane] = l;
+    }
+    __syncthreads();
+    float top = sm_m[0][mine];
+#pragma unroll
+    for (int w = 1; w < kWaves; ++w) top = fmaxf(top, sm_m[w][mine]);
+    const float sink = g.shape.sinks ? g.shape.sinks[head] : -INFINITY;
+    top = fmaxf(top, sink);
+    const auto weight = [&](float of) { return of == -INFINITY ? 0.f : expf(of - top); };
+    float denom = g.shape.sinks ? expf(sink - top) : 0.f;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) denom += sm_l[w][mine] * weight(sm_m[w][mine]);
+    const float own = weight(m);
+#pragma unroll
+    for (int i = 0; i < kRuns; ++i) acc[i] *= own;
+#pragma unroll
+    for (int half = kWaves / 2; half > 0; half /= 2) {
+        if (wave >= half && wave < 2 * half) {
+#pragma unroll
+            for (int i = 0; i < kRuns; ++i) sm_acc[wave - half][i][lane] = acc[i];
+        }
+        __syncthreads();
+        if (wave < half) {
+#pragma unroll
+            for (int i = 0; i < kRuns; ++i) acc[i] += sm_acc[wave][i][lane];
+        }
+        __syncthreads();
+    }
+    if (wave != 0) return;
+    // lane l: its query's elements 16 i + h .. + 3
+#pragma unroll
+    for (int i = 0; i < kRuns; ++i) acc[i] /= denom;
+    f32x4 result[kRuns];
+    if (g.shape.turn_cos) {
+#pragma unroll
+        for (int i = 0; i < kRuns; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float partner = g.shape.turn_pairing ? acc[i][r ^ 1] : acc[(i + kRuns / 2) % kRuns][r];
+                result[i][r] = turned_back(acc[i][r], partner, i * 16 + h + r, kDim, pos, g.shape);
+            }
+    } else {
+#pragma unroll
+        for (int i = 0; i < kRuns; ++i) result[i] = acc[i];
+    }
+    if (!real) return;
+    float* orow = g.out + (static_cast<long>(row) * g.q_heads + head) * kDim;
+    const float* gate_row = g.gate ? g.gate + static_cast<long>(row) * g.gate_stride + (g.gate_each ? static_cast<long>(head) * kDim : head) : nullptr;
+    const float open_head = (g.gate && !g.gate_each) ? 1.0f / (1.0f + expf(-gate_row[0])) : 1.0f;
+#pragma unroll
+    for (int i = 0; i < kRuns; ++i) {
+        f32x4 open = {open_head, open_head, open_head, open_head};
+        if (g.gate && g.gate_each) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) open[r] = 1.0f / (1.0f + expf(-gate_row[i * 16 + h + r]));
+        }
+        *reinterpret_cast<f32x4*>(orow + i * 16 + h) = result[i] * open;
+    }
+}
+
+// Whether the kernel takes this shape: 16-byte rows of q and of the results follow from the head's size, tiles of 16 keys lie
+// within a page, and a kv head's query heads fit one tile.  Everything else is the row kernel's.
+bool attention_f32_takes(const void* q, const void* out, const void* k_pool, const void* v_pool, int q_heads, int kv_heads, int head_dim,
+                         int v_dim, int page_tokens) {
+    const auto aligned = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+    return (head_dim == 64 || head_dim == 128) && v_dim == head_dim && page_tokens % kKeys == 0 && q_heads / kv_heads <= kQueries &&
+           kv_heads <= 65535 && aligned(q) && aligned(out) && aligned(k_pool) && aligned(v_pool);
+}
+
+void launch_attention_f32(const float* q, float* out, const float* k_pool, const float* v_pool, const int* positions, const int* row_entry,
+                          const int* block_table, int max_blocks, int rows, int q_heads, int kv_heads, int head_dim, int page_tokens,
+                          float scale, int window, const float* gate, long gate_stride, int keep_first, int gate_each,
+                          const float* slopes, float temp_coef, int temp_every, const ScoreShape& shape, int chunk, hipStream_t stream) {
+    const AttentionF32Args args{q, out, k_pool, v_pool, positions, row_entry, block_table, max_blocks, rows, q_heads, kv_heads,
+                                page_tokens, scale, window, gate, gate_stride, keep_first, gate_each, slopes, temp_coef, temp_every,
+                                shape, chunk};
+    const dim3 grid(rows, kv_heads);
+    // Few rows leave the chip to few workgroups: eight waves share out a row's keys (one row at 780 keys 29 us; the keys are
+    // bound by what one compute unit can read).  Workgroups that fill the chip by themselves (two a compute unit and more) take
+    // four, whose merge is half as long.
+    const bool few = static_cast<long>(rows) * kv_heads < 512;
+#define LEONE_ATTENTION_F32(D)                                                                    \
+    (few ? attention_f32_kernel<D, 8><<<grid, 8 * kWave, 0, stream>>>(args)                       \
+         : attention_f32_kernel<D, 4><<<grid, 4 * kWave, 0, stream>>>(args))
+    if (head_dim == 128) LEONE_ATTENTION_F32(128);
+    else LEONE_ATTENTION_F32(64);
+#undef LEONE_ATTENTION_F32
+}
+
+}  // namespace leone
