@@ -106,20 +106,21 @@ gemm_f32_stream_kernel(const float* __restrict__ a, const float* __restrict__ b,
 
 // ---- many rows -----------------------------------------------------------------------------------------------------
 // A tile of kEdge x kEdge outputs, four waves of a quarter each (32 x 32 x 2 instructions, kEdge / 64 squared of them a
-// wave).  Slabs of 32 elements of K in shared memory, rows 36 floats apart (16-byte reads of 8 neighbouring rows then
-// touch every bank once); the next slab is on its way into registers while one is multiplied.  Half-wave h of a lane's
-// operand holds elements 4 h .. 4 h + 3 of every 8, for A and B alike.
-constexpr int kSlab = 32;
-constexpr int kSlabStride = kSlab + 4;
+// wave).  Slabs of K in shared memory, rows 4 floats further apart than they are long (16-byte reads of 8 neighbouring
+// rows then touch every bank once); the next slab is on its way into registers while one is multiplied, and is long enough
+// (2048 cycles of instructions and more a wave) to arrive meanwhile.  Half-wave h of a lane's operand holds elements
+// 4 h .. 4 h + 3 of every 8, for A and B alike.
+constexpr int slab_of(int edge) { return edge == 128 ? 32 : 64; }
 
 template <int kEdge, bool kVec>
 __global__ void __launch_bounds__(256)
 gemm_f32_tile_kernel(const float* __restrict__ a, const float* __restrict__ b, float* __restrict__ c, int m, int n, int k,
                      int part_k) {
+    constexpr int kSlab = slab_of(kEdge);
     constexpr int kFrag = kEdge / 64;                  // 32 x 32 squares along an edge of a wave's quarter
     constexpr int kLoads = kEdge * kSlab / 4 / 256;    // 16-byte loads a thread, matrix and slab
-    __shared__ float as[2][kEdge][kSlabStride];
-    __shared__ float bs[2][kEdge][kSlabStride];
+    __shared__ float as[2][kEdge][kSlab + 4];
+    __shared__ float bs[2][kEdge][kSlab + 4];
     const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
     const long m0 = static_cast<long>(blockIdx.y) * kEdge, n0 = static_cast<long>(blockIdx.x) * kEdge;
     const int k_first = blockIdx.z * part_k, k_end = k_first + part_k < k ? k_first + part_k : k;
@@ -198,9 +199,8 @@ __global__ void __launch_bounds__(256) gemm_f32_sum_kernel(const float* __restri
 }
 
 // Up to here a product is a stream of weights.  Measured against 2048 x 2048 weights (us, streamed : tiled): 14.6 : about 20 at 24
-// rows; at 64 rows the stream's reads of A, four times the weights', make it 46 : 22.
+// rows; at 64 rows the stream's reads of A, four times the weights', make it 46 : 16.
 constexpr int kStreamRows = 32;
-constexpr int kFewTiles = 512;         // fewer tiles than two a compute unit: smaller ones, then parts of K
 constexpr int kPartMin = 256;          // elements of K in a part at least
 constexpr int kPartsMax = 16;
 
@@ -208,20 +208,34 @@ struct F32Plan {
     int edge = 0, parts = 1, part_k = 0;               // edge 0: the streaming kernel
 };
 
+// The tile and the number of parts that keep the chip busiest.  A compute unit's matrix instructions run at one rate however
+// many tiles it holds, so what is lost is what tiles cover past the edges and what the fullest of the 256 units has more than
+// the others; one tile a unit leaves a wave a SIMD and its waits in the open (measured at two thirds of the rate of three);
+// every part writes and reads a plane.
 F32Plan f32_plan(int m, int n, int k) {
-    F32Plan p;
-    p.part_k = k;
-    if (m <= kStreamRows) return p;
-    const auto tiles = [&](int edge) { return static_cast<long>(ceil_div(m, edge)) * ceil_div(n, edge); };
-    p.edge = tiles(128) >= kFewTiles ? 128 : 64;
-    if (tiles(p.edge) < kFewTiles) {
-        const long wanted = ceil_div(kFewTiles, tiles(p.edge));
-        const long most = k / kPartMin > 1 ? k / kPartMin : 1;
-        const int parts = static_cast<int>(wanted < most ? (wanted < kPartsMax ? wanted : kPartsMax) : (most < kPartsMax ? most : kPartsMax));
-        p.part_k = ceil_div(ceil_div(k, parts), kSlab) * kSlab;
-        p.parts = ceil_div(k, p.part_k);
+    F32Plan best;
+    best.part_k = k;
+    if (m <= kStreamRows) return best;
+    constexpr long kUnits = 256;
+    double most = 0.0;
+    for (int edge : {128, 64}) {
+        const long tiles = static_cast<long>(ceil_div(m, edge)) * ceil_div(n, edge);
+        const double inside = static_cast<double>(m) * n / (static_cast<double>(tiles) * edge * edge);
+        for (int wanted = 1; wanted <= kPartsMax && (wanted == 1 || k / wanted >= kPartMin); ++wanted) {
+            const int part_k = ceil_div(ceil_div(k, wanted), 64) * 64, parts = ceil_div(k, part_k);
+            const long each = (tiles * parts + kUnits - 1) / kUnits;                     // of the fullest unit
+            const double busy = static_cast<double>(tiles) * k / (static_cast<double>(each) * kUnits * part_k);
+            const double hidden = edge == 128 ? 1.0 : each >= 3 ? 0.9 : each == 2 ? 0.8 : 0.65;
+            const double worth = inside * busy * hidden / (1.0 + 0.04 * (parts - 1));
+            if (worth > most * 1.001) {
+                most = worth;
+                best.edge = edge;
+                best.parts = parts;
+                best.part_k = parts == 1 ? k : part_k;
+            }
+        }
     }
-    return p;
+    return best;
 }
 
 }  // namespace leone
