@@ -10,8 +10,9 @@
 //   moe_product  gated: act(W_gate x) * (W_up x) of every pair, by its expert's matrices; plain (experts without a gate):
 //                act(W_up x), or act(W_up (weight x)) where the pair's weight multiplies what the expert reads; else
 //                W_down of that, times the pair's weight if there is one, float.  Three kernels: any type and size (float sums of 8-element runs a lane);
-//                bfloat16 on the matrix cores from registers (tiles of 16 or 64 pairs); bfloat16 on the matrix cores
-//                through shared memory (tiles of 128 pairs x 128 rows).
+//                bfloat16 on the matrix cores from registers (tiles of 16 pairs, the inner size shared out over a
+//                workgroup's waves, or of 64 pairs); bfloat16 on the matrix cores through shared memory (tiles of
+//                128 pairs x 128 rows).
 //   moe_combine  a row's pairs summed in the order of its places; a router output beyond the experts with
 //                matrices hands the row itself on (times its weight); a delta that comes along is added.
 //
@@ -54,6 +55,40 @@ struct RouteRule {
     float scale;
 };
 
+// The choice of a row with one router output a lane, whose groups count by their best alone: a lane ranks its group among
+// the groups and its output among the open ones by counting those ahead of it (higher, or the lower index among equals),
+// each read from its lane by one instruction.  Scores are compared as integers in the order of the floats, so that what is
+// not a number has a place too and every rank is some lane's.  Returns the lane's place among the winners, `top` and more if
+// it is none of them.  (Winner after winner by exchanges over the wave, a dozen of them each, and the tiles' places by one thread, the
+// choice and the plan of 8 rows over 35 outputs in 7 groups took 18.5 us; now 7.6.)
+__device__ inline unsigned route_order(float v) {
+    const unsigned bits = __float_as_uint(v + 0.0f);           // -0 counts as 0
+    return bits & 0x80000000u ? ~bits : bits | 0x80000000u;
+}
+__device__ inline int route_rank(float choice, int lane, int total, int group_count, int group_keep) {
+    unsigned mine = lane < total ? route_order(choice) : 0u;
+    if (group_count > 1) {
+        const int size = total / group_count, group = lane / size;
+        unsigned best = 0u;
+        for (int i = 0; i < size; ++i) {
+            const unsigned other = __shfl(mine, group * size + i, kWave);
+            best = other > best ? other : best;
+        }
+        int ahead = 0;
+        for (int h = 0; h < group_count; ++h) {
+            const unsigned other = __builtin_amdgcn_readlane(best, h * size);
+            ahead += other > best || (other == best && h < group) ? 1 : 0;
+        }
+        if (ahead >= group_keep) mine = route_order(-INFINITY);
+    }
+    int ahead = 0;
+    for (int o = 0; o < total; ++o) {
+        const unsigned other = __builtin_amdgcn_readlane(mine, o);
+        ahead += other > mine || (other == mine && o < lane) ? 1 : 0;
+    }
+    return lane < total ? ahead : total;
+}
+
 template <int kSlots>
 __device__ inline void route_row(int row, int lane, const float* __restrict__ logits, const AnyVec& correction,
                                  int* __restrict__ chosen, float* __restrict__ weight, int total, int top, int group_count,
@@ -88,6 +123,26 @@ __device__ inline void route_row(int row, int lane, const float* __restrict__ lo
         s[i] = s[i] / sum;
         choice[i] = e < total ? s[i] + (correction.ptr ? load_any(correction, e) : 0.f) : -INFINITY;
         taken[i] = e >= total;
+    }
+    if (kSlots == 1 && (group_count == 1 || rule.group_best == 1)) {
+        const int rank = route_rank(choice[0], lane, total, group_count, group_keep);
+        const bool won = rank < top;
+        // the winners' scores are added in the order of their ranks
+        float picked = 0.f;
+        for (int i = 0; i < top; ++i) {
+            const unsigned long long who = __ballot(rank == i);
+            picked += __shfl(s[0], __ffsll(who) - 1, kWave);
+        }
+        const float by = rule.renorm ? picked + 1e-20f : 1.0f;
+        if (won) {
+            chosen[static_cast<long>(row) * places + rank] = lane >= shift_from ? lane + always : lane;
+            weight[static_cast<long>(row) * places + rank] = s[0] / by * rule.scale;
+        }
+        for (int i = lane; i < always; i += kWave) {
+            chosen[static_cast<long>(row) * places + top + i] = shift_from + i;
+            weight[static_cast<long>(row) * places + top + i] = 1.0f;
+        }
+        return;
     }
     if (group_count > 1) {
         // a group's score: lane g % 64 keeps group g's in its place g / 64 (there are no more groups than outputs)
@@ -224,13 +279,23 @@ __device__ inline void plan_tiles(const int* __restrict__ chosen, int pairs, int
         if (e >= 0 && e < experts) atomicAdd(&count[e], 1);
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        int at = 0;
-        for (int e = 0; e < experts; ++e) {
+    if (threadIdx.x < kWave) {                          // the first wave: a run of experts a lane, the runs added up over the lanes
+        const int run = (experts + kWave - 1) / kWave, begin = threadIdx.x * run;
+        const int end = begin + run < experts ? begin + run : experts;
+        int tiles = 0;
+        for (int e = begin; e < end; ++e) tiles += (count[e] + tile - 1) / tile;
+        int at = tiles;
+#pragma unroll
+        for (int off = 1; off < kWave; off <<= 1) {
+            const int before = __shfl_up(at, off, kWave);
+            if (static_cast<int>(threadIdx.x) >= off) at += before;
+        }
+        at -= tiles;
+        for (int e = begin; e < end; ++e) {
             first_tile[e] = at;
-            const int tiles = (count[e] + tile - 1) / tile;
-            for (int t = 0; t < tiles && at + t < max_tiles; ++t) tile_expert[at + t] = e;
-            at += tiles;
+            const int mine = (count[e] + tile - 1) / tile;
+            for (int t = 0; t < mine && at + t < max_tiles; ++t) tile_expert[at + t] = e;
+            at += mine;
             count[e] = 0;
         }
     }
@@ -456,7 +521,7 @@ moe_product_mfma_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__
         }
     // A ring of kDepth steps of 32: a step's operands are asked for kDepth steps before the matrix instructions
     // that use them run, so that a wave that has its SIMD to itself still keeps loads on their way.
-    constexpr int kDepth = kPB * kRT >= 16 ? 4 : kPB >= 4 ? 4 : 8;
+    constexpr int kDepth = 4;
     moe_bf16x8 a[kDepth][kRT], a2[kDepth][kGated ? kRT : 1], xb[kDepth][kPB];
 #define LEONE_MOE_FETCH(D, K0)                                                                                  \
     {                                                                                                           \
@@ -509,6 +574,75 @@ moe_product_mfma_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__
             }
         }
     }
+}
+
+// Tiles of 16 pairs, bfloat16 (steps of few rows): every matrix of a chosen expert is read once for a handful of pairs, so
+// its bytes are the bound.  A workgroup takes 16 rows of the matrix (gated: and their up rows) and its four waves share out
+// the inner size, each with eight steps of 32 on their way at a time; their sums meet in shared memory, in the waves' order.
+// (A wave that walked the whole inner size by itself had a quarter of the loads in flight and four times the chain.)
+// Eight rows of 2,048 over 34 experts of 768, four routed places and two for every row (us, before): gated 38 (47), down 19 (24).
+template <int kMode>
+__global__ void __launch_bounds__(kMoeThreads, 3)
+moe_product_stream_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, void* __restrict__ y,
+                          const float* __restrict__ pair_weight, const int* __restrict__ tile_expert,
+                          const int* __restrict__ tile_pairs, int top, int n, int k, int act, float limit) {
+    constexpr bool kGated = kMode == kMoeGated;
+    constexpr int kDepth = 8;
+    __shared__ moe_floatx4 sums[kGated ? 2 : 1][kMoeWaves][kWave];
+    const int tile = blockIdx.x;
+    const int e = tile_expert[tile];
+    if (e < 0) return;
+    const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+    const int c = lane & 15, g = lane >> 4;
+    const int row0 = blockIdx.y * 16;
+    const int pair = tile_pairs[static_cast<long>(tile) * 16 + c];
+    const long matrix = static_cast<long>(n) * k;
+    const bool row_ok = row0 + c < n;
+    const bf16_t* wa = w + static_cast<long>(e) * (kGated ? 2 : 1) * matrix + static_cast<long>(row_ok ? row0 + c : 0) * k;
+    const bf16_t* xrow = x + static_cast<long>(pair < 0 ? 0 : (kMode != kMoeDown ? pair / top : pair)) * k;
+    const int steps = (k + 31) / 32, share = (steps + kMoeWaves - 1) / kMoeWaves;
+    const int last = (wave + 1) * share < steps ? (wave + 1) * share : steps;
+    moe_floatx4 acc = {0.f, 0.f, 0.f, 0.f}, acc2 = {0.f, 0.f, 0.f, 0.f};
+    moe_bf16x8 a[kDepth], a2[kGated ? kDepth : 1], xb[kDepth];
+#define LEONE_MOE_FETCH(D, S)                                                                                  \
+    {                                                                                                          \
+        const int at = 32 * (S) + 8 * g;                                                                       \
+        const bool in = (S) < last && at < k;                                                                  \
+        a[D] = (row_ok && in) ? __builtin_bit_cast(moe_bf16x8, load_streamed16(wa + at)) : moe_zero8();        \
+        if constexpr (kGated)                                                                                  \
+            a2[D] = (row_ok && in) ? __builtin_bit_cast(moe_bf16x8, load_streamed16(wa + matrix + at)) : moe_zero8(); \
+        xb[D] = (pair >= 0 && in) ? moe_load8(xrow + at) : moe_zero8();                                        \
+    }
+#pragma unroll
+    for (int d = 0; d < kDepth; ++d) LEONE_MOE_FETCH(d, wave * share + d)
+    for (int s = wave * share; s < last; s += kDepth) {
+#pragma unroll
+        for (int d = 0; d < kDepth; ++d) {
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[d], xb[d], acc, 0, 0, 0);          // zeros past the wave's share
+            if constexpr (kGated) acc2 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2[d], xb[d], acc2, 0, 0, 0);
+            LEONE_MOE_FETCH(d, s + kDepth + d)
+        }
+    }
+#undef LEONE_MOE_FETCH
+    sums[0][wave][lane] = acc;
+    if constexpr (kGated) sums[1][wave][lane] = acc2;
+    __syncthreads();
+    // thread t: row t % 16 of pair t / 16, which lane 16 (row / 4) + pair of every wave holds at row % 4
+    const int row = threadIdx.x % 16, which = threadIdx.x / 16;
+    const int to = tile_pairs[static_cast<long>(tile) * 16 + which], r = row0 + row;
+    if (to < 0 || r >= n) return;
+    const int from = 16 * (row / 4) + which, j = row % 4;
+    float total = 0.f, total2 = 0.f;
+#pragma unroll
+    for (int v = 0; v < kMoeWaves; ++v) {
+        total += sums[0][v][from][j];
+        if constexpr (kGated) total2 += sums[1][v][from][j];
+    }
+    const long at = static_cast<long>(to) * n + r;
+    if constexpr (kGated) static_cast<bf16_t*>(y)[at] = from_float<bf16_t>(glu_value(total, total2, act, limit));
+    else if constexpr (kMode == kMoePlain)
+        static_cast<bf16_t*>(y)[at] = from_float<bf16_t>(plain_act(pair_weight ? total * pair_weight[to] : total, act));
+    else static_cast<float*>(y)[at] = pair_weight ? total * pair_weight[to] : total;
 }
 
 // Tiles of 128 pairs, bfloat16: a workgroup takes a tile and 128 rows of its expert's matrix (gated: 128 gate rows and
@@ -785,15 +919,19 @@ extern "C" int leone_moe_product(const void* x, const void* w, void* y, const fl
                       "moe_product: the matrix-core kernel takes bfloat16 with an inner size that is a multiple of 8, not %d", k);
         LEONE_REQUIRE(x && w && y && tile_expert && tile_pairs, "moe_product: null pointer");
         LEONE_REQUIRE(max_tiles > 0 && top > 0 && n > 0 && k > 0, "moe_product: %d tiles, sizes %d x %d", max_tiles, n, k);
-        const dim3 cores(max_tiles, ceil_div(n, tile == 128 ? 128 : 64));
+        const dim3 cores(max_tiles, ceil_div(n, tile == 128 ? 128 : tile == 64 ? 64 : 16));
         LEONE_REQUIRE(cores.y <= 65535, "moe_product: %d rows of a matrix are too many", n);
 #define LEONE_MOE_CORES(PB, RT, G)                                                                                      \
     moe_product_mfma_kernel<PB, RT, G><<<cores, kMoeThreads, 0, stream>>>(static_cast<const bf16_t*>(x), static_cast<const bf16_t*>(w), \
                                                                           y, pair_weight, tile_expert, tile_pairs, top, n, k, act, limit)
         if (tile == 16) {
-            if (gated == kMoeGated) LEONE_MOE_CORES(1, 1, kMoeGated);
-            else if (gated == kMoePlain) LEONE_MOE_CORES(1, 1, kMoePlain);
-            else LEONE_MOE_CORES(1, 1, kMoeDown);
+#define LEONE_MOE_STREAM(MODE)                                                                                            \
+    moe_product_stream_kernel<MODE><<<cores, kMoeThreads, 0, stream>>>(static_cast<const bf16_t*>(x), static_cast<const bf16_t*>(w), \
+                                                                       y, pair_weight, tile_expert, tile_pairs, top, n, k, act, limit)
+            if (gated == kMoeGated) LEONE_MOE_STREAM(kMoeGated);
+            else if (gated == kMoePlain) LEONE_MOE_STREAM(kMoePlain);
+            else LEONE_MOE_STREAM(kMoeDown);
+#undef LEONE_MOE_STREAM
         } else if (tile == 64) {
             if (gated == kMoeGated) LEONE_MOE_CORES(4, 1, kMoeGated);
             else if (gated == kMoePlain) LEONE_MOE_CORES(4, 1, kMoePlain);

@@ -1,0 +1,59 @@
+"""The router's choice by ranks, the tiles of many experts, and the experts' products in tiles of 16 pairs, at their edges."""
+import math
+
+import pytest
+import torch
+
+from tests.plain import zukinex_plain as plain
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+F = torch.float64
+
+
+@pytest.mark.parametrize("total,top,count,keep", [(1, 1, 1, 1), (64, 64, 1, 1), (64, 6, 8, 3), (63, 5, 9, 2), (64, 8, 64, 8), (35, 4, 7, 4)])
+def test_ranks_of_one_output_a_lane(total, top, count, keep):
+    """Scores of few values, so that most of them tie: of equals the lower index wins, in groups and among the open outputs."""
+    from leone_amd import ops
+    gen = torch.Generator().manual_seed(total + top)
+    logits = torch.zeros(90, total)
+    correction = torch.randint(-2, 3, (total,), generator=gen).float() * 0.25
+    chosen, weight = ops.route_topk(logits.to(DEV), correction.to(DEV), top, count, keep)
+    score = torch.full((total,), 1.0 / total) + correction
+    groups = score.view(count, -1).max(-1).values
+    order = sorted(range(count), key=lambda g: (-float(groups[g]), g))[:keep]
+    open_ = [e for e in range(total) if e // (total // count) in order]
+    want = sorted(open_, key=lambda e: (-float(score[e]), e))[:top]
+    assert chosen.cpu().tolist() == [want] * 90
+    assert float((weight.cpu() - 1.0 / top).abs().max()) < 1e-6       # equal scores over their sum: rounded a few times
+
+
+def test_scores_that_are_no_numbers_choose_outputs_all_the_same():
+    from leone_amd import ops
+    logits = torch.randn(6, 35)
+    logits[1], logits[2, 4], logits[3] = math.nan, math.inf, -math.inf
+    chosen, weight = ops.route_topk(logits.to(DEV), None, 4, 7, 4)
+    for row in chosen.cpu().tolist():
+        assert len(set(row)) == 4 and all(0 <= e < 35 for e in row)
+    assert bool(torch.isfinite(weight[[0, 4, 5]]).all()) and bool(torch.isnan(weight[[1, 2, 3]]).all())
+
+
+@pytest.mark.parametrize("experts,rows,top", [(1000, 40, 3), (65, 30, 2), (128, 64, 8), (3, 50, 2)])
+def test_products_in_tiles_of_sixteen(experts, rows, top):
+    """Up to 1,000 experts' tiles; experts with more pairs than a tile; inner sizes below, at and off a wave's share."""
+    from leone_amd import ops
+    gen = torch.Generator().manual_seed(experts)
+    chosen = torch.stack([torch.randperm(experts, generator=gen)[:top] for _ in range(rows)]).to(torch.int32)
+    weight = torch.rand(rows, top, generator=gen)
+    for hidden, ff in ((8, 8), (40, 24), (136, 1000)) if experts < 200 else ((40, 24),):
+        x = torch.randn(rows, hidden, generator=gen).bfloat16()
+        up = (torch.randn(experts, 2, ff, hidden, generator=gen) / math.sqrt(hidden)).bfloat16()
+        down = (torch.randn(experts, hidden, ff, generator=gen) / math.sqrt(ff)).bfloat16()
+        got = ops.routed_experts(x.to(DEV), chosen.to(DEV), weight.to(DEV), up.to(DEV), down.to(DEV)).cpu().double()
+        want = torch.zeros(rows, hidden, dtype=F)
+        for t in range(rows):
+            for e, a in zip(chosen[t].tolist(), weight[t].double()):
+                g, u = (up[e, i].double() @ x[t].double() for i in (0, 1))
+                want[t] += a * (down[e].double() @ (plain.silu(g) * u).bfloat16().double())
+        # the middle is rounded to 8 bits on both sides, now and then to neighbours: 2^-8 of some elements of one place's sum
+        assert float((got - want).norm() / want.norm()) < 2e-3
