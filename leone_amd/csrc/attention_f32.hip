@@ -121,11 +121,12 @@ __global__ void __launch_bounds__(kWaves * kWave) attention_f32_kernel(const Att
     for (; t < tiles; t += kWaves) {
         const int start = start_of(t);
         fetch_values(start, block);
-        f32x4 s = {0.f, 0.f, 0.f, 0.f};
+        f32x4 dots[4] = {};                   // four sums side by side: no instruction waits for the one before it
 #pragma unroll
         for (int i = 0; i < kRuns; ++i)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) s = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[i][j], q[i][j], s, 0, 0, 0);
+            for (int j = 0; j < 4; ++j) dots[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[i][j], q[i][j], dots[j], 0, 0, 0);
+        f32x4 s = (dots[0] + dots[1]) + (dots[2] + dots[3]);
         if (t + kWaves < tiles) {             // the keys' registers are free: the next tile's are on their way from here on
             const int next = start_of(t + kWaves);
             block = block_of(next, mapped_next);

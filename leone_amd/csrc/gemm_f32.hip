@@ -1,8 +1,8 @@
 // Single-precision matrix product for the true 32-bit path:
 // C[M,N] = A[M,K] . B[N,K]^T on the float matrix instructions (products and sums in float, fused; no reduced-precision
 // mode).  The reference's scalar backend folds each output left to right in float (crates/leone/src/cpu.rs:1379-1405,
-// 1622-1640); here an output is the sum of a few such chains (below), in an order that the sizes alone fix, so that a
-// launch repeats bit for bit.  (Off the 64-bit product by 2e-7 to 1.4e-6 of its norm over 1 to 1024 rows and K of 512 to 6144,
+// 1622-1640); here an output is one such chain, or the sum of a few (below), in an order that the sizes alone fix, so that a
+// launch repeats bit for bit.  (Off the 64-bit product by 1e-7 to 1e-6 of its norm over 1 to 1024 rows and K of 512 to 6144,
 // never more than the single chain that stood here: 4e-7 to 1.4e-6.)
 //
 // Two kernels.  Few rows (decoding): a product reads every weight once for 2 M operations, so the weights' bytes are the
@@ -15,6 +15,7 @@
 
 namespace leone {
 
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
@@ -51,7 +52,10 @@ gemm_f32_stream_kernel(const float* __restrict__ a, const float* __restrict__ b,
     const float* arow[kTilesM];
 #pragma unroll
     for (int t = 0; t < kTilesM; ++t) arow[t] = a + static_cast<long>(t * 16 + r < m ? t * 16 + r : m - 1) * k;
-    f32x4 acc[kTilesM] = {};
+    // sums side by side, put together at the end: short chains, and what is added rounds at a smaller sum's size (sixteen waves
+    // have registers for two)
+    constexpr int kSums = kWaves == 16 ? 2 : 4;
+    f32x4 acc[kTilesM][kSums] = {};
     f32x4 w[2][kStreamLoads], x[2][kTilesM][kStreamLoads];
     auto fetch = [&](int at, int into) {
 #pragma unroll
@@ -68,7 +72,7 @@ gemm_f32_stream_kernel(const float* __restrict__ a, const float* __restrict__ b,
             for (int j = 0; j < 4; ++j)
 #pragma unroll
                 for (int t = 0; t < kTilesM; ++t)
-                    acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[from][t][i][j], w[from][i][j], acc[t], 0, 0, 0);
+                    acc[t][j % kSums] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[from][t][i][j], w[from][i][j], acc[t][j % kSums], 0, 0, 0);
     };
     // two runs' registers take turns: a run is asked for before the one ahead of it is multiplied
     constexpr int kStep = kWaves * kStreamRun;
@@ -90,9 +94,12 @@ gemm_f32_stream_kernel(const float* __restrict__ a, const float* __restrict__ b,
         if (at < k) multiply(0);
     }
 #pragma unroll
-    for (int t = 0; t < kTilesM; ++t)
+    for (int t = 0; t < kTilesM; ++t) {
+        f32x4 sum = acc[t][0] + acc[t][1];
+        if constexpr (kSums == 4) sum += acc[t][2] + acc[t][3];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) sums[wave][t][(h + i) * kStreamTile + r] = acc[t][i];
+        for (int i = 0; i < 4; ++i) sums[wave][t][(h + i) * kStreamTile + r] = sum[i];
+    }
     __syncthreads();
     for (int e = threadIdx.x; e < kTilesM * 256; e += kWaves * kWave) {
         const int t = e / 256, row = t * 16 + e % 256 / 16, col = n0 + e % 16;
@@ -108,8 +115,9 @@ gemm_f32_stream_kernel(const float* __restrict__ a, const float* __restrict__ b,
 // A tile of kEdge x kEdge outputs, four waves of a quarter each (32 x 32 x 2 instructions, kEdge / 64 squared of them a
 // wave).  Slabs of K in shared memory, rows 4 floats further apart than they are long (16-byte reads of 8 neighbouring
 // rows then touch every bank once); the next slab is on its way into registers while one is multiplied, and is long enough
-// (2048 cycles of instructions and more a wave) to arrive meanwhile.  Half-wave h of a lane's operand holds elements
-// 4 h .. 4 h + 3 of every 8, for A and B alike.
+// (2048 cycles of instructions and more a wave) to arrive meanwhile.  Of every 8 elements the
+// even ones lie first and then the odd ones: half-wave h reads its four at once, and the four instructions take elements 0
+// and 1, 2 and 3, .. of them, so that an output is one chain of fused products, k ascending.
 constexpr int slab_of(int edge) { return edge == 128 ? 32 : 64; }
 
 template <int kEdge, bool kVec>
@@ -141,8 +149,11 @@ gemm_f32_tile_kernel(const float* __restrict__ a, const float* __restrict__ b, f
 #pragma unroll
         for (int i = 0; i < kLoads; ++i) {
             const int idx = threadIdx.x + i * 256, row = idx / (kSlab / 4), at = (idx % (kSlab / 4)) * 4;
-            *reinterpret_cast<f32x4*>(&as[into][row][at]) = ra[i];
-            *reinterpret_cast<f32x4*>(&bs[into][row][at]) = rb[i];
+            const int even = at / 8 * 8 + at % 8 / 2;
+            *reinterpret_cast<f32x2*>(&as[into][row][even]) = f32x2{ra[i][0], ra[i][2]};
+            *reinterpret_cast<f32x2*>(&as[into][row][even + 4]) = f32x2{ra[i][1], ra[i][3]};
+            *reinterpret_cast<f32x2*>(&bs[into][row][even]) = f32x2{rb[i][0], rb[i][2]};
+            *reinterpret_cast<f32x2*>(&bs[into][row][even + 4]) = f32x2{rb[i][1], rb[i][3]};
         }
     };
     fetch(k_first);
@@ -201,6 +212,7 @@ __global__ void __launch_bounds__(256) gemm_f32_sum_kernel(const float* __restri
 // Up to here a product is a stream of weights.  Measured against 2048 x 2048 weights (us, streamed : tiled): 14.6 : about 20 at 24
 // rows; at 64 rows the stream's reads of A, four times the weights', make it 46 : 16.
 constexpr int kStreamRows = 32;
+constexpr int kStreamK = 256;          // a shorter K is no work to share out over four waves
 constexpr int kPartMin = 256;          // elements of K in a part at least
 constexpr int kPartsMax = 16;
 
@@ -215,7 +227,7 @@ struct F32Plan {
 F32Plan f32_plan(int m, int n, int k) {
     F32Plan best;
     best.part_k = k;
-    if (m <= kStreamRows) return best;
+    if (m <= kStreamRows && k >= kStreamK) return best;
     constexpr long kUnits = 256;
     double most = 0.0;
     for (int edge : {128, 64}) {
@@ -261,13 +273,13 @@ extern "C" int leone_gemm_f32(const float* a, const float* b, float* c, float* p
         // waves share out K in runs of 64; sixteen of them where the workgroups are few, so that the chip has loads enough in flight
         const int runs = ceil_div(k, kStreamRun);
         const int tiles = m <= 16 ? 1 : 2;
-        const int waves = runs >= 16 && tiles == 1 && blocks < 512 ? 16 : runs >= 8 ? 8 : 4;
+        const int waves = runs >= 16 && tiles == 1 && blocks < 512 && vec ? 16 : runs >= 8 ? 8 : 4;
 #define LEONE_STREAM(T, W)                                                                                                \
     (vec ? gemm_f32_stream_kernel<T, W, true><<<blocks, W * kWave, 0, stream>>>(a, b, c, m, n, k)                          \
          : gemm_f32_stream_kernel<T, W, false><<<blocks, W * kWave, 0, stream>>>(a, b, c, m, n, k))
 #define LEONE_STREAM_TILES(T) (waves == 8 ? LEONE_STREAM(T, 8) : LEONE_STREAM(T, 4))
         if (tiles == 1) {
-            if (waves == 16) LEONE_STREAM(1, 16);
+            if (waves == 16) gemm_f32_stream_kernel<1, 16, true><<<blocks, 16 * kWave, 0, stream>>>(a, b, c, m, n, k);
             else LEONE_STREAM_TILES(1);
         } else {
             LEONE_STREAM_TILES(2);
