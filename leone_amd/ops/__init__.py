@@ -1593,7 +1593,7 @@ def scan_max_dim() -> int:
     return int(library().leone_scan_max_dim())
 
 
-MEMORY_CHUNKS_FROM = 32     # portions of at least so many rows go through a memory with one decay a head as ``chunked_memory``
+MEMORY_CHUNKS_FROM = 32     # portions of at least so many rows go through a memory as ``chunked_memory``
 
 
 def chunked_memory_supported(dim: int) -> bool:
@@ -1602,26 +1602,37 @@ def chunked_memory_supported(dim: int) -> bool:
 
 def chunked_memory(rows: torch.Tensor, columns: dict, plan: dict, state: torch.Tensor, out: torch.Tensor, heads: int, kv_heads: int,
                    dim: int, vdim: int, *, q_scale: float, k_scale: float, activation: Optional[str] = None,
-                   decay: Optional[torch.Tensor] = None, delta: Optional[tuple] = None, write_state: bool = True) -> None:
-    """The long portions of a step (``plan``: ``chunk_plan`` with chunks of ``leone_chunk_rows()`` rows) through a matrix memory
-    with one decay a head, chunk by chunk on the matrix cores in float: S <- g S + k u^T, o = S^T q, with ``decay`` (float32
-    ``[heads]``) and u = v, or the delta rule's u = beta (v - g S^T k): ``delta`` = (strengths' pre-activations ``[rows, >=
-    heads]``, step sizes' pre-activations likewise, rate_log and step_bias ``[heads]``, unit_eps).  Fills the portions' rows of
-    ``out`` and moves their states."""
+                   decay: Optional[torch.Tensor] = None, gates: Optional[tuple] = None, delta: Optional[tuple] = None,
+                   rotation: Optional[tuple] = None, write_state: bool = True) -> None:
+    """The long portions of a step (``plan``: ``chunk_plan`` with chunks of ``leone_chunk_rows()`` rows) through a matrix memory,
+    chunk by chunk on the matrix cores in float: S <- g S + k u^T, o = S^T q, with ``decay`` (float32 ``[heads]``) and u = v;
+    with ``gates`` = (coefficients g and b of every row and head ``[rows, heads, 2]``, dot ``[rows, heads]`` for the normaliser's
+    read-out) and u = b v; or the delta rule's u = beta (v - g S^T k): ``delta`` = (strengths' pre-activations ``[rows, >= heads]``,
+    step sizes' pre-activations likewise or ``[rows, >= heads * dim]``, rate_log ``[heads]`` and step_bias ``[heads]`` or
+    ``[heads * dim]``, unit_eps).  ``rotation`` = (cos, sin, positions): q and k are rotated first (not for the delta rule).
+    Fills the portions' rows of ``out`` and moves their states."""
     chunks, links = plan["chunks"], plan["links"]
     n, count = rows.shape[0], chunks.shape[0]
-    size = library().leone_chunk_workspace(dim, vdim, 1 if delta is not None else 0)
-    workspace = torch.empty((count * heads * size,), dtype=torch.float32, device=rows.device)
     beta, step_size, rate_log, step_bias, unit_eps = delta if delta is not None else (None, None, None, None, 0.0)
+    each = delta is not None and dim > 1 and step_bias.numel() == heads * dim
+    size = library().leone_chunk_workspace(dim, vdim + (1 if gates is not None else 0), 0 if delta is None else 2 if each else 1)
+    workspace = torch.empty((count * heads * size,), dtype=torch.float32, device=rows.device)
+    steps = heads * dim if each else heads
     beta_at, beta_stride = _strided_rows(beta, "write strengths", n, heads)
-    step_at, step_stride = _strided_rows(step_size, "step sizes", n, heads)
+    step_at, step_stride = _strided_rows(step_size, "step sizes", n, steps)
+    coef, dot = gates if gates is not None else (None, None)
+    cos, sin, positions = rotation if rotation is not None else (None, None, None)
+    head_stride = state[0].numel() // heads
     call("leone_chunked_memory", _dev(rows, "q, k, v", torch.float32), rows.shape[1], columns["q"], columns["k"], columns["v"],
          1 if activation == "silu" else 0, float(q_scale), float(k_scale), float(unit_eps), beta_at, beta_stride, step_at, step_stride,
-         _dev(rate_log, "rate", None, (heads,)), _dev(step_bias, "step bias", None, (heads,)),
+         1 if each else 0, _dev(rate_log, "rate", None, (heads,)), _dev(step_bias, "step bias", None, (steps,)),
          _code(rate_log, "rate") if rate_log is not None else F32,
-         _dev(decay, "decay", torch.float32, (heads,)) if delta is None else 0, _dev(chunks, "chunks", torch.int32), count,
-         _dev(links, "links", torch.int32), links.shape[0], _dev(workspace, "workspace"), _dev(state, "state", torch.float32),
-         state.stride(0), 1 if write_state else 0, _dev(out, "out", torch.float32, (n, heads * vdim)), heads, kv_heads, dim, vdim, _stream())
+         _dev(decay, "decay", torch.float32, (heads,)) if delta is None and gates is None else 0,
+         _dev(coef, "coefficients", torch.float32, (n, heads, 2)), _dev(cos, "rope cos", torch.float32), _dev(sin, "rope sin", torch.float32),
+         2 * cos.shape[1] if cos is not None else 0, cos.shape[0] if cos is not None else 0, _dev(positions, "positions", torch.int32, (n,)),
+         _dev(chunks, "chunks", torch.int32), count, _dev(links, "links", torch.int32), links.shape[0], _dev(workspace, "workspace"),
+         _dev(state, "state", torch.float32), state.stride(0), head_stride, 1 if write_state else 0,
+         _dev(out, "out", torch.float32, (n, heads * vdim)), _dev(dot, "dot", torch.float32, (n, heads)), heads, kv_heads, dim, vdim, _stream())
 
 
 def outer_scan(proj: torch.Tensor, columns: dict, state: torch.Tensor, step, heads: int, dim: int, vdim: int, *,
@@ -1637,9 +1648,9 @@ def outer_scan(proj: torch.Tensor, columns: dict, state: torch.Tensor, step, hea
     pass through it first.
     Returns o float32 ``[rows, heads * vdim]`` and, with gates, (dot, top) for ``head_norm_gate``.
 
-    Single tokens and short portions are walked row by row.  A long portion (``OUTER_CHUNKS``) is cut into chunks
-    that are walked side by side: every chunk from zeros, the chunks' end states chained, every chunk once more
-    from the state it starts with."""
+    Single tokens and short portions are walked row by row.  A long portion goes through as ``chunked_memory``; where that
+    does not take the size (``OUTER_CHUNKS``) it is cut into chunks that are walked side by side: every chunk from zeros, the
+    chunks' end states chained, every chunk once more from the state it starts with."""
     rows, width = proj.shape
     per_head = dim * vdim + (dim + 1 if gates else 0)
     if state.dtype != torch.float32 or state.dim() != 3 or tuple(state.shape[1:]) != (heads, per_head) or not state.is_contiguous():
@@ -1676,14 +1687,15 @@ def outer_scan(proj: torch.Tensor, columns: dict, state: torch.Tensor, step, hea
              _dev(product, "decay products"), _dev(out, "out"), _dev(dot, "dot"), heads, dim, vdim, _stream())
 
     plan = None
-    if not gates and cos is None and chunked_memory_supported(dim):
+    if chunked_memory_supported(dim):
         plan = chunk_plan(step, library().leone_chunk_rows(), MEMORY_CHUNKS_FROM)
         if plan is not None:
             chunked_memory(proj, columns, plan, state, out, heads, heads, dim, vdim, q_scale=q_scale, k_scale=k_scale,
-                           activation=activation, decay=decay, write_state=write_state)
+                           activation=activation, decay=decay, gates=(coef, dot) if gates else None,
+                           rotation=(cos, sin, step.positions) if cos is not None else None, write_state=write_state)
             if plan["short"].shape[0]:
                 walk(plan["short"], state, state if write_state else None)
-            return out, None
+            return (out, (dot, top)) if gates else (out, None)
     else:
         plan = chunk_plan(step, *OUTER_CHUNKS)
     if plan is None:
@@ -1713,7 +1725,8 @@ def delta_scan(qkv: torch.Tensor, columns: dict, beta: torch.Tensor, step_size: 
     ``[rows, heads]`` and ``step_size`` ``[rows, heads * dim]`` may be slices of wider rows.  ``state`` float32
     ``[slots, heads, dim, vdim]``.  Returns o float32 ``[rows, heads * vdim]``.
 
-    Long portions are walked in chunks side by side, as in ``outer_scan``; what a chunk's rows do to a state that
+    Long portions of heads of up to 128 key channels go through as ``chunked_memory``; those of wider heads are walked in
+    chunks side by side, as in ``outer_scan``; what a chunk's rows do to a state that
     comes in is no mere factor here but a matrix ``[dim, dim]``, which the first walk finds by carrying the unit
     vectors along as further columns."""
     rows = qkv.shape[0]
@@ -1738,7 +1751,7 @@ def delta_scan(qkv: torch.Tensor, columns: dict, beta: torch.Tensor, step_size: 
              _dev(transition, "transitions"), _dev(out, "out"), heads, kv_heads, dim, vdim, _stream())
 
     plan = None
-    if per_head and chunked_memory_supported(dim):
+    if chunked_memory_supported(dim) and dim <= library().leone_chunk_max_delta_dim():
         plan = chunk_plan(step, library().leone_chunk_rows(), MEMORY_CHUNKS_FROM)
         if plan is not None:
             chunked_memory(qkv, columns, plan, state, out, heads, kv_heads, dim, vdim, q_scale=q_scale, k_scale=1.0,

@@ -1,0 +1,144 @@
+"""Matrix memories over long portions as products over chunks of 64 rows, with gates, with a rotation, and with a decay for every
+key channel, against the recurrence token by token in double precision."""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+F = torch.float64
+# portions (rows, position they start at): below, at and above a chunk, a last chunk of one row, and a single token beside them
+ENTRIES = [[(70, 0)], [(64, 5), (3, 0), (129, 0)], [(33, 3), (1, 9), (200, 40)]]
+
+
+def step_of(entries):
+    from leone_amd.parts.context import EntryInfo, StepContext
+    slots = [2, 0, 3][:len(entries)]
+    infos, positions, owners = [], [], []
+    for i, (slot, (count, start)) in enumerate(zip(slots, entries)):
+        infos.append(EntryInfo(f"r{i}", slot, len(positions), count, start))
+        positions += range(start, start + count)
+        owners += [i] * count
+    on = lambda values: torch.tensor(values, dtype=torch.int32, device=DEV)
+    return slots, StepContext(rows=len(positions), dtype=torch.float32, device=torch.device(DEV), positions=on(positions), row_entry=on(owners),
+                              entries=infos, entry_slots=on(slots), want_rows=None)
+
+
+def close(got, want, what):
+    # float sums of up to 260 products and decays of as many rows, each rounded to 2^-24 and growing like a random walk: a few
+    # 1e-6 of the result's size; five times that
+    error = float((got.to(F) - want).norm() / (want.norm() + 1e-30))
+    assert error < 2e-5, (what, error)
+
+
+def turned(x, positions, cos, sin):
+    half = cos.shape[1]
+    c, s = cos[positions].to(F), sin[positions].to(F)
+    a, b = x[:, :half], x[:, half:2 * half]
+    return torch.cat([a * c - b * s, b * c + a * s, x[:, 2 * half:]], 1)
+
+
+@pytest.mark.parametrize("entries", ENTRIES, ids=str)
+@pytest.mark.parametrize("heads,dim,vdim,rot", [(2, 256, 64, 0), (1, 24, 17, 8), (3, 64, 15, 64), (2, 130, 16, 130), (1, 200, 500, 0)])
+@pytest.mark.parametrize("gated", [True, False])
+def test_gates_and_rotations(gated, heads, dim, vdim, rot, entries):
+    from leone_amd import ops
+    gen = torch.Generator().manual_seed(dim + rot)
+    slots, step = step_of(entries)
+    rows = step.rows
+    width = 2 * heads * dim + heads * vdim
+    x = torch.randn(rows, width + 2 * heads, generator=gen)
+    x[:, width + heads:] += 2.0
+    x[rows // 3, width + heads:] = -30.0                      # a row that forgets, and one that writes with all its might
+    x[rows // 2, width:width + heads] = 12.0
+    per_head = dim * vdim + (dim + 1 if gated else 0)
+    state = torch.randn(4, heads, per_head, generator=gen)
+    for slot, (_, start) in zip(slots, entries):
+        if start == 0:
+            state[slot] = math.nan
+    bias = torch.randn(2, heads, generator=gen)
+    decay = torch.tensor([0.97, 0.0, 1.0])[:heads]
+    cos, sin = ops.rope_table(1e4, rot, 300, DEV) if rot else (None, None)
+    columns = {"q": 0, "k": heads * dim, "v": 2 * heads * dim, "i": width, "f": width + heads}
+    dev_state = state.to(DEV)
+    out, under = ops.outer_scan(x.to(DEV), columns, dev_state, step, heads, dim, vdim, q_scale=dim ** -0.5, k_scale=0.7, cos=cos, sin=sin,
+                                **(dict(gates={"i_bias": bias[0].to(DEV), "f_bias": bias[1].to(DEV), "cap": 15.0}) if gated
+                                   else dict(decay=decay.to(DEV))))
+    out, x = out.view(rows, heads, vdim).cpu(), x.to(F)
+    at = 0
+    for slot, (count, start) in zip(slots, entries):
+        span = slice(at, at + count)
+        at += count
+        for h in range(heads):
+            q, k = (x[span, b + h * dim:b + (h + 1) * dim] for b in (0, heads * dim))
+            if rot:
+                q, k = (turned(t, range(start, start + count), cos.cpu(), sin.cpu()) for t in (q, k))
+            q, k, v = q * dim ** -0.5, k * 0.7, x[span, 2 * heads * dim + h * vdim:2 * heads * dim + (h + 1) * vdim]
+            before = state[slot, h].to(F) if start else torch.zeros(per_head, dtype=F)
+            memory, norm, top = before[:dim * vdim].view(dim, vdim), before[dim * vdim:dim * vdim + dim], before[-1] if gated else None
+            li = 15.0 * torch.tanh((x[span, width + h] + bias[0, h].to(F)) / 15.0)
+            lf = torch.nn.functional.logsigmoid(15.0 * torch.tanh((x[span, width + heads + h] + bias[1, h].to(F)) / 15.0))
+            want, dots, tops = [], [], []
+            for t in range(count):
+                a, b = decay[h].to(F), 1.0
+                if gated:
+                    new = torch.maximum(lf[t] + top, li[t])
+                    a, b, top = torch.exp(lf[t] + top - new), torch.exp(li[t] - new), new
+                    norm = a * norm + b * k[t]
+                    dots.append(norm @ q[t])
+                    tops.append(top)
+                memory = a * memory + b * torch.outer(k[t], v[t])
+                want.append(memory.T @ q[t])
+            close(out[span, h], torch.stack(want), "out")
+            close(dev_state[slot, h, :dim * vdim].cpu(), memory.reshape(-1), "state")
+            if gated:
+                close(under[0][span, h].cpu(), torch.stack(dots), "normaliser's read-out")
+                close(under[1][span, h].cpu(), torch.stack(tops), "running maximum")
+                close(dev_state[slot, h, dim * vdim:dim * vdim + dim].cpu(), norm, "normaliser")
+
+
+@pytest.mark.parametrize("entries", ENTRIES, ids=str)
+@pytest.mark.parametrize("heads,kv_heads,dim,vdim", [(2, 1, 128, 128), (3, 3, 7, 11), (2, 2, 64, 40), (4, 2, 100, 130)])
+@pytest.mark.parametrize("kind", ["mild", "strong", "extreme"])
+def test_a_decay_for_every_channel(kind, heads, kv_heads, dim, vdim, entries):
+    """Decays near 1, decays that leave nothing after a few rows, and channels that forget everything at one row beside ones
+    that keep everything (which the rows before must not blur)."""
+    from leone_amd import ops
+    gen = torch.Generator().manual_seed(dim)
+    slots, step = step_of(entries)
+    rows, kv = step.rows, kv_heads * dim
+    x = torch.randn(rows, 2 * kv + heads * vdim, generator=gen)
+    beta, size = torch.randn(rows, heads, generator=gen), torch.randn(rows, heads * dim, generator=gen)
+    rate_log, bias = torch.rand(heads, generator=gen) - 1.0, torch.rand(heads * dim, generator=gen) * 3 - 4
+    if kind == "strong":
+        rate_log = rate_log + 3.0
+    if kind == "extreme":
+        size = torch.where(torch.rand(rows, heads * dim, generator=gen) < 0.1, 300.0, -40.0)
+    state = torch.randn(4, heads, dim, vdim, generator=gen)
+    for slot, (_, start) in zip(slots, entries):
+        if start == 0:
+            state[slot] = math.nan
+    dev_state = state.to(DEV)
+    wide = torch.cat([size, beta], 1).to(DEV)                   # both as slices of wider rows
+    out = ops.delta_scan(x.to(DEV), {"q": 0, "k": kv, "v": 2 * kv}, wide[:, heads * dim:], wide[:, :heads * dim], rate_log.to(DEV), bias.to(DEV),
+                         dev_state, step, heads, kv_heads, dim, vdim, dim ** -0.5, 1e-6).view(rows, heads, vdim).cpu()
+    x, at = x.to(F), 0
+    for slot, (count, start) in zip(slots, entries):
+        span = slice(at, at + count)
+        at += count
+        for h in range(heads):
+            g = (h // (heads // kv_heads)) * dim
+            q, k = (t / torch.sqrt((t * t).sum(-1, keepdim=True) + 1e-6) for t in (x[span, g:g + dim], x[span, kv + g:kv + g + dim]))
+            v = x[span, 2 * kv + h * vdim:2 * kv + (h + 1) * vdim]
+            mine = slice(h * dim, (h + 1) * dim)
+            decay = torch.exp(-torch.exp(rate_log[h].to(F)) * torch.nn.functional.softplus((size[span, mine] + bias[mine]).to(F)))
+            strength = torch.sigmoid(beta[span, h].to(F))
+            memory = state[slot, h].to(F) if start else torch.zeros(dim, vdim, dtype=F)
+            want = []
+            for t in range(count):
+                memory = decay[t][:, None] * memory
+                memory = memory + torch.outer(k[t], strength[t] * (v[t] - memory.T @ k[t]))
+                want.append(memory.T @ q[t] * dim ** -0.5)
+            close(out[span, h], torch.stack(want), "out")
+            close(dev_state[slot, h].cpu(), memory, "state")
