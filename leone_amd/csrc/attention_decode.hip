@@ -24,12 +24,18 @@
 // cost far more than the second launch, 8.8 against 6.0 ms a step.)
 //
 // A step in which every row is another request (single decoded tokens) can leave the work on the new token's
-// heads to this kernel (`FromProjection`): it takes the fused q/k/v projection as it comes, normalises and
-// rotates the query heads it needs in registers (per-head RMSNorm, half-split rotation:
-// crates/leone/src/backend.rs:2182-2208, crates/leone/src/cpu.rs:1721-1779), and the workgroup whose keys
-// end with the row's own position does the same for the new key, writes it and the new value into the cache
-// and only then walks its tiles.  One launch fewer a layer; the values are those of the separate kernel
-// (rowwise.hip).  Head sizes that are multiples of 64 only: there a lane holds both halves of its pairs.
+// heads to this kernel (`FromProjection`): it takes the fused q/k/v projection as it comes.  The first wave
+// normalises and rotates the query heads (per-head RMSNorm, half-split rotation:
+// crates/leone/src/backend.rs:2182-2208, crates/leone/src/cpu.rs:1721-1779) for all four, the second and third do the
+// same for the new key and value, write them into the cache and leave them in shared memory, from where the
+// wave with the row's last tile puts them in their places.  One launch fewer a layer; the values are those of the
+// separate kernel (rowwise.hip).  Head sizes that are multiples of 64 only: there a lane holds both halves of its pairs.
+//
+// With few keys a call is a chain of trips to memory, and their order is what it costs: what norms and rotation
+// start from is asked for first, before the row's position is known; then the angles; then the block table; then every
+// wave's first tile, whose way from memory covers the arithmetic on the heads.  Two rows of 100 keys, 8 heads over 2:
+// 9.1 us with the launch (11.1 when every wave made the queries for itself and all waited for the new key to come
+// back from the cache).
 //
 // Operand layouts of the 16x16x32 instruction (lane l, c = l % 16, g = l / 16):
 //   A: row c,    k-slots 8g .. 8g+7        B: column c, k-slots 8g .. 8g+7
@@ -131,6 +137,35 @@ struct ScoreBias {
     int temp_every = 0;
 };
 
+// Which row the workgroup takes when there are more workgroups than compute units.  Rows differ in length, and a unit that
+// happens to get two long ones is what the step waits for: the rows are ranked by their positions, the longest go to the first
+// 256 workgroups, and of the 512 that the chip holds at a time the second half start with the shortest, so that a unit's two
+// make up for each other; beyond that many the longest come first throughout.  The heads of a row are neighbouring workgroups,
+// so that every die gets its share of every row.  64 rows of 300 to 2,304 keys, 8 kv heads: 67 us, in the rows' own order
+// 81.
+constexpr int kOrderedRows = 2 * kWave;
+constexpr int kOrderedUnits = 256;
+__device__ inline int ordered_row(const int* __restrict__ positions, int rows, int head_blocks, int splits, int lane, int& head_block) {
+    const int id = blockIdx.x + rows * blockIdx.y;
+    head_block = id % head_blocks;
+    const int place = id / head_blocks, first = (kOrderedUnits + head_blocks - 1) / head_blocks;
+    const bool paired = splits == 1 && rows * head_blocks <= 2 * kOrderedUnits;
+    const int wanted = paired && place >= first ? rows - 1 - (place - first) : place;
+    int mine[2], ahead[2] = {0, 0};
+#pragma unroll
+    for (int i = 0; i < 2; ++i) mine[i] = lane + i * kWave < rows ? positions[lane + i * kWave] : -1;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+        for (int o = 0; o < kWave && o + i * kWave < rows; ++o) {
+            const int other = __builtin_amdgcn_readlane(mine[i], o), at = o + i * kWave;
+#pragma unroll
+            for (int j = 0; j < 2; ++j) ahead[j] += other > mine[j] || (other == mine[j] && at < lane + j * kWave) ? 1 : 0;
+        }
+    const unsigned long long low = __ballot(lane < rows && ahead[0] == wanted);
+    const unsigned long long high = __ballot(lane + kWave < rows && ahead[1] == wanted);
+    return low ? __ffsll(low) - 1 : kWave + __ffsll(high) - 1;
+}
+
 // kShaped: capped scores, sinks, results turned back (ScoreShape); without it none of that is in the kernel.
 template <int kD16, bool kFused, bool kShaped>
 __global__ void __launch_bounds__(kDecodeThreads, kD16 <= 4 ? 3 : kD16 <= 8 ? 2 : 1)
@@ -139,26 +174,64 @@ attention_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__
                         const int* __restrict__ row_entry, const int* __restrict__ block_table, int max_blocks,
                         float* __restrict__ part_acc, float* __restrict__ part_ml, bf16_t* __restrict__ out,
                         int q_heads, int kv_heads, int page_shift, float to_log2, int window, int splits,
-                        FromProjection from, int keep_first, ScoreBias bias, ScoreShape shape, int chunk) {
+                        FromProjection from, int keep_first, ScoreBias bias, ScoreShape shape, int chunk, int ordered) {
     constexpr int kD = kD16 * 16;
     constexpr int kSteps = (kD16 + 1) / 2;           // 32-element steps of the q.k product
     extern __shared__ float smem[];                   // [waves][columns][kD] accumulators, then m and l
 
     const int group = q_heads / kv_heads;
     const int col_tiles = (group + 15) / 16;
-    const int row = blockIdx.x;
-    const int kvh = blockIdx.y / col_tiles;
-    const int col0 = (blockIdx.y % col_tiles) * 16;
-    const int cols = group - col0 < 16 ? group - col0 : 16;   // query heads handled here
-    const int split = blockIdx.z;
     const int wave = threadIdx.x / kWave;
     const int lane = threadIdx.x % kWave;
+    int row = blockIdx.x, head_block = blockIdx.y;
+    if (ordered) row = ordered_row(positions, gridDim.x, gridDim.y, gridDim.z, lane, head_block);
+    const int kvh = head_block / col_tiles;
+    const int col0 = (head_block % col_tiles) * 16;
+    const int cols = group - col0 < 16 ? group - col0 : 16;   // query heads handled here
+    const int split = blockIdx.z;
     const int c = lane & 15, g = lane >> 4;
     const int page_tokens = 1 << page_shift;
     const int page_mask = page_tokens - 1;
 
+    // What the heads' norms and rotation start from is asked for before anything else is known: the first wave takes the
+    // query heads, the second the new key, the third the new value (`FromProjection`).
+    [[maybe_unused]] constexpr int kHalfSteps = kSteps / 2;
+    [[maybe_unused]] float head_run[kFused ? kSteps : 1][8], head_gain[kFused ? kSteps : 1][8];
+    [[maybe_unused]] const bool head_ok = c < cols;
+    if constexpr (kFused) {
+        // Lane (c, g) of the first wave holds elements 32s + 8g .. + 7 of query head c for every step s; with a head size
+        // that is a multiple of 64 the partner of such a run in the other half of the head is the same lane's run of step
+        // s + kSteps / 2.  The new key lies the same way over the lanes (0, g) of the second wave.
+        static_assert(!kFused || kD16 % 4 == 0, "the fused query path needs a head size that is a multiple of 64");
+        const long width = static_cast<long>(q_heads + 2 * kv_heads) * kD;
+        if (wave == 0 || (wave == 1 && from.k_out != nullptr)) {
+            const long head_at = static_cast<long>(wave == 0 ? kvh * group + col0 + (head_ok ? c : 0) : q_heads + kvh) * kD;
+            const AnyVec gain = wave == 0 ? from.q_gain : from.k_gain;
+#pragma unroll
+            for (int s = 0; s < kSteps; ++s) {
+                if (gain.ptr) load_any8(gain, 32 * s + 8 * g, head_gain[s]);
+                load_projection8(from, width, row, head_at + 32 * s + 8 * g, head_run[s]);
+            }
+        } else if (wave == 2 && from.k_out != nullptr) {
+            if (8 * lane < kD)      // values are copied as they are: lane l has elements 8 l .. 8 l + 7 (a head has at most 256)
+                load_projection8(from, width, row, static_cast<long>(q_heads + kv_heads + kvh) * kD + 8 * lane, head_run[0]);
+        }
+    }
+
     const int n = positions[row] + 1;                                    // keys 0 .. n-1 exist
     const int lo = first_key(n - 1, window, chunk);                      // first key in reach
+    // (asked for ahead of any key: loads come back in the order they were asked for)
+    [[maybe_unused]] float angle_cos[kFused ? kHalfSteps : 1][8], angle_sin[kFused ? kHalfSteps : 1][8];
+    if constexpr (kFused) {
+        if (from.cos_table != nullptr && (wave == 0 || (wave == 1 && from.k_out != nullptr))) {
+            const long angles = static_cast<long>(n - 1 < from.table_positions ? n - 1 : from.table_positions - 1) * (kD / 2);
+#pragma unroll
+            for (int s = 0; s < kHalfSteps; ++s) {
+                load_any8(AnyVec{from.cos_table, kF32}, angles + 32 * s + 8 * g, angle_cos[s]);
+                load_any8(AnyVec{from.sin_table, kF32}, angles + 32 * s + 8 * g, angle_sin[s]);
+            }
+        }
+    }
     // this lane's column is query head kvh * group + col0 + c
     const float to_log2_row = bias.temp_every > 0
         ? to_log2 * (1.0f + bias.temp_coef * logf(static_cast<float>(n / bias.temp_every + 1))) : to_log2;
@@ -205,88 +278,6 @@ attention_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__
         const int b = key >> page_shift;
         return b >= first_page ? pages[b - first_page] : pages[n_win_pages + b - kept_first_page];
     };
-    if constexpr (kFused) {
-        // The workgroup whose keys end with the row's own position makes that position's key and value and
-        // writes them into the cache; its waves read them from there after the barrier.  (With more than 16
-        // query heads a kv head several workgroups do, each for itself: the same bytes.)
-        if (from.k_out != nullptr && my_begin < my_end && my_end == n_tiles) {
-            const long width = static_cast<long>(q_heads + 2 * kv_heads) * kD;
-            const int pos = n - 1;
-            const int page = table[pos >> page_shift];
-            if (page >= 0) {                              // the host reserves the page before the launch
-                const long base = (static_cast<long>(page) * kv_heads + kvh) * page_tokens * kD;
-                const int token = pos & page_mask;
-                constexpr int kHalfRuns = kD16;           // runs of 8 elements in half a head
-                if (wave == 0) {
-                    // lane L < kHalfRuns: elements 8L .. 8L+7 and their partners in the other half
-                    const bool mine = lane < kHalfRuns;
-                    float a[8], b[8];
-                    float ss = 0.f;
-                    // gains and angles are asked for together with the projection, not after the sum of squares
-                    float ga[8], gb[8], cs[8], sn[8];
-                    if (mine) {
-                        if (from.k_gain.ptr) {
-                            load_any8(from.k_gain, 8 * lane, ga);
-                            load_any8(from.k_gain, kD / 2 + 8 * lane, gb);
-                        }
-                        if (from.cos_table != nullptr) {
-                            const int tpos = pos < from.table_positions ? pos : from.table_positions - 1;
-                            load_any8(AnyVec{from.cos_table, kF32}, static_cast<long>(tpos) * (kD / 2) + 8 * lane, cs);
-                            load_any8(AnyVec{from.sin_table, kF32}, static_cast<long>(tpos) * (kD / 2) + 8 * lane, sn);
-                        }
-                        load_projection8(from, width, row, static_cast<long>(q_heads + kvh) * kD + 8 * lane, a);
-                        load_projection8(from, width, row, static_cast<long>(q_heads + kvh) * kD + kD / 2 + 8 * lane, b);
-#pragma unroll
-                        for (int i = 0; i < 8; ++i) {
-                            ss = fmaf(a[i], a[i], ss);
-                            ss = fmaf(b[i], b[i], ss);
-                        }
-                    }
-                    ss = wave_sum(ss);
-                    if (mine) {
-                        if (from.k_gain.ptr) {
-                            const float inv = 1.0f / sqrtf(ss / static_cast<float>(kD) + from.eps);
-#pragma unroll
-                            for (int i = 0; i < 8; ++i) {
-                                a[i] = (a[i] * ga[i]) * inv;
-                                b[i] = (b[i] * gb[i]) * inv;
-                            }
-                        }
-                        if (from.cos_table != nullptr) {
-#pragma unroll
-                            for (int i = 0; i < 8; ++i) {
-                                const float ru = a[i] * cs[i] - b[i] * sn[i];
-                                const float rv = a[i] * sn[i] + b[i] * cs[i];
-                                a[i] = ru;
-                                b[i] = rv;
-                            }
-                        }
-                        uint4 lo, hi;
-                        unsigned* wl = reinterpret_cast<unsigned*>(&lo);
-                        unsigned* wh = reinterpret_cast<unsigned*>(&hi);
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            wl[i] = bf16_bits_from_float(a[2 * i]) | (static_cast<unsigned>(bf16_bits_from_float(a[2 * i + 1])) << 16);
-                            wh[i] = bf16_bits_from_float(b[2 * i]) | (static_cast<unsigned>(bf16_bits_from_float(b[2 * i + 1])) << 16);
-                        }
-                        *reinterpret_cast<uint4*>(from.k_out + base + key_offset(token, 8 * lane, page_tokens)) = lo;
-                        *reinterpret_cast<uint4*>(from.k_out + base + key_offset(token, kD / 2 + 8 * lane, page_tokens)) = hi;
-                    }
-                } else if (wave == 1) {
-                    // values are copied as they are, one element of one token at a time
-                    const long value_at = static_cast<long>(q_heads + kv_heads + kvh) * kD;
-                    for (int e = 8 * lane; e < kD; e += 8 * kWave) {
-                        float v[8];
-                        load_projection8(from, width, row, value_at + e, v);
-#pragma unroll
-                        for (int i = 0; i < 8; ++i)
-                            from.v_out[base + value_offset(token, e + i, kD)] = from_float<bf16_t>(v[i]);
-                    }
-                }
-            }
-            __threadfence_block();                         // the waves of this workgroup read what was written
-        }
-    }
     __syncthreads();
 
     // One 32-key tile in two steps: `issue` asks for its keys and values, `finish` does the arithmetic.  The
@@ -331,61 +322,73 @@ attention_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__
 
     // Q^T operand: column c is query head kvh*group + col0 + c.
     bf16x8 qreg[kSteps];
+    // The workgroup whose keys end with the row's own position writes that position's key and value into the cache (with
+    // more than 16 query heads a kv head several do: the same bytes) and puts them into the tile that holds them itself: no
+    // wave waits for a write to come back.
+    const bool writes = kFused && from.k_out != nullptr && my_begin < my_end && my_end == n_tiles;
+    // They stand, until the waves merge, where the wave that works on the last tile puts its results; the queries in the
+    // next wave's place, until every wave has taken them.
+    [[maybe_unused]] const int last_wave = writes ? (n_tiles - 1 - my_begin) % kDecodeWaves : 0;
+    [[maybe_unused]] bf16_t* new_key = reinterpret_cast<bf16_t*>(smem + static_cast<long>(last_wave) * cols * kD);
+    [[maybe_unused]] bf16_t* new_value = new_key + kD;
     if constexpr (kFused) {
-        // Lane (c, g) holds elements 32s + 8g .. + 7 of head c for every step s; with a head size that is a
-        // multiple of 64 the partner of such a run in the other half of the head is the same lane's run of
-        // step s + kSteps / 2.
-        static_assert(!kFused || kD16 % 4 == 0, "the fused query path needs a head size that is a multiple of 64");
-        constexpr int kHalfSteps = kSteps / 2;
-        const bool head_ok = c < cols;
-        const long width = static_cast<long>(q_heads + 2 * kv_heads) * kD;
-        const long head_at = static_cast<long>(kvh * group + col0 + (head_ok ? c : 0)) * kD;
-        // everything is asked for first (heads, gains, angles), 16 or 32 bytes at a time, then worked on
-        float v[kSteps][8], gain[kSteps][8], cs[kHalfSteps][8], sn[kHalfSteps][8];
-        const int tpos = n - 1 < from.table_positions ? n - 1 : from.table_positions - 1;
-#pragma unroll
-        for (int s = 0; s < kSteps; ++s) {
-            load_projection8(from, width, row, head_at + 32 * s + 8 * g, v[s]);
-            if (from.q_gain.ptr) load_any8(from.q_gain, 32 * s + 8 * g, gain[s]);
-        }
-        if (from.cos_table != nullptr) {
-#pragma unroll
-            for (int s = 0; s < kHalfSteps; ++s) {
-                load_any8(AnyVec{from.cos_table, kF32}, static_cast<long>(tpos) * (kD / 2) + 32 * s + 8 * g, cs[s]);
-                load_any8(AnyVec{from.sin_table, kF32}, static_cast<long>(tpos) * (kD / 2) + 32 * s + 8 * g, sn[s]);
-            }
-        }
-        float ss = 0.f;
-#pragma unroll
-        for (int s = 0; s < kSteps; ++s)
-#pragma unroll
-            for (int i = 0; i < 8; ++i) ss = fmaf(v[s][i], v[s][i], ss);
-        ss += __shfl_xor(ss, 16, kWave);                  // the four lanes that share head c
-        ss += __shfl_xor(ss, 32, kWave);
-        if (from.q_gain.ptr) {
-            const float inv = 1.0f / sqrtf(ss / static_cast<float>(kD) + from.eps);
+        bf16_t* queries = reinterpret_cast<bf16_t*>(smem + static_cast<long>((last_wave + 1) % kDecodeWaves) * cols * kD);
+        const int pos = n - 1;
+        const int page = writes ? table[pos >> page_shift] : -1;             // the host reserves the page before the launch
+        const long base = (static_cast<long>(page < 0 ? 0 : page) * kv_heads + kvh) * page_tokens * kD;
+        const int token = pos & page_mask;
+        if (wave == 0 || (wave == 1 && writes)) {
+            const AnyVec gain = wave == 0 ? from.q_gain : from.k_gain;
+            float ss = 0.f;
 #pragma unroll
             for (int s = 0; s < kSteps; ++s)
 #pragma unroll
-                for (int i = 0; i < 8; ++i) v[s][i] = (v[s][i] * gain[s][i]) * inv;
-        }
-        if (from.cos_table != nullptr) {
+                for (int i = 0; i < 8; ++i) ss = fmaf(head_run[s][i], head_run[s][i], ss);
+            ss += __shfl_xor(ss, 16, kWave);                  // the four lanes that share head c
+            ss += __shfl_xor(ss, 32, kWave);
+            if (gain.ptr) {
+                const float inv = 1.0f / sqrtf(ss / static_cast<float>(kD) + from.eps);
 #pragma unroll
-            for (int s = 0; s < kHalfSteps; ++s) {
+                for (int s = 0; s < kSteps; ++s)
 #pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    const float a = v[s][i], b = v[s + kHalfSteps][i];
-                    v[s][i] = a * cs[s][i] - b * sn[s][i];
-                    v[s + kHalfSteps][i] = a * sn[s][i] + b * cs[s][i];
+                    for (int i = 0; i < 8; ++i) head_run[s][i] = (head_run[s][i] * head_gain[s][i]) * inv;
+            }
+            if (from.cos_table != nullptr) {
+#pragma unroll
+                for (int s = 0; s < kHalfSteps; ++s)
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) {
+                        const float a = head_run[s][i], b = head_run[s + kHalfSteps][i];
+                        head_run[s][i] = a * angle_cos[s][i] - b * angle_sin[s][i];
+                        head_run[s + kHalfSteps][i] = a * angle_sin[s][i] + b * angle_cos[s][i];
+                    }
+            }
+#pragma unroll
+            for (int s = 0; s < kSteps; ++s) {
+                bf16x8 rounded;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) rounded[i] = static_cast<__bf16>(head_run[s][i]);
+                const uint4 bits = __builtin_bit_cast(uint4, rounded);
+                if (wave == 0) {
+                    if (head_ok) *reinterpret_cast<uint4*>(queries + c * kD + 32 * s + 8 * g) = bits;
+                } else if (c == 0) {
+                    *reinterpret_cast<uint4*>(new_key + 32 * s + 8 * g) = bits;
+                    if (page >= 0) *reinterpret_cast<uint4*>(from.k_out + base + key_offset(token, 32 * s + 8 * g, page_tokens)) = bits;
                 }
             }
+        } else if (wave == 2 && writes && 8 * lane < kD) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const bf16_t value = from_float<bf16_t>(head_run[0][i]);
+                new_value[8 * lane + i] = value;
+                if (page >= 0) from.v_out[base + value_offset(token, 8 * lane + i, kD)] = value;
+            }
         }
+        __syncthreads();
 #pragma unroll
-        for (int s = 0; s < kSteps; ++s)
-#pragma unroll
-            for (int i = 0; i < 8; ++i) qreg[s][i] = head_ok ? static_cast<__bf16>(v[s][i]) : static_cast<__bf16>(0.0f);
+        for (int s = 0; s < kSteps; ++s) qreg[s] = head_ok ? load8(queries + c * kD + 32 * s + 8 * g) : zero8();
+        __syncthreads();                                      // taken: the place is that wave's own from here on
     } else {
-        const bool head_ok = c < cols;
         const bf16_t* qrow = q + (static_cast<long>(row) * q_heads + kvh * group + col0 + (head_ok ? c : 0)) * kD;
 #pragma unroll
         for (int s = 0; s < kSteps; ++s) {
@@ -415,32 +418,50 @@ attention_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__
             unmapped = true;
             any = false;
         }
-        if (!full || kD16 % 2 != 0 || __any(unmapped)) {
-            // what was read in place of nothing counts as zero
+        if constexpr (kD16 % 2 != 0) {
+            // the last step reaches past the head: what was read in place of nothing counts as zero there
 #pragma unroll
             for (int s = 0; s < kSteps; ++s) {
                 const bool in_head = 32 * s + 8 * g < kD;
                 if (!(va && in_head)) r.xa[s] = zero8();
                 if (!(vb && in_head)) r.xb[s] = zero8();
             }
-            const bool whole = (run0 >= lo || run0 + 8 <= keep) && run0 + 8 <= n;
+        }
+        if (!full || __any(unmapped)) {
+            // A key out of reach spoils its own scores only, which are set below.  Values out of reach may be anything, even
+            // NaN: a weight of zero is not enough.  Bits of this lane's eight keys, two a word:
+            unsigned keep_bits[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                keep_bits[i] = any ? (in_reach(run0 + 2 * i) ? 0x0000ffffu : 0u) | (in_reach(run0 + 2 * i + 1) ? 0xffff0000u : 0u) : 0u;
 #pragma unroll
             for (int dt = 0; dt < kD16; ++dt) {
-                if (!any) {
-                    r.xv[dt] = zero8();
-                } else if (!whole) {
-                    // slots outside [lo, n) may hold anything, even NaN: clear them, a zero weight is not enough
-                    uint4 raw = __builtin_bit_cast(uint4, r.xv[dt]);
-                    unsigned* w = reinterpret_cast<unsigned*>(&raw);
+                uint4 raw = __builtin_bit_cast(uint4, r.xv[dt]);
+                raw.x &= keep_bits[0], raw.y &= keep_bits[1], raw.z &= keep_bits[2], raw.w &= keep_bits[3];
+                r.xv[dt] = __builtin_bit_cast(bf16x8, raw);
+            }
+        }
+        if constexpr (kFused) {
+            if (writes && u == n_tiles - 1) {              // the row's own key and value, which the cache may not show yet
+                const int pos = n - 1;
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const int e0 = run0 + 2 * i, e1 = e0 + 1;
-                        unsigned mask = 0u;
-                        if (in_reach(e0)) mask |= 0x0000ffffu;
-                        if (in_reach(e1)) mask |= 0xffff0000u;
-                        w[i] &= mask;
+                for (int s = 0; s < kSteps; ++s) {
+                    if (ka == pos) r.xa[s] = load8(new_key + 32 * s + 8 * g);
+                    if (kb == pos) r.xb[s] = load8(new_key + 32 * s + 8 * g);
+                }
+                if (run0 <= pos && pos < run0 + 8) {
+                    const int at = (pos - run0) >> 1;
+                    const bool high = (pos - run0) & 1;
+#pragma unroll
+                    for (int dt = 0; dt < kD16; ++dt) {
+                        uint4 raw = __builtin_bit_cast(uint4, r.xv[dt]);
+                        unsigned* w = reinterpret_cast<unsigned*>(&raw);
+                        const unsigned value = new_value[16 * dt + c].bits;
+#pragma unroll
+                        for (int i = 0; i < 4; ++i)
+                            if (i == at) w[i] = high ? (w[i] & 0x0000ffffu) | (value << 16) : (w[i] & 0xffff0000u) | value;
+                        r.xv[dt] = __builtin_bit_cast(bf16x8, raw);
                     }
-                    r.xv[dt] = __builtin_bit_cast(bf16x8, raw);
                 }
             }
         }
@@ -650,13 +671,14 @@ static void launch_decode(const void* q, const void* k_pool, const void* v_pool,
     const int group = q_heads / kv_heads;
     dim3 grid(rows, kv_heads * ((group + 15) / 16), splits);
     const size_t smem = decode_smem_bytes(kD16 * 16, group, max_blocks);
+    const int ordered = rows > 1 && rows <= kOrderedRows && static_cast<long>(grid.x) * grid.y * grid.z > kOrderedUnits ? 1 : 0;
     const float to_log2 = scale * 1.4426950408889634f;
     if constexpr (kD16 % 4 == 0) {
         if (from != nullptr) {
             attention_decode_kernel<kD16, true, false><<<grid, kDecodeThreads, smem, stream>>>(
                 nullptr, static_cast<const bf16_t*>(k_pool), static_cast<const bf16_t*>(v_pool), positions, row_entry,
                 block_table, max_blocks, part_acc, part_ml, static_cast<bf16_t*>(out), q_heads, kv_heads, page_shift,
-                to_log2, window, splits, *from, keep_first, bias, ScoreShape{}, chunk);
+                to_log2, window, splits, *from, keep_first, bias, ScoreShape{}, chunk, ordered);
             return;
         }
     }
@@ -664,7 +686,7 @@ static void launch_decode(const void* q, const void* k_pool, const void* v_pool,
     attention_decode_kernel<kD16, false, SHAPED><<<grid, kDecodeThreads, smem, stream>>>(                                    \
         static_cast<const bf16_t*>(q), static_cast<const bf16_t*>(k_pool), static_cast<const bf16_t*>(v_pool),               \
         positions, row_entry, block_table, max_blocks, part_acc, part_ml, static_cast<bf16_t*>(out), q_heads, kv_heads,      \
-        page_shift, to_log2, window, splits, FromProjection{}, keep_first, bias, shape, chunk)
+        page_shift, to_log2, window, splits, FromProjection{}, keep_first, bias, shape, chunk, ordered)
     if (shape.any()) LEONE_DECODE_LAUNCH(true);
     else LEONE_DECODE_LAUNCH(false);
 #undef LEONE_DECODE_LAUNCH
