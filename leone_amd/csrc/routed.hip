@@ -11,8 +11,7 @@
 //                act(W_up x), or act(W_up (weight x)) where the pair's weight multiplies what the expert reads; else
 //                W_down of that, times the pair's weight if there is one, float.  Three kernels: any type and size (float sums of 8-element runs a lane);
 //                bfloat16 on the matrix cores from registers (tiles of 16 pairs, the inner size shared out over a
-//                workgroup's waves, or of 64 pairs); bfloat16 on the matrix cores through shared memory (tiles of
-//                128 pairs x 128 rows).
+//                workgroup's waves); bfloat16 on the matrix cores through shared memory (tiles of 64 pairs).
 //   moe_combine  a row's pairs summed in the order of its places; a router output beyond the experts with
 //                matrices hands the row itself on (times its weight); a delta that comes along is added.
 //
@@ -464,11 +463,9 @@ moe_product_kernel(const T* __restrict__ x, const T* __restrict__ w, void* __res
 }
 
 
-// The same products on the matrix cores, bfloat16: a workgroup takes a tile of 16 * kPB pairs of one expert and 64
-// rows of its matrix, a wave 16 of those rows against all the tile's pairs (v_mfma_f32_16x16x32_bf16: the rows are
-// one operand, 16 pairs the other; lane (c, g) holds elements 8 g .. 8 g + 7 of a step of 32 of row c and of pair c,
-// and gets rows 4 g .. 4 g + 3 of pair c).  Inner sizes are multiples of 8; a step's lanes beyond the inner size
-// bring zeros.
+// The same products on the matrix cores, bfloat16 (v_mfma_f32_16x16x32_bf16: rows of the matrix are one operand, 16 pairs the
+// other; lane (c, g) holds elements 8 g .. 8 g + 7 of a step of 32 of row c and of pair c, and gets rows 4 g .. 4 g + 3 of
+// pair c).  Inner sizes are multiples of 8; what lies beyond the inner size counts as zeros.
 typedef __bf16 moe_bf16x8 __attribute__((ext_vector_type(8)));
 typedef float moe_floatx4 __attribute__((ext_vector_type(4)));
 
@@ -478,102 +475,6 @@ __device__ inline moe_bf16x8 moe_load8(const bf16_t* p) {
 __device__ inline moe_bf16x8 moe_zero8() {
     const uint4 z = {0u, 0u, 0u, 0u};
     return __builtin_bit_cast(moe_bf16x8, z);
-}
-
-template <int kPB, int kRT, int kMode>
-__global__ void __launch_bounds__(kMoeThreads)
-moe_product_mfma_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, void* __restrict__ y,
-                        const float* __restrict__ pair_weight, const int* __restrict__ tile_expert,
-                        const int* __restrict__ tile_pairs, int top, int n, int k, int act, float limit) {
-    constexpr bool kGated = kMode == kMoeGated;
-    // kPB blocks of 16 pairs a tile; kRT blocks of 16 rows a wave (a workgroup takes 64 * kRT rows): the more of
-    // both, the fewer times the rows of the matrix and of x are fetched again by other workgroups.
-    constexpr int kTile = 16 * kPB;
-    const int tile = blockIdx.x;
-    const int e = tile_expert[tile];
-    if (e < 0) return;
-    const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-    const int c = lane & 15, g = lane >> 4;
-    const int row0 = (blockIdx.y * kMoeWaves + wave) * 16 * kRT;
-    if (row0 >= n) return;
-    int pair[kPB];
-    const bf16_t* xrow[kPB];
-#pragma unroll
-    for (int b = 0; b < kPB; ++b) {
-        pair[b] = tile_pairs[static_cast<long>(tile) * kTile + 16 * b + c];
-        xrow[b] = x + static_cast<long>(pair[b] < 0 ? 0 : (kMode != kMoeDown ? pair[b] / top : pair[b])) * k;
-    }
-    const long matrix = static_cast<long>(n) * k;
-    bool row_ok[kRT];
-    const bf16_t* wa[kRT];
-#pragma unroll
-    for (int t = 0; t < kRT; ++t) {
-        row_ok[t] = row0 + 16 * t + c < n;
-        wa[t] = w + static_cast<long>(e) * (kGated ? 2 : 1) * matrix + static_cast<long>(row_ok[t] ? row0 + 16 * t + c : 0) * k;
-    }
-    moe_floatx4 acc[kRT][kPB], acc2[kGated ? kRT : 1][kPB];
-#pragma unroll
-    for (int t = 0; t < kRT; ++t)
-#pragma unroll
-        for (int b = 0; b < kPB; ++b) {
-            acc[t][b] = moe_floatx4{0.f, 0.f, 0.f, 0.f};
-            if constexpr (kGated) acc2[t][b] = moe_floatx4{0.f, 0.f, 0.f, 0.f};
-        }
-    // A ring of kDepth steps of 32: a step's operands are asked for kDepth steps before the matrix instructions
-    // that use them run, so that a wave that has its SIMD to itself still keeps loads on their way.
-    constexpr int kDepth = 4;
-    moe_bf16x8 a[kDepth][kRT], a2[kDepth][kGated ? kRT : 1], xb[kDepth][kPB];
-#define LEONE_MOE_FETCH(D, K0)                                                                                  \
-    {                                                                                                           \
-        const int at = (K0) + 8 * g;                                                                            \
-        const bool in = at < k;                                                                                 \
-        _Pragma("unroll") for (int t = 0; t < kRT; ++t) {                                                       \
-            a[D][t] = (row_ok[t] && in) ? moe_load8(wa[t] + at) : moe_zero8();                                  \
-            if constexpr (kGated) a2[D][t] = (row_ok[t] && in) ? moe_load8(wa[t] + matrix + at) : moe_zero8();  \
-        }                                                                                                       \
-        _Pragma("unroll") for (int b = 0; b < kPB; ++b)                                                         \
-            xb[D][b] = (pair[b] >= 0 && in) ? moe_load8(xrow[b] + at) : moe_zero8();                            \
-    }
-#pragma unroll
-    for (int d = 0; d < kDepth; ++d) LEONE_MOE_FETCH(d, 32 * d)
-    for (int k0 = 0; k0 < k; k0 += 32 * kDepth) {
-#pragma unroll
-        for (int d = 0; d < kDepth; ++d) {
-            if (k0 + 32 * d < k) {                                   // the same for the whole workgroup
-#pragma unroll
-                for (int t = 0; t < kRT; ++t) {
-#pragma unroll
-                    for (int b = 0; b < kPB; ++b) {
-                        acc[t][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[d][t], xb[d][b], acc[t][b], 0, 0, 0);
-                        if constexpr (kGated)
-                            acc2[t][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2[d][t], xb[d][b], acc2[t][b], 0, 0, 0);
-                    }
-                }
-            }
-            LEONE_MOE_FETCH(d, k0 + 32 * (kDepth + d))
-        }
-    }
-#undef LEONE_MOE_FETCH
-#pragma unroll
-    for (int b = 0; b < kPB; ++b) {
-        if (pair[b] < 0) continue;
-        const float scale = kGated || !pair_weight ? 1.f : pair_weight[pair[b]];
-#pragma unroll
-        for (int t = 0; t < kRT; ++t) {
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int r = row0 + 16 * t + 4 * g + j;
-                if (r >= n) continue;
-                if constexpr (kGated)
-                    static_cast<bf16_t*>(y)[static_cast<long>(pair[b]) * n + r] =
-                        from_float<bf16_t>(glu_value(acc[t][b][j], acc2[t][b][j], act, limit));
-                else if constexpr (kMode == kMoePlain)
-                    static_cast<bf16_t*>(y)[static_cast<long>(pair[b]) * n + r] = from_float<bf16_t>(plain_act(acc[t][b][j] * scale, act));
-                else
-                    static_cast<float*>(y)[static_cast<long>(pair[b]) * n + r] = acc[t][b][j] * scale;
-            }
-        }
-    }
 }
 
 // Tiles of 16 pairs, bfloat16 (steps of few rows): every matrix of a chosen expert is read once for a handful of pairs, so
@@ -645,34 +546,42 @@ moe_product_stream_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict
     else static_cast<float*>(y)[at] = pair_weight ? total * pair_weight[to] : total;
 }
 
-// Tiles of 128 pairs, bfloat16: a workgroup takes a tile and 128 rows of its expert's matrix (gated: 128 gate rows and
-// their up rows), in chunks of 64 of the inner size that go through shared memory: a row's chunk is one line of 128
-// bytes, fetched whole by eight neighbouring threads (rows of a matrix lie a power of two apart, so lines that are
-// only half used at a time push one another out of the caches before their other half is asked for).  While the
-// waves work on a chunk the next is on its way from memory into registers.  In shared memory a chunk lies as two
-// halves of 32 elements, rows one after the other within a half: the 16 rows of an operand are one kilobyte that the
-// 64 lanes read in one piece.  The four waves take 64 rows x 64 pairs each: 4 + 4 operands for 16 matrix instructions.
-constexpr int kBigPairs = 128;
+// Tiles of 64 pairs, bfloat16: a workgroup takes a tile and 128 rows of its expert's matrix (gated: 64 gate rows and their
+// up rows), in chunks of 64 of the inner size that go through shared memory: a row's chunk is one line of 128 bytes, fetched
+// whole by eight neighbouring threads (rows of a matrix lie a power of two apart, so lines that are only half used at a time
+// push one another out of the caches before their other half is asked for).  In shared memory a chunk lies as two halves of 32
+// elements, rows one after the other within a half: the 16 rows of an operand are one kilobyte that the 64 lanes read in one
+// piece.  The four waves take 64 rows x 32 pairs each.
+//
+// What bounds it is the way from memory: a chunk is worked off in half a microsecond and takes two to arrive.  So two chunks
+// are on their way in registers while a third is worked on and a fourth lies ready behind it in shared memory, and the tile
+// is small enough for two to three workgroups a compute unit.  (One chunk ahead, with tiles of 128 pairs x 256 rows, had 0.34
+// PFLOP/s; tiles of 64 pairs straight from memory into registers were slower still; tiles of 128 pairs worked this way take
+// eight waves, of which fewer workgroups fit: 312 us at the largest of these.)  Measured, both products of 32 experts, width
+// 2,048 and 768 (us, before): 1,093 pairs 88 (161), 2,533 pairs 135 (282), 7,358 pairs 216 (237).
+constexpr int kBigPairs = 64;
 constexpr int kBigRows = 128;
 constexpr int kBigChunk = 64;
 
 template <int kMode>
-__global__ void __launch_bounds__(kMoeThreads, 2)
+__global__ void __launch_bounds__(kMoeThreads, 3)
 moe_product_tiled_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, void* __restrict__ y,
                          const float* __restrict__ pair_weight, const int* __restrict__ tile_expert,
                          const int* __restrict__ tile_pairs, int top, int n, int k, int act, float limit, int n_tiles, int n_blocks) {
     constexpr bool kGated = kMode == kMoeGated;
-    constexpr int kWRows = kGated ? 2 * kBigRows : kBigRows;          // rows of the matrix in a chunk
-    constexpr int kXPieces = kBigPairs * 8 / kMoeThreads;             // 16-byte pieces of x a thread brings per chunk
-    constexpr int kWPieces = kWRows * 8 / kMoeThreads;
-    __shared__ uint4 sx[2 * kBigPairs * 4];                           // [half][row][4 pieces]
-    __shared__ uint4 sw[2 * kWRows * 4];
+    constexpr int kOwnRows = kGated ? kBigRows / 2 : kBigRows;        // rows of the result
+    constexpr int kBring = kMoeThreads / 8;                           // rows of 8 pieces that the workgroup brings at once
+    constexpr int kXPieces = kBigPairs / kBring;                         // 16-byte pieces of x a thread brings per chunk
+    constexpr int kWPieces = kBigRows / kBring;
+    constexpr int kPB = 2;                                            // blocks of 16 pairs a wave
+    __shared__ uint4 sx[2][2 * kBigPairs * 4];                           // [chunk][half][row][4 pieces]
+    __shared__ uint4 sw[2][2 * kBigRows * 4];
     // Workgroups go to the eight dies in turn, and each die has a cache of its own: the work is numbered so that a
     // die gets a run of neighbouring (row block, tile) places, tiles fastest: the tiles of one expert, which read the
-    // same rows of its matrix, then lie on one die.
+    // same rows of its matrix, then lie on one die.  (Groups of two or four tiles with all their row blocks measured the same.)
     const int per_die = (n_tiles * n_blocks + 7) / 8;
     const int place = static_cast<int>(blockIdx.x % 8) * per_die + static_cast<int>(blockIdx.x / 8);
-    if (place >= n_tiles * n_blocks) return;
+    if (place >= n_tiles * n_blocks || static_cast<int>(blockIdx.x / 8) >= per_die) return;
     const int tile = place % n_tiles;
     const int row_block = place / n_tiles;
     const int e = tile_expert[tile];
@@ -680,128 +589,121 @@ moe_product_tiled_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict_
     const int tid = threadIdx.x;
     const int wave = tid / kWave, lane = tid % kWave;
     const int c = lane & 15, g = lane >> 4;
-    const int wr = wave >> 1, wp = wave & 1;
-    const int row_base = row_block * kBigRows;
+    const int wr = wave / 2, wp = wave % 2;               // a wave's 64 rows and 32 pairs
+    const int row_base = row_block * kOwnRows;
     const long matrix = static_cast<long>(n) * k;
     const int* my_pairs = tile_pairs + static_cast<long>(tile) * kBigPairs;
 
-    // what this thread brings: piece p = tid + 256 i is part p % 8 of row p / 8 (row tid / 8 + 32 i)
+    // what this thread brings: part tid % 8 of every kBring-th row from tid / 8 on
     const int part = tid & 7;
     const int half = part >> 2, quarter = part & 3;
     const bf16_t* x_from[kXPieces];
     const bf16_t* w_from[kWPieces];
 #pragma unroll
     for (int i = 0; i < kXPieces; ++i) {
-        const int pair = my_pairs[tid / 8 + 32 * i];
+        const int pair = my_pairs[tid / 8 + kBring * i];
         x_from[i] = pair < 0 ? nullptr : x + static_cast<long>(kMode != kMoeDown ? pair / top : pair) * k + 8 * part;
     }
 #pragma unroll
     for (int i = 0; i < kWPieces; ++i) {
-        const int local = tid / 8 + 32 * i;                           // gated: rows 0..127 gate, 128..255 up
-        const int row = row_base + (local % kBigRows);
+        const int local = tid / 8 + kBring * i;                           // gated: rows 0..63 gate, 64..127 up
+        const int row = row_base + local % kOwnRows;
         w_from[i] = row >= n ? nullptr
-                             : w + static_cast<long>(e) * (kGated ? 2 : 1) * matrix + (local >= kBigRows ? matrix : 0) +
+                             : w + static_cast<long>(e) * (kGated ? 2 : 1) * matrix + (local >= kOwnRows ? matrix : 0) +
                                    static_cast<long>(row) * k + 8 * part;
     }
-    uint4 hx[kXPieces], hw[kWPieces];
-
-    moe_floatx4 acc[4][4], acc2[kGated ? 4 : 1][4];
+    struct Pieces {
+        uint4 x[kXPieces], w[kWPieces];
+    };
+    auto bring = [&](int chunk, Pieces& to) {
+        const bool in = chunk * kBigChunk + 8 * part < k;
 #pragma unroll
-    for (int ta = 0; ta < 4; ++ta)
-#pragma unroll
-        for (int tb = 0; tb < 4; ++tb) {
-            acc[ta][tb] = moe_floatx4{0.f, 0.f, 0.f, 0.f};
-            if constexpr (kGated) acc2[ta][tb] = moe_floatx4{0.f, 0.f, 0.f, 0.f};
+        for (int i = 0; i < kWPieces; ++i) {
+            to.w[i] = uint4{0u, 0u, 0u, 0u};
+            if (w_from[i] && in) to.w[i] = *reinterpret_cast<const uint4*>(w_from[i] + static_cast<long>(chunk) * kBigChunk);
         }
-    const int chunks = (k + kBigChunk - 1) / kBigChunk;
-#define LEONE_MOE_BRING(K0)                                                                                              \
-    {                                                                                                                    \
-        const bool in = (K0) + 8 * part < k;                                                                             \
-        _Pragma("unroll") for (int i = 0; i < kXPieces; ++i) {                                                           \
-            hx[i] = uint4{0u, 0u, 0u, 0u};                                                                               \
-            if (x_from[i] && in) hx[i] = *reinterpret_cast<const uint4*>(x_from[i] + (K0));                              \
-        }                                                                                                                \
-        _Pragma("unroll") for (int i = 0; i < kWPieces; ++i) {                                                           \
-            hw[i] = uint4{0u, 0u, 0u, 0u};                                                                               \
-            if (w_from[i] && in) hw[i] = *reinterpret_cast<const uint4*>(w_from[i] + (K0));                              \
-        }                                                                                                                \
-    }
-    LEONE_MOE_BRING(0)
-    for (int ck = 0; ck < chunks; ++ck) {
 #pragma unroll
-        for (int i = 0; i < kXPieces; ++i) sx[(half * kBigPairs + tid / 8 + 32 * i) * 4 + quarter] = hx[i];
+        for (int i = 0; i < kXPieces; ++i) {
+            to.x[i] = uint4{0u, 0u, 0u, 0u};
+            if (x_from[i] && in) to.x[i] = *reinterpret_cast<const uint4*>(x_from[i] + static_cast<long>(chunk) * kBigChunk);
+        }
+    };
+    auto put = [&](const Pieces& from, int at) {
 #pragma unroll
-        for (int i = 0; i < kWPieces; ++i) sw[(half * kWRows + tid / 8 + 32 * i) * 4 + quarter] = hw[i];
-        __syncthreads();
-        if (ck + 1 < chunks) LEONE_MOE_BRING((ck + 1) * kBigChunk)
+        for (int i = 0; i < kXPieces; ++i) sx[at][(half * kBigPairs + tid / 8 + kBring * i) * 4 + quarter] = from.x[i];
+#pragma unroll
+        for (int i = 0; i < kWPieces; ++i) sw[at][(half * kBigRows + tid / 8 + kBring * i) * 4 + quarter] = from.w[i];
+    };
+    // a wave's four blocks of 16 rows: gated, two of gate rows and two of their up rows
+    auto row_of = [&](int t) { return kGated ? (t / 2) * kOwnRows + 32 * wr + 16 * (t % 2) : 64 * wr + 16 * t; };
+    moe_floatx4 acc[4][kPB] = {};
+    auto work = [&](int at) {
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-            moe_bf16x8 a[4], a2[kGated ? 4 : 1], b[4];
+            moe_bf16x8 a[4], b[kPB];
 #pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                a[t] = __builtin_bit_cast(moe_bf16x8, sw[(h * kWRows + 64 * wr + 16 * t + c) * 4 + g]);
-                if constexpr (kGated) a2[t] = __builtin_bit_cast(moe_bf16x8, sw[(h * kWRows + kBigRows + 64 * wr + 16 * t + c) * 4 + g]);
-                b[t] = __builtin_bit_cast(moe_bf16x8, sx[(h * kBigPairs + 64 * wp + 16 * t + c) * 4 + g]);
-            }
+            for (int t = 0; t < 4; ++t) a[t] = __builtin_bit_cast(moe_bf16x8, sw[at][(h * kBigRows + row_of(t) + c) * 4 + g]);
+#pragma unroll
+            for (int t = 0; t < kPB; ++t) b[t] = __builtin_bit_cast(moe_bf16x8, sx[at][(h * kBigPairs + 32 * wp + 16 * t + c) * 4 + g]);
 #pragma unroll
             for (int ta = 0; ta < 4; ++ta)
 #pragma unroll
-                for (int tb = 0; tb < 4; ++tb) {
-                    acc[ta][tb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[ta], b[tb], acc[ta][tb], 0, 0, 0);
-                    if constexpr (kGated) acc2[ta][tb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2[ta], b[tb], acc2[ta][tb], 0, 0, 0);
-                }
+                for (int tb = 0; tb < kPB; ++tb) acc[ta][tb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[ta], b[tb], acc[ta][tb], 0, 0, 0);
         }
-        __syncthreads();                               // everyone has read the chunk before the next is put down
+    };
+    const int chunks = (k + kBigChunk - 1) / kBigChunk;
+    Pieces even, odd;                                  // chunks 1, 3, .. of the loop below come in `odd`, 2, 4, .. in `even`
+    bring(0, even);
+    bring(1, odd);
+    put(even, 0);
+    bring(2, even);                                    // past the last chunk: zeros, and nothing read
+    for (int ck = 0; ck < chunks; ck += 2) {
+        __syncthreads();                               // chunk ck lies ready, and nobody reads the other place any more
+        put(odd, 1);
+        bring(ck + 3, odd);
+        work(0);
+        if (ck + 1 >= chunks) break;
+        __syncthreads();
+        put(even, 0);
+        bring(ck + 4, even);
+        work(1);
     }
-#undef LEONE_MOE_BRING
     // lane (c, g) holds rows 4 g .. 4 g + 3 of pair c of every (ta, tb)
 #pragma unroll
-    for (int tb = 0; tb < 4; ++tb) {
-        const int pair = my_pairs[64 * wp + 16 * tb + c];
+    for (int tb = 0; tb < kPB; ++tb) {
+        const int pair = my_pairs[32 * wp + 16 * tb + c];
         if (pair < 0) continue;
         const float scale = kGated || !pair_weight ? 1.f : pair_weight[pair];
 #pragma unroll
-        for (int ta = 0; ta < 4; ++ta) {
-            const int r = row_base + 64 * wr + 16 * ta + 4 * g;
+        for (int ta = 0; ta < (kGated ? 2 : 4); ++ta) {
+            const int r = row_base + row_of(ta) + 4 * g;
             if (r >= n) continue;
-            float v0, v1, v2, v3;
+            float v[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                v[j] = kGated ? glu_value(acc[ta][tb][j], acc[kGated ? ta + 2 : ta][tb][j], act, limit)
+                              : kMode == kMoePlain ? plain_act(acc[ta][tb][j] * scale, act) : acc[ta][tb][j] * scale;
+            const bool whole = r + 3 < n && n % 4 == 0;
             if constexpr (kMode != kMoeDown) {
-                if constexpr (kGated) {
-                    v0 = glu_value(acc[ta][tb][0], acc2[ta][tb][0], act, limit);
-                    v1 = glu_value(acc[ta][tb][1], acc2[ta][tb][1], act, limit);
-                    v2 = glu_value(acc[ta][tb][2], acc2[ta][tb][2], act, limit);
-                    v3 = glu_value(acc[ta][tb][3], acc2[ta][tb][3], act, limit);
-                } else {
-                    v0 = plain_act(acc[ta][tb][0] * scale, act);
-                    v1 = plain_act(acc[ta][tb][1] * scale, act);
-                    v2 = plain_act(acc[ta][tb][2] * scale, act);
-                    v3 = plain_act(acc[ta][tb][3] * scale, act);
-                }
                 bf16_t* to = static_cast<bf16_t*>(y) + static_cast<long>(pair) * n + r;
-                if (r + 3 < n && n % 4 == 0) {
+                if (whole) {
                     uint2 packed;
-                    packed.x = bf16_bits_from_float(v0) | (static_cast<uint32_t>(bf16_bits_from_float(v1)) << 16);
-                    packed.y = bf16_bits_from_float(v2) | (static_cast<uint32_t>(bf16_bits_from_float(v3)) << 16);
+                    packed.x = bf16_bits_from_float(v[0]) | (static_cast<uint32_t>(bf16_bits_from_float(v[1])) << 16);
+                    packed.y = bf16_bits_from_float(v[2]) | (static_cast<uint32_t>(bf16_bits_from_float(v[3])) << 16);
                     *reinterpret_cast<uint2*>(to) = packed;
                 } else {
-                    to[0] = from_float<bf16_t>(v0);
-                    if (r + 1 < n) to[1] = from_float<bf16_t>(v1);
-                    if (r + 2 < n) to[2] = from_float<bf16_t>(v2);
-                    if (r + 3 < n) to[3] = from_float<bf16_t>(v3);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        if (r + j < n) to[j] = from_float<bf16_t>(v[j]);
                 }
             } else {
-                v0 = acc[ta][tb][0] * scale;
-                v1 = acc[ta][tb][1] * scale;
-                v2 = acc[ta][tb][2] * scale;
-                v3 = acc[ta][tb][3] * scale;
                 float* to = static_cast<float*>(y) + static_cast<long>(pair) * n + r;
-                if (r + 3 < n && n % 4 == 0) {
-                    *reinterpret_cast<float4*>(to) = float4{v0, v1, v2, v3};
+                if (whole) {
+                    *reinterpret_cast<float4*>(to) = float4{v[0], v[1], v[2], v[3]};
                 } else {
-                    to[0] = v0;
-                    if (r + 1 < n) to[1] = v1;
-                    if (r + 2 < n) to[2] = v2;
-                    if (r + 3 < n) to[3] = v3;
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        if (r + j < n) to[j] = v[j];
                 }
             }
         }
@@ -876,7 +778,7 @@ extern "C" int leone_route_plan(const float* logits, const void* correction, int
     LEONE_REQUIRE(group_count >= 1 && total % group_count == 0 && group_keep >= 1 && group_keep <= group_count,
                   "route_plan: %d groups (dividing %d outputs), %d kept", group_count, total, group_keep);
     LEONE_REQUIRE(experts > 0 && experts <= 1024, "route_plan: %d experts (at most 1024)", experts);
-    LEONE_REQUIRE(tile == kTilePairs || tile == 16 || tile == 64 || tile == 128, "route_plan: tiles of %d pairs", tile);
+    LEONE_REQUIRE(tile == kTilePairs || tile == 16 || tile == kBigPairs, "route_plan: tiles of %d pairs", tile);
     const long pairs = static_cast<long>(rows) * (top + always);
     const long needed = pairs / tile + experts;
     LEONE_REQUIRE(max_tiles >= (needed < pairs ? needed : pairs), "route_plan: %d tiles cannot hold %ld pairs of %d experts", max_tiles,
@@ -890,7 +792,7 @@ extern "C" int leone_route_plan(const float* logits, const void* correction, int
 
 extern "C" int leone_moe_plan(const int* chosen, int pairs, int experts, int* tile_expert, int* tile_pairs, int max_tiles,
                               int tile, hipStream_t stream) {
-    LEONE_REQUIRE(tile == kTilePairs || tile == 16 || tile == 64 || tile == 128, "moe_plan: tiles of %d pairs", tile);
+    LEONE_REQUIRE(tile == kTilePairs || tile == 16 || tile == kBigPairs, "moe_plan: tiles of %d pairs", tile);
     LEONE_REQUIRE(chosen && tile_expert && tile_pairs, "moe_plan: null pointer");
     LEONE_REQUIRE(pairs > 0 && experts > 0 && experts <= 1024, "moe_plan: %d pairs, %d experts (at most 1024)", pairs, experts);
     const long needed = static_cast<long>(pairs) / tile + experts;
@@ -914,42 +816,35 @@ extern "C" int leone_moe_product(const void* x, const void* w, void* y, const fl
                       (act == kActReluSquared && gated != kMoeGated),
                   "moe_product: unknown activation %d (limit %g)", act, limit);
     if (tile != kTilePairs) {
-        LEONE_REQUIRE(tile == 16 || tile == 64 || tile == 128, "moe_product: tiles of %d pairs", tile);
+        LEONE_REQUIRE(tile == 16 || tile == kBigPairs, "moe_product: tiles of %d pairs", tile);
         LEONE_REQUIRE(dtype == kBF16 && k % 8 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0,
                       "moe_product: the matrix-core kernel takes bfloat16 with an inner size that is a multiple of 8, not %d", k);
         LEONE_REQUIRE(x && w && y && tile_expert && tile_pairs, "moe_product: null pointer");
         LEONE_REQUIRE(max_tiles > 0 && top > 0 && n > 0 && k > 0, "moe_product: %d tiles, sizes %d x %d", max_tiles, n, k);
-        const dim3 cores(max_tiles, ceil_div(n, tile == 128 ? 128 : tile == 64 ? 64 : 16));
-        LEONE_REQUIRE(cores.y <= 65535, "moe_product: %d rows of a matrix are too many", n);
-#define LEONE_MOE_CORES(PB, RT, G)                                                                                      \
-    moe_product_mfma_kernel<PB, RT, G><<<cores, kMoeThreads, 0, stream>>>(static_cast<const bf16_t*>(x), static_cast<const bf16_t*>(w), \
-                                                                          y, pair_weight, tile_expert, tile_pairs, top, n, k, act, limit)
         if (tile == 16) {
+            const dim3 grid(max_tiles, ceil_div(n, 16));
+            LEONE_REQUIRE(grid.y <= 65535, "moe_product: %d rows of a matrix are too many", n);
 #define LEONE_MOE_STREAM(MODE)                                                                                            \
-    moe_product_stream_kernel<MODE><<<cores, kMoeThreads, 0, stream>>>(static_cast<const bf16_t*>(x), static_cast<const bf16_t*>(w), \
-                                                                       y, pair_weight, tile_expert, tile_pairs, top, n, k, act, limit)
+    moe_product_stream_kernel<MODE><<<grid, kMoeThreads, 0, stream>>>(static_cast<const bf16_t*>(x), static_cast<const bf16_t*>(w), \
+                                                                      y, pair_weight, tile_expert, tile_pairs, top, n, k, act, limit)
             if (gated == kMoeGated) LEONE_MOE_STREAM(kMoeGated);
             else if (gated == kMoePlain) LEONE_MOE_STREAM(kMoePlain);
             else LEONE_MOE_STREAM(kMoeDown);
 #undef LEONE_MOE_STREAM
-        } else if (tile == 64) {
-            if (gated == kMoeGated) LEONE_MOE_CORES(4, 1, kMoeGated);
-            else if (gated == kMoePlain) LEONE_MOE_CORES(4, 1, kMoePlain);
-            else LEONE_MOE_CORES(4, 1, kMoeDown);
         } else {
-            const long places = static_cast<long>(cores.x) * cores.y;
+            const int blocks = ceil_div(n, gated == kMoeGated ? kBigRows / 2 : kBigRows);
+            const long places = static_cast<long>(max_tiles) * blocks;
             LEONE_REQUIRE(places + 7 <= 0x7fffffffL, "moe_product: too many tiles");
             const int grid = static_cast<int>((places + 7) / 8 * 8);
-#define LEONE_MOE_TILED(MODE)                                                                                               \
+#define LEONE_MOE_TILED(MODE)                                                                                                  \
     moe_product_tiled_kernel<MODE><<<grid, kMoeThreads, 0, stream>>>(static_cast<const bf16_t*>(x), static_cast<const bf16_t*>(w), \
                                                                      y, pair_weight, tile_expert, tile_pairs, top, n, k, act, limit, \
-                                                                     static_cast<int>(cores.x), static_cast<int>(cores.y))
+                                                                     max_tiles, blocks)
             if (gated == kMoeGated) LEONE_MOE_TILED(kMoeGated);
             else if (gated == kMoePlain) LEONE_MOE_TILED(kMoePlain);
             else LEONE_MOE_TILED(kMoeDown);
 #undef LEONE_MOE_TILED
         }
-#undef LEONE_MOE_CORES
         LEONE_LAUNCH_CHECK("moe_product");
         return 0;
     }

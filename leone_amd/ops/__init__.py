@@ -1868,17 +1868,20 @@ def route_topk(logits: torch.Tensor, correction: Optional[torch.Tensor], top: in
     return chosen, weight
 
 
-MOE_WIDE_TILE_PAIRS = 32      # from this many (row, place) pairs an expert on average, the experts' products take tiles of 64 pairs
+MOE_WIDE_TILE_PAIRS = 12      # from this many (row, place) pairs an expert on average, the experts' products take tiles of 64 pairs
 ROUTE_PLAN_ROWS = 64          # up to here the router's choice and the tiles are made in one launch
 
 
 def _expert_tiles(x: torch.Tensor, rows: int, top: int, experts: int, hidden: int, ff: int):
     """(pairs a tile, tiles at most, tile_expert, tile_pairs) for a step of ``rows`` rows."""
     pairs = rows * top
-    # bfloat16 with inner sizes in runs of 8 goes to the matrix cores: tiles of 128 or 64 pairs where an expert gets
-    # many (its matrices are read once a tile), of 16 where it gets few; anything else in tiles of the plain kernel's size
+    # bfloat16 with inner sizes in runs of 8 goes to the matrix cores: tiles of 64 pairs where an expert gets many (its
+    # matrices are read once a tile), of 16 where it gets few; anything else in tiles of the plain kernel's size.  Both
+    # products of 32 experts (us, tiles of 16 and 64), width 1,024: 11 pairs an expert 37 and 39, 23 pairs 58 and 42;
+    # width 2,048: 7 pairs 85 and 78, 34 pairs 238 and 88; width 4,096: 4 pairs 276 and 238, 11 pairs 362 and 259, but one
+    # pair 49 and 85.  Below the line a narrow model's few pairs decide, where the smaller tile has more workgroups.
     if x.dtype == torch.bfloat16 and hidden % 8 == 0 and ff % 8 == 0:
-        tile = 128 if pairs >= 4 * MOE_WIDE_TILE_PAIRS * experts else 64 if pairs >= MOE_WIDE_TILE_PAIRS * experts else 16
+        tile = 64 if pairs >= MOE_WIDE_TILE_PAIRS * experts else 16
     else:
         tile = library().leone_moe_tile_pairs()
     max_tiles = min(pairs, pairs // tile + experts)

@@ -1,4 +1,4 @@
-"""The router's choice by ranks, the tiles of many experts, and the experts' products in tiles of 16 pairs, at their edges."""
+"""The router's choice by ranks, the tiles of many experts, and the experts' products in tiles of 16 and 64 pairs, at their edges."""
 import math
 
 import pytest
@@ -56,4 +56,36 @@ def test_products_in_tiles_of_sixteen(experts, rows, top):
                 g, u = (up[e, i].double() @ x[t].double() for i in (0, 1))
                 want[t] += a * (down[e].double() @ (plain.silu(g) * u).bfloat16().double())
         # the middle is rounded to 8 bits on both sides, now and then to neighbours: 2^-8 of some elements of one place's sum
+        assert float((got - want).norm() / want.norm()) < 2e-3
+
+
+@pytest.mark.parametrize("counts,hidden,ff", [((63, 64, 65, 129, 0, 1), 8, 8), ((64, 128, 1), 64, 56), ((129, 2, 64), 72, 136),
+                                              ((65, 63), 136, 64), ((200,), 200, 72), ((33,) + (0,) * 40, 264, 40)])
+@pytest.mark.parametrize("gated", [True, False])
+def test_products_in_tiles_of_sixty_four(counts, hidden, ff, gated):
+    """Tiles just full, one short and one over; inner sizes below, at and off a chunk of 64, odd and even numbers of chunks; result
+    rows off a workgroup's 64 and 128; the last case, few pairs for its experts, takes several tiles of 16 for one expert."""
+    from leone_amd import ops
+    experts, pairs = len(counts), sum(counts)
+    top = 1 if pairs % 2 else 2
+    gen = torch.Generator().manual_seed(pairs + hidden)
+    which = torch.tensor([e for e, count in enumerate(counts) for _ in range(count)])[torch.randperm(pairs, generator=gen)]
+    chosen = which.view(-1, top).to(torch.int32)
+    weight = torch.rand(pairs // top, top, generator=gen) + 0.1
+    x = torch.randn(pairs // top, hidden, generator=gen).bfloat16()
+    up = (torch.randn(experts, 2 if gated else 1, ff, hidden, generator=gen) / math.sqrt(hidden)).bfloat16()
+    down = (torch.randn(experts, hidden, ff, generator=gen) / math.sqrt(ff)).bfloat16()
+    for weigh_input in (False,) if gated else (False, True):
+        got = ops.routed_experts(x.to(DEV), chosen.to(DEV), weight.to(DEV), (up if gated else up[:, 0]).to(DEV), down.to(DEV),
+                                 "silu" if gated else "relu2", weigh_input=weigh_input).cpu().double()
+        rows = x.double().repeat_interleave(top, 0)
+        a = weight.double().view(-1, 1)
+        first = torch.stack([up[e, 0].double() @ r for e, r in zip(which, rows)])
+        if gated:
+            middle = plain.silu(first) * torch.stack([up[e, 1].double() @ r for e, r in zip(which, rows)])
+        else:
+            middle = (a * first if weigh_input else first).clamp(min=0).square()
+        each = torch.stack([down[e].double() @ m for e, m in zip(which, middle.bfloat16().double())])
+        want = (each if weigh_input else a * each).view(-1, top, hidden).sum(1)
+        # as above: middles that are rounded to neighbours, 2^-8 of some elements of one place's sum
         assert float((got - want).norm() / want.norm()) < 2e-3
