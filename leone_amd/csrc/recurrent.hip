@@ -12,8 +12,8 @@
 //                with q and k made unit vectors per head first.
 //
 // A workgroup of four waves owns a run of columns of one head of one segment (a request's rows in the step, or a
-// chunk of them) and walks the segment's rows in order: a single decoded token and a prompt portion are the same
-// kernel.  A column's dim elements are spread over 1, 2, 4 or 8 lanes, 32 to a lane in registers (so that several
+// chunk of them) and walks the segment's rows in order (steps of single rows have kernels of
+// their own, outer_step and delta_step, where the size allows).  A column's dim elements are spread over 1, 2, 4 or 8 lanes, 32 to a lane in registers (so that several
 // waves fit a SIMD and hide each other's waits); the lanes of a column add their parts of a read-out by shuffles.
 // The vectors every lane needs (q_t, k_t, the decays) are prepared 16 tokens at a time in shared memory.
 // Everything here is float.
@@ -269,6 +269,128 @@ __global__ void __launch_bounds__(kScanThreads) outer_scan_kernel(OuterScanArgs 
     }
 }
 
+// The same for segments of single rows (decode steps), where the state's bytes in and out are the bound and the chain of trips to
+// memory in front of them is what costs.  A workgroup takes 64 columns of a head, so that a wave's loads are whole lines of
+// 256 bytes (the other kernel's are pieces of 32), and its waves take 32 key channels each; a row's q and k are made by
+// the lanes of the wave that needs them.  A segment's row, gates, values and state are
+// all asked for before the first is used.  The waves' sums meet in shared memory in the order in which the other kernel's
+// lanes meet.  Eight rows of four heads of 256 x 512 with a normaliser: 9.6 us (18.3 walked).
+// The float at a wave's own row (in bytes from a base that all waves share) and a lane's own column: one base and one offset of 32
+// bits a load, so that no row needs an address of its own.
+__device__ inline const float& float_at(const float* base, unsigned row_bytes, unsigned col_bytes) {
+    return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(base) + (row_bytes + col_bytes));
+}
+__device__ inline float& float_at(float* base, unsigned row_bytes, unsigned col_bytes) {
+    return *reinterpret_cast<float*>(reinterpret_cast<char*>(base) + (row_bytes + col_bytes));
+}
+
+template <int kGroups>
+__device__ inline float sum_groups(const float* of, int stride) {
+    float v[kGroups];
+#pragma unroll
+    for (int g = 0; g < kGroups; ++g) v[g] = of[g * stride];
+#pragma unroll
+    for (int step = 1; step < kGroups; step <<= 1)
+#pragma unroll
+        for (int g = 0; g + step < kGroups; g += 2 * step) v[g] += v[g + step];
+    return v[0];
+}
+
+// x turned by its row's angle, from loads that are already under way
+struct Turned {
+    float own, other, c, s;
+};
+__device__ inline float turn(const Turned& t, int i, int silu, int rot_half) {
+    const float x = silu_if(t.own, silu);
+    if (i >= 2 * rot_half) return x;
+    return i < rot_half ? x * t.c - silu_if(t.other, silu) * t.s : x * t.c + silu_if(t.other, silu) * t.s;
+}
+
+template <int kGroups>
+__global__ void __launch_bounds__(kGroups * kWave) outer_step_kernel(OuterScanArgs p) {
+    __shared__ float sums[2][kGroups][kWave + 1];             // the columns' shares; one more for the normaliser's
+    __shared__ __align__(16) float2 skq[kGroups][kLaneRows];  // a wave's own k and q
+    __shared__ float snorm[kGroups][kLaneRows];
+    const int head = blockIdx.y, tid = threadIdx.x, lane = tid % kWave;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);      // one for all lanes: the state's rows have one address a wave
+    const Segment seg = p.segments[blockIdx.x];
+    const int first = seg.first, n = seg.end - seg.first;
+    const int ch0 = wave * kLaneRows;
+    const int col = blockIdx.z * kWave + lane;
+    const int ccol = min(col, p.vdim - 1);
+    const unsigned row_bytes = 4u * p.vdim;
+    const bool norm = p.norm_column && blockIdx.z == 0;
+    const int ch = ch0 + lane % kLaneRows;                    // the channel whose q, k and normaliser this lane holds
+    const int half = p.rot_half;
+    const int other = ch < half ? ch + half : ch < 2 * half ? ch - half : ch;
+    const int turned = ch < half ? ch : ch < 2 * half ? ch - half : 0;
+    const float* from = seg.in < 0 ? nullptr : p.state_in + seg.in * p.in_stride + head * p.head_stride;
+    const float fixed = p.coef ? 0.f : p.decay[head];
+    float S[kLaneRows], N = 0.f;
+#pragma unroll
+    for (int i = 0; i < kLaneRows; ++i) S[i] = 0.f;
+
+    for (int t = 0; t < n; ++t) {
+        const long row = first + t;
+        const float* base = p.proj + row * p.stride;
+        const float* qs = base + p.q_off + head * p.dim;
+        const float* ks = base + p.k_off + head * p.dim;
+        int pos = 0;
+        if (p.cos_table) pos = p.positions[row];
+        Turned q{qs[ch], qs[other], 1.f, 0.f}, k{ks[ch], ks[other], 1.f, 0.f};
+        const float v_raw = base[p.v_off + head * p.vdim + ccol];
+        const long at = row * p.heads + head;
+        float a = fixed, b = 1.f;
+        if (p.coef) {
+            a = p.coef[2 * at];
+            b = p.coef[2 * at + 1];
+        }
+        if (p.cos_table) {
+            const long angle = static_cast<long>(min(pos, p.table_positions - 1)) * half + turned;
+            q.c = k.c = p.cos_table[angle];
+            q.s = k.s = p.sin_table[angle];
+        }
+        if (t == 0 && from) {
+#pragma unroll
+            for (int i = 0; i < kLaneRows; ++i) S[i] = float_at(from, (ch0 + i) * row_bytes, 4u * ccol);
+            if (norm) N = from[static_cast<long>(p.dim) * p.vdim + ch];
+        }
+        const float qv = turn(q, ch, p.silu, half) * p.q_scale;
+        const float kv = turn(k, ch, p.silu, half) * p.k_scale;
+        const float bv = b * silu_if(v_raw, p.silu);
+        if (lane < kLaneRows) skq[wave][lane] = float2{kv, qv};
+        if (norm) {
+            N = fmaf(a, N, kv * b);
+            if (lane < kLaneRows) snorm[wave][lane] = N;
+        }
+        __syncthreads();
+        float acc = 0.f;
+#pragma unroll
+        for (int i = 0; i < kLaneRows; ++i) {
+            const float2 kq = skq[wave][i];
+            S[i] = fmaf(a, S[i], kq.x * bv);
+            acc = fmaf(S[i], kq.y, acc);
+        }
+        float (*to)[kWave + 1] = sums[t & 1];                  // read behind one barrier, written again behind the next
+        to[wave][lane] = acc;
+        if (norm) {
+            float sum = 0.f;
+#pragma unroll
+            for (int i = 0; i < kLaneRows; ++i) sum = fmaf(snorm[wave][i], skq[wave][i].y, sum);
+            if (lane == 0) to[wave][kWave] = sum;
+        }
+        __syncthreads();
+        if (wave == 0 && col < p.vdim) p.out[at * p.vdim + col] = sum_groups<kGroups>(&to[0][lane], kWave + 1);
+        if (norm && tid == kGroups * kWave - 1) p.dot[at] = sum_groups<kGroups>(&to[0][kWave], kWave + 1);
+    }
+    if (!p.state_out || seg.out < 0 || n <= 0) return;         // (a segment without rows leaves its state as it is)
+    float* into = p.state_out + seg.out * p.out_stride + head * p.head_stride;
+#pragma unroll
+    for (int i = 0; i < kLaneRows; ++i)
+        if (col < p.vdim) float_at(into, (ch0 + i) * row_bytes, 4u * ccol) = S[i];
+    if (norm && lane < kLaneRows) into[static_cast<long>(p.dim) * p.vdim + ch] = N;
+}
+
 // The chunks' end states chained: for a long portion whose chunks are [g0, g1) of `work` (each holding what its
 // own rows wrote, from zeros), S = the request's state (zeros at a sequence's start); for every chunk in order:
 // what the chunk holds is replaced by S (the state it starts from), and S <- product[chunk] * S + what it held.
@@ -430,6 +552,95 @@ __global__ void __launch_bounds__(kScanThreads) delta_scan_kernel(DeltaScanArgs 
         if (ch0 + i < p.dim) to[static_cast<long>(ch0 + i) * p.vdim + col] = S[i];
 }
 
+// The same for segments of single rows (decode steps), split as in outer_step_kernel: 64 columns of a head a workgroup, 32 key
+// channels a wave, everything asked for before the first use.  Eight rows of 16 heads of 128 x 128: 8.9 us (14.5 walked).
+template <int kGroups>
+__global__ void __launch_bounds__(kGroups * kWave) delta_step_kernel(DeltaScanArgs p) {
+    constexpr int kRowLanes = kScanThreads / kScanTokens;     // lanes that share a row's sums of squares, as in the other kernel
+    constexpr int kOwn = kGroups * kLaneRows / kRowLanes;
+    __shared__ float saw[kGroups][kWave], sums[kGroups][kWave];
+    __shared__ float4 sgkq[kGroups][kLaneRows];               // a wave's own decays, k and q
+    const int head = blockIdx.y, tid = threadIdx.x, lane = tid % kWave;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const Segment seg = p.segments[blockIdx.x];
+    const int first = seg.first, n = seg.end - seg.first;
+    const int kvh = head / (p.heads / p.kv_heads);
+    const int ch0 = wave * kLaneRows;
+    const int col = blockIdx.z * kWave + lane;
+    const int ccol = min(col, p.vdim - 1);
+    const unsigned row_bytes = 4u * p.vdim;
+    const int ch = ch0 + lane % kLaneRows;
+    const long head_size = static_cast<long>(p.dim) * p.vdim;
+    const float* from = seg.in < 0 ? nullptr : p.state_in + seg.in * p.in_stride + head * head_size;
+    const long step_at = p.per_head ? head : static_cast<long>(head) * p.dim + ch;
+    float S[kLaneRows];
+#pragma unroll
+    for (int i = 0; i < kLaneRows; ++i) S[i] = 0.f;
+
+    for (int t = 0; t < n; ++t) {
+        const long row = first + t;
+        const float* base = p.qkv + row * p.stride;
+        const float* qs = base + p.q_off + kvh * p.dim;
+        const float* ks = base + p.k_off + kvh * p.dim;
+        float qr[kOwn], kr[kOwn];
+#pragma unroll
+        for (int m = 0; m < kOwn; ++m) {
+            qr[m] = qs[lane % kRowLanes + m * kRowLanes];
+            kr[m] = ks[lane % kRowLanes + m * kRowLanes];
+        }
+        const float q_raw = qs[ch], k_raw = ks[ch];
+        const float v = base[p.v_off + head * p.vdim + ccol];
+        const float step_raw = p.step[row * p.step_stride + step_at], beta_raw = p.beta[row * p.beta_stride + head];
+        if (t == 0 && from) {
+#pragma unroll
+            for (int i = 0; i < kLaneRows; ++i) S[i] = float_at(from, (ch0 + i) * row_bytes, 4u * ccol);
+        }
+        const float rate = expf(load_any(p.rate_log, head)), bias = load_any(p.step_bias, step_at);
+        float qq = 0.f, kk = 0.f;
+#pragma unroll
+        for (int m = 0; m < kOwn; ++m) {
+            qq = fmaf(qr[m], qr[m], qq);
+            kk = fmaf(kr[m], kr[m], kk);
+        }
+#pragma unroll
+        for (int off = kRowLanes / 2; off > 0; off >>= 1) {
+            qq += __shfl_xor(qq, off, kWave);
+            kk += __shfl_xor(kk, off, kWave);
+        }
+        const float qinv = p.q_scale / sqrtf(qq + p.unit_eps);
+        const float kinv = 1.0f / sqrtf(kk + p.unit_eps);
+        const float gv = expf(-rate * softplus_f(step_raw + bias));
+        if (lane < kLaneRows) sgkq[wave][lane] = float4{gv, k_raw * kinv, q_raw * qinv, 0.f};
+        __syncthreads();
+        const float strength = 1.0f / (1.0f + expf(-beta_raw));
+        float seen = 0.f;
+#pragma unroll
+        for (int i = 0; i < kLaneRows; ++i) {
+            const float4 gkq = sgkq[wave][i];
+            S[i] *= gkq.x;
+            seen = fmaf(S[i], gkq.y, seen);
+        }
+        saw[wave][lane] = seen;                                // last read ahead of the barrier that the row before ended with
+        __syncthreads();
+        const float u = strength * (v - sum_groups<kGroups>(&saw[0][lane], kWave));
+        float acc = 0.f;
+#pragma unroll
+        for (int i = 0; i < kLaneRows; ++i) {
+            const float4 gkq = sgkq[wave][i];
+            S[i] = fmaf(gkq.y, u, S[i]);
+            acc = fmaf(S[i], gkq.z, acc);
+        }
+        sums[wave][lane] = acc;
+        __syncthreads();
+        if (wave == 0 && col < p.vdim) p.out[(row * p.heads + head) * p.vdim + col] = sum_groups<kGroups>(&sums[0][lane], kWave);
+    }
+    if (!p.state_out || seg.out < 0 || n <= 0 || col >= p.vdim) return;
+    float* to = p.state_out + seg.out * p.out_stride + head * head_size;
+#pragma unroll
+    for (int i = 0; i < kLaneRows; ++i)
+        float_at(to, (ch0 + i) * row_bytes, 4u * ccol) = S[i];
+}
+
 // The chunks of a long portion chained for the delta rule: a chunk's rows turn a state S that comes in into
 // transition[chunk] . S + (what the chunk holds: its end state from zeros).  As in outer_chain_kernel every chunk's
 // place in `work` ends up holding the state the chunk starts from, and the last state is the request's new one.
@@ -515,7 +726,13 @@ extern "C" int leone_exp_gates(const float* proj, long stride, int i_off, int f_
     return 0;
 }
 
-extern "C" int leone_outer_scan(const float* proj, long stride, int q_off, int k_off, int v_off, const float* coef,
+// Whether heads of such sizes are taken by the kernels for single rows: waves of 32 key channels each, without a rest (of 1, 2, 4
+// or 8 waves), offsets within a head's state of 32 bits.  Other heads are walked by the general kernels in single rows too.
+extern "C" int leone_step_fits(int dim, int vdim) {
+    return dim == lane_groups(dim) * kLaneRows && ceil_div(vdim, kWave) <= 65535 && static_cast<long>(dim) * vdim < (1L << 30);
+}
+
+static int run_outer_scan(bool single, const float* proj, long stride, int q_off, int k_off, int v_off, const float* coef,
                                 const float* decay, int no_input, int accumulate, int norm_column, float q_scale,
                                 float k_scale, int silu, const float* cos_table, const float* sin_table, int rotary_dim,
                                 int table_positions, const int* positions, const int* segments, int n_segments,
@@ -544,9 +761,46 @@ extern "C" int leone_outer_scan(const float* proj, long stride, int q_off, int k
     const int per_block = (kScanThreads / kWave) * (kWave / groups) * kLaneCols;          // columns a workgroup
     const dim3 grid(n_segments, heads, ceil_div(vdim + (norm_column ? 1 : 0), per_block));
     const size_t shared = (2 * kScanTokens * groups * kLaneRows + 2 * kScanTokens) * sizeof(float);
+    if (single) {
+        LEONE_REQUIRE(leone_step_fits(dim, vdim) && !no_input && !accumulate && !decay_product,
+                      "outer_step: single rows write their read-outs and nothing else, of heads of 32, 64, 128 or 256 key channels (not %d x %d)",
+                      dim, vdim);
+        const dim3 columns(n_segments, heads, ceil_div(vdim, kWave));
+        if (groups == 1) outer_step_kernel<1><<<columns, kWave, 0, stream>>>(a);
+        else if (groups == 2) outer_step_kernel<2><<<columns, 2 * kWave, 0, stream>>>(a);
+        else if (groups == 4) outer_step_kernel<4><<<columns, 4 * kWave, 0, stream>>>(a);
+        else outer_step_kernel<8><<<columns, 8 * kWave, 0, stream>>>(a);
+        LEONE_LAUNCH_CHECK("outer_step");
+        return 0;
+    }
     outer_scan_kernel<<<grid, kScanThreads, shared, stream>>>(a, groups);
     LEONE_LAUNCH_CHECK("outer_scan");
     return 0;
+}
+
+extern "C" int leone_outer_scan(const float* proj, long stride, int q_off, int k_off, int v_off, const float* coef,
+                                const float* decay, int no_input, int accumulate, int norm_column, float q_scale,
+                                float k_scale, int silu, const float* cos_table, const float* sin_table, int rotary_dim,
+                                int table_positions, const int* positions, const int* segments, int n_segments,
+                                const float* state_in, long in_stride, float* state_out, long out_stride, long head_stride,
+                                float* decay_product, float* out, float* dot, int heads, int dim, int vdim,
+                                hipStream_t stream) {
+    return run_outer_scan(false, proj, stride, q_off, k_off, v_off, coef, decay, no_input, accumulate, norm_column,
+        q_scale, k_scale, silu, cos_table, sin_table, rotary_dim, table_positions, positions, segments, n_segments,
+        state_in, in_stride, state_out, out_stride, head_stride, decay_product, out, dot, heads, dim, vdim, stream);
+}
+
+// leone_outer_scan where every segment is a single row.
+extern "C" int leone_outer_step(const float* proj, long stride, int q_off, int k_off, int v_off, const float* coef,
+                                const float* decay, int no_input, int accumulate, int norm_column, float q_scale,
+                                float k_scale, int silu, const float* cos_table, const float* sin_table, int rotary_dim,
+                                int table_positions, const int* positions, const int* segments, int n_segments,
+                                const float* state_in, long in_stride, float* state_out, long out_stride, long head_stride,
+                                float* decay_product, float* out, float* dot, int heads, int dim, int vdim,
+                                hipStream_t stream) {
+    return run_outer_scan(true, proj, stride, q_off, k_off, v_off, coef, decay, no_input, accumulate, norm_column,
+        q_scale, k_scale, silu, cos_table, sin_table, rotary_dim, table_positions, positions, segments, n_segments,
+        state_in, in_stride, state_out, out_stride, head_stride, decay_product, out, dot, heads, dim, vdim, stream);
 }
 
 extern "C" int leone_outer_chain(const int* links, int n_links, float* work, long work_stride, const float* product,
@@ -562,7 +816,7 @@ extern "C" int leone_outer_chain(const int* links, int n_links, float* work, lon
     return 0;
 }
 
-extern "C" int leone_delta_scan(const float* qkv, long stride, int q_off, int k_off, int v_off, const float* beta,
+static int run_delta_scan(bool single, const float* qkv, long stride, int q_off, int k_off, int v_off, const float* beta,
                                 long beta_stride, const float* step, long step_stride, int per_head, const void* rate_log,
                                 const void* step_bias, int vec_dtype, float q_scale, float unit_eps, int no_input,
                                 int accumulate, const int* segments, int n_segments, const float* state_in, long in_stride,
@@ -586,9 +840,44 @@ extern "C" int leone_delta_scan(const float* qkv, long stride, int q_off, int k_
     const int groups = lane_groups(dim);
     const dim3 grid(n_segments, heads, ceil_div(vdim + (transition ? dim : 0), (kScanThreads / kWave) * (kWave / groups)));
     const size_t shared = (3 * kScanTokens * groups * kLaneRows + kScanTokens) * sizeof(float);
+    if (single) {
+        LEONE_REQUIRE(leone_step_fits(dim, vdim) && !no_input && !accumulate && !transition,
+                      "delta_step: single rows write their read-outs and nothing else, of heads of 32, 64, 128 or 256 key channels (not %d x %d)",
+                      dim, vdim);
+        const dim3 columns(n_segments, heads, ceil_div(vdim, kWave));
+        if (groups == 1) delta_step_kernel<1><<<columns, kWave, 0, stream>>>(a);
+        else if (groups == 2) delta_step_kernel<2><<<columns, 2 * kWave, 0, stream>>>(a);
+        else if (groups == 4) delta_step_kernel<4><<<columns, 4 * kWave, 0, stream>>>(a);
+        else delta_step_kernel<8><<<columns, 8 * kWave, 0, stream>>>(a);
+        LEONE_LAUNCH_CHECK("delta_step");
+        return 0;
+    }
     delta_scan_kernel<<<grid, kScanThreads, shared, stream>>>(a, groups);
     LEONE_LAUNCH_CHECK("delta_scan");
     return 0;
+}
+
+extern "C" int leone_delta_scan(const float* qkv, long stride, int q_off, int k_off, int v_off, const float* beta,
+                                long beta_stride, const float* step, long step_stride, int per_head, const void* rate_log,
+                                const void* step_bias, int vec_dtype, float q_scale, float unit_eps, int no_input,
+                                int accumulate, const int* segments, int n_segments, const float* state_in, long in_stride,
+                                float* state_out, long out_stride, float* transition, float* out, int heads, int kv_heads,
+                                int dim, int vdim, hipStream_t stream) {
+    return run_delta_scan(false, qkv, stride, q_off, k_off, v_off, beta, beta_stride, step, step_stride, per_head,
+        rate_log, step_bias, vec_dtype, q_scale, unit_eps, no_input, accumulate, segments, n_segments, state_in,
+        in_stride, state_out, out_stride, transition, out, heads, kv_heads, dim, vdim, stream);
+}
+
+// leone_delta_scan where every segment is a single row.
+extern "C" int leone_delta_step(const float* qkv, long stride, int q_off, int k_off, int v_off, const float* beta,
+                                long beta_stride, const float* step, long step_stride, int per_head, const void* rate_log,
+                                const void* step_bias, int vec_dtype, float q_scale, float unit_eps, int no_input,
+                                int accumulate, const int* segments, int n_segments, const float* state_in, long in_stride,
+                                float* state_out, long out_stride, float* transition, float* out, int heads, int kv_heads,
+                                int dim, int vdim, hipStream_t stream) {
+    return run_delta_scan(true, qkv, stride, q_off, k_off, v_off, beta, beta_stride, step, step_stride, per_head,
+        rate_log, step_bias, vec_dtype, q_scale, unit_eps, no_input, accumulate, segments, n_segments, state_in,
+        in_stride, state_out, out_stride, transition, out, heads, kv_heads, dim, vdim, stream);
 }
 
 extern "C" int leone_delta_chain(const int* links, int n_links, float* work, long work_stride, const float* transition,

@@ -1675,7 +1675,10 @@ def outer_scan(proj: torch.Tensor, columns: dict, state: torch.Tensor, step, hea
     rotary_dim = 2 * cos.shape[1] if cos is not None else 0
 
     def walk(segments, state_in, state_out, no_input=False, accumulate=False, product=None):
-        call("leone_outer_scan", _dev(proj, "projection", torch.float32), width, columns["q"], columns["k"], columns["v"],
+        # every entry with a single row: the kernel that is made for it, if it takes the size (no chunks are walked then);
+        # eight rows of four heads of 256 x 512: 18.3 us walked, 9.6 in that kernel
+        single = segments.shape[0] == rows and not accumulate and product is None and library().leone_step_fits(dim, vdim)
+        call("leone_outer_step" if single else "leone_outer_scan", _dev(proj, "projection", torch.float32), width, columns["q"], columns["k"], columns["v"],
              _dev(coef, "coefficients"), _dev(decay, "decay", torch.float32, (heads,)) if decay is not None else 0,
              1 if no_input else 0, 1 if accumulate else 0, 1 if gates else 0, float(q_scale), float(k_scale),
              1 if activation == "silu" else 0,
@@ -1742,7 +1745,10 @@ def delta_scan(qkv: torch.Tensor, columns: dict, beta: torch.Tensor, step_size: 
     step_at, step_stride = _strided_rows(step_size, "delta_scan step", rows, heads if per_head else heads * dim)
 
     def walk(segments, state_in, state_out, no_input=False, accumulate=False, transition=None):
-        call("leone_delta_scan", _dev(qkv, "q, k, v", torch.float32), qkv.shape[1], columns["q"], columns["k"], columns["v"],
+        # every entry with a single row: the kernel that is made for it, if it takes the size (no chunks are walked then);
+        # eight rows of 16 heads of 128 x 128: 14.5 us walked, 8.9 in that kernel
+        single = segments.shape[0] == rows and not accumulate and transition is None and library().leone_step_fits(dim, vdim)
+        call("leone_delta_step" if single else "leone_delta_scan", _dev(qkv, "q, k, v", torch.float32), qkv.shape[1], columns["q"], columns["k"], columns["v"],
              beta_at, beta_stride, step_at, step_stride, 1 if per_head else 0, _dev(rate_log, "rate", None, (heads,)),
              _dev(step_bias, "step bias", None, (heads if per_head else heads * dim,)), _code(rate_log, "rate"), float(q_scale), float(unit_eps),
              1 if no_input else 0, 1 if accumulate else 0, _dev(segments, "segments", torch.int32), segments.shape[0],

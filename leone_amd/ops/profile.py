@@ -44,9 +44,11 @@ OPERATIONS = {
     "leone_relu_squared": "relu squared",
     "leone_head_gate": "head gate",
     "leone_outer_scan": "outer scan",
+    "leone_outer_step": "outer scan",
     "leone_outer_chain": "outer scan",
     "leone_exp_gates": "exp gates",
     "leone_delta_scan": "delta scan",
+    "leone_delta_step": "delta scan",
     "leone_delta_chain": "delta scan",
     "leone_embed_placed": "embed",
     "leone_glu": "swiglu",
