@@ -28,8 +28,9 @@
 // normalises and rotates the query heads (per-head RMSNorm, half-split rotation:
 // crates/leone/src/backend.rs:2182-2208, crates/leone/src/cpu.rs:1721-1779) for all four, the second and third do the
 // same for the new key and value, write them into the cache and leave them in shared memory, from where the
-// wave with the row's last tile puts them in their places.  One launch fewer a layer; the values are those of the
-// separate kernel (rowwise.hip).  Head sizes that are multiples of 64 only: there a lane holds both halves of its pairs.
+// wave with the row's last tile puts them in their places.  One launch fewer a layer; what the cache gets has, for heads of 64 and
+// 128 elements, the bits the separate kernel writes (rowwise.hip, its kernel in runs; of wider heads the sum of squares is added in
+// another order there).  Head sizes that are multiples of 64 only: there a lane holds both halves of its pairs.
 //
 // With few keys a call is a chain of trips to memory, and their order is what it costs: what norms and rotation
 // start from is asked for first, before the row's position is known; then the angles; then the block table; then every
@@ -340,12 +341,29 @@ attention_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__
         if (wave == 0 || (wave == 1 && writes)) {
             const AnyVec gain = wave == 0 ? from.q_gain : from.k_gain;
             float ss = 0.f;
+            if (wave == 0) {
 #pragma unroll
-            for (int s = 0; s < kSteps; ++s)
+                for (int s = 0; s < kSteps; ++s)
 #pragma unroll
-                for (int i = 0; i < 8; ++i) ss = fmaf(head_run[s][i], head_run[s][i], ss);
-            ss += __shfl_xor(ss, 16, kWave);                  // the four lanes that share head c
-            ss += __shfl_xor(ss, 32, kWave);
+                    for (int i = 0; i < 8; ++i) ss = fmaf(head_run[s][i], head_run[s][i], ss);
+                ss += __shfl_xor(ss, 16, kWave);              // the four lanes that share head c
+                ss += __shfl_xor(ss, 32, kWave);
+            } else {
+                // A key's squares are added in the separate kernel's order (a run's elements in turn with their partners', the
+                // runs' sums by halves), so that the cache holds the same bits whichever of the two wrote it.
+                float runs[4] = {0.f, 0.f, 0.f, 0.f};
+                static_assert(kHalfSteps <= 4, "runs of half a head, four a step");
+#pragma unroll
+                for (int s = 0; s < kHalfSteps; ++s)
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) {
+                        runs[s] = fmaf(head_run[s][i], head_run[s][i], runs[s]);
+                        runs[s] = fmaf(head_run[s + kHalfSteps][i], head_run[s + kHalfSteps][i], runs[s]);
+                    }
+                ss = (runs[0] + runs[2]) + (runs[1] + runs[3]);
+                ss += __shfl_xor(ss, 32, kWave);
+                ss += __shfl_xor(ss, 16, kWave);
+            }
             if (gain.ptr) {
                 const float inv = 1.0f / sqrtf(ss / static_cast<float>(kD) + from.eps);
 #pragma unroll
