@@ -1,15 +1,19 @@
 // Single-precision matrix product for the true 32-bit path:
 // C[M,N] = A[M,K] . B[N,K]^T on the float matrix instructions (products and sums in float, fused; no reduced-precision
 // mode).  The reference's scalar backend folds each output left to right in float (crates/leone/src/cpu.rs:1379-1405,
-// 1622-1640); here an output is one such chain, or the sum of a few (below), in an order that the sizes alone fix, so that a
-// launch repeats bit for bit.  (Off the 64-bit product by 1e-7 to 1e-6 of its norm over 1 to 1024 rows and K of 512 to 6144,
-// never more than the single chain that stood here: 4e-7 to 1.4e-6.)
+// 1622-1640).
 //
-// Two kernels.  Few rows (decoding): a product reads every weight once for 2 M operations, so the weights' bytes are the
-// bound and what matters is how much of them is in flight: a workgroup owns 16 rows of B, its waves share out K, and a wave
-// keeps eight 1 KB loads in the air.  Many rows (prompt portions): tiles staged through shared memory, bound by the matrix
-// instructions (256 operations a cycle and compute unit).  With few tiles K is cut into parts, whose results (planes in
-// a buffer of the caller's) a second kernel adds in order.
+// An output's bits depend on its row of A, its row of B and K alone, never on the rows that share the launch (what a request gets
+// does not depend on who is beside it): K is cut into segments by a rule on K (f32_segments), a segment's sum is that of chains of
+// 16 fused products, k ascending, added in order, and so is the segments' sum.  Both kernels below work that way.  What is added rounds
+// at the sum's size, so the short sums are also off by less than one chain over K (error against 64 bits over the result's norm, 1 to 1,024 rows:
+// K 512 1.0e-7, 2048 1.2e-7, 6144 1.6e-7; one chain 2.9e-7, 8.1e-7 and 9.9e-7).  A K below 256 is one chain, the scalar backend's fold.
+//
+// Few rows (decoding): a product reads every weight once for 2 M operations, so the weights' bytes are the
+// bound and what matters is how much of them is in flight: a workgroup owns 16 rows of B, its waves take a segment each, and a
+// wave keeps eight 1 KB loads of B in the air.  Many rows (prompt portions): tiles staged through shared memory, bound by
+// the matrix instructions (256 operations a cycle and compute unit).  With few tiles the segments are shared out over
+// workgroups, which leave them as planes in a buffer of the caller's for a second kernel to add.
 #include "common.h"
 #include "leone_hip.h"
 
@@ -33,17 +37,37 @@ __device__ inline f32x4 load_four(const float* __restrict__ row, int at, int k) 
     return v;
 }
 
+// The same where all four lie before the row's end.
+template <bool kVec>
+__device__ inline f32x4 load_whole(const float* __restrict__ at) {
+    if (kVec) return *reinterpret_cast<const f32x4*>(at);
+    return f32x4{at[0], at[1], at[2], at[3]};
+}
+
 // ---- few rows ------------------------------------------------------------------------------------------------------
-// Lane l of a wave holds, of 16 rows of B, row l % 16's elements 4 (l / 16) .. + 3 of every run of 16: one 16-byte load
-// a lane is 64 bytes of each of 16 rows, and the element j of all lanes is one 16 x 16 x 4 instruction.  A's rows lie the
-// same way, out of the caches (rows past the last are the last one again and not written).
+// Lane l of a wave loads, of 16 rows of B, row l % 16's elements 4 (l / 16) .. + 3 of every run of 16: one 16-byte load
+// a lane is 64 bytes of each of 16 rows.  A's rows lie the same way, out of the caches (rows past the last are the last one again
+// and not written).  The 16 x 16 x 4 instruction adds its four products in the order of the lanes' quarters, so the four quarters'
+// registers are transposed by lane swaps first: instruction j then takes elements 4 j .. 4 j + 3 in turn.
 constexpr int kStreamTile = 16;                        // rows of B a workgroup
 constexpr int kStreamRun = 64;                         // elements of K a wave takes at a time
 constexpr int kStreamLoads = kStreamRun / 16;
+constexpr int kChain = 16;                             // elements of K a chain of products: what a wave's 16-byte loads bring
 
-template <int kTilesM, int kWaves, bool kVec>
+// Register j of quarter g becomes register g of quarter j.
+__device__ inline f32x4 transpose_quarters(const f32x4 v) {
+    typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+    const auto bits = [](float f) { return __float_as_uint(f); };
+    const u32x2 p = __builtin_amdgcn_permlane32_swap(bits(v[0]), bits(v[2]), false, false);
+    const u32x2 q = __builtin_amdgcn_permlane32_swap(bits(v[1]), bits(v[3]), false, false);
+    const u32x2 r = __builtin_amdgcn_permlane16_swap(p[0], q[0], false, false);
+    const u32x2 s = __builtin_amdgcn_permlane16_swap(p[1], q[1], false, false);
+    return f32x4{__uint_as_float(r[0]), __uint_as_float(r[1]), __uint_as_float(s[0]), __uint_as_float(s[1])};
+}
+
+template <int kTilesM, int kWaves, int kDepth, bool kVec>
 __global__ void __launch_bounds__(kWaves * kWave)
-gemm_f32_stream_kernel(const float* __restrict__ a, const float* __restrict__ b, float* __restrict__ c, int m, int n, int k) {
+gemm_f32_stream_kernel(const float* __restrict__ a, const float* __restrict__ b, float* __restrict__ c, int m, int n, int k, int segment) {
     __shared__ float sums[kWaves][kTilesM][kStreamTile * kStreamTile];
     const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
     const int n0 = blockIdx.x * kStreamTile;
@@ -52,113 +76,158 @@ gemm_f32_stream_kernel(const float* __restrict__ a, const float* __restrict__ b,
     const float* arow[kTilesM];
 #pragma unroll
     for (int t = 0; t < kTilesM; ++t) arow[t] = a + static_cast<long>(t * 16 + r < m ? t * 16 + r : m - 1) * k;
-    // sums side by side, put together at the end: short chains, and what is added rounds at a smaller sum's size (sixteen waves
-    // have registers for two)
-    constexpr int kSums = kWaves == 16 ? 2 : 4;
-    f32x4 acc[kTilesM][kSums] = {};
-    f32x4 w[2][kStreamLoads], x[2][kTilesM][kStreamLoads];
-    auto fetch = [&](int at, int into) {
+    f32x4 sum[kTilesM] = {};
+    f32x4 w[kDepth][kStreamLoads], x[kDepth][kTilesM][kStreamLoads];
+    const int first = wave * segment, end = first + segment < k ? first + segment : k;
+    const auto fetch = [&](int at, int into) {         // a run that lies whole before the segment's end
 #pragma unroll
-        for (int i = 0; i < kStreamLoads; ++i) w[into][i] = load_four<kVec>(brow, at + i * 16 + h, k);
+        for (int i = 0; i < kStreamLoads; ++i) w[into][i] = load_whole<kVec>(brow + at + i * 16 + h);
 #pragma unroll
         for (int t = 0; t < kTilesM; ++t)
 #pragma unroll
-            for (int i = 0; i < kStreamLoads; ++i) x[into][t][i] = load_four<kVec>(arow[t], at + i * 16 + h, k);
+            for (int i = 0; i < kStreamLoads; ++i) x[into][t][i] = load_whole<kVec>(arow[t] + at + i * 16 + h);
     };
-    auto multiply = [&](int from) {
+    const auto multiply = [&](int from) {
 #pragma unroll
-        for (int i = 0; i < kStreamLoads; ++i)
+        for (int i = 0; i < kStreamLoads; ++i) {
+            const f32x4 wt = transpose_quarters(w[from][i]);
+            f32x4 xt[kTilesM];
+#pragma unroll
+            for (int t = 0; t < kTilesM; ++t) xt[t] = transpose_quarters(x[from][t][i]);
+            f32x4 acc[kTilesM] = {};
 #pragma unroll
             for (int j = 0; j < 4; ++j)
 #pragma unroll
-                for (int t = 0; t < kTilesM; ++t)
-                    acc[t][j % kSums] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[from][t][i][j], w[from][i][j], acc[t][j % kSums], 0, 0, 0);
-    };
-    // two runs' registers take turns: a run is asked for before the one ahead of it is multiplied
-    constexpr int kStep = kWaves * kStreamRun;
-    int at = wave * kStreamRun;
-    if (at < k) {
-        fetch(at, 0);
-        for (; at + kStep < k; at += 2 * kStep) {
-            fetch(at + kStep, 1);
-            multiply(0);
-            if (at + 2 * kStep < k) {
-                fetch(at + 2 * kStep, 0);
-                multiply(1);
-            } else {
-                multiply(1);
-                at += 2 * kStep;
-                break;
-            }
+                for (int t = 0; t < kTilesM; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(xt[t][j], wt[j], acc[t], 0, 0, 0);
+#pragma unroll
+            for (int t = 0; t < kTilesM; ++t) sum[t] += acc[t];
         }
-        if (at < k) multiply(0);
+    };
+    // whole runs, kDepth of them on their way at a time; the loop's body asks for a run on every pass, so that the compiler can
+    // count the loads in flight
+    int left = end > first ? (end - first) / kStreamRun : 0, at = first;
+    if (left >= kDepth) {
+#pragma unroll
+        for (int d = 0; d < kDepth; ++d) fetch(at + d * kStreamRun, d);
+        for (; left >= 2 * kDepth; left -= kDepth, at += kDepth * kStreamRun)
+#pragma unroll
+            for (int d = 0; d < kDepth; ++d) {
+                multiply(d);
+                fetch(at + (kDepth + d) * kStreamRun, d);
+            }
+#pragma unroll
+        for (int d = 0; d < kDepth; ++d) {
+            multiply(d);
+            if (kDepth + d < left) fetch(at + (kDepth + d) * kStreamRun, d);
+        }
+        left -= kDepth, at += kDepth * kStreamRun;
+    } else {
+#pragma unroll
+        for (int d = 0; d < kDepth - 1; ++d)
+            if (d < left) fetch(at + d * kStreamRun, d);
     }
 #pragma unroll
-    for (int t = 0; t < kTilesM; ++t) {
-        f32x4 sum = acc[t][0] + acc[t][1];
-        if constexpr (kSums == 4) sum += acc[t][2] + acc[t][3];
+    for (int d = 0; d < kDepth - 1; ++d)
+        if (d < left) multiply(d);
+    at += left * kStreamRun;
+    if (at < end) {                                    // the rest of the last segment, filled up with zeros
 #pragma unroll
-        for (int i = 0; i < 4; ++i) sums[wave][t][(h + i) * kStreamTile + r] = sum[i];
+        for (int i = 0; i < kStreamLoads; ++i) w[0][i] = load_four<kVec>(brow, at + i * 16 + h, end);
+#pragma unroll
+        for (int t = 0; t < kTilesM; ++t)
+#pragma unroll
+            for (int i = 0; i < kStreamLoads; ++i) x[0][t][i] = load_four<kVec>(arow[t], at + i * 16 + h, end);
+        multiply(0);
     }
+#pragma unroll
+    for (int t = 0; t < kTilesM; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sums[wave][t][(h + i) * kStreamTile + r] = sum[t][i];
     __syncthreads();
     for (int e = threadIdx.x; e < kTilesM * 256; e += kWaves * kWave) {
         const int t = e / 256, row = t * 16 + e % 256 / 16, col = n0 + e % 16;
         if (row >= m || col >= n) continue;
         float total = sums[0][t][e % 256];
 #pragma unroll
-        for (int v = 1; v < kWaves; ++v) total += sums[v][t][e % 256];
+        for (int v = 1; v < kWaves; ++v) total += sums[v][t][e % 256];        // (segments past K's end are zeros)
         c[static_cast<long>(row) * n + col] = total;
     }
 }
 
 // ---- many rows -----------------------------------------------------------------------------------------------------
-// A tile of kEdge x kEdge outputs, four waves of a quarter each (32 x 32 x 2 instructions, kEdge / 64 squared of them a
-// wave).  Slabs of K in shared memory, rows 4 floats further apart than they are long (16-byte reads of 8 neighbouring
+// A tile of kRows x 64 outputs, four waves of a quarter each (32 x 32 x 2 instructions, kRows / 64 of them a wave).  Slabs of K in
+// shared memory, rows 4 floats further apart than they are long (16-byte reads of 8 neighbouring
 // rows then touch every bank once); the next slab is on its way into registers while one is multiplied, and is long enough
-// (2048 cycles of instructions and more a wave) to arrive meanwhile.  Of every 8 elements the
+// (2048 cycles of instructions a wave) to arrive meanwhile.  Of every 8 elements the
 // even ones lie first and then the odd ones: half-wave h reads its four at once, and the four instructions take elements 0
-// and 1, 2 and 3, .. of them, so that an output is one chain of fused products, k ascending.
-constexpr int slab_of(int edge) { return edge == 128 ? 32 : 64; }
+// and 1, 2 and 3, .. of them: k ascending.  A chain, a segment's sum of chains and the sum of segments each have registers of their
+// own, which is what bounds the tile: 128 x 128 would need more than the 256 that two waves a SIMD leave each other.  1,024 rows
+// against 12288 x 2048: 470 us, 110 TFLOP/s (one chain an output in tiles of 128 x 128: 452); 777 rows 440 (408).
+//
+// kCut: blockIdx.z takes `each` segments and leaves a plane of c for every one of them; else one workgroup walks them all.  kChains:
+// segments are sums of chains of kChain elements, else one chain.
+constexpr int slab_of(int rows) { return rows == 128 ? 32 : 64; }
+constexpr int kTileCols = 64;
 
-template <int kEdge, bool kVec>
-__global__ void __launch_bounds__(256)
+template <int kRows, bool kVec, bool kCut, bool kChains>
+__global__ void __launch_bounds__(256, 2)
 gemm_f32_tile_kernel(const float* __restrict__ a, const float* __restrict__ b, float* __restrict__ c, int m, int n, int k,
-                     int part_k) {
-    constexpr int kSlab = slab_of(kEdge);
-    constexpr int kFrag = kEdge / 64;                  // 32 x 32 squares along an edge of a wave's quarter
-    constexpr int kLoads = kEdge * kSlab / 4 / 256;    // 16-byte loads a thread, matrix and slab
-    __shared__ float as[2][kEdge][kSlab + 4];
-    __shared__ float bs[2][kEdge][kSlab + 4];
+                     int segment, int each) {
+    constexpr int kSlab = slab_of(kRows);
+    constexpr int kFrag = kRows / 64;                  // 32 x 32 squares of a wave, one under the other
+    constexpr int kLoadsA = kRows * kSlab / 4 / 256, kLoadsB = kTileCols * kSlab / 4 / 256;    // 16-byte loads a thread and slab
+    __shared__ float as[2][kRows][kSlab + 4];
+    __shared__ float bs[2][kTileCols][kSlab + 4];
     const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-    const long m0 = static_cast<long>(blockIdx.y) * kEdge, n0 = static_cast<long>(blockIdx.x) * kEdge;
-    const int k_first = blockIdx.z * part_k, k_end = k_first + part_k < k ? k_first + part_k : k;
-    c += static_cast<long>(blockIdx.z) * m * n;
-    const int wm = (wave / 2) * (kEdge / 2), wn = (wave % 2) * (kEdge / 2);
-    f32x16 acc[kFrag][kFrag] = {};
-    f32x4 ra[kLoads], rb[kLoads];
-    auto fetch = [&](int k0) {
+    const int m0 = blockIdx.y * kRows, n0 = blockIdx.x * kTileCols;
+    const long part = static_cast<long>(segment) * each;
+    const int k_first = static_cast<int>(blockIdx.z * part), k_end = k - k_first > part ? static_cast<int>(k_first + part) : k;
+    const int wm = (wave / 2) * (kRows / 2), wn = (wave % 2) * (kTileCols / 2);
+    f32x16 acc[kFrag] = {}, sum[kFrag] = {}, total[kFrag] = {};
+    f32x4 ra[kLoadsA], rb[kLoadsB];
+    const auto fetch = [&](int k0) {
 #pragma unroll
-        for (int i = 0; i < kLoads; ++i) {
-            const int idx = threadIdx.x + i * 256, row = idx / (kSlab / 4), at = k0 + (idx % (kSlab / 4)) * 4;
-            const long gm = m0 + row < m ? m0 + row : m - 1, gn = n0 + row < n ? n0 + row : n - 1;
-            ra[i] = load_four<kVec>(a + gm * k, at, k_end);
-            rb[i] = load_four<kVec>(b + gn * k, at, k_end);
+        for (int i = 0; i < kLoadsA; ++i) {
+            const int idx = threadIdx.x + i * 256, row = m0 + idx / (kSlab / 4), at = k0 + (idx % (kSlab / 4)) * 4;
+            ra[i] = load_four<kVec>(a + static_cast<long>(row < m ? row : m - 1) * k, at, k_end);
+        }
+#pragma unroll
+        for (int i = 0; i < kLoadsB; ++i) {
+            const int idx = threadIdx.x + i * 256, row = n0 + idx / (kSlab / 4), at = k0 + (idx % (kSlab / 4)) * 4;
+            rb[i] = load_four<kVec>(b + static_cast<long>(row < n ? row : n - 1) * k, at, k_end);
         }
     };
-    auto keep = [&](int into) {
+    const auto put = [&](float* row, int at, const f32x4& v) {
+        const int even = at / 8 * 8 + at % 8 / 2;
+        *reinterpret_cast<f32x2*>(row + even) = f32x2{v[0], v[2]};
+        *reinterpret_cast<f32x2*>(row + even + 4) = f32x2{v[1], v[3]};
+    };
+    const auto keep = [&](int into) {
 #pragma unroll
-        for (int i = 0; i < kLoads; ++i) {
-            const int idx = threadIdx.x + i * 256, row = idx / (kSlab / 4), at = (idx % (kSlab / 4)) * 4;
-            const int even = at / 8 * 8 + at % 8 / 2;
-            *reinterpret_cast<f32x2*>(&as[into][row][even]) = f32x2{ra[i][0], ra[i][2]};
-            *reinterpret_cast<f32x2*>(&as[into][row][even + 4]) = f32x2{ra[i][1], ra[i][3]};
-            *reinterpret_cast<f32x2*>(&bs[into][row][even]) = f32x2{rb[i][0], rb[i][2]};
-            *reinterpret_cast<f32x2*>(&bs[into][row][even + 4]) = f32x2{rb[i][1], rb[i][3]};
+        for (int i = 0; i < kLoadsA; ++i) {
+            const int idx = threadIdx.x + i * 256;
+            put(as[into][idx / (kSlab / 4)], (idx % (kSlab / 4)) * 4, ra[i]);
         }
+#pragma unroll
+        for (int i = 0; i < kLoadsB; ++i) {
+            const int idx = threadIdx.x + i * 256;
+            put(bs[into][idx / (kSlab / 4)], (idx % (kSlab / 4)) * 4, rb[i]);
+        }
+    };
+    const auto store = [&](const f32x16 (&of)[kFrag], float* to) {
+        const int col = n0 + wn + lane % 32;
+#pragma unroll
+        for (int i = 0; i < kFrag; ++i)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const int row = m0 + wm + i * 32 + 8 * (e / 4) + 4 * (lane / 32) + e % 4;
+                if (row < m && col < n) to[static_cast<long>(row) * n + col] = of[i][e];
+            }
     };
     fetch(k_first);
     keep(0);
-    int at = 0;
+    int at = 0, segment_left = segment;                // segments are whole slabs
+    float* plane = c + static_cast<long>(blockIdx.z) * each * m * n;
     for (int k0 = k_first; k0 < k_end; k0 += kSlab, at ^= 1) {
         const bool more = k0 + kSlab < k_end;
         if (more) fetch(k0 + kSlab);
@@ -166,37 +235,46 @@ gemm_f32_tile_kernel(const float* __restrict__ a, const float* __restrict__ b, f
         const int row = lane % 32, h = (lane / 32) * 4;
 #pragma unroll
         for (int s = 0; s < kSlab; s += 8) {
-            f32x4 av[kFrag], bv[kFrag];
+            f32x4 av[kFrag];
+            const f32x4 bv = *reinterpret_cast<const f32x4*>(&bs[at][wn + row][s + h]);
 #pragma unroll
-            for (int i = 0; i < kFrag; ++i) {
-                av[i] = *reinterpret_cast<const f32x4*>(&as[at][wm + i * 32 + row][s + h]);
-                bv[i] = *reinterpret_cast<const f32x4*>(&bs[at][wn + i * 32 + row][s + h]);
-            }
+            for (int i = 0; i < kFrag; ++i) av[i] = *reinterpret_cast<const f32x4*>(&as[at][wm + i * 32 + row][s + h]);
 #pragma unroll
             for (int e = 0; e < 4; ++e)
 #pragma unroll
-                for (int i = 0; i < kFrag; ++i)
+                for (int i = 0; i < kFrag; ++i) acc[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[i][e], bv[e], acc[i], 0, 0, 0);
+            if (kChains && (s + 8) % kChain == 0) {
 #pragma unroll
-                    for (int j = 0; j < kFrag; ++j)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[i][e], bv[j][e], acc[i][j], 0, 0, 0);
+                for (int i = 0; i < kFrag; ++i) {
+                    sum[i] += acc[i];
+                    acc[i] = f32x16{};
+                }
+            }
         }
         if (more) keep(at ^ 1);        // read last two slabs ago, and every wave has passed a barrier since
-    }
-#pragma unroll
-    for (int i = 0; i < kFrag; ++i)
-#pragma unroll
-        for (int j = 0; j < kFrag; ++j)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                const long gm = m0 + wm + i * 32 + 8 * (e / 4) + 4 * (lane / 32) + e % 4, gn = n0 + wn + j * 32 + lane % 32;
-                if (gm < m && gn < n) c[gm * n + gn] = acc[i][j][e];
+        segment_left -= kSlab;
+        if (segment_left == 0 || !more) {
+            segment_left = segment;
+            if constexpr (kCut) {
+                store(sum, plane);
+                plane += static_cast<long>(m) * n;
             }
+#pragma unroll
+            for (int i = 0; i < kFrag; ++i) {
+                if constexpr (!kCut) total[i] += kChains ? sum[i] : acc[i];
+                sum[i] = f32x16{};
+            }
+        }
+    }
+    if constexpr (!kCut) store(total, c);
 }
 
-// C = the planes' sum, in order.
+// C = the planes' sum, in order.  kVec: planes and c are aligned to 16 bytes and `count` is a multiple of 4.
+template <bool kVec>
 __global__ void __launch_bounds__(256) gemm_f32_sum_kernel(const float* __restrict__ planes, float* __restrict__ c, long count, int parts) {
     const long at = (static_cast<long>(blockIdx.x) * 256 + threadIdx.x) * 4;
-    if (at + 4 <= count && count % 4 == 0) {
+    if (kVec) {
+        if (at >= count) return;
         f32x4 total = *reinterpret_cast<const f32x4*>(planes + at);
         for (int p = 1; p < parts; ++p) total += *reinterpret_cast<const f32x4*>(planes + p * count + at);
         *reinterpret_cast<f32x4*>(c + at) = total;
@@ -209,41 +287,50 @@ __global__ void __launch_bounds__(256) gemm_f32_sum_kernel(const float* __restri
     }
 }
 
-// Up to here a product is a stream of weights.  Measured against 2048 x 2048 weights (us, streamed : tiled): 14.6 : about 20 at 24
-// rows; at 64 rows the stream's reads of A, four times the weights', make it 46 : 16.
+// Up to here a product is a stream of weights.  Measured against 2048 x 2048 and 12288 x 2048 weights (us, streamed : tiled): 14.1 :
+// 14.3 and 40 : 43 at 24 rows, 15 : 14.5 and 43 : 44 at 32; beyond, the stream's reads of A, then four times the weights', cost more.
 constexpr int kStreamRows = 32;
-constexpr int kStreamK = 256;          // a shorter K is no work to share out over four waves
-constexpr int kPartMin = 256;          // elements of K in a part at least
-constexpr int kPartsMax = 16;
+constexpr int kStreamK = 256;          // a shorter K is no work to share out over four waves: one segment, in tiles whatever the rows
+
+// The segments of K: by K alone.  Eight from 512 elements on (a wave each of a streaming workgroup), four from 256, multiples
+// of 64 elements (a streaming wave's run, and whole slabs of a tile).
+struct F32Segments {
+    int length, count;
+};
+F32Segments f32_segments(int k) {
+    const int wanted = k < kStreamK ? 1 : k < 2 * kStreamK ? 4 : 8;
+    const int length = ceil_div(ceil_div(k, wanted), kStreamRun) * kStreamRun;
+    return {length, ceil_div(k, length)};
+}
 
 struct F32Plan {
-    int edge = 0, parts = 1, part_k = 0;               // edge 0: the streaming kernel
+    int rows = 0, parts = 1, each = 1;                 // rows of a tile, 0: the streaming kernel; parts workgroups of `each` segments along K
 };
 
-// The tile and the number of parts that keep the chip busiest.  A compute unit's matrix instructions run at one rate however
-// many tiles it holds, so what is lost is what tiles cover past the edges and what the fullest of the 256 units has more than
-// the others; one tile a unit leaves a wave a SIMD and its waits in the open (measured at two thirds of the rate of three);
-// every part writes and reads a plane.
+// The tile and the cut of K that take least time.  A compute unit's matrix instructions run at one rate however many tiles it
+// holds, so the product takes as long as the fullest of the 256 units has work for; one tile a unit leaves a wave a SIMD and
+// its waits in the open.  A cut K costs a plane written and read for every segment (mostly in the caches) and a second launch.
+// Constants fitted to every tile and cut timed at 33 to 1,024 rows against 512 x 512 to 32768 x 2048 and 2048 x 6144 weights: the
+// choice is within 6 % of the best at each.
 F32Plan f32_plan(int m, int n, int k) {
     F32Plan best;
-    best.part_k = k;
+    const F32Segments segments = f32_segments(k);
+    best.each = segments.count;
     if (m <= kStreamRows && k >= kStreamK) return best;
     constexpr long kUnits = 256;
-    double most = 0.0;
-    for (int edge : {128, 64}) {
-        const long tiles = static_cast<long>(ceil_div(m, edge)) * ceil_div(n, edge);
-        const double inside = static_cast<double>(m) * n / (static_cast<double>(tiles) * edge * edge);
-        for (int wanted = 1; wanted <= kPartsMax && (wanted == 1 || k / wanted >= kPartMin); ++wanted) {
-            const int part_k = ceil_div(ceil_div(k, wanted), 64) * 64, parts = ceil_div(k, part_k);
-            const long each = (tiles * parts + kUnits - 1) / kUnits;                     // of the fullest unit
-            const double busy = static_cast<double>(tiles) * k / (static_cast<double>(each) * kUnits * part_k);
-            const double hidden = edge == 128 ? 1.0 : each >= 3 ? 0.9 : each == 2 ? 0.8 : 0.65;
-            const double worth = inside * busy * hidden / (1.0 + 0.04 * (parts - 1));
-            if (worth > most * 1.001) {
-                most = worth;
-                best.edge = edge;
-                best.parts = parts;
-                best.part_k = parts == 1 ? k : part_k;
+    constexpr double kUnitRate = 0.6e6, kPlaneRate = 30e6, kLaunch = 6.0;      // operations and bytes a microsecond; microseconds
+    double least = 0.0;
+    for (int rows : {128, 64}) {
+        const long tiles = static_cast<long>(ceil_div(m, rows)) * ceil_div(n, kTileCols);
+        for (int wanted = 1; wanted <= segments.count; wanted *= 2) {
+            const int each = ceil_div(segments.count, wanted), parts = ceil_div(segments.count, each);
+            const long held = (tiles * parts + kUnits - 1) / kUnits;           // of the fullest unit
+            const double hidden = rows == 128 ? (held >= 2 ? 0.87 : 0.4) : (held >= 2 ? 0.82 : 0.65);
+            const double product = 2.0 * held * rows * kTileCols * segments.length * each / (kUnitRate * hidden);
+            const double planes = parts == 1 ? 0.0 : kLaunch + 8.0 * segments.count * m * n / kPlaneRate;
+            if (best.rows == 0 || product + planes < least * 0.999) {
+                least = product + planes;
+                best.rows = rows, best.parts = parts, best.each = each;
             }
         }
     }
@@ -258,7 +345,7 @@ using namespace leone;
 extern "C" int leone_gemm_f32_planes(int m, int n, int k) {
     if (m <= 0 || n <= 0 || k <= 0) return 0;
     const F32Plan p = f32_plan(m, n, k);
-    return p.parts > 1 ? p.parts : 0;
+    return p.parts > 1 ? f32_segments(k).count : 0;
 }
 
 // planes: room for leone_gemm_f32_planes(m, n, k) results (null if that is 0).
@@ -266,46 +353,54 @@ extern "C" int leone_gemm_f32(const float* a, const float* b, float* c, float* p
     LEONE_REQUIRE(a && b && c, "gemm_f32: null pointer");
     LEONE_REQUIRE(m > 0 && n > 0 && k > 0, "gemm_f32: sizes %d x %d x %d must be positive", m, n, k);
     const F32Plan p = f32_plan(m, n, k);
-    LEONE_REQUIRE(p.parts == 1 || planes, "gemm_f32: %d planes are needed for %d x %d x %d", p.parts, m, n, k);
-    const bool vec = k % 4 == 0 && reinterpret_cast<uintptr_t>(a) % 16 == 0 && reinterpret_cast<uintptr_t>(b) % 16 == 0;
-    if (p.edge == 0) {
+    const F32Segments segments = f32_segments(k);
+    LEONE_REQUIRE(p.parts == 1 || planes, "gemm_f32: %d planes are needed for %d x %d x %d", segments.count, m, n, k);
+    const auto aligned = [](const void* at) { return reinterpret_cast<uintptr_t>(at) % 16 == 0; };
+    const bool vec = k % 4 == 0 && aligned(a) && aligned(b);
+    if (p.rows == 0) {
         const int blocks = ceil_div(n, kStreamTile);
-        // waves share out K in runs of 64; sixteen of them where the workgroups are few, so that the chip has loads enough in flight
-        const int runs = ceil_div(k, kStreamRun);
-        const int tiles = m <= 16 ? 1 : 2;
-        const int waves = runs >= 16 && tiles == 1 && blocks < 512 && vec ? 16 : runs >= 8 ? 8 : 4;
-#define LEONE_STREAM(T, W)                                                                                                \
-    (vec ? gemm_f32_stream_kernel<T, W, true><<<blocks, W * kWave, 0, stream>>>(a, b, c, m, n, k)                          \
-         : gemm_f32_stream_kernel<T, W, false><<<blocks, W * kWave, 0, stream>>>(a, b, c, m, n, k))
-#define LEONE_STREAM_TILES(T) (waves == 8 ? LEONE_STREAM(T, 8) : LEONE_STREAM(T, 4))
-        if (tiles == 1) {
-            if (waves == 16) gemm_f32_stream_kernel<1, 16, true><<<blocks, 16 * kWave, 0, stream>>>(a, b, c, m, n, k);
-            else LEONE_STREAM_TILES(1);
+#define LEONE_STREAM(T, W, D)                                                                                                          \
+    (vec ? gemm_f32_stream_kernel<T, W, D, true><<<blocks, W * kWave, 0, stream>>>(a, b, c, m, n, k, segments.length)                  \
+         : gemm_f32_stream_kernel<T, W, D, false><<<blocks, W * kWave, 0, stream>>>(a, b, c, m, n, k, segments.length))
+        // Runs on their way a wave: two leave room for more waves, whose loads count as well (one row against 12288 x 2048 18.4 us,
+        // with four 24.4); two tiles of A take long enough over a run for three (24 rows against 2048 x 6144 37.8, with four 43.1).
+        if (segments.count <= 4) {
+            if (m <= kStreamTile) LEONE_STREAM(1, 4, 2);
+            else LEONE_STREAM(2, 4, 3);
         } else {
-            LEONE_STREAM_TILES(2);
+            if (m <= kStreamTile) LEONE_STREAM(1, 8, 2);
+            else LEONE_STREAM(2, 8, 3);
         }
-#undef LEONE_STREAM_TILES
 #undef LEONE_STREAM
         LEONE_LAUNCH_CHECK("gemm_f32");
         return 0;
     }
-    const int grid_y = ceil_div(m, p.edge);
+    const int grid_y = ceil_div(m, p.rows);
     LEONE_REQUIRE(grid_y <= 65535, "gemm_f32: %d rows exceed the launch limit", m);
-    const dim3 grid(ceil_div(n, p.edge), grid_y, p.parts);
-    float* into = p.parts > 1 ? planes : c;
-#define LEONE_TILE(E, V) gemm_f32_tile_kernel<E, V><<<grid, 256, 0, stream>>>(a, b, into, m, n, k, p.part_k)
-    if (p.edge == 128) {
+    const dim3 grid(ceil_div(n, kTileCols), grid_y, p.parts);
+#define LEONE_TILE_CHAIN(E, V, CHAIN)                                                                                                  \
+    (p.parts > 1 ? gemm_f32_tile_kernel<E, V, true, CHAIN><<<grid, 256, 0, stream>>>(a, b, planes, m, n, k, segments.length, p.each)   \
+                 : gemm_f32_tile_kernel<E, V, false, CHAIN><<<grid, 256, 0, stream>>>(a, b, c, m, n, k, segments.length, p.each))
+#define LEONE_TILE(E, V)                                                                                                               \
+    (segments.count > 1 ? LEONE_TILE_CHAIN(E, V, true)                                                                               \
+                        : gemm_f32_tile_kernel<E, V, false, false><<<grid, 256, 0, stream>>>(a, b, c, m, n, k, segments.length, p.each))
+    if (p.rows == 128) {
         if (vec) LEONE_TILE(128, true);
         else LEONE_TILE(128, false);
     } else {
         if (vec) LEONE_TILE(64, true);
         else LEONE_TILE(64, false);
     }
+#undef LEONE_TILE_CHAIN
 #undef LEONE_TILE
     LEONE_LAUNCH_CHECK("gemm_f32");
     if (p.parts > 1) {
         const long count = static_cast<long>(m) * n;
-        gemm_f32_sum_kernel<<<ceil_div(count, 1024), 256, 0, stream>>>(planes, c, count, p.parts);
+        const int blocks = ceil_div(count, 1024);
+        if (count % 4 == 0 && aligned(planes) && aligned(c))
+            gemm_f32_sum_kernel<true><<<blocks, 256, 0, stream>>>(planes, c, count, segments.count);
+        else
+            gemm_f32_sum_kernel<false><<<blocks, 256, 0, stream>>>(planes, c, count, segments.count);
         LEONE_LAUNCH_CHECK("gemm_f32 sum");
     }
     return 0;

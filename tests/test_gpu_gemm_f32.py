@@ -50,3 +50,31 @@ def test_rows_do_not_depend_on_their_neighbours():
         keep = [i for i in range(m) if i not in (1, 2)]
         assert torch.equal(clean[keep], spoilt[keep])
         assert bool(torch.isinf(spoilt[1]).all()) and bool(torch.isnan(spoilt[2]).all())
+
+
+@pytest.mark.parametrize("n,k", [(40, 200), (96, 256), (70, 333), (512, 512), (100, 1000), (530, 2052), (2048, 2048), (256, 6144)])
+def test_a_row_is_the_same_whatever_rows_are_beside_it(n, k):
+    """To the bit, over both kernels, their tiles and cuts of K, and whether the operands are aligned."""
+    from leone_amd import ops
+    gen = torch.Generator(device=DEV).manual_seed(k)
+    a, b = torch.randn(1024, k, generator=gen, device=DEV), torch.randn(n, k, generator=gen, device=DEV)
+    alone = torch.cat([ops.gemm_f32(a[i:i + 1].contiguous(), b) for i in (0, 1, 15)])
+    for m in (16, 17, 32, 33, 64, 65, 128, 200, 300, 777, 1024):
+        together = ops.gemm_f32(a[:m].contiguous(), b)
+        assert torch.equal(together[[0, 1, 15]], alone), m
+        moved = torch.empty(m * k + 1, device=DEV)[1:].view(m, k).copy_(a[:m])
+        assert torch.equal(ops.gemm_f32(moved, b), together), m
+
+
+def test_results_off_sixteen_bytes():
+    """Where K is cut, the sum over its parts writes a result that lies anywhere."""
+    from leone_amd import ops
+    m, n, k = 40, 128, 2048
+    assert ops.library().leone_gemm_f32_planes(m, n, k) > 1
+    a, b = torch.randn(m, k, device=DEV), torch.randn(n, k, device=DEV)
+    want = ops.gemm_f32(a, b)
+    for shift in (1, 2, 3):
+        room = torch.full((m * n + 8,), 7.0, device=DEV)
+        ops.gemm_f32(a, b, out=room[shift:shift + m * n].view(m, n))
+        assert torch.equal(room[shift:shift + m * n].view(m, n), want)
+        assert bool((room[:shift] == 7.0).all()) and bool((room[shift + m * n:] == 7.0).all())
