@@ -3,17 +3,21 @@
 //
 // A query row alone reads every key for itself, which bounds a row by the walk along its keys (one dot product and one
 // step of the softmax a key).  Here a workgroup takes up to 16 queries that read the same keys - the query heads of one
-// kv head, of a few neighbouring rows of one request - and its waves share out the keys, 16 at a time, each wave with a
-// running softmax of its own; the waves' results are merged through shared memory in a fixed order.  What bounds it is
+// kv head, of a few neighbouring rows of one request - and its waves share out the keys, 16 at a time, in eight shares with a
+// running softmax each; the shares' results are merged through shared memory in a fixed order.  What bounds it is
 // the matrix instructions: 64 of 32 cycles for 16 keys of 128 elements, whose loads (16 KB a wave) are in flight meanwhile.
+//
+// A row's result depends on its own query and on the keys that it sees alone, to the bit, whichever rows share the workgroup or the
+// launch: a tile of keys belongs to a share by the keys' positions, a share's tiles are taken in their order, and tiles that a row
+// does not see add nothing to it.
 //
 // Lane l of a wave holds, of a product, row or column l % 16, and inner elements 4 (l / 16) .. + 3 of every 16: with the
 // cache's runs of 8 a 16-byte load a lane brings 16 keys x 16 elements, or 16 value elements x 16 tokens.  Scores are made
 // as keys x queries, so that a lane's four scores belong to its own query and to the four keys it holds values of: they
 // are the operand of the second product as they stand.
 //
-// Measured (us; the row kernel of attention.hip before): 16 heads over 4 of 128 elements, one row at 780 keys 29 (314), a prompt
-// of 777 rows 81 (1375).
+// Measured (us; the row kernel of attention.hip before): 16 heads over 4 of 128 elements, one row at 780 keys 25 (314), a prompt
+// of 777 rows 73 (1375).
 #include "common.h"
 #include "leone_hip.h"
 #include "score_shape.h"
@@ -26,6 +30,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kQueries = 16;
 constexpr int kKeys = 16;
+constexpr int kShares = 8;
 
 struct AttentionF32Args {
     const float* q;
@@ -48,10 +53,11 @@ struct AttentionF32Args {
     int chunk;
 };
 
+// kWaves waves with kShares / kWaves shares each.
 template <int kDim, int kWaves>
-__global__ void __launch_bounds__(kWaves * kWave) attention_f32_kernel(const AttentionF32Args g) {
-    constexpr int kRuns = kDim / 16;
-    __shared__ float sm_m[kWaves][kQueries], sm_l[kWaves][kQueries];
+__global__ void __launch_bounds__(kWaves * kWave, kDim == 64 ? 3 : 2) attention_f32_kernel(const AttentionF32Args g) {
+    constexpr int kRuns = kDim / 16, kOwn = kShares / kWaves;
+    __shared__ float sm_m[kShares][kQueries], sm_l[kShares][kQueries];
     __shared__ f32x4 sm_acc[kWaves / 2][kRuns][kWave];
 
     // The rows of this workgroup: from this one on, those of the same request up to the next multiple of `most`; the
@@ -89,14 +95,17 @@ __global__ void __launch_bounds__(kWaves * kWave) attention_f32_kernel(const Att
     }
     const int low_tile = low / kKeys;
     const int kept_tiles = min((g.keep_first + kKeys - 1) / kKeys, low_tile);
-    const int tiles = kept_tiles + high / kKeys + 1 - low_tile;
+    const int tiles = high / kKeys + 1;
     const int* table = g.block_table + static_cast<long>(entry) * g.max_blocks;
     const long page_floats = static_cast<long>(g.page_tokens) * kDim;
 
     f32x4 kf[kRuns], vf[kRuns], acc[kRuns] = {};
+    [[maybe_unused]] f32x4 ready[kOwn == 2 ? kRuns : 1];      // the first of two shares
     float m = -INFINITY, l = 0.f;
     bool mapped = true, mapped_next = true;
-    const auto start_of = [&](int t) { return (t < kept_tiles ? t : low_tile + t - kept_tiles) * kKeys; };
+    // share n's tiles are those whose number is n modulo kShares, wave w has the shares that are w modulo kWaves; past the kept
+    // tiles, from the first that a row sees on
+    const auto skip = [&](int t) { return t < kept_tiles || t >= low_tile ? t : t + (low_tile - t + kShares - 1) / kShares * kShares; };
     const auto block_of = [&](int start, bool& there) {
         const int page = table[start / g.page_tokens];
         there = page >= 0;
@@ -112,138 +121,163 @@ __global__ void __launch_bounds__(kWaves * kWave) attention_f32_kernel(const Att
 #pragma unroll
         for (int i = 0; i < kRuns; ++i) vf[i] = *reinterpret_cast<const f32x4*>(at + i * 128);
     };
-    int t = wave;
-    long block = 0;
-    if (t < tiles) {
-        block = block_of(start_of(t), mapped);
-        fetch_keys(start_of(t), block);
-    }
-    for (; t < tiles; t += kWaves) {
-        const int start = start_of(t);
-        fetch_values(start, block);
-        f32x4 dots[4] = {};                   // four sums side by side: no instruction waits for the one before it
+#pragma unroll 1
+    for (int own = wave; own < kShares; own += kWaves) {
+        if constexpr (kOwn == 2) {
+            if (own != wave) {
 #pragma unroll
-        for (int i = 0; i < kRuns; ++i)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) dots[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[i][j], q[i][j], dots[j], 0, 0, 0);
-        f32x4 s = (dots[0] + dots[1]) + (dots[2] + dots[3]);
-        if (t + kWaves < tiles) {             // the keys' registers are free: the next tile's are on their way from here on
-            const int next = start_of(t + kWaves);
-            block = block_of(next, mapped_next);
-            fetch_keys(next, block);
-        }
-        float top = -INFINITY;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int key = start + h + r;
-            const bool seen = key <= pos && (key >= first || key < g.keep_first);
-            float v = s[r] * scale;
-            if (g.shape.cap > 0.f) v = g.shape.cap * tanhf(v / g.shape.cap);
-            v -= slope * static_cast<float>(pos - key);
-            // an unmapped block poisons the result of every row that sees it
-            s[r] = seen ? (mapped ? v : __builtin_nanf("")) : -INFINITY;
-            top = fmaxf(top, s[r]);
-        }
-        top = fmaxf(top, __shfl_xor(top, 16, kWave));
-        top = fmaxf(top, __shfl_xor(top, 32, kWave));
-        const float m_new = fmaxf(m, top);
-        const float reference = m_new == -INFINITY ? 0.f : m_new;      // nothing seen yet: every weight is 0
-        const float alpha = expf(m - reference);
-        float sum = 0.f;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            s[r] = expf(s[r] - reference);
-            sum += s[r];
-        }
-        sum += __shfl_xor(sum, 16, kWave);
-        sum += __shfl_xor(sum, 32, kWave);
-        l = l * alpha + sum;
-        m = m_new;
-        if (!mapped || start + kKeys > high + 1) {       // places nobody has written: their weight is 0, but not what they may hold
-#pragma unroll
-            for (int i = 0; i < kRuns; ++i)
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    if (!mapped || start + h + r > high) vf[i][r] = 0.f;
-        }
-        f32x4 odd = {0.f, 0.f, 0.f, 0.f};                // stays 0 unless a value is infinite or NaN
-#pragma unroll
-        for (int i = 0; i < kRuns; ++i) {
-            acc[i] *= alpha;
-            odd += vf[i] * 0.f;
-        }
-        if (__any(!(odd[0] + odd[1] + odd[2] + odd[3] == 0.f))) {
-            // such a value is for the rows that see it, and no weight of 0 keeps it from the others: one key after the other
-            for (int from = 0; from < 4; ++from)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const int key = start + 4 * from + j;
-                    const bool seen = key <= pos && (key >= first || key < g.keep_first);
-                    const float p = __shfl(s[j], from * 16 + mine, kWave);
-#pragma unroll
-                    for (int i = 0; i < kRuns; ++i)
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) {
-                            const float v = __shfl(vf[i][j], from * 16 + h + r, kWave);
-                            if (seen) acc[i][r] = fmaf(p, v, acc[i][r]);
-                        }
+                for (int i = 0; i < kRuns; ++i) {
+                    ready[i] = acc[i];
+                    acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
                 }
-        } else {
+                m = -INFINITY, l = 0.f;
+                mapped = true;
+            }
+        }
+        int t = skip(own);
+        long block = 0;
+        if (t < tiles) {
+            block = block_of(t * kKeys, mapped);
+            fetch_keys(t * kKeys, block);
+        }
+        while (t < tiles) {
+            const int start = t * kKeys;
+            t = skip(t + kShares);
+            fetch_values(start, block);
+            f32x4 dots[4] = {};                   // four sums side by side: no instruction waits for the one before it
 #pragma unroll
             for (int i = 0; i < kRuns; ++i)
 #pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[i][j], s[j], acc[i], 0, 0, 0);
+                for (int j = 0; j < 4; ++j) dots[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[i][j], q[i][j], dots[j], 0, 0, 0);
+            f32x4 s = (dots[0] + dots[1]) + (dots[2] + dots[3]);
+            if (t < tiles) {                      // the keys' registers are free: the next tile's are on their way from here on
+                block = block_of(t * kKeys, mapped_next);
+                fetch_keys(t * kKeys, block);
+            }
+            float top = -INFINITY;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int key = start + h + r;
+                const bool seen = key <= pos && (key >= first || key < g.keep_first);
+                float v = s[r] * scale;
+                if (g.shape.cap > 0.f) v = g.shape.cap * tanhf(v / g.shape.cap);
+                v -= slope * static_cast<float>(pos - key);
+                // an unmapped block poisons the result of every row that sees it
+                s[r] = seen ? (mapped ? v : __builtin_nanf("")) : -INFINITY;
+                top = fmaxf(top, s[r]);
+            }
+            top = fmaxf(top, __shfl_xor(top, 16, kWave));
+            top = fmaxf(top, __shfl_xor(top, 32, kWave));
+            const float m_new = fmaxf(m, top);
+            const float reference = m_new == -INFINITY ? 0.f : m_new;      // nothing seen yet: every weight is 0
+            const float alpha = expf(m - reference);
+            float sum = 0.f;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                s[r] = expf(s[r] - reference);
+                sum += s[r];
+            }
+            sum += __shfl_xor(sum, 16, kWave);
+            sum += __shfl_xor(sum, 32, kWave);
+            l = l * alpha + sum;
+            m = m_new;
+            if (!mapped || start + kKeys > high + 1) {       // places nobody has written: their weight is 0, but not what they may hold
+#pragma unroll
+                for (int i = 0; i < kRuns; ++i)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        if (!mapped || start + h + r > high) vf[i][r] = 0.f;
+            }
+            f32x4 odd = {0.f, 0.f, 0.f, 0.f};                // stays 0 unless a value is infinite or NaN
+#pragma unroll
+            for (int i = 0; i < kRuns; ++i) {
+                acc[i] *= alpha;
+                odd += vf[i] * 0.f;
+            }
+            if (__any(!(odd[0] + odd[1] + odd[2] + odd[3] == 0.f))) {
+                // such a value is for the rows that see it, and no weight of 0 keeps it from the others: one key after the other, in
+                // the order of the instructions below
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+#pragma unroll 1
+                    for (int from = 0; from < 4; ++from) {
+                        const int key = start + 4 * from + j;
+                        const bool seen = key <= pos && (key >= first || key < g.keep_first);
+                        const float p = __shfl(s[j], from * 16 + mine, kWave);
+#pragma unroll
+                        for (int i = 0; i < kRuns; ++i)
+#pragma unroll
+                            for (int r = 0; r < 4; ++r) {
+                                const float v = __shfl(vf[i][j], from * 16 + h + r, kWave);
+                                if (seen) acc[i][r] = fmaf(p, v, acc[i][r]);
+                            }
+                    }
+            } else {
+#pragma unroll
+                for (int i = 0; i < kRuns; ++i)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[i][j], s[j], acc[i], 0, 0, 0);
+            }
+            mapped = mapped_next;
         }
-        mapped = mapped_next;
+        if (lane < kQueries) {
+            sm_m[own][lane] = m;
+            sm_l[own][lane] = l;
+        }
     }
 
-    // ---- the waves' results, merged -------------------------------------------------------------------------------
-    if (lane < kQueries) {
-        sm_m[wave][lane] = m;
-        sm_l[wave][lane] = l;
-    }
+    // ---- the shares' results, merged: by halves, a share's result rounded before it is added --------------------------
     __syncthreads();
     float top = sm_m[0][mine];
 #pragma unroll
-    for (int w = 1; w < kWaves; ++w) top = fmaxf(top, sm_m[w][mine]);
+    for (int w = 1; w < kShares; ++w) top = fmaxf(top, sm_m[w][mine]);
     const float sink = g.shape.sinks ? g.shape.sinks[head] : -INFINITY;
     top = fmaxf(top, sink);
     const auto weight = [&](float of) { return of == -INFINITY ? 0.f : expf(of - top); };
     float denom = g.shape.sinks ? expf(sink - top) : 0.f;
 #pragma unroll
-    for (int w = 0; w < kWaves; ++w) denom += sm_l[w][mine] * weight(sm_m[w][mine]);
-    const float own = weight(m);
+    for (int w = 0; w < kShares; ++w) denom += sm_l[w][mine] * weight(sm_m[w][mine]);
+    f32x4 result[kRuns];
+    {
+#pragma clang fp contract(off)
+        static_assert(kOwn <= 2 && kShares == kOwn * kWaves, "a wave's two shares are the first halves that meet");
+        const float own = weight(m);
 #pragma unroll
-    for (int i = 0; i < kRuns; ++i) acc[i] *= own;
+        for (int i = 0; i < kRuns; ++i) result[i] = acc[i] * own;
+        if constexpr (kOwn == 2) {
+            const float first_own = weight(sm_m[wave][mine]);
 #pragma unroll
-    for (int half = kWaves / 2; half > 0; half /= 2) {
-        if (wave >= half && wave < 2 * half) {
-#pragma unroll
-            for (int i = 0; i < kRuns; ++i) sm_acc[wave - half][i][lane] = acc[i];
+            for (int i = 0; i < kRuns; ++i) result[i] = ready[i] * first_own + result[i];
         }
-        __syncthreads();
-        if (wave < half) {
 #pragma unroll
-            for (int i = 0; i < kRuns; ++i) acc[i] += sm_acc[wave][i][lane];
+        for (int half = kWaves / 2; half > 0; half /= 2) {
+            if (wave >= half && wave < 2 * half) {
+#pragma unroll
+                for (int i = 0; i < kRuns; ++i) sm_acc[wave - half][i][lane] = result[i];
+            }
+            __syncthreads();
+            if (wave < half) {
+#pragma unroll
+                for (int i = 0; i < kRuns; ++i) result[i] += sm_acc[wave][i][lane];
+            }
+            __syncthreads();
         }
-        __syncthreads();
     }
     if (wave != 0) return;
     // lane l: its query's elements 16 i + h .. + 3
 #pragma unroll
-    for (int i = 0; i < kRuns; ++i) acc[i] /= denom;
-    f32x4 result[kRuns];
+    for (int i = 0; i < kRuns; ++i) result[i] /= denom;
     if (g.shape.turn_cos) {
+        f32x4 turned[kRuns];
 #pragma unroll
         for (int i = 0; i < kRuns; ++i)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const float partner = g.shape.turn_pairing ? acc[i][r ^ 1] : acc[(i + kRuns / 2) % kRuns][r];
-                result[i][r] = turned_back(acc[i][r], partner, i * 16 + h + r, kDim, pos, g.shape);
+                const float partner = g.shape.turn_pairing ? result[i][r ^ 1] : result[(i + kRuns / 2) % kRuns][r];
+                turned[i][r] = turned_back(result[i][r], partner, i * 16 + h + r, kDim, pos, g.shape);
             }
-    } else {
 #pragma unroll
-        for (int i = 0; i < kRuns; ++i) result[i] = acc[i];
+        for (int i = 0; i < kRuns; ++i) result[i] = turned[i];
     }
     if (!real) return;
     float* orow = g.out + (static_cast<long>(row) * g.q_heads + head) * kDim;
@@ -277,16 +311,13 @@ void launch_attention_f32(const float* q, float* out, const float* k_pool, const
                                 page_tokens, scale, window, gate, gate_stride, keep_first, gate_each, slopes, temp_coef, temp_every,
                                 shape, chunk};
     const dim3 grid(rows, kv_heads);
-    // Few rows leave the chip to few workgroups: eight waves share out a row's keys (one row at 780 keys 29 us; the keys are
-    // bound by what one compute unit can read).  Workgroups that fill the chip by themselves (two a compute unit and more) take
-    // four, whose merge is half as long.
-    const bool few = static_cast<long>(rows) * kv_heads < 512;
-#define LEONE_ATTENTION_F32(D)                                                                    \
-    (few ? attention_f32_kernel<D, 8><<<grid, 8 * kWave, 0, stream>>>(args)                       \
-         : attention_f32_kernel<D, 4><<<grid, 4 * kWave, 0, stream>>>(args))
-    if (head_dim == 128) LEONE_ATTENTION_F32(128);
-    else LEONE_ATTENTION_F32(64);
-#undef LEONE_ATTENTION_F32
+    // Eight waves, a share each, where the launch is small or heads are of 128 elements (777 rows of 16 heads over 4: 73 us, with
+    // four waves 83); four waves with two shares each for many rows of 64, whose workgroups are short (1,500 rows of 8 heads
+    // over 2: 161 us, with eight 192; 200 rows: 15.7 and 14.5).  rows * kv_heads are launched; of the rows that share a workgroup
+    // all but the first's leave at once, which costs less the fewer waves they have.
+    if (head_dim == 128) attention_f32_kernel<128, 8><<<grid, 8 * kWave, 0, stream>>>(args);
+    else if (static_cast<long>(rows) * kv_heads < 512) attention_f32_kernel<64, 8><<<grid, 8 * kWave, 0, stream>>>(args);
+    else attention_f32_kernel<64, 4><<<grid, 4 * kWave, 0, stream>>>(args);
 }
 
 }  // namespace leone

@@ -93,3 +93,28 @@ def test_what_is_not_finite_stays_with_the_rows_that_see_it():
     inf, nan = float("inf"), float("nan")
     agree(both(MIXED, 4, 2, 64, spoil=[(0, 20, nan), (1, 100, inf), (1, 101, -inf), (2, 149, inf), (3, 8, nan)]))
     agree(both(MIXED, 4, 2, 64, unmapped=[(0, 0), (1, 64)], window=25))
+
+
+@pytest.mark.parametrize("options", [dict(), dict(window=20), dict(window=33, keep_first=5), dict(window=130, keep_first=40), dict(chunk=24)], ids=str)
+@pytest.mark.parametrize("size,group,kv_heads", [(64, 1, 3), (64, 4, 2), (128, 3, 2), (128, 16, 1)])
+def test_a_row_is_the_same_whatever_rows_are_beside_it(size, group, kv_heads, options):
+    """To the bit: each row alone, the rows of a step, and enough rows that other launches are taken; with values that are not finite
+    behind some of them as well."""
+    rows = [(r + 6 * copy, p) for copy in range(8) for r, p in MIXED]
+    for spoil in (None, [(0, 20, float("nan")), (1, 145, float("inf"))]):
+        many = both(rows, group, kv_heads, size, spoil=spoil, **options)
+        # the rows' queries and requests' keys are made in order, so those of fewer rows have to be cut out of the many
+        gen = torch.Generator().manual_seed(17)
+        requests = 1 + max(r for r, _ in rows)
+        k, v = (torch.randn(requests, 150, kv_heads, size, generator=gen) for _ in range(2))
+        for request, position, value in spoil or []:
+            v[request, position, 0, 5] = value
+        q = (2.0 * torch.randn(len(rows), group * kv_heads * size, generator=gen)).to(DEV)
+        from leone_amd import ops
+        k_pool, v_pool, table = pools(k, v, 16, 16)
+        for chosen in (range(len(MIXED)), range(5, 30), [0], [3], [40], [95], [99]):
+            chosen = list(chosen)
+            got = ops.attention_rows(q[chosen].contiguous(), k_pool, v_pool, torch.tensor([rows[i][1] for i in chosen], dtype=torch.int32, device=DEV),
+                                     torch.tensor([rows[i][0] for i in chosen], dtype=torch.int32, device=DEV), table, group * kv_heads,
+                                     size ** -0.5, **options)
+            assert torch.equal(got.nan_to_num(7e7), many[1][chosen].nan_to_num(7e7)), chosen[:3]
