@@ -25,6 +25,9 @@
 // matrices (us a layer of 2,048 rows, before): gates, 4 heads of 256 x 512 165 (566); fixed decays with rotation, 4 heads of
 // 128 x 256 110 (250); a decay a channel, 16 heads of 128 x 128 241 (1034).
 //
+// A row's read-out holds nothing of the rows behind it, not even where those are infinite or not numbers, and a decay that is not
+// a number makes the memory none from its row on, as the recurrences do row by row.
+//
 // Products are v_mfma_f32_16x16x4_f32.  Lane l = 16 g + c holds A[row c][k-slot g], B[k-slot g][column c] and rows 4 g + v of
 // column c of the result in register v.  Which inner element a k-slot stands for is free as long as both operands agree:
 // instruction v of a run of 16 takes element 4 g + v for slot g, so that an operand is one 16-byte read a lane, and a result
@@ -209,10 +212,10 @@ __global__ void __launch_bounds__(kChunkThreads, 2) chunk_prepare_kernel(ChunkAr
                 strength[lane] = 1.0f / (1.0f + expf(-p.beta[row * p.beta_stride + head]));
             } else {
                 const float d = p.coef ? p.coef[2 * (row * p.heads + head)] : p.decay[head];
-                l = d > 0.f ? log(static_cast<double>(d)) : kNothingLeft;
+                l = d <= 0.f ? static_cast<double>(kNothingLeft) : log(static_cast<double>(d));
                 strength[lane] = p.coef ? p.coef[2 * (row * p.heads + head) + 1] : 1.f;
             }
-            l = fmax(l, static_cast<double>(kNothingLeft));
+            if (l < kNothingLeft) l = kNothingLeft;              // (a decay that is not a number stays one)
         } else {
             strength[lane] = 0.f;
         }
@@ -285,9 +288,10 @@ __global__ void __launch_bounds__(kChunkThreads, 2) chunk_prepare_kernel(ChunkAr
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
             const int t = 16 * ti + 4 * g + v;
-            const float decayed = t >= i ? between(cum[t], cum[i]) * k_norm[i] : 0.f;
-            if (block == 0) mix[4 * ((ti * 4 + tj) * kWave + 16 * (c / 4) + 4 * g + v) + c % 4] = decayed * q_norm[t] * qk[v];
-            if (kDelta) sa[256 * pair + 16 * (4 * g + v) + c] = -decayed * k_norm[t] * strength[t] * kk[v];
+            // (chosen and not multiplied by zero: what is not finite in a later row's key is none of an earlier row's)
+            const float decayed = between(cum[t], cum[i]) * k_norm[i];
+            if (block == 0) mix[4 * ((ti * 4 + tj) * kWave + 16 * (c / 4) + 4 * g + v) + c % 4] = t >= i ? decayed * q_norm[t] * qk[v] : 0.f;
+            if (kDelta) sa[256 * pair + 16 * (4 * g + v) + c] = t >= i ? -decayed * k_norm[t] * strength[t] * kk[v] : 0.f;
         }
     }
     float* q_in = p.q_in + at * kChunkRows * kDim;
@@ -594,28 +598,24 @@ __device__ inline void fetch_chunk(const ChunkArgs& p, int chunk, int head, int 
         for (int r = 0; r < 4; ++r) o.k[t][r] = k_out[(t * 4 + r) * kWave];
 }
 
+// What the walk shares over a workgroup.
+template <bool kDelta>
+struct WalkShared {
+    float part[kDelta ? 2 : 1][kChunkThreads / kWave][kChunkRows * kPartStride];
+    float u[kChunkRows * kPartStride];
+};
+
 // A workgroup walks the chunks of one portion for one head and 16 columns; wave w holds key channels 16 kT w .. of the columns
 // and makes what they give to every row of W S and Q S; the parts meet in shared memory, where wave w takes rows 16 w ..
-template <bool kDelta, int kT, bool kChannel>
-__global__ void __launch_bounds__(kChunkThreads, 1) chunk_walk_kernel(ChunkArgs p) {
+// Returns whether a read-out of this lane came out as no number.  Not kCareful: if only because M's zeros met an infinity or a
+// NaN of a later row, which is none of the row's; kCareful: such sums are made without the rows behind.
+template <bool kDelta, int kT, bool kChannel, bool kCareful>
+__device__ inline bool walk_chunks(const ChunkArgs& p, WalkShared<kDelta>& shared, int g0, int g1, int head, int wave, int c, int g, int col,
+                                   bool held, bool is_norm, floatx4 (&S)[kT]) {
     constexpr int kWaves = kChunkThreads / kWave;
-    __shared__ float part[kDelta ? 2 : 1][kWaves][kChunkRows * kPartStride];
-    __shared__ float su[kChunkRows * kPartStride];
-    const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave, c = lane & 15, g = lane >> 4;
-    const int link = blockIdx.x, head = blockIdx.y, col = 16 * blockIdx.z + c;
-    const int slot = p.links[4 * link], fresh = p.links[4 * link + 1], g0 = p.links[4 * link + 2], g1 = p.links[4 * link + 3];
-    float* state = p.state + slot * p.slot_stride + head * p.head_stride;
-    const bool is_norm = p.dot != nullptr && col == p.vdim, held = col < p.vdim || is_norm;
-    const auto place = [&](int i) { return is_norm ? static_cast<long>(p.dim) * p.vdim + i : static_cast<long>(i) * p.vdim + col; };
-    floatx4 S[kT];
-#pragma unroll
-    for (int t = 0; t < kT; ++t)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const int i = 16 * (wave * kT + t) + 4 * g + v;
-            S[t][v] = (!fresh && i < p.dim && held) ? state[place(i)] : 0.f;
-        }
-    if (g0 >= g1) return;
+    auto& part = shared.part;
+    float* su = shared.u;
+    bool odd = false;
     ChunkOperands<kDelta, kT, kChannel> ahead;
     fetch_chunk<kDelta, kT, kChannel>(p, g0, head, wave, c, g, col, ahead);
     for (int chunk = g0; chunk < g1; ++chunk) {
@@ -675,6 +675,7 @@ __global__ void __launch_bounds__(kChunkThreads, 1) chunk_walk_kernel(ChunkArgs 
 #pragma unroll
                 for (int t = 0; t < kT; ++t) wrote[t] = mfma4(element(now.k[t][s], v), u[s][v], wrote[t]);
             }
+        [[maybe_unused]] const floatx4 before = o;
         o += (mu[0] + mu[1]) + (mu[2] + mu[3]);
 #pragma unroll
         for (int t = 0; t < kT; ++t)
@@ -683,12 +684,61 @@ __global__ void __launch_bounds__(kChunkThreads, 1) chunk_walk_kernel(ChunkArgs 
                 if constexpr (kChannel) S[t][v] = fmaf(S[t][v], element(now.totals[t], v), wrote[t][v]);
                 else S[t][v] = fmaf(S[t][v], now.total, wrote[t][v]);
             }
+        const bool none = o[0] != o[0] || o[1] != o[1] || o[2] != o[2] || o[3] != o[3];
+        if constexpr (!kCareful) {
+            odd = odd || none;
+        } else if (__any(none)) {
+            // the same sums an element at a time, M from memory
+            const float* mix = p.mix + (static_cast<long>(chunk) * p.heads + head) * kChunkRows * kChunkRows + 16 * wave * kChunkRows;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                float sums[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int s = 0; s < 4; ++s)
+#pragma unroll 1
+                    for (int e = 0; e < 16; ++e) {
+                        const int i = 4 * (e % 4) + e / 4;                                // in the order of the instructions
+                        if (16 * s + i <= 16 * wave + 4 * g + v)
+                            sums[s] = fmaf(mix[4 * (s * kWave + 16 * (e % 4) + 4 * g + v) + e / 4], su[(16 * s + i) * kPartStride + c], sums[s]);
+                    }
+                o[v] = before[v] + ((sums[0] + sums[1]) + (sums[2] + sums[3]));
+            }
+        }
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
             const int t = 16 * wave + 4 * g + v;
             const long row_head = static_cast<long>(now.first + t) * p.heads + head;
             if (now.first + t < now.end && held) *(is_norm ? p.dot + row_head : p.out + row_head * p.vdim + col) = o[v];
         }
+    }
+    return odd;
+}
+
+template <bool kDelta, int kT, bool kChannel>
+__global__ void __launch_bounds__(kChunkThreads, 1) chunk_walk_kernel(ChunkArgs p) {
+    __shared__ WalkShared<kDelta> shared;
+    const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave, c = lane & 15, g = lane >> 4;
+    const int link = blockIdx.x, head = blockIdx.y, col = 16 * blockIdx.z + c;
+    const int slot = p.links[4 * link], fresh = p.links[4 * link + 1], g0 = p.links[4 * link + 2], g1 = p.links[4 * link + 3];
+    float* state = p.state + slot * p.slot_stride + head * p.head_stride;
+    const bool is_norm = p.dot != nullptr && col == p.vdim, held = col < p.vdim || is_norm;
+    const auto place = [&](int i) { return is_norm ? static_cast<long>(p.dim) * p.vdim + i : static_cast<long>(i) * p.vdim + col; };
+    floatx4 S[kT];
+    const auto load = [&]() {
+#pragma unroll
+        for (int t = 0; t < kT; ++t)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int i = 16 * (wave * kT + t) + 4 * g + v;
+                S[t][v] = (!fresh && i < p.dim && held) ? state[place(i)] : 0.f;
+            }
+    };
+    if (g0 >= g1) return;
+    load();
+    // (once more from the start where a read-out is no number: a look at every chunk within the walk cost it 4 %)
+    if (__syncthreads_or(walk_chunks<kDelta, kT, kChannel, false>(p, shared, g0, g1, head, wave, c, g, col, held, is_norm, S))) {
+        load();
+        walk_chunks<kDelta, kT, kChannel, true>(p, shared, g0, g1, head, wave, c, g, col, held, is_norm, S);
     }
     if (!p.write_state) return;
 #pragma unroll

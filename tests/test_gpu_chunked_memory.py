@@ -142,3 +142,56 @@ def test_a_decay_for_every_channel(kind, heads, kv_heads, dim, vdim, entries):
                 want.append(memory.T @ q[t] * dim ** -0.5)
             close(out[span, h], torch.stack(want), "out")
             close(dev_state[slot, h].cpu(), memory, "state")
+
+
+PLANTS = ["v inf", "v nan", "k nan", "q nan", "gate nan", "strength nan"]
+
+
+@pytest.mark.parametrize("at", [0, 15, 16, 37, 63, 64, 100, 129])
+@pytest.mark.parametrize("plant", PLANTS)
+@pytest.mark.parametrize("kind", ["gates", "fixed", "one", "channel"])
+def test_what_is_not_finite_reaches_no_row_before_it(kind, plant, at, monkeypatch):
+    """An infinity or a NaN in one row of a portion: the rows before it keep their bits, and from it on the same read-outs and
+    states are finite as when the rows are walked one by one."""
+    from leone_amd import ops
+    heads, dim, vdim = 2, 40, 24
+    gen = torch.Generator().manual_seed(5)
+    slots, step = step_of([(130, 3)])
+    rows, width = 130, heads * (2 * dim + vdim)
+    x = torch.randn(rows, width + 2 * heads, generator=gen)
+    beta, size = torch.randn(rows, heads, generator=gen), torch.randn(rows, heads * (dim if kind == "channel" else 1), generator=gen)
+    first = torch.randn(4, heads, dim * vdim + (dim + 1 if kind == "gates" else 0), generator=gen)
+
+    def run(spoilt):
+        rows_in, gate, strength, state = x.clone(), size.clone(), beta.clone(), first.to(DEV)
+        if spoilt:
+            value = math.inf if plant.endswith("inf") else math.nan
+            if plant[0] in "qkv":
+                rows_in[at, {"q": 0, "k": heads * dim, "v": 2 * heads * dim}[plant[0]] + 7] = value       # of head 0
+            elif plant == "gate nan":
+                gate[at, 0], rows_in[at, width + heads] = value, value
+            else:
+                strength[at, 0], rows_in[at, width] = value, value
+        columns = {"q": 0, "k": heads * dim, "v": 2 * heads * dim, "i": width, "f": width + heads}
+        if kind in ("one", "channel"):
+            state = state.view(4, heads, dim, vdim)
+            out = ops.delta_scan(rows_in.to(DEV), columns, strength.to(DEV), gate.to(DEV), torch.zeros(heads, device=DEV),
+                                 torch.zeros(gate.shape[1], device=DEV), state, step, heads, heads, dim, vdim, dim ** -0.5, 1e-6)
+            return out, state.reshape(4, -1), out
+        if kind == "gates":
+            bias = torch.zeros(2, heads, device=DEV)
+            out, under = ops.outer_scan(rows_in.to(DEV), columns, state, step, heads, dim, vdim, q_scale=dim ** -0.5,
+                                        gates={"i_bias": bias[0], "f_bias": bias[1], "cap": 15.0})
+            return out, state.view(4, -1), under[0]
+        cos, sin = ops.rope_table(1e4, 16, 300, DEV)
+        out, _ = ops.outer_scan(rows_in.to(DEV), columns, state, step, heads, dim, vdim, q_scale=dim ** -0.5, cos=cos, sin=sin,
+                                decay=torch.tensor([0.97, 0.9], device=DEV))
+        return out, state.view(4, -1), out
+
+    clean, spoilt = run(False), run(True)
+    monkeypatch.setattr(ops, "MEMORY_CHUNKS_FROM", 1 << 30)
+    walked = run(True)
+    for now, was, by_rows in zip(spoilt, clean, walked):
+        assert torch.equal(torch.isfinite(now), torch.isfinite(by_rows))
+    for i in (0, 2):
+        assert torch.equal(spoilt[i][:at], clean[i][:at])
