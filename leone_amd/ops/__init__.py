@@ -1593,7 +1593,13 @@ def scan_max_dim() -> int:
     return int(library().leone_scan_max_dim())
 
 
-MEMORY_CHUNKS_FROM = 32     # portions of at least so many rows go through a memory as ``chunked_memory``
+# Portions of at least so many rows go through a memory as ``chunked_memory``.  Alone and eight portions at a time (us, walked row by row and
+# in chunks): gates, 4 heads of 256 x 512, 32 rows 70 and 42, 73 and 68; 16 of 32 x 64 47 and 35; fixed decays with rotation, 4 of
+# 128 x 256, 60 and 25, 61 and 29; a decay a channel, 8 of 64 x 64, 34 and 34, 35 and 35, from 48 rows 48 and 36.
+MEMORY_CHUNKS_FROM = 32
+# With a decay for every channel and more than 64 of them a chunk takes longest to make: 16 heads of 128 x 128, alone and eight at a time,
+# 32 rows 44 and 54, 46 and 72; 48 rows 63 and 58, 64 and 76; 64 rows 82 and 61, 85 and 80.
+WIDE_CHANNEL_CHUNKS_FROM = 64
 
 
 def chunked_memory_supported(dim: int) -> bool:
@@ -1758,7 +1764,11 @@ def delta_scan(qkv: torch.Tensor, columns: dict, beta: torch.Tensor, step_size: 
 
     plan = None
     if chunked_memory_supported(dim) and dim <= library().leone_chunk_max_delta_dim():
-        plan = chunk_plan(step, library().leone_chunk_rows(), MEMORY_CHUNKS_FROM)
+        chunked_from = MEMORY_CHUNKS_FROM
+        # (the step's other memories' plan serves where no portion is in between)
+        if not per_head and dim > 64 and any(chunked_from <= e.count < WIDE_CHANNEL_CHUNKS_FROM for e in step.entries):
+            chunked_from = WIDE_CHANNEL_CHUNKS_FROM
+        plan = chunk_plan(step, library().leone_chunk_rows(), chunked_from)
         if plan is not None:
             chunked_memory(qkv, columns, plan, state, out, heads, kv_heads, dim, vdim, q_scale=q_scale, k_scale=1.0,
                            delta=(beta, step_size, rate_log, step_bias, unit_eps), write_state=write_state)

@@ -225,3 +225,18 @@ def test_chunks_are_as_exact_as_rows(dim, monkeypatch):
                                     gates={"i_bias": bias[0], "f_bias": bias[1], "cap": 15.0})
             off[how] += float((out.view(rows, heads, vdim).transpose(0, 1).to(F) - want).norm() / want.norm()) / 6
     assert off["rows"] < 4e-7 and off["chunks"] <= 1.02 * off["rows"], off
+
+
+@pytest.mark.parametrize("dim,from_rows", [(64, 32), (72, 64), (128, 64)])
+def test_where_channel_wise_portions_go_in_chunks(dim, from_rows, monkeypatch):
+    """Shorter portions are walked, which is faster there, and come out the same."""
+    from leone_amd import ops
+    seen, through = [], ops.chunked_memory
+    monkeypatch.setattr(ops, "chunked_memory", lambda *a, **b: (seen.append(1), through(*a, **b)))
+    for rows, chunked in ((from_rows - 1, False), (from_rows, True)):
+        x, beta, size = (torch.randn(rows, n, device=DEV) for n in (3 * dim, 1, dim))
+        state = torch.zeros(4, 1, dim, dim, device=DEV)
+        seen.clear()
+        ops.delta_scan(x, {"q": 0, "k": dim, "v": 2 * dim}, beta, size, torch.zeros(1, device=DEV), torch.zeros(dim, device=DEV), state,
+                       step_of([(rows, 0)])[1], 1, 1, dim, dim, dim ** -0.5, 1e-6)
+        assert bool(seen) == chunked
