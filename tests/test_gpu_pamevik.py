@@ -111,26 +111,79 @@ def test_engine_agrees_with_plain_however_the_work_is_cut(cases, name, dtype_nam
     assert all(engine.cache.free_pages(g) == engine.cache.groups[g].num_pages for g in range(len(engine.cache.groups)))
 
 
+@pytest.mark.parametrize("how", ["products", "walks"])
 @pytest.mark.parametrize("schedule", ["whole", "portions", "mixed"])
 @pytest.mark.parametrize("name", ["P", "Q", "R"])
-def test_long_portions_walked_in_chunks_side_by_side(cases, monkeypatch, name, schedule):
-    """A portion of many rows has its recurrences walked in chunks side by side instead of row by row; with the
-    chunks made 8 rows and every portion from 16 rows on cut so, these requests go through that path: chunks that
-    end in the middle of a portion, a last chunk of one row, long portions beside single tokens in one step, a
-    portion that continues a request.  The logits must not know."""
+def test_long_portions_in_chunks(cases, monkeypatch, name, schedule, how):
+    """A portion of many rows has its recurrences worked off in chunks instead of row by row.  With every portion from 16 rows on
+    treated so these requests go through that path: as products over chunks of 64 rows, or, the delta rule as its heads
+    of more key channels take it, in chunks of 8 rows walked side by side and chained by a matrix; chunks that end in the
+    middle of a portion, short last chunks, long portions beside single tokens in one step, a portion that continues
+    a request.  The logits must not know."""
     from leone_amd import ops
-    monkeypatch.setattr(ops, "OUTER_CHUNKS", (8, 16))
-    monkeypatch.setattr(ops, "DELTA_CHUNKS", (8, 16))
+    monkeypatch.setattr(ops, "MEMORY_CHUNKS_FROM", 16)
+    monkeypatch.setattr(ops, "WIDE_CHANNEL_CHUNKS_FROM", 16)
+    counts = {"products": 0, "walks": 0}
+    call, memory = ops.call, ops.chunked_memory
+    monkeypatch.setattr(ops, "chunked_memory", lambda *a, **b: (counts.update(products=counts["products"] + 1), memory(*a, **b)))
+    monkeypatch.setattr(ops, "call", lambda entry, *a: (counts.update(walks=counts["walks"] + (entry == "leone_delta_chain")), call(entry, *a))[1])
+    if how == "walks":
+        monkeypatch.setattr(ops, "chunked_memory_supported", lambda dim: False)
+        monkeypatch.setattr(ops, "DELTA_CHUNKS", (8, 16))
+    # chunks add up in another order than row by row; where a read-out is small against its parts a position comes out a few
+    # times further off than its neighbours (measured 5e-5 to 1e-4 at one position of model Q, means 3e-6 to 5e-6), so
+    # single positions get ten times the bound here and the mean keeps it
+    monkeypatch.setitem(OUTLIER, "float32", 10.0)
     folder, requests, expected = cases(name, "float32")
     steps = (SCHEDULES[schedule] if schedule != "portions" else
              (lambda r: schedules.portions(r, sizes=(17, 2, 33, 16, 40, 1, 25))))(requests)
     engine = make_engine(folder, "float32", max_tokens=schedules.max_live_tokens(steps, 16))
     outputs = run_steps(engine, steps)
-    # chained chunks add up in another order than row by row; where a read-out is small against its parts a
-    # position comes out a few times further off than its neighbours (measured 1e-4 at one position of one model,
-    # means 3e-6 to 5e-6), so single positions get ten times the bound here and the mean keeps it
-    monkeypatch.setitem(OUTLIER, "float32", 10.0)
-    compare(steps, outputs, expected, TOLERANCE["float32"], f"{name} chunked {schedule}")
+    compare(steps, outputs, expected, TOLERANCE["float32"], f"{name} {how} {schedule}")
+    assert counts[how] > 0 and counts["walks" if how == "products" else "products"] == 0, counts
+
+
+@pytest.mark.parametrize("heads,kv_heads,dim,vdim", [(2, 1, 136, 40), (1, 1, 200, 64), (2, 2, 256, 33)])
+@pytest.mark.parametrize("each", [True, False])
+def test_delta_rule_over_many_key_channels(each, heads, kv_heads, dim, vdim):
+    """More than 128 key channels: portions from 512 rows on are walked in chunks of 256 side by side, chained by the matrix that each
+    makes of a state, beside a short portion and one that starts a request; against the recurrence in double precision."""
+    from leone_amd import ops
+    from leone_amd.parts.context import EntryInfo, StepContext
+    dev, f64 = "cuda:0", torch.float64
+    entries = [(3, 530, 7), (0, 20, 0), (2, 700, 0)]                     # slot, rows, position
+    gen = torch.Generator().manual_seed(dim)
+    rows, kv = sum(n for _, n, _ in entries), kv_heads * dim
+    x = torch.randn(rows, 2 * kv + heads * vdim, generator=gen)
+    beta, size = torch.randn(rows, heads, generator=gen), torch.randn(rows, heads * (dim if each else 1), generator=gen)
+    rate_log, bias = torch.rand(heads, generator=gen) - 1.0, torch.rand(size.shape[1], generator=gen) * 3 - 4
+    state = torch.randn(4, heads, dim, vdim, generator=gen)
+    on = lambda values: torch.tensor(values, dtype=torch.int32, device=dev)
+    first = [sum(n for _, n, _ in entries[:i]) for i in range(len(entries))]
+    step = StepContext(rows=rows, dtype=torch.float32, device=torch.device(dev), positions=on([s + i for _, n, s in entries for i in range(n)]),
+                       row_entry=on([i for i, (_, n, _) in enumerate(entries) for _ in range(n)]),
+                       entries=[EntryInfo(f"r{i}", slot, at, n, start) for i, (at, (slot, n, start)) in enumerate(zip(first, entries))],
+                       entry_slots=on([slot for slot, _, _ in entries]), want_rows=None)
+    dev_state = state.to(dev)
+    out = ops.delta_scan(x.to(dev), {"q": 0, "k": kv, "v": 2 * kv}, beta.to(dev), size.to(dev), rate_log.to(dev), bias.to(dev), dev_state, step,
+                         heads, kv_heads, dim, vdim, dim ** -0.5, 1e-6).view(rows, heads, vdim).cpu().to(f64)
+    x = x.to(f64)
+    unit = lambda t: t / torch.sqrt((t * t).sum(-1, keepdim=True) + 1e-6)
+    q, k = (unit(x[:, b:b + kv].view(rows, kv_heads, dim)).repeat_interleave(heads // kv_heads, 1) for b in (0, kv))
+    v = x[:, 2 * kv:].view(rows, heads, vdim)
+    decay = torch.exp(-torch.exp(rate_log.to(f64))[:, None] * torch.nn.functional.softplus((size + bias).to(f64)).view(rows, heads, -1))
+    strength = torch.sigmoid(beta.to(f64))
+    for at, (slot, n, start) in zip(first, entries):
+        memory = state[slot].to(f64) if start else torch.zeros(heads, dim, vdim, dtype=f64)
+        want = []
+        for t in range(at, at + n):
+            memory = memory * decay[t][:, :, None]
+            u = strength[t][:, None] * (v[t] - torch.einsum("hd,hdv->hv", k[t], memory))
+            memory = memory + k[t][:, :, None] * u[:, None]
+            want.append(torch.einsum("hd,hdv->hv", q[t], memory) * dim ** -0.5)
+        # float sums of up to 256 products through up to 700 rows of a contracting recurrence: 2e-7 to 1e-6 of the norm; ten times that
+        for got, exact in ((out[at:at + n], torch.stack(want)), (dev_state[slot].cpu().to(f64), memory)):
+            assert float((got - exact).norm() / exact.norm()) < 1e-5
 
 
 @pytest.mark.parametrize("dtype_name", list(DTYPES))

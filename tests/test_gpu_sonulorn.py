@@ -67,14 +67,13 @@ def test_engine_agrees_with_plain_however_the_work_is_cut(cases, name, dtype_nam
 @pytest.mark.parametrize("schedule", ["whole", "portions", "mixed"])
 @pytest.mark.parametrize("name", ["A", "B"])
 def test_long_portions_of_the_memories_in_chunks(cases, monkeypatch, name, schedule, how):
-    """From portions of 16 rows on, the memories work in chunks: as products over chunks of 64 rows, or (what heads of more key
-    channels take) in chunks of 8 rows walked side by side and chained, by a factor for the fixed decays and by a matrix for
-    the delta rule.  The results differ by rounding only."""
+    """From portions of 16 rows on, the memories work in chunks: as products over chunks of 64 rows, or (what the delta rule over more
+    key channels takes) in chunks of 8 rows walked side by side and chained by a matrix, the fixed decays then row by row.  The
+    results differ by rounding only."""
     from leone_amd import ops
     monkeypatch.setattr(ops, "MEMORY_CHUNKS_FROM", 16)
     if how == "walks":
         monkeypatch.setattr(ops, "chunked_memory_supported", lambda dim: False)
-        monkeypatch.setattr(ops, "OUTER_CHUNKS", (8, 16))
         monkeypatch.setattr(ops, "DELTA_CHUNKS", (8, 16))
     folder, requests, expected = cases(name, "float32")
     steps = SCHEDULES[schedule](requests)
