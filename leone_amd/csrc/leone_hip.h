@@ -263,36 +263,33 @@ int leone_scan_max_dim();
 int leone_exp_gates(const float* proj, long stride, int i_off, int f_off, const void* i_bias, const void* f_bias,
                     int bias_dtype, float cap, const int* spans, int entries, float* state, long slot_stride,
                     long head_stride, long top_at, int write_state, float* coef, float* top, int heads, hipStream_t stream);
-int leone_outer_scan(const float* proj, long stride, int q_off, int k_off, int v_off, const float* coef,
-                     const float* decay, int no_input, int accumulate, int norm_column, float q_scale, float k_scale, int silu,
-                     const float* cos_table, const float* sin_table, int rotary_dim, int table_positions,
-                     const int* positions, const int* segments, int n_segments, const float* state_in, long in_stride,
-                     float* state_out, long out_stride, long head_stride, float* decay_product, float* out, float* dot,
-                     int heads, int dim, int vdim, hipStream_t stream);
+int leone_outer_scan(const float* proj, long stride, int q_off, int k_off, int v_off, const float* coef, const float* decay,
+                     int norm_column, float q_scale, float k_scale, int silu, const float* cos_table,
+                     const float* sin_table, int rotary_dim, int table_positions, const int* positions,
+                     const int* segments, int n_segments, const float* state_in, long in_stride, float* state_out,
+                     long out_stride, long head_stride, float* out, float* dot, int heads, int dim, int vdim,
+                     hipStream_t stream);
 // Whether heads of such sizes are taken by leone_outer_step and leone_delta_step.
 int leone_step_fits(int dim, int vdim);
-// leone_outer_scan where every segment is a single row (no_input and accumulate 0, no decay_product).
-int leone_outer_step(const float* proj, long stride, int q_off, int k_off, int v_off, const float* coef,
-                     const float* decay, int no_input, int accumulate, int norm_column, float q_scale, float k_scale, int silu,
-                     const float* cos_table, const float* sin_table, int rotary_dim, int table_positions,
-                     const int* positions, const int* segments, int n_segments, const float* state_in, long in_stride,
-                     float* state_out, long out_stride, long head_stride, float* decay_product, float* out, float* dot,
-                     int heads, int dim, int vdim, hipStream_t stream);
-int leone_outer_chain(const int* links, int n_links, float* work, long work_stride, const float* product, float* state,
-                      long slot_stride, long head_stride, int per_head, int heads, int write_state, hipStream_t stream);
+// leone_outer_scan where every segment is a single row.
+int leone_outer_step(const float* proj, long stride, int q_off, int k_off, int v_off, const float* coef, const float* decay,
+                     int norm_column, float q_scale, float k_scale, int silu, const float* cos_table,
+                     const float* sin_table, int rotary_dim, int table_positions, const int* positions,
+                     const int* segments, int n_segments, const float* state_in, long in_stride, float* state_out,
+                     long out_stride, long head_stride, float* out, float* dot, int heads, int dim, int vdim,
+                     hipStream_t stream);
 int leone_delta_scan(const float* qkv, long stride, int q_off, int k_off, int v_off, const float* beta,
                      long beta_stride, const float* step, long step_stride, int per_head, const void* rate_log,
                      const void* step_bias, int vec_dtype, float q_scale, float unit_eps, int no_input, int accumulate,
                      const int* segments, int n_segments, const float* state_in, long in_stride, float* state_out,
                      long out_stride, float* transition, float* out, int heads, int kv_heads, int dim, int vdim,
                      hipStream_t stream);
-// leone_delta_scan where every segment is a single row (no_input and accumulate 0, no transition).
+// leone_delta_scan where every segment is a single row.
 int leone_delta_step(const float* qkv, long stride, int q_off, int k_off, int v_off, const float* beta,
                      long beta_stride, const float* step, long step_stride, int per_head, const void* rate_log,
-                     const void* step_bias, int vec_dtype, float q_scale, float unit_eps, int no_input, int accumulate,
-                     const int* segments, int n_segments, const float* state_in, long in_stride, float* state_out,
-                     long out_stride, float* transition, float* out, int heads, int kv_heads, int dim, int vdim,
-                     hipStream_t stream);
+                     const void* step_bias, int vec_dtype, float q_scale, float unit_eps, const int* segments,
+                     int n_segments, const float* state_in, long in_stride, float* state_out, long out_stride,
+                     float* out, int heads, int kv_heads, int dim, int vdim, hipStream_t stream);
 int leone_delta_chain(const int* links, int n_links, float* work, long work_stride, const float* transition, float* state,
                       long slot_stride, int heads, int dim, int vdim, int write_state, hipStream_t stream);
 

@@ -35,9 +35,10 @@ inline int lane_groups(int dim) { return dim <= 32 ? 1 : dim <= 64 ? 2 : dim <= 
 // A segment is a run of consecutive rows of one request that one wave walks in order: rows [first, end), the
 // state it starts from (index `in` into the launch's input states, negative: zeros) and where the state it ends
 // with goes (index `out` into the launch's output states, negative: nowhere).  A decoded token or a short portion
-// is one segment from and into the request's state slot.  A long portion is cut into chunks that are walked side
+// is one segment from and into the request's state slot; long portions go through chunked_memory.hip.  What that does not take,
+// the delta rule over more than 128 key channels, is cut into chunks that are walked side
 // by side, three launches instead of one: every chunk from zeros (what the chunk's own rows write, and what they
-// read of it), then the chunks' end states chained into the state each chunk starts from (outer_chain), then every
+// read of it), then the chunks' end states chained into the state each chunk starts from (delta_chain), then every
 // chunk once more from that state with nothing written into it (`no_input`), added to the first walk's read-outs.
 struct Segment {
     int first, end, in, out;
@@ -49,8 +50,6 @@ struct OuterScanArgs {
     int q_off, k_off, v_off;    // columns of head 0; head h of q and k at + h * dim, of v at + h * vdim
     const float* coef;          // [rows, heads, 2]: a_t and b_t, or null: a = decay[head], b = 1
     const float* decay;         // [heads]
-    int no_input;               // b is taken as 0: the state is only carried through the rows and read
-    int accumulate;             // read-outs are added to what out and dot hold
     int norm_column;            // one more column whose value is always 1 (the normaliser), read out into dot
     float q_scale, k_scale;
     int silu;                   // q, k and v pass through silu first
@@ -64,7 +63,6 @@ struct OuterScanArgs {
     float* state_out;
     long out_stride;
     long head_stride;           // floats from head to head in a state: S [dim, vdim], then the normaliser [dim]
-    float* decay_product;       // [segments, heads]: the product of a_t over the segment's rows, or null
     float* out;                 // [rows, heads, vdim]
     float* dot;                 // [rows, heads]
     int heads, dim, vdim;
@@ -177,7 +175,6 @@ __global__ void __launch_bounds__(kScanThreads) outer_scan_kernel(OuterScanArgs 
         }
     }
     const float fixed = p.coef ? 0.f : p.decay[head];
-    float carried = 1.f;                                      // the product of the segment's decays
 
     for (int t0 = 0; t0 < n; t0 += kScanTokens) {
         const int here = min(kScanTokens, n - t0);
@@ -191,7 +188,7 @@ __global__ void __launch_bounds__(kScanThreads) outer_scan_kernel(OuterScanArgs 
                 const float* s = p.cos_table ? p.sin_table + static_cast<long>(pos) * p.rot_half : nullptr;
                 const float* base = p.proj + row * p.stride;
                 qv = rotated(base + p.q_off + head * p.dim, i, p.silu, c, s, p.rot_half) * p.q_scale;
-                if (!p.no_input) kv = rotated(base + p.k_off + head * p.dim, i, p.silu, c, s, p.rot_half) * p.k_scale;
+                kv = rotated(base + p.k_off + head * p.dim, i, p.silu, c, s, p.rot_half) * p.k_scale;
             }
             sq[idx] = qv;
             sk[idx] = kv;
@@ -199,7 +196,7 @@ __global__ void __launch_bounds__(kScanThreads) outer_scan_kernel(OuterScanArgs 
         if (tid < here) {
             const long at = static_cast<long>(first + t0 + tid) * p.heads + head;
             sa[tid] = p.coef ? p.coef[2 * at] : fixed;
-            sb[tid] = p.no_input ? 0.f : (p.coef ? p.coef[2 * at + 1] : 1.f);
+            sb[tid] = p.coef ? p.coef[2 * at + 1] : 1.f;
         }
         __syncthreads();
         if (col[0] < cols) {                                   // the lanes of a column are in or out together
@@ -208,52 +205,34 @@ __global__ void __launch_bounds__(kScanThreads) outer_scan_kernel(OuterScanArgs 
                 const float a = sa[t];
                 const float* kt = sk + t * dkp + ch0;
                 const float* qt = sq + t * dkp + ch0;
-                float acc[kLaneCols];
-                if (p.no_input) {                              // nothing is written: the state decays and is read
+                float acc[kLaneCols], bv[kLaneCols];
 #pragma unroll
-                    for (int c = 0; c < kLaneCols; ++c) acc[c] = 0.f;
+                for (int c = 0; c < kLaneCols; ++c) {
+                    const float v = is_value[c] ? silu_if(p.proj[row * p.stride + p.v_off + head * p.vdim + col[c]], p.silu) : 1.f;
+                    bv[c] = sb[t] * v;
+                    acc[c] = 0.f;
+                }
 #pragma unroll
-                    for (int i = 0; i < kLaneRows; ++i) {
-                        const float q = qt[i];
-#pragma unroll
-                        for (int c = 0; c < kLaneCols; ++c) {
-                            S[c][i] *= a;
-                            acc[c] = fmaf(S[c][i], q, acc[c]);
-                        }
-                    }
-                } else {
-                    float bv[kLaneCols];
+                for (int i = 0; i < kLaneRows; ++i) {
+                    const float k = kt[i], q = qt[i];
 #pragma unroll
                     for (int c = 0; c < kLaneCols; ++c) {
-                        const float v = is_value[c] ? silu_if(p.proj[row * p.stride + p.v_off + head * p.vdim + col[c]], p.silu) : 1.f;
-                        bv[c] = sb[t] * v;
-                        acc[c] = 0.f;
-                    }
-#pragma unroll
-                    for (int i = 0; i < kLaneRows; ++i) {
-                        const float k = kt[i], q = qt[i];
-#pragma unroll
-                        for (int c = 0; c < kLaneCols; ++c) {
-                            S[c][i] = fmaf(a, S[c][i], k * bv[c]);
-                            acc[c] = fmaf(S[c][i], q, acc[c]);
-                        }
+                        S[c][i] = fmaf(a, S[c][i], k * bv[c]);
+                        acc[c] = fmaf(S[c][i], q, acc[c]);
                     }
                 }
-                carried *= a;
 #pragma unroll
                 for (int c = 0; c < kLaneCols; ++c) {
                     for (int off = per_wave; off < kWave; off <<= 1) acc[c] += __shfl_xor(acc[c], off, kWave);
                     if (part == 0 && col[c] < cols) {
                         const long at = row * p.heads + head;
-                        float* dst = is_value[c] ? p.out + at * p.vdim + col[c] : p.dot + at;
-                        *dst = p.accumulate ? *dst + acc[c] : acc[c];
+                        *(is_value[c] ? p.out + at * p.vdim + col[c] : p.dot + at) = acc[c];
                     }
                 }
             }
         }
         __syncthreads();
     }
-    if (p.decay_product && blockIdx.z == 0 && tid == 0) p.decay_product[static_cast<long>(blockIdx.x) * p.heads + head] = carried;
     if (!p.state_out || seg.out < 0) return;
     float* to = p.state_out + seg.out * p.out_stride + head * p.head_stride;
 #pragma unroll
@@ -389,28 +368,6 @@ __global__ void __launch_bounds__(kGroups * kWave) outer_step_kernel(OuterScanAr
     for (int i = 0; i < kLaneRows; ++i)
         if (col < p.vdim) float_at(into, (ch0 + i) * row_bytes, 4u * ccol) = S[i];
     if (norm && lane < kLaneRows) into[static_cast<long>(p.dim) * p.vdim + ch] = N;
-}
-
-// The chunks' end states chained: for a long portion whose chunks are [g0, g1) of `work` (each holding what its
-// own rows wrote, from zeros), S = the request's state (zeros at a sequence's start); for every chunk in order:
-// what the chunk holds is replaced by S (the state it starts from), and S <- product[chunk] * S + what it held.
-// The last S is the request's new state.  links[l] = (slot, fresh, g0, g1).
-__global__ void outer_chain_kernel(const int* __restrict__ links, float* __restrict__ work, long work_stride,
-                                   const float* __restrict__ product, float* __restrict__ state, long slot_stride,
-                                   long head_stride, int per_head, int heads, int write_state) {
-    const int l = blockIdx.x, head = blockIdx.y;
-    const int el = blockIdx.z * blockDim.x + threadIdx.x;
-    if (el >= per_head) return;
-    const int slot = links[4 * l], fresh = links[4 * l + 1], g0 = links[4 * l + 2], g1 = links[4 * l + 3];
-    float* mine = state + slot * slot_stride + head * head_stride + el;
-    float S = fresh ? 0.f : *mine;
-    for (int g = g0; g < g1; ++g) {
-        float* at = work + g * work_stride + head * head_stride + el;
-        const float wrote = *at;
-        *at = S;
-        S = fmaf(product[static_cast<long>(g) * heads + head], S, wrote);
-    }
-    if (write_state) *mine = S;
 }
 
 struct DeltaScanArgs {
@@ -641,9 +598,10 @@ __global__ void __launch_bounds__(kGroups * kWave) delta_step_kernel(DeltaScanAr
         float_at(to, (ch0 + i) * row_bytes, 4u * ccol) = S[i];
 }
 
-// The chunks of a long portion chained for the delta rule: a chunk's rows turn a state S that comes in into
-// transition[chunk] . S + (what the chunk holds: its end state from zeros).  As in outer_chain_kernel every chunk's
-// place in `work` ends up holding the state the chunk starts from, and the last state is the request's new one.
+// The chunks of a long portion chained for the delta rule, its chunks [g0, g1) of `work`: a chunk's rows turn a state S that comes
+// in into transition[chunk] . S + (what the chunk holds: its end state from zeros).  From the request's state on (zeros at a
+// sequence's start) every chunk's place in `work` ends up holding the state the chunk starts from, and the last state is the
+// request's new one.  links[l] = (slot, fresh, g0, g1).
 // A workgroup owns a run of columns of one head; a column's channels are spread over lanes as in the scans, and
 // the whole column passes through shared memory so that every lane sees all of it.
 __global__ void __launch_bounds__(kScanThreads)
@@ -733,12 +691,11 @@ extern "C" int leone_step_fits(int dim, int vdim) {
 }
 
 static int run_outer_scan(bool single, const float* proj, long stride, int q_off, int k_off, int v_off, const float* coef,
-                                const float* decay, int no_input, int accumulate, int norm_column, float q_scale,
-                                float k_scale, int silu, const float* cos_table, const float* sin_table, int rotary_dim,
-                                int table_positions, const int* positions, const int* segments, int n_segments,
-                                const float* state_in, long in_stride, float* state_out, long out_stride, long head_stride,
-                                float* decay_product, float* out, float* dot, int heads, int dim, int vdim,
-                                hipStream_t stream) {
+                                const float* decay, int norm_column, float q_scale, float k_scale, int silu,
+                                const float* cos_table, const float* sin_table, int rotary_dim, int table_positions,
+                                const int* positions, const int* segments, int n_segments, const float* state_in,
+                                long in_stride, float* state_out, long out_stride, long head_stride, float* out, float* dot,
+                                int heads, int dim, int vdim, hipStream_t stream) {
     LEONE_REQUIRE(proj && positions && segments && out, "outer_scan: null pointer");
     LEONE_REQUIRE(n_segments > 0 && heads > 0 && heads <= 65535 && dim > 0 && vdim > 0, "outer_scan: %d segments, %d heads of %d x %d",
                   n_segments, heads, dim, vdim);
@@ -753,18 +710,16 @@ static int run_outer_scan(bool single, const float* proj, long stride, int q_off
                   (!state_out || out_stride >= heads * head_stride), "outer_scan: states of %ld floats a head do not fit", head_stride);
     LEONE_REQUIRE(stride >= q_off + heads * dim && stride >= k_off + heads * dim && stride >= v_off + heads * vdim &&
                   q_off >= 0 && k_off >= 0 && v_off >= 0, "outer_scan: the projection's rows of %ld do not hold the named columns", stride);
-    OuterScanArgs a{proj, stride, q_off, k_off, v_off, coef, decay, no_input, accumulate, norm_column, q_scale, k_scale,
+    OuterScanArgs a{proj, stride, q_off, k_off, v_off, coef, decay, norm_column, q_scale, k_scale,
                     silu, cos_table, sin_table, cos_table ? rotary_dim / 2 : 0, cos_table ? table_positions : 1, positions,
                     reinterpret_cast<const Segment*>(segments), state_in, in_stride, state_out, out_stride, head_stride,
-                    decay_product, out, dot, heads, dim, vdim};
+                    out, dot, heads, dim, vdim};
     const int groups = lane_groups(dim);
     const int per_block = (kScanThreads / kWave) * (kWave / groups) * kLaneCols;          // columns a workgroup
     const dim3 grid(n_segments, heads, ceil_div(vdim + (norm_column ? 1 : 0), per_block));
     const size_t shared = (2 * kScanTokens * groups * kLaneRows + 2 * kScanTokens) * sizeof(float);
     if (single) {
-        LEONE_REQUIRE(leone_step_fits(dim, vdim) && !no_input && !accumulate && !decay_product,
-                      "outer_step: single rows write their read-outs and nothing else, of heads of 32, 64, 128 or 256 key channels (not %d x %d)",
-                      dim, vdim);
+        LEONE_REQUIRE(leone_step_fits(dim, vdim), "outer_step: heads have 32, 64, 128 or 256 key channels (not %d x %d)", dim, vdim);
         const dim3 columns(n_segments, heads, ceil_div(vdim, kWave));
         if (groups == 1) outer_step_kernel<1><<<columns, kWave, 0, stream>>>(a);
         else if (groups == 2) outer_step_kernel<2><<<columns, 2 * kWave, 0, stream>>>(a);
@@ -779,41 +734,26 @@ static int run_outer_scan(bool single, const float* proj, long stride, int q_off
 }
 
 extern "C" int leone_outer_scan(const float* proj, long stride, int q_off, int k_off, int v_off, const float* coef,
-                                const float* decay, int no_input, int accumulate, int norm_column, float q_scale,
-                                float k_scale, int silu, const float* cos_table, const float* sin_table, int rotary_dim,
-                                int table_positions, const int* positions, const int* segments, int n_segments,
-                                const float* state_in, long in_stride, float* state_out, long out_stride, long head_stride,
-                                float* decay_product, float* out, float* dot, int heads, int dim, int vdim,
-                                hipStream_t stream) {
-    return run_outer_scan(false, proj, stride, q_off, k_off, v_off, coef, decay, no_input, accumulate, norm_column,
-        q_scale, k_scale, silu, cos_table, sin_table, rotary_dim, table_positions, positions, segments, n_segments,
-        state_in, in_stride, state_out, out_stride, head_stride, decay_product, out, dot, heads, dim, vdim, stream);
+                                const float* decay, int norm_column, float q_scale, float k_scale, int silu,
+                                const float* cos_table, const float* sin_table, int rotary_dim, int table_positions,
+                                const int* positions, const int* segments, int n_segments, const float* state_in,
+                                long in_stride, float* state_out, long out_stride, long head_stride, float* out, float* dot,
+                                int heads, int dim, int vdim, hipStream_t stream) {
+    return run_outer_scan(false, proj, stride, q_off, k_off, v_off, coef, decay, norm_column, q_scale, k_scale, silu, cos_table,
+        sin_table, rotary_dim, table_positions, positions, segments, n_segments, state_in, in_stride, state_out, out_stride,
+        head_stride, out, dot, heads, dim, vdim, stream);
 }
 
 // leone_outer_scan where every segment is a single row.
 extern "C" int leone_outer_step(const float* proj, long stride, int q_off, int k_off, int v_off, const float* coef,
-                                const float* decay, int no_input, int accumulate, int norm_column, float q_scale,
-                                float k_scale, int silu, const float* cos_table, const float* sin_table, int rotary_dim,
-                                int table_positions, const int* positions, const int* segments, int n_segments,
-                                const float* state_in, long in_stride, float* state_out, long out_stride, long head_stride,
-                                float* decay_product, float* out, float* dot, int heads, int dim, int vdim,
-                                hipStream_t stream) {
-    return run_outer_scan(true, proj, stride, q_off, k_off, v_off, coef, decay, no_input, accumulate, norm_column,
-        q_scale, k_scale, silu, cos_table, sin_table, rotary_dim, table_positions, positions, segments, n_segments,
-        state_in, in_stride, state_out, out_stride, head_stride, decay_product, out, dot, heads, dim, vdim, stream);
-}
-
-extern "C" int leone_outer_chain(const int* links, int n_links, float* work, long work_stride, const float* product,
-                                 float* state, long slot_stride, long head_stride, int per_head, int heads, int write_state,
-                                 hipStream_t stream) {
-    LEONE_REQUIRE(links && work && product && state && n_links > 0 && heads > 0 && heads <= 65535 && per_head > 0,
-                  "outer_chain: null pointer or empty sizes");
-    LEONE_REQUIRE(head_stride >= per_head && work_stride >= heads * head_stride && slot_stride >= heads * head_stride &&
-                  ceil_div(per_head, 256) <= 65535, "outer_chain: states of %ld floats a head do not fit", head_stride);
-    outer_chain_kernel<<<dim3(n_links, heads, ceil_div(per_head, 256)), 256, 0, stream>>>(
-        links, work, work_stride, product, state, slot_stride, head_stride, per_head, heads, write_state);
-    LEONE_LAUNCH_CHECK("outer_chain");
-    return 0;
+                                const float* decay, int norm_column, float q_scale, float k_scale, int silu,
+                                const float* cos_table, const float* sin_table, int rotary_dim, int table_positions,
+                                const int* positions, const int* segments, int n_segments, const float* state_in,
+                                long in_stride, float* state_out, long out_stride, long head_stride, float* out, float* dot,
+                                int heads, int dim, int vdim, hipStream_t stream) {
+    return run_outer_scan(true, proj, stride, q_off, k_off, v_off, coef, decay, norm_column, q_scale, k_scale, silu, cos_table,
+        sin_table, rotary_dim, table_positions, positions, segments, n_segments, state_in, in_stride, state_out, out_stride,
+        head_stride, out, dot, heads, dim, vdim, stream);
 }
 
 static int run_delta_scan(bool single, const float* qkv, long stride, int q_off, int k_off, int v_off, const float* beta,
@@ -841,9 +781,7 @@ static int run_delta_scan(bool single, const float* qkv, long stride, int q_off,
     const dim3 grid(n_segments, heads, ceil_div(vdim + (transition ? dim : 0), (kScanThreads / kWave) * (kWave / groups)));
     const size_t shared = (3 * kScanTokens * groups * kLaneRows + kScanTokens) * sizeof(float);
     if (single) {
-        LEONE_REQUIRE(leone_step_fits(dim, vdim) && !no_input && !accumulate && !transition,
-                      "delta_step: single rows write their read-outs and nothing else, of heads of 32, 64, 128 or 256 key channels (not %d x %d)",
-                      dim, vdim);
+        LEONE_REQUIRE(leone_step_fits(dim, vdim), "delta_step: heads have 32, 64, 128 or 256 key channels (not %d x %d)", dim, vdim);
         const dim3 columns(n_segments, heads, ceil_div(vdim, kWave));
         if (groups == 1) delta_step_kernel<1><<<columns, kWave, 0, stream>>>(a);
         else if (groups == 2) delta_step_kernel<2><<<columns, 2 * kWave, 0, stream>>>(a);
@@ -871,13 +809,12 @@ extern "C" int leone_delta_scan(const float* qkv, long stride, int q_off, int k_
 // leone_delta_scan where every segment is a single row.
 extern "C" int leone_delta_step(const float* qkv, long stride, int q_off, int k_off, int v_off, const float* beta,
                                 long beta_stride, const float* step, long step_stride, int per_head, const void* rate_log,
-                                const void* step_bias, int vec_dtype, float q_scale, float unit_eps, int no_input,
-                                int accumulate, const int* segments, int n_segments, const float* state_in, long in_stride,
-                                float* state_out, long out_stride, float* transition, float* out, int heads, int kv_heads,
-                                int dim, int vdim, hipStream_t stream) {
+                                const void* step_bias, int vec_dtype, float q_scale, float unit_eps, const int* segments,
+                                int n_segments, const float* state_in, long in_stride, float* state_out, long out_stride,
+                                float* out, int heads, int kv_heads, int dim, int vdim, hipStream_t stream) {
     return run_delta_scan(true, qkv, stride, q_off, k_off, v_off, beta, beta_stride, step, step_stride, per_head,
-        rate_log, step_bias, vec_dtype, q_scale, unit_eps, no_input, accumulate, segments, n_segments, state_in,
-        in_stride, state_out, out_stride, transition, out, heads, kv_heads, dim, vdim, stream);
+        rate_log, step_bias, vec_dtype, q_scale, unit_eps, 0, 0, segments, n_segments, state_in,
+        in_stride, state_out, out_stride, nullptr, out, heads, kv_heads, dim, vdim, stream);
 }
 
 extern "C" int leone_delta_chain(const int* links, int n_links, float* work, long work_stride, const float* transition,

@@ -1408,15 +1408,13 @@ def entry_spans(step) -> torch.Tensor:
     return spans
 
 
-# Rows of a chunk when a long portion's recurrence is walked chunk by chunk, side by side, and the portions that
-# are (at least so many rows): (chunk, from).  The outer-product recurrences chain their chunks by a factor, the
-# delta rule by a matrix product a chunk, so its chunks are longer.
-OUTER_CHUNKS = (64, 256)
+# Rows of a chunk when a long portion of the delta rule over more than 128 key channels is walked chunk by chunk, side by side, and
+# the portions that are (at least so many rows): (chunk, from).  The chunks are chained by a matrix product each.
 DELTA_CHUNKS = (256, 512)
 
 
 def chunk_plan(step, chunk: int, chunked_from: int):
-    """How the recurrences of a step with long portions are walked (``outer_scan``): None if the step has none (or
+    """How the recurrences of a step with long portions are cut into chunks: None if the step has none (or
     is replayed from a recording: then the host does not know its entries).  Else int32 tables on the device:
     ``chunks`` ``[c, 4]`` (first row, end, -1, chunk index) of the long portions' chunks, ``again`` the same chunks
     reading (chunk index, -1), ``links`` ``[l, 4]`` (state slot, whether the sequence starts here, first chunk, end)
@@ -1654,9 +1652,7 @@ def outer_scan(proj: torch.Tensor, columns: dict, state: torch.Tensor, step, hea
     pass through it first.
     Returns o float32 ``[rows, heads * vdim]`` and, with gates, (dot, top) for ``head_norm_gate``.
 
-    Single tokens and short portions are walked row by row.  A long portion goes through as ``chunked_memory``; where that
-    does not take the size (``OUTER_CHUNKS``) it is cut into chunks that are walked side by side: every chunk from zeros, the
-    chunks' end states chained, every chunk once more from the state it starts with."""
+    Single tokens and short portions are walked row by row, a long portion goes through as ``chunked_memory``."""
     rows, width = proj.shape
     per_head = dim * vdim + (dim + 1 if gates else 0)
     if state.dtype != torch.float32 or state.dim() != 3 or tuple(state.shape[1:]) != (heads, per_head) or not state.is_contiguous():
@@ -1680,46 +1676,28 @@ def outer_scan(proj: torch.Tensor, columns: dict, state: torch.Tensor, step, hea
              _dev(coef, "coefficients"), _dev(top, "top"), heads, _stream())
     rotary_dim = 2 * cos.shape[1] if cos is not None else 0
 
-    def walk(segments, state_in, state_out, no_input=False, accumulate=False, product=None):
-        # every entry with a single row: the kernel that is made for it, if it takes the size (no chunks are walked then);
-        # eight rows of four heads of 256 x 512: 18.3 us walked, 9.6 in that kernel
-        single = segments.shape[0] == rows and not accumulate and product is None and library().leone_step_fits(dim, vdim)
+    def walk(segments):
+        # every entry with a single row: the kernel that is made for it, if it takes the size; eight rows of four heads of
+        # 256 x 512: 18.3 us walked, 9.6 in that kernel
+        single = segments.shape[0] == rows and library().leone_step_fits(dim, vdim)
         call("leone_outer_step" if single else "leone_outer_scan", _dev(proj, "projection", torch.float32), width, columns["q"], columns["k"], columns["v"],
              _dev(coef, "coefficients"), _dev(decay, "decay", torch.float32, (heads,)) if decay is not None else 0,
-             1 if no_input else 0, 1 if accumulate else 0, 1 if gates else 0, float(q_scale), float(k_scale),
-             1 if activation == "silu" else 0,
+             1 if gates else 0, float(q_scale), float(k_scale), 1 if activation == "silu" else 0,
              _dev(cos, "rope cos", torch.float32), _dev(sin, "rope sin", torch.float32), rotary_dim,
              cos.shape[0] if cos is not None else 0, _dev(step.positions, "positions", torch.int32, (rows,)),
-             _dev(segments, "segments", torch.int32), segments.shape[0],
-             _dev(state_in, "state read"), state_in.stride(0) if state_in is not None else 0,
-             _dev(state_out, "state written"), state_out.stride(0) if state_out is not None else 0, per_head,
-             _dev(product, "decay products"), _dev(out, "out"), _dev(dot, "dot"), heads, dim, vdim, _stream())
+             _dev(segments, "segments", torch.int32), segments.shape[0], _dev(state, "state read"), state.stride(0),
+             _dev(state if write_state else None, "state written"), state.stride(0) if write_state else 0, per_head,
+             _dev(out, "out"), _dev(dot, "dot"), heads, dim, vdim, _stream())
 
-    plan = None
-    if chunked_memory_supported(dim):
-        plan = chunk_plan(step, library().leone_chunk_rows(), MEMORY_CHUNKS_FROM)
-        if plan is not None:
-            chunked_memory(proj, columns, plan, state, out, heads, heads, dim, vdim, q_scale=q_scale, k_scale=k_scale,
-                           activation=activation, decay=decay, gates=(coef, dot) if gates else None,
-                           rotation=(cos, sin, step.positions) if cos is not None else None, write_state=write_state)
-            if plan["short"].shape[0]:
-                walk(plan["short"], state, state if write_state else None)
-            return (out, (dot, top)) if gates else (out, None)
-    else:
-        plan = chunk_plan(step, *OUTER_CHUNKS)
+    plan = chunk_plan(step, library().leone_chunk_rows(), MEMORY_CHUNKS_FROM) if chunked_memory_supported(dim) else None
     if plan is None:
-        walk(spans, state, state if write_state else None)
+        walk(spans)
     else:
-        chunks = plan["chunks"]
-        work = torch.empty((chunks.shape[0], heads, per_head), dtype=torch.float32, device=device)
-        product = torch.empty((chunks.shape[0], heads), dtype=torch.float32, device=device)
-        walk(chunks, None, work, product=product)
-        call("leone_outer_chain", _dev(plan["links"], "links", torch.int32), plan["links"].shape[0], _dev(work, "work"),
-             work.stride(0), _dev(product, "decay products"), _dev(state, "state"), state.stride(0), per_head,
-             dim * vdim + (dim if gates else 0), heads, 1 if write_state else 0, _stream())
-        walk(plan["again"], work, None, no_input=True, accumulate=True)
+        chunked_memory(proj, columns, plan, state, out, heads, heads, dim, vdim, q_scale=q_scale, k_scale=k_scale,
+                       activation=activation, decay=decay, gates=(coef, dot) if gates else None,
+                       rotation=(cos, sin, step.positions) if cos is not None else None, write_state=write_state)
         if plan["short"].shape[0]:
-            walk(plan["short"], state, state if write_state else None)
+            walk(plan["short"])
     return (out, (dot, top)) if gates else (out, None)
 
 
@@ -1735,9 +1713,9 @@ def delta_scan(qkv: torch.Tensor, columns: dict, beta: torch.Tensor, step_size: 
     ``[slots, heads, dim, vdim]``.  Returns o float32 ``[rows, heads * vdim]``.
 
     Long portions of heads of up to 128 key channels go through as ``chunked_memory``; those of wider heads are walked in
-    chunks side by side, as in ``outer_scan``; what a chunk's rows do to a state that
-    comes in is no mere factor here but a matrix ``[dim, dim]``, which the first walk finds by carrying the unit
-    vectors along as further columns."""
+    chunks side by side (``DELTA_CHUNKS``): every chunk from zeros, the chunks' end states chained, every chunk once more from the
+    state it starts with.  What a chunk's rows do to a state that comes in is a matrix ``[dim, dim]``, which the first walk
+    finds by carrying the unit vectors along as further columns."""
     rows = qkv.shape[0]
     if state.dtype != torch.float32 or tuple(state.shape[1:]) != (heads, dim, vdim) or not state.is_contiguous():
         raise KernelError(f"delta_scan: state {tuple(state.shape)} is not [slots, {heads}, {dim}, {vdim}] float32")
@@ -1754,13 +1732,14 @@ def delta_scan(qkv: torch.Tensor, columns: dict, beta: torch.Tensor, step_size: 
         # every entry with a single row: the kernel that is made for it, if it takes the size (no chunks are walked then);
         # eight rows of 16 heads of 128 x 128: 14.5 us walked, 8.9 in that kernel
         single = segments.shape[0] == rows and not accumulate and transition is None and library().leone_step_fits(dim, vdim)
+        in_chunks = () if single else (1 if no_input else 0, 1 if accumulate else 0)
         call("leone_delta_step" if single else "leone_delta_scan", _dev(qkv, "q, k, v", torch.float32), qkv.shape[1], columns["q"], columns["k"], columns["v"],
              beta_at, beta_stride, step_at, step_stride, 1 if per_head else 0, _dev(rate_log, "rate", None, (heads,)),
              _dev(step_bias, "step bias", None, (heads if per_head else heads * dim,)), _code(rate_log, "rate"), float(q_scale), float(unit_eps),
-             1 if no_input else 0, 1 if accumulate else 0, _dev(segments, "segments", torch.int32), segments.shape[0],
+             *in_chunks, _dev(segments, "segments", torch.int32), segments.shape[0],
              _dev(state_in, "state read"), state_in.stride(0) if state_in is not None else 0,
              _dev(state_out, "state written"), state_out.stride(0) if state_out is not None else 0,
-             _dev(transition, "transitions"), _dev(out, "out"), heads, kv_heads, dim, vdim, _stream())
+             *(() if single else (_dev(transition, "transitions"),)), _dev(out, "out"), heads, kv_heads, dim, vdim, _stream())
 
     plan = None
     if chunked_memory_supported(dim) and dim <= library().leone_chunk_max_delta_dim():
@@ -1993,7 +1972,7 @@ def routed_feed_forward(x: torch.Tensor, logits: torch.Tensor, correction: Optio
 
 
 # ---- a forget gate per key channel, attention through a shared latent, the stream as a sum over depth -----------
-GATED_CHUNKS = (64, 256)     # rows of a chunk and the portions that are walked in chunks (as ``OUTER_CHUNKS``)
+GATED_CHUNKS = (64, 256)     # rows of a chunk and the portions that are walked in chunks (as ``DELTA_CHUNKS``)
 
 
 def gated_scan(proj: torch.Tensor, columns: dict, f_bias: torch.Tensor, lower: torch.Tensor, state: torch.Tensor, step,

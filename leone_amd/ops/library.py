@@ -75,16 +75,15 @@ _PROTOTYPES = {
     "leone_head_gate": [P, c_int, P, ctypes.c_long, c_int, c_int, c_int, P],
     "leone_exp_gates": [P, ctypes.c_long, c_int, c_int, P, P, c_int, c_float, P, c_int, P, ctypes.c_long, ctypes.c_long,
                         ctypes.c_long, c_int, P, P, c_int, P],
-    "leone_outer_scan": [P, ctypes.c_long, c_int, c_int, c_int, P, P, c_int, c_int, c_int, c_float, c_float, c_int, P, P, c_int, c_int,
-                         P, P, c_int, P, ctypes.c_long, P, ctypes.c_long, ctypes.c_long, P, P, P, c_int, c_int, c_int, P],
+    "leone_outer_scan": [P, ctypes.c_long, c_int, c_int, c_int, P, P, c_int, c_float, c_float, c_int, P, P, c_int, c_int,
+                         P, P, c_int, P, ctypes.c_long, P, ctypes.c_long, ctypes.c_long, P, P, c_int, c_int, c_int, P],
     "leone_step_fits": [c_int, c_int],
-    "leone_outer_step": [P, ctypes.c_long, c_int, c_int, c_int, P, P, c_int, c_int, c_int, c_float, c_float, c_int, P, P, c_int, c_int,
-                         P, P, c_int, P, ctypes.c_long, P, ctypes.c_long, ctypes.c_long, P, P, P, c_int, c_int, c_int, P],
-    "leone_outer_chain": [P, c_int, P, ctypes.c_long, P, P, ctypes.c_long, ctypes.c_long, c_int, c_int, c_int, P],
+    "leone_outer_step": [P, ctypes.c_long, c_int, c_int, c_int, P, P, c_int, c_float, c_float, c_int, P, P, c_int, c_int,
+                         P, P, c_int, P, ctypes.c_long, P, ctypes.c_long, ctypes.c_long, P, P, c_int, c_int, c_int, P],
     "leone_delta_scan": [P, ctypes.c_long, c_int, c_int, c_int, P, ctypes.c_long, P, ctypes.c_long, c_int, P, P, c_int, c_float,
                          c_float, c_int, c_int, P, c_int, P, ctypes.c_long, P, ctypes.c_long, P, P, c_int, c_int, c_int, c_int, P],
     "leone_delta_step": [P, ctypes.c_long, c_int, c_int, c_int, P, ctypes.c_long, P, ctypes.c_long, c_int, P, P, c_int, c_float,
-                         c_float, c_int, c_int, P, c_int, P, ctypes.c_long, P, ctypes.c_long, P, P, c_int, c_int, c_int, c_int, P],
+                         c_float, P, c_int, P, ctypes.c_long, P, ctypes.c_long, P, c_int, c_int, c_int, c_int, P],
     "leone_embed_placed": [P, c_int, P, P, c_int, c_int, c_int, c_float, P, P, c_int, P, P],
     "leone_glu": [P, P, c_int, c_int, c_int, c_int, c_float, P],
     "leone_add_normed": [P, P, c_int, ctypes.c_long, P, c_int, c_float, P, c_int, P, c_int, c_float, P, c_int, c_int, P],

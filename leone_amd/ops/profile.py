@@ -45,7 +45,6 @@ OPERATIONS = {
     "leone_head_gate": "head gate",
     "leone_outer_scan": "outer scan",
     "leone_outer_step": "outer scan",
-    "leone_outer_chain": "outer scan",
     "leone_exp_gates": "exp gates",
     "leone_delta_scan": "delta scan",
     "leone_delta_step": "delta scan",
