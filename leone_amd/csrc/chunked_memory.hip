@@ -87,7 +87,13 @@ struct ChunkArgs {
 __device__ inline float chunk_act(float x, int silu) { return silu ? x / (1.0f + expf(-x)) : x; }
 __device__ inline float chunk_softplus(float z) { return z > 20.f ? z : log1pf(expf(z)); }
 constexpr float kNothingLeft = -1e4f;   // a logarithm whose exponential is zero and of which 64 add up without overflow
-__device__ inline float between(double later, double earlier) { return static_cast<float>(exp(later - earlier)); }
+// exp(later - earlier), the difference's rounding to float made good (an exponential in double took a chunk's tiles 0.4 us longer;
+// read-outs and states are as far from 64 bits either way).
+__device__ inline float between(double later, double earlier) {
+    const double of = later - earlier;
+    const float rounded = static_cast<float>(of), result = expf(rounded);
+    return result == INFINITY ? result : fmaf(result, static_cast<float>(of - rounded), result);
+}
 __device__ inline float element(const float4& f, int v) { return v == 0 ? f.x : v == 1 ? f.y : v == 2 ? f.z : f.w; }
 __device__ inline floatx4 mfma4(float a, float b, floatx4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
@@ -183,25 +189,20 @@ __global__ void __launch_bounds__(kChunkThreads, 2) chunk_prepare_kernel(ChunkAr
     const long at = static_cast<long>(chunk) * p.heads + head;
     const int block = blockIdx.z * kDim;        // delta rule: the value columns solved here; the first workgroup writes all the rest
 
-    // reads in batches, of the last row or channel again where there is none, so that no read waits for the one before
+    // Reads in batches, of the last row or channel again where there is none, so that no read waits for the one before; the first
+    // batch is on its way while wave 0 makes the decays, a logarithm in double among them.
     constexpr int kBatch = 8;
     static_assert(kChunkRows * kDim % (kBatch * kChunkThreads) == 0, "whole batches");
-    for (int from = tid; from < kChunkRows * kDim; from += kBatch * kChunkThreads) {
-        float q[kBatch], k[kBatch];
+    float q_read[kBatch], k_read[kBatch];
+    const auto read_rows = [&](int from) {
 #pragma unroll
         for (int e = 0; e < kBatch; ++e) {
             const int t = (from + e * kChunkThreads) / kDim, i = (from + e * kChunkThreads) % kDim;
             const float* base = p.rows + static_cast<long>(first + min(t, n - 1)) * p.stride + kvh * p.dim + min(i, p.dim - 1);
-            q[e] = base[p.q_off], k[e] = base[p.k_off];
+            q_read[e] = base[p.q_off], k_read[e] = base[p.k_off];
         }
-#pragma unroll
-        for (int e = 0; e < kBatch; ++e) {
-            const int t = (from + e * kChunkThreads) / kDim, i = (from + e * kChunkThreads) % kDim;
-            const bool there = t < n && i < p.dim;
-            sq[t * row_p + i] = there ? chunk_act(q[e], p.silu) : 0.f;
-            sk[t * row_p + i] = there ? chunk_act(k[e], p.silu) : 0.f;
-        }
-    }
+    };
+    read_rows(tid);
     if (wave == 0) {
         // the decays' logarithms summed up over the chunk; rows past its end decay nothing and write nothing
         double l = 0.;
@@ -227,6 +228,16 @@ __global__ void __launch_bounds__(kChunkThreads, 2) chunk_prepare_kernel(ChunkAr
         cum[lane] = l;
         so_far[lane] = between(l, 0.);
         to_end[lane] = between(__shfl(l, kWave - 1, kWave), l);
+    }
+    for (int from = tid; from < kChunkRows * kDim; from += kBatch * kChunkThreads) {
+        if (from != tid) read_rows(from);
+#pragma unroll
+        for (int e = 0; e < kBatch; ++e) {
+            const int t = (from + e * kChunkThreads) / kDim, i = (from + e * kChunkThreads) % kDim;
+            const bool there = t < n && i < p.dim;
+            sq[t * row_p + i] = there ? chunk_act(q_read[e], p.silu) : 0.f;
+            sk[t * row_p + i] = there ? chunk_act(k_read[e], p.silu) : 0.f;
+        }
     }
     __syncthreads();
     if (!kDelta && p.cos_table != nullptr) {
@@ -325,17 +336,22 @@ __global__ void __launch_bounds__(kChunkThreads, 2) chunk_prepare_kernel(ChunkAr
     const auto taken_v = [&](float v, int t, int j) { return t < n && j < p.vdim ? chunk_act(v, p.silu) : 0.f; };
     if constexpr (!kDelta) {
         constexpr int kRows = kChunkThreads / kWave, kEach = kChunkRows / kRows;
+        const int norm = p.dot != nullptr ? p.vdim : -1;        // the normaliser's column
+        float by[kEach];
+#pragma unroll
+        for (int e = 0; e < kEach; ++e) by[e] = strength[wave + kRows * e];
         for (int j = lane; j < p.vdim_p; j += kWave) {
+            if (j == norm) continue;
             float v[kEach];
 #pragma unroll
             for (int e = 0; e < kEach; ++e) v[e] = read_v(wave + kRows * e, j);
 #pragma unroll
             for (int e = 0; e < kEach; ++e) {
                 const int t = wave + kRows * e;
-                const float value = j == p.vdim && p.dot != nullptr ? (t < n ? 1.f : 0.f) : taken_v(v[e], t, j);
-                values[t * p.vdim_p + j] = value * strength[t];
+                values[t * p.vdim_p + j] = taken_v(v[e], t, j) * by[e];
             }
         }
+        if (norm >= 0 && tid < kChunkRows) values[tid * p.vdim_p + norm] = strength[tid];      // (0 past the chunk's end)
     } else {
         float* solved_k = p.solved_k + at * kChunkRows * kDim;
         __syncthreads();                    // M is made and K written: their places take the right sides, K and a block of V
@@ -562,6 +578,11 @@ __global__ void __launch_bounds__(kChunkThreads, 1) chunk_prepare_channel_kernel
                     block == 0 ? p.solved_k + at * kChunkRows * kDim : nullptr);
 }
 
+// Workgroups of chunk_walk a compute unit, where its registers allow: 256 a lane for two of them.  (Eight portions of 512 rows with
+// one workgroup and with two a unit, us: fixed decays, 4 heads of 128 x 256, 69 and 58; the delta rule, 8 heads of 64 x 128, 90 and 80.)
+template <bool kDelta, int kT>
+constexpr int kWalkers = kT * (kDelta ? 2 : 1) <= 2 ? 2 : 1;
+
 // What a wave needs of a chunk, all of it asked for a chunk ahead.
 template <bool kDelta, int kT, bool kChannel>
 struct ChunkOperands {
@@ -624,35 +645,37 @@ __device__ inline bool walk_chunks(const ChunkArgs& p, WalkShared<kDelta>& share
     float* su = shared.u;
     bool odd = false;
     ChunkOperands<kDelta, kT, kChannel> ahead;
-    fetch_chunk<kDelta, kT, kChannel>(p, g0, head, wave, c, g, col, ahead);
+    if constexpr (!kCareful) fetch_chunk<kDelta, kT, kChannel>(p, g0, head, wave, c, g, col, ahead);
     for (int chunk = g0; chunk < g1; ++chunk) {
+        if constexpr (kCareful) fetch_chunk<kDelta, kT, kChannel>(p, chunk, head, wave, c, g, col, ahead);
         const ChunkOperands<kDelta, kT, kChannel> now = ahead;
-        fetch_chunk<kDelta, kT, kChannel>(p, chunk + 1 < g1 ? chunk + 1 : chunk, head, wave, c, g, col, ahead);
+        if constexpr (!kCareful) fetch_chunk<kDelta, kT, kChannel>(p, chunk + 1 < g1 ? chunk + 1 : chunk, head, wave, c, g, col, ahead);
         // Sums are kept short and put together at the end (two a row of W S and Q S, one a tile of M U, the chunk's own part of S
         // by itself): what is added to a sum is rounded at the sum's size.
-        floatx4 ws[4], qs[4], ws2[4] = {}, qs2[4] = {};
+        // (sums of all four tiles of rows side by side take registers that a second workgroup a unit needs)
+        constexpr int kSide = kWalkers<kDelta, kT> == 1 ? 4 : kDelta ? 1 : 2;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) ws[r] = qs[r] = floatx4{0.f, 0.f, 0.f, 0.f};
+        for (int r0 = 0; r0 < 4; r0 += kSide) {
+            floatx4 ws[kSide][2] = {}, qs[kSide][2] = {};
 #pragma unroll
-        for (int t = 0; t < kT; ++t)
+            for (int t = 0; t < kT; ++t)
 #pragma unroll
-            for (int v = 0; v < 4; ++v)
+                for (int v = 0; v < 4; ++v)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    floatx4& w = v < 2 ? ws[r] : ws2[r];
-                    floatx4& q = v < 2 ? qs[r] : qs2[r];
-                    if constexpr (kDelta) w = mfma4(element(now.w[r][t], v), S[t][v], w);
-                    q = mfma4(element(now.q[r][t], v), S[t][v], q);
+                    for (int r = 0; r < kSide; ++r) {
+                        if constexpr (kDelta) ws[r][v / 2] = mfma4(element(now.w[r0 + r][t], v), S[t][v], ws[r][v / 2]);
+                        qs[r][v / 2] = mfma4(element(now.q[r0 + r][t], v), S[t][v], qs[r][v / 2]);
+                    }
+#pragma unroll
+            for (int r = 0; r < kSide; ++r) {
+                const floatx4 w = ws[r][0] + ws[r][1], q = qs[r][0] + qs[r][1];
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    part[0][wave][(16 * (r0 + r) + 4 * g + v) * kPartStride + c] = q[v];
+                    if constexpr (kDelta) part[kDelta ? 1 : 0][wave][(16 * (r0 + r) + 4 * g + v) * kPartStride + c] = w[v];
                 }
-#pragma unroll
-        for (int r = 0; r < 4; ++r) ws[r] += ws2[r], qs[r] += qs2[r];
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                part[0][wave][(16 * r + 4 * g + v) * kPartStride + c] = qs[r][v];
-                if constexpr (kDelta) part[kDelta ? 1 : 0][wave][(16 * r + 4 * g + v) * kPartStride + c] = ws[r][v];
             }
+        }
         __syncthreads();
         floatx4 o = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -722,7 +745,7 @@ __device__ inline bool walk_chunks(const ChunkArgs& p, WalkShared<kDelta>& share
 }
 
 template <bool kDelta, int kT, bool kChannel>
-__global__ void __launch_bounds__(kChunkThreads, 1) chunk_walk_kernel(ChunkArgs p) {
+__global__ void __launch_bounds__(kChunkThreads, (kWalkers<kDelta, kT>)) chunk_walk_kernel(ChunkArgs p) {
     __shared__ WalkShared<kDelta> shared;
     const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave, c = lane & 15, g = lane >> 4;
     const int link = blockIdx.x, head = blockIdx.y, col = 16 * blockIdx.z + c;
