@@ -17,7 +17,7 @@
 // are the operand of the second product as they stand.
 //
 // Measured (us; the row kernel of attention.hip before): 16 heads over 4 of 128 elements, one row at 780 keys 25 (314), a prompt
-// of 777 rows 73 (1375).
+// of 777 rows 71 (1375), of 2,048 rows 295 (8589).
 #include "common.h"
 #include "leone_hip.h"
 #include "score_shape.h"
@@ -61,9 +61,13 @@ __global__ void __launch_bounds__(kWaves * kWave, kDim == 64 ? 3 : 2) attention_
     __shared__ f32x4 sm_acc[kWaves / 2][kRuns][kWave];
 
     // The rows of this workgroup: from this one on, those of the same request up to the next multiple of `most`; the
-    // workgroups of the rows that another one takes have nothing to do.
+    // workgroups of the rows that another one takes have nothing to do.  Rows are numbered so that those at the multiples come first,
+    // one behind the other: workgroups go to the eight dies in turn, and every 4th or 16th would have left the work of a portion to one
+    // or two of them (2,048 rows of 16 heads over 4 of 128: 1330 us, numbered so 295).
     const int group = g.q_heads / g.kv_heads, most = kQueries / group;
-    const int first_row = blockIdx.x, kvh = blockIdx.y;
+    const int multiples = (g.rows + most - 1) / most;
+    const int first_row = blockIdx.x % multiples * most + blockIdx.x / multiples, kvh = blockIdx.y;
+    if (first_row >= g.rows) return;
     const int entry = g.row_entry[first_row];
     if (first_row % most != 0 && g.row_entry[first_row - 1] == entry) return;
     int count = 1;
@@ -310,11 +314,12 @@ void launch_attention_f32(const float* q, float* out, const float* k_pool, const
     const AttentionF32Args args{q, out, k_pool, v_pool, positions, row_entry, block_table, max_blocks, rows, q_heads, kv_heads,
                                 page_tokens, scale, window, gate, gate_stride, keep_first, gate_each, slopes, temp_coef, temp_every,
                                 shape, chunk};
-    const dim3 grid(rows, kv_heads);
-    // Eight waves, a share each, where the launch is small or heads are of 128 elements (777 rows of 16 heads over 4: 73 us, with
-    // four waves 83); four waves with two shares each for many rows of 64, whose workgroups are short (1,500 rows of 8 heads
-    // over 2: 161 us, with eight 192; 200 rows: 15.7 and 14.5).  rows * kv_heads are launched; of the rows that share a workgroup
-    // all but the first's leave at once, which costs less the fewer waves they have.
+    const int most = kQueries / (q_heads / kv_heads);
+    const dim3 grid(ceil_div(rows, most) * most, kv_heads);
+    // Eight waves, a share each, where the launch is small or heads are of 128 elements; four waves with two shares each for many
+    // rows of 64, whose workgroups are short (us, eight waves and four: 8 heads over 2, 1,500 rows 66 and 58, 300 decoded rows at 500
+    // keys 38 and 32; 16 over 8, 777 rows 57 and 45; but 300 rows behind 1,200 keys of 8 over 2 30 and 48, which the host cannot tell
+    // from decoded rows).  As many workgroups are launched as there are rows: those of the rows that share one leave at once.
     if (head_dim == 128) attention_f32_kernel<128, 8><<<grid, 8 * kWave, 0, stream>>>(args);
     else if (static_cast<long>(rows) * kv_heads < 512) attention_f32_kernel<64, 8><<<grid, 8 * kWave, 0, stream>>>(args);
     else attention_f32_kernel<64, 4><<<grid, 4 * kWave, 0, stream>>>(args);
