@@ -481,7 +481,9 @@ __device__ inline moe_bf16x8 moe_zero8() {
 // its bytes are the bound.  A workgroup takes 16 rows of the matrix (gated: and their up rows) and its four waves share out
 // the inner size, each with eight steps of 32 on their way at a time; their sums meet in shared memory, in the waves' order.
 // (A wave that walked the whole inner size by itself had a quarter of the loads in flight and four times the chain.)
-// Eight rows of 2,048 over 34 experts of 768, four routed places and two for every row (us, before): gated 38 (47), down 19 (24).
+// The loads are ordinary ones: each is half of a line in 16 rows, whose other half a load behind it takes from the cache, and marked
+// as not to be kept (as where the weights are streamed in whole lines) lines came twice.  Both products of 32 experts of 2,048 x 768, us,
+// marked and not: four rows 42 and 35, eight 65 and 56; 8 experts of 4,096 x 2,048, four rows 99 and 68.
 template <int kMode>
 __global__ void __launch_bounds__(kMoeThreads, 3)
 moe_product_stream_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, void* __restrict__ y,
@@ -509,9 +511,9 @@ moe_product_stream_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict
     {                                                                                                          \
         const int at = 32 * (S) + 8 * g;                                                                       \
         const bool in = (S) < last && at < k;                                                                  \
-        a[D] = (row_ok && in) ? __builtin_bit_cast(moe_bf16x8, load_streamed16(wa + at)) : moe_zero8();        \
+        a[D] = (row_ok && in) ? moe_load8(wa + at) : moe_zero8();        \
         if constexpr (kGated)                                                                                  \
-            a2[D] = (row_ok && in) ? __builtin_bit_cast(moe_bf16x8, load_streamed16(wa + matrix + at)) : moe_zero8(); \
+            a2[D] = (row_ok && in) ? moe_load8(wa + matrix + at) : moe_zero8(); \
         xb[D] = (pair >= 0 && in) ? moe_load8(xrow + at) : moe_zero8();                                        \
     }
 #pragma unroll
@@ -581,7 +583,7 @@ moe_product_tiled_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict_
     // same rows of its matrix, then lie on one die.  (Groups of two or four tiles with all their row blocks measured the same.)
     const int per_die = (n_tiles * n_blocks + 7) / 8;
     const int place = static_cast<int>(blockIdx.x % 8) * per_die + static_cast<int>(blockIdx.x / 8);
-    if (place >= n_tiles * n_blocks || static_cast<int>(blockIdx.x / 8) >= per_die) return;
+    if (place >= n_tiles * n_blocks) return;
     const int tile = place % n_tiles;
     const int row_block = place / n_tiles;
     const int e = tile_expert[tile];
