@@ -9,9 +9,9 @@
 //                weight 1 (a shared expert cut to the experts' size) may stand behind the routed ones.
 //   moe_product  gated: act(W_gate x) * (W_up x) of every pair, by its expert's matrices; plain (experts without a gate):
 //                act(W_up x), or act(W_up (weight x)) where the pair's weight multiplies what the expert reads; else
-//                W_down of that, times the pair's weight if there is one, float.  Three kernels: any type and size (float sums of 8-element runs a lane);
+//                W_down of that, times the pair's weight if there is one, float.  Four kernels: any type and size (float sums of 8-element runs a lane);
 //                bfloat16 on the matrix cores from registers (tiles of 16 pairs, the inner size shared out over a
-//                workgroup's waves); bfloat16 on the matrix cores through shared memory (tiles of 64 pairs).
+//                workgroup's waves); bfloat16 on the matrix cores through shared memory (tiles of 64 and of 128 pairs).
 //   moe_combine  a row's pairs summed in the order of its places; a router output beyond the experts with
 //                matrices hands the row itself on (times its weight); a delta that comes along is added.
 //
@@ -565,6 +565,34 @@ constexpr int kBigPairs = 64;
 constexpr int kBigRows = 128;
 constexpr int kBigChunk = 64;
 
+// Rows r .. r + 3 of a pair's result, r < n.
+template <int kMode>
+__device__ inline void store_rows(void* y, int pair, int r, int n, const float (&v)[4]) {
+    const bool whole = r + 3 < n && n % 4 == 0;
+    if constexpr (kMode != kMoeDown) {
+        bf16_t* to = static_cast<bf16_t*>(y) + static_cast<long>(pair) * n + r;
+        if (whole) {
+            uint2 packed;
+            packed.x = bf16_bits_from_float(v[0]) | (static_cast<uint32_t>(bf16_bits_from_float(v[1])) << 16);
+            packed.y = bf16_bits_from_float(v[2]) | (static_cast<uint32_t>(bf16_bits_from_float(v[3])) << 16);
+            *reinterpret_cast<uint2*>(to) = packed;
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (r + j < n) to[j] = from_float<bf16_t>(v[j]);
+        }
+    } else {
+        float* to = static_cast<float*>(y) + static_cast<long>(pair) * n + r;
+        if (whole) {
+            *reinterpret_cast<float4*>(to) = float4{v[0], v[1], v[2], v[3]};
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (r + j < n) to[j] = v[j];
+        }
+    }
+}
+
 template <int kMode>
 __global__ void __launch_bounds__(kMoeThreads, 3)
 moe_product_tiled_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, void* __restrict__ y,
@@ -685,29 +713,133 @@ moe_product_tiled_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict_
             for (int j = 0; j < 4; ++j)
                 v[j] = kGated ? glu_value(acc[ta][tb][j], acc[kGated ? ta + 2 : ta][tb][j], act, limit)
                               : kMode == kMoePlain ? plain_act(acc[ta][tb][j] * scale, act) : acc[ta][tb][j] * scale;
-            const bool whole = r + 3 < n && n % 4 == 0;
-            if constexpr (kMode != kMoeDown) {
-                bf16_t* to = static_cast<bf16_t*>(y) + static_cast<long>(pair) * n + r;
-                if (whole) {
-                    uint2 packed;
-                    packed.x = bf16_bits_from_float(v[0]) | (static_cast<uint32_t>(bf16_bits_from_float(v[1])) << 16);
-                    packed.y = bf16_bits_from_float(v[2]) | (static_cast<uint32_t>(bf16_bits_from_float(v[3])) << 16);
-                    *reinterpret_cast<uint2*>(to) = packed;
-                } else {
+            store_rows<kMode>(y, pair, r, n, v);
+        }
+    }
+}
+
+// Tiles of 128 pairs, bfloat16, where an expert gets hundreds: 128 rows of the matrix (gated: and their up rows), whose chunks lie
+// in shared memory as above, one at a time, the next on its way in registers.  The four waves take 64 rows x 64 pairs each, four and four
+// operands (gated: eight and four) for 16 (32) matrix instructions, and a matrix is read half as often: with many tiles an expert that
+// counts for more than chunks in flight.  Both products, us, tiles of 64 and of 128: 32 experts of 2,048 x 768, 300 pairs an expert 247 and 257, 500 388
+// and 351, 700 533 and 468; of 4,096 x 1,024, 500 910 and 790; 64 of 2,048 x 1,408, 700 1594 and 1332.
+constexpr int kWidePairs = 128;
+constexpr int kWideRows = 128;
+
+template <int kMode>
+__global__ void __launch_bounds__(kMoeThreads, 2)
+moe_product_wide_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, void* __restrict__ y,
+                         const float* __restrict__ pair_weight, const int* __restrict__ tile_expert,
+                         const int* __restrict__ tile_pairs, int top, int n, int k, int act, float limit, int n_tiles, int n_blocks) {
+    constexpr bool kGated = kMode == kMoeGated;
+    constexpr int kWRows = kGated ? 2 * kWideRows : kWideRows;          // rows of the matrix in a chunk
+    constexpr int kXPieces = kWidePairs * 8 / kMoeThreads;             // 16-byte pieces of x a thread brings per chunk
+    constexpr int kWPieces = kWRows * 8 / kMoeThreads;
+    __shared__ uint4 sx[2 * kWidePairs * 4];                           // [half][row][4 pieces]
+    __shared__ uint4 sw[2 * kWRows * 4];
+    // Workgroups go to the eight dies in turn, and each die has a cache of its own: the work is numbered so that a
+    // die gets a run of neighbouring (row block, tile) places, tiles fastest: the tiles of one expert, which read the
+    // same rows of its matrix, then lie on one die.
+    const int per_die = (n_tiles * n_blocks + 7) / 8;
+    const int place = static_cast<int>(blockIdx.x % 8) * per_die + static_cast<int>(blockIdx.x / 8);
+    if (place >= n_tiles * n_blocks) return;
+    const int tile = place % n_tiles;
+    const int row_block = place / n_tiles;
+    const int e = tile_expert[tile];
+    if (e < 0) return;
+    const int tid = threadIdx.x;
+    const int wave = tid / kWave, lane = tid % kWave;
+    const int c = lane & 15, g = lane >> 4;
+    const int wr = wave >> 1, wp = wave & 1;
+    const int row_base = row_block * kWideRows;
+    const long matrix = static_cast<long>(n) * k;
+    const int* my_pairs = tile_pairs + static_cast<long>(tile) * kWidePairs;
+
+    // what this thread brings: piece p = tid + 256 i is part p % 8 of row p / 8 (row tid / 8 + 32 i)
+    const int part = tid & 7;
+    const int half = part >> 2, quarter = part & 3;
+    const bf16_t* x_from[kXPieces];
+    const bf16_t* w_from[kWPieces];
 #pragma unroll
-                    for (int j = 0; j < 4; ++j)
-                        if (r + j < n) to[j] = from_float<bf16_t>(v[j]);
-                }
-            } else {
-                float* to = static_cast<float*>(y) + static_cast<long>(pair) * n + r;
-                if (whole) {
-                    *reinterpret_cast<float4*>(to) = float4{v[0], v[1], v[2], v[3]};
-                } else {
+    for (int i = 0; i < kXPieces; ++i) {
+        const int pair = my_pairs[tid / 8 + 32 * i];
+        x_from[i] = pair < 0 ? nullptr : x + static_cast<long>(kMode != kMoeDown ? pair / top : pair) * k + 8 * part;
+    }
 #pragma unroll
-                    for (int j = 0; j < 4; ++j)
-                        if (r + j < n) to[j] = v[j];
-                }
+    for (int i = 0; i < kWPieces; ++i) {
+        const int local = tid / 8 + 32 * i;                           // gated: rows 0..127 gate, 128..255 up
+        const int row = row_base + (local % kWideRows);
+        w_from[i] = row >= n ? nullptr
+                             : w + static_cast<long>(e) * (kGated ? 2 : 1) * matrix + (local >= kWideRows ? matrix : 0) +
+                                   static_cast<long>(row) * k + 8 * part;
+    }
+    uint4 hx[kXPieces], hw[kWPieces];
+
+    moe_floatx4 acc[4][4], acc2[kGated ? 4 : 1][4];
+#pragma unroll
+    for (int ta = 0; ta < 4; ++ta)
+#pragma unroll
+        for (int tb = 0; tb < 4; ++tb) {
+            acc[ta][tb] = moe_floatx4{0.f, 0.f, 0.f, 0.f};
+            if constexpr (kGated) acc2[ta][tb] = moe_floatx4{0.f, 0.f, 0.f, 0.f};
+        }
+    const int chunks = (k + kBigChunk - 1) / kBigChunk;
+#define LEONE_MOE_BRING(K0)                                                                                              \
+    {                                                                                                                    \
+        const bool in = (K0) + 8 * part < k;                                                                             \
+        _Pragma("unroll") for (int i = 0; i < kXPieces; ++i) {                                                           \
+            hx[i] = uint4{0u, 0u, 0u, 0u};                                                                               \
+            if (x_from[i] && in) hx[i] = *reinterpret_cast<const uint4*>(x_from[i] + (K0));                              \
+        }                                                                                                                \
+        _Pragma("unroll") for (int i = 0; i < kWPieces; ++i) {                                                           \
+            hw[i] = uint4{0u, 0u, 0u, 0u};                                                                               \
+            if (w_from[i] && in) hw[i] = *reinterpret_cast<const uint4*>(w_from[i] + (K0));                              \
+        }                                                                                                                \
+    }
+    LEONE_MOE_BRING(0)
+    for (int ck = 0; ck < chunks; ++ck) {
+#pragma unroll
+        for (int i = 0; i < kXPieces; ++i) sx[(half * kWidePairs + tid / 8 + 32 * i) * 4 + quarter] = hx[i];
+#pragma unroll
+        for (int i = 0; i < kWPieces; ++i) sw[(half * kWRows + tid / 8 + 32 * i) * 4 + quarter] = hw[i];
+        __syncthreads();
+        if (ck + 1 < chunks) LEONE_MOE_BRING((ck + 1) * kBigChunk)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            moe_bf16x8 a[4], a2[kGated ? 4 : 1], b[4];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                a[t] = __builtin_bit_cast(moe_bf16x8, sw[(h * kWRows + 64 * wr + 16 * t + c) * 4 + g]);
+                if constexpr (kGated) a2[t] = __builtin_bit_cast(moe_bf16x8, sw[(h * kWRows + kWideRows + 64 * wr + 16 * t + c) * 4 + g]);
+                b[t] = __builtin_bit_cast(moe_bf16x8, sx[(h * kWidePairs + 64 * wp + 16 * t + c) * 4 + g]);
             }
+#pragma unroll
+            for (int ta = 0; ta < 4; ++ta)
+#pragma unroll
+                for (int tb = 0; tb < 4; ++tb) {
+                    acc[ta][tb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[ta], b[tb], acc[ta][tb], 0, 0, 0);
+                    if constexpr (kGated) acc2[ta][tb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2[ta], b[tb], acc2[ta][tb], 0, 0, 0);
+                }
+        }
+        __syncthreads();                               // everyone has read the chunk before the next is put down
+    }
+#undef LEONE_MOE_BRING
+    // lane (c, g) holds rows 4 g .. 4 g + 3 of pair c of every (ta, tb)
+#pragma unroll
+    for (int tb = 0; tb < 4; ++tb) {
+        const int pair = my_pairs[64 * wp + 16 * tb + c];
+        if (pair < 0) continue;
+        const float scale = kGated || !pair_weight ? 1.f : pair_weight[pair];
+#pragma unroll
+        for (int ta = 0; ta < 4; ++ta) {
+            const int r = row_base + 64 * wr + 16 * ta + 4 * g;
+            if (r >= n) continue;
+            float v[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                v[j] = kGated ? glu_value(acc[ta][tb][j], acc2[kGated ? ta : 0][tb][j], act, limit)
+                              : kMode == kMoePlain ? plain_act(acc[ta][tb][j] * scale, act) : acc[ta][tb][j] * scale;
+            store_rows<kMode>(y, pair, r, n, v);
         }
     }
 }
@@ -780,7 +912,7 @@ extern "C" int leone_route_plan(const float* logits, const void* correction, int
     LEONE_REQUIRE(group_count >= 1 && total % group_count == 0 && group_keep >= 1 && group_keep <= group_count,
                   "route_plan: %d groups (dividing %d outputs), %d kept", group_count, total, group_keep);
     LEONE_REQUIRE(experts > 0 && experts <= 1024, "route_plan: %d experts (at most 1024)", experts);
-    LEONE_REQUIRE(tile == kTilePairs || tile == 16 || tile == kBigPairs, "route_plan: tiles of %d pairs", tile);
+    LEONE_REQUIRE(tile == kTilePairs || tile == 16 || tile == kBigPairs || tile == kWidePairs, "route_plan: tiles of %d pairs", tile);
     const long pairs = static_cast<long>(rows) * (top + always);
     const long needed = pairs / tile + experts;
     LEONE_REQUIRE(max_tiles >= (needed < pairs ? needed : pairs), "route_plan: %d tiles cannot hold %ld pairs of %d experts", max_tiles,
@@ -794,7 +926,7 @@ extern "C" int leone_route_plan(const float* logits, const void* correction, int
 
 extern "C" int leone_moe_plan(const int* chosen, int pairs, int experts, int* tile_expert, int* tile_pairs, int max_tiles,
                               int tile, hipStream_t stream) {
-    LEONE_REQUIRE(tile == kTilePairs || tile == 16 || tile == kBigPairs, "moe_plan: tiles of %d pairs", tile);
+    LEONE_REQUIRE(tile == kTilePairs || tile == 16 || tile == kBigPairs || tile == kWidePairs, "moe_plan: tiles of %d pairs", tile);
     LEONE_REQUIRE(chosen && tile_expert && tile_pairs, "moe_plan: null pointer");
     LEONE_REQUIRE(pairs > 0 && experts > 0 && experts <= 1024, "moe_plan: %d pairs, %d experts (at most 1024)", pairs, experts);
     const long needed = static_cast<long>(pairs) / tile + experts;
@@ -809,7 +941,7 @@ extern "C" int leone_moe_plan(const int* chosen, int pairs, int experts, int* ti
 // gated == 0: x [pairs, k], w [experts, n, k], y float32 [pairs, n] = pair_weight[pair] * product (null: 1).
 // gated == 2: x [rows, k], w [experts, n, k], y [pairs, n] of dtype = act(pair_weight[pair] * product) (null: 1).
 // tile: pairs a tile holds, as leone_moe_plan was told: leone_moe_tile_pairs() for the kernel that takes any type and
-// size; 16 or 64 for the matrix-core kernel (bfloat16, n and k multiples of 8).
+// size; 16, 64 or 128 for the matrix-core kernels (bfloat16, n and k multiples of 8).
 extern "C" int leone_moe_product(const void* x, const void* w, void* y, const float* pair_weight, int dtype, int gated,
                                  const int* tile_expert, const int* tile_pairs, int max_tiles, int tile, int top, int n, int k,
                                  int act, float limit, hipStream_t stream) {
@@ -818,7 +950,7 @@ extern "C" int leone_moe_product(const void* x, const void* w, void* y, const fl
                       (act == kActReluSquared && gated != kMoeGated),
                   "moe_product: unknown activation %d (limit %g)", act, limit);
     if (tile != kTilePairs) {
-        LEONE_REQUIRE(tile == 16 || tile == kBigPairs, "moe_product: tiles of %d pairs", tile);
+        LEONE_REQUIRE(tile == 16 || tile == kBigPairs || tile == kWidePairs, "moe_product: tiles of %d pairs", tile);
         LEONE_REQUIRE(dtype == kBF16 && k % 8 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0,
                       "moe_product: the matrix-core kernel takes bfloat16 with an inner size that is a multiple of 8, not %d", k);
         LEONE_REQUIRE(x && w && y && tile_expert && tile_pairs, "moe_product: null pointer");
@@ -834,17 +966,19 @@ extern "C" int leone_moe_product(const void* x, const void* w, void* y, const fl
             else LEONE_MOE_STREAM(kMoeDown);
 #undef LEONE_MOE_STREAM
         } else {
-            const int blocks = ceil_div(n, gated == kMoeGated ? kBigRows / 2 : kBigRows);
+            const int blocks = ceil_div(n, tile == kWidePairs ? kWideRows : gated == kMoeGated ? kBigRows / 2 : kBigRows);
             const long places = static_cast<long>(max_tiles) * blocks;
             LEONE_REQUIRE(places + 7 <= 0x7fffffffL, "moe_product: too many tiles");
             const int grid = static_cast<int>((places + 7) / 8 * 8);
-#define LEONE_MOE_TILED(MODE)                                                                                                  \
-    moe_product_tiled_kernel<MODE><<<grid, kMoeThreads, 0, stream>>>(static_cast<const bf16_t*>(x), static_cast<const bf16_t*>(w), \
-                                                                     y, pair_weight, tile_expert, tile_pairs, top, n, k, act, limit, \
-                                                                     max_tiles, blocks)
-            if (gated == kMoeGated) LEONE_MOE_TILED(kMoeGated);
-            else if (gated == kMoePlain) LEONE_MOE_TILED(kMoePlain);
-            else LEONE_MOE_TILED(kMoeDown);
+#define LEONE_MOE_TILED(KERNEL, MODE)                                                                                         \
+    KERNEL<MODE><<<grid, kMoeThreads, 0, stream>>>(static_cast<const bf16_t*>(x), static_cast<const bf16_t*>(w), y, pair_weight,   \
+                                                   tile_expert, tile_pairs, top, n, k, act, limit, max_tiles, blocks)
+#define LEONE_MOE_TILES(MODE)                                                                                                 \
+    (tile == kBigPairs ? LEONE_MOE_TILED(moe_product_tiled_kernel, MODE) : LEONE_MOE_TILED(moe_product_wide_kernel, MODE))
+            if (gated == kMoeGated) LEONE_MOE_TILES(kMoeGated);
+            else if (gated == kMoePlain) LEONE_MOE_TILES(kMoePlain);
+            else LEONE_MOE_TILES(kMoeDown);
+#undef LEONE_MOE_TILES
 #undef LEONE_MOE_TILED
         }
         LEONE_LAUNCH_CHECK("moe_product");

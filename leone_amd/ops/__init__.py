@@ -1863,20 +1863,24 @@ def route_topk(logits: torch.Tensor, correction: Optional[torch.Tensor], top: in
     return chosen, weight
 
 
-MOE_WIDE_TILE_PAIRS = 12      # from this many (row, place) pairs an expert on average, the experts' products take tiles of 64 pairs
 ROUTE_PLAN_ROWS = 64          # up to here the router's choice and the tiles are made in one launch
 
 
 def _expert_tiles(x: torch.Tensor, rows: int, top: int, experts: int, hidden: int, ff: int):
     """(pairs a tile, tiles at most, tile_expert, tile_pairs) for a step of ``rows`` rows."""
     pairs = rows * top
-    # bfloat16 with inner sizes in runs of 8 goes to the matrix cores: tiles of 64 pairs where an expert gets many (its
-    # matrices are read once a tile), of 16 where it gets few; anything else in tiles of the plain kernel's size.  Both
-    # products of 32 experts (us, tiles of 16 and 64), width 1,024: 11 pairs an expert 37 and 39, 23 pairs 58 and 42;
-    # width 2,048: 7 pairs 85 and 78, 34 pairs 238 and 88; width 4,096: 4 pairs 276 and 238, 11 pairs 362 and 259, but one
-    # pair 49 and 85.  Below the line a narrow model's few pairs decide, where the smaller tile has more workgroups.
+    # bfloat16 with inner sizes in runs of 8 goes to the matrix cores: the more pairs an expert gets on average, the larger the
+    # tiles (its matrices are read once a tile); anything else in tiles of the plain kernel's size.  Both products, us:
+    #   tiles of 16 and 64: 32 experts of 1,024 x 512, 6 pairs an expert 31 and 32, 11 pairs 36 and 35; of 2,048 x 768, 3 pairs 66 and 61, 11 pairs
+    #   84 and 71; of 4,096 x 1,024, 4 pairs 168 and 187, 6 pairs 181 and 189, 11 pairs 208 and 189; 64 of 2,048 x 1,408, 3 pairs 220 and
+    #   225, 6 pairs 244 and 228, 11 pairs 287 and 232; but where tiles of 64 do not give every unit a workgroup, 8 of 1,024 x 4,096, 6 pairs
+    #   50 and 67, 12 pairs 55 and 70, 16 pairs 83 and 74
+    #   tiles of 64 and 128: 32 of 2,048 x 768, 200 pairs 188 and 182, 300 pairs 247 and 257, 500 pairs 388 and 351; of 4,096 x 1,024, 200 pairs 436 and 368,
+    #   256 pairs 509 and 495; 128 of 2,048 x 768, 300 pairs 956 and 912; but of 1,024 x 512, 500 pairs 160 and 178, 700 pairs 212 and 217
     if x.dtype == torch.bfloat16 and hidden % 8 == 0 and ff % 8 == 0:
-        tile = 64 if pairs >= MOE_WIDE_TILE_PAIRS * experts else 16
+        fills = experts * -(-hidden // 128) >= compute_units(x.device)
+        each = pairs / experts
+        tile = 128 if each >= (200 if hidden > 1024 else 700) else 64 if each >= (6 if fills else 14) else 16
     else:
         tile = library().leone_moe_tile_pairs()
     max_tiles = min(pairs, pairs // tile + experts)

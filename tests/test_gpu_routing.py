@@ -89,3 +89,20 @@ def test_products_in_tiles_of_sixty_four(counts, hidden, ff, gated):
         want = (each if weigh_input else a * each).view(-1, top, hidden).sum(1)
         # as above: middles that are rounded to neighbours, 2^-8 of some elements of one place's sum
         assert float((got - want).norm() / want.norm()) < 2e-3
+
+
+@pytest.mark.parametrize("counts,hidden,ff", [((1283, 127), 72, 136), ((128, 1300, 0, 1401), 136, 64), ((1401,), 8, 200)])
+@pytest.mark.parametrize("gated", [True, False])
+def test_products_in_tiles_of_a_hundred_and_twenty_eight(counts, hidden, ff, gated):
+    """As above where an expert gets many."""
+    test_products_in_tiles_of_sixty_four(counts, hidden, ff, gated)
+
+
+def test_tiles_by_pairs_and_width():
+    """The size of a tile by the pairs an expert gets on average, the width, and whether tiles of 64 give every unit a workgroup."""
+    from leone_amd import ops
+    for hidden, experts, lines in ((1024, 32, (6, 700)), (2048, 32, (6, 200)), (4096, 8, (6, 200)), (1024, 8, (14, 700))):
+        for line, below, above in zip(lines, (16, 64), (64, 128)):
+            x = torch.empty(1, hidden, dtype=torch.bfloat16, device=DEV)
+            assert ops._expert_tiles(x, line * experts - 1, 1, experts, hidden, 512)[0] == below
+            assert ops._expert_tiles(x, line * experts, 1, experts, hidden, 512)[0] == above
