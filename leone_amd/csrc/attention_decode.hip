@@ -138,23 +138,32 @@ struct ScoreBias {
     int temp_every = 0;
 };
 
-// Which row the workgroup takes when there are more workgroups than compute units and none share out a row's keys.  Rows differ in length, and a unit that
-// happens to get two long ones is what the step waits for: the rows are ranked by their positions, the longest go to the first
-// 256 workgroups, and of the 512 that the chip holds at a time the second half start with the shortest, so that a unit's two
-// make up for each other; beyond that many the longest come first throughout.  The heads of a row are neighbouring workgroups,
-// so that every die gets its share of every row.  64 rows of 300 to 2,304 keys, 8 kv heads: 67 us, in the rows' own order
-// 81.
+// Which row the workgroup takes when there are more workgroups than compute units, up to two for each, and none share out a row's keys.  Rows
+// differ in length, and a unit that happens to get two long ones is what the step waits for: the rows are ranked by their
+// positions, the longest go to the first 256 workgroups, and the others start with the shortest, so that a unit's two make up for each other.  The heads of
+// a row are neighbouring workgroups, so that every die gets its share of every row.  Ranking takes 2 to 4 us, so
+// rows of about the same length stay in their own order (us, ranked and not, 32 heads over 8 of 128, 64 rows: of 100 keys 17.6 and 13.0, of 100 to 900
+// 30 and 32, of 100 to 1,700 44 and 51; 8 heads of 64, 64 rows of 100 to 900 20.1 and 19.1, of 100 to 1,700 27.8 and 28.8); with more
+// than two workgroups a unit it gains nothing (128 rows of 8 heads of 64, 100 keys 31 and 13, 100 to 1,700 62 and 60).
 constexpr int kOrderedRows = 2 * kWave;
 constexpr int kOrderedUnits = 256;
+constexpr int kEvenKeys = 1024;
 __device__ inline int ordered_row(const int* __restrict__ positions, int rows, int head_blocks, int lane, int& head_block) {
     const int id = blockIdx.x + rows * blockIdx.y;
     head_block = id % head_blocks;
     const int place = id / head_blocks, first = (kOrderedUnits + head_blocks - 1) / head_blocks;
-    const bool paired = rows * head_blocks <= 2 * kOrderedUnits;
-    const int wanted = paired && place >= first ? rows - 1 - (place - first) : place;
+    const int wanted = place >= first ? rows - 1 - (place - first) : place;
     int mine[2], ahead[2] = {0, 0};
 #pragma unroll
     for (int i = 0; i < 2; ++i) mine[i] = lane + i * kWave < rows ? positions[lane + i * kWave] : -1;
+    int longest = max(mine[0], mine[1]), shortest = mine[1] < 0 ? mine[0] : min(mine[0], mine[1]);
+    if (shortest < 0) shortest = 0x7fffffff;                   // (no row)
+#pragma unroll
+    for (int off = kWave / 2; off > 0; off >>= 1) {
+        longest = max(longest, __shfl_xor(longest, off, kWave));
+        shortest = min(shortest, __shfl_xor(shortest, off, kWave));
+    }
+    if (longest - shortest < kEvenKeys) return place;
 #pragma unroll
     for (int i = 0; i < 2; ++i)
         for (int o = 0; o < kWave && o + i * kWave < rows; ++o) {
@@ -690,7 +699,8 @@ static void launch_decode(const void* q, const void* k_pool, const void* v_pool,
     dim3 grid(rows, kv_heads * ((group + 15) / 16), splits);
     const size_t smem = decode_smem_bytes(kD16 * 16, group, max_blocks);
     // (Where keys are shared out over splits, rows are even enough: ranking them cost 11 rows of 150 to 3,000 keys 0.7 us a call.)
-    const int ordered = rows > 1 && rows <= kOrderedRows && grid.z == 1 && static_cast<long>(grid.x) * grid.y > kOrderedUnits ? 1 : 0;
+    const long blocks = static_cast<long>(grid.x) * grid.y;
+    const int ordered = rows > 1 && rows <= kOrderedRows && grid.z == 1 && blocks > kOrderedUnits && blocks <= 2 * kOrderedUnits ? 1 : 0;
     const float to_log2 = scale * 1.4426950408889634f;
     if constexpr (kD16 % 4 == 0) {
         if (from != nullptr) {

@@ -62,3 +62,16 @@ def test_the_rows_own_key_at_every_place_of_a_tile(dim, group, planes):
     for splits in (1, 2):
         got, want = projected(lengths, 2, group, dim, planes, splits, seed=dim)
         assert bool(torch.isfinite(got.float()).all()) and torch.equal(got, want)
+
+
+# ranked: up to two workgroups a unit and lengths more than 1,024 apart; one key less and it is not
+@pytest.mark.parametrize("rows,kv_heads", [(33, 8), (64, 8), (65, 5), (128, 4)])
+def test_rows_of_very_different_lengths(rows, kv_heads):
+    gen = torch.Generator().manual_seed(rows)
+    lengths = torch.randint(2, 1100, (rows,), generator=gen).tolist()
+    lengths[rows // 2:rows // 2 + 2] = [77, 77]
+    for longest in (1024, 1025, 1200):
+        lengths[0], lengths[-1] = longest, 1
+        lengths[1:-1] = [min(n, longest) for n in lengths[1:-1]]
+        got, want = projected(lengths, kv_heads, 2, 64, 0, 1)
+        assert torch.equal(got, want)
