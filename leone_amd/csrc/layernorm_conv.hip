@@ -309,7 +309,7 @@ __global__ void causal_conv_state_kernel(const TIn* __restrict__ in, long in_str
 }
 
 // One wave per (row, head).
-template <typename TOut>
+template <typename TOut, int kKept>
 __global__ void head_norm_gate_kernel(const float* __restrict__ o, const float* __restrict__ dot, const float* __restrict__ top,
                                       AnyVec gain, int gain_per_head, const float* __restrict__ gate, long gate_stride,
                                       int act, float eps, TOut* __restrict__ out, int heads, int vdim, int gate_first) {
@@ -322,7 +322,7 @@ __global__ void head_norm_gate_kernel(const float* __restrict__ o, const float* 
     const float* gate_row = gate ? gate + static_cast<long>(row) * gate_stride + static_cast<long>(head) * vdim : nullptr;
     // Few rows are a chain of trips to memory: the run, its gate, its gains and what divides it are asked for side by side
     // (at indexes held inside the run, so that no branch stands between the loads).  Eight rows of four heads of 512: 4.8 us (8.8 before).
-    constexpr int kKept = 8;                                   // values a lane keeps between the two passes
+    // kKept: the values a lane keeps between the two passes.
     const long gain_at = gain_per_head ? static_cast<long>(head) * vdim : 0;
     float kept[kKept], open[kKept] = {}, by[kKept];
     const float read = dot ? dot[at] : 0.f, highest = dot ? top[at] : 0.f;
@@ -628,12 +628,16 @@ extern "C" int leone_head_norm_gate_ordered(const float* o, const float* dot, co
         return 0;
     }
     const dim3 grid(rows, ceil_div(heads, 4));
-    if (out_dtype == kF32)
-        head_norm_gate_kernel<float><<<grid, 4 * kWave, 0, stream>>>(o, dot, top, vg, gain_per_head, gate, gate_stride, act, eps,
-                                                                     static_cast<float*>(out), heads, vdim, gate_first);
-    else
-        head_norm_gate_kernel<bf16_t><<<grid, 4 * kWave, 0, stream>>>(o, dot, top, vg, gain_per_head, gate, gate_stride, act, eps,
-                                                                      static_cast<bf16_t*>(out), heads, vdim, gate_first);
+    // Heads of 64 and 128 hold one and two values a lane: asking for eight reads the same ones again (us, 2,048 rows of 32 heads of
+    // 64, eight and one: 26.8 and 19.6; 16 of 128, eight and two: 17.9 and 14.1).
+#define LEONE_HEAD(T, KEPT)                                                                                                    \
+    head_norm_gate_kernel<T, KEPT><<<grid, 4 * kWave, 0, stream>>>(o, dot, top, vg, gain_per_head, gate, gate_stride, act, eps, \
+                                                                   static_cast<T*>(out), heads, vdim, gate_first)
+#define LEONE_HEAD_KEPT(T) (vdim <= kWave ? LEONE_HEAD(T, 1) : vdim <= 2 * kWave ? LEONE_HEAD(T, 2) : LEONE_HEAD(T, 8))
+    if (out_dtype == kF32) LEONE_HEAD_KEPT(float);
+    else LEONE_HEAD_KEPT(bf16_t);
+#undef LEONE_HEAD_KEPT
+#undef LEONE_HEAD
     LEONE_LAUNCH_CHECK("head_norm_gate");
     return 0;
 }
