@@ -128,7 +128,8 @@ __device__ inline void load_projection8(const FromProjection& f, long row_width,
 
 // kD16 = head_dim / 16.
 // Two tiles of keys and values are held at a time (one on its way, one being worked on): up to a head size of
-// 64 that fits three waves a SIMD, up to 128 two; larger heads need all registers.
+// 64 that fits three waves a SIMD (four would spill: 64 rows of 8 heads at 1,000 keys 40 us instead of 26), up to 176 two; larger heads need
+// all registers.
 // Scores that fall with the distance (slopes float [q_heads] or null: head h's score at distance d is lowered by
 // slopes[h] * d) and queries that count more the further on they stand (temp_every > 0: the row's scores times
 // 1 + temp_coef * ln(floor((pos + 1) / temp_every) + 1)).
@@ -178,7 +179,7 @@ __device__ inline int ordered_row(const int* __restrict__ positions, int rows, i
 
 // kShaped: capped scores, sinks, results turned back (ScoreShape); without it none of that is in the kernel.
 template <int kD16, bool kFused, bool kShaped>
-__global__ void __launch_bounds__(kDecodeThreads, kD16 <= 4 ? 3 : kD16 <= 8 ? 2 : 1)
+__global__ void __launch_bounds__(kDecodeThreads, kD16 <= 4 ? 3 : kD16 <= 11 ? 2 : 1)
 attention_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_pool,
                         const bf16_t* __restrict__ v_pool, const int* __restrict__ positions,
                         const int* __restrict__ row_entry, const int* __restrict__ block_table, int max_blocks,
