@@ -1870,17 +1870,19 @@ def _expert_tiles(x: torch.Tensor, rows: int, top: int, experts: int, hidden: in
     """(pairs a tile, tiles at most, tile_expert, tile_pairs) for a step of ``rows`` rows."""
     pairs = rows * top
     # bfloat16 with inner sizes in runs of 8 goes to the matrix cores: the more pairs an expert gets on average, the larger the
-    # tiles (its matrices are read once a tile); anything else in tiles of the plain kernel's size.  Both products, us:
-    #   tiles of 16 and 64: 32 experts of 1,024 x 512, 6 pairs an expert 31 and 32, 11 pairs 36 and 35; of 2,048 x 768, 3 pairs 66 and 61, 11 pairs
-    #   84 and 71; of 4,096 x 1,024, 4 pairs 168 and 187, 6 pairs 181 and 189, 11 pairs 208 and 189; 64 of 2,048 x 1,408, 3 pairs 220 and
-    #   225, 6 pairs 244 and 228, 11 pairs 287 and 232; but where tiles of 64 do not give every unit a workgroup, 8 of 1,024 x 4,096, 6 pairs
-    #   50 and 67, 12 pairs 55 and 70, 16 pairs 83 and 74
-    #   tiles of 64 and 128: 32 of 2,048 x 768, 200 pairs 188 and 182, 300 pairs 247 and 257, 500 pairs 388 and 351; of 4,096 x 1,024, 200 pairs 436 and 368,
-    #   256 pairs 509 and 495; 128 of 2,048 x 768, 300 pairs 956 and 912; but of 1,024 x 512, 500 pairs 160 and 178, 700 pairs 212 and 217
+    # tiles (its matrices are read once a tile); anything else in tiles of the plain kernel's size.  Both products, matrices from
+    # memory, us:
+    #   tiles of 16 and 64: 32 experts of 1,024 x 512, 8 pairs an expert 38 and 38, 11 pairs 42 and 41; 34 of 2,048 x 768, 6 pairs 86 and 88, 8 pairs
+    #   89 and 88, 11 pairs 95 and 89; 64 of 2,048 x 1,408, 8 pairs 259 and 231; 32 of 4,096 x 1,024, 4 pairs 168 and 188, 8 pairs 197
+    #   and 188; but where tiles of 64 do not give every unit a workgroup, 8 of 1,024 x 4,096, 11 pairs 69 and 94, 16 pairs 101 and 94
+    #   tiles of 64 and 128, by the work of a matrix: 34 of 2,048 x 768, 300 pairs (16e9 products) 257 and 269, 500 pairs (27e9) 395 and
+    #   348; 8 of 4,096 x 2,048, 200 pairs (13e9) 231 and 239, 300 pairs (21e9) 282 and 247; 64 of 2,048 x 1,408, 160 pairs (30e9) 476 and 473,
+    #   200 pairs (37e9) 570 and 517; 8 of 1,024 x 4,096, 500 pairs (17e9) 229 and 234, 700 pairs (23e9) 290 and 259
     if x.dtype == torch.bfloat16 and hidden % 8 == 0 and ff % 8 == 0:
-        fills = experts * -(-hidden // 128) >= compute_units(x.device)
         each = pairs / experts
-        tile = 128 if each >= (200 if hidden > 1024 else 700) else 64 if each >= (6 if fills else 14) else 16
+        fills = experts * -(-hidden // 128) >= compute_units(x.device)
+        few = 14 if not fills else 12 if hidden <= 1024 else 8
+        tile = 128 if each >= 160 and pairs * hidden * ff >= 20e9 else 64 if each >= few else 16
     else:
         tile = library().leone_moe_tile_pairs()
     max_tiles = min(pairs, pairs // tile + experts)

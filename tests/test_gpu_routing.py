@@ -91,18 +91,28 @@ def test_products_in_tiles_of_sixty_four(counts, hidden, ff, gated):
         assert float((got - want).norm() / want.norm()) < 2e-3
 
 
-@pytest.mark.parametrize("counts,hidden,ff", [((1283, 127), 72, 136), ((128, 1300, 0, 1401), 136, 64), ((1401,), 8, 200)])
+@pytest.mark.parametrize("counts,hidden,ff", [((127, 128, 129, 256, 0, 1, 300), 72, 136), ((65, 257), 136, 64), ((200,), 8, 200)])
 @pytest.mark.parametrize("gated", [True, False])
-def test_products_in_tiles_of_a_hundred_and_twenty_eight(counts, hidden, ff, gated):
-    """As above where an expert gets many."""
+def test_products_in_tiles_of_a_hundred_and_twenty_eight(counts, hidden, ff, gated, monkeypatch):
+    """As above, at sizes too small for these tiles by the rule."""
+    from leone_amd import ops
+    kinds = []
+
+    def tiles(x, rows, top, experts, hidden, ff):
+        most = min(rows * top, rows * top // 128 + experts)
+        kinds.append(most)
+        return 128, most, torch.empty(most, dtype=torch.int32, device=DEV), torch.empty(most, 128, dtype=torch.int32, device=DEV)
+    monkeypatch.setattr(ops, "_expert_tiles", tiles)
     test_products_in_tiles_of_sixty_four(counts, hidden, ff, gated)
+    assert kinds
 
 
 def test_tiles_by_pairs_and_width():
     """The size of a tile by the pairs an expert gets on average, the width, and whether tiles of 64 give every unit a workgroup."""
     from leone_amd import ops
-    for hidden, experts, lines in ((1024, 32, (6, 700)), (2048, 32, (6, 200)), (4096, 8, (6, 200)), (1024, 8, (14, 700))):
+    for hidden, experts, ff, lines in ((1024, 32, 512, (12, 1193)), (2048, 34, 768, (8, 374)), (4096, 8, 2048, (8, 299)), (1024, 8, 4096, (14, 597)),
+                                       (2048, 128, 768, (8, 160))):
         for line, below, above in zip(lines, (16, 64), (64, 128)):
             x = torch.empty(1, hidden, dtype=torch.bfloat16, device=DEV)
-            assert ops._expert_tiles(x, line * experts - 1, 1, experts, hidden, 512)[0] == below
-            assert ops._expert_tiles(x, line * experts, 1, experts, hidden, 512)[0] == above
+            assert ops._expert_tiles(x, (line - 1) * experts, 1, experts, hidden, ff)[0] == below
+            assert ops._expert_tiles(x, line * experts, 1, experts, hidden, ff)[0] == above
