@@ -481,10 +481,15 @@ __device__ inline moe_bf16x8 moe_zero8() {
 // its bytes are the bound.  A workgroup takes 16 rows of the matrix (gated: and their up rows) and its four waves share out
 // the inner size, each with eight steps of 32 on their way at a time; their sums meet in shared memory, in the waves' order.
 // (A wave that walked the whole inner size by itself had a quarter of the loads in flight and four times the chain.)
-// The loads are ordinary ones: each is half of a line in 16 rows, whose other half a load behind it takes from the cache, and marked
-// as not to be kept (as where the weights are streamed in whole lines) lines came twice.  Both products of 32 experts of 2,048 x 768, us,
-// marked and not: four rows 42 and 35, eight 65 and 56; 8 experts of 4,096 x 2,048, four rows 99 and 68.
-template <int kMode>
+// Eight rows of 2,048 over 34 experts of 768, four routed places and two for every row (us, before): gated 38 (47), down 19 (24).
+//
+// A load is half of a line in 16 rows; the other half comes with the load behind it.  kStreamed: loads marked as not to be kept, which
+// leaves the caches to others (a decoding step of a model with 32 experts of 2,048 x 768: 6.96 ms, unmarked 7.09, its first products alone unmarked
+// 7.14); with longer rows some lines came twice (32 experts of 4,096 x 1,024, both products, 16 rows 172 us, the first one
+// unmarked 158; 8 of 1,024 x 4,096, eight rows 58, the second one unmarked 46 to 56).
+constexpr int kStreamedInner = 2048;
+
+template <int kMode, bool kStreamed>
 __global__ void __launch_bounds__(kMoeThreads, 3)
 moe_product_stream_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, void* __restrict__ y,
                           const float* __restrict__ pair_weight, const int* __restrict__ tile_expert,
@@ -507,13 +512,14 @@ moe_product_stream_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict
     const int last = (wave + 1) * share < steps ? (wave + 1) * share : steps;
     moe_floatx4 acc = {0.f, 0.f, 0.f, 0.f}, acc2 = {0.f, 0.f, 0.f, 0.f};
     moe_bf16x8 a[kDepth], a2[kGated ? kDepth : 1], xb[kDepth];
+    const auto weights = [](const bf16_t* p) { return kStreamed ? __builtin_bit_cast(moe_bf16x8, load_streamed16(p)) : moe_load8(p); };
 #define LEONE_MOE_FETCH(D, S)                                                                                  \
     {                                                                                                          \
         const int at = 32 * (S) + 8 * g;                                                                       \
         const bool in = (S) < last && at < k;                                                                  \
-        a[D] = (row_ok && in) ? moe_load8(wa + at) : moe_zero8();        \
+        a[D] = (row_ok && in) ? weights(wa + at) : moe_zero8();        \
         if constexpr (kGated)                                                                                  \
-            a2[D] = (row_ok && in) ? moe_load8(wa + matrix + at) : moe_zero8(); \
+            a2[D] = (row_ok && in) ? weights(wa + matrix + at) : moe_zero8(); \
         xb[D] = (pair >= 0 && in) ? moe_load8(xrow + at) : moe_zero8();                                        \
     }
 #pragma unroll
@@ -958,9 +964,12 @@ extern "C" int leone_moe_product(const void* x, const void* w, void* y, const fl
         if (tile == 16) {
             const dim3 grid(max_tiles, ceil_div(n, 16));
             LEONE_REQUIRE(grid.y <= 65535, "moe_product: %d rows of a matrix are too many", n);
-#define LEONE_MOE_STREAM(MODE)                                                                                            \
-    moe_product_stream_kernel<MODE><<<grid, kMoeThreads, 0, stream>>>(static_cast<const bf16_t*>(x), static_cast<const bf16_t*>(w), \
-                                                                      y, pair_weight, tile_expert, tile_pairs, top, n, k, act, limit)
+            const bool streamed = k <= kStreamedInner;
+#define LEONE_MOE_STREAM(MODE)                                                                                                 \
+    (streamed ? moe_product_stream_kernel<MODE, true><<<grid, kMoeThreads, 0, stream>>>(                                      \
+                    static_cast<const bf16_t*>(x), static_cast<const bf16_t*>(w), y, pair_weight, tile_expert, tile_pairs, top, n, k, act, limit) \
+              : moe_product_stream_kernel<MODE, false><<<grid, kMoeThreads, 0, stream>>>(                                     \
+                    static_cast<const bf16_t*>(x), static_cast<const bf16_t*>(w), y, pair_weight, tile_expert, tile_pairs, top, n, k, act, limit))
             if (gated == kMoeGated) LEONE_MOE_STREAM(kMoeGated);
             else if (gated == kMoePlain) LEONE_MOE_STREAM(kMoePlain);
             else LEONE_MOE_STREAM(kMoeDown);
