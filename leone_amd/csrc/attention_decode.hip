@@ -139,13 +139,14 @@ struct ScoreBias {
     int temp_every = 0;
 };
 
-// Which row the workgroup takes when there are more workgroups than compute units, up to two for each, and none share out a row's keys.  Rows
-// differ in length, and a unit that happens to get two long ones is what the step waits for: the rows are ranked by their
-// positions, the longest go to the first 256 workgroups, and the others start with the shortest, so that a unit's two make up for each other.  The heads of
-// a row are neighbouring workgroups, so that every die gets its share of every row.  Ranking takes 2 to 4 us, so
-// rows of about the same length stay in their own order (us, ranked and not, 32 heads over 8 of 128, 64 rows: of 100 keys 17.6 and 13.0, of 100 to 900
-// 30 and 32, of 100 to 1,700 44 and 51; 8 heads of 64, 64 rows of 100 to 900 20.1 and 19.1, of 100 to 1,700 27.8 and 28.8); with more
-// than two workgroups a unit it gains nothing (128 rows of 8 heads of 64, 100 keys 31 and 13, 100 to 1,700 62 and 60).
+// Which row the workgroup takes when there are more workgroups than compute units, up to two for each, and none share out a
+// row's keys.  Rows differ in length, and a unit that happens to get two long ones is what the step waits for: the rows are
+// ranked by their positions, the longest go to the first 256 workgroups, and the others start with the shortest, so that a
+// unit's two make up for each other.  The heads of a row are neighbouring workgroups, so that every die gets its share of every
+// row.  Ranking takes 2 to 4 us, so rows of about the same length stay in their own order (us, ranked and not, 32 heads over 8
+// of 128, 64 rows: of 100 keys 17.6 and 13.0, of 100 to 900 30 and 32, of 100 to 1,700 44 and 51; 8 heads of 64, 64 rows of 100
+// to 900 20.1 and 19.1, of 100 to 1,700 27.8 and 28.8); with more than two workgroups a unit it gains nothing (128 rows of 8
+// heads of 64, 100 keys 31 and 16, 100 to 1,700 62 and 59).
 constexpr int kOrderedRows = 2 * kWave;
 constexpr int kOrderedUnits = 256;
 constexpr int kEvenKeys = 1024;

@@ -724,11 +724,12 @@ moe_product_tiled_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict_
     }
 }
 
-// Tiles of 128 pairs, bfloat16, where an expert gets hundreds: 128 rows of the matrix (gated: and their up rows), whose chunks lie
-// in shared memory as above, one at a time, the next on its way in registers.  The four waves take 64 rows x 64 pairs each, four and four
-// operands (gated: eight and four) for 16 (32) matrix instructions, and a matrix is read half as often: with many tiles an expert that
-// counts for more than chunks in flight.  Both products, us, tiles of 64 and of 128: 32 experts of 2,048 x 768, 300 pairs an expert 247 and 257, 500 388
-// and 351, 700 533 and 468; of 4,096 x 1,024, 500 910 and 790; 64 of 2,048 x 1,408, 700 1594 and 1332.
+// Tiles of 128 pairs, bfloat16, where an expert gets hundreds: 128 rows of the matrix (gated: and their up rows), whose chunks
+// lie in shared memory as above, one at a time, the next on its way in registers.  The four waves take 64 rows x 64 pairs each,
+// four and four operands (gated: eight and four) for 16 (32) matrix instructions, and a matrix is read half as often: with many
+// tiles an expert that counts for more than chunks in flight.  Both products, us, tiles of 64 and of 128: 32 experts of 2,048 x
+// 768, 300 pairs an expert 247 and 257, 500 388 and 351, 700 533 and 468; of 4,096 x 1,024, 500 910 and 790; 64 of 2,048 x
+// 1,408, 700 1594 and 1332.
 constexpr int kWidePairs = 128;
 constexpr int kWideRows = 128;
 
