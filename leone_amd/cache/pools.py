@@ -5,6 +5,8 @@ from typing import Dict, List, Union
 
 import torch
 
+from ..ops.state import StateSlots
+from ..parts.base import StateNeed
 from ..parts.context import CacheView
 from .manager import GroupSpec
 
@@ -39,6 +41,10 @@ class DevicePools:
                 self.group_of_slot[slot] = [n.group_key() for n in self.group_needs].index(key)
             else:
                 self.state[slot] = need.allocate_slots(max_requests, self.device)
+        # The state that is one plain tensor is moved by one launch for all of it; any other need moves its own.
+        plain = [slot for slot, storage in self.state.items() if type(needs[slot]) is StateNeed and StateSlots.takes(storage)]
+        self._slots = StateSlots([self.state[slot] for slot in plain]) if plain else None
+        self._others = {slot: storage for slot, storage in self.state.items() if slot not in plain}
         self.group_specs: List[GroupSpec] = []
         for gi, need in enumerate(self.group_needs):
             pages = num_pages[gi] if isinstance(num_pages, dict) else num_pages
@@ -67,28 +73,40 @@ class DevicePools:
         return out
 
     def zero_state(self, slot_index: int) -> None:
-        for slot, storage in self.state.items():
+        if self._slots is not None:
+            self._slots.zero([slot_index])
+        for slot, storage in self._others.items():
             self.needs[slot].zero(storage, slot_index)
 
     def copy_state(self, from_slot: int, to_slot: int) -> None:
         """Gives request slot ``to_slot`` a copy of what ``from_slot`` holds (a request that takes over another's
-        prefix at the other's latest position), through the needs' own ``snapshot`` and ``restore``."""
+        prefix at the other's latest position); needs of other kinds through their own ``snapshot`` and ``restore``."""
+        if self._slots is not None:
+            self._slots.copy(from_slot, to_slot)
+        if not self._others:
+            return
         source = torch.tensor([from_slot], dtype=torch.long, device=self.device)
         target = torch.tensor([to_slot], dtype=torch.long, device=self.device)
-        for slot, storage in self.state.items():
+        for slot, storage in self._others.items():
             self.needs[slot].restore(storage, target, self.needs[slot].snapshot(storage, source))
 
     def snapshot_state(self, slot_indices: List[int]):
         """What the per-request storage of these request slots holds, to be put back by ``restore_state``."""
         if not self.state:
             return None
-        index = torch.tensor(sorted(set(slot_indices)), dtype=torch.long, device=self.device)
-        return index, {slot: self.needs[slot].snapshot(storage, index) for slot, storage in self.state.items()}
+        slots = sorted(set(slot_indices))
+        packed = self._slots.save(slots) if self._slots is not None else None
+        if not self._others:
+            return slots, packed, None, {}
+        index = torch.tensor(slots, dtype=torch.long, device=self.device)
+        return slots, packed, index, {slot: self.needs[slot].snapshot(storage, index) for slot, storage in self._others.items()}
 
     def restore_state(self, saved) -> None:
         if saved is None:
             return
-        index, kept = saved
+        slots, packed, index, kept = saved
+        if packed is not None:
+            self._slots.restore(slots, packed)
         for slot, value in kept.items():
             self.needs[slot].restore(self.state[slot], index, value)
 

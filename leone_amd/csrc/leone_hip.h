@@ -493,4 +493,9 @@ int leone_time_mix_read(const float* r, long stride, const float* decay, const i
 // The weight-streaming product of several inputs against matrices that lie together (see gemm_fused.hip).
 int leone_gemm_planes_bf16(const void* x, int planes, int plane_rows, const void* w, int w_tiled, void* y, int out_dtype, int m,
                            int n, int k, hipStream_t stream);
+// Request slots of many state tensors cleared, copied, saved and put back in one launch (see state_slots.hip).
+int leone_state_chunk();
+int leone_state_slots_max();
+int leone_state_slots(const void* table, int tensors, long chunks, int move, const int* ids, const int* to, int count, void* packed,
+                      long packed_bytes, hipStream_t stream);
 }

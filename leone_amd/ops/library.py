@@ -23,6 +23,7 @@ _lib: ctypes.CDLL | None = None
 P = c_void_p
 _PROTOTYPES = {
     "leone_embed": [P, c_int, P, P, c_int, c_int, c_int, c_float, P],
+    "leone_state_slots": [P, c_int, ctypes.c_long, c_int, P, P, c_int, P, ctypes.c_long, P],
     "leone_soft_cap": [P, ctypes.c_long, c_float, P],
     "leone_add_rmsnorm": [P, P, c_int, c_int, ctypes.c_long, P, c_int, c_float, P, c_int, P, c_int, c_int, P, P],
     "leone_swiglu": [P, P, c_int, c_int, c_int, P],
@@ -165,6 +166,10 @@ def library() -> ctypes.CDLL:
             lib.leone_top_candidates_max.argtypes = []
             lib.leone_argmax_chunk.restype = c_int
             lib.leone_argmax_chunk.argtypes = []
+            lib.leone_state_chunk.restype = c_int
+            lib.leone_state_chunk.argtypes = []
+            lib.leone_state_slots_max.restype = c_int
+            lib.leone_state_slots_max.argtypes = []
             lib.leone_gemm_f32_planes.restype = c_int
             lib.leone_gemm_f32_planes.argtypes = [c_int, c_int, c_int]
             lib.leone_sample_truncated_stages.restype = c_int
