@@ -160,11 +160,8 @@ __device__ inline int ordered_row(const int* __restrict__ positions, int rows, i
     for (int i = 0; i < 2; ++i) mine[i] = lane + i * kWave < rows ? positions[lane + i * kWave] : -1;
     int longest = max(mine[0], mine[1]), shortest = mine[1] < 0 ? mine[0] : min(mine[0], mine[1]);
     if (shortest < 0) shortest = 0x7fffffff;                   // (no row)
-#pragma unroll
-    for (int off = kWave / 2; off > 0; off >>= 1) {
-        longest = max(longest, __shfl_xor(longest, off, kWave));
-        shortest = min(shortest, __shfl_xor(shortest, off, kWave));
-    }
+    longest = join_span<kWave>(longest, [](int a, int b) { return max(a, b); });
+    shortest = join_span<kWave>(shortest, [](int a, int b) { return min(a, b); });
     if (longest - shortest < kEvenKeys) return place;
 #pragma unroll
     for (int i = 0; i < 2; ++i)
@@ -357,8 +354,8 @@ attention_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__
                 for (int s = 0; s < kSteps; ++s)
 #pragma unroll
                     for (int i = 0; i < 8; ++i) ss = fmaf(head_run[s][i], head_run[s][i], ss);
-                ss += __shfl_xor(ss, 16, kWave);              // the four lanes that share head c
-                ss += __shfl_xor(ss, 32, kWave);
+                ss = add_lanes<16>(ss);              // the four lanes that share head c
+                ss = add_lanes<32>(ss);
             } else {
                 // A key's squares are added in the separate kernel's order (a run's elements in turn with their partners', the
                 // runs' sums by halves), so that the cache holds the same bits whichever of the two wrote it.
@@ -372,8 +369,8 @@ attention_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__
                         runs[s] = fmaf(head_run[s + kHalfSteps][i], head_run[s + kHalfSteps][i], runs[s]);
                     }
                 ss = (runs[0] + runs[2]) + (runs[1] + runs[3]);
-                ss += __shfl_xor(ss, 32, kWave);
-                ss += __shfl_xor(ss, 16, kWave);
+                ss = add_lanes<32>(ss);
+                ss = add_lanes<16>(ss);
             }
             if (gain.ptr) {
                 const float inv = 1.0f / sqrtf(ss / static_cast<float>(kD) + from.eps);
@@ -513,8 +510,8 @@ attention_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__
             sc[j] = (full || in_reach(key)) ? fmaf(raw, kShaped && shape.cap > 0.f ? 1.0f : to_log2_row, slope_log2 * static_cast<float>(key - (n - 1))) : -INFINITY;
             tile_max = fmaxf(tile_max, sc[j]);
         }
-        tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 16, kWave));
-        tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 32, kWave));
+        tile_max = max_lanes<16>(tile_max);
+        tile_max = max_lanes<32>(tile_max);
         const float m_new = fmaxf(m_run, ceilf(tile_max));   // finite: every tile of the range holds a key in reach
         const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);   // an exact power of two (0 from -inf)
         float psum = 0.f;
@@ -524,8 +521,8 @@ attention_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__
             pt[j] = static_cast<__bf16>(__builtin_amdgcn_exp2f(sc[j] - m_new));
             psum += static_cast<float>(pt[j]);
         }
-        psum += __shfl_xor(psum, 16, kWave);
-        psum += __shfl_xor(psum, 32, kWave);
+        psum = add_lanes<16>(psum);
+        psum = add_lanes<32>(psum);
         l_run = l_run * alpha + psum;
         m_run = m_new;
         // ---- O^T += V^T . P^T ------------------------------------------------------------------

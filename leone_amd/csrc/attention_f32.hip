@@ -91,12 +91,8 @@ __global__ void __launch_bounds__(kWaves * kWave, kDim == 64 ? 3 : 2) attention_
     for (int i = 0; i < kRuns; ++i) q[i] = *reinterpret_cast<const f32x4*>(qr + i * 16 + h);
 
     // what the rows together see: tiles of 16 keys from the earliest row's first one on, and those of the kept first keys
-    int low = first, high = pos;
-#pragma unroll
-    for (int off = 8; off > 0; off >>= 1) {
-        low = min(low, __shfl_xor(low, off, kWave));
-        high = max(high, __shfl_xor(high, off, kWave));
-    }
+    const int low = join_span<16>(first, [](int a, int b) { return min(a, b); });
+    const int high = join_span<16>(pos, [](int a, int b) { return max(a, b); });
     const int low_tile = low / kKeys;
     const int kept_tiles = min((g.keep_first + kKeys - 1) / kKeys, low_tile);
     const int tiles = high / kKeys + 1;
@@ -170,8 +166,8 @@ __global__ void __launch_bounds__(kWaves * kWave, kDim == 64 ? 3 : 2) attention_
                 s[r] = seen ? (mapped ? v : __builtin_nanf("")) : -INFINITY;
                 top = fmaxf(top, s[r]);
             }
-            top = fmaxf(top, __shfl_xor(top, 16, kWave));
-            top = fmaxf(top, __shfl_xor(top, 32, kWave));
+            top = max_lanes<16>(top);
+            top = max_lanes<32>(top);
             const float m_new = fmaxf(m, top);
             const float reference = m_new == -INFINITY ? 0.f : m_new;      // nothing seen yet: every weight is 0
             const float alpha = expf(m - reference);
@@ -181,8 +177,8 @@ __global__ void __launch_bounds__(kWaves * kWave, kDim == 64 ? 3 : 2) attention_
                 s[r] = expf(s[r] - reference);
                 sum += s[r];
             }
-            sum += __shfl_xor(sum, 16, kWave);
-            sum += __shfl_xor(sum, 32, kWave);
+            sum = add_lanes<16>(sum);
+            sum = add_lanes<32>(sum);
             l = l * alpha + sum;
             m = m_new;
             if (!mapped || start + kKeys > high + 1) {       // places nobody has written: their weight is 0, but not what they may hold

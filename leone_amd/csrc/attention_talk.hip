@@ -601,8 +601,8 @@ attention_talk_prefill_kernel(TalkArgs a, const int* __restrict__ tiles, int n_t
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
                         float top = fmaxf(fmaxf(d[0][i], d[1][i]), fmaxf(d[2][i], d[3][i]));
-                        top = fmaxf(top, __shfl_xor(top, 16, kWave));
-                        top = fmaxf(top, __shfl_xor(top, 32, kWave));
+                        top = max_lanes<16>(top);
+                        top = max_lanes<32>(top);
                         if (g == 0) smax[(wave * kH + 4 * b + i) * 16 + c] = top;
                     }
                 } else {
@@ -703,8 +703,8 @@ attention_talk_prefill_kernel(TalkArgs a, const int* __restrict__ tiles, int n_t
     for (int w = 0; w < kHW; ++w) {
         const int h = head_of(w);
         float l = l_run[w];
-        l += __shfl_xor(l, 16, kWave);
-        l += __shfl_xor(l, 32, kWave);
+        l = add_lanes<16>(l);
+        l = add_lanes<32>(l);
         if (poisoned) l = __builtin_nanf("");
         if (out0 + h >= heads || c >= rows) continue;
         const long rh = (static_cast<long>(row0) + c) * heads + out0 + h;

@@ -261,10 +261,10 @@ __global__ void __launch_bounds__(kChunkThreads, 2) chunk_prepare_kernel(ChunkAr
                 qq = fmaf(sq[t * row_p + i], sq[t * row_p + i], qq);
                 kk = fmaf(sk[t * row_p + i], sk[t * row_p + i], kk);
             }
-            qq += __shfl_xor(qq, 1, kWave);
-            kk += __shfl_xor(kk, 1, kWave);
-            qq += __shfl_xor(qq, 2, kWave);
-            kk += __shfl_xor(kk, 2, kWave);
+            qq = add_lanes<1>(qq);
+            kk = add_lanes<1>(kk);
+            qq = add_lanes<2>(qq);
+            kk = add_lanes<2>(kk);
         }
         if (sub == 0) {
             q_norm[t] = kDelta ? p.q_scale / sqrtf(qq + p.unit_eps) : p.q_scale;
@@ -421,10 +421,10 @@ __global__ void __launch_bounds__(kChunkThreads, 1) chunk_prepare_channel_kernel
             qq = fmaf(sq[t * row_p + i], sq[t * row_p + i], qq);
             kk = fmaf(sk[t * row_p + i], sk[t * row_p + i], kk);
         }
-        qq += __shfl_xor(qq, 1, kWave);
-        kk += __shfl_xor(kk, 1, kWave);
-        qq += __shfl_xor(qq, 2, kWave);
-        kk += __shfl_xor(kk, 2, kWave);
+        qq = add_lanes<1>(qq);
+        kk = add_lanes<1>(kk);
+        qq = add_lanes<2>(qq);
+        kk = add_lanes<2>(kk);
         if (sub == 0) {
             q_norm[t] = p.q_scale / sqrtf(qq + p.unit_eps);
             k_norm[t] = p.k_scale / sqrtf(kk + p.unit_eps);
@@ -463,10 +463,10 @@ __global__ void __launch_bounds__(kChunkThreads, 1) chunk_prepare_channel_kernel
                 ks.z = fmaf(y.z, key[j].z, ks.z), ks.w = fmaf(y.w, key[j].w, ks.w);
             }
             float qk = (qs.x + qs.y) + (qs.z + qs.w), kk = (ks.x + ks.y) + (ks.z + ks.w);
-            qk += __shfl_xor(qk, 16, kWave);
-            kk += __shfl_xor(kk, 16, kWave);
-            qk += __shfl_xor(qk, 32, kWave);
-            kk += __shfl_xor(kk, 32, kWave);
+            qk = add_lanes<16>(qk);
+            kk = add_lanes<16>(kk);
+            qk = add_lanes<32>(qk);
+            kk = add_lanes<32>(kk);
             if (g == 0) {
                 if (block == 0) mix[4 * ((wave * 4 + wave) * kWave + 16 * (c / 4) + t) + c % 4] = t >= c ? qk : 0.f;
                 to_a[16 * t + c] = t > c ? -strength[16 * wave + t] * kk : 0.f;

@@ -95,15 +95,77 @@ __device__ inline void load_any8(const AnyVec& v, long at, float out[8]) {
     }
 }
 
+// ---- values of other lanes -----------------------------------------------------------------------------------------
+// A shuffle (ds_bpermute) is a trip through the shared-memory unit, some 60 cycles that the next addition waits for, and a wave's
+// sum is six of them one after the other.  Lanes of the same row of 16 are reached by an operand's own permutation (DPP) instead,
+// the other rows and halves by the lane swaps: a few cycles each.  Which lanes meet, and in which order, is the shuffles', so the
+// results are the same bits.  Every lane of the wave has to take part.
+//
+// A lane's value and that of lane ^ kOff, in an order that may differ between the two: for operations that do not mind it.
+template <typename T>
+struct Pair {
+    T a, b;
+};
+template <int kOff, typename T>
+__device__ inline Pair<T> lane_pair(T v) {
+    static_assert(kOff == 1 || kOff == 2 || kOff == 4 || kOff == 8 || kOff == 16 || kOff == 32, "a power of two");
+    static_assert(sizeof(T) == 4 || sizeof(T) == 8, "one register or two");
+    if constexpr (sizeof(T) == 8) {
+        typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+        const u32x2 own = __builtin_bit_cast(u32x2, v);
+        const Pair<unsigned> low = lane_pair<kOff>(own[0]), high = lane_pair<kOff>(own[1]);
+        return {__builtin_bit_cast(T, u32x2{low.a, high.a}), __builtin_bit_cast(T, u32x2{low.b, high.b})};
+    } else {
+        const unsigned own = __builtin_bit_cast(unsigned, v);
+        if constexpr (kOff >= 16) {
+            // of every two rows (or of the two halves), the first one's values here and the second one's there
+            typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+            u32x2 both;
+            if constexpr (kOff == 32) both = __builtin_amdgcn_permlane32_swap(own, own, false, false);
+            else both = __builtin_amdgcn_permlane16_swap(own, own, false, false);
+            const unsigned first = both[0], second = both[1];       // (a bit_cast of a vector's element takes the vector's first)
+            return {__builtin_bit_cast(T, first), __builtin_bit_cast(T, second)};
+        } else {
+            constexpr int kRotate8 = 0x128, kShl4 = 0x104, kShr4 = 0x114, kSwap1 = 0xb1, kSwap2 = 0x4e;
+            int other;
+            if constexpr (kOff == 4) {       // the first and third four lanes take from four above, the others from four below
+                other = __builtin_amdgcn_update_dpp(own, own, kShl4, 0xf, 0x5, false);
+                other = __builtin_amdgcn_update_dpp(other, own, kShr4, 0xf, 0xa, false);
+            } else {
+                other = __builtin_amdgcn_update_dpp(own, own, kOff == 8 ? kRotate8 : kOff == 2 ? kSwap2 : kSwap1, 0xf, 0xf, false);
+            }
+            return {v, __builtin_bit_cast(T, other)};
+        }
+    }
+}
+template <int kOff, typename T, typename Op>
+__device__ inline T join_lanes(T v, Op op) {
+    const Pair<T> both = lane_pair<kOff>(v);
+    return op(both.a, both.b);
+}
+template <int kOff>
+__device__ inline float add_lanes(float v) {
+    return join_lanes<kOff>(v, [](float a, float b) { return a + b; });
+}
+template <int kOff>
+__device__ inline float max_lanes(float v) {
+    return join_lanes<kOff>(v, [](float a, float b) { return fmaxf(a, b); });
+}
+// Over every kSpan neighbouring lanes, the furthest apart first; each of them gets the result.
+template <int kSpan, typename T, typename Op>
+__device__ inline T join_span(T v, Op op) {
+    if constexpr (kSpan == 1) return v;
+    else return join_span<kSpan / 2>(join_lanes<kSpan / 2>(v, op), op);
+}
+template <int kSpan>
+__device__ inline float add_span(float v) {
+    return join_span<kSpan>(v, [](float a, float b) { return a + b; });
+}
 __device__ inline float wave_sum(float v) {
-#pragma unroll
-    for (int off = kWave / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, kWave);
-    return v;
+    return join_span<kWave>(v, [](float a, float b) { return a + b; });
 }
 __device__ inline float wave_max(float v) {
-#pragma unroll
-    for (int off = kWave / 2; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, kWave));
-    return v;
+    return join_span<kWave>(v, [](float a, float b) { return fmaxf(a, b); });
 }
 
 // Sum over a block of kThreads (a multiple of 64, at most 1024); every thread

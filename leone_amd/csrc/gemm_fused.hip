@@ -205,8 +205,8 @@ gemm_fused_kernel(FusedArgs a) {
         }
     }
     if (kIn == kInNorm) {
-        ss += __shfl_xor(ss, 16, kWave);             // the four lanes that share X row c
-        ss += __shfl_xor(ss, 32, kWave);
+        ss = add_lanes<16>(ss);             // the four lanes that share X row c
+        ss = add_lanes<32>(ss);
         if (g == 0) squares[wave][c] = ss;
     }
     __syncthreads();
@@ -232,8 +232,8 @@ gemm_fused_kernel(FusedArgs a) {
 #pragma unroll
                 for (int u = 0; u < 8; ++u) total += (v[u].x + v[u].y) + (v[u].z + v[u].w);
             }
-            total += __shfl_xor(total, 16, kWave);
-            total += __shfl_xor(total, 32, kWave);
+            total = add_lanes<16>(total);
+            total = add_lanes<32>(total);
         } else {
 #pragma unroll
             for (int v = 0; v < kWaves; ++v) total += squares[v][c];
@@ -248,7 +248,7 @@ gemm_fused_kernel(FusedArgs a) {
         // gates, lanes g + 2 the matching ups
         floatx4 up;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) up[r] = __shfl_xor(sum[r], 32, kWave);
+        for (int r = 0; r < 4; ++r) up[r] = lane_pair<32>(sum[r]).b;      // the upper half's
         if (g < 2 && row < m) {
             bf16_t* out = static_cast<bf16_t*>(a.y) + static_cast<long>(row) * (n / 2) + n0 / 2 + 4 * g;
 #pragma unroll
@@ -273,8 +273,8 @@ gemm_fused_kernel(FusedArgs a) {
                 a.operand_out[static_cast<long>(row) * n + col + r] = from_float<bf16_t>(v * gain_after[r]);
             }
         }
-        squares += __shfl_xor(squares, 16, kWave);
-        squares += __shfl_xor(squares, 32, kWave);
+        squares = add_lanes<16>(squares);
+        squares = add_lanes<32>(squares);
         if (g == 0 && row < m) a.squares_out[static_cast<long>(row) * gridDim.x + blockIdx.x] = squares;
         return;
     }

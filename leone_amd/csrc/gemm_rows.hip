@@ -245,7 +245,7 @@ gemm_rows_kernel(RowsArgs a) {
             // g = 0, 1 hold gates, lanes g + 2 the matching ups
             floatx4 up;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) up[r] = __shfl_xor(acc[t][r], 32, kWave);
+            for (int r = 0; r < 4; ++r) up[r] = lane_pair<32>(acc[t][r]).b;      // the upper half's
             if (g < 2 && row < m && col < n) {
                 bf16_t* out = static_cast<bf16_t*>(a.y) + static_cast<long>(row) * (n / 2) + 8 * tile + 4 * g;
                 float v[4];

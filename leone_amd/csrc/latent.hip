@@ -494,8 +494,8 @@ latent_attention_cores_kernel(const bf16_t* __restrict__ q, float* __restrict__ 
                 sc[j] = (mine && key >= first && key <= pos) ? score * to_log2 : -INFINITY;
                 tile_max = fmaxf(tile_max, sc[j]);
             }
-            tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 16, kWave));
-            tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 32, kWave));
+            tile_max = max_lanes<16>(tile_max);
+            tile_max = max_lanes<32>(tile_max);
             const float m_new = fmaxf(m_run, tile_max);
             const bool none = m_new == -INFINITY;                 // a column that has seen no key yet
             const float alpha = none ? 1.f : __builtin_amdgcn_exp2f(m_run - m_new);
@@ -506,8 +506,8 @@ latent_attention_cores_kernel(const bf16_t* __restrict__ q, float* __restrict__ 
                 pt[j] = static_cast<__bf16>(none ? 0.f : __builtin_amdgcn_exp2f(sc[j] - m_new));
                 psum += static_cast<float>(pt[j]);
             }
-            psum += __shfl_xor(psum, 16, kWave);
-            psum += __shfl_xor(psum, 32, kWave);
+            psum = add_lanes<16>(psum);
+            psum = add_lanes<32>(psum);
             l_run = l_run * alpha + psum;
             m_run = m_new;
             // ---- O^T += V^T P^T ----

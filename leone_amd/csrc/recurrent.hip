@@ -444,11 +444,8 @@ __global__ void __launch_bounds__(kScanThreads) delta_scan_kernel(DeltaScanArgs 
                     qq = fmaf(qs[i], qs[i], qq);
                     kk = fmaf(ks[i], ks[i], kk);
                 }
-#pragma unroll
-                for (int off = kRowLanes / 2; off > 0; off >>= 1) {
-                    qq += __shfl_xor(qq, off, kWave);
-                    kk += __shfl_xor(kk, off, kWave);
-                }
+                qq = add_span<kRowLanes>(qq);
+                kk = add_span<kRowLanes>(kk);
                 const float qinv = p.q_scale / sqrtf(qq + p.unit_eps);
                 const float kinv = 1.0f / sqrtf(kk + p.unit_eps);
                 const float head_decay = p.per_head
@@ -559,11 +556,8 @@ __global__ void __launch_bounds__(kGroups * kWave) delta_step_kernel(DeltaScanAr
             qq = fmaf(qr[m], qr[m], qq);
             kk = fmaf(kr[m], kr[m], kk);
         }
-#pragma unroll
-        for (int off = kRowLanes / 2; off > 0; off >>= 1) {
-            qq += __shfl_xor(qq, off, kWave);
-            kk += __shfl_xor(kk, off, kWave);
-        }
+        qq = add_span<kRowLanes>(qq);
+        kk = add_span<kRowLanes>(kk);
         const float qinv = p.q_scale / sqrtf(qq + p.unit_eps);
         const float kinv = 1.0f / sqrtf(kk + p.unit_eps);
         const float gv = expf(-rate * softplus_f(step_raw + bias));

@@ -32,17 +32,15 @@ constexpr int kMoeWaves = kMoeThreads / kWave;
 constexpr int kColsPerWave = 4;
 constexpr int kMoeCols = kMoeWaves * kColsPerWave;
 
-// The better of two (value, index): the larger value, the lower index among equals.
+// The best (value, index) of a wave: the larger value, the lower index among equals; what has no index (0x7fffffff) loses.
+template <int kSpan = kWave>
 __device__ inline void wave_best(float& v, int& at) {
-#pragma unroll
-    for (int off = kWave / 2; off > 0; off >>= 1) {
-        const float v2 = __shfl_xor(v, off, kWave);
-        const int at2 = __shfl_xor(at, off, kWave);
-        if (v2 > v || (v2 == v && at2 < at)) {
-            v = v2;
-            at = at2;
-        }
-    }
+    const Pair<float> of = lane_pair<kSpan / 2>(v);
+    const Pair<int> where = lane_pair<kSpan / 2>(at);
+    const bool second = of.b > of.a || (of.b == of.a && where.b < where.a) || where.a == 0x7fffffff;
+    v = second ? of.b : of.a;
+    at = second ? where.b : where.a;
+    if constexpr (kSpan > 2) wave_best<kSpan / 2>(v, at);
 }
 
 // One wave a row; a lane holds kSlots router outputs (kSlots * 64 >= total).

@@ -478,8 +478,7 @@ qk_norm_rope_write_runs_kernel(
             ss = fmaf(b[i], b[i], ss);
         }
     }
-#pragma unroll
-    for (int off = kShare / 2; off > 0; off >>= 1) ss += __shfl_xor(ss, off, kWave);
+    ss = add_span<kShare>(ss);
     if (!mine) return;
 
     const int pos = positions[row];

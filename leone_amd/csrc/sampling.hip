@@ -30,13 +30,7 @@ __device__ inline Best better(Best a, Best b) {
 }
 
 __device__ inline Best block_best(Best mine, Best* scratch) {
-#pragma unroll
-    for (int off = kWave / 2; off > 0; off >>= 1) {
-        Best other;
-        other.value = __shfl_xor(mine.value, off, kWave);
-        other.index = __shfl_xor(mine.index, off, kWave);
-        mine = better(mine, other);
-    }
+    mine = join_span<kWave>(mine, better);
     const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
     __syncthreads();
     if (lane == 0) scratch[wave] = mine;
@@ -240,11 +234,7 @@ __device__ inline int rank_among(const unsigned long long* keys, int n, unsigned
 
 // The greatest key of the workgroup, for every thread; `scratch` holds one place a wave.
 __device__ inline unsigned long long block_max_key(unsigned long long mine, unsigned long long* scratch) {
-#pragma unroll
-    for (int off = kWave / 2; off > 0; off >>= 1) {
-        const unsigned long long other = __shfl_xor(mine, off, kWave);
-        mine = other > mine ? other : mine;
-    }
+    mine = join_span<kWave>(mine, [](unsigned long long a, unsigned long long b) { return b > a ? b : a; });
     __syncthreads();                                        // what the call before this one left has been read
     if (threadIdx.x % kWave == 0) scratch[threadIdx.x / kWave] = mine;
     __syncthreads();
@@ -320,11 +310,7 @@ __device__ inline Selection select_best(const float* __restrict__ row, int vocab
     });
     // A cell is kCellThreads neighbouring threads; its best key goes to keys[cell].
     unsigned long long best = best_id < 0 ? 0ull : candidate_key(best_value, best_id);
-#pragma unroll
-    for (int off = 1; off < kCellThreads; off <<= 1) {
-        const unsigned long long other = __shfl_xor(best, off, kWave);
-        best = other > best ? other : best;
-    }
+    best = join_span<kCellThreads>(best, [](unsigned long long a, unsigned long long b) { return b > a ? b : a; });
     if (threadIdx.x % kCellThreads == 0) keys[threadIdx.x / kCellThreads] = best;
     if (threadIdx.x == 0) {
         counters[0] = counters[1] = 0;
@@ -337,8 +323,7 @@ __device__ inline Selection select_best(const float* __restrict__ row, int vocab
         const unsigned long long mine = keys[threadIdx.x];
         if (mine != 0ull && rank_among(keys, kCandidateMaxK, mine) == k - 1) *bound_at = mine;
     }
-#pragma unroll
-    for (int off = kWave / 2; off > 0; off >>= 1) finite += __shfl_xor(finite, off, kWave);
+    finite = join_span<kWave>(finite, [](int a, int b) { return a + b; });
     if (threadIdx.x % kWave == 0) atomicAdd(&counters[1], finite);
     __syncthreads();
     const unsigned long long bound = *bound_at;
