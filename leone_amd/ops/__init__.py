@@ -1673,7 +1673,7 @@ def outer_scan(proj: torch.Tensor, columns: dict, state: torch.Tensor, step, hea
              _dev(gates["i_bias"], "i bias", None, (heads,)), _dev(gates["f_bias"], "f bias", None, (heads,)),
              _code(gates["i_bias"], "i bias"), float(gates["cap"]), _dev(spans, "spans"), spans.shape[0],
              _dev(state, "state"), state.stride(0), per_head, dim * vdim + dim, 1 if write_state else 0,
-             _dev(coef, "coefficients"), _dev(top, "top"), heads, _stream())
+             _dev(coef, "coefficients"), _dev(top, "top"), rows, heads, _stream())
     rotary_dim = 2 * cos.shape[1] if cos is not None else 0
 
     def walk(segments):

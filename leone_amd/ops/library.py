@@ -75,7 +75,7 @@ _PROTOTYPES = {
     "leone_relu_squared": [P, P, c_int, ctypes.c_long, P],
     "leone_head_gate": [P, c_int, P, ctypes.c_long, c_int, c_int, c_int, P],
     "leone_exp_gates": [P, ctypes.c_long, c_int, c_int, P, P, c_int, c_float, P, c_int, P, ctypes.c_long, ctypes.c_long,
-                        ctypes.c_long, c_int, P, P, c_int, P],
+                        ctypes.c_long, c_int, P, P, c_int, c_int, P],
     "leone_outer_scan": [P, ctypes.c_long, c_int, c_int, c_int, P, P, c_int, c_float, c_float, c_int, P, P, c_int, c_int,
                          P, P, c_int, P, ctypes.c_long, P, ctypes.c_long, ctypes.c_long, P, P, c_int, c_int, c_int, P],
     "leone_step_fits": [c_int, c_int],
