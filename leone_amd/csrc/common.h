@@ -101,6 +101,13 @@ __device__ inline void load_any8(const AnyVec& v, long at, float out[8]) {
 // the other rows and halves by the lane swaps: a few cycles each.  Which lanes meet, and in which order, is the shuffles', so the
 // results are the same bits.  Every lane of the wave has to take part.
 //
+// The value of the lane that the permutation kControl of a row's 16 lanes names (one that stays within the row).
+template <int kControl, typename T>
+__device__ inline T of_lane(T v) {
+    static_assert(sizeof(T) == 4, "one register");
+    const int own = __builtin_bit_cast(int, v);
+    return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(0, own, kControl, 0xf, 0xf, true));
+}
 // A lane's value and that of lane ^ kOff, in an order that may differ between the two: for operations that do not mind it.
 template <typename T>
 struct Pair {
@@ -127,14 +134,13 @@ __device__ inline Pair<T> lane_pair(T v) {
             return {__builtin_bit_cast(T, first), __builtin_bit_cast(T, second)};
         } else {
             constexpr int kRotate8 = 0x128, kShl4 = 0x104, kShr4 = 0x114, kSwap1 = 0xb1, kSwap2 = 0x4e;
-            int other;
             if constexpr (kOff == 4) {       // the first and third four lanes take from four above, the others from four below
-                other = __builtin_amdgcn_update_dpp(own, own, kShl4, 0xf, 0x5, false);
+                int other = __builtin_amdgcn_update_dpp(own, own, kShl4, 0xf, 0x5, false);
                 other = __builtin_amdgcn_update_dpp(other, own, kShr4, 0xf, 0xa, false);
+                return {v, __builtin_bit_cast(T, other)};
             } else {
-                other = __builtin_amdgcn_update_dpp(own, own, kOff == 8 ? kRotate8 : kOff == 2 ? kSwap2 : kSwap1, 0xf, 0xf, false);
+                return {v, of_lane<kOff == 8 ? kRotate8 : kOff == 2 ? kSwap2 : kSwap1>(v)};
             }
-            return {v, __builtin_bit_cast(T, other)};
         }
     }
 }

@@ -104,119 +104,234 @@ add_layernorm_kernel(float* __restrict__ x, const float* __restrict__ delta, Any
     }
 }
 
-// The same for few rows of up to 1,024 kPer elements.  A step of few rows is a chain of trips to memory, about two microseconds
-// each when the lines are cold: here the row, the delta, the gains, the biases, the filter's taps and the state's last inputs
-// are all asked for before the first sum (each at an index held inside the row, so that no branch stands between the loads), and
-// the row stays in registers.  One type for all of the norm's and the filter's vectors, so that a load is not followed by its
-// conversion.  Sums run in the other kernel's order: the results are the same bits.  Eight rows of 1,536 with a folded filter
-// of 4 taps, in bfloat16: 8.1 us (11.7 before).
+// Eight neighbouring elements of a row as they were loaded: a value is unpacked where it is used, so that no load is waited for by
+// its own conversion.  kVec: the row is aligned to 16 bytes and holds whole runs; else the elements one by one, at indices held
+// inside the row.
+constexpr int kRun = 8;
+template <typename T, bool kVec>
+struct Run {
+    T v[kRun];
+    __device__ inline void load(const T* __restrict__ row, int at, int length) {
+#pragma unroll
+        for (int i = 0; i < kRun; ++i) v[i] = row[at + i < length ? at + i : length - 1];
+    }
+    __device__ inline float get(int i) const { return to_float(v[i]); }
+};
+template <>
+struct Run<float, true> {
+    float4 v[2];
+    __device__ inline void load(const float* __restrict__ row, int at, int length) {
+        const float4* from = reinterpret_cast<const float4*>(row + (at < length ? at : 0));
+        v[0] = from[0];
+        v[1] = from[1];
+    }
+    __device__ inline float get(int i) const {
+        const float4 half = v[i / 4];
+        return i % 4 == 0 ? half.x : i % 4 == 1 ? half.y : i % 4 == 2 ? half.z : half.w;
+    }
+};
+template <>
+struct Run<bf16_t, true> {
+    uint4 v;
+    __device__ inline void load(const bf16_t* __restrict__ row, int at, int length) {
+        v = *reinterpret_cast<const uint4*>(row + (at < length ? at : 0));
+    }
+    __device__ inline float get(int i) const {
+        const unsigned word = i / 2 == 0 ? v.x : i / 2 == 1 ? v.y : i / 2 == 2 ? v.z : v.w;
+        return __uint_as_float(i % 2 ? word & 0xffff0000u : word << 16);
+    }
+};
+template <typename T, bool kVec>
+__device__ inline void store_run(T* __restrict__ row, int at, int length, const float (&v)[kRun]) {
+    if constexpr (!kVec) {
+#pragma unroll
+        for (int i = 0; i < kRun; ++i)
+            if (at + i < length) row[at + i] = from_float<T>(v[i]);
+    } else if (at < length) {
+        if constexpr (sizeof(T) == 4) {
+            reinterpret_cast<float4*>(row + at)[0] = float4{v[0], v[1], v[2], v[3]};
+            reinterpret_cast<float4*>(row + at)[1] = float4{v[4], v[5], v[6], v[7]};
+        } else {
+            unsigned w[kRun / 2];
+#pragma unroll
+            for (int i = 0; i < kRun / 2; ++i)
+                w[i] = bf16_bits_from_float(v[2 * i]) | static_cast<unsigned>(bf16_bits_from_float(v[2 * i + 1])) << 16;
+            *reinterpret_cast<uint4*>(row + at) = uint4{w[0], w[1], w[2], w[3]};
+        }
+    }
+}
+
+// The same for rows of up to 1,024 kPer elements, a workgroup of two waves a row, in runs of 8 elements a thread.  A step of few rows
+// is a chain of trips to memory, about two microseconds each when the lines are cold: here the row, the delta, the gains, the
+// biases, the filter's taps and the state's last inputs are all asked for before the first sum, and the row stays in registers.
+// Many rows are bound by their bytes: 16-byte accesses, every row's on their way at once.
+// Sums run in the other kernel's order with 1,024 threads, so that few rows get the bits they get there: elements 1,024 apart in
+// turn, then those 32, 16, .. 1 apart meet, then every 64's sums in turn.  The runs of 64 elements lie on the eight lanes so that
+// each of the lanes' three meetings is an operand's permutation.
+// kTaps: of the folded filter; 0: none, -1: `taps` of them, up to kHeldTaps.
+// Eight rows of 2,048 with two norms and a filter of 4 taps, in bfloat16: 6.1 us (7.8 with 1,024 threads of single elements);
+// 2,048 rows with two norms 13.9 (25.8).
 constexpr int kHeldTaps = 4;
-template <typename TOut, typename TW, int kPer>
-__global__ void __launch_bounds__(kNormThreadsFew)
+constexpr int kHeldThreads = 128;
+template <typename TOut, typename TW, bool kVec, int kPer, int kTaps>
+__global__ void __launch_bounds__(kHeldThreads)
 add_layernorm_held_kernel(float* __restrict__ x, const float* __restrict__ delta, const TW* __restrict__ dw, const TW* __restrict__ db,
                           float deps, const TW* __restrict__ w, const TW* __restrict__ b, float eps, TOut* __restrict__ y,
                           const int* __restrict__ rows, int hidden, const TW* __restrict__ conv, int taps, float* conv_state,
                           int write_state, const int* __restrict__ positions, const int* __restrict__ row_entry,
                           const int* __restrict__ entry_slots) {
-    __shared__ float scratch[kNormThreadsFew / kWave];
-    const int tid = threadIdx.x;
+    constexpr int kLanes = 64 / kRun, kGroups = kHeldThreads / kLanes;        // lanes that share 64 elements, sums of 64 elements
+    __shared__ float4 scratch[4][kGroups / 4];
     const long src = rows ? rows[blockIdx.x] : blockIdx.x;
     float* xr = x + src * hidden;
+    const int sub = threadIdx.x % kLanes, place = threadIdx.x - sub + (sub & 1) * 4 + (sub & 2) + sub / 4;
     int at[kPer];
-    bool in[kPer];
 #pragma unroll
-    for (int n = 0; n < kPer; ++n) {
-        in[n] = tid + n * kNormThreadsFew < hidden;
-        at[n] = in[n] ? tid + n * kNormThreadsFew : hidden - 1;
-    }
-    float v[kPer], d[kPer], old[kHeldTaps - 1][kPer];
-    TW gd[kPer], bd[kPer], g[kPer], o[kPer], f[kHeldTaps][kPer];
+    for (int n = 0; n < kPer; ++n) at[n] = (n * kHeldThreads + place) * kRun;
+    const bool filtered = kTaps > 0 || (kTaps < 0 && conv);
+    if constexpr (kTaps > 0) taps = kTaps;
     int pos = 0, entry = 0;
-    if (conv) {
+    if (filtered) {
         pos = positions[blockIdx.x];
         entry = row_entry[blockIdx.x];
     }
+    Run<float, kVec> stream[kPer], more[kPer], old[kTaps == 0 ? 1 : kHeldTaps - 1][kPer];
+    Run<TW, kVec> delta_gain[kPer], delta_bias[kPer], gain[kPer], bias[kPer], filter[kTaps == 0 ? 1 : kHeldTaps][kPer];
 #pragma unroll
-    for (int n = 0; n < kPer; ++n) v[n] = xr[at[n]];
+    for (int n = 0; n < kPer; ++n) stream[n].load(xr, at[n], hidden);
     if (delta) {
 #pragma unroll
-        for (int n = 0; n < kPer; ++n) d[n] = delta[src * hidden + at[n]];
+        for (int n = 0; n < kPer; ++n) more[n].load(delta + src * hidden, at[n], hidden);
     }
     if (dw) {
 #pragma unroll
         for (int n = 0; n < kPer; ++n) {
-            gd[n] = dw[at[n]];
-            bd[n] = db[at[n]];
+            delta_gain[n].load(dw, at[n], hidden);
+            delta_bias[n].load(db, at[n], hidden);
         }
     }
     if (y) {
 #pragma unroll
         for (int n = 0; n < kPer; ++n) {
-            g[n] = w[at[n]];
-            o[n] = b[at[n]];
+            gain[n].load(w, at[n], hidden);
+            bias[n].load(b, at[n], hidden);
         }
     }
     float* keep = nullptr;
-    if (conv) {
+    if (filtered) {
 #pragma unroll
-        for (int j = 0; j < kHeldTaps; ++j)
+        for (int n = 0; n < kPer; ++n) {
+            if constexpr (kTaps == kHeldTaps) {      // a channel's taps lie side by side: four runs of two channels each
 #pragma unroll
-            for (int n = 0; n < kPer; ++n)
-                if (j < taps) f[j][n] = conv[static_cast<long>(at[n]) * taps + j];
+                for (int j = 0; j < kHeldTaps; ++j)
+                    filter[j][n].load(conv, at[n] < hidden ? at[n] * kHeldTaps + j * kRun : 0, hidden * kHeldTaps);
+            } else if constexpr (kTaps < 0) {
+#pragma unroll
+                for (int j = 0; j < kHeldTaps; ++j)
+#pragma unroll
+                    for (int i = 0; i < kRun; ++i)
+                        if (j < taps) filter[j][n].v[i] = conv[static_cast<long>(at[n] + i < hidden ? at[n] + i : hidden - 1) * taps + j];
+            }
+        }
         keep = conv_state + static_cast<long>(entry_slots[entry]) * (taps - 1) * hidden;
 #pragma unroll
-        for (int j = 0; j + 1 < kHeldTaps; ++j)
+        for (int j = 0; j + 1 < (kTaps == 0 ? 1 : kHeldTaps); ++j)
 #pragma unroll
             for (int n = 0; n < kPer; ++n)
-                if (j + 1 < taps) old[j][n] = keep[static_cast<long>(j) * hidden + at[n]];
+                if (j + 1 < taps) old[j][n].load(keep + static_cast<long>(j) * hidden, at[n], hidden);
     }
-    auto mean_of = [&](const float (&values)[kPer], float eps_, float& mean, float& rstd) {
-        float sum = 0.f;
+    const auto inside = [&](int n, int i) { return at[n] + (kVec ? 0 : i) < hidden; };
+    const auto row_sum = [&](float (&part)[kRun], float4* meet) {
 #pragma unroll
-        for (int n = 0; n < kPer; ++n) sum += in[n] ? values[n] : 0.f;
-        mean = block_sum<kNormThreadsFew>(sum, scratch) / static_cast<float>(hidden);
-        float q = 0.f;
-#pragma unroll
-        for (int n = 0; n < kPer; ++n) {
-            const float off = in[n] ? values[n] - mean : 0.f;
-            q = fmaf(off, off, q);
+        for (int i = 0; i < kRun; ++i) {
+            constexpr int kSwap1 = 0xb1, kSwap2 = 0x4e, kMirror8 = 0x141;     // elements 32, 16 and 8 apart
+            part[i] += of_lane<kSwap1>(part[i]);
+            part[i] += of_lane<kSwap2>(part[i]);
+            part[i] += of_lane<kMirror8>(part[i]);
         }
-        rstd = 1.0f / sqrtf(block_sum<kNormThreadsFew>(q, scratch) / static_cast<float>(hidden) + eps_);
+#pragma unroll
+        for (int off = kRun / 2; off > 0; off /= 2)
+#pragma unroll
+            for (int i = 0; i < off; ++i) part[i] += part[i + off];
+        if (sub == 0) reinterpret_cast<float*>(meet)[threadIdx.x / kLanes] = part[0];
+        __syncthreads();
+        float total = 0.f;
+#pragma unroll
+        for (int q = 0; q < kGroups / 4; ++q) {
+            const float4 four = meet[q];
+            total += four.x;
+            total += four.y;
+            total += four.z;
+            total += four.w;
+        }
+        return total;
     };
-    float mean = 0.f, rstd = 1.f;
+    const auto moments = [&](const float (&v)[kPer][kRun], float of_eps, float4 (*meet)[kGroups / 4], float& mean, float& rstd) {
+        float part[kRun] = {};
+#pragma unroll
+        for (int n = 0; n < kPer; ++n)
+#pragma unroll
+            for (int i = 0; i < kRun; ++i) part[i] += inside(n, i) ? v[n][i] : 0.f;
+        mean = row_sum(part, meet[0]) / static_cast<float>(hidden);
+#pragma unroll
+        for (int i = 0; i < kRun; ++i) part[i] = 0.f;
+#pragma unroll
+        for (int n = 0; n < kPer; ++n)
+#pragma unroll
+            for (int i = 0; i < kRun; ++i) {
+                const float off = inside(n, i) ? v[n][i] - mean : 0.f;
+                part[i] = fmaf(off, off, part[i]);
+            }
+        rstd = 1.0f / sqrtf(row_sum(part, meet[1]) / static_cast<float>(hidden) + of_eps);
+    };
+    float v[kPer][kRun];
+#pragma unroll
+    for (int n = 0; n < kPer; ++n)
+#pragma unroll
+        for (int i = 0; i < kRun; ++i) v[n][i] = stream[n].get(i);
     if (delta) {
-        if (dw) mean_of(d, deps, mean, rstd);
+        float d[kPer][kRun], mean = 0.f, rstd = 1.f;
+#pragma unroll
+        for (int n = 0; n < kPer; ++n)
+#pragma unroll
+            for (int i = 0; i < kRun; ++i) d[n][i] = more[n].get(i);
+        if (dw) moments(d, deps, scratch, mean, rstd);
 #pragma unroll
         for (int n = 0; n < kPer; ++n) {
-            const float more = dw ? (d[n] - mean) * rstd * to_float(gd[n]) + to_float(bd[n]) : d[n];
-            v[n] += more;
-            if (!rows && in[n]) xr[at[n]] = v[n];
+#pragma unroll
+            for (int i = 0; i < kRun; ++i) v[n][i] += dw ? (d[n][i] - mean) * rstd * delta_gain[n].get(i) + delta_bias[n].get(i) : d[n][i];
+            if (!rows) store_run<float, kVec>(xr, at[n], hidden, v[n]);
         }
     }
     if (!y) return;
-    mean_of(v, eps, mean, rstd);
+    float mean, rstd;
+    moments(v, eps, scratch + 2, mean, rstd);
     TOut* yr = y + static_cast<long>(blockIdx.x) * hidden;
 #pragma unroll
     for (int n = 0; n < kPer; ++n) {
-        if (!in[n]) continue;
-        const float h = (v[n] - mean) * rstd * to_float(g[n]) + to_float(o[n]);
-        if (!conv) {
-            yr[at[n]] = from_float<TOut>(h);
-            continue;
-        }
-        float acc = 0.f;
+        float h[kRun];
 #pragma unroll
-        for (int j = 0; j < kHeldTaps; ++j) {                // oldest input first, the row itself under the last tap
-            if (j + 1 < taps) {
-                const float was = pos - (taps - 1 - j) < 0 ? 0.f : old[j < kHeldTaps - 1 ? j : 0][n];
-                acc = fmaf(to_float(f[j][n]), was, acc);
-                if (write_state && j > 0) keep[static_cast<long>(j - 1) * hidden + at[n]] = was;
-            } else if (j + 1 == taps) {
-                acc = fmaf(to_float(f[j][n]), h, acc);
-                if (write_state) keep[static_cast<long>(j - 1) * hidden + at[n]] = h;
+        for (int i = 0; i < kRun; ++i) h[i] = (v[n][i] - mean) * rstd * gain[n].get(i) + bias[n].get(i);
+        if (filtered) {
+            // A step of single rows, every row another request: oldest input first, the row itself under the last tap
+            float acc[kRun] = {};
+#pragma unroll
+            for (int j = 0; j < (kTaps == 0 ? 1 : kHeldTaps); ++j) {
+                if (j >= taps) continue;
+                float in[kRun];
+#pragma unroll
+                for (int i = 0; i < kRun; ++i) {
+                    if (j + 1 < taps) in[i] = pos - (taps - 1 - j) < 0 ? 0.f : old[j < kHeldTaps - 1 ? j : 0][n].get(i);
+                    else in[i] = h[i];
+                    const float tap = kTaps < 0 ? filter[j][n].get(i) : filter[i / 2][n].get(i % 2 * kHeldTaps + j);
+                    acc[i] = fmaf(tap, in[i], acc[i]);
+                }
+                if (write_state && j > 0) store_run<float, kVec>(keep + static_cast<long>(j - 1) * hidden, at[n], hidden, in);
             }
+#pragma unroll
+            for (int i = 0; i < kRun; ++i) h[i] += acc[i];
         }
-        yr[at[n]] = from_float<TOut>(h + acc);
+        store_run<TOut, kVec>(yr, at[n], hidden, h);
     }
 }
 
@@ -284,6 +399,108 @@ __global__ void causal_conv_kernel(const TIn* __restrict__ in, long in_stride, T
             for (int j = 0; j + 2 < taps; ++j)
                 keep[static_cast<long>(j) * channels] = pos - (taps - 2 - j) < 0 ? 0.f : keep[static_cast<long>(j + 1) * channels];
             keep[static_cast<long>(taps - 2) * channels] = now;
+        }
+    }
+}
+
+// The same for steps of many rows with four taps, four channels a thread: a row is read once, the inputs before it stay in registers
+// as a window that moves on with every row of the same request, and the rows of a workgroup are all asked for before the first is
+// worked on.  Sums in the other kernel's order: the same bits.  What bounds it are the bytes, read and written once.
+// With cold caches, 2,048 rows of 4,096 channels, float to float: 17.2 us (54.4 with a load for every tap of a row); of 2,048, float
+// to bfloat16: 12.3 (26.5); 600 rows of those 9.6 (19.7).
+constexpr int kWindowTaps = 4;
+constexpr int kWindowThreads = 256;
+constexpr int kWindowChannels = 4;
+template <typename T>
+struct Four {
+    float4 v;
+    __device__ inline void load(const T* from) { v = *reinterpret_cast<const float4*>(from); }
+    __device__ inline float get(int i) const { return i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w; }
+};
+template <>
+struct Four<bf16_t> {
+    uint2 v;
+    __device__ inline void load(const bf16_t* from) { v = *reinterpret_cast<const uint2*>(from); }
+    __device__ inline float get(int i) const {
+        const unsigned word = i / 2 ? v.y : v.x;
+        return __uint_as_float(i % 2 ? word & 0xffff0000u : word << 16);
+    }
+};
+template <typename TIn, typename TOut>
+__global__ void __launch_bounds__(kWindowThreads)
+causal_conv_window_kernel(const TIn* __restrict__ in, long in_stride, TOut* __restrict__ out, long out_stride, AnyVec w, AnyVec bias,
+                          const float* __restrict__ state, const int* __restrict__ positions, const int* __restrict__ row_entry,
+                          const int* __restrict__ entry_slots, int rows, int channels, int add_input, int act) {
+    constexpr int kBefore = kWindowTaps - 1;
+    const int c = (blockIdx.y * kWindowThreads + threadIdx.x) * kWindowChannels;
+    const int r0 = blockIdx.x * kConvRows, count = min(kConvRows, rows - r0);
+    if (c >= channels) return;
+    Four<TIn> mine[kConvRows];
+#pragma unroll
+    for (int k = 0; k < kConvRows; ++k) mine[k].load(in + static_cast<long>(r0 + (k < count ? k : 0)) * in_stride + c);
+    int entries[kConvRows], places[kConvRows];
+#pragma unroll
+    for (int k = 0; k < kConvRows; ++k) {
+        entries[k] = row_entry[r0 + (k < count ? k : 0)];
+        places[k] = positions[r0 + (k < count ? k : 0)];
+    }
+    static_assert(kWindowChannels * kWindowTaps == 16, "a thread's taps are two runs of eight");
+    float taps[kWindowChannels * kWindowTaps], add[kWindowChannels], window[kBefore][kWindowChannels];
+    load_any8(w, static_cast<long>(c) * kWindowTaps, taps);
+    load_any8(w, static_cast<long>(c) * kWindowTaps + 8, taps + 8);
+#pragma unroll
+    for (int i = 0; i < kWindowChannels; ++i) add[i] = bias.ptr ? load_any(bias, c + i) : 0.f;
+    int last_entry = -1, last_pos = 0;
+#pragma unroll
+    for (int k = 0; k < kConvRows; ++k) {
+        if (k >= count) break;
+        const int r = r0 + k, entry = entries[k], pos = places[k];
+        if (k == 0 || entry != last_entry || pos != last_pos + 1) {
+            // a request's first row here: its last inputs are rows of this step as far as there are some, and then its state
+            int inside = 0;
+            while (inside < kBefore && r - inside - 1 >= 0 && row_entry[r - inside - 1] == entry) ++inside;
+            const float* kept = state + static_cast<long>(entry_slots[entry]) * kBefore * channels + c;
+#pragma unroll
+            for (int back = kBefore; back > 0; --back) {
+                if (pos - back < 0) {                           // before the sequence's start
+#pragma unroll
+                    for (int i = 0; i < kWindowChannels; ++i) window[kBefore - back][i] = 0.f;
+                } else if (back <= inside) {
+                    Four<TIn> row;
+                    row.load(in + static_cast<long>(r - back) * in_stride + c);
+#pragma unroll
+                    for (int i = 0; i < kWindowChannels; ++i) window[kBefore - back][i] = row.get(i);
+                } else {
+                    Four<float> was;
+                    was.load(kept + static_cast<long>(kBefore - (back - inside)) * channels);
+#pragma unroll
+                    for (int i = 0; i < kWindowChannels; ++i) window[kBefore - back][i] = was.get(i);
+                }
+            }
+        }
+        last_entry = entry, last_pos = pos;
+        float result[kWindowChannels];
+#pragma unroll
+        for (int i = 0; i < kWindowChannels; ++i) {
+            const float now = mine[k].get(i);
+            float acc = 0.f;
+#pragma unroll
+            for (int j = 0; j < kBefore; ++j) acc = fmaf(taps[i * kWindowTaps + j], window[j][i], acc);        // oldest input first
+            acc = fmaf(taps[i * kWindowTaps + kBefore], now, acc);
+            if (add_input) acc += now;
+            if (bias.ptr) acc += add[i];
+            result[i] = activate(acc, act);
+#pragma unroll
+            for (int j = 0; j + 1 < kBefore; ++j) window[j][i] = window[j + 1][i];
+            window[kBefore - 1][i] = now;
+        }
+        TOut* to = out + static_cast<long>(r) * out_stride + c;
+        if constexpr (sizeof(TOut) == 4) {
+            *reinterpret_cast<float4*>(to) = float4{result[0], result[1], result[2], result[3]};
+        } else {
+            *reinterpret_cast<uint2*>(to) =
+                uint2{bf16_bits_from_float(result[0]) | static_cast<unsigned>(bf16_bits_from_float(result[1])) << 16,
+                      bf16_bits_from_float(result[2]) | static_cast<unsigned>(bf16_bits_from_float(result[3])) << 16};
         }
     }
 }
@@ -505,18 +722,26 @@ extern "C" int leone_add_layernorm(float* x, const float* delta, const void* dw,
                                                                          rows, hidden, vconv, taps, conv_state, write_state,   \
                                                                          positions, row_entry, entry_slots, stage_delta)
     const bool many = n_out >= kNormManyRows;
-    // few rows whose elements fit a workgroup's registers, one type of vectors throughout
-    if (!many && hidden <= 4 * kNormThreadsFew && (!conv || (taps <= kHeldTaps && conv_dtype == w_dtype))) {
-#define LEONE_HELD(T, TW, PER)                                                                                                  \
-    add_layernorm_held_kernel<T, TW, PER><<<n_out, kNormThreadsFew, 0, stream>>>(                                               \
+    // Rows that fit a workgroup's registers, one type of vectors throughout: whole 16-byte runs whatever the number of rows; else
+    // element by element, where few rows wait for their trips to memory.  (us with cold caches, before and so: 2,048 rows of 2,048 33.6
+    // and 22.0, of 1,024 18.6 and 13.7, 512 rows of 2,048 20.0 and 9.3.)
+    const auto aligned = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+    const bool vec = hidden % kRun == 0 && aligned(x) && aligned(delta) && aligned(dw) && aligned(db) && aligned(w) && aligned(b) &&
+                     aligned(y) && (!conv || (taps == kHeldTaps && aligned(conv) && aligned(conv_state)));
+    if (hidden <= 4 * kRun * kHeldThreads && (vec || !many) && (!conv || (taps <= kHeldTaps && conv_dtype == w_dtype))) {
+#define LEONE_HELD(T, TW, VEC, PER, TAPS)                                                                                       \
+    add_layernorm_held_kernel<T, TW, VEC, PER, TAPS><<<n_out, kHeldThreads, 0, stream>>>(                                       \
         x, delta, static_cast<const TW*>(dw), static_cast<const TW*>(db), deps, static_cast<const TW*>(w), static_cast<const TW*>(b), eps, \
         static_cast<T*>(y), rows, hidden, static_cast<const TW*>(conv), taps, conv_state, write_state, positions, row_entry, entry_slots)
-#define LEONE_HELD_PER(T, TW) (hidden <= 2 * kNormThreadsFew ? LEONE_HELD(T, TW, 2) : LEONE_HELD(T, TW, 4))
+#define LEONE_HELD_VEC(T, TW, PER)                                                                                              \
+    (!vec ? LEONE_HELD(T, TW, false, PER, -1) : conv ? LEONE_HELD(T, TW, true, PER, kHeldTaps) : LEONE_HELD(T, TW, true, PER, 0))
+#define LEONE_HELD_PER(T, TW) (hidden <= 2 * kRun * kHeldThreads ? LEONE_HELD_VEC(T, TW, 2) : LEONE_HELD_VEC(T, TW, 4))
         if (y_dtype == kF32 && w_dtype == kF32) LEONE_HELD_PER(float, float);
         else if (y_dtype == kF32) LEONE_HELD_PER(float, bf16_t);
         else if (w_dtype == kF32) LEONE_HELD_PER(bf16_t, float);
         else LEONE_HELD_PER(bf16_t, bf16_t);
 #undef LEONE_HELD_PER
+#undef LEONE_HELD_VEC
 #undef LEONE_HELD
         LEONE_LAUNCH_CHECK("add_layernorm");
         return 0;
@@ -568,11 +793,22 @@ extern "C" int leone_causal_conv_biased(const void* in, int in_dtype, long in_st
     const AnyVec vbias{bias, w_dtype};
     const int per_block = rows >= kNormManyRows ? kConvRows : 1;
     const dim3 grid(ceil_div(rows, per_block), ceil_div(channels, 256));
+    float* const own_state = (write_state && single_rows) ? state : nullptr;
+    // Four channels a thread where rows of the inputs, the outputs and the state can be read and written so.
+    const auto fours = [&](const void* p, long stride, int size) {
+        return stride % kWindowChannels == 0 && reinterpret_cast<uintptr_t>(p) % (kWindowChannels * size) == 0;
+    };
+    const bool window = per_block > 1 && taps == kWindowTaps && !own_state && fours(in, in_stride, in_dtype == kF32 ? 4 : 2) &&
+                        fours(out, out_stride, out_dtype == kF32 ? 4 : 2) && fours(state, channels, 4) &&
+                        reinterpret_cast<uintptr_t>(w) % 16 == 0;
+    const dim3 window_grid(grid.x, ceil_div(channels, kWindowThreads * kWindowChannels));
 #define LEONE_CONV(TIN, TOUT)                                                                                         \
-    causal_conv_kernel<TIN, TOUT><<<grid, 256, 0, stream>>>(static_cast<const TIN*>(in), in_stride, static_cast<TOUT*>(out), \
-                                                            out_stride, vw, vbias, state, positions, row_entry, entry_slots, \
-                                                            rows, channels, taps, add_input, act,                    \
-                                                            (write_state && single_rows) ? state : nullptr, per_block)
+    (window ? causal_conv_window_kernel<TIN, TOUT><<<window_grid, kWindowThreads, 0, stream>>>(                           \
+                  static_cast<const TIN*>(in), in_stride, static_cast<TOUT*>(out), out_stride, vw, vbias, state, positions, \
+                  row_entry, entry_slots, rows, channels, add_input, act)                                             \
+            : causal_conv_kernel<TIN, TOUT><<<grid, 256, 0, stream>>>(static_cast<const TIN*>(in), in_stride, static_cast<TOUT*>(out), \
+                                                                      out_stride, vw, vbias, state, positions, row_entry, entry_slots, \
+                                                                      rows, channels, taps, add_input, act, own_state, per_block))
     if (in_dtype == kF32 && out_dtype == kF32) LEONE_CONV(float, float);
     else if (in_dtype == kF32) LEONE_CONV(float, bf16_t);
     else if (out_dtype == kF32) LEONE_CONV(bf16_t, float);

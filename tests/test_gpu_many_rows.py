@@ -1,0 +1,84 @@
+"""Row-wise kernels at the sizes where many rows, whole runs or several trips of a workgroup take another path: filters of four taps
+with a window in registers, the exponential gates of long portions."""
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _step(spans, slots):
+    """A step of entries with rows [first position, count] each."""
+    positions = torch.cat([torch.arange(p, p + n) for p, n in spans]).to(torch.int32)
+    entry = torch.cat([torch.full((n,), i) for i, (_, n) in enumerate(spans)]).to(torch.int32)
+    entries, first = [], 0
+    for (p, n), slot in zip(spans, slots):
+        entries.append(SimpleNamespace(first_row=first, count=n, start=p, slot=slot))
+        first += n
+    return SimpleNamespace(decode_only=False, rows=first, positions=positions.to(DEV), row_entry=entry.to(DEV), entries=entries,
+                           entry_slots=torch.tensor(slots, dtype=torch.int32, device=DEV), plan=None, device=torch.device(DEV))
+
+
+@pytest.mark.parametrize("channels", [4, 1020, 1028, 1030])
+@pytest.mark.parametrize("kind,out,filters", [(torch.float32, torch.bfloat16, torch.bfloat16), (torch.bfloat16, torch.float32, torch.float32),
+                                              (torch.float32, torch.float32, torch.bfloat16)])
+def test_filters_of_many_rows(channels, kind, out, filters):
+    """Requests of a row, a few and many, at their start and later, boundaries inside a workgroup's rows; inputs that are columns of
+    wider rows (1,030 channels: not in runs of four)."""
+    from leone_amd import ops
+    gen = torch.Generator().manual_seed(channels)
+    spans, slots, taps = [(0, 1), (7, 2), (0, 3), (1, 5), (0, 500), (2, 11), (900, 9)], [3, 0, 6, 1, 5, 2, 4], 4
+    step = _step(spans, slots)
+    wide = torch.randn(step.rows, channels + 8, generator=gen).to(kind)
+    weight, bias = torch.randn(channels, taps, generator=gen).to(filters), torch.randn(channels, generator=gen).to(filters)
+    state = torch.randn(8, taps - 1, channels, generator=gen)
+    kept = state.to(DEV).clone()
+    x = wide.to(DEV)[:, 4:4 + channels]
+    got = ops.causal_conv(x, weight.to(DEV), kept, step, out, add_input=True, bias=bias.to(DEV)).cpu().double()
+    first, want, after = 0, [], state.double().clone()
+    for (p, n), slot in zip(spans, slots):
+        rows = wide[first:first + n, 4:4 + channels].double()
+        before = state[slot].double() * (torch.arange(p - 3, p) >= 0)[:, None]
+        full = torch.cat([before, rows])
+        want.append(rows + bias.double() + sum(full[j:j + n] * weight.double()[:, j] for j in range(taps)))
+        after[slot] = full[-3:]
+        first += n
+    want = torch.cat(want)
+    # six float operations on values of up to some 20; results in bfloat16 have eight significant bits
+    assert float(((got - want).abs() / (want.abs() + 10.0)).max()) < (2.0 ** -8 if out == torch.bfloat16 else 2e-6)
+    assert torch.equal(kept.cpu().double(), after)
+
+
+@pytest.mark.parametrize("counts", [(1, 1), (64, 1), (65, 3), (1024, 1025), (2111,)])
+def test_exponential_gates(counts):
+    """One wave's rows, a workgroup's and one over, from a state and from a sequence's start."""
+    from leone_amd import ops
+    gen = torch.Generator().manual_seed(sum(counts))
+    heads, dim, vdim = 2, 32, 64
+    starts = [0 if i % 2 else 5 for i in range(len(counts))]
+    step = _step(list(zip(starts, counts)), list(range(1, len(counts) + 1)))
+    step.decode_only = all(n == 1 for n in counts)
+    width = 2 * heads * dim + heads * vdim + 2 * heads
+    proj = torch.randn(step.rows, width, generator=gen)
+    columns = {"q": 0, "k": heads * dim, "v": 2 * heads * dim, "i": width - 2 * heads, "f": width - heads}
+    bias = {"i": torch.randn(heads, generator=gen), "f": torch.randn(heads, generator=gen) + 2}
+    per = dim * vdim + dim + 1
+    state = torch.zeros(len(counts) + 1, heads, per)
+    state[:, :, -1] = torch.randn(len(counts) + 1, heads, generator=gen)
+    kept = state.to(DEV).clone()
+    _, (_, top) = ops.outer_scan(proj.to(DEV), columns, kept, step, heads, dim, vdim,
+                                 gates={"i_bias": bias["i"].to(DEV), "f_bias": bias["f"].to(DEV), "cap": 15.0})
+    top, first = top.cpu().double(), 0
+    for e, n in enumerate(counts):
+        raw = proj[first:first + n].double()
+        li = 15 * torch.tanh((raw[:, columns["i"]:columns["i"] + heads] + bias["i"].double()) / 15)
+        lf = torch.nn.functional.logsigmoid(15 * torch.tanh((raw[:, columns["f"]:] + bias["f"].double()) / 15))
+        m = torch.zeros(heads, dtype=torch.float64) if starts[e] == 0 else state[e + 1, :, -1].double()
+        for t in range(n):
+            m = torch.maximum(lf[t] + m, li[t])
+            # sums of up to 64 gates of float a wave, each off by 2^-24 of values up to 100
+            assert float((top[first + t] - m).abs().max()) < 1e-4, (e, t)
+        assert float((kept[e + 1, :, -1].cpu().double() - m).abs().max()) < 1e-4
+        first += n
