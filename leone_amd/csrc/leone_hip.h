@@ -306,6 +306,13 @@ int leone_glu(const void* gate_up, void* out, int dtype, int rows, int ffn, int 
 int leone_add_normed(float* x, const float* delta, int delta_planes, long delta_plane, const void* gain, int gain_dtype,
                      float eps, void* y, int y_dtype, const void* gain2, int gain2_dtype, float eps2, const int* rows,
                      int n_rows, int hidden, hipStream_t stream);
+// The same with the sums that leone_moe_combine makes as the delta, without writing them; for hidden sizes that
+// leone_add_normed_pairs_fits takes, every operand aligned to 16 bytes.
+int leone_add_normed_pairs_fits(int hidden);
+int leone_add_normed_pairs(float* x, const float* pair_out, const int* chosen, const float* weight, int top, const void* from,
+                           int from_dtype, const float* extra, int experts, const void* gain, int gain_dtype, float eps, void* y,
+                           int y_dtype, const void* gain2, int gain2_dtype, float eps2, const int* rows, int n_rows, int hidden,
+                           hipStream_t stream);
 // leone_attention_rows with the keys below keep_first kept in sight of a windowed layer, and with gate_each a
 // gate value for every element of every head ([rows, q_heads * v_dim] within rows of gate_stride).
 int leone_attention_rows_kept(const void* q, void* out, const void* k_pool, const void* v_pool, int dtype,

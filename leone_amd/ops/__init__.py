@@ -1347,7 +1347,35 @@ class NormedDelta:
         self.rows, self.norm = rows, norm
 
     def materialize(self) -> torch.Tensor:
-        return self.norm.apply(self.rows)
+        return self.norm.apply(self.rows.sum() if isinstance(self.rows, PairedRows) else self.rows)
+
+
+class PairedRows:
+    """What routed experts gave, one row a (row, place): still to be summed over each row's places.  ``add_normed`` takes it as a
+    delta and makes the sums on the way; any other consumer asks for ``sum()`` (float32 ``[rows, hidden]``)."""
+
+    def __init__(self, pairs: torch.Tensor, chosen: torch.Tensor, weight: torch.Tensor, x: torch.Tensor, extra: Optional[torch.Tensor],
+                 experts: int):
+        self.pairs, self.chosen, self.weight, self.x, self.extra, self.experts = pairs, chosen, weight, x, extra, experts
+
+    def args(self) -> tuple:
+        rows, hidden = self.x.shape
+        top = self.chosen.shape[1]
+        return (_dev(self.pairs, "pair results", torch.float32, (rows * top, hidden)), _dev(self.chosen, "chosen", torch.int32, (rows, top)),
+                _dev(self.weight, "weights", torch.float32, (rows, top)), top, _dev(self.x, "routed rows"), _code(self.x, "routed rows"),
+                _dev(self.extra, "extra", torch.float32, (rows, hidden)))
+
+    def sum(self) -> torch.Tensor:
+        rows, hidden = self.x.shape
+        pairs, chosen, weight, top, x, kind, extra = self.args()
+        out = torch.empty((rows, hidden), dtype=torch.float32, device=self.x.device)
+        call("leone_moe_combine", pairs, chosen, weight, x, kind, extra, _dev(out, "routed out"), rows, top, self.experts, hidden, _stream())
+        return out
+
+    def folds(self, *operands) -> bool:
+        """Whether ``add_normed`` makes the sums itself beside these operands."""
+        return bool(library().leone_add_normed_pairs_fits(self.x.shape[1])) and \
+            all(t is None or t.data_ptr() % 16 == 0 for t in (self.pairs, self.x, self.extra) + operands)
 
 
 def add_layernorm(x: torch.Tensor, delta: Optional[torch.Tensor], gain: Optional[torch.Tensor],
@@ -1777,11 +1805,17 @@ def add_normed(x: torch.Tensor, delta: Optional[torch.Tensor], gain: Optional[to
                out_dtype: Optional[torch.dtype] = None, then: Optional[tuple] = None,
                rows: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
     """x += rmsnorm(delta) * gain in the float32 stream (``delta`` float32 ``[n, hidden]`` or planes ``[p, n, hidden]``
-    whose sum, in order, is meant; None: nothing is added).  What comes back: with ``out_dtype`` the new rows of
+    whose sum, in order, is meant, or ``PairedRows``; None: nothing is added).  What comes back: with ``out_dtype`` the new rows of
     the stream in that type (what the next sublayer's products read); with ``then = (gain2, eps2, dtype)`` instead
     rmsnorm(x) * gain2 of the new rows, of the rows ``rows`` (int32 indices) only if given, and then the stream
     itself is left as it was."""
     n, hidden = x.shape
+    paired = delta if isinstance(delta, PairedRows) else None
+    if paired is not None:
+        if not paired.folds(x, gain, then[0] if then is not None else None):
+            paired, delta = None, paired.sum()
+        else:
+            delta = paired.pairs
     if delta is not None and delta.dtype != torch.float32:
         delta = delta.float()
     stacked = delta is not None and delta.dim() == 3
@@ -1796,14 +1830,19 @@ def add_normed(x: torch.Tensor, delta: Optional[torch.Tensor], gain: Optional[to
         return x                                   # nothing to add, nothing to convert
     same = then is None and kind == torch.float32          # the stream itself is what the next products read
     y = torch.empty((n_out, hidden), dtype=kind, device=x.device) if (kind is not None and not same) else None
-    call("leone_add_normed", _dev(x, "stream", torch.float32),
-         _dev(delta, "delta", torch.float32, (planes, n, hidden) if stacked else (n, hidden)), planes, n * hidden,
-         _dev(gain, "gain", None, (hidden,)) if delta is not None else 0,
-         _code(gain, "gain") if delta is not None else F32, float(eps),
-         _dev(y, "rows out"), _CODES[kind] if kind is not None else F32,
-         _dev(then[0], "second gain", None, (hidden,)) if then is not None else 0,
-         _code(then[0], "second gain") if then is not None else F32, float(then[1]) if then is not None else 0.0,
-         _dev(rows, "rows", torch.int32) if rows is not None else 0, n_out, hidden, _stream())
+    norms = (_dev(gain, "gain", None, (hidden,)) if delta is not None else 0,
+             _code(gain, "gain") if delta is not None else F32, float(eps),
+             _dev(y, "rows out"), _CODES[kind] if kind is not None else F32,
+             _dev(then[0], "second gain", None, (hidden,)) if then is not None else 0,
+             _code(then[0], "second gain") if then is not None else F32, float(then[1]) if then is not None else 0.0,
+             _dev(rows, "rows", torch.int32) if rows is not None else 0, n_out, hidden, _stream())
+    if paired is not None:
+        if paired.x.shape != x.shape:
+            raise KernelError(f"add_normed: experts' rows {tuple(paired.x.shape)} for a stream of {tuple(x.shape)}")
+        call("leone_add_normed_pairs", _dev(x, "stream", torch.float32), *paired.args(), paired.experts, *norms)
+    else:
+        call("leone_add_normed", _dev(x, "stream", torch.float32),
+             _dev(delta, "delta", torch.float32, (planes, n, hidden) if stacked else (n, hidden)), planes, n * hidden, *norms)
     return x if same else y
 
 
@@ -1902,7 +1941,7 @@ def _check_experts(x: torch.Tensor, w_up: torch.Tensor, w_down: torch.Tensor):
     return rows, hidden, experts, ff, gated
 
 
-def _expert_products(x, chosen, weight, tiles, w_up, w_down, activation, extra, limit=None, weigh_input=False) -> torch.Tensor:
+def _expert_products(x, chosen, weight, tiles, w_up, w_down, activation, extra, limit=None, weigh_input=False, paired=False):
     rows, hidden, experts, ff, gated = _check_experts(x, w_up, w_down)
     if weigh_input and gated:
         raise KernelError("routed experts: a weight on what an expert reads goes with experts without a gate")
@@ -1921,46 +1960,44 @@ def _expert_products(x, chosen, weight, tiles, w_up, w_down, activation, extra, 
     call("leone_moe_product", _dev(hidden_act, "expert hidden"), _dev(w_down, "expert down"), _dev(pair_out, "pair results"),
          0 if weigh_input else weights, _code(x, "routed rows"), 0, _dev(tile_expert, "tiles"),
          _dev(tile_pairs, "tile pairs"), max_tiles, tile, top, hidden, ff, 0, 0.0, _stream())
-    out = torch.empty((rows, hidden), dtype=torch.float32, device=device)
-    call("leone_moe_combine", _dev(pair_out, "pair results"), _dev(chosen, "chosen"), weights,
-         _dev(x, "routed rows"), _code(x, "routed rows"), _dev(extra, "extra", torch.float32, (rows, hidden)),
-         _dev(out, "routed out"), rows, top, experts, hidden, _stream())
-    return out
+    out = PairedRows(pair_out, chosen, weight, x, extra, experts)
+    return out if paired else out.sum()
 
 
 def routed_experts(x: torch.Tensor, chosen: torch.Tensor, weight: torch.Tensor, w_gate_up: torch.Tensor,
                    w_down: torch.Tensor, activation: str = "silu", extra: Optional[torch.Tensor] = None,
-                   limit: Optional[float] = None, weigh_input: bool = False) -> torch.Tensor:
+                   limit: Optional[float] = None, weigh_input: bool = False, paired: bool = False):
     """Every row through the experts chosen for it: float32 ``[rows, hidden]`` = sum over a row's places of
     weight * W_down[e] (act(W_gate[e] x) * (W_up[e] x)), in the places' order; a chosen index from the number of
     experts on stands for an expert that hands the row on as it is; ``extra`` (float32 ``[rows, hidden]``) is added.
     ``w_gate_up`` is ``[experts, 2, ff, hidden]`` (gate rows, then up rows), ``w_down`` ``[experts, hidden, ff]``, both
     of ``x``'s type; experts without a gate come as ``[experts, ff, hidden]`` and compute W_down[e] act(W_up[e] x)
     (``PLAIN_ACTIVATIONS``).  ``weigh_input`` (experts without a gate): the weight multiplies what the expert reads
-    instead of what it gives.  Nothing here depends on the choice except through device arrays."""
+    instead of what it gives.  ``paired``: the sum is left to the consumer (``PairedRows``).  Nothing here depends on the choice
+    except through device arrays."""
     rows, hidden, experts, ff, _ = _check_experts(x, w_gate_up, w_down)
     top = chosen.shape[1]
     tiles = _expert_tiles(x, rows, top, experts, hidden, ff)
     call("leone_moe_plan", _dev(chosen, "chosen", torch.int32, (rows, top)), rows * top, experts, _dev(tiles[2], "tiles"),
          _dev(tiles[3], "tile pairs"), tiles[1], tiles[0], _stream())
-    return _expert_products(x, chosen, weight, tiles, w_gate_up, w_down, activation, extra, limit, weigh_input)
+    return _expert_products(x, chosen, weight, tiles, w_gate_up, w_down, activation, extra, limit, weigh_input, paired)
 
 
 def routed_feed_forward(x: torch.Tensor, logits: torch.Tensor, correction: Optional[torch.Tensor], top: int, group_count: int,
                         group_keep: int, w_gate_up: torch.Tensor, w_down: torch.Tensor, activation: str = "silu",
                         extra: Optional[torch.Tensor] = None, always: int = 0, rule: Optional[RouterRule] = None,
-                        limit: Optional[float] = None, weigh_input: bool = False) -> torch.Tensor:
+                        limit: Optional[float] = None, weigh_input: bool = False, paired: bool = False):
     """``route_topk`` on the router's float32 ``logits`` and ``routed_experts`` with its choice; for steps of few rows
     (up to ``ROUTE_PLAN_ROWS``) the choice and the tiles are made in one launch.  ``always`` (such steps only): the
     last so many experts of the matrices are no choice of the router's but taken by every row with weight 1 (a
-    shared expert cut to the experts' size rides along in the experts' launches)."""
+    shared expert cut to the experts' size rides along in the experts' launches).  ``paired`` as for ``routed_experts``."""
     rows, hidden, experts, ff, _ = _check_experts(x, w_gate_up, w_down)
     total = logits.shape[1]
     if rows > ROUTE_PLAN_ROWS:
         if always:
             raise KernelError(f"routed_feed_forward: experts for every row ride along in steps of up to {ROUTE_PLAN_ROWS} rows only")
         chosen, weight = route_topk(logits, correction, top, group_count, group_keep, rule)
-        return routed_experts(x, chosen, weight, w_gate_up, w_down, activation, extra, limit, weigh_input)
+        return routed_experts(x, chosen, weight, w_gate_up, w_down, activation, extra, limit, weigh_input, paired)
     if total > library().leone_route_max_outputs():
         raise KernelError(f"route_topk: {total} router outputs, the kernel takes {library().leone_route_max_outputs()}")
     if not 0 <= always < experts:
@@ -1974,7 +2011,7 @@ def routed_feed_forward(x: torch.Tensor, logits: torch.Tensor, correction: Optio
          _dev(chosen, "chosen"), _dev(weight, "weights"), rows, total, int(top), int(group_count), int(group_keep), experts,
          _dev(tiles[2], "tiles"), _dev(tiles[3], "tile pairs"), tiles[1], tiles[0], int(always),
          *(rule or _DEFAULT_RULE).args(), _stream())
-    return _expert_products(x, chosen, weight, tiles, w_gate_up, w_down, activation, extra, limit, weigh_input)
+    return _expert_products(x, chosen, weight, tiles, w_gate_up, w_down, activation, extra, limit, weigh_input, paired)
 
 
 # ---- a forget gate per key channel, attention through a shared latent, the stream as a sum over depth -----------

@@ -87,6 +87,8 @@ _PROTOTYPES = {
                          c_float, P, c_int, P, ctypes.c_long, P, ctypes.c_long, P, c_int, c_int, c_int, c_int, P],
     "leone_embed_placed": [P, c_int, P, P, c_int, c_int, c_int, c_float, P, P, c_int, P, P],
     "leone_glu": [P, P, c_int, c_int, c_int, c_int, c_float, P],
+    "leone_add_normed_pairs_fits": [c_int],
+    "leone_add_normed_pairs": [P, P, P, P, c_int, P, c_int, P, c_int, P, c_int, c_float, P, c_int, P, c_int, c_float, P, c_int, c_int, P],
     "leone_add_normed": [P, P, c_int, ctypes.c_long, P, c_int, c_float, P, c_int, P, c_int, c_float, P, c_int, c_int, P],
     "leone_attention_rows_kept": [P, P, P, P, c_int, P, P, P, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float,
                                   c_int, P, ctypes.c_long, c_int, c_int, P],

@@ -52,6 +52,7 @@ OPERATIONS = {
     "leone_embed_placed": "embed",
     "leone_glu": "swiglu",
     "leone_add_normed": "norm",
+    "leone_add_normed_pairs": "norm",
     "leone_attention_rows_kept": "attention",
     "leone_attention_decode_kept": "attention",
     "leone_attention_prefill_kept": "attention",

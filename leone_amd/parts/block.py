@@ -250,7 +250,8 @@ class PostNormBlock(Part):
         if self.feed_forward is None:
             return ops.NormedDelta(mixed, self.norm1)
         h = self.norm1.add_behind(x, mixed, step.dtype)
-        return ops.NormedDelta(self.feed_forward.forward(h, step), self.norm2)
+        feed = getattr(self.feed_forward, "forward_paired", self.feed_forward.forward)
+        return ops.NormedDelta(feed(h, step), self.norm2)
 
 
 @BLOCKS.register("scaled_prenorm")

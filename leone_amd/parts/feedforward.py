@@ -224,13 +224,13 @@ class RoutedGluMlp(Part):
     def streamed_weights(self) -> List[torch.Tensor]:
         return self.shared.streamed_weights() if self.shared is not None else []
 
-    def forward(self, y: torch.Tensor, step: StepContext) -> torch.Tensor:
+    def forward(self, y: torch.Tensor, step: StepContext, paired: bool = False):
         y = ops.materialize(y)
         logits = ops.linear(y, self.w_router, out_dtype=torch.float32)
         if self.always and y.shape[0] <= ops.ROUTE_PLAN_ROWS:
             return ops.routed_feed_forward(y, logits, self.correction, self.top, self.group_count, self.group_keep,
                                            self.w_gate_up_all, self.w_down_all, self.activation, always=self.always,
-                                           rule=self.rule, limit=self.limit)
+                                           rule=self.rule, limit=self.limit, paired=paired)
         extra = None
         if self.shared is not None:
             extra = self.shared.forward(y, step)
@@ -240,4 +240,8 @@ class RoutedGluMlp(Part):
                 extra = extra.float()
         return ops.routed_feed_forward(y, logits, self.correction, self.top, self.group_count, self.group_keep,
                                        self.w_gate_up, self.w_down, self.activation, extra=extra, rule=self.rule,
-                                       limit=self.limit, weigh_input=self.weigh_input)
+                                       limit=self.limit, weigh_input=self.weigh_input, paired=paired)
+
+    def forward_paired(self, y: torch.Tensor, step: StepContext) -> ops.PairedRows:
+        """The same with the sum over a row's places left to the norm behind (``ops.add_normed``)."""
+        return self.forward(y, step, paired=True)

@@ -97,3 +97,36 @@ def test_head_norms_of_few_rows(vdim, act, gate_first):
             v = o.double() * (g if gate_first else 1)
             v = v / ((v ** 2).mean(-1, keepdim=True) + 1e-5).sqrt() * gain.double().view(*((heads, vdim) if per_head else (vdim,)))
             _close(got.view(rows, heads, vdim), v if gate_first else v * g, out)
+
+
+@pytest.mark.parametrize("hidden", [4, 1020, 1024, 2048, 2052, 4096, 4100])
+@pytest.mark.parametrize("places", [1, 4, 8, 9])
+def test_norms_behind_a_sublayer_that_sum_their_places(hidden, places):
+    """The norm of a delta in planes, and of what routed experts left row by row (some places handing the row on, some empty), at the
+    sizes where registers no longer hold a row and where places come in several turns."""
+    from leone_amd import ops
+    gen = torch.Generator().manual_seed(hidden + places)
+    n, experts = 6, 5
+    draw = lambda *size: torch.randn(*size, generator=gen)     # noqa: E731
+    x, pairs, extra = draw(n, hidden), draw(n * places, hidden), draw(n, hidden)
+    chosen = torch.randint(-1, experts + 2, (n, places), generator=gen, dtype=torch.int32)
+    weight, gain, gain2 = torch.rand(n, places, generator=gen), draw(hidden), draw(hidden).bfloat16()
+    for kind, out, planes in ((torch.bfloat16, torch.bfloat16, False), (torch.float32, torch.float32, False), (None, torch.bfloat16, True)):
+        for picked in (False, True):
+            rows = torch.tensor([3, 0, 5], dtype=torch.int32) if picked else None
+            stream = x.to(DEV).clone()
+            if planes:
+                delta, total = pairs.view(places, n, hidden).to(DEV), pairs.view(places, n, hidden).double().sum(0)
+            else:
+                came = draw(n, hidden).to(kind)
+                with_extra = extra if kind == torch.float32 else None
+                delta = ops.PairedRows(pairs.to(DEV), chosen.to(DEV), weight.to(DEV), came.to(DEV), with_extra.to(DEV) if with_extra is not None else None, experts)
+                each = torch.where((chosen >= experts)[..., None], weight.double()[..., None] * came.double()[:, None], pairs.view(n, places, hidden).double())
+                total = (each * (chosen >= 0)[..., None]).sum(1) + (with_extra.double() if with_extra is not None else 0)
+                assert float((delta.sum().cpu().double() - total).abs().max()) < 1e-5
+            normed = lambda v, g, eps: v / ((v ** 2).mean(-1, keepdim=True) + eps).sqrt() * g.double()      # noqa: E731
+            after = x.double() + normed(total, gain, 1e-6)
+            then = (gain2.to(DEV), 1e-5, out) if picked else None
+            y = ops.add_normed(stream, delta, gain.to(DEV), 1e-6, out_dtype=None if picked else out, then=then, rows=rows.to(DEV) if picked else None)
+            _close(y, normed(after, gain2, 1e-5)[rows.long()] if picked else after, out)
+            assert torch.equal(stream.cpu(), x) if picked else float((stream.cpu().double() - after).abs().max()) < 4e-5
