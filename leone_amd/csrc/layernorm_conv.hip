@@ -40,6 +40,28 @@ __device__ inline void mean_rstd(F value, int n, float eps, float* scratch, floa
     rstd = 1.0f / sqrtf(var + eps);
 }
 
+// Four neighbouring elements as they were loaded, unpacked where they are used.
+template <typename T>
+struct Four {
+    float4 v;
+    __device__ inline void load(const T* from) { v = *reinterpret_cast<const float4*>(from); }
+    __device__ inline float get(int i) const { return i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w; }
+};
+template <>
+struct Four<bf16_t> {
+    uint2 v;
+    __device__ inline void load(const bf16_t* from) { v = *reinterpret_cast<const uint2*>(from); }
+    __device__ inline float get(int i) const {
+        const unsigned word = i / 2 ? v.y : v.x;
+        return __uint_as_float(i % 2 ? word & 0xffff0000u : word << 16);
+    }
+};
+__device__ inline void store_four(float* to, const float (&v)[4]) { *reinterpret_cast<float4*>(to) = float4{v[0], v[1], v[2], v[3]}; }
+__device__ inline void store_four(bf16_t* to, const float (&v)[4]) {
+    *reinterpret_cast<uint2*>(to) = uint2{bf16_bits_from_float(v[0]) | static_cast<unsigned>(bf16_bits_from_float(v[1])) << 16,
+                                          bf16_bits_from_float(v[2]) | static_cast<unsigned>(bf16_bits_from_float(v[3])) << 16};
+}
+
 // One workgroup a row; the row lies in shared memory between the passes.
 template <typename TOut, int kNormThreads>
 __global__ void __launch_bounds__(kNormThreads)
@@ -164,13 +186,11 @@ __device__ inline void store_run(T* __restrict__ row, int at, int length, const 
 // The same for rows of up to 1,024 kPer elements, a workgroup of two waves a row, in runs of 8 elements a thread.  A step of few rows
 // is a chain of trips to memory, about two microseconds each when the lines are cold: here the row, the delta, the gains, the
 // biases, the filter's taps and the state's last inputs are all asked for before the first sum, and the row stays in registers.
-// Many rows are bound by their bytes: 16-byte accesses, every row's on their way at once.
 // Sums run in the other kernel's order with 1,024 threads, so that few rows get the bits they get there: elements 1,024 apart in
 // turn, then those 32, 16, .. 1 apart meet, then every 64's sums in turn.  The runs of 64 elements lie on the eight lanes so that
 // each of the lanes' three meetings is an operand's permutation.
 // kTaps: of the folded filter; 0: none, -1: `taps` of them, up to kHeldTaps.
-// Eight rows of 2,048 with two norms and a filter of 4 taps, in bfloat16: 6.1 us (7.8 with 1,024 threads of single elements);
-// 2,048 rows with two norms 13.9 (25.8).
+// Eight rows of 2,048 with two norms and a filter of 4 taps, in bfloat16: 6.1 us (7.8 with 1,024 threads of single elements).
 constexpr int kHeldTaps = 4;
 constexpr int kHeldThreads = 128;
 template <typename TOut, typename TW, bool kVec, int kPer, int kTaps>
@@ -335,6 +355,102 @@ add_layernorm_held_kernel(float* __restrict__ x, const float* __restrict__ delta
     }
 }
 
+// The same for many rows of up to 256 kPer elements in whole 16-byte runs, a wave a row, without a barrier: what bounds them are
+// their bytes, so every row is on its way at once.  Sums in the general kernel's order with 256 threads, for its bits: a lane adds
+// elements 256 apart in turn, those 32, 16, .. 1 apart meet, and the sums of every 64 neighbours are added in turn.  A lane has four
+// neighbours, so the first four meetings are between lanes of a row of 16, the last two in its own registers.
+// With cold caches, two norms (us, before): 2,048 rows of 2,048 20.8 (33.6), of 1,024 12.3 (18.6), 512 rows of 2,048 12.6 (20.0).
+constexpr int kRowThreads = 256;                 // four rows
+template <typename TOut, typename TW, int kPer>
+__global__ void __launch_bounds__(kRowThreads)
+add_layernorm_wave_kernel(float* __restrict__ x, const float* __restrict__ delta, const TW* __restrict__ dw, const TW* __restrict__ db,
+                          float deps, const TW* __restrict__ w, const TW* __restrict__ b, float eps, TOut* __restrict__ y,
+                          const int* __restrict__ rows, int n_out, int hidden) {
+    const int lane = threadIdx.x % kWave;
+    const int out_row = blockIdx.x * (kRowThreads / kWave) + threadIdx.x / kWave;
+    if (out_row >= n_out) return;
+    const long src = rows ? rows[out_row] : out_row;
+    float* xr = x + src * hidden;
+    float v[kPer][4], d[kPer][4];
+    const auto at = [&](int n) { return n * 256 + lane * 4; };
+    const auto place = [&](int n) { return at(n) < hidden ? at(n) : 0; };
+    const auto fetch = [](const float* p, float (&to)[4]) {
+        const float4 four = *reinterpret_cast<const float4*>(p);
+        to[0] = four.x, to[1] = four.y, to[2] = four.z, to[3] = four.w;
+    };
+#pragma unroll
+    for (int n = 0; n < kPer; ++n) fetch(xr + place(n), v[n]);
+    if (delta) {
+#pragma unroll
+        for (int n = 0; n < kPer; ++n) fetch(delta + src * hidden + place(n), d[n]);
+    }
+    const auto row_sum = [&](float (&part)[4]) {
+        constexpr int kRotate8 = 0x128, kRotate4 = 0x124, kSwap1 = 0xb1, kSwap2 = 0x4e;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            part[i] += of_lane<kRotate8>(part[i]);
+            part[i] += of_lane<kRotate4>(part[i]);
+            part[i] += of_lane<kSwap2>(part[i]);
+            part[i] += of_lane<kSwap1>(part[i]);
+        }
+        const float mine = (part[0] + part[2]) + (part[1] + part[3]);
+        float total = 0.f;
+#pragma unroll
+        for (int sixteen = 0; sixteen < 4; ++sixteen)
+            total += __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(mine), sixteen * 16));
+        return total;
+    };
+    const auto moments = [&](const float (&of)[kPer][4], float of_eps, float& mean, float& rstd) {
+        float part[4] = {};
+#pragma unroll
+        for (int n = 0; n < kPer; ++n)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) part[i] += at(n) < hidden ? of[n][i] : 0.f;
+        mean = row_sum(part) / static_cast<float>(hidden);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) part[i] = 0.f;
+#pragma unroll
+        for (int n = 0; n < kPer; ++n)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float off = at(n) < hidden ? of[n][i] - mean : 0.f;
+                part[i] = fmaf(off, off, part[i]);
+            }
+        rstd = 1.0f / sqrtf(row_sum(part) / static_cast<float>(hidden) + of_eps);
+    };
+    if (delta) {
+        float mean = 0.f, rstd = 1.f;
+        if (dw) moments(d, deps, mean, rstd);
+#pragma unroll
+        for (int n = 0; n < kPer; ++n) {
+            if (at(n) >= hidden) continue;
+            Four<TW> gain, bias;
+            if (dw) {
+                gain.load(dw + at(n));
+                bias.load(db + at(n));
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[n][i] += dw ? (d[n][i] - mean) * rstd * gain.get(i) + bias.get(i) : d[n][i];
+            if (!rows) *reinterpret_cast<float4*>(xr + at(n)) = float4{v[n][0], v[n][1], v[n][2], v[n][3]};
+        }
+    }
+    if (!y) return;
+    float mean, rstd;
+    moments(v, eps, mean, rstd);
+    TOut* yr = y + static_cast<long>(out_row) * hidden;
+#pragma unroll
+    for (int n = 0; n < kPer; ++n) {
+        if (at(n) >= hidden) continue;
+        Four<TW> gain, bias;
+        gain.load(w + at(n));
+        bias.load(b + at(n));
+        float h[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) h[i] = (v[n][i] - mean) * rstd * gain.get(i) + bias.get(i);
+        store_four(yr + at(n), h);
+    }
+}
+
 __global__ void entry_spans_kernel(const int* __restrict__ row_entry, const int* __restrict__ positions,
                                    const int* __restrict__ entry_slots, int rows, int* __restrict__ spans) {
     const int r = blockIdx.x * blockDim.x + threadIdx.x;
@@ -411,21 +527,6 @@ __global__ void causal_conv_kernel(const TIn* __restrict__ in, long in_stride, T
 constexpr int kWindowTaps = 4;
 constexpr int kWindowThreads = 256;
 constexpr int kWindowChannels = 4;
-template <typename T>
-struct Four {
-    float4 v;
-    __device__ inline void load(const T* from) { v = *reinterpret_cast<const float4*>(from); }
-    __device__ inline float get(int i) const { return i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w; }
-};
-template <>
-struct Four<bf16_t> {
-    uint2 v;
-    __device__ inline void load(const bf16_t* from) { v = *reinterpret_cast<const uint2*>(from); }
-    __device__ inline float get(int i) const {
-        const unsigned word = i / 2 ? v.y : v.x;
-        return __uint_as_float(i % 2 ? word & 0xffff0000u : word << 16);
-    }
-};
 template <typename TIn, typename TOut>
 __global__ void __launch_bounds__(kWindowThreads)
 causal_conv_window_kernel(const TIn* __restrict__ in, long in_stride, TOut* __restrict__ out, long out_stride, AnyVec w, AnyVec bias,
@@ -494,14 +595,7 @@ causal_conv_window_kernel(const TIn* __restrict__ in, long in_stride, TOut* __re
             for (int j = 0; j + 1 < kBefore; ++j) window[j][i] = window[j + 1][i];
             window[kBefore - 1][i] = now;
         }
-        TOut* to = out + static_cast<long>(r) * out_stride + c;
-        if constexpr (sizeof(TOut) == 4) {
-            *reinterpret_cast<float4*>(to) = float4{result[0], result[1], result[2], result[3]};
-        } else {
-            *reinterpret_cast<uint2*>(to) =
-                uint2{bf16_bits_from_float(result[0]) | static_cast<unsigned>(bf16_bits_from_float(result[1])) << 16,
-                      bf16_bits_from_float(result[2]) | static_cast<unsigned>(bf16_bits_from_float(result[3])) << 16};
-        }
+        store_four(out + static_cast<long>(r) * out_stride + c, result);
     }
 }
 
@@ -722,13 +816,12 @@ extern "C" int leone_add_layernorm(float* x, const float* delta, const void* dw,
                                                                          rows, hidden, vconv, taps, conv_state, write_state,   \
                                                                          positions, row_entry, entry_slots, stage_delta)
     const bool many = n_out >= kNormManyRows;
-    // Rows that fit a workgroup's registers, one type of vectors throughout: whole 16-byte runs whatever the number of rows; else
-    // element by element, where few rows wait for their trips to memory.  (us with cold caches, before and so: 2,048 rows of 2,048 33.6
-    // and 22.0, of 1,024 18.6 and 13.7, 512 rows of 2,048 20.0 and 9.3.)
+    // Rows that fit registers, one type of vectors throughout: few rows by a workgroup each, in whole 16-byte runs where they lie so
+    // and else element by element; many rows by a wave each where they lie in such runs.
     const auto aligned = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
     const bool vec = hidden % kRun == 0 && aligned(x) && aligned(delta) && aligned(dw) && aligned(db) && aligned(w) && aligned(b) &&
                      aligned(y) && (!conv || (taps == kHeldTaps && aligned(conv) && aligned(conv_state)));
-    if (hidden <= 4 * kRun * kHeldThreads && (vec || !many) && (!conv || (taps <= kHeldTaps && conv_dtype == w_dtype))) {
+    if (!many && hidden <= 4 * kRun * kHeldThreads && (!conv || (taps <= kHeldTaps && conv_dtype == w_dtype))) {
 #define LEONE_HELD(T, TW, VEC, PER, TAPS)                                                                                       \
     add_layernorm_held_kernel<T, TW, VEC, PER, TAPS><<<n_out, kHeldThreads, 0, stream>>>(                                       \
         x, delta, static_cast<const TW*>(dw), static_cast<const TW*>(db), deps, static_cast<const TW*>(w), static_cast<const TW*>(b), eps, \
@@ -743,6 +836,21 @@ extern "C" int leone_add_layernorm(float* x, const float* delta, const void* dw,
 #undef LEONE_HELD_PER
 #undef LEONE_HELD_VEC
 #undef LEONE_HELD
+        LEONE_LAUNCH_CHECK("add_layernorm");
+        return 0;
+    }
+    if (many && vec && !conv && hidden <= 4096) {
+#define LEONE_WAVE(T, TW, PER)                                                                                                    \
+    add_layernorm_wave_kernel<T, TW, PER><<<ceil_div(n_out, kRowThreads / kWave), kRowThreads, 0, stream>>>(                      \
+        x, delta, static_cast<const TW*>(dw), static_cast<const TW*>(db), deps, static_cast<const TW*>(w), static_cast<const TW*>(b), eps, \
+        static_cast<T*>(y), rows, n_out, hidden)
+#define LEONE_WAVE_PER(T, TW) (hidden <= 1024 ? LEONE_WAVE(T, TW, 4) : hidden <= 2048 ? LEONE_WAVE(T, TW, 8) : LEONE_WAVE(T, TW, 16))
+        if (y_dtype == kF32 && w_dtype == kF32) LEONE_WAVE_PER(float, float);
+        else if (y_dtype == kF32) LEONE_WAVE_PER(float, bf16_t);
+        else if (w_dtype == kF32) LEONE_WAVE_PER(bf16_t, float);
+        else LEONE_WAVE_PER(bf16_t, bf16_t);
+#undef LEONE_WAVE_PER
+#undef LEONE_WAVE
         LEONE_LAUNCH_CHECK("add_layernorm");
         return 0;
     }

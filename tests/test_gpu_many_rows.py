@@ -82,3 +82,32 @@ def test_exponential_gates(counts):
             assert float((top[first + t] - m).abs().max()) < 1e-4, (e, t)
         assert float((kept[e + 1, :, -1].cpu().double() - m).abs().max()) < 1e-4
         first += n
+
+
+@pytest.mark.parametrize("hidden", [8, 1016, 1032, 2048, 2056, 4096])
+@pytest.mark.parametrize("weights,out", [(torch.bfloat16, torch.bfloat16), (torch.float32, torch.float32), (torch.bfloat16, torch.float32)])
+def test_layer_norms_of_many_rows(hidden, weights, out):
+    """A wave a row, at the lengths where its registers change and where a row ends inside a run of 256, with every set of operands."""
+    from leone_amd import ops
+    gen = torch.Generator().manual_seed(hidden)
+    n = 515
+    x, delta = torch.randn(n, hidden, generator=gen) * 2 + 0.5, torch.randn(n, hidden, generator=gen) - 0.25
+    gain, bias, dgain, dbias = (torch.randn(hidden, generator=gen).to(weights) for _ in range(4))
+
+    def norm(v, g, b, eps):
+        off = v - v.mean(-1, keepdim=True)
+        return off / ((off ** 2).mean(-1, keepdim=True) + eps).sqrt() * g.double() + b.double()
+
+    for with_delta, normed, picked in ((False, False, False), (True, False, False), (True, True, False), (True, True, True)):
+        rows = torch.randint(0, n, (n - 2,), generator=gen, dtype=torch.int32) if picked else None
+        stream = x.to(DEV).clone()
+        y = ops.add_layernorm(stream, delta.to(DEV) if with_delta else None, gain.to(DEV), bias.to(DEV), 1e-5, out,
+                              rows.to(DEV) if picked else None, (dgain.to(DEV), dbias.to(DEV), 1e-6) if normed else None)
+        more = (norm(delta.double(), dgain, dbias, 1e-6) if normed else delta.double()) if with_delta else 0.0
+        total = x.double() + more
+        want = norm(total, gain, bias, 1e-5)
+        want = want[rows.long()] if picked else want
+        # float sums of up to 4,096 terms over 64 lanes, a few roundings behind them; bfloat16 results have eight significant bits (a
+        # row of 8 elements may vary little beside its mean)
+        assert float(((y.cpu().double() - want).abs() / (want.abs() + 1.0)).max()) < (2.0 ** -8 if out == torch.bfloat16 else 0.0) + (4e-6 if hidden > 8 else 2e-5)
+        assert torch.equal(stream.cpu(), x) if picked or not with_delta else float((stream.cpu().double() - total).abs().max()) < 4e-5
