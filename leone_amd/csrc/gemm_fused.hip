@@ -32,6 +32,7 @@
 #include "leone_hip.h"
 
 #include <math.h>
+#include <type_traits>
 
 namespace leone {
 
@@ -109,10 +110,6 @@ gemm_fused_kernel(FusedArgs a) {
     float ss = 0.f;
     const int xr = c < m ? c : m - 1;
     const long xrow_index = (kIn == kInNorm && a.rows) ? a.rows[xr] : xr;
-    // Prepared input: the rows' partial sums of squares ([m][k / 16] floats, k a multiple of 64) go to shared
-    // memory after the walk over K, all threads side by side in 16-byte loads, and wave 0 adds each row's up
-    // in index order.  (Asked for before the walk and kept in registers they cost the kernel a third of the
-    // waves a compute unit holds, and with them the loads in flight that it lives on.)
     constexpr int kQuads = 8;                        // 16-byte loads a thread takes; the entry point checks that they suffice
     extern __shared__ float4 sums_of_squares[];      // [m * k / 64]
     const int quads = kIn == kInPrepared ? m * (k / 64) : 0;
@@ -126,10 +123,9 @@ gemm_fused_kernel(FusedArgs a) {
     floatx4 acc = {0.f, 0.f, 0.f, 0.f};
 
     // One step: 64 elements of K; this lane's run is elements at + 16g .. + 15, `left` of which exist.
-    auto step = [&](int s, bf16x8 a0, bf16x8 a1, bool tail) {
+    auto operand = [&](int s, bool tail, bf16x8 (&b)[2]) {
         const int at = 64 * s;
         const int left = tail ? k - (at + 16 * g) : 16;
-        bf16x8 b[2];
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             if (left < 8 * (h + 1)) {
@@ -149,22 +145,53 @@ gemm_fused_kernel(FusedArgs a) {
                 }
             }
         }
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, b[0], acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, b[1], acc, 0, 0, 0);
     };
 
     // Wave 0, which writes the result, asks for what the epilogue adds to (the stream's values, the next
-    // norm's gains) before the walk over K: after it they would cost one more trip to memory.
-    float stream_before[4] = {0.f, 0.f, 0.f, 0.f}, gain_after[4] = {0.f, 0.f, 0.f, 0.f};
+    // norm's gains) before the walk over K: after it they would cost one more trip to memory.  In whole runs where they lie so, the
+    // gains unpacked where they are used: element by element, each conversion behind its load, they were four trips one after the
+    // other ahead of the walk (1,024 x 1,024 and x 3,072, two rows: 6.5 us each, so 5.2).
+    const int col0 = static_cast<int>(n0) + 4 * g;
+    float4 stream_before = {0.f, 0.f, 0.f, 0.f};
+    [[maybe_unused]] uint4 gain_bits = {0u, 0u, 0u, 0u};
+    const auto at = [](const void* p) { return static_cast<unsigned>(reinterpret_cast<uintptr_t>(p)); };
+    const bool runs = n % 16 == 0 && at(a.y) % 16 == 0 && (kOut != kOutPrepare || (at(a.next_gain) % 16 == 0 && at(a.operand_out) % 8 == 0));
     if ((kOut == kOutPrepare || kOut == kOutResidual) && wave == 0) {
-        const long col = n0 + 4 * g;
-        const float* out = static_cast<const float*>(a.y) + static_cast<long>(c) * n + col;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            if (c < m && col + r < n) {
-                stream_before[r] = out[r];
-                if (kOut == kOutPrepare) gain_after[r] = load_any(AnyVec{a.next_gain, a.next_gain_dtype}, col + r);
+        const float* out = static_cast<const float*>(a.y) + static_cast<long>(xr) * n;
+        if (runs) {
+            stream_before = *reinterpret_cast<const float4*>(out + col0);
+            if (kOut == kOutPrepare && a.next_gain_dtype == kF32) {
+                gain_bits = *reinterpret_cast<const uint4*>(static_cast<const float*>(a.next_gain) + col0);
+            } else if (kOut == kOutPrepare) {
+                const uint2 two = *reinterpret_cast<const uint2*>(static_cast<const bf16_t*>(a.next_gain) + col0);
+                gain_bits.x = two.x, gain_bits.y = two.y;
             }
+        } else {
+            float* before = &stream_before.x;
+            unsigned* bits = &gain_bits.x;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int col = col0 + r < n ? col0 + r : n - 1;
+                before[r] = out[col];
+                if (kOut == kOutPrepare) bits[r] = __float_as_uint(load_any(AnyVec{a.next_gain, a.next_gain_dtype}, col));
+            }
+        }
+    }
+    const auto gain_after = [&](int r) {
+        if (!runs || a.next_gain_dtype == kF32) return __uint_as_float(r == 0 ? gain_bits.x : r == 1 ? gain_bits.y : r == 2 ? gain_bits.z : gain_bits.w);
+        const unsigned word = r / 2 ? gain_bits.y : gain_bits.x;
+        return __uint_as_float(r % 2 ? word & 0xffff0000u : word << 16);
+    };
+    const auto before = [&](int r) { return r == 0 ? stream_before.x : r == 1 ? stream_before.y : r == 2 ? stream_before.z : stream_before.w; };
+
+    // Prepared input: the rows' partial sums of squares ([m][k / 16] floats, k a multiple of 64) go straight into shared memory, all
+    // threads side by side in 16-byte loads that hold no registers over the walk, and wave 0 adds each row's up in index order.
+    if (kIn == kInPrepared) {
+#pragma unroll
+        for (int i = 0; i < kQuads; ++i) {
+            const int first = (i * kWaves + wave) * kWave;
+            if (first + lane < quads)
+                __builtin_amdgcn_global_load_lds(reinterpret_cast<const float4*>(a.squares_in) + first + lane, sums_of_squares + first, 16, 0, 0);
         }
     }
 
@@ -172,38 +199,44 @@ gemm_fused_kernel(FusedArgs a) {
     const int whole = k / 64;                        // steps of 64 elements without a tail
     const int share = (whole + kWaves - 1) / kWaves;
     const int s_end = (wave + 1) * share < whole ? (wave + 1) * share : whole;
-    constexpr int kUnroll = 4;                       // weight loads of four steps are in flight together
+    // The weights of four steps are in flight together.  (With the operand of all four held back as well, 80 registers against 64 and fewer
+    // waves: 8 rows of the 8B sizes 8.79 ms for eight steps against 8.70.)
+    constexpr int kUnroll = 4;
     int s = wave * share;
-    for (; s + kUnroll <= s_end; s += kUnroll) {
-        bf16x8 wa[kUnroll][2];
+    auto steps = [&](auto count) {
+        constexpr int kCount = decltype(count)::value;
+        bf16x8 wa[kCount][2], xa[kCount][2];
 #pragma unroll
-        for (int u = 0; u < kUnroll; ++u) {
+        for (int u = 0; u < kCount; ++u) {
             wa[u][0] = wld(s + u, 0);
             wa[u][1] = wld(s + u, 1);
         }
 #pragma unroll
-        for (int u = 0; u < kUnroll; ++u) step(s + u, wa[u][0], wa[u][1], false);
+        for (int u = 0; u < kCount; ++u) operand(s + u, false, xa[u]);
+#pragma unroll
+        for (int u = 0; u < kCount; ++u)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[u][h], xa[u][h], acc, 0, 0, 0);
+        s += kCount;
+    };
+    while (s + kUnroll <= s_end) steps(std::integral_constant<int, kUnroll>{});
+    switch (s_end - s) {                               // what is left, on its way at once as well
+        case 3: steps(std::integral_constant<int, 3>{}); break;
+        case 2: steps(std::integral_constant<int, 2>{}); break;
+        case 1: steps(std::integral_constant<int, 1>{}); break;
+        default: break;
     }
-    for (; s < s_end; ++s) step(s, wld(s, 0), wld(s, 1), false);
     if (kTail && wave == kWaves - 1) {                 // the last wave also takes the step that holds the end of K
         const int left = k - (64 * whole + 16 * g);
-        step(whole, left >= 8 ? wld(whole, 0) : fz8(), left >= 16 ? wld(whole, 1) : fz8(), true);
+        const bf16x8 w0 = left >= 8 ? wld(whole, 0) : fz8(), w1 = left >= 16 ? wld(whole, 1) : fz8();
+        bf16x8 xa[2];
+        operand(whole, true, xa);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w0, xa[0], acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w1, xa[1], acc, 0, 0, 0);
     }
 #pragma unroll
     for (int r = 0; r < 4; ++r) partial[wave][lane][r] = acc[r];
-    if (kIn == kInPrepared) {
-        float4 held[kQuads];
-#pragma unroll
-        for (int i = 0; i < kQuads; ++i) {
-            const int at = i * kWaves * kWave + static_cast<int>(threadIdx.x);
-            held[i] = at < quads ? reinterpret_cast<const float4*>(a.squares_in)[at] : float4{0.f, 0.f, 0.f, 0.f};
-        }
-#pragma unroll
-        for (int i = 0; i < kQuads; ++i) {
-            const int at = i * kWaves * kWave + static_cast<int>(threadIdx.x);
-            if (at < quads) sums_of_squares[at] = held[i];
-        }
-    }
+    if (kIn == kInPrepared) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     if (kIn == kInNorm) {
         ss = add_lanes<16>(ss);             // the four lanes that share X row c
         ss = add_lanes<32>(ss);
@@ -263,14 +296,27 @@ gemm_fused_kernel(FusedArgs a) {
     if (kOut == kOutPrepare) {
         // every lane takes part in the exchange; rows and columns past the end count as zero
         float* out = static_cast<float*>(a.y) + static_cast<long>(row) * n + col;
-        float squares = 0.f;
+        float squares = 0.f, value[4] = {};
+        unsigned next[4] = {};
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             if (row < m && col + r < n) {
-                const float v = stream_before[r] + sum[r];
-                out[r] = v;
+                const float v = before(r) + sum[r];
+                value[r] = v;
                 squares = fmaf(v, v, squares);
-                a.operand_out[static_cast<long>(row) * n + col + r] = from_float<bf16_t>(v * gain_after[r]);
+                next[r] = bf16_bits_from_float(v * gain_after(r));
+            }
+        }
+        bf16_t* operand = a.operand_out + static_cast<long>(row) * n + col;
+        if (runs && row < m) {
+            *reinterpret_cast<float4*>(out) = float4{value[0], value[1], value[2], value[3]};
+            *reinterpret_cast<uint2*>(operand) = uint2{next[0] | next[1] << 16, next[2] | next[3] << 16};
+        } else {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                if (row >= m || col + r >= n) continue;
+                out[r] = value[r];
+                operand[r].bits = static_cast<uint16_t>(next[r]);
             }
         }
         squares = add_lanes<16>(squares);
@@ -283,7 +329,7 @@ gemm_fused_kernel(FusedArgs a) {
         float* out = static_cast<float*>(a.y) + static_cast<long>(row) * n + col;
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-            if (col + r < n) out[r] = stream_before[r] + sum[r];
+            if (col + r < n) out[r] = before(r) + sum[r];
     } else {
         TOut* out = static_cast<TOut*>(a.y) + static_cast<long>(row) * n + col;
 #pragma unroll
