@@ -503,10 +503,12 @@ attention_prefill_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ out,
 // Merges the key ranges of one row and query head: out = sum_s acc_s 2^(m_s - M) / sum_s l_s 2^(m_s - M),
 // the sums taken in range order; a range that held no key for the row (m_s = -inf) counts as nothing,
 // whatever its accumulator holds.  One wave a (row, head): lane s takes the reference and sum of range s,
-// then all lanes walk the accumulators together.  blockIdx.x is a tile and a quarter of its rows.
+// then all lanes walk the accumulators together.  blockIdx.x is a tile and an eighth of its rows.
+// A wave is a chain of trips to memory: the accumulators of four ranges at a time are asked for before it is known what they weigh.
 constexpr int kMergeWaves = 4;
 constexpr int kMergeThreads = kMergeWaves * kWave;
-constexpr int kMergeBlocksPerTile = kRowsPerWave / kMergeWaves / 2;   // a wave takes two rows, one after the other
+constexpr int kMergeBlocksPerTile = kRowsPerWave / kMergeWaves;
+constexpr int kMergeAhead = 4;                                        // ranges on their way at a time
 constexpr int kMaxPrefillSplits = 32;
 
 __global__ void __launch_bounds__(kMergeThreads)
@@ -520,24 +522,35 @@ attention_prefill_merge_kernel(const float* __restrict__ part_acc, const float* 
         const long rh = static_cast<long>(row0 + r) * q_heads + head;
         const float2 ml = lane < splits ? reinterpret_cast<const float2*>(part_ml)[rh * splits + lane]
                                         : float2{-INFINITY, 0.f};
+        const float* acc = part_acc + rh * splits * head_dim;
+        float ahead[kMergeAhead][4];                             // head_dim <= 256: at most four elements a lane
+        auto ask = [&](int s0) {
+#pragma unroll
+            for (int u = 0; u < kMergeAhead; ++u) {
+                const float* from = acc + static_cast<long>(s0 + u < splits ? s0 + u : splits - 1) * head_dim;
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (kWave * i < head_dim) ahead[u][i] = from[lane + kWave * i < head_dim ? lane + kWave * i : head_dim - 1];
+            }
+        };
+        ask(0);
         const float top = wave_max(ml.x);
         const bool counts = ml.x != -INFINITY;
         const float my_weight = counts ? __builtin_amdgcn_exp2f(ml.x - top) : 0.f;
         // A range without keys for this row has sum 0; a sum that is NaN (a key without a page) still shows.
         const float my_share = counts || ml.y != ml.y ? ml.y * (counts ? my_weight : 1.f) : 0.f;
         float den = 0.f;
-        float num[4] = {0.f, 0.f, 0.f, 0.f};                     // head_dim <= 256: at most four elements a lane
-        const float* acc = part_acc + rh * splits * head_dim;
-        for (int s = 0; s < splits; ++s) {
-            const float weight = __shfl(my_weight, s, kWave);
-            den += __shfl(my_share, s, kWave);
+        float num[4] = {0.f, 0.f, 0.f, 0.f};
+        for (int s0 = 0; s0 < splits; s0 += kMergeAhead) {
+            if (s0 > 0) ask(s0);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int d = lane + kWave * i;
-                if (d < head_dim) {
-                    const float value = acc[static_cast<long>(s) * head_dim + d];   // may be anything where weight is 0
-                    num[i] += weight != 0.f ? value * weight : 0.f;
-                }
+            for (int u = 0; u < kMergeAhead; ++u) {
+                if (s0 + u >= splits) break;
+                const float weight = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(my_weight), s0 + u));
+                den += __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(my_share), s0 + u));
+#pragma unroll
+                for (int i = 0; i < 4; ++i)                      // a value may be anything where its weight is 0
+                    if (kWave * i < head_dim) num[i] += weight != 0.f ? ahead[u][i] * weight : 0.f;
             }
         }
         if (shape.sinks != nullptr) den += __builtin_amdgcn_exp2f(shape.sinks[head] * 1.44269504088896340736f - top);
@@ -568,10 +581,104 @@ attention_prefill_merge_kernel(const float* __restrict__ part_acc, const float* 
     }
 }
 
+// The same for heads of 64, 128 or 256 elements whose results stay as they are: kLanes lanes a row with four elements each, two rows a
+// lane, so that a wave has up to 16 KB on its way and every lane makes its row's weights itself.  Sums in the same order: the same bits.
+// us (a wave a row and an element a lane): 512 rows of 32 heads of 128 in four ranges 9.3 (12.7; 18.5 with a range a trip), 2,048 rows
+// of 16 heads in two 11.3 (18.7).
+template <int kLanes>
+__global__ void __launch_bounds__(kMergeThreads)
+attention_prefill_merge_lanes_kernel(const float* __restrict__ part_acc, const float* __restrict__ part_ml, bf16_t* __restrict__ out,
+                                     const int* __restrict__ tiles, int q_heads, int splits, const float* __restrict__ sinks) {
+    constexpr int kD = 4 * kLanes, kRows = kMergeThreads / kLanes, kEach = 2, kBlocks = kRowsPerWave / (kRows * kEach);
+    static_assert(kBlocks >= 1, "a tile's rows in whole workgroups");
+    const int* tile = tiles + 3 * static_cast<long>(blockIdx.x / kBlocks);
+    const int row0 = tile[1], rows = tile[2], head = blockIdx.y;
+    const int first = (blockIdx.x % kBlocks) * kRows * kEach + threadIdx.x / kLanes, d = 4 * (threadIdx.x % kLanes);
+    if (first >= rows) return;
+    long rh[kEach];
+    float4 ahead[kEach][kMergeAhead];
+    float2 ml[kEach][kMergeAhead];
+#pragma unroll
+    for (int e = 0; e < kEach; ++e) {
+        const int r = first + e * kRows;                          // a row past the tile's last is its first again, and not written
+        rh[e] = static_cast<long>(row0 + (r < rows ? r : first)) * q_heads + head;
+    }
+    const auto ask_weights = [&](int s0) {
+#pragma unroll
+        for (int e = 0; e < kEach; ++e)
+#pragma unroll
+            for (int u = 0; u < kMergeAhead; ++u)
+                if (s0 + u < splits) ml[e][u] = reinterpret_cast<const float2*>(part_ml)[rh[e] * splits + s0 + u];
+    };
+    const auto ask = [&](int s0) {
+#pragma unroll
+        for (int e = 0; e < kEach; ++e)
+#pragma unroll
+            for (int u = 0; u < kMergeAhead; ++u)
+                if (s0 + u < splits) ahead[e][u] = *reinterpret_cast<const float4*>(part_acc + (rh[e] * splits + s0 + u) * kD + d);
+    };
+    ask_weights(0);
+    ask(0);
+    float top[kEach], den[kEach] = {}, num[kEach][4] = {};
+#pragma unroll
+    for (int e = 0; e < kEach; ++e) top[e] = -INFINITY;
+    for (int s0 = 0; s0 < splits; s0 += kMergeAhead) {
+        if (s0 > 0) ask_weights(s0);
+#pragma unroll
+        for (int e = 0; e < kEach; ++e)
+#pragma unroll
+            for (int u = 0; u < kMergeAhead; ++u)
+                if (s0 + u < splits) top[e] = fmaxf(top[e], ml[e][u].x);
+    }
+    for (int s0 = 0; s0 < splits; s0 += kMergeAhead) {
+        if (splits > kMergeAhead) ask_weights(s0);
+        if (s0 > 0) ask(s0);
+#pragma unroll
+        for (int e = 0; e < kEach; ++e)
+#pragma unroll
+            for (int u = 0; u < kMergeAhead; ++u) {
+                if (s0 + u >= splits) continue;
+                const float2 of = ml[e][u];
+                const bool counts = of.x != -INFINITY;
+                const float weight = counts ? __builtin_amdgcn_exp2f(of.x - top[e]) : 0.f;
+                // a range without keys for this row has sum 0; a sum that is NaN (a key without a page) still shows
+                den[e] += counts || of.y != of.y ? of.y * (counts ? weight : 1.f) : 0.f;
+                const float4 v = ahead[e][u];                     // may be anything where the weight is 0
+                num[e][0] += weight != 0.f ? v.x * weight : 0.f;
+                num[e][1] += weight != 0.f ? v.y * weight : 0.f;
+                num[e][2] += weight != 0.f ? v.z * weight : 0.f;
+                num[e][3] += weight != 0.f ? v.w * weight : 0.f;
+            }
+    }
+#pragma unroll
+    for (int e = 0; e < kEach; ++e) {
+        if (first + e * kRows >= rows) continue;
+        if (sinks != nullptr) den[e] += __builtin_amdgcn_exp2f(sinks[head] * 1.44269504088896340736f - top[e]);
+        const uint2 packed = {bf16_bits_from_float(num[e][0] / den[e]) | static_cast<uint32_t>(bf16_bits_from_float(num[e][1] / den[e])) << 16,
+                              bf16_bits_from_float(num[e][2] / den[e]) | static_cast<uint32_t>(bf16_bits_from_float(num[e][3] / den[e])) << 16};
+        *reinterpret_cast<uint2*>(out + rh[e] * kD + d) = packed;
+    }
+}
+
+static void launch_merge(const float* part_acc, const float* part_ml, bf16_t* out, const int* tiles, int n_tiles, int q_heads, int head_dim,
+                         int splits, const int* positions, const ScoreShape& shape, hipStream_t stream) {
+#define LEONE_MERGE_LANES(LANES)                                                                                                \
+    attention_prefill_merge_lanes_kernel<LANES><<<dim3(n_tiles * (kRowsPerWave * LANES / (2 * kMergeThreads)), q_heads), kMergeThreads, 0, \
+                                                  stream>>>(part_acc, part_ml, out, tiles, q_heads, splits, shape.sinks)
+    const bool as_they_are = shape.turn_cos == nullptr && reinterpret_cast<uintptr_t>(part_acc) % 16 == 0 &&
+                             reinterpret_cast<uintptr_t>(part_ml) % 8 == 0 && reinterpret_cast<uintptr_t>(out) % 8 == 0;
+    if (as_they_are && head_dim == 64) LEONE_MERGE_LANES(16);
+    else if (as_they_are && head_dim == 128) LEONE_MERGE_LANES(32);
+    else if (as_they_are && head_dim == 256) LEONE_MERGE_LANES(64);
+    else
+        attention_prefill_merge_kernel<<<dim3(n_tiles * kMergeBlocksPerTile, q_heads), kMergeThreads, 0, stream>>>(
+            part_acc, part_ml, out, tiles, q_heads, head_dim, splits, positions, shape);
+#undef LEONE_MERGE_LANES
+}
+
 void launch_attention_tile_merge(const float* part_acc, const float* part_ml, bf16_t* out, const int* tiles, int n_tiles, int q_heads,
                                  int head_dim, int splits, hipStream_t stream) {
-    attention_prefill_merge_kernel<<<dim3(n_tiles * kMergeBlocksPerTile, q_heads), kMergeThreads, 0, stream>>>(
-        part_acc, part_ml, out, tiles, q_heads, head_dim, splits, nullptr, ScoreShape{});
+    launch_merge(part_acc, part_ml, out, tiles, n_tiles, q_heads, head_dim, splits, nullptr, ScoreShape{}, stream);
 }
 int attention_tile_merge_max_splits() { return kMaxPrefillSplits; }
 
@@ -708,9 +815,8 @@ extern "C" int leone_attention_prefill_shaped(const void* q, void* out, const vo
     if (status) return status;
     LEONE_LAUNCH_CHECK("attention_prefill");
     if (splits > 1) {
-        attention_prefill_merge_kernel<<<dim3(n_groups * kPrefillWaves * kMergeBlocksPerTile, q_heads), kMergeThreads, 0,
-                                         stream>>>(
-            part_acc, part_ml, static_cast<bf16_t*>(out), tiles, q_heads, head_dim, splits, positions, shape);
+        launch_merge(part_acc, part_ml, static_cast<bf16_t*>(out), tiles, n_groups * kPrefillWaves, q_heads, head_dim, splits, positions,
+                     shape, stream);
         LEONE_LAUNCH_CHECK("attention_prefill_merge");
     }
     return 0;
