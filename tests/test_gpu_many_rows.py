@@ -111,3 +111,17 @@ def test_layer_norms_of_many_rows(hidden, weights, out):
         # row of 8 elements may vary little beside its mean)
         assert float(((y.cpu().double() - want).abs() / (want.abs() + 1.0)).max()) < (2.0 ** -8 if out == torch.bfloat16 else 0.0) + (4e-6 if hidden > 8 else 2e-5)
         assert torch.equal(stream.cpu(), x) if picked or not with_delta else float((stream.cpu().double() - total).abs().max()) < 4e-5
+
+
+@pytest.mark.parametrize("kind", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("heads,vdim", [(16, 1), (20, 1), (5, 8), (3, 24), (7, 6)])
+def test_gates_on_attentions_output(kind, heads, vdim):
+    """A gate an element and a gate a head, in runs of eight and where a row does not lie in such runs."""
+    from leone_amd import ops
+    gen = torch.Generator().manual_seed(heads * vdim)
+    rows = 300
+    out, gate = torch.randn(rows, heads * vdim, generator=gen).to(kind), torch.randn(rows, heads + 12, generator=gen) * 3
+    for first in (0, 4, 5):
+        got = ops.head_gate(out.to(DEV).clone(), gate.to(DEV)[:, first:first + heads], heads, vdim).cpu().double()
+        want = out.double() * torch.sigmoid(gate.double()[:, first:first + heads]).repeat_interleave(vdim, 1)
+        assert float(((got - want).abs() / (want.abs() + 1e-3)).max()) < (2.0 ** -8 if kind == torch.bfloat16 else 2e-6)
