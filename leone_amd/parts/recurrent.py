@@ -196,7 +196,7 @@ class ChannelDeltaMixer(Part):
         self.columns = {"q": 0, "k": qk, "v": 2 * qk, "b": 2 * qk + vv, "a1": 2 * qk + vv + self.heads,
                         "g1": 2 * qk + vv + self.heads + self.a_rank}
         self.conv_width = 2 * qk + vv
-        self.w_in = self.w_a2 = self.w_g2 = self.w_o = self.norm = self.rate_log = self.step_bias = None
+        self.w_in = self.w_a2 = self.w_g2 = self.w_low = self.w_o = self.norm = self.rate_log = self.step_bias = None
 
     def tensor_specs(self) -> List[TensorSpec]:
         n, qk, vv = self.names, self.kv_heads * self.dim, self.heads * self.vdim
@@ -211,8 +211,12 @@ class ChannelDeltaMixer(Part):
 
     def bind(self, tensors: Dict[str, torch.Tensor]) -> None:
         self.w_in = torch.cat([tensors.pop(self.names[k]) for k in ("q", "k", "v", "b", "a1", "g1")], dim=0).contiguous()
+        # the wide halves of the two low-rank pairs; of one rank they lie together and are one launch in steps of few rows
         self.w_a2 = tensors.pop(self.names["a2"]).contiguous()
         self.w_g2 = tensors.pop(self.names["g2"]).contiguous()
+        self.w_low = torch.cat([self.w_a2, self.w_g2], dim=0).contiguous() if self.a_rank == self.g_rank else None
+        if self.w_low is not None:
+            self.w_a2, self.w_g2 = self.w_low[:self.heads * self.dim], self.w_low[self.heads * self.dim:]
         self.w_o = tensors.pop(self.names["o"]).contiguous()
         self.norm = tensors.pop(self.names["norm"]).contiguous()
         self.rate_log = tensors.pop(self.names["A_log"]).contiguous()
@@ -232,8 +236,13 @@ class ChannelDeltaMixer(Part):
         proj = ops.linear(h, self.w_in, out_dtype=torch.float32)
         qkv = self.conv.forward(proj[:, :self.conv_width], step, cache["conv"], torch.float32)
         # the two low-rank pairs: their narrow halves came out of the fused product
-        step_size = ops.linear(proj[:, c["a1"]:c["g1"]].to(step.dtype).contiguous(), self.w_a2, out_dtype=torch.float32)
-        gate = ops.linear(proj[:, c["g1"]:].to(step.dtype).contiguous(), self.w_g2, out_dtype=torch.float32)
+        if self.w_low is not None and step.dtype == torch.bfloat16:
+            narrow = torch.empty((2, proj.shape[0], self.a_rank), dtype=step.dtype, device=proj.device)
+            narrow.copy_(proj[:, c["a1"]:].unflatten(1, (2, self.a_rank)).transpose(0, 1))
+            step_size, gate = ops.linear_planes(narrow, self.w_low, [self.w_a2.shape[0], self.w_g2.shape[0]])
+        else:
+            step_size = ops.linear(proj[:, c["a1"]:c["g1"]].to(step.dtype).contiguous(), self.w_a2, out_dtype=torch.float32)
+            gate = ops.linear(proj[:, c["g1"]:].to(step.dtype).contiguous(), self.w_g2, out_dtype=torch.float32)
         memory = cache["memory"]
         o = ops.delta_scan(qkv, {"q": c["q"], "k": c["k"], "v": c["v"]}, proj[:, c["b"]:c["a1"]], step_size,
                            self.rate_log, self.step_bias, memory.state, step, self.heads, self.kv_heads, self.dim,
