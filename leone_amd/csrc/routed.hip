@@ -22,6 +22,7 @@
 #include "leone_hip.h"
 
 #include <math.h>
+#include <type_traits>
 
 namespace leone {
 
@@ -488,7 +489,7 @@ __device__ inline moe_bf16x8 moe_zero8() {
 constexpr int kStreamedInner = 2048;
 
 template <int kMode, bool kStreamed>
-__global__ void __launch_bounds__(kMoeThreads, 3)
+__global__ void __launch_bounds__(kMoeThreads, 4)
 moe_product_stream_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, void* __restrict__ y,
                           const float* __restrict__ pair_weight, const int* __restrict__ tile_expert,
                           const int* __restrict__ tile_pairs, int top, int n, int k, int act, float limit) {
@@ -496,41 +497,76 @@ moe_product_stream_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict
     constexpr int kDepth = 8;
     __shared__ moe_floatx4 sums[kGated ? 2 : 1][kMoeWaves][kWave];
     const int tile = blockIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
+    const int c = lane & 15, g = lane >> 4;
+    const int* my_pairs = tile_pairs + static_cast<long>(tile) * 16;
+    const int own = my_pairs[c], first_pair = my_pairs[0];
     const int e = tile_expert[tile];
     if (e < 0) return;
-    const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-    const int c = lane & 15, g = lane >> 4;
     const int row0 = blockIdx.y * 16;
-    const int pair = tile_pairs[static_cast<long>(tile) * 16 + c];
     const long matrix = static_cast<long>(n) * k;
-    const bool row_ok = row0 + c < n;
-    const bf16_t* wa = w + static_cast<long>(e) * (kGated ? 2 : 1) * matrix + static_cast<long>(row_ok ? row0 + c : 0) * k;
-    const bf16_t* xrow = x + static_cast<long>(pair < 0 ? 0 : (kMode != kMoeDown ? pair / top : pair)) * k;
+    // Lanes past the last row take that one again, lanes without a pair the tile's first: their results are not written.  Nothing
+    // stands between the loads: behind one that may not have been asked for the compiler cannot count those in flight and waits for all.
+    const bf16_t* wa = w + static_cast<long>(e) * (kGated ? 2 : 1) * matrix + static_cast<long>(row0 + c < n ? row0 + c : n - 1) * k;
+    const int pair = own < 0 ? first_pair : own;
+    const bf16_t* xrow = x + static_cast<long>(kMode != kMoeDown ? pair / top : pair) * k;
     const int steps = (k + 31) / 32, share = (steps + kMoeWaves - 1) / kMoeWaves;
-    const int last = (wave + 1) * share < steps ? (wave + 1) * share : steps;
+    const int first = wave * share, last = first + share < steps ? first + share : steps;
     moe_floatx4 acc = {0.f, 0.f, 0.f, 0.f}, acc2 = {0.f, 0.f, 0.f, 0.f};
     moe_bf16x8 a[kDepth], a2[kGated ? kDepth : 1], xb[kDepth];
     const auto weights = [](const bf16_t* p) { return kStreamed ? __builtin_bit_cast(moe_bf16x8, load_streamed16(p)) : moe_load8(p); };
-#define LEONE_MOE_FETCH(D, S)                                                                                  \
-    {                                                                                                          \
-        const int at = 32 * (S) + 8 * g;                                                                       \
-        const bool in = (S) < last && at < k;                                                                  \
-        a[D] = (row_ok && in) ? weights(wa + at) : moe_zero8();        \
-        if constexpr (kGated)                                                                                  \
-            a2[D] = (row_ok && in) ? weights(wa + matrix + at) : moe_zero8(); \
-        xb[D] = (pair >= 0 && in) ? moe_load8(xrow + at) : moe_zero8();                                        \
-    }
+    const auto ask = [&](int d, const bf16_t* of_w, const bf16_t* of_x) {
+        a[d] = weights(of_w);
+        if constexpr (kGated) a2[d] = weights(of_w + matrix);
+        xb[d] = moe_load8(of_x);
+    };
+    const auto multiply = [&](int d) {
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[d], xb[d], acc, 0, 0, 0);
+        if constexpr (kGated) acc2 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2[d], xb[d], acc2, 0, 0, 0);
+    };
+    const int whole = last * 32 <= k ? last : last - 1;          // steps without the inner size's end
+    const bf16_t *from_w = wa + 32 * first + 8 * g, *from_x = xrow + 32 * first + 8 * g;
+    int left = whole > first ? whole - first : 0;
+    if (left >= kDepth) {
 #pragma unroll
-    for (int d = 0; d < kDepth; ++d) LEONE_MOE_FETCH(d, wave * share + d)
-    for (int s = wave * share; s < last; s += kDepth) {
+        for (int d = 0; d < kDepth; ++d) ask(d, from_w + 32 * d, from_x + 32 * d);
+        for (; left >= 2 * kDepth; left -= kDepth) {
+            from_w += 32 * kDepth, from_x += 32 * kDepth;
 #pragma unroll
-        for (int d = 0; d < kDepth; ++d) {
-            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[d], xb[d], acc, 0, 0, 0);          // zeros past the wave's share
-            if constexpr (kGated) acc2 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2[d], xb[d], acc2, 0, 0, 0);
-            LEONE_MOE_FETCH(d, s + kDepth + d)
+            for (int d = 0; d < kDepth; ++d) {
+                multiply(d);
+                ask(d, from_w + 32 * d, from_x + 32 * d);
+            }
         }
+#pragma unroll
+        for (int d = 0; d < kDepth; ++d) multiply(d);
+        from_w += 32 * kDepth, from_x += 32 * kDepth, left -= kDepth;
     }
-#undef LEONE_MOE_FETCH
+    const auto rest = [&](auto count) {
+#pragma unroll
+        for (int d = 0; d < decltype(count)::value; ++d) ask(d, from_w + 32 * d, from_x + 32 * d);
+#pragma unroll
+        for (int d = 0; d < decltype(count)::value; ++d) multiply(d);
+    };
+    switch (left) {
+        case 7: rest(std::integral_constant<int, 7>{}); break;
+        case 6: rest(std::integral_constant<int, 6>{}); break;
+        case 5: rest(std::integral_constant<int, 5>{}); break;
+        case 4: rest(std::integral_constant<int, 4>{}); break;
+        case 3: rest(std::integral_constant<int, 3>{}); break;
+        case 2: rest(std::integral_constant<int, 2>{}); break;
+        case 1: rest(std::integral_constant<int, 1>{}); break;
+        default: break;
+    }
+    if (first < last && whole < last) {                            // the step that holds the inner size's end; zeros beyond it
+        const int wanted = 32 * whole + 8 * g, at = wanted < k ? wanted : k - 8;
+        ask(0, wa + at, xrow + at);
+        if (wanted >= k) {
+            a[0] = xb[0] = moe_zero8();
+            if constexpr (kGated) a2[0] = moe_zero8();
+        }
+        multiply(0);
+    }
     sums[0][wave][lane] = acc;
     if constexpr (kGated) sums[1][wave][lane] = acc2;
     __syncthreads();
@@ -568,6 +604,14 @@ moe_product_stream_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict
 constexpr int kBigPairs = 64;
 constexpr int kBigRows = 128;
 constexpr int kBigChunk = 64;
+
+// Where 16-byte piece `quarter` of a row's half chunk lies in its half: rows of four pieces, the pieces of every fourth row turned
+// about, so that the same piece of 16 neighbouring rows lies in 16 places of the 256 bytes that shared memory gives at a time.  The
+// second half begins 128 bytes past the first one's end: a row's two halves, written side by side, then meet in no bank either.
+// (Rows one after the other as they came: half of shared memory's time went to conflicts, and it was busy for 55 % of the first
+// product's: 121 us for 7,700 pairs, 32 experts of 2,048 x 768.)
+__device__ inline int piece_at(int row, int quarter) { return row * 4 + (quarter ^ ((row >> 2) & 3)); }
+constexpr int half_pieces(int rows) { return rows * 4 + 8; }
 
 // Rows r .. r + 3 of a pair's result, r < n.
 template <int kMode>
@@ -608,8 +652,9 @@ moe_product_tiled_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict_
     constexpr int kXPieces = kBigPairs / kBring;                         // 16-byte pieces of x a thread brings per chunk
     constexpr int kWPieces = kBigRows / kBring;
     constexpr int kPB = 2;                                            // blocks of 16 pairs a wave
-    __shared__ uint4 sx[2][2 * kBigPairs * 4];                           // [chunk][half][row][4 pieces]
-    __shared__ uint4 sw[2][2 * kBigRows * 4];
+    constexpr int kXHalf = half_pieces(kBigPairs), kWHalf = half_pieces(kBigRows);
+    __shared__ uint4 sx[2][2 * kXHalf];                                  // [chunk][half][piece_at]
+    __shared__ uint4 sw[2][2 * kWHalf];
     // Workgroups go to the eight dies in turn, and each die has a cache of its own: the work is numbered so that a
     // die gets a run of neighbouring (row block, tile) places, tiles fastest: the tiles of one expert, which read the
     // same rows of its matrix, then lie on one die.  (Groups of two or four tiles with all their row blocks measured the same.)
@@ -634,39 +679,41 @@ moe_product_tiled_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict_
     const bf16_t* x_from[kXPieces];
     const bf16_t* w_from[kWPieces];
 #pragma unroll
-    for (int i = 0; i < kXPieces; ++i) {
-        const int pair = my_pairs[tid / 8 + kBring * i];
-        x_from[i] = pair < 0 ? nullptr : x + static_cast<long>(kMode != kMoeDown ? pair / top : pair) * k + 8 * part;
+    for (int i = 0; i < kXPieces; ++i) {                                  // (in place of no pair or row, another one: not written)
+        const int own = my_pairs[tid / 8 + kBring * i], pair = own < 0 ? my_pairs[0] : own;
+        x_from[i] = x + static_cast<long>(kMode != kMoeDown ? pair / top : pair) * k;
     }
 #pragma unroll
     for (int i = 0; i < kWPieces; ++i) {
         const int local = tid / 8 + kBring * i;                           // gated: rows 0..63 gate, 64..127 up
         const int row = row_base + local % kOwnRows;
-        w_from[i] = row >= n ? nullptr
-                             : w + static_cast<long>(e) * (kGated ? 2 : 1) * matrix + (local >= kOwnRows ? matrix : 0) +
-                                   static_cast<long>(row) * k + 8 * part;
+        w_from[i] = w + static_cast<long>(e) * (kGated ? 2 : 1) * matrix + (local >= kOwnRows ? matrix : 0) +
+                    static_cast<long>(row < n ? row : n - 1) * k;
     }
     struct Pieces {
         uint4 x[kXPieces], w[kWPieces];
     };
+    const int chunks = (k + kBigChunk - 1) / kBigChunk;
+    // Every call loads, past the inner size's end its last piece again, and in place of no pair the tile's first one: behind a load
+    // that may not have been asked for the compiler cannot count those in flight, and waited for both chunks where one was needed.
     auto bring = [&](int chunk, Pieces& to) {
-        const bool in = chunk * kBigChunk + 8 * part < k;
+        const int wanted = chunk * kBigChunk + 8 * part, at = wanted < k ? wanted : k - 8;
 #pragma unroll
-        for (int i = 0; i < kWPieces; ++i) {
-            to.w[i] = uint4{0u, 0u, 0u, 0u};
-            if (w_from[i] && in) to.w[i] = *reinterpret_cast<const uint4*>(w_from[i] + static_cast<long>(chunk) * kBigChunk);
-        }
+        for (int i = 0; i < kWPieces; ++i) to.w[i] = *reinterpret_cast<const uint4*>(w_from[i] + at);
 #pragma unroll
-        for (int i = 0; i < kXPieces; ++i) {
-            to.x[i] = uint4{0u, 0u, 0u, 0u};
-            if (x_from[i] && in) to.x[i] = *reinterpret_cast<const uint4*>(x_from[i] + static_cast<long>(chunk) * kBigChunk);
-        }
+        for (int i = 0; i < kXPieces; ++i) to.x[i] = *reinterpret_cast<const uint4*>(x_from[i] + at);
     };
-    auto put = [&](const Pieces& from, int at) {
+    auto put = [&](Pieces& from, int chunk, int at) {
+        if (chunk >= chunks - 1 && chunk * kBigChunk + 8 * part >= k) {      // beyond the inner size: zeros
 #pragma unroll
-        for (int i = 0; i < kXPieces; ++i) sx[at][(half * kBigPairs + tid / 8 + kBring * i) * 4 + quarter] = from.x[i];
+            for (int i = 0; i < kXPieces; ++i) from.x[i] = uint4{0u, 0u, 0u, 0u};
 #pragma unroll
-        for (int i = 0; i < kWPieces; ++i) sw[at][(half * kBigRows + tid / 8 + kBring * i) * 4 + quarter] = from.w[i];
+            for (int i = 0; i < kWPieces; ++i) from.w[i] = uint4{0u, 0u, 0u, 0u};
+        }
+#pragma unroll
+        for (int i = 0; i < kXPieces; ++i) sx[at][half * kXHalf + piece_at(tid / 8 + kBring * i, quarter)] = from.x[i];
+#pragma unroll
+        for (int i = 0; i < kWPieces; ++i) sw[at][half * kWHalf + piece_at(tid / 8 + kBring * i, quarter)] = from.w[i];
     };
     // a wave's four blocks of 16 rows: gated, two of gate rows and two of their up rows
     auto row_of = [&](int t) { return kGated ? (t / 2) * kOwnRows + 32 * wr + 16 * (t % 2) : 64 * wr + 16 * t; };
@@ -676,30 +723,48 @@ moe_product_tiled_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict_
         for (int h = 0; h < 2; ++h) {
             moe_bf16x8 a[4], b[kPB];
 #pragma unroll
-            for (int t = 0; t < 4; ++t) a[t] = __builtin_bit_cast(moe_bf16x8, sw[at][(h * kBigRows + row_of(t) + c) * 4 + g]);
+            for (int t = 0; t < 4; ++t) a[t] = __builtin_bit_cast(moe_bf16x8, sw[at][h * kWHalf + piece_at(row_of(t) + c, g)]);
 #pragma unroll
-            for (int t = 0; t < kPB; ++t) b[t] = __builtin_bit_cast(moe_bf16x8, sx[at][(h * kBigPairs + 32 * wp + 16 * t + c) * 4 + g]);
+            for (int t = 0; t < kPB; ++t) b[t] = __builtin_bit_cast(moe_bf16x8, sx[at][h * kXHalf + piece_at(32 * wp + 16 * t + c, g)]);
 #pragma unroll
             for (int ta = 0; ta < 4; ++ta)
 #pragma unroll
                 for (int tb = 0; tb < kPB; ++tb) acc[ta][tb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[ta], b[tb], acc[ta][tb], 0, 0, 0);
         }
     };
-    const int chunks = (k + kBigChunk - 1) / kBigChunk;
     Pieces even, odd;                                  // chunks 1, 3, .. of the loop below come in `odd`, 2, 4, .. in `even`
     bring(0, even);
     bring(1, odd);
-    put(even, 0);
-    bring(2, even);                                    // past the last chunk: zeros, and nothing read
-    for (int ck = 0; ck < chunks; ck += 2) {
+    put(even, 0, 0);
+    bring(2, even);
+    int ck = 0;
+    for (; ck + 4 < chunks; ck += 2) {
         __syncthreads();                               // chunk ck lies ready, and nobody reads the other place any more
-        put(odd, 1);
+        put(odd, ck + 1, 1);
+        __builtin_amdgcn_sched_barrier(0);             // asked for earlier a chunk would take registers of its own, later it would come late
         bring(ck + 3, odd);
+        __builtin_amdgcn_sched_barrier(0);
         work(0);
-        if (ck + 1 >= chunks) break;
         __syncthreads();
-        put(even, 0);
+        put(even, ck + 2, 0);
+        __builtin_amdgcn_sched_barrier(0);
         bring(ck + 4, even);
+        __builtin_amdgcn_sched_barrier(0);
+        work(1);
+    }
+    // the last one to four chunks; behind an odd number of them one of zeros
+    __syncthreads();
+    put(odd, ck + 1, 1);
+    if (ck + 3 < chunks) bring(ck + 3, odd);
+    work(0);
+    __syncthreads();
+    put(even, ck + 2, 0);
+    work(1);
+    if (ck + 2 < chunks) {
+        __syncthreads();
+        put(odd, ck + 3, 1);
+        work(0);
+        __syncthreads();
         work(1);
     }
     // lane (c, g) holds rows 4 g .. 4 g + 3 of pair c of every (ta, tb)
@@ -740,8 +805,9 @@ moe_product_wide_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__
     constexpr int kWRows = kGated ? 2 * kWideRows : kWideRows;          // rows of the matrix in a chunk
     constexpr int kXPieces = kWidePairs * 8 / kMoeThreads;             // 16-byte pieces of x a thread brings per chunk
     constexpr int kWPieces = kWRows * 8 / kMoeThreads;
-    __shared__ uint4 sx[2 * kWidePairs * 4];                           // [half][row][4 pieces]
-    __shared__ uint4 sw[2 * kWRows * 4];
+    constexpr int kXHalf = half_pieces(kWidePairs), kWHalf = half_pieces(kWRows);
+    __shared__ uint4 sx[2 * kXHalf];                                   // [half][piece_at]
+    __shared__ uint4 sw[2 * kWHalf];
     // Workgroups go to the eight dies in turn, and each die has a cache of its own: the work is numbered so that a
     // die gets a run of neighbouring (row block, tile) places, tiles fastest: the tiles of one expert, which read the
     // same rows of its matrix, then lie on one die.
@@ -804,9 +870,9 @@ moe_product_wide_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__
     LEONE_MOE_BRING(0)
     for (int ck = 0; ck < chunks; ++ck) {
 #pragma unroll
-        for (int i = 0; i < kXPieces; ++i) sx[(half * kWidePairs + tid / 8 + 32 * i) * 4 + quarter] = hx[i];
+        for (int i = 0; i < kXPieces; ++i) sx[half * kXHalf + piece_at(tid / 8 + 32 * i, quarter)] = hx[i];
 #pragma unroll
-        for (int i = 0; i < kWPieces; ++i) sw[(half * kWRows + tid / 8 + 32 * i) * 4 + quarter] = hw[i];
+        for (int i = 0; i < kWPieces; ++i) sw[half * kWHalf + piece_at(tid / 8 + 32 * i, quarter)] = hw[i];
         __syncthreads();
         if (ck + 1 < chunks) LEONE_MOE_BRING((ck + 1) * kBigChunk)
 #pragma unroll
@@ -814,9 +880,9 @@ moe_product_wide_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__
             moe_bf16x8 a[4], a2[kGated ? 4 : 1], b[4];
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
-                a[t] = __builtin_bit_cast(moe_bf16x8, sw[(h * kWRows + 64 * wr + 16 * t + c) * 4 + g]);
-                if constexpr (kGated) a2[t] = __builtin_bit_cast(moe_bf16x8, sw[(h * kWRows + kWideRows + 64 * wr + 16 * t + c) * 4 + g]);
-                b[t] = __builtin_bit_cast(moe_bf16x8, sx[(h * kWidePairs + 64 * wp + 16 * t + c) * 4 + g]);
+                a[t] = __builtin_bit_cast(moe_bf16x8, sw[h * kWHalf + piece_at(64 * wr + 16 * t + c, g)]);
+                if constexpr (kGated) a2[t] = __builtin_bit_cast(moe_bf16x8, sw[h * kWHalf + piece_at(kWideRows + 64 * wr + 16 * t + c, g)]);
+                b[t] = __builtin_bit_cast(moe_bf16x8, sx[h * kXHalf + piece_at(64 * wp + 16 * t + c, g)]);
             }
 #pragma unroll
             for (int ta = 0; ta < 4; ++ta)
