@@ -410,9 +410,9 @@ __device__ inline void load_run(const AnyVec& v, int at, float out[8]) {
     }
 }
 
-template <typename T>
-__device__ inline void value_write_block(T* turned, int row_block, int kvh, const T* __restrict__ qkv, T* __restrict__ v_pool,
-                                         const int* __restrict__ positions, const int* __restrict__ row_entry,
+template <typename TIn, typename T>
+__device__ inline void value_write_block(T* turned, int row_block, int kvh, const TIn* __restrict__ qkv, long row_width,
+                                         T* __restrict__ v_pool, const int* __restrict__ positions, const int* __restrict__ row_entry,
                                          const int* __restrict__ block_table, int max_blocks, int rows, int q_heads,
                                          int kv_heads, int head_dim, int page_tokens);
 
@@ -432,8 +432,9 @@ qk_norm_rope_write_runs_kernel(
         if constexpr (std::is_same<TIn, T>::value) {
             extern __shared__ __align__(32) unsigned char turned_raw[];
             const int at = value_blocks - static_cast<int>(gridDim.x - blockIdx.x);
-            value_write_block<T>(reinterpret_cast<T*>(turned_raw), at / kv_heads, at % kv_heads, qkv, v_pool, positions, row_entry,
-                                 block_table, max_blocks, rows, q_heads, kv_heads, kD, page_tokens);
+            value_write_block<T, T>(reinterpret_cast<T*>(turned_raw), at / kv_heads, at % kv_heads, qkv,
+                                    static_cast<long>(q_heads + 2 * kv_heads) * kD, v_pool, positions, row_entry, block_table, max_blocks,
+                                    rows, q_heads, kv_heads, kD, page_tokens);
         }
         return;
     }
@@ -545,14 +546,13 @@ qk_norm_rope_write_runs_kernel(
 // turns them in shared memory and writes head_dim runs that lie side by side.  Rows that do not line
 // up like that (the first and last rows of a portion, single decoded tokens) are written one element
 // at a time.  One thread an element of the head.
-template <typename T>
-__device__ inline void value_write_block(T* turned, int row_block, int kvh, const T* __restrict__ qkv, T* __restrict__ v_pool,
-                                         const int* __restrict__ positions, const int* __restrict__ row_entry,
+template <typename TIn, typename T>
+__device__ inline void value_write_block(T* turned, int row_block, int kvh, const TIn* __restrict__ qkv, long row_width,
+                                         T* __restrict__ v_pool, const int* __restrict__ positions, const int* __restrict__ row_entry,
                                          const int* __restrict__ block_table, int max_blocks, int rows, int q_heads,
                                          int kv_heads, int head_dim, int page_tokens) {
     const int row0 = row_block * 8;
     const int d = threadIdx.x;                                          // blockDim.x >= head_dim; threads beyond it only copy
-    const int qkv_width = (q_heads + 2 * kv_heads) * head_dim;
     const long head_at = static_cast<long>(q_heads + kv_heads + kvh) * head_dim;
     const int n = rows - row0 < 8 ? rows - row0 : 8;
     const int p0 = positions[row0], e0 = row_entry[row0];
@@ -561,8 +561,14 @@ __device__ inline void value_write_block(T* turned, int row_block, int kvh, cons
     // rows in, a run of eight elements a thread
     for (int idx = threadIdx.x; idx < n * (head_dim / 8); idx += blockDim.x) {
         const int r = idx / (head_dim / 8), chunk = idx % (head_dim / 8);
-        *reinterpret_cast<HeadRun<T>*>(turned + r * head_dim + 8 * chunk) =
-            *reinterpret_cast<const HeadRun<T>*>(qkv + static_cast<long>(row0 + r) * qkv_width + head_at + 8 * chunk);
+        const HeadRun<TIn> in = *reinterpret_cast<const HeadRun<TIn>*>(qkv + (row0 + r) * row_width + head_at + 8 * chunk);
+        HeadRun<T> run;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            if constexpr (std::is_same<TIn, T>::value) run.v[i] = in.v[i];
+            else run.v[i] = from_float<T>(to_float(in.v[i]));
+        }
+        *reinterpret_cast<HeadRun<T>*>(turned + r * head_dim + 8 * chunk) = run;
     }
     __syncthreads();
     if (d >= head_dim) return;
@@ -591,8 +597,153 @@ value_write_kernel(const T* __restrict__ qkv, T* __restrict__ v_pool, const int*
                    const int* __restrict__ row_entry, const int* __restrict__ block_table, int max_blocks,
                    int rows, int q_heads, int kv_heads, int head_dim, int page_tokens) {
     extern __shared__ __align__(32) unsigned char turned_raw[];
-    value_write_block<T>(reinterpret_cast<T*>(turned_raw), blockIdx.x, blockIdx.y, qkv, v_pool, positions, row_entry, block_table,
-                         max_blocks, rows, q_heads, kv_heads, head_dim, page_tokens);
+    value_write_block<T, T>(reinterpret_cast<T*>(turned_raw), blockIdx.x, blockIdx.y, qkv, static_cast<long>(q_heads + 2 * kv_heads) * head_dim,
+                            v_pool, positions, row_entry, block_table, max_blocks, rows, q_heads, kv_heads, head_dim, page_tokens);
+}
+
+// The general kernel's work for heads of 64 or 128 elements in runs of 8, kD / 16 lanes a head: rotation of the whole head's halves
+// (kAdjacent false), or of the first pairs of neighbours (or none); rows may be wider than their heads.  A wave a head was bound by
+// its chain of trips to memory, of which many rows have as many as heads; here a wave has 8 or 16 heads on their way.  A head's
+// squares are added in that kernel's order (pairs by halves of the whole, then of the lanes', then of a lane's own): the same bits.
+// us with cold caches, 16 heads over 4 of 128 in float, half of a head turned (the general kernel): 2,114 rows of 5,120 19.5 (35.5),
+// queries alone 13.8 (21.9); 600 rows 10.1 (13.7); 300 rows 8.9 (10.7); 200 rows 8.4 (8.4); 8 rows 9.1 (7.8): few rows have nothing
+// to overlap and wait for a longer chain in a lane, so the line is at 256.
+constexpr int kPairRows = 256;
+template <typename TIn, typename T, int kD16, bool kAdjacent>
+__global__ void __launch_bounds__(256)
+qk_norm_rope_write_pairs_kernel(const TIn* __restrict__ qkv, int planes, long plane, T* __restrict__ q_out, T* __restrict__ k_pool,
+                                T* __restrict__ v_pool, AnyVec q_gain, AnyVec k_gain, float eps, const float* __restrict__ cos_table,
+                                const float* __restrict__ sin_table, int table_positions, const int* __restrict__ positions,
+                                const int* __restrict__ row_entry, const int* __restrict__ block_table, int max_blocks, int rows,
+                                int q_heads, int kv_heads, int page_tokens, int write_cache, int rotary_half, long row_width,
+                                int value_blocks) {
+    constexpr int kD = 16 * kD16, kHalf = kD / 2, kShare = kD16;
+    static_assert(kD16 == 4 || kD16 == 8, "lanes of a head, a power of two");
+    if (static_cast<int>(gridDim.x - blockIdx.x) <= value_blocks) {
+        extern __shared__ __align__(32) unsigned char turned_raw[];
+        const int at = value_blocks - static_cast<int>(gridDim.x - blockIdx.x);
+        value_write_block<TIn, T>(reinterpret_cast<T*>(turned_raw), at / kv_heads, at % kv_heads, qkv, row_width, v_pool, positions,
+                                  row_entry, block_table, max_blocks, rows, q_heads, kv_heads, kD, page_tokens);
+        return;
+    }
+    const int heads_total = q_heads + (write_cache ? (value_blocks > 0 ? 1 : 2) * kv_heads : 0);
+    const long item = (static_cast<long>(blockIdx.x) * blockDim.x + threadIdx.x) / kShare;
+    const int j = threadIdx.x % kShare;
+    const bool mine = item < static_cast<long>(rows) * heads_total;         // (a head's lanes all or none)
+    const int row = mine ? static_cast<int>(item / heads_total) : 0;
+    const int head = mine ? static_cast<int>(item % heads_total) : 0;
+    const bool is_q = head < q_heads, is_k = !is_q && head < q_heads + kv_heads;
+    const TIn* src = qkv + row * row_width + static_cast<long>(head) * kD + 8 * j;
+
+    const int pos = positions[row];
+    HeadRun<TIn> lo = *reinterpret_cast<const HeadRun<TIn>*>(src), hi = *reinterpret_cast<const HeadRun<TIn>*>(src + kHalf);
+    int page = 0;
+    if (!is_q) page = block_table[static_cast<long>(row_entry[row]) * max_blocks + pos / page_tokens];
+    // the lane's pairs: halves of the head, elements 8 j + i and theirs half a head on; neighbours, 8 j + 2 i and the one behind it, and
+    // those half a head on
+    const int tpos = pos < table_positions ? pos : table_positions - 1;     // host checks the bound
+    constexpr int kAngles = kAdjacent ? 4 : 8;
+    float cs[2][kAngles], sn[2][kAngles];
+    bool turned[2] = {false, false};
+    if (cos_table != nullptr) {
+#pragma unroll
+        for (int part = 0; part < (kAdjacent ? 2 : 1); ++part) {
+            const int pair = kAdjacent ? part * (kHalf / 2) + 4 * j : 8 * j;     // rotary_half is a multiple of 4
+            turned[part] = pair < rotary_half;
+            const long at = static_cast<long>(tpos) * rotary_half + (turned[part] ? pair : 0);
+#pragma unroll
+            for (int i = 0; i < kAngles; i += 4) {
+                const float4 c = *reinterpret_cast<const float4*>(cos_table + at + i), s = *reinterpret_cast<const float4*>(sin_table + at + i);
+                cs[part][i] = c.x, cs[part][i + 1] = c.y, cs[part][i + 2] = c.z, cs[part][i + 3] = c.w;
+                sn[part][i] = s.x, sn[part][i + 1] = s.y, sn[part][i + 2] = s.z, sn[part][i + 3] = s.w;
+            }
+        }
+    }
+    float a[8], b[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        a[i] = to_float(lo.v[i]);
+        b[i] = to_float(hi.v[i]);
+    }
+    for (int s = 1; s < planes; ++s) {               // planes of a product cut along K: added in order
+        lo = *reinterpret_cast<const HeadRun<TIn>*>(src + s * plane);
+        hi = *reinterpret_cast<const HeadRun<TIn>*>(src + s * plane + kHalf);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            a[i] += to_float(lo.v[i]);
+            b[i] += to_float(hi.v[i]);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        // rounded as a product stored in the outputs' type would be: the same bits whichever way it came
+        a[i] = to_float(from_float<T>(a[i]));
+        b[i] = to_float(from_float<T>(b[i]));
+    }
+    float squares[8];
+    constexpr int kSums = kAdjacent ? 4 : 8;
+#pragma unroll
+    for (int i = 0; i < kSums; ++i) {
+        if constexpr (kAdjacent) {
+            const float first = fmaf(a[2 * i + 1], a[2 * i + 1], fmaf(a[2 * i], a[2 * i], 0.f));
+            squares[i] = first + fmaf(b[2 * i + 1], b[2 * i + 1], fmaf(b[2 * i], b[2 * i], 0.f));
+        } else {
+            squares[i] = fmaf(b[i], b[i], fmaf(a[i], a[i], 0.f));
+        }
+        squares[i] = add_span<kShare>(squares[i]);
+    }
+#pragma unroll
+    for (int off = kSums / 2; off > 0; off /= 2)
+#pragma unroll
+        for (int i = 0; i < off; ++i) squares[i] += squares[i + off];
+    if (!mine || page < 0) return;                   // host reserves pages before the launch
+    const int token = pos % page_tokens;
+    const int kvh = is_k ? head - q_heads : head - q_heads - kv_heads;
+    T* page_base = is_q ? nullptr : (is_k ? k_pool : v_pool) + (static_cast<long>(page) * kv_heads + kvh) * page_tokens * kD;
+    if (!is_q && !is_k) {      // value head: copied as it is; eight elements of one token lie 16 bytes apart
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            page_base[value_offset(token, 8 * j + i, kD)] = from_float<T>(a[i]);
+            page_base[value_offset(token, kHalf + 8 * j + i, kD)] = from_float<T>(b[i]);
+        }
+        return;
+    }
+    const AnyVec gain = is_q ? q_gain : k_gain;
+    if (gain.ptr) {
+        const float inv = 1.0f / sqrtf(squares[0] / static_cast<float>(kD) + eps);
+        float ga[8], gb[8];
+        load_run(gain, 8 * j, ga);
+        load_run(gain, kHalf + 8 * j, gb);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            a[i] = (a[i] * ga[i]) * inv;
+            b[i] = (b[i] * gb[i]) * inv;
+        }
+    }
+    const auto turn = [](float& u, float& v, float c, float s) {
+        const float ru = fmaf(u, c, -(v * s)), rv = fmaf(v, c, u * s);      // which product is rounded: as in the general kernel
+        u = ru;
+        v = rv;
+    };
+    if constexpr (kAdjacent) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            if (turned[0]) turn(a[2 * i], a[2 * i + 1], cs[0][i], sn[0][i]);
+            if (turned[1]) turn(b[2 * i], b[2 * i + 1], cs[1][i], sn[1][i]);
+        }
+    } else if (turned[0]) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) turn(a[i], b[i], cs[0][i], sn[0][i]);
+    }
+    HeadRun<T> first, second;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        first.v[i] = from_float<T>(a[i]);
+        second.v[i] = from_float<T>(b[i]);
+    }
+    T* dst = is_q ? q_out + (static_cast<long>(row) * q_heads + head) * kD + 8 * j : page_base + key_offset(token, 8 * j, page_tokens);
+    *reinterpret_cast<HeadRun<T>*>(dst) = first;
+    *reinterpret_cast<HeadRun<T>*>(is_q ? dst + kHalf : page_base + key_offset(token, kHalf + 8 * j, page_tokens)) = second;
 }
 
 template <typename TIn, typename T, int kD16>
@@ -846,6 +997,37 @@ extern "C" int leone_qk_norm_rope_write_turned(const void* qkv, int qkv_dtype, i
         }
 #undef LEONE_RUNS_CASE
 #undef LEONE_RUNS_ARGS
+        LEONE_LAUNCH_CHECK("qk_norm_rope_write");
+        return 0;
+    }
+    // heads of 64 or 128 elements whose rows, gains and angles can be read in runs: the whole head's halves turned, or pairs of neighbours
+    const int rotary_half = cos_table ? rotary_dim / 2 : 0;
+    const bool adjacent = pairing == kPairAdjacent || rotary_half == 0;
+    const bool pairs_aligned = (!q_gain || (reinterpret_cast<uintptr_t>(q_gain) % 32 == 0 && reinterpret_cast<uintptr_t>(k_gain) % 32 == 0)) &&
+                               (!cos_table || (reinterpret_cast<uintptr_t>(cos_table) % 16 == 0 && reinterpret_cast<uintptr_t>(sin_table) % 16 == 0)) &&
+                               (!write_cache || reinterpret_cast<uintptr_t>(v_pool) % run_bytes == 0);
+    const long pair_items = static_cast<long>(rows) * (q_heads + 2 * kv_heads) * (head_dim / 16);
+    if (rows >= kPairRows && plain && (head_dim == 64 || head_dim == 128) && v_dim == head_dim && row_width % 8 == 0 && aligned && pairs_aligned &&
+        rotary_half % 4 == 0 && (adjacent || rotary_half == head_dim / 2) && pair_items < 0x7fffffffL * 256) {
+        // many rows are mostly portions of prompts: their values are written in whole runs, eight rows at a time
+        const bool values_apart = write_cache && rows >= 64 && qkv_planes == 1 && static_cast<long>(ceil_div(rows, 8)) * kv_heads < 0x3fffffffL;
+        const long items = static_cast<long>(rows) * (q_heads + (write_cache ? (values_apart ? 1 : 2) * kv_heads : 0));
+        const int value_blocks = values_apart ? ceil_div(rows, 8) * kv_heads : 0;
+        const int blocks = ceil_div(items * (head_dim / 16), 256) + value_blocks;
+        const size_t shared = values_apart ? static_cast<size_t>(8) * head_dim * (dtype == kF32 ? sizeof(float) : sizeof(bf16_t)) : 0;
+#define LEONE_PAIRS(TIN, T, D16, ADJACENT)                                                                                    \
+    qk_norm_rope_write_pairs_kernel<TIN, T, D16, ADJACENT><<<blocks, 256, shared, stream>>>(                                    \
+        static_cast<const TIN*>(qkv), qkv_planes, qkv_plane, static_cast<T*>(q_out), static_cast<T*>(k_pool), static_cast<T*>(v_pool), qg, \
+        kg, eps, cos_table, sin_table, table_positions, positions, row_entry, block_table, max_blocks, rows, q_heads, kv_heads,  \
+        page_tokens, write_cache, rotary_half, row_width, value_blocks)
+#define LEONE_PAIRS_SIZE(TIN, T, ADJACENT) (head_dim == 64 ? LEONE_PAIRS(TIN, T, 4, ADJACENT) : LEONE_PAIRS(TIN, T, 8, ADJACENT))
+#define LEONE_PAIRS_TYPE(TIN, T) (adjacent ? LEONE_PAIRS_SIZE(TIN, T, true) : LEONE_PAIRS_SIZE(TIN, T, false))
+        if (dtype == kF32) LEONE_PAIRS_TYPE(float, float);
+        else if (qkv_dtype == kF32) LEONE_PAIRS_TYPE(float, bf16_t);
+        else LEONE_PAIRS_TYPE(bf16_t, bf16_t);
+#undef LEONE_PAIRS_TYPE
+#undef LEONE_PAIRS_SIZE
+#undef LEONE_PAIRS
         LEONE_LAUNCH_CHECK("qk_norm_rope_write");
         return 0;
     }

@@ -125,3 +125,39 @@ def test_gates_on_attentions_output(kind, heads, vdim):
         got = ops.head_gate(out.to(DEV).clone(), gate.to(DEV)[:, first:first + heads], heads, vdim).cpu().double()
         want = out.double() * torch.sigmoid(gate.double()[:, first:first + heads]).repeat_interleave(vdim, 1)
         assert float(((got - want).abs() / (want.abs() + 1e-3)).max()) < (2.0 ** -8 if kind == torch.bfloat16 else 2e-6)
+
+
+@pytest.mark.parametrize("rows", [256, 259])
+@pytest.mark.parametrize("dim", [64, 128])
+@pytest.mark.parametrize("turned,pairing,normed", [(1.0, "half_split", True), (1.0, "adjacent", True), (0.5, "adjacent", True), (0.0, "adjacent", False)])
+def test_heads_in_runs_of_eight(rows, dim, turned, pairing, normed):
+    """Norms, rotation and cache write in runs of eight against the kernel a wave a head, which takes rows that do not lie in such runs:
+    the same bits, for prompts and decoded tokens at odd places, unmapped pages, layers that bring queries only."""
+    from leone_amd import ops
+    gen = torch.Generator(device=DEV).manual_seed(rows + dim)
+    rand = lambda *size: torch.randn(*size, generator=gen, device=DEV)     # noqa: E731
+    q_heads, kv_heads, page = 6, 2, 16
+    heads = (q_heads + 2 * kv_heads) * dim
+    positions = 5 + torch.arange(rows, dtype=torch.int32, device=DEV)
+    entry = torch.zeros(rows, dtype=torch.int32, device=DEV)
+    if rows > 256:                                       # two requests, the second one from a run's start on
+        positions[33:] = torch.arange(8, 8 + rows - 33, dtype=torch.int32, device=DEV)
+        entry[33:] = 1
+    table = torch.randperm(40, generator=gen, device=DEV).view(2, 20).to(torch.int32)
+    table[1, 2] = -1
+    cos, sin = ops.rope_table(1e6, int(dim * turned), 300, DEV) if turned else (None, None)
+    for kind in (torch.float32, torch.bfloat16):
+        for given in {torch.float32, kind}:
+            gains = [(1 + 0.1 * rand(dim)).to(kind) for _ in range(2)] if normed else [None, None]
+            data = rand(rows, heads + 8).to(given)
+            pools = rand(40, kv_heads, dim // 8, page, 8).to(kind), rand(40, kv_heads, page // 8, dim, 8).to(kind)
+            for queries_only in (False, True):
+                found = []
+                for width in (heads + 8, heads + 4):     # rows that lie in runs, and rows that do not
+                    k_pool, v_pool = (p.clone() for p in pools)
+                    q = ops.qk_norm_rope_write(data[:, :width].contiguous(), q_heads, kv_heads, dim, *gains, 1e-6, cos, sin, positions, entry, table,
+                                               k_pool, v_pool, write_cache=not queries_only, out_dtype=kind, pairing=pairing, value_dim=dim,
+                                               queries_only=queries_only)
+                    found.append((q, k_pool, v_pool))
+                assert all(torch.equal(a, b) for a, b in zip(*found)), (kind, given, queries_only)
+                assert queries_only or not torch.equal(found[0][1], pools[0])
