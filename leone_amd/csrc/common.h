@@ -95,6 +95,23 @@ __device__ inline void load_any8(const AnyVec& v, long at, float out[8]) {
     }
 }
 
+// Four neighbouring elements as they were loaded, unpacked where they are used.
+template <typename T>
+struct Four {
+    float4 v;
+    __device__ inline void load(const T* from) { v = *reinterpret_cast<const float4*>(from); }
+    __device__ inline float get(int i) const { return i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w; }
+};
+template <>
+struct Four<bf16_t> {
+    uint2 v;
+    __device__ inline void load(const bf16_t* from) { v = *reinterpret_cast<const uint2*>(from); }
+    __device__ inline float get(int i) const {
+        const unsigned word = i / 2 ? v.y : v.x;
+        return __uint_as_float(i % 2 ? word & 0xffff0000u : word << 16);
+    }
+};
+
 // ---- values of other lanes -----------------------------------------------------------------------------------------
 // A shuffle (ds_bpermute) is a trip through the shared-memory unit, some 60 cycles that the next addition waits for, and a wave's
 // sum is six of them one after the other.  Lanes of the same row of 16 are reached by an operand's own permutation (DPP) instead,

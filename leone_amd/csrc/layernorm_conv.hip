@@ -40,22 +40,6 @@ __device__ inline void mean_rstd(F value, int n, float eps, float* scratch, floa
     rstd = 1.0f / sqrtf(var + eps);
 }
 
-// Four neighbouring elements as they were loaded, unpacked where they are used.
-template <typename T>
-struct Four {
-    float4 v;
-    __device__ inline void load(const T* from) { v = *reinterpret_cast<const float4*>(from); }
-    __device__ inline float get(int i) const { return i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w; }
-};
-template <>
-struct Four<bf16_t> {
-    uint2 v;
-    __device__ inline void load(const bf16_t* from) { v = *reinterpret_cast<const uint2*>(from); }
-    __device__ inline float get(int i) const {
-        const unsigned word = i / 2 ? v.y : v.x;
-        return __uint_as_float(i % 2 ? word & 0xffff0000u : word << 16);
-    }
-};
 __device__ inline void store_four(float* to, const float (&v)[4]) { *reinterpret_cast<float4*>(to) = float4{v[0], v[1], v[2], v[3]}; }
 __device__ inline void store_four(bf16_t* to, const float (&v)[4]) {
     *reinterpret_cast<uint2*>(to) = uint2{bf16_bits_from_float(v[0]) | static_cast<unsigned>(bf16_bits_from_float(v[1])) << 16,
