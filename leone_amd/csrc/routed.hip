@@ -480,7 +480,8 @@ __device__ inline moe_bf16x8 moe_zero8() {
 // its bytes are the bound.  A workgroup takes 16 rows of the matrix (gated: and their up rows) and its four waves share out
 // the inner size, each with eight steps of 32 on their way at a time; their sums meet in shared memory, in the waves' order.
 // (A wave that walked the whole inner size by itself had a quarter of the loads in flight and four times the chain.)
-// Eight rows of 2,048 over 34 experts of 768, four routed places and two for every row (us, before): gated 38 (47), down 19 (24).
+// Eight rows of 2,048 over 34 experts of 768, four routed places and two for every row (us; with loads that the compiler could not
+// count, for which it waited one by one; one wave an item): gated 30 (38, 47), down 18 (19, 24).
 //
 // A load is half of a line in 16 rows; the other half comes with the load behind it.  kStreamed: loads marked as not to be kept, which
 // leaves the caches to others (a decoding step of a model with 32 experts of 2,048 x 768: 6.96 ms, unmarked 7.09, its first products alone unmarked
@@ -600,7 +601,8 @@ moe_product_stream_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict
 // is small enough for two to three workgroups a compute unit.  (One chunk ahead, with tiles of 128 pairs x 256 rows, had 0.34
 // PFLOP/s; tiles of 64 pairs straight from memory into registers were slower still; tiles of 128 pairs worked this way take
 // eight waves, of which fewer workgroups fit: 312 us at the largest of these.)  Measured, both products of 32 experts, width
-// 2,048 and 768 (us, before): 1,093 pairs 88 (161), 2,533 pairs 135 (282), 7,358 pairs 216 (237).
+// 2,048 and 768, in a model's pass (us; with loads that the compiler could not count): 7,700 pairs 181 (199).  Alone, matrices not
+// in the caches: 1,160 pairs 128 (131), 2,800 pairs 143 (161), 8,456 pairs 259 (279).
 constexpr int kBigPairs = 64;
 constexpr int kBigRows = 128;
 constexpr int kBigChunk = 64;
