@@ -108,7 +108,7 @@ exp_gates_kernel(const float* __restrict__ proj, long stride, int i_off, int f_o
         raw_i = base[i_off + head];
         raw_f = base[f_off + head];
     };
-    fetch(first + tid);
+    if (first < end) fetch(first + tid);             // (an entry without rows has no last row to take instead)
     for (int r0 = first, turn = 0; r0 < end; r0 += kThreads, turn ^= 1) {
         const int r = r0 + tid;
         float li = -INFINITY, lf = 0.f;

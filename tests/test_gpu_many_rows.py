@@ -84,6 +84,30 @@ def test_exponential_gates(counts):
         first += n
 
 
+def test_exponential_gates_of_an_entry_without_rows():
+    """The maximum goes from the state that is read to the one that is written, nothing is read of the rows, and no row's gates change."""
+    from leone_amd import ops
+    from leone_amd.ops.library import call
+    gen = torch.Generator().manual_seed(3)
+    heads, rows = 3, 70
+    proj, bias = torch.randn(rows, 2 * heads, generator=gen).to(DEV), torch.randn(2, heads, generator=gen).to(DEV)
+    state = torch.randn(5, heads, 4, generator=gen)
+
+    def gates(spans, count):
+        spans, kept = torch.tensor(spans, dtype=torch.int32, device=DEV), state.to(DEV).clone()
+        coef, top = torch.zeros(rows, heads, 2, device=DEV), torch.zeros(rows, heads, device=DEV)
+        call("leone_exp_gates", proj.data_ptr(), 2 * heads, 0, heads, bias[0].data_ptr(), bias[1].data_ptr(), ops.F32, 15.0, spans.data_ptr(),
+             spans.shape[0], kept.data_ptr(), kept.stride(0), 4, 3, 1, coef.data_ptr(), top.data_ptr(), count, heads, torch.cuda.current_stream().cuda_stream)
+        return kept, coef, top
+
+    for count in (1, rows):                              # a wave an entry, a workgroup an entry
+        want = gates([[0, count, 1, 1]], count)
+        got = gates([[0, 0, 0, 3], [0, count, 1, 1], [0, 0, -1, 4]], count)
+        assert torch.equal(got[1], want[1]) and torch.equal(got[2], want[2])
+        want[0][3, :, 3], want[0][4, :, 3] = state[0, :, 3].to(DEV), 0.0
+        assert torch.equal(got[0], want[0])
+
+
 @pytest.mark.parametrize("hidden", [8, 1016, 1032, 2048, 2056, 4096])
 @pytest.mark.parametrize("weights,out", [(torch.bfloat16, torch.bfloat16), (torch.float32, torch.float32), (torch.bfloat16, torch.float32)])
 def test_layer_norms_of_many_rows(hidden, weights, out):
