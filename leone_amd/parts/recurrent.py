@@ -211,10 +211,11 @@ class ChannelDeltaMixer(Part):
 
     def bind(self, tensors: Dict[str, torch.Tensor]) -> None:
         self.w_in = torch.cat([tensors.pop(self.names[k]) for k in ("q", "k", "v", "b", "a1", "g1")], dim=0).contiguous()
-        # the wide halves of the two low-rank pairs; of one rank they lie together and are one launch in steps of few rows
+        # the wide halves of the two low-rank pairs; of one rank they lie together and are one launch in steps of few rows, if every
+        # half then begins at 16 bytes, as what the products read does
         self.w_a2 = tensors.pop(self.names["a2"]).contiguous()
         self.w_g2 = tensors.pop(self.names["g2"]).contiguous()
-        self.w_low = torch.cat([self.w_a2, self.w_g2], dim=0).contiguous() if self.a_rank == self.g_rank else None
+        self.w_low = torch.cat([self.w_a2, self.w_g2], dim=0).contiguous() if self.a_rank == self.g_rank and self.a_rank % 8 == 0 else None
         if self.w_low is not None:
             self.w_a2, self.w_g2 = self.w_low[:self.heads * self.dim], self.w_low[self.heads * self.dim:]
         self.w_o = tensors.pop(self.names["o"]).contiguous()
