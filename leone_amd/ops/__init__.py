@@ -1343,16 +1343,25 @@ class NormedDelta:
     ``rows`` (float32 ``[rows, hidden]``) before the sum.  The norm part that runs next takes it in place of a
     delta and does both in one pass (``add_layernorm``); any other consumer asks for ``materialize()``."""
 
-    def __init__(self, rows: torch.Tensor, norm):
-        self.rows, self.norm = rows, norm
+    def __init__(self, rows, norm):
+        self.unsummed, self.norm = rows, norm        # a tensor or ``PairedRows``: for a consumer that takes both
+
+    @property
+    def rows(self) -> torch.Tensor:
+        if isinstance(self.unsummed, PairedRows):
+            self.unsummed = self.unsummed.sum()
+        return self.unsummed
 
     def materialize(self) -> torch.Tensor:
-        return self.norm.apply(self.rows.sum() if isinstance(self.rows, PairedRows) else self.rows)
+        return self.norm.apply(self.rows)
 
 
 class PairedRows:
     """What routed experts gave, one row a (row, place): still to be summed over each row's places.  ``add_normed`` takes it as a
-    delta and makes the sums on the way; any other consumer asks for ``sum()`` (float32 ``[rows, hidden]``)."""
+    delta and makes the sums on the way; any other consumer asks for ``sum()`` (float32 ``[rows, hidden]``).  A feed-forward hands it
+    out if its ``forward`` carries ``gives_pairs`` and is called with ``paired=True``; a norm gets it only if its ``add_behind``
+    carries ``takes_pairs``.  Both are marks on the functions themselves, so that one that takes their place has none.
+    ``x``, the rows that were routed, may be the stream itself: whoever is handed this takes it before the stream changes."""
 
     def __init__(self, pairs: torch.Tensor, chosen: torch.Tensor, weight: torch.Tensor, x: torch.Tensor, extra: Optional[torch.Tensor],
                  experts: int):

@@ -238,7 +238,8 @@ class PostNormBlock(Part):
         if isinstance(pending, ops.PreparedRows):
             pending = None                        # its product has added into the stream already
         if isinstance(pending, ops.NormedDelta) and hasattr(pending.norm, "add_behind"):
-            return pending.norm.add_behind(x, pending.rows, step.dtype)
+            behind = pending.norm.add_behind
+            return behind(x, pending.unsummed if getattr(behind, "takes_pairs", False) else pending.rows, step.dtype)
         if pending is not None:
             delta = pending.materialize() if isinstance(pending, (ops.NormedDelta, ops.ScaledDelta, ops.MixedDelta)) else pending
             x.add_(delta.sum(dim=0) if delta.dim() == 3 else delta)
@@ -250,8 +251,8 @@ class PostNormBlock(Part):
         if self.feed_forward is None:
             return ops.NormedDelta(mixed, self.norm1)
         h = self.norm1.add_behind(x, mixed, step.dtype)
-        feed = getattr(self.feed_forward, "forward_paired", self.feed_forward.forward)
-        return ops.NormedDelta(feed(h, step), self.norm2)
+        feed = self.feed_forward.forward
+        return ops.NormedDelta(feed(h, step, paired=True) if getattr(feed, "gives_pairs", False) else feed(h, step), self.norm2)
 
 
 @BLOCKS.register("scaled_prenorm")

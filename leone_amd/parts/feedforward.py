@@ -242,6 +242,4 @@ class RoutedGluMlp(Part):
                                        self.w_gate_up, self.w_down, self.activation, extra=extra, rule=self.rule,
                                        limit=self.limit, weigh_input=self.weigh_input, paired=paired)
 
-    def forward_paired(self, y: torch.Tensor, step: StepContext) -> ops.PairedRows:
-        """The same with the sum over a row's places left to the norm behind (``ops.add_normed``)."""
-        return self.forward(y, step, paired=True)
+    forward.gives_pairs = True       # ``paired``: the sum over a row's places is left to the norm behind (``ops.PairedRows``)

@@ -66,7 +66,7 @@ class RmsNorm(Part):
             behind = delta.norm
             if isinstance(behind, RmsNorm) and behind.gain.dtype == self.gain.dtype:
                 # the norm behind the last sublayer, the residual sum and this norm in one kernel
-                return ops.add_normed(x, delta.rows, behind.gain, behind.eps, then=(self.gain, self.eps, out_dtype), rows=rows)
+                return ops.add_normed(x, delta.unsummed, behind.gain, behind.eps, then=(self.gain, self.eps, out_dtype), rows=rows)
             delta = delta.materialize()       # a delta that another kind of norm is still to be applied to
         return ops.add_rmsnorm(x, delta, self.gain, self.eps, out_dtype, rows)
 
@@ -82,6 +82,8 @@ class RmsNorm(Part):
         if self.groups > 1:
             raise ValueError("a norm in groups does not stand behind a sublayer")
         return ops.add_normed(x, delta, self.gain, self.eps, out_dtype=out_dtype)
+
+    add_behind.takes_pairs = True
 
     def folded(self, out_dtype: torch.dtype):
         """(gain, eps, type) for a product that can leave this norm's operand behind when it adds into the
