@@ -1346,8 +1346,18 @@ class NormedDelta:
     def __init__(self, rows, norm):
         self.unsummed, self.norm = rows, norm        # a tensor or ``PairedRows``: for a consumer that takes both
 
+    def take(self):
+        """``unsummed`` for a consumer that adds it into the stream.  Experts' places are several times as large as their sum, and the
+        blocks and the model keep this object until the block that consumed it returns: they are let go here."""
+        found = self.unsummed
+        if isinstance(found, PairedRows):
+            self.unsummed = None
+        return found
+
     @property
     def rows(self) -> torch.Tensor:
+        if self.unsummed is None:
+            raise KernelError("what this delta held has been added into the stream")
         if isinstance(self.unsummed, PairedRows):
             self.unsummed = self.unsummed.sum()
         return self.unsummed

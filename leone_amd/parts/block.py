@@ -239,7 +239,7 @@ class PostNormBlock(Part):
             pending = None                        # its product has added into the stream already
         if isinstance(pending, ops.NormedDelta) and hasattr(pending.norm, "add_behind"):
             behind = pending.norm.add_behind
-            return behind(x, pending.unsummed if getattr(behind, "takes_pairs", False) else pending.rows, step.dtype)
+            return behind(x, pending.take() if getattr(behind, "takes_pairs", False) else pending.rows, step.dtype)
         if pending is not None:
             delta = pending.materialize() if isinstance(pending, (ops.NormedDelta, ops.ScaledDelta, ops.MixedDelta)) else pending
             x.add_(delta.sum(dim=0) if delta.dim() == 3 else delta)

@@ -66,7 +66,8 @@ class RmsNorm(Part):
             behind = delta.norm
             if isinstance(behind, RmsNorm) and behind.gain.dtype == self.gain.dtype:
                 # the norm behind the last sublayer, the residual sum and this norm in one kernel
-                return ops.add_normed(x, delta.unsummed, behind.gain, behind.eps, then=(self.gain, self.eps, out_dtype), rows=rows)
+                return ops.add_normed(x, delta.take() if rows is None else delta.unsummed, behind.gain, behind.eps,
+                                      then=(self.gain, self.eps, out_dtype), rows=rows)
             delta = delta.materialize()       # a delta that another kind of norm is still to be applied to
         return ops.add_rmsnorm(x, delta, self.gain, self.eps, out_dtype, rows)
 

@@ -1,4 +1,6 @@
 """Who is handed routed experts' results that are still to be summed over their places."""
+import gc
+import weakref
 from types import SimpleNamespace
 
 import pytest
@@ -72,6 +74,25 @@ def test_the_ordinary_norm_gets_the_places(monkeypatch):
     seen.clear()
     block._take_in(torch.zeros(2, 3), pending, STEP)
     assert seen == [pairs]
+
+
+@pytest.mark.parametrize("where", ["block", "norm"])
+def test_places_are_let_go_once_they_are_in_the_stream(monkeypatch, where):
+    """Whoever still holds the delta, as the model and the block do until the block returns, holds no places with it."""
+    norm = RmsNorm.__new__(RmsNorm)
+    norm.groups, norm.gain, norm.eps = 1, torch.ones(3), 1e-5
+    pending = ops.NormedDelta(ops.PairedRows(torch.ones(4, 3), None, None, torch.zeros(2, 3), None, 1), norm)
+    monkeypatch.setattr(ops, "add_normed", lambda x, delta, *args, **kwargs: x)
+    places = weakref.ref(pending.unsummed.pairs)
+    if where == "block":
+        PostNormBlock._take_in(torch.zeros(2, 3), pending, STEP)
+    else:
+        assert norm.add_norm(torch.zeros(2, 3), pending, torch.float32, torch.tensor([0])) is not None and places() is not None   # nothing added yet
+        norm.add_norm(torch.zeros(2, 3), pending, torch.float32)
+    gc.collect()
+    assert places() is None
+    with pytest.raises(ops.KernelError):
+        pending.rows
 
 
 def test_a_feed_forward_of_its_own_is_called_as_ever(monkeypatch):
