@@ -1,0 +1,56 @@
+"""Registers and scratch of the built kernels, from the notes of their code objects: what a kernel must not take, where taking it costs
+half its waves or sends its operands through memory."""
+import struct
+
+import pytest
+
+msgpack = pytest.importorskip("msgpack")
+
+
+def _code_objects(data: bytes):
+    """The gfx950 code objects of every source's bundle in the library."""
+    magic, at = b"__CLANG_OFFLOAD_BUNDLE__", 0
+    while (at := data.find(magic, at)) >= 0:
+        here = at + len(magic)
+        count, = struct.unpack_from("<Q", data, here)
+        here += 8
+        for _ in range(count):
+            offset, size, length = struct.unpack_from("<QQQ", data, here)
+            target = data[here + 24:here + 24 + length]
+            here += 24 + length
+            if target.endswith(b"gfx950"):
+                yield data[at + offset:at + offset + size]
+        at += len(magic)
+
+
+def _notes(elf: bytes):
+    """The kernels' entries of a code object's note section."""
+    sections, = struct.unpack_from("<Q", elf, 0x28)
+    size, count = struct.unpack_from("<HH", elf, 0x3a)
+    for i in range(count):
+        kind, = struct.unpack_from("<I", elf, sections + i * size + 4)
+        if kind != 7:                                    # SHT_NOTE
+            continue
+        offset, = struct.unpack_from("<Q", elf, sections + i * size + 0x18)
+        name, length, kind = struct.unpack_from("<III", elf, offset)
+        if kind == 32:                                   # NT_AMDGPU_METADATA
+            start = offset + 12 + (name + 3) // 4 * 4
+            yield from msgpack.unpackb(elf[start:start + length], raw=False)["amdhsa.kernels"]
+
+
+@pytest.fixture(scope="module")
+def kernels():
+    from leone_amd.csrc import build
+    with open(build.build(force=False), "rb") as handle:
+        data = handle.read()
+    found = {k[".name"]: k for elf in _code_objects(data) for k in _notes(elf)}
+    assert len(found) > 500
+    return found
+
+
+def test_products_that_carry_out_a_norm(kernels):
+    """Four waves a SIMD (128 registers of 512) and nothing in scratch."""
+    normed = [k for name, k in kernels.items() if "gemm_fused_kernelILi1E" in name]
+    assert len(normed) >= 40
+    for k in normed:
+        assert k[".vgpr_count"] <= 128 and k[".private_segment_fixed_size"] == 0, k[".name"]
