@@ -110,21 +110,13 @@ add_layernorm_kernel(float* __restrict__ x, const float* __restrict__ delta, Any
     }
 }
 
-// Eight neighbouring elements of a row as they were loaded: a value is unpacked where it is used, so that no load is waited for by
-// its own conversion.  kVec: the row is aligned to 16 bytes and holds whole runs; else the elements one by one, at indices held
-// inside the row.
+// Eight neighbouring elements of a row that is aligned to 16 bytes and holds whole runs, as they were loaded: a value is unpacked
+// where it is used, so that no load is waited for by its own conversion.
 constexpr int kRun = 8;
-template <typename T, bool kVec>
-struct Run {
-    T v[kRun];
-    __device__ inline void load(const T* __restrict__ row, int at, int length) {
-#pragma unroll
-        for (int i = 0; i < kRun; ++i) v[i] = row[at + i < length ? at + i : length - 1];
-    }
-    __device__ inline float get(int i) const { return to_float(v[i]); }
-};
+template <typename T>
+struct Run;
 template <>
-struct Run<float, true> {
+struct Run<float> {
     float4 v[2];
     __device__ inline void load(const float* __restrict__ row, int at, int length) {
         const float4* from = reinterpret_cast<const float4*>(row + (at < length ? at : 0));
@@ -137,7 +129,7 @@ struct Run<float, true> {
     }
 };
 template <>
-struct Run<bf16_t, true> {
+struct Run<bf16_t> {
     uint4 v;
     __device__ inline void load(const bf16_t* __restrict__ row, int at, int length) {
         v = *reinterpret_cast<const uint4*>(row + (at < length ? at : 0));
@@ -147,23 +139,133 @@ struct Run<bf16_t, true> {
         return __uint_as_float(i % 2 ? word & 0xffff0000u : word << 16);
     }
 };
-template <typename T, bool kVec>
+template <typename T>
 __device__ inline void store_run(T* __restrict__ row, int at, int length, const float (&v)[kRun]) {
-    if constexpr (!kVec) {
+    if (at >= length) return;
+    if constexpr (sizeof(T) == 4) {
+        reinterpret_cast<float4*>(row + at)[0] = float4{v[0], v[1], v[2], v[3]};
+        reinterpret_cast<float4*>(row + at)[1] = float4{v[4], v[5], v[6], v[7]};
+    } else {
+        unsigned w[kRun / 2];
 #pragma unroll
-        for (int i = 0; i < kRun; ++i)
-            if (at + i < length) row[at + i] = from_float<T>(v[i]);
-    } else if (at < length) {
-        if constexpr (sizeof(T) == 4) {
-            reinterpret_cast<float4*>(row + at)[0] = float4{v[0], v[1], v[2], v[3]};
-            reinterpret_cast<float4*>(row + at)[1] = float4{v[4], v[5], v[6], v[7]};
-        } else {
-            unsigned w[kRun / 2];
+        for (int i = 0; i < kRun / 2; ++i)
+            w[i] = bf16_bits_from_float(v[2 * i]) | static_cast<unsigned>(bf16_bits_from_float(v[2 * i + 1])) << 16;
+        *reinterpret_cast<uint4*>(row + at) = uint4{w[0], w[1], w[2], w[3]};
+    }
+}
+
+// The same for few rows of up to 1,024 kPer elements, a thread an element of every 1,024.  A step of few rows is a chain of trips to
+// memory, about two microseconds each when the lines are cold: here the row, the delta, the gains, the biases, the filter's taps and
+// the state's last inputs are all asked for before the first sum (each at an index held inside the row, so that no branch stands
+// between the loads), and the row stays in registers.  One type for all of the norm's and the filter's vectors, so that a load is
+// not followed by its conversion.  Sums run in the other kernel's order: the results are the same bits.
+constexpr int kHeldTaps = 4;
+template <typename TOut, typename TW, int kPer>
+__global__ void __launch_bounds__(kNormThreadsFew)
+add_layernorm_single_kernel(float* __restrict__ x, const float* __restrict__ delta, const TW* __restrict__ dw, const TW* __restrict__ db,
+                          float deps, const TW* __restrict__ w, const TW* __restrict__ b, float eps, TOut* __restrict__ y,
+                          const int* __restrict__ rows, int hidden, const TW* __restrict__ conv, int taps, float* conv_state,
+                          int write_state, const int* __restrict__ positions, const int* __restrict__ row_entry,
+                          const int* __restrict__ entry_slots) {
+    __shared__ float scratch[kNormThreadsFew / kWave];
+    const int tid = threadIdx.x;
+    const long src = rows ? rows[blockIdx.x] : blockIdx.x;
+    float* xr = x + src * hidden;
+    int at[kPer];
+    bool in[kPer];
 #pragma unroll
-            for (int i = 0; i < kRun / 2; ++i)
-                w[i] = bf16_bits_from_float(v[2 * i]) | static_cast<unsigned>(bf16_bits_from_float(v[2 * i + 1])) << 16;
-            *reinterpret_cast<uint4*>(row + at) = uint4{w[0], w[1], w[2], w[3]};
+    for (int n = 0; n < kPer; ++n) {
+        in[n] = tid + n * kNormThreadsFew < hidden;
+        at[n] = in[n] ? tid + n * kNormThreadsFew : hidden - 1;
+    }
+    float v[kPer], d[kPer], old[kHeldTaps - 1][kPer];
+    TW gd[kPer], bd[kPer], g[kPer], o[kPer], f[kHeldTaps][kPer];
+    int pos = 0, entry = 0;
+    if (conv) {
+        pos = positions[blockIdx.x];
+        entry = row_entry[blockIdx.x];
+    }
+#pragma unroll
+    for (int n = 0; n < kPer; ++n) v[n] = xr[at[n]];
+    if (delta) {
+#pragma unroll
+        for (int n = 0; n < kPer; ++n) d[n] = delta[src * hidden + at[n]];
+    }
+    if (dw) {
+#pragma unroll
+        for (int n = 0; n < kPer; ++n) {
+            gd[n] = dw[at[n]];
+            bd[n] = db[at[n]];
         }
+    }
+    if (y) {
+#pragma unroll
+        for (int n = 0; n < kPer; ++n) {
+            g[n] = w[at[n]];
+            o[n] = b[at[n]];
+        }
+    }
+    float* keep = nullptr;
+    if (conv) {
+#pragma unroll
+        for (int j = 0; j < kHeldTaps; ++j)
+#pragma unroll
+            for (int n = 0; n < kPer; ++n)
+                if (j < taps) f[j][n] = conv[static_cast<long>(at[n]) * taps + j];
+        keep = conv_state + static_cast<long>(entry_slots[entry]) * (taps - 1) * hidden;
+#pragma unroll
+        for (int j = 0; j + 1 < kHeldTaps; ++j)
+#pragma unroll
+            for (int n = 0; n < kPer; ++n)
+                if (j + 1 < taps) old[j][n] = keep[static_cast<long>(j) * hidden + at[n]];
+    }
+    auto mean_of = [&](const float (&values)[kPer], float eps_, float& mean, float& rstd) {
+        float sum = 0.f;
+#pragma unroll
+        for (int n = 0; n < kPer; ++n) sum += in[n] ? values[n] : 0.f;
+        mean = block_sum<kNormThreadsFew>(sum, scratch) / static_cast<float>(hidden);
+        float q = 0.f;
+#pragma unroll
+        for (int n = 0; n < kPer; ++n) {
+            const float off = in[n] ? values[n] - mean : 0.f;
+            q = fmaf(off, off, q);
+        }
+        rstd = 1.0f / sqrtf(block_sum<kNormThreadsFew>(q, scratch) / static_cast<float>(hidden) + eps_);
+    };
+    float mean = 0.f, rstd = 1.f;
+    if (delta) {
+        if (dw) mean_of(d, deps, mean, rstd);
+#pragma unroll
+        for (int n = 0; n < kPer; ++n) {
+            const float more = dw ? (d[n] - mean) * rstd * to_float(gd[n]) + to_float(bd[n]) : d[n];
+            v[n] += more;
+            if (!rows && in[n]) xr[at[n]] = v[n];
+        }
+    }
+    if (!y) return;
+    mean_of(v, eps, mean, rstd);
+    TOut* yr = y + static_cast<long>(blockIdx.x) * hidden;
+#pragma unroll
+    for (int n = 0; n < kPer; ++n) {
+        if (!in[n]) continue;
+        const float h = (v[n] - mean) * rstd * to_float(g[n]) + to_float(o[n]);
+        if (!conv) {
+            yr[at[n]] = from_float<TOut>(h);
+            continue;
+        }
+        float acc = 0.f;
+#pragma unroll
+        for (int j = 0; j < kHeldTaps; ++j) {                // oldest input first, the row itself under the last tap
+            if (j + 1 < taps) {
+                const float was = pos - (taps - 1 - j) < 0 ? 0.f : old[j < kHeldTaps - 1 ? j : 0][n];
+                acc = fmaf(to_float(f[j][n]), was, acc);
+                if (write_state && j > 0) keep[static_cast<long>(j - 1) * hidden + at[n]] = was;
+            } else if (j + 1 == taps) {
+                acc = fmaf(to_float(f[j][n]), h, acc);
+                if (write_state) keep[static_cast<long>(j - 1) * hidden + at[n]] = h;
+            }
+        }
+        yr[at[n]] = from_float<TOut>(h + acc);
     }
 }
 
@@ -173,17 +275,15 @@ __device__ inline void store_run(T* __restrict__ row, int at, int length, const 
 // Sums run in the other kernel's order with 1,024 threads, so that few rows get the bits they get there: elements 1,024 apart in
 // turn, then those 32, 16, .. 1 apart meet, then every 64's sums in turn.  The runs of 64 elements lie on the eight lanes so that
 // each of the lanes' three meetings is an operand's permutation.
-// kTaps: of the folded filter; 0: none, -1: `taps` of them, up to kHeldTaps.
+// kTaps: of the folded filter; 0: none.
 // Eight rows of 2,048 with two norms and a filter of 4 taps, in bfloat16: 6.1 us (7.8 with 1,024 threads of single elements).
-constexpr int kHeldTaps = 4;
 constexpr int kHeldThreads = 128;
-template <typename TOut, typename TW, bool kVec, int kPer, int kTaps>
+template <typename TOut, typename TW, int kPer, int kTaps>
 __global__ void __launch_bounds__(kHeldThreads)
 add_layernorm_held_kernel(float* __restrict__ x, const float* __restrict__ delta, const TW* __restrict__ dw, const TW* __restrict__ db,
                           float deps, const TW* __restrict__ w, const TW* __restrict__ b, float eps, TOut* __restrict__ y,
-                          const int* __restrict__ rows, int hidden, const TW* __restrict__ conv, int taps, float* conv_state,
-                          int write_state, const int* __restrict__ positions, const int* __restrict__ row_entry,
-                          const int* __restrict__ entry_slots) {
+                          const int* __restrict__ rows, int hidden, const TW* __restrict__ conv, float* conv_state, int write_state,
+                          const int* __restrict__ positions, const int* __restrict__ row_entry, const int* __restrict__ entry_slots) {
     constexpr int kLanes = 64 / kRun, kGroups = kHeldThreads / kLanes;        // lanes that share 64 elements, sums of 64 elements
     __shared__ float4 scratch[4][kGroups / 4];
     const long src = rows ? rows[blockIdx.x] : blockIdx.x;
@@ -192,15 +292,15 @@ add_layernorm_held_kernel(float* __restrict__ x, const float* __restrict__ delta
     int at[kPer];
 #pragma unroll
     for (int n = 0; n < kPer; ++n) at[n] = (n * kHeldThreads + place) * kRun;
-    const bool filtered = kTaps > 0 || (kTaps < 0 && conv);
-    if constexpr (kTaps > 0) taps = kTaps;
+    constexpr bool filtered = kTaps > 0;
+    static_assert(kTaps == 0 || kTaps == 4, "a channel's taps are half a run");
     int pos = 0, entry = 0;
     if (filtered) {
         pos = positions[blockIdx.x];
         entry = row_entry[blockIdx.x];
     }
-    Run<float, kVec> stream[kPer], more[kPer], old[kTaps == 0 ? 1 : kHeldTaps - 1][kPer];
-    Run<TW, kVec> delta_gain[kPer], delta_bias[kPer], gain[kPer], bias[kPer], filter[kTaps == 0 ? 1 : kHeldTaps][kPer];
+    Run<float> stream[kPer], more[kPer], old[kTaps == 0 ? 1 : kTaps - 1][kPer];
+    Run<TW> delta_gain[kPer], delta_bias[kPer], gain[kPer], bias[kPer], filter[kTaps == 0 ? 1 : kTaps][kPer];
 #pragma unroll
     for (int n = 0; n < kPer; ++n) stream[n].load(xr, at[n], hidden);
     if (delta) {
@@ -225,26 +325,17 @@ add_layernorm_held_kernel(float* __restrict__ x, const float* __restrict__ delta
     if (filtered) {
 #pragma unroll
         for (int n = 0; n < kPer; ++n) {
-            if constexpr (kTaps == kHeldTaps) {      // a channel's taps lie side by side: four runs of two channels each
 #pragma unroll
-                for (int j = 0; j < kHeldTaps; ++j)
-                    filter[j][n].load(conv, at[n] < hidden ? at[n] * kHeldTaps + j * kRun : 0, hidden * kHeldTaps);
-            } else if constexpr (kTaps < 0) {
-#pragma unroll
-                for (int j = 0; j < kHeldTaps; ++j)
-#pragma unroll
-                    for (int i = 0; i < kRun; ++i)
-                        if (j < taps) filter[j][n].v[i] = conv[static_cast<long>(at[n] + i < hidden ? at[n] + i : hidden - 1) * taps + j];
-            }
+            for (int j = 0; j < kTaps; ++j)          // a channel's taps lie side by side: four runs of two channels each
+                filter[j][n].load(conv, at[n] < hidden ? at[n] * kTaps + j * kRun : 0, hidden * kTaps);
         }
-        keep = conv_state + static_cast<long>(entry_slots[entry]) * (taps - 1) * hidden;
+        keep = conv_state + static_cast<long>(entry_slots[entry]) * (kTaps - 1) * hidden;
 #pragma unroll
-        for (int j = 0; j + 1 < (kTaps == 0 ? 1 : kHeldTaps); ++j)
+        for (int j = 0; j + 1 < kTaps; ++j)
 #pragma unroll
-            for (int n = 0; n < kPer; ++n)
-                if (j + 1 < taps) old[j][n].load(keep + static_cast<long>(j) * hidden, at[n], hidden);
+            for (int n = 0; n < kPer; ++n) old[j][n].load(keep + static_cast<long>(j) * hidden, at[n], hidden);
     }
-    const auto inside = [&](int n, int i) { return at[n] + (kVec ? 0 : i) < hidden; };
+    const auto inside = [&](int n) { return at[n] < hidden; };
     const auto row_sum = [&](float (&part)[kRun], float4* meet) {
 #pragma unroll
         for (int i = 0; i < kRun; ++i) {
@@ -275,7 +366,7 @@ add_layernorm_held_kernel(float* __restrict__ x, const float* __restrict__ delta
 #pragma unroll
         for (int n = 0; n < kPer; ++n)
 #pragma unroll
-            for (int i = 0; i < kRun; ++i) part[i] += inside(n, i) ? v[n][i] : 0.f;
+            for (int i = 0; i < kRun; ++i) part[i] += inside(n) ? v[n][i] : 0.f;
         mean = row_sum(part, meet[0]) / static_cast<float>(hidden);
 #pragma unroll
         for (int i = 0; i < kRun; ++i) part[i] = 0.f;
@@ -283,7 +374,7 @@ add_layernorm_held_kernel(float* __restrict__ x, const float* __restrict__ delta
         for (int n = 0; n < kPer; ++n)
 #pragma unroll
             for (int i = 0; i < kRun; ++i) {
-                const float off = inside(n, i) ? v[n][i] - mean : 0.f;
+                const float off = inside(n) ? v[n][i] - mean : 0.f;
                 part[i] = fmaf(off, off, part[i]);
             }
         rstd = 1.0f / sqrtf(row_sum(part, meet[1]) / static_cast<float>(hidden) + of_eps);
@@ -304,7 +395,7 @@ add_layernorm_held_kernel(float* __restrict__ x, const float* __restrict__ delta
         for (int n = 0; n < kPer; ++n) {
 #pragma unroll
             for (int i = 0; i < kRun; ++i) v[n][i] += dw ? (d[n][i] - mean) * rstd * delta_gain[n].get(i) + delta_bias[n].get(i) : d[n][i];
-            if (!rows) store_run<float, kVec>(xr, at[n], hidden, v[n]);
+            if (!rows) store_run<float>(xr, at[n], hidden, v[n]);
         }
     }
     if (!y) return;
@@ -320,22 +411,20 @@ add_layernorm_held_kernel(float* __restrict__ x, const float* __restrict__ delta
             // A step of single rows, every row another request: oldest input first, the row itself under the last tap
             float acc[kRun] = {};
 #pragma unroll
-            for (int j = 0; j < (kTaps == 0 ? 1 : kHeldTaps); ++j) {
-                if (j >= taps) continue;
+            for (int j = 0; j < kTaps; ++j) {
                 float in[kRun];
 #pragma unroll
                 for (int i = 0; i < kRun; ++i) {
-                    if (j + 1 < taps) in[i] = pos - (taps - 1 - j) < 0 ? 0.f : old[j < kHeldTaps - 1 ? j : 0][n].get(i);
+                    if (j + 1 < kTaps) in[i] = pos - (kTaps - 1 - j) < 0 ? 0.f : old[j < kTaps - 1 ? j : 0][n].get(i);
                     else in[i] = h[i];
-                    const float tap = kTaps < 0 ? filter[j][n].get(i) : filter[i / 2][n].get(i % 2 * kHeldTaps + j);
-                    acc[i] = fmaf(tap, in[i], acc[i]);
+                    acc[i] = fmaf(filter[i / 2][n].get(i % 2 * kTaps + j), in[i], acc[i]);
                 }
-                if (write_state && j > 0) store_run<float, kVec>(keep + static_cast<long>(j - 1) * hidden, at[n], hidden, in);
+                if (write_state && j > 0) store_run<float>(keep + static_cast<long>(j - 1) * hidden, at[n], hidden, in);
             }
 #pragma unroll
             for (int i = 0; i < kRun; ++i) h[i] += acc[i];
         }
-        store_run<TOut, kVec>(yr, at[n], hidden, h);
+        store_run<TOut>(yr, at[n], hidden, h);
     }
 }
 
@@ -782,16 +871,16 @@ head_gate_runs_kernel(T* __restrict__ out, const float* __restrict__ gate, long 
     const int row = i / runs, at = (i - row * runs) * kRun, length = runs * kRun;
     const float* gates = gate + row * gate_stride;
     T* mine = out + static_cast<long>(row) * length;
-    Run<T, true> v;
+    Run<T> v;
     v.load(mine, at, length);
-    Run<float, true> each;
+    Run<float> each;
     float one = 0.f;
     if constexpr (kEach) each.load(gates, at, length);
     else one = gates[at / vdim];
     float result[kRun];
 #pragma unroll
     for (int k = 0; k < kRun; ++k) result[k] = v.get(k) * activate(kEach ? each.get(k) : one, kActSigmoid);
-    store_run<T, true>(mine, at, length, result);
+    store_run<T>(mine, at, length, result);
 }
 
 static bool known(int dtype) { return dtype == kF32 || dtype == kBF16; }
@@ -823,26 +912,39 @@ extern "C" int leone_add_layernorm(float* x, const float* delta, const void* dw,
                                                                          rows, hidden, vconv, taps, conv_state, write_state,   \
                                                                          positions, row_entry, entry_slots, stage_delta)
     const bool many = n_out >= kNormManyRows;
-    // Rows that fit registers, one type of vectors throughout: few rows by a workgroup each, in whole 16-byte runs where they lie so
-    // and else element by element; many rows by a wave each where they lie in such runs.
+    // Rows that fit registers, one type of vectors throughout: few rows by a workgroup each, many rows by a wave each where they lie in
+    // whole 16-byte runs.  Few rows go in such runs too where they lie so, a filter in four taps, and else element by element: in runs
+    // that were loaded by elements a thread takes 490 registers and neighbours lie 32 bytes apart (us, element by element: 8 rows of
+    // 2,049 10.1, so 5.2, of 4,095 12.9, 5.3, of 4,096 with three taps 25.2, 8.1).  Rows of more than 2,048 without a filter go element by
+    // element up to one a compute unit: a thread with four runs of everything is the longer chain (8 rows of 4,096, two norms, vectors in
+    // bfloat16 and in float: in runs 6.2 and 6.5, so 5.4 and 5.1; 256 rows 7.2 and 7.5, 6.5 and 6.4), and with two workgroups a unit
+    // the runs are ahead (384 rows 8.8 and 9.5, so 12.2 and 12.1).
     const auto aligned = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
     const bool vec = hidden % kRun == 0 && aligned(x) && aligned(delta) && aligned(dw) && aligned(db) && aligned(w) && aligned(b) &&
                      aligned(y) && (!conv || (taps == kHeldTaps && aligned(conv) && aligned(conv_state)));
-    if (!many && hidden <= 4 * kRun * kHeldThreads && (!conv || (taps <= kHeldTaps && conv_dtype == w_dtype))) {
-#define LEONE_HELD(T, TW, VEC, PER, TAPS)                                                                                       \
-    add_layernorm_held_kernel<T, TW, VEC, PER, TAPS><<<n_out, kHeldThreads, 0, stream>>>(                                       \
+    if (!many && hidden <= 4 * kNormThreadsFew && (!conv || (taps <= kHeldTaps && conv_dtype == w_dtype))) {
+        constexpr int kTwoRuns = 2 * kRun * kHeldThreads, kSingleRows = 256;
+        static_assert(kTwoRuns == 2 * kNormThreadsFew, "both kernels hold the same rows");
+        const bool single = !vec || (!conv && hidden > kTwoRuns && n_out <= kSingleRows);
+#define LEONE_SINGLE(T, TW, PER)                                                                                                \
+    add_layernorm_single_kernel<T, TW, PER><<<n_out, kNormThreadsFew, 0, stream>>>(                                             \
         x, delta, static_cast<const TW*>(dw), static_cast<const TW*>(db), deps, static_cast<const TW*>(w), static_cast<const TW*>(b), eps, \
         static_cast<T*>(y), rows, hidden, static_cast<const TW*>(conv), taps, conv_state, write_state, positions, row_entry, entry_slots)
-#define LEONE_HELD_VEC(T, TW, PER)                                                                                              \
-    (!vec ? LEONE_HELD(T, TW, false, PER, -1) : conv ? LEONE_HELD(T, TW, true, PER, kHeldTaps) : LEONE_HELD(T, TW, true, PER, 0))
-#define LEONE_HELD_PER(T, TW) (hidden <= 2 * kRun * kHeldThreads ? LEONE_HELD_VEC(T, TW, 2) : LEONE_HELD_VEC(T, TW, 4))
-        if (y_dtype == kF32 && w_dtype == kF32) LEONE_HELD_PER(float, float);
-        else if (y_dtype == kF32) LEONE_HELD_PER(float, bf16_t);
-        else if (w_dtype == kF32) LEONE_HELD_PER(bf16_t, float);
-        else LEONE_HELD_PER(bf16_t, bf16_t);
-#undef LEONE_HELD_PER
-#undef LEONE_HELD_VEC
+#define LEONE_HELD(T, TW, PER, TAPS)                                                                                            \
+    add_layernorm_held_kernel<T, TW, PER, TAPS><<<n_out, kHeldThreads, 0, stream>>>(                                            \
+        x, delta, static_cast<const TW*>(dw), static_cast<const TW*>(db), deps, static_cast<const TW*>(w), static_cast<const TW*>(b), eps, \
+        static_cast<T*>(y), rows, hidden, static_cast<const TW*>(conv), conv_state, write_state, positions, row_entry, entry_slots)
+#define LEONE_FEW_PER(T, TW, PER)                                                                                               \
+    (single ? LEONE_SINGLE(T, TW, PER) : conv ? LEONE_HELD(T, TW, PER, kHeldTaps) : LEONE_HELD(T, TW, PER, 0))
+#define LEONE_FEW(T, TW) (hidden <= kTwoRuns ? LEONE_FEW_PER(T, TW, 2) : LEONE_FEW_PER(T, TW, 4))
+        if (y_dtype == kF32 && w_dtype == kF32) LEONE_FEW(float, float);
+        else if (y_dtype == kF32) LEONE_FEW(float, bf16_t);
+        else if (w_dtype == kF32) LEONE_FEW(bf16_t, float);
+        else LEONE_FEW(bf16_t, bf16_t);
+#undef LEONE_FEW
+#undef LEONE_FEW_PER
 #undef LEONE_HELD
+#undef LEONE_SINGLE
         LEONE_LAUNCH_CHECK("add_layernorm");
         return 0;
     }

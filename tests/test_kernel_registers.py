@@ -54,3 +54,11 @@ def test_products_that_carry_out_a_norm(kernels):
     assert len(normed) >= 40
     for k in normed:
         assert k[".vgpr_count"] <= 128 and k[".private_segment_fixed_size"] == 0, k[".name"]
+
+
+def test_layer_norms_of_few_rows(kernels):
+    """What takes rows element by element has a thread an element of every 1,024: five waves a SIMD, nothing in scratch."""
+    normed = {name: k for name, k in kernels.items() if "add_layernorm_" in name}
+    assert not [name for name, k in normed.items() if k[".private_segment_fixed_size"]]
+    single = [k for name, k in normed.items() if "add_layernorm_single" in name]
+    assert len(single) == 8 and all(k[".vgpr_count"] <= 96 and k[".max_flat_workgroup_size"] == 1024 for k in single)
