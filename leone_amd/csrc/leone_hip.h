@@ -262,7 +262,9 @@ int leone_scan_max_dim();
 // segments: n x (first row, end, index of the state read or -1 for zeros, index of the state written or -1).
 int leone_exp_gates(const float* proj, long stride, int i_off, int f_off, const void* i_bias, const void* f_bias,
                     int bias_dtype, float cap, const int* spans, int entries, float* state, long slot_stride,
-                    long head_stride, long top_at, int write_state, float* coef, float* top, int rows, int heads, hipStream_t stream);
+                    long head_stride, long top_at, int write_state, float* coef, float* top, int longest, int heads, hipStream_t stream);
+// longest: the most rows an entry has.  The threads of a workgroup that are taken for such entries:
+int leone_exp_gates_threads(int longest, int entries, int heads);
 int leone_outer_scan(const float* proj, long stride, int q_off, int k_off, int v_off, const float* coef, const float* decay,
                      int norm_column, float q_scale, float k_scale, int silu, const float* cos_table,
                      const float* sin_table, int rotary_dim, int table_positions, const int* positions,

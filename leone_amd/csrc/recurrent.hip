@@ -89,8 +89,18 @@ __device__ inline float log_sigmoid_f(float z) { return z >= 0.f ? -log1pf(expf(
 // waves' order.  A portion is bound by one workgroup's chain of trips to memory a head: as many rows a trip as a workgroup may have
 // threads, the next trip's rows asked for ahead of this one's scan.  2,048 rows of 4 heads: 10.4 us (28.2 with one wave scanning the
 // 256 rows of a trip).
-constexpr int kGateThreadsFew = kWave;             // steps of single rows
-constexpr int kGateThreadsMany = 1024;
+//
+// How many threads, by the longest entry's rows: as many waves as it has 64 rows, which scan side by side, and up to 1,024 threads
+// while every workgroup has a compute unit of its own.  More workgroups share units with each other, and threads without rows hold
+// them up (us with 64, 256, 512 and 1,024 threads): one portion of 2,000 rows beside 8 single ones, 16 heads 41, 15.2, 11.9, 10.4, beside 63
+// 40, 22.9, 18.7, 25.6; beside 128, 32 heads 43, 19.1, 21.3, 42; 64 entries of 2 rows, 16 heads 3.7, 3.9, 5.6, 9.7; one of 128 rows 4.7, 3.7,
+// 3.8, 3.9.
+constexpr int kGateUnits = 256;
+__host__ inline int gate_threads(int longest, long groups) {
+    if (longest <= kWave) return kWave;
+    if (longest <= 256 || groups > 8 * kGateUnits) return 256;
+    return groups > kGateUnits ? 512 : 1024;
+}
 template <int kThreads>
 __global__ void __launch_bounds__(kThreads)
 exp_gates_kernel(const float* __restrict__ proj, long stride, int i_off, int f_off, AnyVec i_bias, AnyVec f_bias, float cap,
@@ -675,22 +685,27 @@ static bool known_vec(int dtype) { return dtype == kF32 || dtype == kBF16; }
 using namespace leone;
 
 extern "C" int leone_scan_max_dim() { return 256; }
+extern "C" int leone_exp_gates_threads(int longest, int entries, int heads) { return gate_threads(longest, static_cast<long>(entries) * heads); }
 
 extern "C" int leone_exp_gates(const float* proj, long stride, int i_off, int f_off, const void* i_bias, const void* f_bias,
                                int bias_dtype, float cap, const int* spans, int entries, float* state, long slot_stride,
-                               long head_stride, long top_at, int write_state, float* coef, float* top, int rows,
+                               long head_stride, long top_at, int write_state, float* coef, float* top, int longest,
                                int heads, hipStream_t stream) {
     LEONE_REQUIRE(proj && i_bias && f_bias && spans && state && coef && top, "exp_gates: null pointer");
     LEONE_REQUIRE(known_vec(bias_dtype) && cap > 0.f, "exp_gates: unknown bias type or cap %g", cap);
-    LEONE_REQUIRE(entries > 0 && rows > 0 && heads > 0 && heads <= 65535 && i_off >= 0 && f_off >= 0 && stride >= i_off + heads &&
+    LEONE_REQUIRE(entries > 0 && longest > 0 && heads > 0 && heads <= 65535 && i_off >= 0 && f_off >= 0 && stride >= i_off + heads &&
                   stride >= f_off + heads, "exp_gates: %d entries, %d heads, rows of %ld", entries, heads, stride);
     LEONE_REQUIRE(top_at >= 0 && top_at < head_stride && slot_stride >= heads * head_stride, "exp_gates: the maximum's place %ld", top_at);
 #define LEONE_GATES(THREADS)                                                                                                \
     exp_gates_kernel<THREADS><<<dim3(entries, heads), THREADS, 0, stream>>>(proj, stride, i_off, f_off, AnyVec{i_bias, bias_dtype}, \
                                                                             AnyVec{f_bias, bias_dtype}, cap, spans, state, slot_stride, \
                                                                             head_stride, top_at, write_state, coef, top, heads)
-    if (rows <= entries) LEONE_GATES(kGateThreadsFew);
-    else LEONE_GATES(kGateThreadsMany);
+    switch (gate_threads(longest, static_cast<long>(entries) * heads)) {
+        case kWave: LEONE_GATES(kWave); break;
+        case 256: LEONE_GATES(256); break;
+        case 512: LEONE_GATES(512); break;
+        default: LEONE_GATES(1024); break;
+    }
 #undef LEONE_GATES
     LEONE_LAUNCH_CHECK("exp_gates");
     return 0;

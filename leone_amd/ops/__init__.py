@@ -1455,6 +1455,15 @@ def entry_spans(step) -> torch.Tensor:
     return spans
 
 
+def longest_entry(step) -> int:
+    """The most rows an entry of the step has: of a step that is replayed from a recording, whose entries the host does not know,
+    what is left if all others have one."""
+    longest = getattr(step, "longest", None)
+    if longest is None:
+        longest = step.longest = max((e.count for e in step.entries), default=step.rows - step.entry_slots.numel() + 1)
+    return longest
+
+
 # Rows of a chunk when a long portion of the delta rule over more than 128 key channels is walked chunk by chunk, side by side, and
 # the portions that are (at least so many rows): (chunk, from).  The chunks are chained by a matrix product each.
 DELTA_CHUNKS = (256, 512)
@@ -1720,7 +1729,7 @@ def outer_scan(proj: torch.Tensor, columns: dict, state: torch.Tensor, step, hea
              _dev(gates["i_bias"], "i bias", None, (heads,)), _dev(gates["f_bias"], "f bias", None, (heads,)),
              _code(gates["i_bias"], "i bias"), float(gates["cap"]), _dev(spans, "spans"), spans.shape[0],
              _dev(state, "state"), state.stride(0), per_head, dim * vdim + dim, 1 if write_state else 0,
-             _dev(coef, "coefficients"), _dev(top, "top"), rows, heads, _stream())
+             _dev(coef, "coefficients"), _dev(top, "top"), longest_entry(step), heads, _stream())
     rotary_dim = 2 * cos.shape[1] if cos is not None else 0
 
     def walk(segments):

@@ -1,0 +1,16 @@
+"""Where the lines of rules lie that choose between kernels with the same results."""
+import pytest
+
+
+@pytest.fixture(scope="module")
+def lib():
+    from leone_amd.ops.library import library
+    return library()
+
+
+@pytest.mark.parametrize("longest,entries,heads,threads", [
+    (1, 64, 16, 64), (2, 64, 16, 64), (64, 1, 4, 64),            # a wave has an entry's rows: no more threads than that
+    (65, 1, 4, 256), (256, 8, 16, 256), (2000, 129, 32, 256),    # few trips, or many workgroups that share units
+    (257, 1, 4, 1024), (2000, 16, 16, 1024), (257, 64, 16, 512), (2000, 128, 16, 512)])
+def test_threads_of_the_exponential_gates(lib, longest, entries, heads, threads):
+    assert lib.leone_exp_gates_threads(longest, entries, heads) == threads

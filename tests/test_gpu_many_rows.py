@@ -51,9 +51,10 @@ def test_filters_of_many_rows(channels, kind, out, filters):
     assert torch.equal(kept.cpu().double(), after)
 
 
-@pytest.mark.parametrize("counts", [(1, 1), (64, 1), (65, 3), (1024, 1025), (2111,)])
+@pytest.mark.parametrize("counts", [(1, 1), (64, 1), (65, 3), (256, 257), (1024, 1025), (2111,), (300,) + (1,) * 130, (1100,) + (1, 2) * 520])
 def test_exponential_gates(counts):
-    """One wave's rows, a workgroup's and one over, from a state and from a sequence's start."""
+    """One wave's rows, a workgroup's and one over, from a state and from a sequence's start; long entries beside many short ones, with
+    every number of threads."""
     from leone_amd import ops
     gen = torch.Generator().manual_seed(sum(counts))
     heads, dim, vdim = 2, 32, 64
@@ -93,16 +94,16 @@ def test_exponential_gates_of_an_entry_without_rows():
     proj, bias = torch.randn(rows, 2 * heads, generator=gen).to(DEV), torch.randn(2, heads, generator=gen).to(DEV)
     state = torch.randn(5, heads, 4, generator=gen)
 
-    def gates(spans, count):
+    def gates(spans, longest):
         spans, kept = torch.tensor(spans, dtype=torch.int32, device=DEV), state.to(DEV).clone()
         coef, top = torch.zeros(rows, heads, 2, device=DEV), torch.zeros(rows, heads, device=DEV)
         call("leone_exp_gates", proj.data_ptr(), 2 * heads, 0, heads, bias[0].data_ptr(), bias[1].data_ptr(), ops.F32, 15.0, spans.data_ptr(),
-             spans.shape[0], kept.data_ptr(), kept.stride(0), 4, 3, 1, coef.data_ptr(), top.data_ptr(), count, heads, torch.cuda.current_stream().cuda_stream)
+             spans.shape[0], kept.data_ptr(), kept.stride(0), 4, 3, 1, coef.data_ptr(), top.data_ptr(), longest, heads, torch.cuda.current_stream().cuda_stream)
         return kept, coef, top
 
-    for count in (1, rows):                              # a wave an entry, a workgroup an entry
-        want = gates([[0, count, 1, 1]], count)
-        got = gates([[0, 0, 0, 3], [0, count, 1, 1], [0, 0, -1, 4]], count)
+    for longest in (1, rows, 300):                       # a wave an entry, a few, and as many as a workgroup may have
+        want = gates([[0, rows, 1, 1]], longest)
+        got = gates([[0, 0, 0, 3], [0, rows, 1, 1], [0, 0, -1, 4]], longest)
         assert torch.equal(got[1], want[1]) and torch.equal(got[2], want[2])
         want[0][3, :, 3], want[0][4, :, 3] = state[0, :, 3].to(DEV), 0.0
         assert torch.equal(got[0], want[0])
