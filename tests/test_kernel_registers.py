@@ -62,3 +62,9 @@ def test_layer_norms_of_few_rows(kernels):
     assert not [name for name, k in normed.items() if k[".private_segment_fixed_size"]]
     single = [k for name, k in normed.items() if "add_layernorm_single" in name]
     assert len(single) == 8 and all(k[".vgpr_count"] <= 96 and k[".max_flat_workgroup_size"] == 1024 for k in single)
+
+
+def test_norms_behind_a_sublayer_of_short_rows(kernels):
+    """Rows of up to 1,024 elements take a run a thread: eight waves a SIMD, or seven with eight places on their way."""
+    held = [k for name, k in kernels.items() if "add_normed_held_kernel" in name and "Li1ELi" in name]
+    assert sorted(k[".vgpr_count"] <= 64 for k in held) == [False, False, True, True] and all(k[".vgpr_count"] <= 72 for k in held)
