@@ -608,8 +608,14 @@ value_write_kernel(const T* __restrict__ qkv, T* __restrict__ v_pool, const int*
 // squares are added in that kernel's order (pairs by halves of the whole, then of the lanes', then of a lane's own): the same bits.
 // us with cold caches, 16 heads over 4 of 128 in float, half of a head turned (the general kernel): 2,114 rows of 5,120 19.5 (35.5),
 // queries alone 13.8 (21.9); 600 rows 10.1 (13.7); 300 rows 8.9 (10.7); 200 rows 8.4 (8.4); 8 rows 9.1 (7.8): few rows have nothing
-// to overlap and wait for a longer chain in a lane, so the line is at 256.
+// to overlap and wait for a longer chain in a lane, so the line is at 256 rows, and at as many heads as fill the chip: with warm
+// caches, rows x heads of 128, with keys and values 1,536 4.5 (4.2), 2,560 4.6 (4.6), 3,584 4.6 (5.0), 5,120 4.7 (5.8); queries alone
+// 2,048 4.3 (3.6), 4,096 4.4 (4.2), 5,120 4.4 (4.6).
 constexpr int kPairRows = 256;
+constexpr long kPairHeads = 3584, kPairQueries = 4608;
+static bool heads_in_pairs(int rows, long heads, int write_cache) {
+    return rows >= kPairRows && rows * heads >= (write_cache ? kPairHeads : kPairQueries);
+}
 template <typename TIn, typename T, int kD16, bool kAdjacent>
 __global__ void __launch_bounds__(256)
 qk_norm_rope_write_pairs_kernel(const TIn* __restrict__ qkv, int planes, long plane, T* __restrict__ q_out, T* __restrict__ k_pool,
@@ -929,6 +935,8 @@ extern "C" int leone_qk_norm_rope_write(const void* qkv, int qkv_dtype, int qkv_
                                            write_cache, v_dim, row_width, nullptr, kF32, nullptr, nullptr, 0, 0, 0, stream);
 }
 
+extern "C" int leone_heads_in_pairs(int rows, int heads, int write_cache) { return heads_in_pairs(rows, heads, write_cache); }
+
 extern "C" int leone_qk_norm_rope_write_turned(const void* qkv, int qkv_dtype, int qkv_planes, long qkv_plane, void* q_out,
                                                void* k_pool, void* v_pool, int dtype, const void* q_gain, const void* k_gain,
                                                int gain_dtype, float eps, const float* cos_table, const float* sin_table,
@@ -1008,7 +1016,7 @@ extern "C" int leone_qk_norm_rope_write_turned(const void* qkv, int qkv_dtype, i
                                (!cos_table || (reinterpret_cast<uintptr_t>(cos_table) % 16 == 0 && reinterpret_cast<uintptr_t>(sin_table) % 16 == 0)) &&
                                (!write_cache || reinterpret_cast<uintptr_t>(v_pool) % run_bytes == 0);
     const long pair_items = static_cast<long>(rows) * (q_heads + 2 * kv_heads) * (head_dim / 16);
-    if (rows >= kPairRows && plain && (head_dim == 64 || head_dim == 128) && v_dim == head_dim && row_width % 8 == 0 && aligned && pairs_aligned &&
+    if (heads_in_pairs(rows, q_heads + (write_cache ? 2L * kv_heads : 0L), write_cache) && plain && (head_dim == 64 || head_dim == 128) && v_dim == head_dim && row_width % 8 == 0 && aligned && pairs_aligned &&
         rotary_half % 4 == 0 && (adjacent || rotary_half == head_dim / 2) && pair_items < 0x7fffffffL * 256) {
         // many rows are mostly portions of prompts: their values are written in whole runs, eight rows at a time
         const bool values_apart = write_cache && rows >= 64 && qkv_planes == 1 && static_cast<long>(ceil_div(rows, 8)) * kv_heads < 0x3fffffffL;

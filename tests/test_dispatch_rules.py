@@ -14,3 +14,9 @@ def lib():
     (257, 1, 4, 1024), (2000, 16, 16, 1024), (257, 64, 16, 512), (2000, 128, 16, 512)])
 def test_threads_of_the_exponential_gates(lib, longest, entries, heads, threads):
     assert lib.leone_exp_gates_threads(longest, entries, heads) == threads
+
+
+@pytest.mark.parametrize("rows,heads,write_cache,runs", [(255, 100, 1, 0), (256, 14, 1, 1), (256, 13, 1, 0), (512, 4, 1, 0), (512, 8, 0, 0), (512, 9, 0, 1), (256, 17, 0, 0),
+                                                         (256, 18, 0, 1), (2114, 24, 1, 1), (1 << 30, 24, 1, 1)])
+def test_heads_of_wide_rows_in_runs(lib, rows, heads, write_cache, runs):
+    assert lib.leone_heads_in_pairs(rows, heads, write_cache) == runs

@@ -161,7 +161,8 @@ def test_heads_in_runs_of_eight(rows, dim, turned, pairing, normed):
     from leone_amd import ops
     gen = torch.Generator(device=DEV).manual_seed(rows + dim)
     rand = lambda *size: torch.randn(*size, generator=gen, device=DEV)     # noqa: E731
-    q_heads, kv_heads, page = 6, 2, 16
+    q_heads, kv_heads, page = 18, 2, 16                  # enough heads for the kernel in runs with and without keys and values
+    assert ops.library().leone_heads_in_pairs(rows, q_heads, 0) and ops.library().leone_heads_in_pairs(rows, q_heads + 2 * kv_heads, 1)
     heads = (q_heads + 2 * kv_heads) * dim
     positions = 5 + torch.arange(rows, dtype=torch.int32, device=DEV)
     entry = torch.zeros(rows, dtype=torch.int32, device=DEV)
