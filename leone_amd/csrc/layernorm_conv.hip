@@ -863,6 +863,10 @@ __global__ void head_gate_kernel(T* __restrict__ out, const float* __restrict__ 
 // The same in runs of eight elements of a row (`runs` of them), which have one gate (kEach: a gate each).  What bounds it are its
 // bytes: 2,114 rows of 2,048 with cold caches, a gate an element 15.0 us, a gate a head of 128 7.8 (element by element, with two
 // divisions each, 22.6 and 16.9).
+// A gate an element is eight exponentials one after the other in a thread, which few values wait for: up to so many go element by element.
+// (us with warm caches, runs and elements: in bfloat16 16 x 2,048 2.8 and 2.4, 128 x 2,048 2.9 and 2.7, 192 x 2,048 3.0 and 3.0, 512 x 512 3.0
+// and 2.7; in float 384 x 512 2.6 and 2.6, 128 x 2,048 2.6 and 2.7.  A gate a head: 16 x 2,048 2.4 and 2.4.)
+static bool gates_in_runs(int dtype, bool each, long n) { return !each || n >= (dtype == kBF16 ? 192L << 11 : 96L << 11); }
 template <typename T, bool kEach>
 __global__ void __launch_bounds__(256)
 head_gate_runs_kernel(T* __restrict__ out, const float* __restrict__ gate, long gate_stride, int runs, int vdim, int n) {
@@ -1139,6 +1143,7 @@ extern "C" int leone_relu_squared(const void* in, void* out, int dtype, long n, 
     return 0;
 }
 
+extern "C" int leone_gates_in_runs(int dtype, int each, long n) { return gates_in_runs(dtype, each != 0, n); }
 extern "C" int leone_head_gate(void* out, int dtype, const float* gate, long gate_stride, int rows, int heads, int vdim,
                                hipStream_t stream) {
     LEONE_REQUIRE(out && gate && known(dtype) && rows > 0 && heads > 0 && vdim > 0, "head_gate: needs values and gates");
@@ -1146,7 +1151,7 @@ extern "C" int leone_head_gate(void* out, int dtype, const float* gate, long gat
     LEONE_REQUIRE((n + 255) / 256 <= 0x7fffffffL, "head_gate: too many values");
     // Runs of eight where a row's elements and its gates can be read so: every run in one head, or a gate an element.
     const bool each = vdim == 1, aligned = reinterpret_cast<uintptr_t>(out) % 16 == 0;
-    if (aligned && n <= 0x7fffffffL &&
+    if (aligned && n <= 0x7fffffffL && gates_in_runs(dtype, each, n) &&
         (each ? heads % kRun == 0 && gate_stride % 4 == 0 && reinterpret_cast<uintptr_t>(gate) % 16 == 0 : vdim % kRun == 0)) {
         const int runs = static_cast<int>(static_cast<long>(heads) * vdim / kRun), items = static_cast<int>(n / kRun), blocks = ceil_div(items, 256);
 #define LEONE_GATE_RUNS(T, EACH) \

@@ -499,6 +499,8 @@ int leone_time_mix_scan(const float* r, const float* k, const float* v, long str
 int leone_time_mix_read_rows();
 int leone_time_mix_read(const float* r, long stride, const float* decay, const int* segments, int n_segments, const float* state,
                         long state_stride, float* out, int heads, int dim, int vdim, hipStream_t stream);
+// Whether n values with a gate each (or a gate a head) go through head_gate in runs of eight, if they lie so.
+int leone_gates_in_runs(int dtype, int each, long n);
 // Whether heads of rows that are wider than them, or whose pairs are neighbours, go through qk_norm_rope_write in runs of eight.
 int leone_heads_in_pairs(int rows, int heads, int write_cache);
 // The weight-streaming product of several inputs against matrices that lie together (see gemm_fused.hip).

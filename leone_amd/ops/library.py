@@ -79,6 +79,7 @@ _PROTOTYPES = {
     "leone_outer_scan": [P, ctypes.c_long, c_int, c_int, c_int, P, P, c_int, c_float, c_float, c_int, P, P, c_int, c_int,
                          P, P, c_int, P, ctypes.c_long, P, ctypes.c_long, ctypes.c_long, P, P, c_int, c_int, c_int, P],
     "leone_heads_in_pairs": [c_int, c_int, c_int],
+    "leone_gates_in_runs": [c_int, c_int, ctypes.c_long],
     "leone_exp_gates_threads": [c_int, c_int, c_int],
     "leone_step_fits": [c_int, c_int],
     "leone_outer_step": [P, ctypes.c_long, c_int, c_int, c_int, P, P, c_int, c_float, c_float, c_int, P, P, c_int, c_int,

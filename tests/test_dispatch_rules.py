@@ -20,3 +20,10 @@ def test_threads_of_the_exponential_gates(lib, longest, entries, heads, threads)
                                                          (256, 18, 0, 1), (2114, 24, 1, 1), (1 << 30, 24, 1, 1)])
 def test_heads_of_wide_rows_in_runs(lib, rows, heads, write_cache, runs):
     assert lib.leone_heads_in_pairs(rows, heads, write_cache) == runs
+
+
+@pytest.mark.parametrize("kind,each,n,runs", [("BF16", 1, 8 * 2048, 0), ("BF16", 1, 192 * 2048 - 8, 0), ("BF16", 1, 192 * 2048, 1), ("F32", 1, 96 * 2048 - 8, 0),
+                                              ("F32", 1, 96 * 2048, 1), ("BF16", 0, 8, 1), ("F32", 1, 1 << 33, 1)])
+def test_gates_in_runs(lib, kind, each, n, runs):
+    from leone_amd import ops
+    assert lib.leone_gates_in_runs(getattr(ops, kind), each, n) == runs

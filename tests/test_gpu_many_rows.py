@@ -139,9 +139,9 @@ def test_layer_norms_of_many_rows(hidden, weights, out):
 
 
 @pytest.mark.parametrize("kind", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("heads,vdim", [(16, 1), (20, 1), (5, 8), (3, 24), (7, 6)])
+@pytest.mark.parametrize("heads,vdim", [(16, 1), (20, 1), (1312, 1), (1316, 1), (5, 8), (3, 24), (7, 6)])
 def test_gates_on_attentions_output(kind, heads, vdim):
-    """A gate an element and a gate a head, in runs of eight and where a row does not lie in such runs."""
+    """A gate an element, of few and of many values, and a gate a head, in runs of eight and where a row does not lie in such runs."""
     from leone_amd import ops
     gen = torch.Generator().manual_seed(heads * vdim)
     rows = 300
