@@ -370,10 +370,13 @@ int leone_route_plan(const float* logits, const void* correction, int correction
                      hipStream_t stream);
 int leone_moe_plan(const int* chosen, int pairs, int experts, int* tile_expert, int* tile_pairs, int max_tiles, int tile,
                    hipStream_t stream);
-// tile: leone_moe_tile_pairs() (any type and size), or 16, 64 or 128 (matrix cores: bfloat16, n and k multiples of 8).
+// tile: leone_moe_tile_pairs() (any type and size), or 16, 64 or 128 (matrix cores: bfloat16, n and k multiples of 8).  experts: how many
+// there are.
 int leone_moe_product(const void* x, const void* w, void* y, const float* pair_weight, int dtype, int gated,
-                      const int* tile_expert, const int* tile_pairs, int max_tiles, int tile, int top, int n, int k, int act,
-                      float limit, hipStream_t stream);
+                      const int* tile_expert, const int* tile_pairs, int max_tiles, int tile, int experts, int top, int n, int k,
+                      int act, float limit, hipStream_t stream);
+// Whether tiles of 64 pairs keep one chunk of such experts' matrices on its way, not two.
+int leone_moe_one_chunk_ahead(int experts, int gated, int n, int k);
 int leone_moe_combine(const float* pair_out, const int* chosen, const float* weight, const void* x, int dtype,
                       const float* extra, float* out, int rows, int top, int experts, int hidden, hipStream_t stream);
 // A matrix memory whose forget gate per head and key channel also says what is written (see gated_scan.hip).

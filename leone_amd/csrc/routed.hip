@@ -643,11 +643,24 @@ __device__ inline void store_rows(void* y, int pair, int r, int n, const float (
     }
 }
 
+// One chunk is on its way at a time, not two, where the experts' matrices give nearly every unit one workgroup (7/8 of the units up to all of
+// them) and their rows lie whole multiples of 4 KB apart: the units then walk the inner size abreast, and what more they ask for falls on
+// the same channels.  Both products from memory, us (one chunk, two): 8 experts of 4,096 x 2,048, 16 pairs an expert 116 and 130, 50 pairs
+// 126 and 143, 150 pairs 152 and 162; 16 of 8,192 x 1,024, 16 pairs 205 and 254; 16 of 2,048 x 1,024 62 and 67.  With rows
+// 12 KB apart (6,144) 166 and 170, 10 KB (5,120) 136 and 138; with half the workgroups (4 of 4,096 x 2,048) 87 and 65, with twice as many (32
+// of 4,096 x 1,024) 189 and 173; matrices of few rows (32 of 4,096 x 512) 100 and 96.
+constexpr int kMoeUnits = 256;
+static bool one_chunk_ahead(int experts, int blocks, int n, int k) {
+    const long groups = static_cast<long>(experts) * blocks;
+    return 8 * groups > 7 * kMoeUnits && groups <= kMoeUnits && k % 2048 == 0 && n >= 1024;
+}
+
 template <int kMode>
 __global__ void __launch_bounds__(kMoeThreads, 3)
 moe_product_tiled_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, void* __restrict__ y,
                          const float* __restrict__ pair_weight, const int* __restrict__ tile_expert,
-                         const int* __restrict__ tile_pairs, int top, int n, int k, int act, float limit, int n_tiles, int n_blocks) {
+                         const int* __restrict__ tile_pairs, int top, int n, int k, int act, float limit, int n_tiles, int n_blocks,
+                         int one_ahead) {
     constexpr bool kGated = kMode == kMoeGated;
     constexpr int kOwnRows = kGated ? kBigRows / 2 : kBigRows;        // rows of the result
     constexpr int kBring = kMoeThreads / 8;                           // rows of 8 pieces that the workgroup brings at once
@@ -742,12 +755,14 @@ moe_product_tiled_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict_
     int ck = 0;
     for (; ck + 4 < chunks; ck += 2) {
         __syncthreads();                               // chunk ck lies ready, and nobody reads the other place any more
+        if (one_ahead) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         put(odd, ck + 1, 1);
         __builtin_amdgcn_sched_barrier(0);             // asked for earlier a chunk would take registers of its own, later it would come late
         bring(ck + 3, odd);
         __builtin_amdgcn_sched_barrier(0);
         work(0);
         __syncthreads();
+        if (one_ahead) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         put(even, ck + 2, 0);
         __builtin_amdgcn_sched_barrier(0);
         bring(ck + 4, even);
@@ -802,7 +817,7 @@ template <int kMode>
 __global__ void __launch_bounds__(kMoeThreads, 2)
 moe_product_wide_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, void* __restrict__ y,
                          const float* __restrict__ pair_weight, const int* __restrict__ tile_expert,
-                         const int* __restrict__ tile_pairs, int top, int n, int k, int act, float limit, int n_tiles, int n_blocks) {
+                         const int* __restrict__ tile_pairs, int top, int n, int k, int act, float limit, int n_tiles, int n_blocks, int) {
     constexpr bool kGated = kMode == kMoeGated;
     constexpr int kWRows = kGated ? 2 * kWideRows : kWideRows;          // rows of the matrix in a chunk
     constexpr int kXPieces = kWidePairs * 8 / kMoeThreads;             // 16-byte pieces of x a thread brings per chunk
@@ -997,6 +1012,10 @@ extern "C" int leone_route_plan(const float* logits, const void* correction, int
     return 0;
 }
 
+extern "C" int leone_moe_one_chunk_ahead(int experts, int gated, int n, int k) {
+    return one_chunk_ahead(experts, ceil_div(n, gated == kMoeGated ? kBigRows / 2 : kBigRows), n, k);
+}
+
 extern "C" int leone_moe_plan(const int* chosen, int pairs, int experts, int* tile_expert, int* tile_pairs, int max_tiles,
                               int tile, hipStream_t stream) {
     LEONE_REQUIRE(tile == kTilePairs || tile == 16 || tile == kBigPairs || tile == kWidePairs, "moe_plan: tiles of %d pairs", tile);
@@ -1013,11 +1032,12 @@ extern "C" int leone_moe_plan(const int* chosen, int pairs, int experts, int* ti
 // gated != 0: x [rows, k], w [experts, 2, n, k], y [pairs, n] of dtype = act(gate) * up (act: GateAct).
 // gated == 0: x [pairs, k], w [experts, n, k], y float32 [pairs, n] = pair_weight[pair] * product (null: 1).
 // gated == 2: x [rows, k], w [experts, n, k], y [pairs, n] of dtype = act(pair_weight[pair] * product) (null: 1).
+// experts: how many there are, for the rule that looks at how many workgroups their matrices give (see one_chunk_ahead).
 // tile: pairs a tile holds, as leone_moe_plan was told: leone_moe_tile_pairs() for the kernel that takes any type and
 // size; 16, 64 or 128 for the matrix-core kernels (bfloat16, n and k multiples of 8).
 extern "C" int leone_moe_product(const void* x, const void* w, void* y, const float* pair_weight, int dtype, int gated,
-                                 const int* tile_expert, const int* tile_pairs, int max_tiles, int tile, int top, int n, int k,
-                                 int act, float limit, hipStream_t stream) {
+                                 const int* tile_expert, const int* tile_pairs, int max_tiles, int tile, int experts, int top, int n,
+                                 int k, int act, float limit, hipStream_t stream) {
     LEONE_REQUIRE(gated >= kMoeDown && gated <= kMoePlain, "moe_product: unknown kind of product %d", gated);
     LEONE_REQUIRE(act == kGateSilu || act == kGateGeluTanh || (act == kGateClampedSwish && limit > 0.f && gated != kMoePlain) ||
                       (act == kActReluSquared && gated != kMoeGated),
@@ -1045,10 +1065,10 @@ extern "C" int leone_moe_product(const void* x, const void* w, void* y, const fl
             const int blocks = ceil_div(n, tile == kWidePairs ? kWideRows : gated == kMoeGated ? kBigRows / 2 : kBigRows);
             const long places = static_cast<long>(max_tiles) * blocks;
             LEONE_REQUIRE(places + 7 <= 0x7fffffffL, "moe_product: too many tiles");
-            const int grid = static_cast<int>((places + 7) / 8 * 8);
+            const int grid = static_cast<int>((places + 7) / 8 * 8), one_ahead = one_chunk_ahead(experts, blocks, n, k);
 #define LEONE_MOE_TILED(KERNEL, MODE)                                                                                         \
     KERNEL<MODE><<<grid, kMoeThreads, 0, stream>>>(static_cast<const bf16_t*>(x), static_cast<const bf16_t*>(w), y, pair_weight,   \
-                                                   tile_expert, tile_pairs, top, n, k, act, limit, max_tiles, blocks)
+                                                   tile_expert, tile_pairs, top, n, k, act, limit, max_tiles, blocks, one_ahead)
 #define LEONE_MOE_TILES(MODE)                                                                                                 \
     (tile == kBigPairs ? LEONE_MOE_TILED(moe_product_tiled_kernel, MODE) : LEONE_MOE_TILED(moe_product_wide_kernel, MODE))
             if (gated == kMoeGated) LEONE_MOE_TILES(kMoeGated);

@@ -1983,11 +1983,11 @@ def _expert_products(x, chosen, weight, tiles, w_up, w_down, activation, extra, 
     # the weight stands on the input's side (a product of weight * x is weight times the product) or on the result's
     call("leone_moe_product", _dev(x, "routed rows"), _dev(w_up, "expert up"), _dev(hidden_act, "expert hidden"),
          weights if weigh_input else 0, _code(x, "routed rows"), 1 if gated else 2, _dev(tile_expert, "tiles"),
-         _dev(tile_pairs, "tile pairs"), max_tiles, tile, top, ff, hidden, act, limit, _stream())
+         _dev(tile_pairs, "tile pairs"), max_tiles, tile, experts, top, ff, hidden, act, limit, _stream())
     pair_out = torch.empty((pairs, hidden), dtype=torch.float32, device=device)
     call("leone_moe_product", _dev(hidden_act, "expert hidden"), _dev(w_down, "expert down"), _dev(pair_out, "pair results"),
          0 if weigh_input else weights, _code(x, "routed rows"), 0, _dev(tile_expert, "tiles"),
-         _dev(tile_pairs, "tile pairs"), max_tiles, tile, top, hidden, ff, 0, 0.0, _stream())
+         _dev(tile_pairs, "tile pairs"), max_tiles, tile, experts, top, hidden, ff, 0, 0.0, _stream())
     out = PairedRows(pair_out, chosen, weight, x, extra, experts)
     return out if paired else out.sum()
 

@@ -27,3 +27,9 @@ def test_heads_of_wide_rows_in_runs(lib, rows, heads, write_cache, runs):
 def test_gates_in_runs(lib, kind, each, n, runs):
     from leone_amd import ops
     assert lib.leone_gates_in_runs(getattr(ops, kind), each, n) == runs
+
+
+@pytest.mark.parametrize("experts,gated,n,k,one", [(8, 1, 2048, 4096, 1), (8, 0, 4096, 2048, 1), (16, 1, 1024, 2048, 1), (8, 1, 1856, 4096, 1), (8, 1, 1792, 4096, 0),
+                                                   (8, 1, 2049, 4096, 0), (32, 1, 768, 2048, 0), (8, 1, 2048, 5120, 0), (4, 1, 2048, 4096, 0), (32, 1, 512, 4096, 0)])
+def test_chunks_of_experts_matrices_on_their_way(lib, experts, gated, n, k, one):
+    assert lib.leone_moe_one_chunk_ahead(experts, gated, n, k) == one

@@ -116,3 +116,27 @@ def test_tiles_by_pairs_and_width():
             x = torch.empty(1, hidden, dtype=torch.bfloat16, device=DEV)
             assert ops._expert_tiles(x, (line - 1) * experts, 1, experts, hidden, ff)[0] == below
             assert ops._expert_tiles(x, line * experts, 1, experts, hidden, ff)[0] == above
+
+
+def test_products_with_one_chunk_ahead():
+    """Experts whose matrices give every unit one workgroup, with rows whole multiples of 4 KB apart; some with more pairs than a tile."""
+    from leone_amd import ops
+    from leone_amd.ops.library import library
+    experts, hidden, ff = 16, 2048, 1024
+    assert library().leone_moe_one_chunk_ahead(experts, 1, ff, hidden)
+    gen = torch.Generator().manual_seed(16)
+    counts = [3, 64, 1, 65, 0, 130] + [20] * 10
+    which = torch.tensor([e for e, count in enumerate(counts) for _ in range(count)])[torch.randperm(sum(counts), generator=gen)]
+    rows = len(which)
+    weight, x = torch.rand(rows, 1, generator=gen) + 0.1, torch.randn(rows, hidden, generator=gen).bfloat16()
+    up = (torch.randn(experts, 2, ff, hidden, generator=gen) / math.sqrt(hidden)).bfloat16()
+    down = (torch.randn(experts, hidden, ff, generator=gen) / math.sqrt(ff)).bfloat16()
+    assert ops._expert_tiles(x.to(DEV), rows, 1, experts, hidden, ff)[0] == 64
+    got = ops.routed_experts(x.to(DEV), which.view(-1, 1).to(torch.int32).to(DEV), weight.to(DEV), up.to(DEV), down.to(DEV)).cpu().double()
+    want = torch.empty(rows, hidden, dtype=F)
+    for e in range(experts):
+        mine = which == e
+        gate, more = (x[mine].double() @ up[e, i].double().T for i in (0, 1))
+        want[mine] = weight[mine].double() * ((plain.silu(gate) * more).bfloat16().double() @ down[e].double().T)
+    # as above: middles that are rounded to neighbours
+    assert float((got - want).norm() / want.norm()) < 2e-3
