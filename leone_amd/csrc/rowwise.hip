@@ -117,13 +117,14 @@ add_rmsnorm_vec_kernel(float* __restrict__ x, const TD* __restrict__ delta, int 
     float v[kChunks][4];
     Four<TG> gv[kChunks];
     float ss = 0.f;
-    // Everything a thread needs is asked for before anything is added: the row, the gains, and the planes four
+    // Everything a thread needs is asked for before anything is added: the row, the gains, and the planes three or four
     // at a time (a plane beyond the last is the last one again and is not added), so that the trips to memory
     // overlap instead of following one another plane by plane.  The planes are added in their order.  Places past the row's end
     // load its first elements, and nothing is unpacked behind its load: under a condition, a conversion in it, every load
     // was waited for before the next was asked for (64 rows of 4,096 in four planes 7.0 us, so 5.3; 2,048 rows in bfloat16 13.1 and 11.0).
-    const auto at = [&](int i) { return 4 * (static_cast<int>(threadIdx.x) + i * kThreads); };
-    const auto place = [&](int i) { return at(i) < hidden ? at(i) : 0; };
+    const auto at = [&](unsigned i) { return 4u * (threadIdx.x + i * kThreads); };
+    const unsigned length = static_cast<unsigned>(hidden);
+    const auto place = [&](unsigned i) { return at(i) < length ? at(i) : 0u; };
     Four<float> before[kChunks];
 #pragma unroll
     for (int i = 0; i < kChunks; ++i) before[i].load(xr + place(i));
@@ -145,17 +146,20 @@ add_rmsnorm_vec_kernel(float* __restrict__ x, const TD* __restrict__ delta, int 
 #pragma unroll
             for (int j = 0; j < 4; ++j) v[i][j] += d[i].get(j);
     } else if (dr) {
-        for (int p0 = 0; p0 < planes; p0 += 4) {
-            Four<TD> d[kChunks][4];
+        // float planes under float gains three at a time in long rows: four took 264 registers of 512, one wave a SIMD, whether there
+        // were planes or not (2,048 rows of 5,120 without a delta 21.4 us, so 16.5; 512 in four planes 15.7 and 13.5)
+        constexpr int kAhead = sizeof(TD) + sizeof(TG) == 8 && kChunks >= 4 ? 3 : 4;
+        for (int p0 = 0; p0 < planes; p0 += kAhead) {
+            Four<TD> d[kChunks][kAhead];
 #pragma unroll
             for (int i = 0; i < kChunks; ++i)
 #pragma unroll
-                for (int q = 0; q < 4; ++q) d[i][q].load(dr + (p0 + q < planes ? p0 + q : planes - 1) * plane + place(i));
+                for (int q = 0; q < kAhead; ++q) d[i][q].load(dr + (p0 + q < planes ? p0 + q : planes - 1) * plane + place(i));
             if (p0 == 0) unpack();
 #pragma unroll
             for (int i = 0; i < kChunks; ++i)
 #pragma unroll
-                for (int q = 0; q < 4; ++q)
+                for (int q = 0; q < kAhead; ++q)
                     if (p0 + q < planes) {
 #pragma unroll
                         for (int j = 0; j < 4; ++j) v[i][j] += d[i][q].get(j);
@@ -166,7 +170,7 @@ add_rmsnorm_vec_kernel(float* __restrict__ x, const TD* __restrict__ delta, int 
     }
 #pragma unroll
     for (int i = 0; i < kChunks; ++i) {
-        if (at(i) < hidden) {
+        if (at(i) < length) {
             if (dr && !rows) store4(xr + at(i), v[i]);
 #pragma unroll
             for (int j = 0; j < 4; ++j) ss = fmaf(v[i][j], v[i][j], ss);
@@ -180,7 +184,7 @@ add_rmsnorm_vec_kernel(float* __restrict__ x, const TD* __restrict__ delta, int 
     }
 #pragma unroll
     for (int i = 0; i < kChunks; ++i) {
-        if (at(i) < hidden) {
+        if (at(i) < length) {
             float o[4];
 #pragma unroll
             for (int j = 0; j < 4; ++j) o[j] = (v[i][j] * gv[i].get(j)) * inv;

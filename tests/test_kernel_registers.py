@@ -68,3 +68,12 @@ def test_norms_behind_a_sublayer_of_short_rows(kernels):
     """Rows of up to 1,024 elements take a run a thread: eight waves a SIMD, or seven with eight places on their way."""
     held = [k for name, k in kernels.items() if "add_normed_held_kernel" in name and "Li1ELi" in name]
     assert sorted(k[".vgpr_count"] <= 64 for k in held) == [False, False, True, True] and all(k[".vgpr_count"] <= 72 for k in held)
+
+
+def test_rms_norms_in_registers(kernels):
+    """Rows of up to 4,096 elements keep four waves a SIMD, rows of up to 8,192 two, whatever the types."""
+    for chunks, most in ((4, 128), (8, 256)):
+        normed = [k for name, k in kernels.items() if "add_rmsnorm_vec_kernel" in name and f"Li256ELi{chunks}E" in name]
+        assert len(normed) == 8
+        for k in normed:
+            assert k[".vgpr_count"] <= most and k[".private_segment_fixed_size"] == 0, k[".name"]
