@@ -104,7 +104,7 @@ __device__ inline void store4(bf16_t* p, const float v[4]) {
 }
 
 template <typename TD, typename TG, typename TY, int kThreads, int kChunks>
-__global__ void __launch_bounds__(kThreads)
+__global__ void __launch_bounds__(kThreads, kChunks == 8 ? 2 : kChunks == 4 ? 4 : 8)
 add_rmsnorm_vec_kernel(float* __restrict__ x, const TD* __restrict__ delta, int planes, long plane,
                        const TG* __restrict__ gain, float eps, TY* __restrict__ y, const int* __restrict__ rows,
                        int hidden, float* __restrict__ squares_out) {
