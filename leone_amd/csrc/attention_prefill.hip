@@ -503,22 +503,23 @@ attention_prefill_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ out,
 // Merges the key ranges of one row and query head: out = sum_s acc_s 2^(m_s - M) / sum_s l_s 2^(m_s - M),
 // the sums taken in range order; a range that held no key for the row (m_s = -inf) counts as nothing,
 // whatever its accumulator holds.  One wave a (row, head): lane s takes the reference and sum of range s,
-// then all lanes walk the accumulators together.  blockIdx.x is a tile and an eighth of its rows.
+// then all lanes walk the accumulators together.  blockIdx.x is a tile and a share of its rows.
 // A wave is a chain of trips to memory: the accumulators of four ranges at a time are asked for before it is known what they weigh.
 constexpr int kMergeWaves = 4;
 constexpr int kMergeThreads = kMergeWaves * kWave;
-constexpr int kMergeBlocksPerTile = kRowsPerWave / kMergeWaves;
 constexpr int kMergeAhead = 4;                                        // ranges on their way at a time
 constexpr int kMaxPrefillSplits = 32;
 
+template <int kRowsEach>
 __global__ void __launch_bounds__(kMergeThreads)
 attention_prefill_merge_kernel(const float* __restrict__ part_acc, const float* __restrict__ part_ml,
                                bf16_t* __restrict__ out, const int* __restrict__ tiles, int q_heads, int head_dim,
                                int splits, const int* __restrict__ positions, ScoreShape shape) {
-    const int* tile = tiles + 3 * static_cast<long>(blockIdx.x / kMergeBlocksPerTile);
+    constexpr int kBlocks = kRowsPerWave / (kMergeWaves * kRowsEach);
+    const int* tile = tiles + 3 * static_cast<long>(blockIdx.x / kBlocks);
     const int row0 = tile[1], rows = tile[2], head = blockIdx.y;
     const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-    for (int r = (blockIdx.x % kMergeBlocksPerTile) * kMergeWaves + wave; r < rows; r += kMergeWaves * kMergeBlocksPerTile) {
+    for (int r = (blockIdx.x % kBlocks) * kMergeWaves + wave; r < rows; r += kMergeWaves * kBlocks) {
         const long rh = static_cast<long>(row0 + r) * q_heads + head;
         const float2 ml = lane < splits ? reinterpret_cast<const float2*>(part_ml)[rh * splits + lane]
                                         : float2{-INFINITY, 0.f};
@@ -665,14 +666,19 @@ static void launch_merge(const float* part_acc, const float* part_ml, bf16_t* ou
 #define LEONE_MERGE_LANES(LANES)                                                                                                \
     attention_prefill_merge_lanes_kernel<LANES><<<dim3(n_tiles * (kRowsPerWave * LANES / (2 * kMergeThreads)), q_heads), kMergeThreads, 0, \
                                                   stream>>>(part_acc, part_ml, out, tiles, q_heads, splits, shape.sinks)
+#define LEONE_MERGE_ROWS(EACH)                                                                                                  \
+    attention_prefill_merge_kernel<EACH><<<dim3(n_tiles * (kRowsPerWave / (kMergeWaves * EACH)), q_heads), kMergeThreads, 0, stream>>>( \
+        part_acc, part_ml, out, tiles, q_heads, head_dim, splits, positions, shape)
     const bool as_they_are = shape.turn_cos == nullptr && reinterpret_cast<uintptr_t>(part_acc) % 16 == 0 &&
                              reinterpret_cast<uintptr_t>(part_ml) % 8 == 0 && reinterpret_cast<uintptr_t>(out) % 8 == 0;
     if (as_they_are && head_dim == 64) LEONE_MERGE_LANES(16);
     else if (as_they_are && head_dim == 128) LEONE_MERGE_LANES(32);
     else if (as_they_are && head_dim == 256) LEONE_MERGE_LANES(64);
-    else
-        attention_prefill_merge_kernel<<<dim3(n_tiles * kMergeBlocksPerTile, q_heads), kMergeThreads, 0, stream>>>(
-            part_acc, part_ml, out, tiles, q_heads, head_dim, splits, positions, shape);
+    // A row a wave; two one after the other where there are many waves that have little to read each, heads of up to 32 in two ranges (2,048
+    // rows of 16 heads of 16 and of 32, attention and merge, us: a row 46.5 and 49.6, two 44.1 and 46.7; 512 rows of 4 heads 12.4 and 13.1).
+    else if (head_dim <= 32 && splits <= 2 && static_cast<long>(n_tiles) * q_heads >= 1024) LEONE_MERGE_ROWS(2);
+    else LEONE_MERGE_ROWS(1);
+#undef LEONE_MERGE_ROWS
 #undef LEONE_MERGE_LANES
 }
 

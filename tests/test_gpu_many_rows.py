@@ -1,5 +1,6 @@
 """Row-wise kernels at the sizes where many rows, whole runs or several trips of a workgroup take another path: filters of four taps
 with a window in registers, the exponential gates of long portions."""
+import math
 from types import SimpleNamespace
 
 import pytest
@@ -187,3 +188,26 @@ def test_heads_in_runs_of_eight(rows, dim, turned, pairing, normed):
                     found.append((q, k_pool, v_pool))
                 assert all(torch.equal(a, b) for a, b in zip(*found)), (kind, given, queries_only)
                 assert queries_only or not torch.equal(found[0][1], pools[0])
+
+
+@pytest.mark.parametrize("dim,q_heads,kv_heads,rows", [(16, 32, 4, 1050), (32, 30, 2, 1089), (16, 16, 4, 600)])
+def test_two_key_ranges_of_small_heads(dim, q_heads, kv_heads, rows):
+    """Key ranges of a long portion merged two rows a wave, the last tile not full, and of a shorter one a row a wave."""
+    from leone_amd import ops
+    gen = torch.Generator().manual_seed(dim + rows)
+    page = 16
+    pages = -(-rows // page)
+    keys, values = (torch.randn(pages * page, kv_heads, dim, generator=gen).bfloat16() for _ in range(2))
+    k_pool = keys.view(pages, page, kv_heads, dim // 8, 8).permute(0, 2, 3, 1, 4).contiguous()
+    v_pool = values.view(pages, page // 8, 8, kv_heads, dim).permute(0, 3, 1, 4, 2).contiguous()
+    q = torch.randn(rows, q_heads, dim, generator=gen).bfloat16()
+    out = torch.empty(rows, q_heads * dim, dtype=torch.bfloat16, device=DEV)
+    table = torch.arange(pages, dtype=torch.int32, device=DEV).view(1, -1)
+    ops.attention_prefill(q.view(rows, -1).to(DEV), out, k_pool.to(DEV), v_pool.to(DEV), torch.arange(rows, dtype=torch.int32, device=DEV),
+                          ops.prefill_tiles([(0, 0, rows)]).to(DEV), table, q_heads, dim ** -0.5, splits=2)
+    hidden = torch.triu(torch.ones(rows, rows, dtype=torch.bool), 1)
+    for h in range(q_heads):
+        scores = (q[:, h].double() @ keys[:rows, h * kv_heads // q_heads].double().T) * dim ** -0.5
+        want = torch.softmax(scores.masked_fill(hidden, -math.inf), -1) @ values[:rows, h * kv_heads // q_heads].double()
+        # weights and results are rounded to eight bits: 2^-8 of the largest value, a few times over
+        assert float((out.view(rows, q_heads, dim)[:, h].cpu().double() - want).abs().max()) < 0.03
