@@ -360,7 +360,9 @@ attention_prefill_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ out,
         top *= to_log2;
         if (__any(top > m_ref + kRaise)) {                     // -inf + 8 is -inf: the first scores always raise
             // Some score outgrew its reference: every row takes its true maximum so far as the new one.
-            const float row_top = max_lanes<32>(top);
+            // (over the halves by a shuffle where heads are small: with the swap the loop around it is scheduled worse, 40 rows of heads of 32 behind
+            // 2,000 keys 44.4 us and 42.8, 512 of 64 behind 6,000 190 and 185; heads of 96 the other way, 232 with the swap and 239)
+            const float row_top = kD16 <= 4 ? fmaxf(top, __shfl_xor(top, 32, kWave)) : max_lanes<32>(top);
             const float m_new = fmaxf(m_ref, ceilf(row_top));           // a whole number: see the rounding of the weights below
             const float alpha = m_new == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m_ref - m_new);   // 2^-inf = 0
             m_ref = m_new;
@@ -428,7 +430,7 @@ attention_prefill_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ out,
     }
 
     const bool poisoned = unmapped_seen != 0;                    // every write to it came before the last barrier
-    const float l_row = add_lanes<32>(l_run);    // both halves of the keys
+    const float l_row = kD16 <= 4 ? l_run + __shfl_xor(l_run, 32, kWave) : add_lanes<32>(l_run);    // both halves of the keys
     if (splits > 1) {
         if (!row_ok) return;
         const long slot = (static_cast<long>(tile_row0 + j) * q_heads + head) * splits + blockIdx.y;
