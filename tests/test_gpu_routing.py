@@ -118,25 +118,56 @@ def test_tiles_by_pairs_and_width():
             assert ops._expert_tiles(x, line * experts, 1, experts, hidden, ff)[0] == above
 
 
+def _through_experts(x, which, weight, up, down, gated, weigh_input=False):
+    """Pair by pair through the experts in 64 bits, the middle rounded as the kernels hand it on.  up: [experts, 1 or 2, ff, hidden]."""
+    want = torch.empty(len(which), down.shape[1], dtype=F)
+    for e in range(up.shape[0]):
+        mine = which == e
+        a, first = weight[mine].double(), x[mine].double() @ up[e, 0].double().T
+        middle = plain.silu(first) * (x[mine].double() @ up[e, 1].double().T) if gated else (a * first if weigh_input else first).clamp(min=0).square()
+        each = middle.bfloat16().double() @ down[e].double().T
+        want[mine] = each if weigh_input else a * each
+    return want
+
+
+def _dealt(counts, hidden, ff, gated, seed):
+    gen = torch.Generator().manual_seed(seed)
+    which = torch.tensor([e for e, count in enumerate(counts) for _ in range(count)])[torch.randperm(sum(counts), generator=gen)]
+    return (torch.randn(len(which), hidden, generator=gen).bfloat16(), which, torch.rand(len(which), 1, generator=gen) + 0.1,
+            (torch.randn(len(counts), 2 if gated else 1, ff, hidden, generator=gen) / math.sqrt(hidden)).bfloat16(),
+            (torch.randn(len(counts), hidden, ff, generator=gen) / math.sqrt(ff)).bfloat16())
+
+
+def _check_pairs(counts, hidden, ff, gated, tile):
+    from leone_amd import ops
+    x, which, weight, up, down = _dealt(counts, hidden, ff, gated, hidden + ff)
+    assert ops._expert_tiles(x.to(DEV), len(which), 1, len(counts), hidden, ff)[0] == tile
+    for weigh_input in (False,) if gated else (False, True):
+        got = ops.routed_experts(x.to(DEV), which.view(-1, 1).to(torch.int32).to(DEV), weight.to(DEV), (up if gated else up[:, 0]).to(DEV),
+                                 down.to(DEV), "silu" if gated else "relu2", weigh_input=weigh_input).cpu().double()
+        want = _through_experts(x, which, weight, up, down, gated, weigh_input)
+        # as above: middles that are rounded to neighbours
+        assert float((got - want).norm() / want.norm()) < 2e-3
+
+
+@pytest.mark.parametrize("hidden,ff", [(264, 576), (328, 520), (392, 512), (448, 328), (512, 640), (520, 448), (576, 264), (704, 136)])
+@pytest.mark.parametrize("gated", [True, False])
+def test_tiles_of_sixty_four_over_many_chunks(hidden, ff, gated):
+    """Inner sizes of 3 to 11 chunks of 64, on and off a whole one: the loop over two chunks none, one and several times and every
+    number of chunks behind it, for the first product and the second."""
+    _check_pairs([63, 64, 65, 130, 1], hidden, ff, gated, 64)
+
+
+@pytest.mark.parametrize("hidden,ff", [(1032, 1408), (1408, 2056), (2048, 1032), (2056, 2568), (2568, 2048), (40, 4104), (4104, 24), (1984, 1000)])
+@pytest.mark.parametrize("gated", [True, False])
+def test_tiles_of_sixteen_over_long_rows(hidden, ff, gated):
+    """Inner sizes whose share of a wave is one batch of eight steps and a remainder, two and more batches, and ends inside a step; of
+    more than 2,048 by ordinary loads."""
+    _check_pairs([5, 0, 17, 2], hidden, ff, gated, 16)
+
+
 def test_products_with_one_chunk_ahead():
     """Experts whose matrices give every unit one workgroup, with rows whole multiples of 4 KB apart; some with more pairs than a tile."""
-    from leone_amd import ops
     from leone_amd.ops.library import library
-    experts, hidden, ff = 16, 2048, 1024
-    assert library().leone_moe_one_chunk_ahead(experts, 1, ff, hidden)
-    gen = torch.Generator().manual_seed(16)
-    counts = [3, 64, 1, 65, 0, 130] + [20] * 10
-    which = torch.tensor([e for e, count in enumerate(counts) for _ in range(count)])[torch.randperm(sum(counts), generator=gen)]
-    rows = len(which)
-    weight, x = torch.rand(rows, 1, generator=gen) + 0.1, torch.randn(rows, hidden, generator=gen).bfloat16()
-    up = (torch.randn(experts, 2, ff, hidden, generator=gen) / math.sqrt(hidden)).bfloat16()
-    down = (torch.randn(experts, hidden, ff, generator=gen) / math.sqrt(ff)).bfloat16()
-    assert ops._expert_tiles(x.to(DEV), rows, 1, experts, hidden, ff)[0] == 64
-    got = ops.routed_experts(x.to(DEV), which.view(-1, 1).to(torch.int32).to(DEV), weight.to(DEV), up.to(DEV), down.to(DEV)).cpu().double()
-    want = torch.empty(rows, hidden, dtype=F)
-    for e in range(experts):
-        mine = which == e
-        gate, more = (x[mine].double() @ up[e, i].double().T for i in (0, 1))
-        want[mine] = weight[mine].double() * ((plain.silu(gate) * more).bfloat16().double() @ down[e].double().T)
-    # as above: middles that are rounded to neighbours
-    assert float((got - want).norm() / want.norm()) < 2e-3
+    assert library().leone_moe_one_chunk_ahead(16, 1, 1024, 2048)
+    _check_pairs([3, 64, 1, 65, 0, 130] + [20] * 10, 2048, 1024, True, 64)
