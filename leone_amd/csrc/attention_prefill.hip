@@ -585,7 +585,7 @@ attention_prefill_merge_kernel(const float* __restrict__ part_acc, const float* 
 }
 
 // The same for heads of 64, 128 or 256 elements whose results stay as they are: kLanes lanes a row with four elements each, two rows a
-// lane, so that a wave has up to 16 KB on its way and every lane makes its row's weights itself.  Sums in the same order: the same bits.
+// lane, so that a wave has up to 8 KB on its way and every lane makes its row's weights itself.  Sums in the same order: the same bits.
 // us (a wave a row and an element a lane): 512 rows of 32 heads of 128 in four ranges 9.3 (12.7; 18.5 with a range a trip), 2,048 rows
 // of 16 heads in two 11.3 (18.7).
 template <int kLanes>

@@ -116,7 +116,8 @@ struct Four<bf16_t> {
 // A shuffle (ds_bpermute) is a trip through the shared-memory unit, some 60 cycles that the next addition waits for, and a wave's
 // sum is six of them one after the other.  Lanes of the same row of 16 are reached by an operand's own permutation (DPP) instead,
 // the other rows and halves by the lane swaps: a few cycles each.  Which lanes meet, and in which order, is the shuffles', so the
-// results are the same bits.  Every lane of the wave has to take part.
+// results are the same bits.  Lanes 1, 2, 4 and 8 apart: every lane of a row of 16 that takes part has the whole row beside it; 16 and
+// 32 apart: every lane of the wave takes part (a swap with a lane that does not gives nothing defined).
 //
 // The value of the lane that the permutation kControl of a row's 16 lanes names (one that stays within the row).
 template <int kControl, typename T>

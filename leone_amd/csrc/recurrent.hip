@@ -468,6 +468,8 @@ __global__ void __launch_bounds__(kScanThreads) delta_scan_kernel(DeltaScanArgs 
                     qq = fmaf(qs[i], qs[i], qq);
                     kk = fmaf(ks[i], ks[i], kk);
                 }
+                // (on a chunk's last rows only some of the lanes are here, whole rows of 16 of them)
+                static_assert(kRowLanes <= 16 && 16 % kRowLanes == 0, "a row's lanes meet within a row of 16 lanes");
                 qq = add_span<kRowLanes>(qq);
                 kk = add_span<kRowLanes>(kk);
                 const float qinv = p.q_scale / sqrtf(qq + p.unit_eps);

@@ -2,7 +2,7 @@
 // saved to and put back from a packed buffer in one launch.
 //
 // A model has a few dozen state tensors of some KB to some MB a slot.  One call of torch for each is bound by the host (10 to 20 us a
-// tensor and direction), not by the bytes.  Twenty tensors, 2.2 MB a request: eight requests that fork and decode 12 tokens 7,684 us
+// tensor and direction), not by the bytes.  Twenty tensors, 11.9 MB a request: eight requests that fork and decode 12 tokens 7,684 us
 // with a call a tensor, 5,713 so; a prompt of 2,048 tokens, whose slot is cleared and saved first, 3,969 and 3,502.  The tensors'
 // addresses stand in a table on the device; the bytes of all of them are one range of chunks, a workgroup each, so that the launch
 // is as wide as there is work and small tensors do not wait for each other.

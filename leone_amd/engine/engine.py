@@ -384,7 +384,7 @@ class Engine:
         self.poison_freed_pages()              # what a scheduler on the same manager has freed since the last step
         # A failed step gives its pages back (rollback) and leaves per-request state as it found it.  A step that is
         # replayed from a recording it already has cannot fail half way (it is refused before the replay or not at
-        # all), so the copy of the state, a kernel for every state tensor of the model, is left out there.
+        # all), so the copy of the state, a launch and all its bytes, is left out there.
         replayed = self.graphs and not profile.recording() and all(len(e.tokens) == 1 for e in entries)
         saved_state = None if (replayed and self._has_recording(entries)) else \
             self.pools.snapshot_state([self.cache.slot(e.request) for e in entries])
