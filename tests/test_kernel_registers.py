@@ -77,3 +77,11 @@ def test_rms_norms_in_registers(kernels):
         assert len(normed) == 8
         for k in normed:
             assert k[".vgpr_count"] <= most and k[".private_segment_fixed_size"] == 0, k[".name"]
+
+
+def test_gated_products_of_many_rows(kernels):
+    """Six tiles of rows a wave, and four under a row-major weight, leave three waves a SIMD (168 registers of 512) where one wave takes
+    a tile of the weight."""
+    gated = [k for name, k in kernels.items() if "gemm_rows_kernelILi6ELi4ELi1ELi2ELi1ELi2E" in name
+             or ("gemm_rows_kernelILi4ELi4ELi1ELi4ELi1ELi2E" in name and "Lb0EEE" in name)]
+    assert len(gated) == 3 and all(k[".vgpr_count"] <= 168 for k in gated)
