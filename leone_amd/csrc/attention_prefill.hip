@@ -664,7 +664,7 @@ attention_prefill_merge_lanes_kernel(const float* __restrict__ part_acc, const f
 }
 
 static void launch_merge(const float* part_acc, const float* part_ml, bf16_t* out, const int* tiles, int n_tiles, int q_heads, int head_dim,
-                         int splits, const int* positions, const ScoreShape& shape, hipStream_t stream) {
+                         int splits, int tile_rows, const int* positions, const ScoreShape& shape, hipStream_t stream) {
 #define LEONE_MERGE_LANES(LANES)                                                                                                \
     attention_prefill_merge_lanes_kernel<LANES><<<dim3(n_tiles * (kRowsPerWave * LANES / (2 * kMergeThreads)), q_heads), kMergeThreads, 0, \
                                                   stream>>>(part_acc, part_ml, out, tiles, q_heads, splits, shape.sinks)
@@ -676,17 +676,18 @@ static void launch_merge(const float* part_acc, const float* part_ml, bf16_t* ou
     if (as_they_are && head_dim == 64) LEONE_MERGE_LANES(16);
     else if (as_they_are && head_dim == 128) LEONE_MERGE_LANES(32);
     else if (as_they_are && head_dim == 256) LEONE_MERGE_LANES(64);
-    // A row a wave; two one after the other where there are many waves that have little to read each, heads of up to 32 in two ranges (2,048
-    // rows of 16 heads of 16 and of 32, attention and merge, us: a row 46.5 and 49.6, two 44.1 and 46.7; 512 rows of 4 heads 12.4 and 13.1).
-    else if (head_dim <= 32 && splits <= 2 && static_cast<long>(n_tiles) * q_heads >= 1024) LEONE_MERGE_ROWS(2);
+    // A row a wave, which in tiles of up to 16 rows is half as many workgroups (1,024 rows of 32 heads of 96 in such tiles, attention and
+    // merge, us: 132.7, 147.2 with all of them); two rows one after the other where there are many waves that have little to read each, heads of up
+    // to 32 in two ranges (2,048 rows of 16 heads of 16 and of 32: a row 46.5 and 49.6, two 44.1 and 46.7; 512 rows of 4 heads 12.4 and 13.1).
+    else if (tile_rows <= kRowsPerWave / 2 || (head_dim <= 32 && splits <= 2 && static_cast<long>(n_tiles) * q_heads >= 1024)) LEONE_MERGE_ROWS(2);
     else LEONE_MERGE_ROWS(1);
 #undef LEONE_MERGE_ROWS
 #undef LEONE_MERGE_LANES
 }
 
 void launch_attention_tile_merge(const float* part_acc, const float* part_ml, bf16_t* out, const int* tiles, int n_tiles, int q_heads,
-                                 int head_dim, int splits, hipStream_t stream) {
-    launch_merge(part_acc, part_ml, out, tiles, n_tiles, q_heads, head_dim, splits, nullptr, ScoreShape{}, stream);
+                                 int head_dim, int splits, int tile_rows, hipStream_t stream) {
+    launch_merge(part_acc, part_ml, out, tiles, n_tiles, q_heads, head_dim, splits, tile_rows, nullptr, ScoreShape{}, stream);
 }
 int attention_tile_merge_max_splits() { return kMaxPrefillSplits; }
 
@@ -823,8 +824,8 @@ extern "C" int leone_attention_prefill_shaped(const void* q, void* out, const vo
     if (status) return status;
     LEONE_LAUNCH_CHECK("attention_prefill");
     if (splits > 1) {
-        launch_merge(part_acc, part_ml, static_cast<bf16_t*>(out), tiles, n_groups * kPrefillWaves, q_heads, head_dim, splits, positions,
-                     shape, stream);
+        launch_merge(part_acc, part_ml, static_cast<bf16_t*>(out), tiles, n_groups * kPrefillWaves, q_heads, head_dim, splits, kRowsPerWave,
+                     positions, shape, stream);
         LEONE_LAUNCH_CHECK("attention_prefill_merge");
     }
     return 0;

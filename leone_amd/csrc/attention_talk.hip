@@ -856,7 +856,7 @@ extern "C" int leone_attention_talk_prefill(const void* q, void* out, const void
 #undef LEONE_TALK_PREFILL
     LEONE_LAUNCH_CHECK("attention_talk_prefill");
     if (splits > 1) {
-        launch_attention_tile_merge(part_acc, part_ml, static_cast<bf16_t*>(out), tiles, n_tiles, q_heads, v_dim, splits, stream);
+        launch_attention_tile_merge(part_acc, part_ml, static_cast<bf16_t*>(out), tiles, n_tiles, q_heads, v_dim, splits, kTalkRows, stream);
         LEONE_LAUNCH_CHECK("attention_talk_prefill merge");
     }
     return 0;
