@@ -601,8 +601,8 @@ attention_talk_prefill_kernel(TalkArgs a, const int* __restrict__ tiles, int n_t
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
                         float top = fmaxf(fmaxf(d[0][i], d[1][i]), fmaxf(d[2][i], d[3][i]));
-                        top = max_lanes<16>(top);
-                        top = max_lanes<32>(top);
+                        top = kIn > 16 ? fmaxf(top, __shfl_xor(top, 16, kWave)) : max_lanes<16>(top);
+                        top = kIn > 16 ? fmaxf(top, __shfl_xor(top, 32, kWave)) : max_lanes<32>(top);
                         if (g == 0) smax[(wave * kH + 4 * b + i) * 16 + c] = top;
                     }
                 } else {
@@ -703,8 +703,10 @@ attention_talk_prefill_kernel(TalkArgs a, const int* __restrict__ tiles, int n_t
     for (int w = 0; w < kHW; ++w) {
         const int h = head_of(w);
         float l = l_run[w];
-        l = add_lanes<16>(l);
-        l = add_lanes<32>(l);
+        // (of more than 16 heads by shuffles, as the maxima above: what the swaps hold goes to scratch there, 124 bytes a lane and 100; 1,024 rows
+        // of 32 heads of 128 over 8 204 us, so 201)
+        l = kIn > 16 ? l + __shfl_xor(l, 16, kWave) : add_lanes<16>(l);
+        l = kIn > 16 ? l + __shfl_xor(l, 32, kWave) : add_lanes<32>(l);
         if (poisoned) l = __builtin_nanf("");
         if (out0 + h >= heads || c >= rows) continue;
         const long rh = (static_cast<long>(row0) + c) * heads + out0 + h;

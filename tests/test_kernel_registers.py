@@ -85,3 +85,10 @@ def test_gated_products_of_many_rows(kernels):
     gated = [k for name, k in kernels.items() if "gemm_rows_kernelILi6ELi4ELi1ELi2ELi1ELi2E" in name
              or ("gemm_rows_kernelILi4ELi4ELi1ELi4ELi1ELi2E" in name and "Lb0EEE" in name)]
     assert len(gated) == 3 and all(k[".vgpr_count"] <= 168 for k in gated)
+
+
+def test_attention_with_mixed_scores(kernels):
+    """What 32 heads of 128 with keys of their own leave to scratch, and no more; smaller ones leave less or nothing."""
+    found = {name: k[".private_segment_fixed_size"] for name, k in kernels.items() if "attention_talk_prefill_kernel" in name}
+    assert len(found) == 16 and max(found.values()) <= 100
+    assert not any(size for name, size in found.items() if "Li64E" in name)
