@@ -88,7 +88,8 @@ def test_gated_products_of_many_rows(kernels):
 
 
 def test_attention_with_mixed_scores(kernels):
-    """What 32 heads of 128 with keys of their own leave to scratch, and no more; smaller ones leave less or nothing."""
-    found = {name: k[".private_segment_fixed_size"] for name, k in kernels.items() if "attention_talk_prefill_kernel" in name}
-    assert len(found) == 16 and max(found.values()) <= 100
-    assert not any(size for name, size in found.items() if "Li64E" in name)
+    """What 32 heads of 128 leave to scratch, with keys of their own and with keys that four share, and no more; smaller ones less or nothing."""
+    found = {name.split("attention_talk_prefill_kernel")[1][:24]: k[".private_segment_fixed_size"] for name, k in kernels.items()
+             if "attention_talk_prefill_kernel" in name}
+    assert len(found) == 16 and found.pop("ILi128ELi32ELi4ELi1EEEvN") <= 100 and found.pop("ILi128ELi32ELi4ELi4EEEvN") <= 176
+    assert max(found.values()) <= 80 and not any(size for name, size in found.items() if name.startswith("ILi64E"))
