@@ -46,13 +46,18 @@ class StateSlots:
         most = library().leone_state_slots_max()
         # On the tensors' device whatever the caller's is: requests are admitted and forked from any thread, and a thread that has
         # not chosen a device stands on the first.
-        with torch.cuda.device(self.table.device):
-            for at in range(0, len(ids), most):
-                some, there = ids[at:at + most], to[at:at + most]
-                array = ctypes.c_int * len(some)
-                call("leone_state_slots", self.table.data_ptr(), len(self.tensors), self.chunks, move, array(*some),
-                     array(*there) if there else None, len(some), 0 if packed is None else packed[at:].data_ptr(), self.packed_bytes,
-                     _stream())
+        if torch.cuda.current_device() == self.table.device.index:
+            self._launch(move, ids, to, packed, most)
+        else:
+            with torch.cuda.device(self.table.device):
+                self._launch(move, ids, to, packed, most)
+
+    def _launch(self, move: int, ids: Sequence[int], to: Sequence[int], packed, most: int) -> None:
+        for at in range(0, len(ids), most):
+            some, there = ids[at:at + most], to[at:at + most]
+            array = ctypes.c_int * len(some)
+            call("leone_state_slots", self.table.data_ptr(), len(self.tensors), self.chunks, move, array(*some),
+                 array(*there) if there else None, len(some), 0 if packed is None else packed[at:].data_ptr(), self.packed_bytes, _stream())
 
     def zero(self, slots: Sequence[int]) -> None:
         self._move(self.ZERO, list(slots))

@@ -19,6 +19,7 @@ def test_slots_move_on_their_tensors_device(monkeypatch, move):
         current[0] = before
 
     monkeypatch.setattr(torch.cuda, "device", device)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: int(current[0][-1]))
     monkeypatch.setattr(state, "library", lambda: SimpleNamespace(leone_state_slots_max=lambda: 64))
     monkeypatch.setattr(state, "_stream", lambda: current[0])
     monkeypatch.setattr(state, "call", lambda name, *args: seen.append(args[-1]))
