@@ -4,16 +4,20 @@
 // 1622-1640).
 //
 // An output's bits depend on its row of A, its row of B and K alone, never on the rows that share the launch (what a request gets
-// does not depend on who is beside it): K is cut into segments by a rule on K (f32_segments), a segment's sum is that of chains of
-// 16 fused products, k ascending, added in order, and so is the segments' sum.  Both kernels below work that way.  What is added rounds
-// at the sum's size, so the short sums are also off by less than one chain over K (error against 64 bits over the result's norm, 1 to 1,024 rows:
-// K 512 1.0e-7, 2048 1.2e-7, 6144 1.6e-7; one chain 2.9e-7, 8.1e-7 and 9.9e-7).  A K below 256 is one chain, the scalar backend's fold.
+// does not depend on who is beside it): K is cut into segments by a rule on K (f32_segments), a segment's sum is that of the sums of 32
+// products, k ascending, added in order, and so is the segments' sum.  A K below 256 is one chain of float products, the scalar
+// backend's fold.
+//
+// The matrix instructions take floats at a sixteenth of the rate of bfloat16.  From a K of 256 on, numbers are therefore taken apart
+// into three bfloat16 each, which hold all of their 24 bits, and a product is made of the six products of parts that reach a float's last
+// bit: 2.7 times the float rate, and the sums of 32 round less often than chains of float products do (error against 64 bits over the
+// result's norm, 1 to 1,024 rows: K 512 0.7e-7, 2048 0.9e-7, 6144 1.2e-7; chains of 16 float products 1.0e-7, 1.2e-7 and 1.6e-7).
 //
 // Few rows (decoding): a product reads every weight once for 2 M operations, so the weights' bytes are the
 // bound and what matters is how much of them is in flight: a workgroup owns 16 rows of B, its waves take a segment each, and a
-// wave keeps eight 1 KB loads of B in the air.  Many rows (prompt portions): tiles staged through shared memory, bound by
-// the matrix instructions (256 operations a cycle and compute unit).  With few tiles the segments are shared out over
-// workgroups, which leave them as planes in a buffer of the caller's for a second kernel to add.
+// wave keeps its next loads of B in the air.  Many rows (prompt portions): tiles, whose rows of A are staged through shared memory.
+// With few tiles the segments are shared out over workgroups, which leave them as planes in a buffer of the caller's for a second
+// kernel to add.
 #include "common.h"
 #include "leone_hip.h"
 
@@ -44,31 +48,88 @@ __device__ inline f32x4 load_whole(const float* __restrict__ at) {
     return f32x4{at[0], at[1], at[2], at[3]};
 }
 
+// ---- three parts a number --------------------------------------------------------------------------------------------
+// The 16 x 16 x 32 instruction takes eight bfloat16 a lane and adds in float.  A float is the sum of three bfloat16 (8 bits each,
+// rounded to nearest, so that what is left is at most half of the last bit and of either sign); a product of two floats is six of
+// the nine products of their parts, the other three lie below a quarter of a float's last bit.
+typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+
+// The next part of two numbers, taken off them.
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+__device__ inline unsigned next_part(float& a, float& b) {
+    unsigned bits = __builtin_bit_cast(unsigned, bf16x2{static_cast<__bf16>(a), static_cast<__bf16>(b)});
+    asm("" : "+v"(bits));          // (one conversion of both, not another of each for what is taken off)
+    a -= __uint_as_float(bits << 16);
+    b -= __uint_as_float(bits & 0xffff0000u);
+    return bits;
+}
+// Four numbers' parts, highest first.
+struct FourParts {
+    u32x2 part[3];
+};
+__device__ inline FourParts parts_of(f32x4 v) {
+    FourParts r;
+#pragma unroll
+    for (int p = 0; p < 3; ++p) {
+        float a = v[0], b = v[1], c = v[2], d = v[3];
+        const unsigned low = next_part(a, b), high = next_part(c, d);
+        r.part[p] = u32x2{low, high};
+        v = f32x4{a, b, c, d};
+    }
+    return r;
+}
+// A lane's operand of one instruction: eight numbers in three parts.
+struct Operand {
+    bf16x8 part[3];
+};
+__device__ inline Operand operand_of(const f32x4& first, const f32x4& second) {
+    const FourParts a = parts_of(first), b = parts_of(second);
+    Operand r;
+#pragma unroll
+    for (int p = 0; p < 3; ++p) r.part[p] = __builtin_bit_cast(bf16x8, u32x4{a.part[p][0], a.part[p][1], b.part[p][0], b.part[p][1]});
+    return r;
+}
+// The sum of 32 products, the smallest parts first.  What the instruction loses when it brings its products to one exponent it takes
+// off, whatever their sign (sums of 2,048 come out 5e-8 of their root mean square too low), so every other 32 elements of a segment
+// are multiplied with A's sign turned and their sum is subtracted.
+constexpr int kTerms = 6, kTermA[kTerms] = {2, 0, 1, 1, 0, 0}, kTermB[kTerms] = {0, 2, 1, 0, 1, 0};
+__device__ inline f32x4 add_term(int term, const Operand& a, const Operand& b, const f32x4& sum) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.part[kTermA[term]], b.part[kTermB[term]], sum, 0, 0, 0);
+}
+// An infinity has no parts (what is left of it is not a number), and neither have numbers that round to one; the parts of a number
+// below 2^-108 can lie below what the instruction takes for zero, which is off by at most 2^-126 of the other factor.  A segment's
+// sum that comes out infinite, NaN or that small is therefore made again, one product after the other.
+constexpr unsigned kLeastBits = 0x1f800000u, kMostBits = 0x7f7fffffu;      // 2^-64 and the largest number
+__device__ inline bool in_doubt(float v) {
+    const unsigned size = __float_as_uint(v) & 0x7fffffffu;
+    return size != 0 && size - kLeastBits > kMostBits - kLeastBits;
+}
+__device__ float plain_segment(const float* __restrict__ a, const float* __restrict__ b, int first, int end) {
+    float sum = 0.f;
+    for (int at = first; at < end; at += 16) {
+        float chain = 0.f;
+        for (int e = at; e < at + 16 && e < end; ++e) chain = fmaf(a[e], b[e], chain);
+        sum += chain;
+    }
+    return sum;
+}
+
 // ---- few rows ------------------------------------------------------------------------------------------------------
 // Lane l of a wave loads, of 16 rows of B, row l % 16's elements 4 (l / 16) .. + 3 of every run of 16: one 16-byte load
 // a lane is 64 bytes of each of 16 rows.  A's rows lie the same way, out of the caches (rows past the last are the last one again
-// and not written).  The 16 x 16 x 4 instruction adds its four products in the order of the lanes' quarters, so the four quarters'
-// registers are transposed by lane swaps first: instruction j then takes elements 4 j .. 4 j + 3 in turn.
+// and not written).  Two such runs are a lane's eight numbers of an instruction.
 constexpr int kStreamTile = 16;                        // rows of B a workgroup
-constexpr int kStreamRun = 64;                         // elements of K a wave takes at a time
+constexpr int kStreamRun = 32;                         // elements of K a wave takes at a time
 constexpr int kStreamLoads = kStreamRun / 16;
-constexpr int kChain = 16;                             // elements of K a chain of products: what a wave's 16-byte loads bring
+constexpr int kChain = 32;                             // elements of K whose products are added up before they meet a sum
 
-// Register j of quarter g becomes register g of quarter j.
-__device__ inline f32x4 transpose_quarters(const f32x4 v) {
-    typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
-    const auto bits = [](float f) { return __float_as_uint(f); };
-    const u32x2 p = __builtin_amdgcn_permlane32_swap(bits(v[0]), bits(v[2]), false, false);
-    const u32x2 q = __builtin_amdgcn_permlane32_swap(bits(v[1]), bits(v[3]), false, false);
-    const u32x2 r = __builtin_amdgcn_permlane16_swap(p[0], q[0], false, false);
-    const u32x2 s = __builtin_amdgcn_permlane16_swap(p[1], q[1], false, false);
-    return f32x4{__uint_as_float(r[0]), __uint_as_float(r[1]), __uint_as_float(s[0]), __uint_as_float(s[1])};
-}
-
-template <int kTilesM, int kWaves, int kDepth, bool kVec>
-__global__ void __launch_bounds__(kWaves * kWave)
+template <int kTilesM, int kWaves, int kDepth, int kEach, bool kVec>
+__global__ void __launch_bounds__(kWaves * kWave, kEach)
 gemm_f32_stream_kernel(const float* __restrict__ a, const float* __restrict__ b, float* __restrict__ c, int m, int n, int k, int segment) {
     __shared__ float sums[kWaves][kTilesM][kStreamTile * kStreamTile];
+    static_assert(kDepth % 2 == 0, "a register's runs are all even ones or all odd ones");
     const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
     const int n0 = blockIdx.x * kStreamTile;
     const int r = lane % 16, h = (lane / 16) * 4;
@@ -87,20 +148,18 @@ gemm_f32_stream_kernel(const float* __restrict__ a, const float* __restrict__ b,
 #pragma unroll
             for (int i = 0; i < kStreamLoads; ++i) x[into][t][i] = load_whole<kVec>(arow[t] + at + i * 16 + h);
     };
-    const auto multiply = [&](int from) {
+    const auto multiply = [&](int from, bool odd) {     // (see kTerms)
 #pragma unroll
-        for (int i = 0; i < kStreamLoads; ++i) {
-            const f32x4 wt = transpose_quarters(w[from][i]);
-            f32x4 xt[kTilesM];
+        for (int i = 0; i < kStreamLoads; i += 2) {
+            const Operand wp = operand_of(w[from][i], w[from][i + 1]);
 #pragma unroll
-            for (int t = 0; t < kTilesM; ++t) xt[t] = transpose_quarters(x[from][t][i]);
-            f32x4 acc[kTilesM] = {};
+            for (int t = 0; t < kTilesM; ++t) {
+                const Operand xp = odd ? operand_of(-x[from][t][i], -x[from][t][i + 1]) : operand_of(x[from][t][i], x[from][t][i + 1]);
+                f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
-#pragma unroll
-                for (int t = 0; t < kTilesM; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(xt[t][j], wt[j], acc[t], 0, 0, 0);
-#pragma unroll
-            for (int t = 0; t < kTilesM; ++t) sum[t] += acc[t];
+                for (int e = 0; e < kTerms; ++e) acc = add_term(e, xp, wp, acc);
+                sum[t] = odd ? sum[t] - acc : sum[t] + acc;
+            }
         }
     };
     // whole runs, kDepth of them on their way at a time; the loop's body asks for a run on every pass, so that the compiler can
@@ -112,12 +171,12 @@ gemm_f32_stream_kernel(const float* __restrict__ a, const float* __restrict__ b,
         for (; left >= 2 * kDepth; left -= kDepth, at += kDepth * kStreamRun)
 #pragma unroll
             for (int d = 0; d < kDepth; ++d) {
-                multiply(d);
+                multiply(d, d % 2);
                 fetch(at + (kDepth + d) * kStreamRun, d);
             }
 #pragma unroll
         for (int d = 0; d < kDepth; ++d) {
-            multiply(d);
+            multiply(d, d % 2);
             if (kDepth + d < left) fetch(at + (kDepth + d) * kStreamRun, d);
         }
         left -= kDepth, at += kDepth * kStreamRun;
@@ -128,7 +187,7 @@ gemm_f32_stream_kernel(const float* __restrict__ a, const float* __restrict__ b,
     }
 #pragma unroll
     for (int d = 0; d < kDepth - 1; ++d)
-        if (d < left) multiply(d);
+        if (d < left) multiply(d, d % 2);
     at += left * kStreamRun;
     if (at < end) {                                    // the rest of the last segment, filled up with zeros
 #pragma unroll
@@ -137,12 +196,16 @@ gemm_f32_stream_kernel(const float* __restrict__ a, const float* __restrict__ b,
         for (int t = 0; t < kTilesM; ++t)
 #pragma unroll
             for (int i = 0; i < kStreamLoads; ++i) x[0][t][i] = load_four<kVec>(arow[t], at + i * 16 + h, end);
-        multiply(0);
+        left % 2 ? multiply(0, true) : multiply(0, false);
     }
 #pragma unroll
     for (int t = 0; t < kTilesM; ++t)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) sums[wave][t][(h + i) * kStreamTile + r] = sum[t][i];
+        for (int i = 0; i < 4; ++i) {
+            const int row = t * 16 + h + i;
+            if (in_doubt(sum[t][i])) sum[t][i] = plain_segment(a + static_cast<long>(row < m ? row : m - 1) * k, brow, first, end);
+            sums[wave][t][(h + i) * kStreamTile + r] = sum[t][i];
+        }
     __syncthreads();
     for (int e = threadIdx.x; e < kTilesM * 256; e += kWaves * kWave) {
         const int t = e / 256, row = t * 16 + e % 256 / 16, col = n0 + e % 16;
@@ -155,46 +218,208 @@ gemm_f32_stream_kernel(const float* __restrict__ a, const float* __restrict__ b,
 }
 
 // ---- many rows -----------------------------------------------------------------------------------------------------
-// A tile of kRows x 64 outputs, four waves of a quarter each (32 x 32 x 2 instructions, kRows / 64 of them a wave).  Slabs of K in
-// shared memory, rows 4 floats further apart than they are long (16-byte reads of 8 neighbouring
-// rows then touch every bank once); the next slab is on its way into registers while one is multiplied, and is long enough
-// (2048 cycles of instructions a wave) to arrive meanwhile.  Of every 8 elements the
-// even ones lie first and then the odd ones: half-wave h reads its four at once, and the four instructions take elements 0
-// and 1, 2 and 3, .. of them: k ascending.  A chain, a segment's sum of chains and the sum of segments each have registers of their
-// own, which is what bounds the tile: 128 x 128 would need more than the 256 that two waves a SIMD leave each other.  1,024 rows
-// against 12288 x 2048: 470 us, 110 TFLOP/s (one chain an output in tiles of 128 x 128: 452); 777 rows 440 (408).
+// A tile of 64 x kCols outputs, four waves side by side.  A wave's columns are its own: it takes their elements of B from memory as
+// the kernel above does, and takes them apart in registers.  All four waves need A's rows: slabs of 32 elements of K in shared memory,
+// in parts (64 bytes a row and part); a lane's eight numbers of an instruction, elements 4 g .. + 3 and 16 + 4 g .. + 3 of the slab for
+// g = lane / 16, lie together, and the four lanes' places of a row change with every second row, so that eight neighbouring lanes touch
+// every bank once.  While a slab is multiplied, A's next one is taken apart between the instructions, and the one after that and B's
+// next one are on their way into registers.
 //
-// kCut: blockIdx.z takes `each` segments and leaves a plane of c for every one of them; else one workgroup walks them all.  kChains:
-// segments are sums of chains of kChain elements, else one chain.
-constexpr int slab_of(int rows) { return rows == 128 ? 32 : 64; }
-constexpr int kTileCols = 64;
+// What bounds it is that the matrix instructions (six for what one product of floats needs), the taking apart (half of the vector
+// instructions) and the trips through shared memory follow one another within a wave; three workgroups a unit make up for it to half of
+// the instructions' rate.  Columns of their own keep B out of shared memory: 777 rows against 12288 x 2048 take 243 us (161 TFLOP/s
+// in floats), with both operands in shared memory 303, on the float instructions 437; against 2048 x 6144 137, 150 and 219.
+//
+// kCut: blockIdx.z takes `each` segments and leaves a plane of c for every one of them; else one workgroup walks them all.
+constexpr int kSlab = kChain;
+constexpr int kTileRows = 64;
 
-template <int kRows, bool kVec, bool kCut, bool kChains>
-__global__ void __launch_bounds__(256, 2)
+template <int kCols, bool kVec, bool kCut>
+__global__ void __launch_bounds__(256, 3)
 gemm_f32_tile_kernel(const float* __restrict__ a, const float* __restrict__ b, float* __restrict__ c, int m, int n, int k,
                      int segment, int each) {
-    constexpr int kSlab = slab_of(kRows);
-    constexpr int kFrag = kRows / 64;                  // 32 x 32 squares of a wave, one under the other
-    constexpr int kLoadsA = kRows * kSlab / 4 / 256, kLoadsB = kTileCols * kSlab / 4 / 256;    // 16-byte loads a thread and slab
-    __shared__ float as[2][kRows][kSlab + 4];
-    __shared__ float bs[2][kTileCols][kSlab + 4];
+    constexpr int kFragA = kTileRows / 16, kFragB = kCols / 64;                      // 16 x 16 squares of a wave
+    constexpr int kLoadsA = kTileRows / 32;                                          // 16-byte loads a thread and slab
+    __shared__ u32x2 slabs[2][3][kTileRows][8];
     const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-    const int m0 = blockIdx.y * kRows, n0 = blockIdx.x * kTileCols;
+    const int m0 = blockIdx.y * kTileRows, n0 = blockIdx.x * kCols + wave * (kCols / 4);
+    const int r = lane % 16, g = lane / 16;
     const long part = static_cast<long>(segment) * each;
     const int k_first = static_cast<int>(blockIdx.z * part), k_end = k - k_first > part ? static_cast<int>(k_first + part) : k;
-    const int wm = (wave / 2) * (kRows / 2), wn = (wave % 2) * (kTileCols / 2);
-    f32x16 acc[kFrag] = {}, sum[kFrag] = {}, total[kFrag] = {};
+    const int four = threadIdx.x % 8, from_row = threadIdx.x / 8;                // this thread's four elements of every 32nd row of A
+    const float *arow[kLoadsA], *brow[kFragB];
+#pragma unroll
+    for (int i = 0; i < kLoadsA; ++i) arow[i] = a + static_cast<long>(m0 + from_row + i * 32 < m ? m0 + from_row + i * 32 : m - 1) * k;
+#pragma unroll
+    for (int j = 0; j < kFragB; ++j) brow[j] = b + static_cast<long>(n0 + j * 16 + r < n ? n0 + j * 16 + r : n - 1) * k;
+    f32x4 sum[kFragA][kFragB] = {};
+    [[maybe_unused]] f32x4 total[kFragA][kFragB] = {};
+    f32x4 ra[kLoadsA], rb[kFragB][2];
+    // (past the last element of a row: its last ones, and not used)
+    const auto load_at = [&](const float* row, int at) {
+        if (kVec) return *reinterpret_cast<const f32x4*>(row + (at < k ? at : k - 4));
+        f32x4 v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = row[at + e < k ? at + e : k - 1];
+        return v;
+    };
+    const auto fetch_a = [&](int k0) {
+#pragma unroll
+        for (int i = 0; i < kLoadsA; ++i) ra[i] = load_at(arow[i], k0 + four * 4);
+    };
+    const auto fetch_b = [&](int k0) {
+#pragma unroll
+        for (int j = 0; j < kFragB; ++j)
+#pragma unroll
+            for (int half = 0; half < 2; ++half) rb[j][half] = load_at(brow[j], k0 + half * 16 + g * 4);
+    };
+    const auto cut_off = [&](int k0) {                  // what lies past K in a slab of A counts as zero
+        if (k0 + kSlab <= k) return;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (k0 + four * 4 + e >= k) {
+#pragma unroll
+                for (int i = 0; i < kLoadsA; ++i) ra[i][e] = 0.f;
+            }
+    };
+    const auto cut_off_b = [&](int k0) {                // and of B
+        if (k0 + kSlab <= k) return;
+#pragma unroll
+        for (int half = 0; half < 2; ++half)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (k0 + half * 16 + g * 4 + e >= k) {
+#pragma unroll
+                    for (int j = 0; j < kFragB; ++j) rb[j][half][e] = 0.f;
+                }
+    };
+    const auto place = [](int row, int of) { return of ^ (row / 2 % 4); };       // of lane group `of`'s sixteen bytes
+    const int kept_at = place(from_row, four % 4) * 2 + four / 4;                // (32 rows further it is the same)
+    const auto keep = [&](int into, int i, float sign) {
+        const FourParts v = parts_of(ra[i] * sign);
+#pragma unroll
+        for (int p = 0; p < 3; ++p) slabs[into][p][from_row + i * 32][kept_at] = v.part[p];
+    };
+    const int col = n0 + r;                                                      // of the first square; rows 4 g .. + 3
+    const auto row_of = [&](int i, int e) { return m0 + i * 16 + 4 * g + e; };
+    const auto store = [&](const f32x4 (&of)[kFragA][kFragB], float* to) {
+#pragma unroll
+        for (int i = 0; i < kFragA; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int j = 0; j < kFragB; ++j)
+                    if (row_of(i, e) < m && col + j * 16 < n) to[static_cast<long>(row_of(i, e)) * n + col + j * 16] = of[i][j][e];
+    };
+    fetch_a(k_first);
+    fetch_b(k_first);
+    cut_off(k_first);
+#pragma unroll
+    for (int i = 0; i < kLoadsA; ++i) keep(0, i, 1.0f);
+    fetch_a(k_first + kSlab);
+    float sign = 1.0f;                                 // of the slab that is multiplied (see kTerms)
+    int at = 0, segment_first = k_first;               // segments are an even number of slabs
+    float* plane = c + static_cast<long>(blockIdx.z) * each * m * n;
+    const int mine = place(r, g) * 2;
+    for (int k0 = k_first; k0 < k_end; k0 += kSlab, at ^= 1) {
+        cut_off_b(k0);
+        Operand bp[kFragB];
+#pragma unroll
+        for (int j = 0; j < kFragB; ++j) bp[j] = operand_of(rb[j][0], rb[j][1]);
+        fetch_b(k0 + kSlab);
+        __syncthreads();               // this slab is there, and nobody reads the one before it any more
+        cut_off(k0 + kSlab);
+#pragma unroll
+        for (int i = 0; i < kFragA; ++i) {
+            Operand ap;
+#pragma unroll
+            for (int p = 0; p < 3; ++p)
+                ap.part[p] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(&slabs[at][p][i * 16 + r][mine]));
+            f32x4 acc[kFragB] = {};
+#pragma unroll
+            for (int e = 0; e < kTerms; ++e)
+#pragma unroll
+                for (int j = 0; j < kFragB; ++j) acc[j] = add_term(e, ap, bp[j], acc[j]);
+#pragma unroll
+            for (int l = i * kLoadsA / kFragA; l < (i + 1) * kLoadsA / kFragA; ++l) keep(at ^ 1, l, -sign);
+#pragma unroll
+            for (int j = 0; j < kFragB; ++j) sum[i][j] = acc[j] * sign + sum[i][j];        // (one instruction, and exact)
+        }
+        fetch_a(k0 + 2 * kSlab);
+        sign = -sign;
+        if (k0 + kSlab >= k_end || k0 + kSlab == segment_first + segment) {
+            unsigned furthest = 0;                       // from the sums that are not in doubt; a sum of 0 is looked at below
+#pragma unroll
+            for (int i = 0; i < kFragA; ++i)
+#pragma unroll
+                for (int j = 0; j < kFragB; ++j)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) furthest = max(furthest, (__float_as_uint(sum[i][j][e]) & 0x7fffffffu) - kLeastBits);
+            if (__any(furthest > kMostBits - kLeastBits)) {
+                const int end = segment_first + segment < k_end ? segment_first + segment : k_end;
+#pragma unroll 1
+                for (int x = 0; x < kFragA * kFragB * 4; ++x) {
+                    const int i = x / (kFragB * 4), j = x / 4 % kFragB, e = x % 4;
+                    float v = 0.f;
+#pragma unroll
+                    for (int y = 0; y < kFragA * kFragB * 4; ++y) v = x == y ? sum[y / (kFragB * 4)][y / 4 % kFragB][y % 4] : v;
+                    if (in_doubt(v) && row_of(i, e) < m && col + j * 16 < n)
+                        v = plain_segment(a + static_cast<long>(row_of(i, e)) * k, b + static_cast<long>(col + j * 16) * k, segment_first, end);
+#pragma unroll
+                    for (int y = 0; y < kFragA * kFragB * 4; ++y) {
+                        float& to = reinterpret_cast<float*>(&sum[y / (kFragB * 4)][y / 4 % kFragB])[y % 4];
+                        to = x == y ? v : to;
+                    }
+                }
+            }
+            segment_first += segment;
+            if constexpr (kCut) {
+                store(sum, plane);
+                plane += static_cast<long>(m) * n;
+            }
+#pragma unroll
+            for (int i = 0; i < kFragA; ++i)
+#pragma unroll
+                for (int j = 0; j < kFragB; ++j) {
+                    if constexpr (!kCut) total[i][j] += sum[i][j];
+                    sum[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+                }
+        }
+    }
+    if constexpr (!kCut) store(total, c);
+}
+
+// ---- a short K -----------------------------------------------------------------------------------------------------
+// K below 256 is one chain of float products, k ascending, in tiles of kRows x 64 outputs whatever the rows: 32 x 32 x 2 instructions
+// on the floats themselves, a quarter of the tile a wave.  Slabs of K in shared memory, rows 4 floats further apart than they are long (16-byte reads of 8
+// neighbouring rows then touch every bank once).  Of every 8 elements the even ones lie first and then the odd ones: half-wave h
+// reads its four at once, and the four instructions take elements 0 and 1, 2 and 3, .. of them.
+constexpr int kChainCols = 64;
+constexpr int chain_slab_of(int rows) { return rows == 128 ? 32 : 64; }
+
+template <int kRows, bool kVec>
+__global__ void __launch_bounds__(256, 2)
+gemm_f32_chain_kernel(const float* __restrict__ a, const float* __restrict__ b, float* __restrict__ c, int m, int n, int k) {
+    constexpr int kLong = chain_slab_of(kRows);
+    constexpr int kFrag = kRows / 64;                  // 32 x 32 squares of a wave, one under the other
+    constexpr int kLoadsA = kRows * kLong / 4 / 256, kLoadsB = kChainCols * kLong / 4 / 256;    // 16-byte loads a thread and slab
+    __shared__ float as[2][kRows][kLong + 4];
+    __shared__ float bs[2][kChainCols][kLong + 4];
+    const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+    const int m0 = blockIdx.y * kRows, n0 = blockIdx.x * kChainCols;
+    const int wm = (wave / 2) * (kRows / 2), wn = (wave % 2) * (kChainCols / 2);
+    f32x16 acc[kFrag] = {};
     f32x4 ra[kLoadsA], rb[kLoadsB];
     const auto fetch = [&](int k0) {
 #pragma unroll
         for (int i = 0; i < kLoadsA; ++i) {
-            const int idx = threadIdx.x + i * 256, row = m0 + idx / (kSlab / 4), at = k0 + (idx % (kSlab / 4)) * 4;
-            ra[i] = load_four<kVec>(a + static_cast<long>(row < m ? row : m - 1) * k, at, k_end);
+            const int idx = threadIdx.x + i * 256, row = m0 + idx / (kLong / 4), at = k0 + (idx % (kLong / 4)) * 4;
+            ra[i] = load_four<kVec>(a + static_cast<long>(row < m ? row : m - 1) * k, at, k);
         }
 #pragma unroll
         for (int i = 0; i < kLoadsB; ++i) {
-            const int idx = threadIdx.x + i * 256, row = n0 + idx / (kSlab / 4), at = k0 + (idx % (kSlab / 4)) * 4;
-            rb[i] = load_four<kVec>(b + static_cast<long>(row < n ? row : n - 1) * k, at, k_end);
+            const int idx = threadIdx.x + i * 256, row = n0 + idx / (kLong / 4), at = k0 + (idx % (kLong / 4)) * 4;
+            rb[i] = load_four<kVec>(b + static_cast<long>(row < n ? row : n - 1) * k, at, k);
         }
     };
     const auto put = [&](float* row, int at, const f32x4& v) {
@@ -206,35 +431,24 @@ gemm_f32_tile_kernel(const float* __restrict__ a, const float* __restrict__ b, f
 #pragma unroll
         for (int i = 0; i < kLoadsA; ++i) {
             const int idx = threadIdx.x + i * 256;
-            put(as[into][idx / (kSlab / 4)], (idx % (kSlab / 4)) * 4, ra[i]);
+            put(as[into][idx / (kLong / 4)], (idx % (kLong / 4)) * 4, ra[i]);
         }
 #pragma unroll
         for (int i = 0; i < kLoadsB; ++i) {
             const int idx = threadIdx.x + i * 256;
-            put(bs[into][idx / (kSlab / 4)], (idx % (kSlab / 4)) * 4, rb[i]);
+            put(bs[into][idx / (kLong / 4)], (idx % (kLong / 4)) * 4, rb[i]);
         }
     };
-    const auto store = [&](const f32x16 (&of)[kFrag], float* to) {
-        const int col = n0 + wn + lane % 32;
-#pragma unroll
-        for (int i = 0; i < kFrag; ++i)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                const int row = m0 + wm + i * 32 + 8 * (e / 4) + 4 * (lane / 32) + e % 4;
-                if (row < m && col < n) to[static_cast<long>(row) * n + col] = of[i][e];
-            }
-    };
-    fetch(k_first);
+    fetch(0);
     keep(0);
-    int at = 0, segment_left = segment;                // segments are whole slabs
-    float* plane = c + static_cast<long>(blockIdx.z) * each * m * n;
-    for (int k0 = k_first; k0 < k_end; k0 += kSlab, at ^= 1) {
-        const bool more = k0 + kSlab < k_end;
-        if (more) fetch(k0 + kSlab);
+    int at = 0;
+    for (int k0 = 0; k0 < k; k0 += kLong, at ^= 1) {
+        const bool more = k0 + kLong < k;
+        if (more) fetch(k0 + kLong);
         __syncthreads();
         const int row = lane % 32, h = (lane / 32) * 4;
 #pragma unroll
-        for (int s = 0; s < kSlab; s += 8) {
+        for (int s = 0; s < kLong; s += 8) {
             f32x4 av[kFrag];
             const f32x4 bv = *reinterpret_cast<const f32x4*>(&bs[at][wn + row][s + h]);
 #pragma unroll
@@ -243,30 +457,17 @@ gemm_f32_tile_kernel(const float* __restrict__ a, const float* __restrict__ b, f
             for (int e = 0; e < 4; ++e)
 #pragma unroll
                 for (int i = 0; i < kFrag; ++i) acc[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[i][e], bv[e], acc[i], 0, 0, 0);
-            if (kChains && (s + 8) % kChain == 0) {
-#pragma unroll
-                for (int i = 0; i < kFrag; ++i) {
-                    sum[i] += acc[i];
-                    acc[i] = f32x16{};
-                }
-            }
         }
         if (more) keep(at ^ 1);        // read last two slabs ago, and every wave has passed a barrier since
-        segment_left -= kSlab;
-        if (segment_left == 0 || !more) {
-            segment_left = segment;
-            if constexpr (kCut) {
-                store(sum, plane);
-                plane += static_cast<long>(m) * n;
-            }
-#pragma unroll
-            for (int i = 0; i < kFrag; ++i) {
-                if constexpr (!kCut) total[i] += kChains ? sum[i] : acc[i];
-                sum[i] = f32x16{};
-            }
-        }
     }
-    if constexpr (!kCut) store(total, c);
+    const int col = n0 + wn + lane % 32;
+#pragma unroll
+    for (int i = 0; i < kFrag; ++i)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            const int row = m0 + wm + i * 32 + 8 * (e / 4) + 4 * (lane / 32) + e % 4;
+            if (row < m && col < n) c[static_cast<long>(row) * n + col] = acc[i][e];
+        }
 }
 
 // C = the planes' sum, in order.  kVec: planes and c are aligned to 16 bytes and `count` is a multiple of 4.
@@ -287,54 +488,133 @@ __global__ void __launch_bounds__(256) gemm_f32_sum_kernel(const float* __restri
     }
 }
 
-// Up to here a product is a stream of weights.  Measured against 2048 x 2048 and 12288 x 2048 weights (us, streamed : tiled): 14.1 :
-// 14.3 and 40 : 43 at 24 rows, 15 : 14.5 and 43 : 44 at 32; beyond, the stream's reads of A, then four times the weights', cost more.
+// Up to here a product is a stream of weights.  Measured (us, streamed : tiled) against 2048 x 2048 weights 11.4 : 12.1 at 17 rows,
+// 13.7 : 12.5 at 32, 3072 x 512 5.9 : 9.7 at 32, 6144 x 1024 13.9 : 14.4; beyond, the stream's reads of A, then four times the
+// weights', cost more.  A long K leaves the tiles' workgroups enough to do from the second tile of rows on: 1024 x 3072 15.1 : 14.6
+// and 18.9 : 15.0 at 17 and 32 rows, 2048 x 6144 27.9 : 26.4 and 35.5 : 26.8.
 constexpr int kStreamRows = 32;
-constexpr int kStreamK = 256;          // a shorter K is no work to share out over four waves: one segment, in tiles whatever the rows
+constexpr int kStreamLongK = 3072;
+constexpr int kStreamK = 256;          // a shorter K is no work to share out over four waves: one chain, in tiles whatever the rows
 
 // The segments of K: by K alone.  Eight from 512 elements on (a wave each of a streaming workgroup), four from 256, multiples
-// of 64 elements (a streaming wave's run, and whole slabs of a tile).
+// of 64 elements (whole slabs of a tile).
 struct F32Segments {
     int length, count;
 };
 F32Segments f32_segments(int k) {
     const int wanted = k < kStreamK ? 1 : k < 2 * kStreamK ? 4 : 8;
-    const int length = ceil_div(ceil_div(k, wanted), kStreamRun) * kStreamRun;
+    const int length = ceil_div(ceil_div(k, wanted), 64) * 64;
     return {length, ceil_div(k, length)};
 }
 
 struct F32Plan {
-    int rows = 0, parts = 1, each = 1;                 // rows of a tile, 0: the streaming kernel; parts workgroups of `each` segments along K
+    int rows = 0, cols = 0, parts = 1, each = 1;       // of a tile, no rows: the streaming kernel; parts workgroups of `each` segments along K
 };
 
-// The tile and the cut of K that take least time.  A compute unit's matrix instructions run at one rate however many tiles it
-// holds, so the product takes as long as the fullest of the 256 units has work for; one tile a unit leaves a wave a SIMD and
-// its waits in the open.  A cut K costs a plane written and read for every segment (mostly in the caches) and a second launch.
-// Constants fitted to every tile and cut timed at 33 to 1,024 rows against 512 x 512 to 32768 x 2048 and 2048 x 6144 weights: the
-// choice is within 6 % of the best at each.
-F32Plan f32_plan(int m, int n, int k) {
+// A short K: the tile that takes least time.  A compute unit's float instructions run at one rate however many tiles it holds, so the
+// product takes as long as the fullest of the 256 units has work for; one tile a unit leaves a wave a SIMD and its waits in the open.
+F32Plan f32_chain_plan(int m, int n) {
     F32Plan best;
-    const F32Segments segments = f32_segments(k);
-    best.each = segments.count;
-    if (m <= kStreamRows && k >= kStreamK) return best;
-    constexpr long kUnits = 256;
-    constexpr double kUnitRate = 0.6e6, kPlaneRate = 30e6, kLaunch = 6.0;      // operations and bytes a microsecond; microseconds
     double least = 0.0;
     for (int rows : {128, 64}) {
-        const long tiles = static_cast<long>(ceil_div(m, rows)) * ceil_div(n, kTileCols);
+        const long held = (static_cast<long>(ceil_div(m, rows)) * ceil_div(n, kChainCols) + 255) / 256;
+        const double time = held * rows / (rows == 128 ? (held >= 2 ? 0.87 : 0.4) : (held >= 2 ? 0.82 : 0.65));
+        if (best.rows == 0 || time < least * 0.999) {
+            least = time;
+            best.rows = rows, best.cols = kChainCols;
+        }
+    }
+    return best;
+}
+
+// The tile's width and the cut of K that take least time.  Up to four workgroups of a unit work side by side: a slab takes them the longer
+// of a workgroup's own way through it and of what they ask of the unit together.  A cut K costs a plane written and read for every
+// segment (mostly in the caches) and a second launch.  Constants (microseconds; bytes a microsecond) fitted to both tiles and every cut
+// timed at 17 to 2,048 rows against the matrices of layers of 512, 1,024 and 2,048 channels: the choice is 0.4 % off the best on
+// average and 10 % at worst.
+F32Plan f32_plan(int m, int n, int k) {
+    F32Plan best;
+    if (k < kStreamK) return f32_chain_plan(m, n);
+    const F32Segments segments = f32_segments(k);
+    best.each = segments.count;
+    if (m <= (k < kStreamLongK ? kStreamRows : kStreamTile)) return best;
+    constexpr long kUnits = 256, kBeside = 4;
+    constexpr double kPlaneRate = 8.5e6, kLaunch = 4.4;
+    double least = 0.0;
+    for (int cols : {128, 64}) {
+        const double own = cols == 128 ? 1.06 : 0.66, shared = cols == 128 ? 0.76 : 0.47;
+        const long tiles = static_cast<long>(ceil_div(m, kTileRows)) * ceil_div(n, cols);
         for (int wanted = 1; wanted <= segments.count; wanted *= 2) {
             const int each = ceil_div(segments.count, wanted), parts = ceil_div(segments.count, each);
             const long held = (tiles * parts + kUnits - 1) / kUnits;           // of the fullest unit
-            const double hidden = rows == 128 ? (held >= 2 ? 0.87 : 0.4) : (held >= 2 ? 0.82 : 0.65);
-            const double product = 2.0 * held * rows * kTileCols * segments.length * each / (kUnitRate * hidden);
+            const double slabs = static_cast<double>(segments.length) * each / kSlab;
+            const auto side_by_side = [&](long workgroups) { return workgroups * shared > own ? workgroups * shared : own; };
+            const double product = slabs * ((held / kBeside) * side_by_side(kBeside) + (held % kBeside ? side_by_side(held % kBeside) : 0.0));
             const double planes = parts == 1 ? 0.0 : kLaunch + 8.0 * segments.count * m * n / kPlaneRate;
             if (best.rows == 0 || product + planes < least * 0.999) {
                 least = product + planes;
-                best.rows = rows, best.parts = parts, best.each = each;
+                best.rows = kTileRows, best.cols = cols, best.parts = parts, best.each = each;
             }
         }
     }
     return best;
+}
+
+int launch_f32(const F32Plan& p, const float* a, const float* b, float* c, float* planes, int m, int n, int k, hipStream_t stream) {
+    const F32Segments segments = f32_segments(k);
+    LEONE_REQUIRE(p.parts == 1 || planes, "gemm_f32: %d planes are needed for %d x %d x %d", segments.count, m, n, k);
+    const auto aligned = [](const void* at) { return reinterpret_cast<uintptr_t>(at) % 16 == 0; };
+    const bool vec = k % 4 == 0 && aligned(a) && aligned(b);
+    if (p.rows == 0) {
+        const int blocks = ceil_div(n, kStreamTile);
+#define LEONE_STREAM(T, W, D, E)                                                                                                       \
+    (vec ? gemm_f32_stream_kernel<T, W, D, E, true><<<blocks, W * kWave, 0, stream>>>(a, b, c, m, n, k, segments.length)               \
+         : gemm_f32_stream_kernel<T, W, D, E, false><<<blocks, W * kWave, 0, stream>>>(a, b, c, m, n, k, segments.length))
+        // Runs on their way a wave: two leave room for more waves, whose loads count as well, and segments of few runs have no use for
+        // more; of a large matrix four (us, two and four runs: one row against 12288 x 2048 21.2 and 19.0, 32768 x 2048 48.1 and 44.0,
+        // 2048 x 6144 17.7 and 17.2; but 2048 x 2048 7.1 and 7.4, 1024 x 3072 10.9 and 11.5, five rows against 32768 x 512 16.4 and
+        // 18.7).  Two tiles of A fill the registers: 24 rows against 12288 x 2048 32.5 with two, 37.0 with three.
+        const bool large = segments.length >= 256 && static_cast<long>(n) * k >= 8l << 20;
+        if (segments.count <= 4) {
+            if (m <= kStreamTile) LEONE_STREAM(1, 4, 2, 4);
+            else LEONE_STREAM(2, 4, 2, 2);
+        } else if (m > kStreamTile) {
+            LEONE_STREAM(2, 8, 2, 2);
+        } else if (large) {
+            LEONE_STREAM(1, 8, 4, 4);
+        } else {
+            LEONE_STREAM(1, 8, 2, 4);
+        }
+#undef LEONE_STREAM
+        LEONE_LAUNCH_CHECK("gemm_f32");
+        return 0;
+    }
+    const int grid_y = ceil_div(m, p.rows);
+    LEONE_REQUIRE(grid_y <= 65535, "gemm_f32: %d rows exceed the launch limit", m);
+    const dim3 grid(ceil_div(n, p.cols), grid_y, p.parts);
+#define LEONE_CHAIN(R)                                                                                                                 \
+    (vec ? gemm_f32_chain_kernel<R, true><<<grid, 256, 0, stream>>>(a, b, c, m, n, k)                                                  \
+         : gemm_f32_chain_kernel<R, false><<<grid, 256, 0, stream>>>(a, b, c, m, n, k))
+#define LEONE_TILE_CUT(C, V)                                                                                                           \
+    (p.parts > 1 ? gemm_f32_tile_kernel<C, V, true><<<grid, 256, 0, stream>>>(a, b, planes, m, n, k, segments.length, p.each)          \
+                 : gemm_f32_tile_kernel<C, V, false><<<grid, 256, 0, stream>>>(a, b, c, m, n, k, segments.length, p.each))
+#define LEONE_TILE(C) (vec ? LEONE_TILE_CUT(C, true) : LEONE_TILE_CUT(C, false))
+    if (k < kStreamK) p.rows == 128 ? LEONE_CHAIN(128) : LEONE_CHAIN(64);
+    else p.cols == 128 ? LEONE_TILE(128) : LEONE_TILE(64);
+#undef LEONE_CHAIN
+#undef LEONE_TILE
+#undef LEONE_TILE_CUT
+    LEONE_LAUNCH_CHECK("gemm_f32");
+    if (p.parts > 1) {
+        const long count = static_cast<long>(m) * n;
+        const int blocks = ceil_div(count, 1024);
+        if (count % 4 == 0 && aligned(planes) && aligned(c))
+            gemm_f32_sum_kernel<true><<<blocks, 256, 0, stream>>>(planes, c, count, segments.count);
+        else
+            gemm_f32_sum_kernel<false><<<blocks, 256, 0, stream>>>(planes, c, count, segments.count);
+        LEONE_LAUNCH_CHECK("gemm_f32 sum");
+    }
+    return 0;
 }
 
 }  // namespace leone
@@ -352,56 +632,5 @@ extern "C" int leone_gemm_f32_planes(int m, int n, int k) {
 extern "C" int leone_gemm_f32(const float* a, const float* b, float* c, float* planes, int m, int n, int k, hipStream_t stream) {
     LEONE_REQUIRE(a && b && c, "gemm_f32: null pointer");
     LEONE_REQUIRE(m > 0 && n > 0 && k > 0, "gemm_f32: sizes %d x %d x %d must be positive", m, n, k);
-    const F32Plan p = f32_plan(m, n, k);
-    const F32Segments segments = f32_segments(k);
-    LEONE_REQUIRE(p.parts == 1 || planes, "gemm_f32: %d planes are needed for %d x %d x %d", segments.count, m, n, k);
-    const auto aligned = [](const void* at) { return reinterpret_cast<uintptr_t>(at) % 16 == 0; };
-    const bool vec = k % 4 == 0 && aligned(a) && aligned(b);
-    if (p.rows == 0) {
-        const int blocks = ceil_div(n, kStreamTile);
-#define LEONE_STREAM(T, W, D)                                                                                                          \
-    (vec ? gemm_f32_stream_kernel<T, W, D, true><<<blocks, W * kWave, 0, stream>>>(a, b, c, m, n, k, segments.length)                  \
-         : gemm_f32_stream_kernel<T, W, D, false><<<blocks, W * kWave, 0, stream>>>(a, b, c, m, n, k, segments.length))
-        // Runs on their way a wave: two leave room for more waves, whose loads count as well (one row against 12288 x 2048 18.4 us,
-        // with four 24.4); two tiles of A take long enough over a run for three (24 rows against 2048 x 6144 37.8, with four 43.1).
-        if (segments.count <= 4) {
-            if (m <= kStreamTile) LEONE_STREAM(1, 4, 2);
-            else LEONE_STREAM(2, 4, 3);
-        } else {
-            if (m <= kStreamTile) LEONE_STREAM(1, 8, 2);
-            else LEONE_STREAM(2, 8, 3);
-        }
-#undef LEONE_STREAM
-        LEONE_LAUNCH_CHECK("gemm_f32");
-        return 0;
-    }
-    const int grid_y = ceil_div(m, p.rows);
-    LEONE_REQUIRE(grid_y <= 65535, "gemm_f32: %d rows exceed the launch limit", m);
-    const dim3 grid(ceil_div(n, kTileCols), grid_y, p.parts);
-#define LEONE_TILE_CHAIN(E, V, CHAIN)                                                                                                  \
-    (p.parts > 1 ? gemm_f32_tile_kernel<E, V, true, CHAIN><<<grid, 256, 0, stream>>>(a, b, planes, m, n, k, segments.length, p.each)   \
-                 : gemm_f32_tile_kernel<E, V, false, CHAIN><<<grid, 256, 0, stream>>>(a, b, c, m, n, k, segments.length, p.each))
-#define LEONE_TILE(E, V)                                                                                                               \
-    (segments.count > 1 ? LEONE_TILE_CHAIN(E, V, true)                                                                               \
-                        : gemm_f32_tile_kernel<E, V, false, false><<<grid, 256, 0, stream>>>(a, b, c, m, n, k, segments.length, p.each))
-    if (p.rows == 128) {
-        if (vec) LEONE_TILE(128, true);
-        else LEONE_TILE(128, false);
-    } else {
-        if (vec) LEONE_TILE(64, true);
-        else LEONE_TILE(64, false);
-    }
-#undef LEONE_TILE_CHAIN
-#undef LEONE_TILE
-    LEONE_LAUNCH_CHECK("gemm_f32");
-    if (p.parts > 1) {
-        const long count = static_cast<long>(m) * n;
-        const int blocks = ceil_div(count, 1024);
-        if (count % 4 == 0 && aligned(planes) && aligned(c))
-            gemm_f32_sum_kernel<true><<<blocks, 256, 0, stream>>>(planes, c, count, segments.count);
-        else
-            gemm_f32_sum_kernel<false><<<blocks, 256, 0, stream>>>(planes, c, count, segments.count);
-        LEONE_LAUNCH_CHECK("gemm_f32 sum");
-    }
-    return 0;
+    return launch_f32(f32_plan(m, n, k), a, b, c, planes, m, n, k, stream);
 }

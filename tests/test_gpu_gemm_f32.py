@@ -78,3 +78,32 @@ def test_results_off_sixteen_bytes():
         ops.gemm_f32(a, b, out=room[shift:shift + m * n].view(m, n))
         assert torch.equal(room[shift:shift + m * n].view(m, n), want)
         assert bool((room[:shift] == 7.0).all()) and bool((room[shift + m * n:] == 7.0).all())
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 17, 257), (16, 129, 511), (33, 128, 513), (65, 130, 609), (200, 127, 1100), (70, 300, 2048)])
+@pytest.mark.parametrize("scale", [1e-37, 1e-30, 1e-12, 1.0, 1e12])
+def test_numbers_of_every_size(m, n, k, scale):
+    """Numbers in three parts: none of their 24 bits is lost, whatever the numbers' size and wherever the row ends."""
+    from leone_amd import ops
+    gen = torch.Generator(device=DEV).manual_seed(n)
+    a, b = torch.randn(m, k, generator=gen, device=DEV) * scale, torch.randn(n, k, generator=gen, device=DEV)
+    want = a.double() @ b.double().T
+    error = float((ops.gemm_f32(a, b).double() - want).norm() / want.norm())
+    # a product that loses more than a float's last bit is off by 2^-24 of itself, at random; sums round as sums of floats do
+    assert error < 2.0 ** -24 * (1.0 + math.sqrt(math.log2(k))), error
+
+
+def test_numbers_that_are_no_sums_of_parts():
+    """The largest numbers round to infinity in 16 bits and an infinity has nothing left over: plain sums all the same."""
+    from leone_amd import ops
+    for m, n, k in ((3, 20, 300), (40, 140, 600), (300, 70, 512)):
+        a, b = torch.zeros(m, k, device=DEV), torch.randn(n, k, device=DEV)
+        a[0, 5], a[1, k - 1], a[2, 7] = 3.4e38, -3.4028234e38, math.inf
+        b[:, 5] = b[:, k - 1] = 0.25
+        b[:, 7] = 1.0 + 2.0 ** -20
+        b[3, 7] = 0.0
+        got = ops.gemm_f32(a, b)
+        assert torch.equal(got[0], torch.full_like(got[0], 3.4e38) * 0.25)
+        assert torch.equal(got[1], torch.full_like(got[1], -3.4028234e38) * 0.25)
+        keep = [j for j in range(n) if j != 3]
+        assert bool((got[2, keep] == math.inf).all()) and bool(torch.isnan(got[2, 3])) and not bool(got[3:].any())
