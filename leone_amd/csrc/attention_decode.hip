@@ -88,19 +88,11 @@ struct FromProjection {
     bf16_t* v_out;
 };
 
-// Eight elements of the projection from element offset `at` of row `row`: planes added in order, then rounded
-// to bfloat16 as a stored projection would be.
-__device__ inline void load_projection8(const FromProjection& f, long row_width, long row, long at, float out[8]) {
-    if (!f.is_float) {
-        const uint4 raw = *reinterpret_cast<const uint4*>(static_cast<const bf16_t*>(f.qkv) + row * row_width + at);
-        const unsigned w[4] = {raw.x, raw.y, raw.z, raw.w};
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            out[2 * i] = __uint_as_float(w[i] << 16);
-            out[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
-        }
-        return;
-    }
+// Eight elements of the projection from element offset `at` of row `row`, as they stand in a bfloat16 projection; planes are added in
+// order, then rounded to bfloat16 as a stored projection would be.
+__device__ inline uint4 load_projection8(const FromProjection& f, long row_width, long row, long at) {
+    if (!f.is_float) return *reinterpret_cast<const uint4*>(static_cast<const bf16_t*>(f.qkv) + row * row_width + at);
+    float out[8];
     // The planes are asked for four at a time before any is added (a plane beyond the last is the last one again
     // and is not added): one trip to memory for up to five planes instead of one a plane.  Added in their order.
     const float* src = static_cast<const float*>(f.qkv) + row * row_width + at;
@@ -122,9 +114,45 @@ __device__ inline void load_projection8(const FromProjection& f, long row_width,
                 out[4] += hi[q].x; out[5] += hi[q].y; out[6] += hi[q].z; out[7] += hi[q].w;
             }
     }
+    bf16x8 rounded;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) out[i] = to_float(from_float<bf16_t>(out[i]));
+    for (int i = 0; i < 8; ++i) rounded[i] = static_cast<__bf16>(out[i]);
+    return __builtin_bit_cast(uint4, rounded);
 }
+__device__ inline void unpack8(const uint4& raw, float out[8]) {
+    const unsigned w[4] = {raw.x, raw.y, raw.z, raw.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        out[2 * i] = __uint_as_float(w[i] << 16);
+        out[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
+    }
+}
+// Eight gains as they were loaded (bfloat16 in the first sixteen bytes), unpacked where they are used.
+struct EightGains {
+    uint4 low, high;
+    __device__ void load(const AnyVec& v, int at) {
+        if (v.dtype == kF32) {
+            const uint4* from = reinterpret_cast<const uint4*>(static_cast<const float*>(v.ptr) + at);
+            low = from[0], high = from[1];
+        } else {
+            low = *reinterpret_cast<const uint4*>(static_cast<const bf16_t*>(v.ptr) + at);
+        }
+    }
+    __device__ void get(int dtype, float out[8]) const {
+        if (dtype == kF32) {
+            const unsigned w[8] = {low.x, low.y, low.z, low.w, high.x, high.y, high.z, high.w};
+#pragma unroll
+            for (int i = 0; i < 8; ++i) out[i] = __uint_as_float(w[i]);
+        } else {
+            unpack8(low, out);
+        }
+    }
+};
+// How a launch's heads and splits are laid out: what the kernel would divide for.
+struct DecodeShape {
+    int group, col_tiles;                // query heads a kv head; workgroups that share them
+    unsigned splits_inverse;             // 2^32 / splits, rounded up (0: one split)
+};
 
 // kD16 = head_dim / 16.
 // Two tiles of keys and values are held at a time (one on its way, one being worked on): up to a head size of
@@ -183,19 +211,19 @@ attention_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__
                         const int* __restrict__ row_entry, const int* __restrict__ block_table, int max_blocks,
                         float* __restrict__ part_acc, float* __restrict__ part_ml, bf16_t* __restrict__ out,
                         int q_heads, int kv_heads, int page_shift, float to_log2, int window, int splits,
-                        FromProjection from, int keep_first, ScoreBias bias, ScoreShape shape, int chunk, int ordered) {
+                        FromProjection from, int keep_first, ScoreBias bias, ScoreShape shape, int chunk, int ordered,
+                        DecodeShape heads) {
     constexpr int kD = kD16 * 16;
     constexpr int kSteps = (kD16 + 1) / 2;           // 32-element steps of the q.k product
     extern __shared__ float smem[];                   // [waves][columns][kD] accumulators, then m and l
 
-    const int group = q_heads / kv_heads;
-    const int col_tiles = (group + 15) / 16;
-    const int wave = threadIdx.x / kWave;
+    const int group = heads.group;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);      // (the same for the whole wave: scalar registers)
     const int lane = threadIdx.x % kWave;
     int row = blockIdx.x, head_block = blockIdx.y;
     if (ordered) row = ordered_row(positions, gridDim.x, gridDim.y, lane, head_block);
-    const int kvh = head_block / col_tiles;
-    const int col0 = (head_block % col_tiles) * 16;
+    const int kvh = heads.col_tiles == 1 ? head_block : head_block / heads.col_tiles;
+    const int col0 = (head_block - kvh * heads.col_tiles) * 16;
     const int cols = group - col0 < 16 ? group - col0 : 16;   // query heads handled here
     const int split = blockIdx.z;
     const int c = lane & 15, g = lane >> 4;
@@ -205,7 +233,8 @@ attention_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__
     // What the heads' norms and rotation start from is asked for before anything else is known: the first wave takes the
     // query heads, the second the new key, the third the new value (`FromProjection`).
     [[maybe_unused]] constexpr int kHalfSteps = kSteps / 2;
-    [[maybe_unused]] float head_run[kFused ? kSteps : 1][8], head_gain[kFused ? kSteps : 1][8];
+    [[maybe_unused]] uint4 head_raw[kFused ? kSteps : 1];
+    [[maybe_unused]] EightGains head_gain[kFused ? kSteps : 1];
     [[maybe_unused]] const bool head_ok = c < cols;
     if constexpr (kFused) {
         // Lane (c, g) of the first wave holds elements 32s + 8g .. + 7 of query head c for every step s; with a head size
@@ -218,12 +247,12 @@ attention_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__
             const AnyVec gain = wave == 0 ? from.q_gain : from.k_gain;
 #pragma unroll
             for (int s = 0; s < kSteps; ++s) {
-                if (gain.ptr) load_any8(gain, 32 * s + 8 * g, head_gain[s]);
-                load_projection8(from, width, row, head_at + 32 * s + 8 * g, head_run[s]);
+                if (gain.ptr) head_gain[s].load(gain, 32 * s + 8 * g);
+                head_raw[s] = load_projection8(from, width, row, head_at + 32 * s + 8 * g);
             }
         } else if (wave == 2 && from.k_out != nullptr) {
             if (8 * lane < kD)      // values are copied as they are: lane l has elements 8 l .. 8 l + 7 (a head has at most 256)
-                load_projection8(from, width, row, static_cast<long>(q_heads + kv_heads + kvh) * kD + 8 * lane, head_run[0]);
+                head_raw[0] = load_projection8(from, width, row, static_cast<long>(q_heads + kv_heads + kvh) * kD + 8 * lane);
         }
     }
 
@@ -258,7 +287,7 @@ attention_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__
     const int n_tiles = kept_tiles + t_end - t_begin;
     auto tile_of = [&](int u) { return u < kept_tiles ? u : t_begin + (u - kept_tiles); };
     auto in_reach = [&](int key) { return key < n && (key >= lo || key < keep); };
-    const int per_split = (n_tiles + splits - 1) / splits;
+    const int per_split = heads.splits_inverse ? static_cast<int>(__umulhi(n_tiles + splits - 1, heads.splits_inverse)) : n_tiles;
     const int my_begin = split * per_split;                         // places in the row's list of tiles
     const int my_end = my_begin + per_split < n_tiles ? my_begin + per_split : n_tiles;
 
@@ -287,7 +316,6 @@ attention_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__
         const int b = key >> page_shift;
         return b >= first_page ? pages[b - first_page] : pages[n_win_pages + b - kept_first_page];
     };
-    __syncthreads();
 
     // One 32-key tile in two steps: `issue` asks for its keys and values, `finish` does the arithmetic.  The
     // next tile of the wave is asked for before the present one is finished, so that a wave always has loads
@@ -300,34 +328,52 @@ attention_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__
     // the last tile of a row are not.
     struct Tile {
         bf16x8 xa[kSteps], xb[kSteps], xv[kD16];
+        int page;                                        // where a tile's keys lie on one page: which, -1: none
     };
-    auto issue = [&](int u, bool exists, Tile& r) {
+    const int block_elements = page_tokens * kD;         // one page of one kv head
+    const int key_step = 4 * page_tokens * 8;            // 32 elements of a key further
+    const bool one_page = page_shift >= 5;               // a tile's keys lie on one page
+    // (The page ids are in shared memory once the waves have met; the first tile is asked for before.)
+    auto issue = [&](int u, bool exists, Tile& r, bool first_tile) {
         const int key0 = (exists ? tile_of(u) : 0) * kTileKeys;
-        // A-operand row c of half a is key 8*(c/4) + c%4, of half b four keys further
-        const int ka = key0 + 8 * (c >> 2) + (c & 3);
-        const int run0 = key0 + 8 * g;                   // this lane's eight keys for the second product
-        const bool near = exists && ka < n && (ka + 4 >= lo || ka < keep);   // ka or kb = ka + 4 in reach: they share a page (pages hold multiples of 8 keys)
-        const bool any = exists && run0 < n && (run0 + 8 > lo || run0 < keep);
-        const int page_k = near ? page_at(ka) : -1;
-        const int page_v = any ? page_at(run0) : -1;
-        const bf16_t* pk = page_k < 0 ? k_pool
-                                      : k_pool + (static_cast<long>(page_k) * kv_heads + kvh) * page_tokens * kD + (ka & page_mask) * 8;
-        const bf16_t* pv = page_v < 0 ? v_pool
-                                      : v_pool + (static_cast<long>(page_v) * kv_heads + kvh) * page_tokens * kD +
-                                            static_cast<long>((run0 & page_mask) >> 3) * kD * 8;
-#pragma unroll
-        for (int s = 0; s < kSteps; ++s) {
-            const bool in_head = 32 * s + 8 * g < kD;
-            const long run = in_head ? static_cast<long>(4 * s + g) * page_tokens * 8 : 0;   // elements 32s+8g .. +7 of the key
-            r.xa[s] = load8_streamed(pk + run);
-            r.xb[s] = load8_streamed(pk + run + 32);           // four keys further
+        const int ka_place = 8 * (c >> 2) + (c & 3);     // A-operand row c of half a is key 8*(c/4) + c%4, of half b four keys further
+        const bf16_t *pk, *pv;
+        if (one_page) {
+            // a tile of the list holds a key in reach, so its page counts; what else lies there may be read, and is masked in `finish`
+            int page = -1;
+            if (exists) page = first_tile ? table[key0 >> page_shift] : __builtin_amdgcn_readfirstlane(page_at(key0));
+            r.page = page;
+            const long block = (static_cast<long>(page < 0 ? 0 : page) * kv_heads + kvh) * block_elements;
+            const int token = page < 0 ? 0 : key0 & page_mask;
+            pk = k_pool + block + token * 8 + (g * page_tokens + ka_place) * 8;
+            pv = v_pool + block + token * kD + (g * kD + c) * 8;
+        } else {
+            const auto page_of = [&](int key) { return first_tile ? table[key >> page_shift] : page_at(key); };
+            const int ka = key0 + ka_place;
+            const int run0 = key0 + 8 * g;                   // this lane's eight keys for the second product
+            const bool near = exists && ka < n && (ka + 4 >= lo || ka < keep);   // ka or kb = ka + 4 in reach: they share a page (pages hold multiples of 8 keys)
+            const bool any = exists && run0 < n && (run0 + 8 > lo || run0 < keep);
+            const int page_k = near ? page_of(ka) : -1;
+            const int page_v = any ? page_of(run0) : -1;
+            pk = k_pool + g * page_tokens * 8;
+            if (page_k >= 0) pk += (static_cast<long>(page_k) * kv_heads + kvh) * block_elements + (ka & page_mask) * 8;
+            pv = v_pool + c * 8;
+            if (page_v >= 0) pv += (static_cast<long>(page_v) * kv_heads + kvh) * block_elements + ((run0 & page_mask) >> 3) * kD * 8;
         }
 #pragma unroll
-        for (int dt = 0; dt < kD16; ++dt) r.xv[dt] = load8_streamed(pv + (16 * dt + c) * 8);
+        for (int s = 0; s < kSteps; ++s) {
+            const bf16_t* at = pk + static_cast<long>(s) * key_step;   // elements 32s+8g .. +7 of the key
+            if (32 * s + 32 > kD && g >= 2) at = k_pool;               // (not in the head: the last step of an odd kD16)
+            r.xa[s] = load8_streamed(at);
+            r.xb[s] = load8_streamed(at + 32);                         // four keys further
+        }
+#pragma unroll
+        for (int dt = 0; dt < kD16; ++dt) r.xv[dt] = load8_streamed(pv + 16 * dt * 8);
     };
     // The wave's first tile is asked for before the queries are made: neither waits for the other.
     Tile one, two;
-    if (my_begin + wave < my_end) issue(my_begin + wave, true, one);
+    if (my_begin + wave < my_end) issue(my_begin + wave, true, one, true);
+    if constexpr (!kFused) __syncthreads();            // the page ids are there (else where the queries are)
 
     // Q^T operand: column c is query head kvh*group + col0 + c.
     bf16x8 qreg[kSteps];
@@ -348,6 +394,9 @@ attention_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__
         const int token = pos & page_mask;
         if (wave == 0 || (wave == 1 && writes)) {
             const AnyVec gain = wave == 0 ? from.q_gain : from.k_gain;
+            float head_run[kSteps][8];
+#pragma unroll
+            for (int s = 0; s < kSteps; ++s) unpack8(head_raw[s], head_run[s]);
             float ss = 0.f;
             if (wave == 0) {
 #pragma unroll
@@ -375,9 +424,12 @@ attention_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__
             if (gain.ptr) {
                 const float inv = 1.0f / sqrtf(ss / static_cast<float>(kD) + from.eps);
 #pragma unroll
-                for (int s = 0; s < kSteps; ++s)
+                for (int s = 0; s < kSteps; ++s) {
+                    float gains[8];
+                    head_gain[s].get(gain.dtype, gains);
 #pragma unroll
-                    for (int i = 0; i < 8; ++i) head_run[s][i] = (head_run[s][i] * head_gain[s][i]) * inv;
+                    for (int i = 0; i < 8; ++i) head_run[s][i] = (head_run[s][i] * gains[i]) * inv;
+                }
             }
             if (from.cos_table != nullptr) {
 #pragma unroll
@@ -403,11 +455,12 @@ attention_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__
                 }
             }
         } else if (wave == 2 && writes && 8 * lane < kD) {
+            const unsigned w[4] = {head_raw[0].x, head_raw[0].y, head_raw[0].z, head_raw[0].w};
+            *reinterpret_cast<uint4*>(new_value + 8 * lane) = head_raw[0];
+            if (page >= 0) {
+                bf16_t* to = from.v_out + base + value_offset(token, 8 * lane, kD);
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const bf16_t value = from_float<bf16_t>(head_run[0][i]);
-                new_value[8 * lane + i] = value;
-                if (page >= 0) from.v_out[base + value_offset(token, 8 * lane + i, kD)] = value;
+                for (int i = 0; i < 8; ++i) to[8 * i] = bf16_t{static_cast<uint16_t>(i % 2 ? w[i / 2] >> 16 : w[i / 2] & 0xffffu)};
             }
         }
         __syncthreads();
@@ -436,11 +489,11 @@ attention_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__
         const int kb = ka + 4;
         const int run0 = key0 + 8 * g;
         bool va = in_reach(ka), vb = in_reach(kb), any = run0 < n && (run0 + 8 > lo || run0 < keep);
-        if ((va || vb) && page_at(ka) < 0) {
+        if ((va || vb) && (one_page ? r.page : page_at(ka)) < 0) {
             unmapped = true;                              // never read outside the pool; the result is poisoned below
             va = vb = false;
         }
-        if (any && page_at(run0) < 0) {
+        if (any && (one_page ? r.page : page_at(run0)) < 0) {
             unmapped = true;
             any = false;
         }
@@ -504,12 +557,24 @@ attention_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__
         float tile_max = -INFINITY;
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-            const int key = run0 + j;
-            float raw = j < 4 ? sa[j & 3] : sb[j & 3];
-            if (kShaped && shape.cap > 0.f) raw = cap_log2 * tanh_fast(raw * to_cap);
-            sc[j] = (full || in_reach(key)) ? fmaf(raw, kShaped && shape.cap > 0.f ? 1.0f : to_log2_row, slope_log2 * static_cast<float>(key - (n - 1))) : -INFINITY;
-            tile_max = fmaxf(tile_max, sc[j]);
+            sc[j] = j < 4 ? sa[j & 3] : sb[j & 3];
+            if (kShaped && shape.cap > 0.f) sc[j] = cap_log2 * tanh_fast(sc[j] * to_cap);
+            else sc[j] *= to_log2_row;
         }
+        if (bias.slopes) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const float raw = j < 4 ? sa[j & 3] : sb[j & 3], lowered = slope_log2 * static_cast<float>(run0 + j - (n - 1));
+                sc[j] = kShaped && shape.cap > 0.f ? sc[j] + lowered : fmaf(raw, to_log2_row, lowered);
+            }
+        }
+        if (!full) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                if (!in_reach(run0 + j)) sc[j] = -INFINITY;
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) tile_max = fmaxf(tile_max, sc[j]);
         tile_max = max_lanes<16>(tile_max);
         tile_max = max_lanes<32>(tile_max);
         const float m_new = fmaxf(m_run, ceilf(tile_max));   // finite: every tile of the range holds a key in reach
@@ -538,7 +603,7 @@ attention_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__
     // for a tile that does not exist (see `issue`).
     if constexpr (kD16 > 8) {                           // two tiles of such heads do not fit the registers
         for (int t = my_begin + wave; t < my_end; t += kDecodeWaves) {
-            if (t != my_begin + wave) issue(t, true, one);
+            if (t != my_begin + wave) issue(t, true, one, false);
             finish(t, one);
         }
     } else {
@@ -546,11 +611,11 @@ attention_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__
         if (t < my_end) {
             while (true) {
                 const int t1 = t + kDecodeWaves;
-                issue(t1, t1 < my_end, two);
+                issue(t1, t1 < my_end, two, false);
                 finish(t, one);
                 if (t1 >= my_end) break;
                 const int t2 = t1 + kDecodeWaves;
-                issue(t2, t2 < my_end, one);
+                issue(t2, t2 < my_end, one, false);
                 finish(t1, two);
                 if (t2 >= my_end) break;
                 t = t2;
@@ -570,8 +635,7 @@ attention_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__
     if (c < cols) {
 #pragma unroll
         for (int dt = 0; dt < kD16; ++dt)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) sm_acc[(wave * cols + c) * kD + 16 * dt + 4 * g + r] = acc[dt][r];
+            *reinterpret_cast<floatx4*>(&sm_acc[(wave * cols + c) * kD + 16 * dt + 4 * g]) = acc[dt];
     }
     __syncthreads();
     for (int i = threadIdx.x; i < cols * kD; i += kDecodeThreads) {
@@ -701,12 +765,13 @@ static void launch_decode(const void* q, const void* k_pool, const void* v_pool,
     const long blocks = static_cast<long>(grid.x) * grid.y;
     const int ordered = rows > 1 && rows <= kOrderedRows && grid.z == 1 && blocks > kOrderedUnits && blocks <= 2 * kOrderedUnits ? 1 : 0;
     const float to_log2 = scale * 1.4426950408889634f;
+    const DecodeShape heads{group, (group + 15) / 16, splits > 1 ? static_cast<unsigned>(((1ull << 32) + splits - 1) / splits) : 0u};
     if constexpr (kD16 % 4 == 0) {
         if (from != nullptr) {
             attention_decode_kernel<kD16, true, false><<<grid, kDecodeThreads, smem, stream>>>(
                 nullptr, static_cast<const bf16_t*>(k_pool), static_cast<const bf16_t*>(v_pool), positions, row_entry,
                 block_table, max_blocks, part_acc, part_ml, static_cast<bf16_t*>(out), q_heads, kv_heads, page_shift,
-                to_log2, window, splits, *from, keep_first, bias, ScoreShape{}, chunk, ordered);
+                to_log2, window, splits, *from, keep_first, bias, ScoreShape{}, chunk, ordered, heads);
             return;
         }
     }
@@ -714,7 +779,7 @@ static void launch_decode(const void* q, const void* k_pool, const void* v_pool,
     attention_decode_kernel<kD16, false, SHAPED><<<grid, kDecodeThreads, smem, stream>>>(                                    \
         static_cast<const bf16_t*>(q), static_cast<const bf16_t*>(k_pool), static_cast<const bf16_t*>(v_pool),               \
         positions, row_entry, block_table, max_blocks, part_acc, part_ml, static_cast<bf16_t*>(out), q_heads, kv_heads,      \
-        page_shift, to_log2, window, splits, FromProjection{}, keep_first, bias, shape, chunk, ordered)
+        page_shift, to_log2, window, splits, FromProjection{}, keep_first, bias, shape, chunk, ordered, heads)
     if (shape.any()) LEONE_DECODE_LAUNCH(true);
     else LEONE_DECODE_LAUNCH(false);
 #undef LEONE_DECODE_LAUNCH
