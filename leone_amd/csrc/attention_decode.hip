@@ -221,7 +221,11 @@ attention_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);      // (the same for the whole wave: scalar registers)
     const int lane = threadIdx.x % kWave;
     int row = blockIdx.x, head_block = blockIdx.y;
-    if (ordered) row = ordered_row(positions, gridDim.x, gridDim.y, lane, head_block);
+    if (ordered) {
+        row = __builtin_amdgcn_readfirstlane(ordered_row(positions, gridDim.x, gridDim.y, lane, head_block));
+        head_block = __builtin_amdgcn_readfirstlane(head_block);
+    }
+    const int pos = positions[row], entry = row_entry[row];
     const int kvh = heads.col_tiles == 1 ? head_block : head_block / heads.col_tiles;
     const int col0 = (head_block - kvh * heads.col_tiles) * 16;
     const int cols = group - col0 < 16 ? group - col0 : 16;   // query heads handled here
@@ -256,7 +260,7 @@ attention_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__
         }
     }
 
-    const int n = positions[row] + 1;                                    // keys 0 .. n-1 exist
+    const int n = pos + 1;                                               // keys 0 .. n-1 exist
     const int lo = first_key(n - 1, window, chunk);                      // first key in reach
     // (asked for ahead of any key: loads come back in the order they were asked for)
     [[maybe_unused]] float angle_cos[kFused ? kHalfSteps : 1][8], angle_sin[kFused ? kHalfSteps : 1][8];
@@ -276,7 +280,7 @@ attention_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__
     const float cap_log2 = shape.cap * 1.4426950408889634f;                // capped scores, in units of log2
     const float to_cap = kShaped && shape.cap > 0.f ? to_log2_row / cap_log2 : 0.f;
     const float slope_log2 = (bias.slopes && c < cols) ? bias.slopes[kvh * group + col0 + c] * 1.4426950408889634f : 0.f;
-    const int* table = block_table + static_cast<long>(row_entry[row]) * max_blocks;
+    const int* table = block_table + static_cast<long>(entry) * max_blocks;
     const int t_begin = lo / kTileKeys, t_end = (n + kTileKeys - 1) / kTileKeys;
     // A windowed layer may keep its first keys in sight: keys below `keep` count as in reach wherever they lie.
     // The tiles that hold such keys and lie wholly before the window's first tile come first in the row's list of
@@ -302,7 +306,12 @@ attention_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__
     if (has_window) {
         const int last_key = (win_end * kTileKeys < n ? win_end * kTileKeys : n) - 1;
         n_win_pages = (last_key >> page_shift) - first_page + 1;
-        for (int i = threadIdx.x; i < n_win_pages; i += kDecodeThreads) pages[i] = table[first_page + i];
+        // (the last wave has no heads to make: its loads come back before the others' projections)
+        if (kFused && n_win_pages <= kWave) {
+            if (wave == kDecodeWaves - 1 && lane < n_win_pages) pages[lane] = table[first_page + lane];
+        } else {
+            for (int i = threadIdx.x; i < n_win_pages; i += kDecodeThreads) pages[i] = table[first_page + i];
+        }
     }
     const int kept_first_page = (my_begin * kTileKeys) >> page_shift;
     if (my_begin < kept_tiles && my_begin < my_end) {
@@ -370,6 +379,11 @@ attention_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__
 #pragma unroll
         for (int dt = 0; dt < kD16; ++dt) r.xv[dt] = load8_streamed(pv + 16 * dt * 8);
     };
+    // The workgroup whose keys end with the row's own position writes that position's key and value into the cache (with
+    // more than 16 query heads a kv head several do: the same bytes) and puts them into the tile that holds them itself: no
+    // wave waits for a write to come back.
+    const bool writes = kFused && from.k_out != nullptr && my_begin < my_end && my_end == n_tiles;
+    [[maybe_unused]] const int page = writes ? table[pos >> page_shift] : -1;   // the host reserves the page before the launch
     // The wave's first tile is asked for before the queries are made: neither waits for the other.
     Tile one, two;
     if (my_begin + wave < my_end) issue(my_begin + wave, true, one, true);
@@ -377,19 +391,13 @@ attention_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__
 
     // Q^T operand: column c is query head kvh*group + col0 + c.
     bf16x8 qreg[kSteps];
-    // The workgroup whose keys end with the row's own position writes that position's key and value into the cache (with
-    // more than 16 query heads a kv head several do: the same bytes) and puts them into the tile that holds them itself: no
-    // wave waits for a write to come back.
-    const bool writes = kFused && from.k_out != nullptr && my_begin < my_end && my_end == n_tiles;
-    // They stand, until the waves merge, where the wave that works on the last tile puts its results; the queries in the
+    // The new key and value stand, until the waves merge, where the wave that works on the last tile puts its results; the queries in the
     // next wave's place, until every wave has taken them.
     [[maybe_unused]] const int last_wave = writes ? (n_tiles - 1 - my_begin) % kDecodeWaves : 0;
     [[maybe_unused]] bf16_t* new_key = reinterpret_cast<bf16_t*>(smem + static_cast<long>(last_wave) * cols * kD);
     [[maybe_unused]] bf16_t* new_value = new_key + kD;
     if constexpr (kFused) {
         bf16_t* queries = reinterpret_cast<bf16_t*>(smem + static_cast<long>((last_wave + 1) % kDecodeWaves) * cols * kD);
-        const int pos = n - 1;
-        const int page = writes ? table[pos >> page_shift] : -1;             // the host reserves the page before the launch
         const long base = (static_cast<long>(page < 0 ? 0 : page) * kv_heads + kvh) * page_tokens * kD;
         const int token = pos & page_mask;
         if (wave == 0 || (wave == 1 && writes)) {
@@ -522,7 +530,6 @@ attention_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__
         }
         if constexpr (kFused) {
             if (writes && u == n_tiles - 1) {              // the row's own key and value, which the cache may not show yet
-                const int pos = n - 1;
 #pragma unroll
                 for (int s = 0; s < kSteps; ++s) {
                     if (ka == pos) r.xa[s] = load8(new_key + 32 * s + 8 * g);
@@ -638,37 +645,81 @@ attention_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__
             *reinterpret_cast<floatx4*>(&sm_acc[(wave * cols + c) * kD + 16 * dt + 4 * g]) = acc[dt];
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < cols * kD; i += kDecodeThreads) {
-        const int col = i / kD, d = i % kD;
-        const int partner = kShaped && shape.turn_cos != nullptr && splits == 1 ? turn_partner(d, kD / 2, shape.turn_pairing) : d;
-        float top = -INFINITY;
+    // Four elements of a head a thread (of one that is turned back, an element: it needs its pair's other one).
+    const bool turned = kShaped && shape.turn_cos != nullptr && splits == 1;
+    const bool wide = ((reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(part_acc)) & 15) == 0;
+    if (!turned) {
+        for (int i = threadIdx.x * 4; i < cols * kD; i += kDecodeThreads * 4) {
+            const int col = i / kD, d = i % kD;
+            float top = -INFINITY;
 #pragma unroll
-        for (int w = 0; w < kDecodeWaves; ++w) top = fmaxf(top, sm_m[w * cols + col]);
-        float num = 0.f, den = 0.f, num_partner = 0.f;
-        if (top != -INFINITY) {
+            for (int w = 0; w < kDecodeWaves; ++w) top = fmaxf(top, sm_m[w * cols + col]);
+            floatx4 num = {0.f, 0.f, 0.f, 0.f};
+            float den = 0.f;
+            if (top != -INFINITY) {
 #pragma unroll
-            for (int w = 0; w < kDecodeWaves; ++w) {
-                const float mw = sm_m[w * cols + col];
-                const float wgt = mw == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mw - top);
-                num += sm_acc[(w * cols + col) * kD + d] * wgt;
-                if (kShaped) num_partner += sm_acc[(w * cols + col) * kD + partner] * wgt;
-                den += sm_l[w * cols + col] * wgt;
+                for (int w = 0; w < kDecodeWaves; ++w) {
+                    const float mw = sm_m[w * cols + col];
+                    const float wgt = mw == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mw - top);
+                    const floatx4 part = *reinterpret_cast<const floatx4*>(&sm_acc[(w * cols + col) * kD + d]);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) num[e] += part[e] * wgt;
+                    den += sm_l[w * cols + col] * wgt;
+                }
+            }
+            const int head = kvh * group + col0 + col;
+            const long rh = static_cast<long>(row) * q_heads + head;
+            if (splits == 1) {                            // nothing to merge with: this is the result
+                if (kShaped && shape.sinks != nullptr) den += __builtin_amdgcn_exp2f(shape.sinks[head] * 1.4426950408889634f - top);
+                typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+                bf16x4 result;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) result[e] = static_cast<__bf16>(num[e] / den);
+                __bf16* to = reinterpret_cast<__bf16*>(out) + rh * kD + d;
+                if (wide) {
+                    *reinterpret_cast<bf16x4*>(to) = result;
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) to[e] = result[e];
+                }
+                continue;
+            }
+            const long slot = rh * splits + split;
+            if (wide) {
+                *reinterpret_cast<floatx4*>(part_acc + slot * kD + d) = num;
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) part_acc[slot * kD + d + e] = num[e];
+            }
+            if (d == 0) {
+                part_ml[slot * 2] = top;
+                part_ml[slot * 2 + 1] = den;
             }
         }
-        const int head = kvh * group + col0 + col;
-        const long rh = static_cast<long>(row) * q_heads + head;
-        if (splits == 1) {                            // nothing to merge with: this is the result
-            if (kShaped && shape.sinks != nullptr) den += __builtin_amdgcn_exp2f(shape.sinks[head] * 1.4426950408889634f - top);
-            float value = num / den;
-            if (kShaped && shape.turn_cos != nullptr) value = turned_back(value, num_partner / den, d, kD, n - 1, shape);
-            out[rh * kD + d] = from_float<bf16_t>(value);
-            continue;
-        }
-        const long slot = rh * splits + split;
-        part_acc[slot * kD + d] = num;
-        if (d == 0) {
-            part_ml[slot * 2] = top;
-            part_ml[slot * 2 + 1] = den;
+        return;
+    }
+    if constexpr (kShaped) {
+        for (int i = threadIdx.x; i < cols * kD; i += kDecodeThreads) {
+            const int col = i / kD, d = i % kD;
+            const int partner = turn_partner(d, kD / 2, shape.turn_pairing);
+            float top = -INFINITY;
+#pragma unroll
+            for (int w = 0; w < kDecodeWaves; ++w) top = fmaxf(top, sm_m[w * cols + col]);
+            float num = 0.f, den = 0.f, num_partner = 0.f;
+            if (top != -INFINITY) {
+#pragma unroll
+                for (int w = 0; w < kDecodeWaves; ++w) {
+                    const float mw = sm_m[w * cols + col];
+                    const float wgt = mw == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mw - top);
+                    num += sm_acc[(w * cols + col) * kD + d] * wgt;
+                    num_partner += sm_acc[(w * cols + col) * kD + partner] * wgt;
+                    den += sm_l[w * cols + col] * wgt;
+                }
+            }
+            const int head = kvh * group + col0 + col;
+            if (shape.sinks != nullptr) den += __builtin_amdgcn_exp2f(shape.sinks[head] * 1.4426950408889634f - top);
+            out[(static_cast<long>(row) * q_heads + head) * kD + d] =
+                from_float<bf16_t>(turned_back(num / den, num_partner / den, d, kD, n - 1, shape));
         }
     }
 }
