@@ -386,7 +386,7 @@ attention_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__
     [[maybe_unused]] const int page = writes ? table[pos >> page_shift] : -1;   // the host reserves the page before the launch
     // The wave's first tile is asked for before the queries are made: neither waits for the other.
     Tile one, two;
-    if (my_begin + wave < my_end) issue(my_begin + wave, true, one, true);
+    if ((!kFused || wave >= 2) && my_begin + wave < my_end) issue(my_begin + wave, true, one, true);
     if constexpr (!kFused) __syncthreads();            // the page ids are there (else where the queries are)
 
     // Q^T operand: column c is query head kvh*group + col0 + c.
@@ -471,6 +471,7 @@ attention_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__
                 for (int i = 0; i < 8; ++i) to[8 * i] = bf16_t{static_cast<uint16_t>(i % 2 ? w[i / 2] >> 16 : w[i / 2] & 0xffffu)};
             }
         }
+        if (wave < 2 && my_begin + wave < my_end) issue(my_begin + wave, true, one, true);
         __syncthreads();
 #pragma unroll
         for (int s = 0; s < kSteps; ++s) qreg[s] = head_ok ? load8(queries + c * kD + 32 * s + 8 * g) : zero8();
@@ -615,7 +616,9 @@ attention_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__
         }
     } else {
         int t = my_begin + wave;
-        if (t < my_end) {
+        if (t < my_end && t + kDecodeWaves >= my_end) {
+            finish(t, one);
+        } else if (t < my_end) {
             while (true) {
                 const int t1 = t + kDecodeWaves;
                 issue(t1, t1 < my_end, two, false);
