@@ -116,6 +116,12 @@ __device__ float plain_segment(const float* __restrict__ a, const float* __restr
     return sum;
 }
 
+// What is done with finished sums: nothing, or (B's rows are 8 gates, their 8 ups, and so on) act(gate) * up of every pair.
+struct Epilogue {
+    int gated = 0, act = 0;
+    float limit = 0.f;
+};
+
 // ---- few rows ------------------------------------------------------------------------------------------------------
 // Lane l of a wave loads, of 16 rows of B, row l % 16's elements 4 (l / 16) .. + 3 of every run of 16: one 16-byte load
 // a lane is 64 bytes of each of 16 rows.  A's rows lie the same way, out of the caches (rows past the last are the last one again
@@ -127,7 +133,8 @@ constexpr int kChain = 32;                             // elements of K whose pr
 
 template <int kTilesM, int kWaves, int kDepth, int kEach, bool kVec>
 __global__ void __launch_bounds__(kWaves * kWave, kEach)
-gemm_f32_stream_kernel(const float* __restrict__ a, const float* __restrict__ b, float* __restrict__ c, int m, int n, int k, int segment) {
+gemm_f32_stream_kernel(const float* __restrict__ a, const float* __restrict__ b, float* __restrict__ c, int m, int n, int k, int segment,
+                       Epilogue then) {
     __shared__ float sums[kWaves][kTilesM][kStreamTile * kStreamTile];
     static_assert(kDepth % 2 == 0, "a register's runs are all even ones or all odd ones");
     const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
@@ -207,6 +214,17 @@ gemm_f32_stream_kernel(const float* __restrict__ a, const float* __restrict__ b,
             sums[wave][t][(h + i) * kStreamTile + r] = sum[t][i];
         }
     __syncthreads();
+    if (then.gated) {                                  // the tile's 16 rows of B are eight gates and their ups
+        for (int e = threadIdx.x; e < kTilesM * 128; e += kWaves * kWave) {
+            const int t = e / 128, row = t * 16 + e % 128 / 8, at = e % 128 / 8 * kStreamTile + e % 8;
+            if (row >= m) continue;
+            float gate = sums[0][t][at], up = sums[0][t][at + 8];
+#pragma unroll
+            for (int v = 1; v < kWaves; ++v) gate += sums[v][t][at], up += sums[v][t][at + 8];
+            c[static_cast<long>(row) * (n / 2) + n0 / 2 + e % 8] = glu_value(gate, up, then.act, then.limit);
+        }
+        return;
+    }
     for (int e = threadIdx.x; e < kTilesM * 256; e += kWaves * kWave) {
         const int t = e / 256, row = t * 16 + e % 256 / 16, col = n0 + e % 16;
         if (row >= m || col >= n) continue;
@@ -237,7 +255,7 @@ constexpr int kTileRows = 64;
 template <int kCols, bool kVec, bool kCut>
 __global__ void __launch_bounds__(256, 3)
 gemm_f32_tile_kernel(const float* __restrict__ a, const float* __restrict__ b, float* __restrict__ c, int m, int n, int k,
-                     int segment, int each) {
+                     int segment, int each, Epilogue then) {
     constexpr int kFragA = kTileRows / 16, kFragB = kCols / 64;                      // 16 x 16 squares of a wave
     constexpr int kLoadsA = kTileRows / 32;                                          // 16-byte loads a thread and slab
     __shared__ u32x2 slabs[2][3][kTileRows][8];
@@ -386,7 +404,21 @@ gemm_f32_tile_kernel(const float* __restrict__ a, const float* __restrict__ b, f
                 }
         }
     }
-    if constexpr (!kCut) store(total, c);
+    if constexpr (!kCut) {
+        if (!then.gated) return store(total, c);
+        // lanes 0 .. 7 of a row of 16 hold gates, the lane eight further its up
+#pragma unroll
+        for (int i = 0; i < kFragA; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int j = 0; j < kFragB; ++j) {
+                    const float up = lane_pair<8>(total[i][j][e]).b;
+                    if (r < 8 && row_of(i, e) < m && col + j * 16 < n)
+                        c[static_cast<long>(row_of(i, e)) * (n / 2) + (n0 + j * 16) / 2 + r] =
+                            glu_value(total[i][j][e], up, then.act, then.limit);
+                }
+    }
 }
 
 // ---- a short K -----------------------------------------------------------------------------------------------------
@@ -488,6 +520,28 @@ __global__ void __launch_bounds__(256) gemm_f32_sum_kernel(const float* __restri
     }
 }
 
+// The same of sums that are gates and ups: four results a thread, of rows of n / 2.  kVec: planes and c are aligned to 16 bytes.
+template <bool kVec>
+__global__ void __launch_bounds__(256)
+gemm_f32_sum_gated_kernel(const float* __restrict__ planes, float* __restrict__ c, long count, int n, int parts, Epilogue then) {
+    const long at = (static_cast<long>(blockIdx.x) * 256 + threadIdx.x) * 4;
+    if (at >= count / 2) return;
+    const long row = at / (n / 2);
+    const int col = static_cast<int>(at - row * (n / 2));                   // n / 2 is a multiple of 8
+    const float* from = planes + row * n + col / 8 * 16 + col % 8;
+    const auto four = [](const float* p) { return kVec ? *reinterpret_cast<const f32x4*>(p) : f32x4{p[0], p[1], p[2], p[3]}; };
+    f32x4 gate = four(from), up = four(from + 8), result;
+    for (int p = 1; p < parts; ++p) gate += four(from + p * count), up += four(from + p * count + 8);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) result[e] = glu_value(gate[e], up[e], then.act, then.limit);
+    if (kVec) {
+        *reinterpret_cast<f32x4*>(c + at) = result;
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) c[at + e] = result[e];
+    }
+}
+
 // Up to here a product is a stream of weights.  Measured (us, streamed : tiled) against 2048 x 2048 weights 11.4 : 12.1 at 17 rows,
 // 13.7 : 12.5 at 32, 3072 x 512 5.9 : 9.7 at 32, 6144 x 1024 13.9 : 14.4; beyond, the stream's reads of A, then four times the
 // weights', cost more.  A long K leaves the tiles' workgroups enough to do from the second tile of rows on: 1024 x 3072 15.1 : 14.6
@@ -560,7 +614,8 @@ F32Plan f32_plan(int m, int n, int k) {
     return best;
 }
 
-int launch_f32(const F32Plan& p, const float* a, const float* b, float* c, float* planes, int m, int n, int k, hipStream_t stream) {
+int launch_f32(const F32Plan& p, const float* a, const float* b, float* c, float* planes, int m, int n, int k, const Epilogue& then,
+               hipStream_t stream) {
     const F32Segments segments = f32_segments(k);
     LEONE_REQUIRE(p.parts == 1 || planes, "gemm_f32: %d planes are needed for %d x %d x %d", segments.count, m, n, k);
     const auto aligned = [](const void* at) { return reinterpret_cast<uintptr_t>(at) % 16 == 0; };
@@ -568,8 +623,8 @@ int launch_f32(const F32Plan& p, const float* a, const float* b, float* c, float
     if (p.rows == 0) {
         const int blocks = ceil_div(n, kStreamTile);
 #define LEONE_STREAM(T, W, D, E)                                                                                                       \
-    (vec ? gemm_f32_stream_kernel<T, W, D, E, true><<<blocks, W * kWave, 0, stream>>>(a, b, c, m, n, k, segments.length)               \
-         : gemm_f32_stream_kernel<T, W, D, E, false><<<blocks, W * kWave, 0, stream>>>(a, b, c, m, n, k, segments.length))
+    (vec ? gemm_f32_stream_kernel<T, W, D, E, true><<<blocks, W * kWave, 0, stream>>>(a, b, c, m, n, k, segments.length, then)         \
+         : gemm_f32_stream_kernel<T, W, D, E, false><<<blocks, W * kWave, 0, stream>>>(a, b, c, m, n, k, segments.length, then))
         // Runs on their way a wave: two leave room for more waves, whose loads count as well, and segments of few runs have no use for
         // more; of a large matrix four (us, two and four runs: one row against 12288 x 2048 21.2 and 19.0, 32768 x 2048 48.1 and 44.0,
         // 2048 x 6144 17.7 and 17.2; but 2048 x 2048 7.1 and 7.4, 1024 x 3072 10.9 and 11.5, five rows against 32768 x 512 16.4 and
@@ -596,8 +651,8 @@ int launch_f32(const F32Plan& p, const float* a, const float* b, float* c, float
     (vec ? gemm_f32_chain_kernel<R, true><<<grid, 256, 0, stream>>>(a, b, c, m, n, k)                                                  \
          : gemm_f32_chain_kernel<R, false><<<grid, 256, 0, stream>>>(a, b, c, m, n, k))
 #define LEONE_TILE_CUT(C, V)                                                                                                           \
-    (p.parts > 1 ? gemm_f32_tile_kernel<C, V, true><<<grid, 256, 0, stream>>>(a, b, planes, m, n, k, segments.length, p.each)          \
-                 : gemm_f32_tile_kernel<C, V, false><<<grid, 256, 0, stream>>>(a, b, c, m, n, k, segments.length, p.each))
+    (p.parts > 1 ? gemm_f32_tile_kernel<C, V, true><<<grid, 256, 0, stream>>>(a, b, planes, m, n, k, segments.length, p.each, then)    \
+                 : gemm_f32_tile_kernel<C, V, false><<<grid, 256, 0, stream>>>(a, b, c, m, n, k, segments.length, p.each, then))
 #define LEONE_TILE(C) (vec ? LEONE_TILE_CUT(C, true) : LEONE_TILE_CUT(C, false))
     if (k < kStreamK) p.rows == 128 ? LEONE_CHAIN(128) : LEONE_CHAIN(64);
     else p.cols == 128 ? LEONE_TILE(128) : LEONE_TILE(64);
@@ -607,6 +662,13 @@ int launch_f32(const F32Plan& p, const float* a, const float* b, float* c, float
     LEONE_LAUNCH_CHECK("gemm_f32");
     if (p.parts > 1) {
         const long count = static_cast<long>(m) * n;
+        if (then.gated) {
+            const int blocks = ceil_div(count / 2, 1024);
+            if (aligned(planes) && aligned(c)) gemm_f32_sum_gated_kernel<true><<<blocks, 256, 0, stream>>>(planes, c, count, n, segments.count, then);
+            else gemm_f32_sum_gated_kernel<false><<<blocks, 256, 0, stream>>>(planes, c, count, n, segments.count, then);
+            LEONE_LAUNCH_CHECK("gemm_f32 sum");
+            return 0;
+        }
         const int blocks = ceil_div(count, 1024);
         if (count % 4 == 0 && aligned(planes) && aligned(c))
             gemm_f32_sum_kernel<true><<<blocks, 256, 0, stream>>>(planes, c, count, segments.count);
@@ -632,5 +694,20 @@ extern "C" int leone_gemm_f32_planes(int m, int n, int k) {
 extern "C" int leone_gemm_f32(const float* a, const float* b, float* c, float* planes, int m, int n, int k, hipStream_t stream) {
     LEONE_REQUIRE(a && b && c, "gemm_f32: null pointer");
     LEONE_REQUIRE(m > 0 && n > 0 && k > 0, "gemm_f32: sizes %d x %d x %d must be positive", m, n, k);
-    return launch_f32(f32_plan(m, n, k), a, b, c, planes, m, n, k, stream);
+    return launch_f32(f32_plan(m, n, k), a, b, c, planes, m, n, k, Epilogue{}, stream);
+}
+
+// Whether leone_gemm_f32_glu takes a matrix: whole tiles of eight gates and their ups, and a K that is no chain.
+extern "C" int leone_gemm_f32_glu_fits(int n, int k) { return n > 0 && n % 16 == 0 && k >= kStreamK; }
+
+// C[M, N / 2] = act(gate) * up of the same product, B's rows being eight gates, their eight ups, and so on (act, limit: as leone_glu).
+// The bits are those of the product and leone_glu behind it; one launch and the product's way to memory and back are saved (us, before
+// and with it: one row against 12288 x 2048 23.4 and 18.9; 777 rows 255 and 240).
+extern "C" int leone_gemm_f32_glu(const float* a, const float* b, float* c, float* planes, int m, int n, int k, int act, float limit,
+                                  hipStream_t stream) {
+    LEONE_REQUIRE(a && b && c, "gemm_f32_glu: null pointer");
+    LEONE_REQUIRE(m > 0 && leone_gemm_f32_glu_fits(n, k), "gemm_f32_glu: sizes %d x %d x %d", m, n, k);
+    LEONE_REQUIRE(act == kGateSilu || act == kGateGeluTanh || (act == kGateClampedSwish && limit > 0.f),
+                  "gemm_f32_glu: unknown activation %d (limit %g)", act, limit);
+    return launch_f32(f32_plan(m, n, k), a, b, c, planes, m, n, k, Epilogue{1, act, limit}, stream);
 }

@@ -98,6 +98,9 @@ int leone_attention_prefill(const void* q, void* out, const void* k_pool, const 
 // C[M,N] = A[M,K] . B[N,K]^T in float.
 int leone_gemm_f32_planes(int m, int n, int k);      // planes [m, n] of floats that leone_gemm_f32 needs beside C, 0 for none
 int leone_gemm_f32(const float* a, const float* b, float* c, float* planes, int m, int n, int k, hipStream_t stream);
+int leone_gemm_f32_glu_fits(int n, int k);              // whether leone_gemm_f32_glu takes [n, k]
+int leone_gemm_f32_glu(const float* a, const float* b, float* c, float* planes, int m, int n, int k, int act, float limit,
+                       hipStream_t stream);
 
 // Tiled weights.  The two weight-streaming products below read W either row by row ([N,K]) or, with w_tiled, from
 // a copy laid out in the order in which their waves ask for it, for K a multiple of 64: rows in tiles of 16

@@ -724,6 +724,23 @@ def gemm_f32(a: torch.Tensor, b: torch.Tensor, out: Optional[torch.Tensor] = Non
     return out
 
 
+def gemm_f32_glu(a: torch.Tensor, b: torch.Tensor, activation: str = "silu", limit: Optional[float] = None) -> torch.Tensor:
+    """``swiglu(gemm_f32(a, b), ...)`` to the bit, in the product's own launch where it takes ``b`` [8 gates, their 8 ups, ..; K]."""
+    m, k = a.shape
+    n, k2 = b.shape
+    if k != k2:
+        raise KernelError(f"gemm_f32: inner sizes {k} and {k2} differ")
+    if not library().leone_gemm_f32_glu_fits(n, k):
+        return swiglu(gemm_f32(a, b), activation=activation, limit=limit)
+    out = torch.empty((m, n // 2), dtype=torch.float32, device=a.device)
+    parts = library().leone_gemm_f32_planes(m, n, k)
+    planes = torch.empty((parts, m, n), dtype=torch.float32, device=a.device) if parts else None
+    with profile.span("gemm f32", b):
+        call("leone_gemm_f32_glu", _dev(a, "gemm a", torch.float32), _dev(b, "gemm b", torch.float32), _dev(out, "gemm out"),
+             _dev(planes, "gemm planes"), m, n, k, _glu_code(activation, limit), float(limit or 0.0), _stream())
+    return out
+
+
 # Up to here norm, gate and residual are folded into the weight-streaming kernel for few rows; beyond, the
 # multi-row kernel runs with the row-wise kernels between.  Measured in whole decode steps at the 8B layer sizes
 # with the second copies of the weights (ms a step, folded : multi-row): 5.98 : 6.40 at 11 rows, 6.17 : 6.47 at
@@ -1173,6 +1190,8 @@ def linear(x, weight: torch.Tensor, out_dtype: Optional[torch.dtype] = None,
     if dtype == torch.float32:
         if out_dtype != torch.float32:
             raise KernelError("linear: the float32 path produces float32")
+        if gated:
+            return gemm_f32_glu(x, weight, activation, limit)
         y = gemm_f32(x, weight)
     elif not x.is_cuda:
         raise KernelError("linear: tensor is not on the GPU")

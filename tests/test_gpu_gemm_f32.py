@@ -107,3 +107,17 @@ def test_numbers_that_are_no_sums_of_parts():
         assert torch.equal(got[1], torch.full_like(got[1], -3.4028234e38) * 0.25)
         keep = [j for j in range(n) if j != 3]
         assert bool((got[2, keep] == math.inf).all()) and bool(torch.isnan(got[2, 3])) and not bool(got[3:].any())
+
+
+@pytest.mark.parametrize("n,k", [(16, 256), (48, 511), (144, 520), (1040, 1024), (96, 255), (3072, 2048)])
+def test_gates_and_ups_in_the_products_own_launch(n, k):
+    """To the bit what the product and the activation behind it give, in every kernel, also where K is cut or too short."""
+    from leone_amd import ops
+    b = torch.randn(n, k, device=DEV) / math.sqrt(k)
+    for m in (1, 5, 16, 17, 33, 64, 130, 300):
+        a = torch.randn(m, k, device=DEV)
+        for options in ({}, {"activation": "gelu_tanh"}, {"activation": "clamped_swish", "limit": 0.5}):
+            assert torch.equal(ops.gemm_f32_glu(a, b, **options), ops.swiglu(ops.gemm_f32(a, b), **options)), (m, options)
+    a[0, 3], a[1, 5] = math.inf, math.nan
+    got, want = ops.gemm_f32_glu(a, b), ops.swiglu(ops.gemm_f32(a, b))
+    assert torch.equal(torch.nan_to_num(got, 1.0, 2.0, 3.0), torch.nan_to_num(want, 1.0, 2.0, 3.0))
