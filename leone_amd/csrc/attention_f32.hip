@@ -16,8 +16,12 @@
 // as keys x queries, so that a lane's four scores belong to its own query and to the four keys it holds values of: they
 // are the operand of the second product as they stand.
 //
-// Measured (us; the row kernel of attention.hip before): 16 heads over 4 of 128 elements, one row at 780 keys 25 (314), a prompt
-// of 777 rows 71 (1375), of 2,048 rows 295 (8589).
+// Everything that is the same for a wave (its share, the tile, the page) is in scalar registers, and a tile that every row sees whole
+// needs neither masks nor a look for values that are no numbers: of the instructions between the products, which the other wave of a
+// SIMD has to cover, that is a third.
+//
+// Measured (us; with those, the row kernel of attention.hip): 16 heads over 4 of 128 elements, one row at 780 keys 23.5 (24.9, 314), a prompt
+// of 777 rows 64 (71, 1375), of 2,048 rows 260 (292, 8589).
 #include "common.h"
 #include "leone_hip.h"
 #include "score_shape.h"
@@ -40,7 +44,9 @@ struct AttentionF32Args {
     const int* positions;
     const int* row_entry;
     const int* block_table;
-    int max_blocks, rows, q_heads, kv_heads, page_tokens;
+    int max_blocks, rows, q_heads, kv_heads, group, most;      // most: rows that a workgroup takes
+    unsigned multiples_inverse;                                // 2^32 / (rows / most, rounded up), rounded up; 0: divide
+    int page_tokens, page_shift;                               // page_shift: -1 if page_tokens is no power of two
     float scale;
     int window;
     const float* gate;
@@ -64,40 +70,58 @@ __global__ void __launch_bounds__(kWaves * kWave, kDim == 64 ? 3 : 2) attention_
     // workgroups of the rows that another one takes have nothing to do.  Rows are numbered so that those at the multiples come first,
     // one behind the other: workgroups go to the eight dies in turn, and every 4th or 16th would have left the work of a portion to one
     // or two of them (2,048 rows of 16 heads over 4 of 128: 1330 us, numbered so 295).
-    const int group = g.q_heads / g.kv_heads, most = kQueries / group;
+    const int group = g.group, most = g.most;
     const int multiples = (g.rows + most - 1) / most;
-    const int first_row = blockIdx.x % multiples * most + blockIdx.x / multiples, kvh = blockIdx.y;
+    const int turn = multiples == 1 ? blockIdx.x : g.multiples_inverse ? __umulhi(blockIdx.x, g.multiples_inverse) : blockIdx.x / multiples;
+    const int first_row = (blockIdx.x - turn * multiples) * most + turn, kvh = blockIdx.y;       // (turn 0: a multiple of `most`)
     if (first_row >= g.rows) return;
-    const int entry = g.row_entry[first_row];
-    if (first_row % most != 0 && g.row_entry[first_row - 1] == entry) return;
-    int count = 1;
-    while ((first_row + count) % most != 0 && first_row + count < g.rows && g.row_entry[first_row + count] == entry) ++count;
-
-    const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
     const int mine = lane % 16, h = (lane / 16) * 4;
-    // this lane's query: lanes past the last one repeat it and write nothing
+
+    // A lane's query, if the workgroup takes so many rows (past the last row it is the last one again), is asked for ahead of what the
+    // rows are; that comes by scalar loads where, as in decoding, the row is alone.
+    const auto clamped = [&](int row) { return row < g.rows ? row : g.rows - 1; };
+    const int place = mine / group;                           // which of the rows this lane's query belongs to
+    const int row = clamped(first_row + place), head = kvh * group + (mine - place * group);
+    const int entry = g.row_entry[first_row], entry_before = g.row_entry[first_row > 0 ? first_row - 1 : 0];
+    const int entry_after = g.row_entry[clamped(first_row + 1)], first_pos = g.positions[first_row];
+    if (turn != 0 && entry_before == entry) return;
+    // rows of the same request, one behind the other, up to the next multiple
+    const int room = most - turn < g.rows - first_row ? most - turn : g.rows - first_row;
+    int count = 1, pos = first_pos;
+    if (room > 1 && entry_after == entry) {
+        const unsigned others = static_cast<unsigned>(__ballot(g.row_entry[clamped(first_row + mine)] != entry)) & 0xffffu;
+        const int same = others ? __builtin_ctz(others) : 16;
+        count = same < room ? same : room;
+        pos = g.positions[first_row + (place < count ? place : count - 1)];
+    }
+    // lanes past the last query stand where the last row does and write nothing
     const bool real = mine < count * group;
-    const int query = real ? mine : count * group - 1;
-    const int row = first_row + query / group, head = kvh * group + query % group;
-    const int pos = g.positions[row];
+    f32x4 q[kRuns];
+    {
+        const float* qr = g.q + (static_cast<long>(row) * g.q_heads + head) * kDim;
+#pragma unroll
+        for (int i = 0; i < kRuns; ++i) q[i] = *reinterpret_cast<const f32x4*>(qr + i * 16 + h);
+    }
     float scale = g.scale;
     if (g.temp_every > 0) scale *= 1.0f + g.temp_coef * logf(static_cast<float>((pos + 1) / g.temp_every + 1));
     const float slope = g.slopes ? g.slopes[head] : 0.f;
     const int first = first_key(pos, g.window, g.chunk);
 
-    f32x4 q[kRuns];
-    const float* qr = g.q + (static_cast<long>(row) * g.q_heads + head) * kDim;
-#pragma unroll
-    for (int i = 0; i < kRuns; ++i) q[i] = *reinterpret_cast<const f32x4*>(qr + i * 16 + h);
-
     // what the rows together see: tiles of 16 keys from the earliest row's first one on, and those of the kept first keys
-    const int low = join_span<16>(first, [](int a, int b) { return min(a, b); });
-    const int high = join_span<16>(pos, [](int a, int b) { return max(a, b); });
+    // and what each of them sees: a tile between the two needs no masks
+    int low = __builtin_amdgcn_readfirstlane(first), high = __builtin_amdgcn_readfirstlane(pos), whole_from = low, whole_to = high;
+    if (count > 1) {
+        const auto least = [](int v) { return __builtin_amdgcn_readfirstlane(join_span<16>(v, [](int a, int b) { return min(a, b); })); };
+        const auto most_of = [](int v) { return __builtin_amdgcn_readfirstlane(join_span<16>(v, [](int a, int b) { return max(a, b); })); };
+        low = least(first), high = most_of(pos), whole_from = most_of(first), whole_to = least(pos);
+    }
     const int low_tile = low / kKeys;
     const int kept_tiles = min((g.keep_first + kKeys - 1) / kKeys, low_tile);
     const int tiles = high / kKeys + 1;
     const int* table = g.block_table + static_cast<long>(entry) * g.max_blocks;
     const long page_floats = static_cast<long>(g.page_tokens) * kDim;
+    const auto page_of = [&](int key) { return g.page_shift >= 0 ? key >> g.page_shift : key / g.page_tokens; };
 
     f32x4 kf[kRuns], vf[kRuns], acc[kRuns] = {};
     [[maybe_unused]] f32x4 ready[kOwn == 2 ? kRuns : 1];      // the first of two shares
@@ -106,18 +130,22 @@ __global__ void __launch_bounds__(kWaves * kWave, kDim == 64 ? 3 : 2) attention_
     // share n's tiles are those whose number is n modulo kShares, wave w has the shares that are w modulo kWaves; past the kept
     // tiles, from the first that a row sees on
     const auto skip = [&](int t) { return t < kept_tiles || t >= low_tile ? t : t + (low_tile - t + kShares - 1) / kShares * kShares; };
+    int in_page = 0;                              // of the tile that is fetched: its first key's place in its page
     const auto block_of = [&](int start, bool& there) {
-        const int page = table[start / g.page_tokens];
+        const int block = page_of(start), page = table[block];
+        in_page = start - block * g.page_tokens;
         there = page >= 0;
         return (static_cast<long>(there ? page : 0) * g.kv_heads + kvh) * page_floats;
     };
-    const auto fetch_keys = [&](int start, long block) {
-        const float* at = g.k_pool + block + (static_cast<long>(h / 8) * g.page_tokens + start % g.page_tokens + mine) * 8 + h % 8;
+    const long run_step = 2l * g.page_tokens * 8;             // from a key's 16 elements to its next
+    const int key_lane = (h / 8) * g.page_tokens * 8 + mine * 8 + h % 8, value_lane = ((h / 8) * kDim + mine) * 8 + h % 8;
+    const auto fetch_keys = [&](long block) {
+        const float* at = g.k_pool + block + in_page * 8 + key_lane;
 #pragma unroll
-        for (int i = 0; i < kRuns; ++i) kf[i] = *reinterpret_cast<const f32x4*>(at + static_cast<long>(2 * i) * g.page_tokens * 8);
+        for (int i = 0; i < kRuns; ++i) kf[i] = *reinterpret_cast<const f32x4*>(at + i * run_step);
     };
-    const auto fetch_values = [&](int start, long block) {
-        const float* at = g.v_pool + block + (static_cast<long>((start % g.page_tokens + h) / 8) * kDim + mine) * 8 + h % 8;
+    const auto fetch_values = [&](long block, int first_place) {
+        const float* at = g.v_pool + block + static_cast<long>(first_place) * kDim + value_lane;      // (a tile begins a run of 8)
 #pragma unroll
         for (int i = 0; i < kRuns; ++i) vf[i] = *reinterpret_cast<const f32x4*>(at + i * 128);
     };
@@ -138,12 +166,14 @@ __global__ void __launch_bounds__(kWaves * kWave, kDim == 64 ? 3 : 2) attention_
         long block = 0;
         if (t < tiles) {
             block = block_of(t * kKeys, mapped);
-            fetch_keys(t * kKeys, block);
+            fetch_keys(block);
         }
         while (t < tiles) {
             const int start = t * kKeys;
             t = skip(t + kShares);
-            fetch_values(start, block);
+            fetch_values(block, in_page);
+            // whether every row sees all of the tile's keys
+            const bool whole = mapped && start + kKeys - 1 <= whole_to && (start >= whole_from || start + kKeys <= g.keep_first);
             f32x4 dots[4] = {};                   // four sums side by side: no instruction waits for the one before it
 #pragma unroll
             for (int i = 0; i < kRuns; ++i)
@@ -152,13 +182,13 @@ __global__ void __launch_bounds__(kWaves * kWave, kDim == 64 ? 3 : 2) attention_
             f32x4 s = (dots[0] + dots[1]) + (dots[2] + dots[3]);
             if (t < tiles) {                      // the keys' registers are free: the next tile's are on their way from here on
                 block = block_of(t * kKeys, mapped_next);
-                fetch_keys(t * kKeys, block);
+                fetch_keys(block);
             }
             float top = -INFINITY;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int key = start + h + r;
-                const bool seen = key <= pos && (key >= first || key < g.keep_first);
+                const bool seen = whole || (key <= pos && (key >= first || key < g.keep_first));
                 float v = s[r] * scale;
                 if (g.shape.cap > 0.f) v = g.shape.cap * tanhf(v / g.shape.cap);
                 v -= slope * static_cast<float>(pos - key);
@@ -188,13 +218,18 @@ __global__ void __launch_bounds__(kWaves * kWave, kDim == 64 ? 3 : 2) attention_
                     for (int r = 0; r < 4; ++r)
                         if (!mapped || start + h + r > high) vf[i][r] = 0.f;
             }
-            f32x4 odd = {0.f, 0.f, 0.f, 0.f};                // stays 0 unless a value is infinite or NaN
+            {
 #pragma unroll
-            for (int i = 0; i < kRuns; ++i) {
-                acc[i] *= alpha;
-                odd += vf[i] * 0.f;
+                for (int i = 0; i < kRuns; ++i) acc[i] *= alpha;
             }
-            if (__any(!(odd[0] + odd[1] + odd[2] + odd[3] == 0.f))) {
+            bool odd_value = false;
+            if (!whole) {
+                f32x4 odd = {0.f, 0.f, 0.f, 0.f};            // stays 0 unless a value is infinite or NaN
+#pragma unroll
+                for (int i = 0; i < kRuns; ++i) odd += vf[i] * 0.f;
+                odd_value = __any(!(odd[0] + odd[1] + odd[2] + odd[3] == 0.f));
+            }
+            if (odd_value) {
                 // such a value is for the rows that see it, and no weight of 0 keeps it from the others: one key after the other, in
                 // the order of the instructions below
 #pragma unroll
@@ -307,10 +342,13 @@ void launch_attention_f32(const float* q, float* out, const float* k_pool, const
                           const int* block_table, int max_blocks, int rows, int q_heads, int kv_heads, int head_dim, int page_tokens,
                           float scale, int window, const float* gate, long gate_stride, int keep_first, int gate_each,
                           const float* slopes, float temp_coef, int temp_every, const ScoreShape& shape, int chunk, hipStream_t stream) {
+    const int group = q_heads / kv_heads, most = kQueries / group;
+    const long multiples = ceil_div(rows, most);
+    const int page_shift = (page_tokens & (page_tokens - 1)) == 0 ? __builtin_ctz(page_tokens) : -1;
     const AttentionF32Args args{q, out, k_pool, v_pool, positions, row_entry, block_table, max_blocks, rows, q_heads, kv_heads,
-                                page_tokens, scale, window, gate, gate_stride, keep_first, gate_each, slopes, temp_coef, temp_every,
+                                group, most, multiples > 1 && multiples * rows < 1l << 32 ? static_cast<unsigned>(((1ull << 32) + multiples - 1) / multiples) : 0u,
+                                page_tokens, page_shift, scale, window, gate, gate_stride, keep_first, gate_each, slopes, temp_coef, temp_every,
                                 shape, chunk};
-    const int most = kQueries / (q_heads / kv_heads);
     const dim3 grid(ceil_div(rows, most) * most, kv_heads);
     // Eight waves, a share each, where the launch is small or heads are of 128 elements; four waves with two shares each for many
     // rows of 64, whose workgroups are short (us, eight waves and four: 8 heads over 2, 1,500 rows 66 and 58, 300 decoded rows at 500
