@@ -203,6 +203,9 @@ int leone_sample_truncated_stages();
 int leone_sample_truncated_params();
 int leone_sample_truncated(const float* logits, const double* params, int* out, int rows, int vocab,
                            hipStream_t stream);
+long leone_choose_workspace(int rows, int vocab);                 // doubles that leone_choose_tokens needs
+int leone_choose_tokens(const float* logits, const double* kinds, int of_kinds, const double* temperature, const double* uniform,
+                        const double* params, int* out, double* work, int rows, int vocab, hipStream_t stream);
 
 // ---- layers that keep state of their own per request (layernorm_conv.hip, recurrent.hip) ----------------------
 // x += LayerNorm(delta; dw, db, deps) if delta comes (dw null: added as it is), then y = LayerNorm(x; w, b, eps)

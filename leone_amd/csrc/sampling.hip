@@ -45,12 +45,8 @@ __device__ inline Best block_best(Best mine, Best* scratch) {
 // `better` prefers the lower index on equal values, so the result does not depend on the cut.
 constexpr int kArgmaxChunk = 4096;
 
-__global__ void __launch_bounds__(kSampleThreads)
-argmax_partial_kernel(const float* __restrict__ logits, float* __restrict__ part_value,
-                      int* __restrict__ part_index, int vocab, int chunks) {
+__device__ inline void argmax_of_chunk(const float* __restrict__ row, int chunk, float* part_value, int* part_index, int vocab) {
     __shared__ Best scratch[kSampleThreads / kWave];
-    const int chunk = blockIdx.x;
-    const float* row = logits + static_cast<long>(blockIdx.y) * vocab;
     const int end = (chunk + 1) * kArgmaxChunk < vocab ? (chunk + 1) * kArgmaxChunk : vocab;
     Best mine{0.f, -1};
     for (int i = chunk * kArgmaxChunk + threadIdx.x; i < end; i += kSampleThreads) {
@@ -60,20 +56,48 @@ argmax_partial_kernel(const float* __restrict__ logits, float* __restrict__ part
     }
     const Best total = block_best(mine, scratch);
     if (threadIdx.x == 0) {
-        part_value[blockIdx.y * chunks + chunk] = total.value;
-        part_index[blockIdx.y * chunks + chunk] = total.index;
+        *part_value = total.value;
+        *part_index = total.index;
     }
+}
+// The best of a row's chunks, for every thread.
+__device__ inline int best_of_chunks(const float* __restrict__ part_value, const int* __restrict__ part_index, int chunks) {
+    __shared__ Best scratch[kSampleThreads / kWave];
+    Best mine{0.f, -1};
+    for (int i = threadIdx.x; i < chunks; i += kSampleThreads) mine = better(mine, Best{part_value[i], part_index[i]});
+    return block_best(mine, scratch).index;
+}
+
+__global__ void __launch_bounds__(kSampleThreads)
+argmax_partial_kernel(const float* __restrict__ logits, float* __restrict__ part_value,
+                      int* __restrict__ part_index, int vocab, int chunks) {
+    const long at = static_cast<long>(blockIdx.y) * chunks + blockIdx.x;
+    argmax_of_chunk(logits + static_cast<long>(blockIdx.y) * vocab, blockIdx.x, part_value + at, part_index + at, vocab);
 }
 
 __global__ void __launch_bounds__(kSampleThreads)
 argmax_final_kernel(const float* __restrict__ part_value, const int* __restrict__ part_index,
                     int* __restrict__ out, int chunks) {
-    __shared__ Best scratch[kSampleThreads / kWave];
-    Best mine{0.f, -1};
-    for (int i = threadIdx.x; i < chunks; i += kSampleThreads)
-        mine = better(mine, Best{part_value[blockIdx.x * chunks + i], part_index[blockIdx.x * chunks + i]});
-    const Best total = block_best(mine, scratch);
-    if (threadIdx.x == 0) out[blockIdx.x] = total.index;
+    const long at = static_cast<long>(blockIdx.x) * chunks;
+    const int best = best_of_chunks(part_value + at, part_index + at, chunks);
+    if (threadIdx.x == 0) out[blockIdx.x] = best;
+}
+
+// What one thread does with the elements of an array in turn, until it says no: eight of them are on their way from shared memory at a
+// time, where each would wait out that way by itself (a walk over 64 double sums 3.5 us, so 0.6).
+template <typename T, typename Use>
+__device__ inline void in_turn(const T* of, int n, Use use) {
+    int i = 0;
+    for (; i + 8 <= n; i += 8) {
+        T v[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = of[i + e];
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+            if (!use(i + e, v[e])) return;
+    }
+    for (; i < n; ++i)
+        if (!use(i, of[i])) return;
 }
 
 // Temperature sampling, three steps: the row's highest logit (the two argmax kernels), then the sum of
@@ -99,30 +123,39 @@ __device__ inline void chunk_sums_in_order(const double w[4], double* thread_sum
     __syncthreads();
     if (threadIdx.x % kWave == 0) {
         double sum = 0.0;
-        for (int i = 0; i < kWave; ++i) sum += thread_sum[threadIdx.x + i];
+        in_turn(thread_sum + threadIdx.x, kWave, [&](int, double s) {
+            sum += s;
+            return true;
+        });
         wave_sum[threadIdx.x / kWave] = sum;
     }
     __syncthreads();
 }
 
-__global__ void __launch_bounds__(kSampleThreads)
-temperature_sums_kernel(const float* __restrict__ logits, const double* __restrict__ temperature,
-                        const int* __restrict__ best, double* __restrict__ sums, int vocab, int chunks) {
+__device__ inline void temperature_sum_of_chunk(const float* __restrict__ row, int chunk, double t, int top, double* __restrict__ to, int vocab) {
     __shared__ double thread_sum[kSampleThreads];
     __shared__ double wave_sum[kSampleThreads / kWave];
-    const int r = blockIdx.y, chunk = blockIdx.x;
-    const float* row = logits + static_cast<long>(r) * vocab;
-    const int top = best[r];
-    if (top < 0) return;                                    // no finite logit: the row's answer is -1
-    const double t = temperature[r];
     double w[4];
     chunk_weights(row, vocab, chunk, t, static_cast<double>(row[top]) / t, w);
     chunk_sums_in_order(w, thread_sum, wave_sum);
     if (threadIdx.x == 0) {
         double sum = 0.0;
-        for (int v = 0; v < kSampleThreads / kWave; ++v) sum += wave_sum[v];
-        sums[static_cast<long>(r) * chunks + chunk] = sum;
+        in_turn(wave_sum, kSampleThreads / kWave, [&](int, double v) {
+            sum += v;
+            return true;
+        });
+        *to = sum;
     }
+}
+
+__global__ void __launch_bounds__(kSampleThreads)
+temperature_sums_kernel(const float* __restrict__ logits, const double* __restrict__ temperature,
+                        const int* __restrict__ best, double* __restrict__ sums, int vocab, int chunks) {
+    const int r = blockIdx.y, chunk = blockIdx.x;
+    const int top = best[r];
+    if (top < 0) return;                                    // no finite logit: the row's answer is -1
+    temperature_sum_of_chunk(logits + static_cast<long>(r) * vocab, chunk, temperature[r], top, sums + static_cast<long>(r) * chunks + chunk,
+                             vocab);
 }
 
 // In `sum[0, n)`, walked from the left with `running` as the sum before: the first positive entry that takes
@@ -130,47 +163,44 @@ temperature_sums_kernel(const float* __restrict__ logits, const double* __restri
 __device__ inline int walk_to(const double* sum, int n, double target, double& running) {
     int at = -1;
     double before = running;
-    for (int i = 0; i < n; ++i) {
-        const double s = sum[i];
-        if (!(s > 0.0)) continue;
+    in_turn(sum, n, [&](int i, double s) {
+        if (!(s > 0.0)) return true;
         at = i;
         before = running;
-        if (target < running + s) break;
+        if (target < running + s) return false;
         running += s;
-    }
+        return true;
+    });
     running = before;
     return at;
 }
 
-__global__ void __launch_bounds__(kSampleThreads)
-temperature_pick_kernel(const float* __restrict__ logits, const double* __restrict__ temperature,
-                        const double* __restrict__ uniform, const int* __restrict__ best,
-                        const double* __restrict__ sums, int* __restrict__ out, int vocab, int chunks) {
+// mine: the row's sums of chunks; top: its highest logit.
+__device__ inline void temperature_pick_row(const float* __restrict__ row, double t, double uniform, int top, const double* __restrict__ mine,
+                                            int* __restrict__ out, int vocab, int chunks) {
     __shared__ double thread_sum[kSampleThreads];
     __shared__ double wave_sum[kSampleThreads / kWave];
     __shared__ int chosen_chunk, chosen_thread;
     __shared__ double chosen_before, target;
-    const int r = blockIdx.x;
-    const float* row = logits + static_cast<long>(r) * vocab;
-    const int top = best[r];
     if (top < 0) {
-        if (threadIdx.x == 0) out[r] = -1;
+        if (threadIdx.x == 0) *out = -1;
         return;
     }
-    const double* mine = sums + static_cast<long>(r) * chunks;
     if (threadIdx.x == 0) {
         double total = 0.0;
-        for (int c = 0; c < chunks; ++c) total += mine[c];
-        target = uniform[r] * total;
+        in_turn(mine, chunks, [&](int, double s) {
+            total += s;
+            return true;
+        });
+        target = uniform * total;
         double running = 0.0;
         chosen_chunk = walk_to(mine, chunks, target, running);   // the highest logit weighs 1: some chunk is positive
         chosen_before = running;
-        if (chosen_chunk < 0) out[r] = top;                      // sums that are not numbers (a temperature the host let through)
+        if (chosen_chunk < 0) *out = top;                      // sums that are not numbers (a temperature the host let through)
     }
     __syncthreads();
     const int chunk = chosen_chunk;
     if (chunk < 0) return;
-    const double t = temperature[r];
     double w[4];
     chunk_weights(row, vocab, chunk, t, static_cast<double>(row[top]) / t, w);
     chunk_sums_in_order(w, thread_sum, wave_sum);
@@ -180,14 +210,23 @@ temperature_pick_kernel(const float* __restrict__ logits, const double* __restri
         const int lane = wave < 0 ? -1 : walk_to(thread_sum + wave * kWave, kWave, target, running);
         chosen_thread = lane < 0 ? -1 : wave * kWave + lane;
         chosen_before = running;
-        if (lane < 0) out[r] = top;
+        if (lane < 0) *out = top;
     }
     __syncthreads();
     if (static_cast<int>(threadIdx.x) == chosen_thread) {
         double running = chosen_before;
         const int at = walk_to(w, 4, target, running);
-        out[r] = at < 0 ? top : chunk * kArgmaxChunk + 4 * static_cast<int>(threadIdx.x) + at;
+        *out = at < 0 ? top : chunk * kArgmaxChunk + 4 * static_cast<int>(threadIdx.x) + at;
     }
+}
+
+__global__ void __launch_bounds__(kSampleThreads)
+temperature_pick_kernel(const float* __restrict__ logits, const double* __restrict__ temperature,
+                        const double* __restrict__ uniform, const int* __restrict__ best,
+                        const double* __restrict__ sums, int* __restrict__ out, int vocab, int chunks) {
+    const int r = blockIdx.x;
+    temperature_pick_row(logits + static_cast<long>(r) * vocab, temperature[r], uniform[r], best[r], sums + static_cast<long>(r) * chunks,
+                         out + r, vocab, chunks);
 }
 
 // ---- the best k logits of a row ---------------------------------------------------------------------------
@@ -410,9 +449,7 @@ top_candidates_kernel(const float* __restrict__ logits, int k, float* __restrict
 constexpr int kDrawStages = 8;
 constexpr int kDrawParams = 3 + 2 * kDrawStages;
 
-__global__ void __launch_bounds__(kSampleThreads)
-sample_truncated_kernel(const float* __restrict__ logits, const double* __restrict__ params, int* __restrict__ out,
-                        int vocab) {
+__device__ inline void sample_truncated_row(const float* __restrict__ row, const double* __restrict__ mine, int* __restrict__ out, int vocab) {
     __shared__ __align__(16) unsigned long long keys[kCandidateRoom];
     __shared__ int counters[2];
     __shared__ unsigned long long bound;
@@ -420,20 +457,18 @@ sample_truncated_kernel(const float* __restrict__ logits, const double* __restri
     __shared__ double share[kCandidateMaxK];
     __shared__ double mass;
     __shared__ int keep;
-    const float* row = logits + static_cast<long>(blockIdx.x) * vocab;
-    const double* mine = params + static_cast<long>(blockIdx.x) * kDrawParams;
     // The caller checks the table before it uploads it; whatever the memory holds, the kernel stays in its arrays.
     const int stages = mine[2] >= 1.0 ? (mine[2] < kDrawStages ? static_cast<int>(mine[2]) : kDrawStages) : 0;
     const bool cut = stages > 0 && static_cast<int>(mine[3]) == 0 && mine[4] >= 1.0 && mine[4] <= kCandidateMaxK;
     if (!cut) {
-        if (threadIdx.x == 0) out[blockIdx.x] = -1;
+        if (threadIdx.x == 0) *out = -1;
         return;
     }
     const int k = static_cast<int>(mine[4]);
     const Selection chosen = select_best(row, vocab, k, keys, counters, &bound);
     const int have = chosen.kept;
     if (have == 0) {
-        if (threadIdx.x == 0) out[blockIdx.x] = -1;
+        if (threadIdx.x == 0) *out = -1;
         return;
     }
     const double t = mine[0];
@@ -459,11 +494,12 @@ sample_truncated_kernel(const float* __restrict__ logits, const double* __restri
         if (!(k < chosen.size)) {
             double carry = 0.0;
             total = 0.0;
-            for (int j = 0; j < have; ++j) {
-                const double y = share[by_id[j]] - carry, sum = total + y;
+            in_turn(by_id, have, [&](int, int rank) {
+                const double y = share[rank] - carry, sum = total + y;
                 carry = (sum - total) - y;
                 total = sum;
-            }
+                return true;
+            });
         }
         mass = total;
     }
@@ -482,25 +518,25 @@ sample_truncated_kernel(const float* __restrict__ logits, const double* __restri
                 n = value >= static_cast<double>(kept) ? kept : static_cast<int>(value);
             } else if (kind == 1) {
                 double sum = 0.0;
-                for (int i = 0; i < seen; ++i) {
-                    sum += share[i];
-                    if (sum >= value) {
-                        n = i + 1;
-                        break;
-                    }
-                }
+                in_turn(share, seen, [&](int i, double p) {
+                    sum += p;
+                    if (sum >= value) n = i + 1;
+                    return !(sum >= value);
+                });
             } else {
                 const double floor = value * share[0];
-                for (int i = 0; i < seen; ++i)
-                    if (!(share[i] >= floor)) {
-                        n = i;
-                        break;
-                    }
+                in_turn(share, seen, [&](int i, double p) {
+                    if (!(p >= floor)) n = i;
+                    return p >= floor;
+                });
             }
             n = n < 1 ? 1 : n;
             n = n > have ? have : n;                        // the first stage has cut to what is held, or the row is held whole
             double sum = 0.0;
-            for (int i = 0; i < n; ++i) sum += share[i];
+            in_turn(share, n, [&](int, double p) {
+                sum += p;
+                return true;
+            });
             mass = sum;
             keep = n;
         }
@@ -513,21 +549,74 @@ sample_truncated_kernel(const float* __restrict__ logits, const double* __restri
         __syncthreads();
     }
 
+    // the shares in id order, of those that are kept, for the walk
+    __shared__ double in_id_order[kCandidateMaxK];
+    if (static_cast<int>(threadIdx.x) < have) in_id_order[threadIdx.x] = by_id[threadIdx.x] < kept ? share[by_id[threadIdx.x]] : 0.0;
+    __syncthreads();
     if (threadIdx.x == 0) {
         const double u = mine[1];
         double running = 0.0;
-        int token = -1;
-        for (int j = 0; j < have; ++j) {
-            const int rank = by_id[j];
-            if (rank >= kept) continue;
-            const double p = share[rank];
-            if (!(p > 0.0)) continue;
-            token = candidate_id(keys[rank]);
+        int last = -1;
+        in_turn(in_id_order, have, [&](int j, double p) {
+            if (!(p > 0.0)) return true;
+            last = j;
             running += p;
-            if (u < running) break;
-        }
-        out[blockIdx.x] = token;
+            return !(u < running);
+        });
+        *out = last < 0 ? -1 : candidate_id(keys[by_id[last]]);
     }
+}
+
+__global__ void __launch_bounds__(kSampleThreads)
+sample_truncated_kernel(const float* __restrict__ logits, const double* __restrict__ params, int* __restrict__ out,
+                        int vocab) {
+    sample_truncated_row(logits + static_cast<long>(blockIdx.x) * vocab, params + static_cast<long>(blockIdx.x) * kDrawParams, out + blockIdx.x,
+                         vocab);
+}
+
+// ---- rows of different kinds in one call ------------------------------------------------------------------
+//
+// A batch whose rows are chosen in different ways takes three launches: the best of the chunks; the rows' best (the answer of a greedy
+// row) and the sums of the chunks; the draws, of both kinds side by side.  Each row is worked on by what its kind needs and nothing
+// else.  (Every kind's kernels over all rows, one behind the other, and a selection between their answers were nine launches: five
+// rows of three kinds over 32,768 logits 68 us, so 40.)
+enum ChoiceKind : int { kGreedyRow = 0, kTemperatureRow = 1, kTruncatedRow = 2 };
+__device__ inline int kind_of(const double* kinds, int row) { return static_cast<int>(kinds[row]); }
+
+__global__ void __launch_bounds__(kSampleThreads)
+choose_partial_kernel(const float* __restrict__ logits, const double* __restrict__ kinds, float* __restrict__ part_value,
+                      int* __restrict__ part_index, int vocab, int chunks) {
+    if (kind_of(kinds, blockIdx.y) == kTruncatedRow) return;
+    const long at = static_cast<long>(blockIdx.y) * chunks + blockIdx.x;
+    argmax_of_chunk(logits + static_cast<long>(blockIdx.y) * vocab, blockIdx.x, part_value + at, part_index + at, vocab);
+}
+
+__global__ void __launch_bounds__(kSampleThreads)
+choose_sums_kernel(const float* __restrict__ logits, const double* __restrict__ kinds, const double* __restrict__ temperature,
+                   const float* __restrict__ part_value, const int* __restrict__ part_index, int* __restrict__ best,
+                   double* __restrict__ sums, int* __restrict__ out, int vocab, int chunks) {
+    const int r = blockIdx.y, kind = kind_of(kinds, r);
+    if (kind == kTruncatedRow || (kind == kGreedyRow && blockIdx.x != 0)) return;
+    const long at = static_cast<long>(r) * chunks;
+    const int top = best_of_chunks(part_value + at, part_index + at, chunks);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        best[r] = top;
+        if (kind == kGreedyRow) out[r] = top;
+    }
+    if (kind == kGreedyRow || top < 0) return;
+    temperature_sum_of_chunk(logits + static_cast<long>(r) * vocab, blockIdx.x, temperature[r], top, sums + at + blockIdx.x, vocab);
+}
+
+__global__ void __launch_bounds__(kSampleThreads)
+choose_draw_kernel(const float* __restrict__ logits, const double* __restrict__ kinds, const double* __restrict__ temperature,
+                   const double* __restrict__ uniform, const double* __restrict__ params, const int* __restrict__ best,
+                   const double* __restrict__ sums, int* __restrict__ out, int vocab, int chunks) {
+    const int r = blockIdx.x, kind = kind_of(kinds, r);
+    const float* row = logits + static_cast<long>(r) * vocab;
+    if (kind == kTemperatureRow)
+        temperature_pick_row(row, temperature[r], uniform[r], best[r], sums + static_cast<long>(r) * chunks, out + r, vocab, chunks);
+    else if (kind == kTruncatedRow)
+        sample_truncated_row(row, params + static_cast<long>(r) * kDrawParams, out + r, vocab);
 }
 
 }  // namespace leone
@@ -662,5 +751,41 @@ extern "C" int leone_sample_temperature(const float* logits, const double* tempe
     LEONE_LAUNCH_CHECK("sample_temperature");
     temperature_pick_kernel<<<rows, kSampleThreads, 0, stream>>>(logits, temperature, uniform, best, sums, out, vocab, chunks);
     LEONE_LAUNCH_CHECK("sample_temperature");
+    return 0;
+}
+
+// How many doubles leone_choose_tokens needs beside its arguments.
+extern "C" long leone_choose_workspace(int rows, int vocab) {
+    const long chunks = ceil_div(vocab, kArgmaxChunk);
+    return 2 * rows * chunks + (rows + 1) / 2;
+}
+
+// A token for every row by its kind: 0 the highest logit (leone_argmax), 1 by temperature[row] and uniform[row]
+// (leone_sample_temperature), 2 by params (leone_sample_truncated).  temperature and uniform, or params, may be null if no row is of
+// their kind (`of_kinds`: the kinds that occur, bit 1 << kind).  work: leone_choose_workspace(rows, vocab) doubles.
+extern "C" int leone_choose_tokens(const float* logits, const double* kinds, int of_kinds, const double* temperature, const double* uniform,
+                                   const double* params, int* out, double* work, int rows, int vocab, hipStream_t stream) {
+    LEONE_REQUIRE(logits && kinds && out && work, "choose_tokens: null pointer");
+    LEONE_REQUIRE(of_kinds > 0 && of_kinds < 8, "choose_tokens: kinds %d", of_kinds);
+    LEONE_REQUIRE(!(of_kinds & (1 << kTemperatureRow)) || (temperature && uniform), "choose_tokens: rows by temperature need theirs");
+    LEONE_REQUIRE(!(of_kinds & (1 << kTruncatedRow)) || params, "choose_tokens: rows with truncation stages need theirs");
+    LEONE_REQUIRE(rows > 0 && rows <= 65535 && vocab > 0 && vocab <= (1 << 30), "choose_tokens: rows %d vocab %d out of range", rows, vocab);
+    const int chunks = ceil_div(vocab, kArgmaxChunk);
+    const long places = static_cast<long>(rows) * chunks;
+    double* sums = work;
+    float* part_value = reinterpret_cast<float*>(work + places);
+    int* part_index = reinterpret_cast<int*>(part_value + places);
+    int* best = part_index + places;
+    if (of_kinds != 1 << kTruncatedRow) {
+        choose_partial_kernel<<<dim3(chunks, rows), kSampleThreads, 0, stream>>>(logits, kinds, part_value, part_index, vocab, chunks);
+        LEONE_LAUNCH_CHECK("choose_tokens");
+        choose_sums_kernel<<<dim3(chunks, rows), kSampleThreads, 0, stream>>>(logits, kinds, temperature, part_value, part_index, best, sums, out,
+                                                                             vocab, chunks);
+        LEONE_LAUNCH_CHECK("choose_tokens");
+    }
+    if (of_kinds != 1 << kGreedyRow) {
+        choose_draw_kernel<<<rows, kSampleThreads, 0, stream>>>(logits, kinds, temperature, uniform, params, best, sums, out, vocab, chunks);
+        LEONE_LAUNCH_CHECK("choose_tokens");
+    }
     return 0;
 }

@@ -73,7 +73,7 @@ def device_kind(policy: SamplingParams) -> Optional[str]:
 class DeviceChoice:
     """What the device kernels need to choose a step's tokens, uploaded before the step's logits exist (so that
     the upload does not stand between the step and the kernels that choose): temperatures and uniform values, the
-    table of truncation stages, and which kernel's answer each row takes.  ``kinds`` holds for every sampled row
+    table of truncation stages, and each row's kind.  ``kinds`` holds for every sampled row
     its ``device_kind`` or None; rows with None get nothing of meaning."""
 
     def __init__(self, rows: Sequence[PlannedEntry], policies: Sequence[SamplingParams],
@@ -92,12 +92,11 @@ class DeviceChoice:
         if "truncated" in kinds:
             pieces.append(ops.truncated_rows([(p.temperature, u, p.truncations) if kind == "truncated" else None
                                               for p, u, kind in zip(policies, draws, kinds)]).reshape(-1))
-        # which rows take the answer of the second and third kernel (a batch of one kind needs none)
-        self.names = [name for name in ("greedy", "temperature", "truncated") if name in kinds]
-        for name in self.names[1:]:
-            pieces.append(np.array([1.0 if kind == name else 0.0 for kind in kinds], dtype=np.float64))
-        self.scaled = self.truncated = None
-        self.masks = {}
+        # which rows are of which kind (a batch of one kind needs no list)
+        self.names = [name for name in ops.CHOICE_KINDS if name in kinds]
+        if len(self.names) > 1:
+            pieces.append(np.array([ops.CHOICE_KINDS.get(kind, 0) for kind in kinds], dtype=np.float64))
+        self.scaled = self.truncated = self.codes = None
         if pieces:
             flat = np.concatenate(pieces)
             if staging is not None:
@@ -114,23 +113,19 @@ class DeviceChoice:
                 width = 3 + 2 * ops.TRUNCATED_STAGES
                 self.truncated = on_device[at:at + count * width].view(count, width)
                 at += count * width
-            for name in self.names[1:]:
-                self.masks[name] = on_device[at:at + count] != 0.0
-                at += count
+            if len(self.names) > 1:
+                self.codes = on_device[at:at + count]
 
     def choose(self, logits: torch.Tensor) -> torch.Tensor:
-        """int32 [rows] on the device: the token each row's kernel chose, -1 for a row without a finite logit.
-        Each kernel runs once, over all rows."""
-        out = None
-        for name in self.names:
-            if name == "greedy":
-                chosen = ops.argmax(logits)
-            elif name == "temperature":
-                chosen = ops.sample_temperature(logits, self.scaled[0], self.scaled[1])
-            else:
-                chosen = ops.sample_truncated(logits, self.truncated)
-            out = chosen if out is None else torch.where(self.masks[name], chosen, out)
-        return out
+        """int32 [rows] on the device: the token each row's kernel chose, -1 for a row without a finite logit; None if no row is
+        chosen here."""
+        if len(self.names) > 1:
+            return ops.choose_tokens(logits, self.codes, self.names, self.scaled, self.truncated)
+        if "temperature" in self.names:
+            return ops.sample_temperature(logits, self.scaled[0], self.scaled[1])
+        if "truncated" in self.names:
+            return ops.sample_truncated(logits, self.truncated)
+        return ops.argmax(logits) if self.names else None
 
 
 def plan_device_choice(entries: Sequence[PlannedEntry], params: Dict[Hashable, SamplingParams], device,

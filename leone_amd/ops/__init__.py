@@ -1363,6 +1363,27 @@ def sample_truncated(logits: torch.Tensor, draws) -> torch.Tensor:
     return out
 
 
+CHOICE_KINDS = {"greedy": 0, "temperature": 1, "truncated": 2}
+
+
+def choose_tokens(logits: torch.Tensor, kinds: torch.Tensor, names, scaled: Optional[torch.Tensor] = None,
+                  params: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """One token a row (int32 on the device), every row by its own kind, in one call: what ``argmax``, ``sample_temperature`` and
+    ``sample_truncated`` would give it.  ``kinds`` float64 [rows] on the device holds ``CHOICE_KINDS``, ``names`` says which occur,
+    ``scaled`` float64 [2, rows] temperatures and uniform values, ``params`` the table of ``truncated_table``."""
+    rows, vocab = logits.shape
+    library_, of_kinds = library(), sum(1 << CHOICE_KINDS[name] for name in names)
+    if params is not None and params.shape != (rows, 3 + 2 * TRUNCATED_STAGES):
+        raise KernelError(f"choose_tokens: {rows} rows of logits, a table of {tuple(params.shape)}")
+    out = torch.empty((rows,), dtype=torch.int32, device=logits.device)
+    work = torch.empty((library_.leone_choose_workspace(rows, vocab),), dtype=torch.float64, device=logits.device)
+    at = _dev(scaled, "choose scaled", torch.float64, (2, rows))
+    call("leone_choose_tokens", _dev(logits, "choose logits", torch.float32), _dev(kinds, "choose kinds", torch.float64, (rows,)), of_kinds,
+         at, at + 8 * rows if at else 0, _dev(params, "choose stages", torch.float64), _dev(out, "choose out"), _dev(work, "choose workspace"),
+         rows, vocab, _stream())
+    return out
+
+
 __all__ = [name for name in dir() if not name.startswith("_")]
 
 

@@ -55,6 +55,7 @@ _PROTOTYPES = {
     "leone_sample_temperature": [P, P, P, P, P, P, P, P, c_int, c_int, P],
     "leone_top_candidates": [P, P, P, P, c_int, c_int, c_int, P],
     "leone_sample_truncated": [P, P, P, c_int, c_int, P],
+    "leone_choose_tokens": [P, P, c_int, P, P, P, P, P, c_int, c_int, P],
     "leone_add_layernorm": [P, P, P, P, c_float, P, P, c_int, c_float, P, c_int, P, c_int, c_int, P, c_int, c_int, P, c_int,
                             P, P, P, P],
     "leone_entry_spans": [P, P, P, c_int, P, P],
@@ -185,6 +186,8 @@ def library() -> ctypes.CDLL:
             lib.leone_sample_truncated_stages.argtypes = []
             lib.leone_sample_truncated_params.restype = c_int
             lib.leone_sample_truncated_params.argtypes = []
+            lib.leone_choose_workspace.restype = ctypes.c_long
+            lib.leone_choose_workspace.argtypes = [c_int, c_int]
             lib.leone_peak_mfma_flops.restype = ctypes.c_double
             lib.leone_peak_mfma_flops.argtypes = [c_int, c_int]
             lib.leone_chunk_rows.restype = c_int

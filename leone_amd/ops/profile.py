@@ -35,6 +35,7 @@ OPERATIONS = {
     "leone_swiglu": "swiglu",
     "leone_argmax": "argmax",
     "leone_sample_temperature": "sample",
+    "leone_choose_tokens": "sample",
     "leone_top_candidates": "sample",
     "leone_add_layernorm": "layer norm",
     "leone_entry_spans": "entry spans",

@@ -517,3 +517,25 @@ def test_command_line_eval_and_doctor(folders, tmp_path):
                             capture_output=True, text=True, timeout=300)
     assert doctor.returncode == 0, doctor.stdout + doctor.stderr
     assert "Qwen3ForCausalLM" in doctor.stdout and "tensor names and shapes: ok" in doctor.stdout
+
+
+@pytest.mark.parametrize("vocab", [1, 50, 4096, 4097, 32768, 151936])
+@pytest.mark.parametrize("names", [("greedy", "temperature"), ("greedy", "truncated"), ("temperature", "truncated"), ("greedy", "temperature", "truncated")])
+def test_rows_of_different_kinds_in_one_call(vocab, names):
+    """Every row's token is the one its own kind's kernel gives it, whoever is beside it; also for a row without a finite logit."""
+    from leone_amd import ops
+    gen = np.random.default_rng(vocab)
+    rows = 7
+    logits = (gen.standard_normal((rows, vocab)) * 3).astype(np.float32)
+    logits[2], logits[3, ::2] = np.nan, np.inf
+    logits = torch.from_numpy(logits).cuda()
+    scaled = torch.from_numpy(np.stack([gen.uniform(0.3, 2.0, rows), gen.random(rows)])).cuda()
+    draws = [(0.8, float(gen.random()), [("top_k", float(k)), ("top_p", 0.9), ("min_p", 0.02)]) for k in (1, 40, 40, 256, 9, 64, 5)]
+    table = ops.truncated_table(draws, "cuda")
+    alone = {"greedy": ops.argmax(logits), "temperature": ops.sample_temperature(logits, scaled[0], scaled[1]),
+             "truncated": ops.sample_truncated(logits, table)}
+    for shift in range(3):
+        kinds = [names[(r + shift) % len(names)] for r in range(rows)]
+        codes = torch.tensor([float(ops.CHOICE_KINDS[kind]) for kind in kinds], dtype=torch.float64, device="cuda")
+        got = ops.choose_tokens(logits, codes, names, scaled if "temperature" in names else None, table if "truncated" in names else None)
+        assert got.tolist() == [int(alone[kind][r]) for r, kind in enumerate(kinds)]
