@@ -753,6 +753,48 @@ attention_reduce_kernel(const float* __restrict__ part_acc, const float* __restr
     __shared__ float wave_top[kReduceThreads / kWave];
     const long rh = blockIdx.x;                      // row * q_heads + head
     const float* ml = part_ml + rh * splits * 2;
+    if constexpr (!kShaped) {
+        // Up to 64 splits: a lane of each wave has one's maximum and sum, and they are handed on by lane; eight partial results are on
+        // their way before those are known, and the next eight while they are added.  (By shared memory and two barriers, with a trip
+        // to memory a split: eight decode steps of one request with 17 splits 5.83 ms, so 5.70; of eight requests with 4, 8.52 and 8.45.)
+        if (splits <= kWave) {
+            const int lane = threadIdx.x % kWave;
+            constexpr int kAhead = 8;
+            const int own = lane < splits ? lane : splits - 1;
+            const float own_top = ml[2 * own], own_sum = ml[2 * own + 1];
+            // (every lane takes part in what is handed on, also those past the head's end)
+            for (int d0 = 0; d0 < head_dim; d0 += kReduceThreads) {
+                const int d = d0 + threadIdx.x;
+                const float* from = part_acc + rh * splits * head_dim + (d < head_dim ? d : head_dim - 1);
+                const auto part = [&](int s) { return from[static_cast<long>(s < splits ? s : splits - 1) * head_dim]; };
+                float v[kAhead];
+#pragma unroll
+                for (int u = 0; u < kAhead; ++u) v[u] = part(u);
+                const float top = wave_max(own_top);
+                const float mine = own_top == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(own_top - top);
+                const auto weight_of = [&](int s) { return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(mine), s)); };
+                float den = 0.f, num = 0.f;
+                for (int s0 = 0; s0 < splits; s0 += kAhead) {
+                    float next[kAhead];
+                    if (s0 + kAhead < splits) {
+#pragma unroll
+                        for (int u = 0; u < kAhead; ++u) next[u] = part(s0 + kAhead + u);
+                    }
+#pragma unroll
+                    for (int u = 0; u < kAhead; ++u)
+                        if (s0 + u < splits) {
+                            const float w = weight_of(s0 + u);
+                            den += __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(own_sum), s0 + u)) * w;
+                            num += v[u] * w;
+                        }
+#pragma unroll
+                    for (int u = 0; u < kAhead; ++u) v[u] = next[u];
+                }
+                if (d < head_dim) out[rh * head_dim + d] = from_float<bf16_t>(num / den * gate.factor(rh, d, head_dim, q_heads));
+            }
+            return;
+        }
+    }
     float top = -INFINITY;
     for (int s = threadIdx.x; s < splits; s += kReduceThreads) top = fmaxf(top, ml[2 * s]);
     top = wave_max(top);
