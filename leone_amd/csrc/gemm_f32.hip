@@ -701,8 +701,9 @@ extern "C" int leone_gemm_f32(const float* a, const float* b, float* c, float* p
 extern "C" int leone_gemm_f32_glu_fits(int n, int k) { return n > 0 && n % 16 == 0 && k >= kStreamK; }
 
 // C[M, N / 2] = act(gate) * up of the same product, B's rows being eight gates, their eight ups, and so on (act, limit: as leone_glu).
-// The bits are those of the product and leone_glu behind it; one launch and the product's way to memory and back are saved (us, before
-// and with it: one row against 12288 x 2048 23.4 and 18.9; 777 rows 255 and 240).
+// The bits are those of the product and leone_glu behind it; one launch and the product's way to memory and back are saved (us, two launches
+// and one: one row against 12288 x 2048 22.7 and 20.5, five against 3072 x 512 7.0 and 4.2, 200 20.6 and 18.6, 777 against 12288 x 2048
+// 271 and 264).
 extern "C" int leone_gemm_f32_glu(const float* a, const float* b, float* c, float* planes, int m, int n, int k, int act, float limit,
                                   hipStream_t stream) {
     LEONE_REQUIRE(a && b && c, "gemm_f32_glu: null pointer");

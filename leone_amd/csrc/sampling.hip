@@ -84,7 +84,7 @@ argmax_final_kernel(const float* __restrict__ part_value, const int* __restrict_
 }
 
 // What one thread does with the elements of an array in turn, until it says no: eight of them are on their way from shared memory at a
-// time, where each would wait out that way by itself (a walk over 64 double sums 3.5 us, so 0.6).
+// time, where each would wait out that way by itself (temperature sampling of five rows of 32,768 26.5 us, so 21.6).
 template <typename T, typename Use>
 __device__ inline void in_turn(const T* of, int n, Use use) {
     int i = 0;
@@ -579,7 +579,7 @@ sample_truncated_kernel(const float* __restrict__ logits, const double* __restri
 // A batch whose rows are chosen in different ways takes three launches: the best of the chunks; the rows' best (the answer of a greedy
 // row) and the sums of the chunks; the draws, of both kinds side by side.  Each row is worked on by what its kind needs and nothing
 // else.  (Every kind's kernels over all rows, one behind the other, and a selection between their answers were nine launches: five
-// rows of three kinds over 32,768 logits 68 us, so 40.)
+// rows of three kinds over 32,768 logits 65 us, so 34.5.)
 enum ChoiceKind : int { kGreedyRow = 0, kTemperatureRow = 1, kTruncatedRow = 2 };
 __device__ inline int kind_of(const double* kinds, int row) { return static_cast<int>(kinds[row]); }
 
