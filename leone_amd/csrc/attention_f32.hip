@@ -346,7 +346,7 @@ void launch_attention_f32(const float* q, float* out, const float* k_pool, const
     const long multiples = ceil_div(rows, most);
     const int page_shift = (page_tokens & (page_tokens - 1)) == 0 ? __builtin_ctz(page_tokens) : -1;
     const AttentionF32Args args{q, out, k_pool, v_pool, positions, row_entry, block_table, max_blocks, rows, q_heads, kv_heads,
-                                group, most, multiples > 1 && multiples * rows < 1l << 32 ? static_cast<unsigned>(((1ull << 32) + multiples - 1) / multiples) : 0u,
+                                group, most, multiples > 1 && multiples * (rows + kQueries) < 1l << 32 ? static_cast<unsigned>(((1ull << 32) + multiples - 1) / multiples) : 0u,
                                 page_tokens, page_shift, scale, window, gate, gate_stride, keep_first, gate_each, slopes, temp_coef, temp_every,
                                 shape, chunk};
     const dim3 grid(ceil_div(rows, most) * most, kv_heads);
