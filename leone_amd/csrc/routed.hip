@@ -58,7 +58,8 @@ struct RouteRule {
 // each read from its lane by one instruction.  Scores are compared as integers in the order of the floats, so that what is
 // not a number has a place too and every rank is some lane's.  Returns the lane's place among the winners, `top` and more if
 // it is none of them.  (Winner after winner by exchanges over the wave, a dozen of them each, and the tiles' places by one thread, the
-// choice and the plan of 8 rows over 35 outputs in 7 groups took 18.5 us; now 7.6.)
+// choice and the plan of 8 rows over 35 outputs in 7 groups took 18.5 us; by ranks 6.6, recorded one behind the other; what
+// route_plan_kernel says of its waits made it 5.4.)
 __device__ inline unsigned route_order(float v) {
     const unsigned bits = __float_as_uint(v + 0.0f);           // -0 counts as 0
     return bits & 0x80000000u ? ~bits : bits | 0x80000000u;
@@ -90,11 +91,18 @@ __device__ inline int route_rank(float choice, int lane, int total, int group_co
 template <int kSlots>
 __device__ inline void route_row(int row, int lane, const float* __restrict__ logits, const AnyVec& correction,
                                  int* __restrict__ chosen, float* __restrict__ weight, int total, int top, int group_count,
-                                 int group_keep, const RouteRule rule, int shift_from = 0x7fffffff, int always = 0) {
+                                 int group_keep, const RouteRule rule, int shift_from = 0x7fffffff, int always = 0,
+                                 int* here = nullptr, int room = 0) {
     // `always` experts that every row takes with weight 1 stand behind the routed ones in the matrices (indices
     // shift_from .. shift_from + always - 1): a row's places are its `top` choices and then these; a chosen router
     // output from shift_from on (one that hands the row on) is numbered behind them.
+    // here: a second copy of the first `room` choices of all rows, for the workgroup's own use.
     const int places = top + always;
+    const auto choose = [&](int place, int e) {
+        const long at = static_cast<long>(row) * places + place;
+        chosen[at] = e;
+        if (at < room) here[at] = e;
+    };
     const float* z = logits + static_cast<long>(row) * total;
     float s[kSlots], choice[kSlots];
     bool taken[kSlots];
@@ -103,7 +111,12 @@ __device__ inline void route_row(int row, int lane, const float* __restrict__ lo
     for (int i = 0; i < kSlots; ++i) {
         const int e = lane + i * kWave;
         s[i] = e < total ? z[e] : -INFINITY;
-        top_z = fmaxf(top_z, s[i]);
+        if constexpr (kSlots > 1) top_z = fmaxf(top_z, s[i]);
+    }
+    float early = 0.f;                                     // one output a lane: the correction on its way together with the logits
+    if constexpr (kSlots == 1) {
+        early = lane < total && correction.ptr ? load_any(correction, lane) : 0.f;
+        top_z = fmaxf(top_z, s[0]);
     }
     top_z = wave_max(top_z);
     float sum = 0.f;
@@ -119,7 +132,7 @@ __device__ inline void route_row(int row, int lane, const float* __restrict__ lo
     for (int i = 0; i < kSlots; ++i) {
         const int e = lane + i * kWave;
         s[i] = s[i] / sum;
-        choice[i] = e < total ? s[i] + (correction.ptr ? load_any(correction, e) : 0.f) : -INFINITY;
+        choice[i] = e < total ? s[i] + (kSlots == 1 ? early : correction.ptr ? load_any(correction, e) : 0.f) : -INFINITY;
         taken[i] = e >= total;
     }
     if (kSlots == 1 && (group_count == 1 || rule.group_best == 1)) {
@@ -129,15 +142,15 @@ __device__ inline void route_row(int row, int lane, const float* __restrict__ lo
         float picked = 0.f;
         for (int i = 0; i < top; ++i) {
             const unsigned long long who = __ballot(rank == i);
-            picked += __shfl(s[0], __ffsll(who) - 1, kWave);
+            picked += __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(s[0]), __ffsll(who) - 1));
         }
         const float by = rule.renorm ? picked + 1e-20f : 1.0f;
         if (won) {
-            chosen[static_cast<long>(row) * places + rank] = lane >= shift_from ? lane + always : lane;
+            choose(rank, lane >= shift_from ? lane + always : lane);
             weight[static_cast<long>(row) * places + rank] = s[0] / by * rule.scale;
         }
         for (int i = lane; i < always; i += kWave) {
-            chosen[static_cast<long>(row) * places + top + i] = shift_from + i;
+            choose(top + i, shift_from + i);
             weight[static_cast<long>(row) * places + top + i] = 1.0f;
         }
         return;
@@ -239,39 +252,42 @@ __device__ inline void route_row(int row, int lane, const float* __restrict__ lo
             my_e = at;
         }
         if (n >= kWave && lane == 0) {       // more than 64 places: written as they come, scaled below
-            chosen[static_cast<long>(row) * places + n] = at >= shift_from ? at + always : at;
+            choose(n, at >= shift_from ? at + always : at);
             weight[static_cast<long>(row) * places + n] = got;
         }
     }
     const float denom = rule.renorm ? picked_sum + 1e-20f : 1.0f;
     if (lane < top && lane < kWave) {
-        chosen[static_cast<long>(row) * places + lane] = my_e >= shift_from ? my_e + always : my_e;
+        choose(lane, my_e >= shift_from ? my_e + always : my_e);
         weight[static_cast<long>(row) * places + lane] = my_s / denom * rule.scale;
     }
     if (top > kWave && lane == 0)
         for (int n = kWave; n < top; ++n)
             weight[static_cast<long>(row) * places + n] = weight[static_cast<long>(row) * places + n] / denom * rule.scale;
     for (int i = lane; i < always; i += kWave) {
-        chosen[static_cast<long>(row) * places + top + i] = shift_from + i;
+        choose(top + i, shift_from + i);
         weight[static_cast<long>(row) * places + top + i] = 1.0f;
     }
 }
 
+template <int kSlots>
 __global__ void __launch_bounds__(kWave)
 route_topk_kernel(const float* __restrict__ logits, AnyVec correction, int* __restrict__ chosen, float* __restrict__ weight,
                   int total, int top, int group_count, int group_keep, RouteRule rule) {
-    if (total <= kWave) route_row<1>(blockIdx.x, threadIdx.x, logits, correction, chosen, weight, total, top, group_count, group_keep, rule);
-    else if (total <= 2 * kWave) route_row<2>(blockIdx.x, threadIdx.x, logits, correction, chosen, weight, total, top, group_count, group_keep, rule);
-    else route_row<kRouteSlots>(blockIdx.x, threadIdx.x, logits, correction, chosen, weight, total, top, group_count, group_keep, rule);
+    route_row<kSlots>(blockIdx.x, threadIdx.x, logits, correction, chosen, weight, total, top, group_count, group_keep, rule);
 }
 
-// One workgroup.  counts and places live in shared memory (experts <= 1024).
-__device__ inline void plan_tiles(const int* __restrict__ chosen, int pairs, int experts, int* __restrict__ tile_expert,
+// One workgroup.  counts and places live in shared memory (experts <= 1024).  clear_tiles, the choices, a barrier, plan_tiles.
+__device__ inline void clear_tiles(int experts, int* __restrict__ tile_expert, int* __restrict__ tile_pairs, int max_tiles, int tile,
+                                   int* count, int first_thread = 0) {
+    const int mine = threadIdx.x - first_thread, all = blockDim.x - first_thread;
+    for (int e = mine; e < experts; e += all) count[e] = 0;
+    for (int t = mine; t < max_tiles; t += all) tile_expert[t] = -1;
+    for (long i = mine; i < static_cast<long>(max_tiles) * tile; i += all) tile_pairs[i] = -1;
+}
+
+__device__ inline void plan_tiles(const int* chosen, int pairs, int experts, int* __restrict__ tile_expert,
                                   int* __restrict__ tile_pairs, int max_tiles, int tile, int* count, int* first_tile) {
-    for (int e = threadIdx.x; e < experts; e += blockDim.x) count[e] = 0;
-    for (int t = threadIdx.x; t < max_tiles; t += blockDim.x) tile_expert[t] = -1;
-    for (long i = threadIdx.x; i < static_cast<long>(max_tiles) * tile; i += blockDim.x) tile_pairs[i] = -1;
-    __syncthreads();
     for (int p = threadIdx.x; p < pairs; p += blockDim.x) {
         const int e = chosen[p];
         if (e >= 0 && e < experts) atomicAdd(&count[e], 1);
@@ -314,25 +330,38 @@ moe_plan_kernel(const int* __restrict__ chosen, int pairs, int experts, int* __r
                 int* __restrict__ tile_pairs, int max_tiles, int tile) {
     __shared__ int count[1024];
     __shared__ int first_tile[1024];
+    clear_tiles(experts, tile_expert, tile_pairs, max_tiles, tile, count);
+    __syncthreads();
     plan_tiles(chosen, pairs, experts, tile_expert, tile_pairs, max_tiles, tile, count, first_tile);
 }
 
-// The router's choice and the tiles in one launch, for steps of few rows (a wave a row, 16 waves in turn).
+// The router's choice and the tiles in one launch, for steps of few rows (a wave a row, 16 waves in turn).  One workgroup and so
+// bound by its chain of waits: the waves without a row clear the tiles meanwhile (a wave with one would wait for its stores along with
+// its logits), and the choices are handed to the plan through shared memory (kPlanPairs of them; more are read back from where
+// they were written).  kSlots: outputs a lane; each number is a kernel of its own, without the others' registers.  One behind the
+// other in a recording: 8 rows over 64 outputs 7.5 -> 6.1 us, 64 rows over 64 in 8 groups 28.4 -> 26.0, 64 over 256 (4 outputs a lane,
+// not 8) 47.7 -> 36.5; over 512, where the copy in shared memory gave nothing and is not made, 49.8 -> 50.7.
+constexpr int kPlanPairs = 2048;
+
+template <int kSlots>
 __global__ void __launch_bounds__(1024)
 route_plan_kernel(const float* __restrict__ logits, AnyVec correction, int* __restrict__ chosen, float* __restrict__ weight,
                   int rows, int total, int top, int group_count, int group_keep, int experts, int* __restrict__ tile_expert,
                   int* __restrict__ tile_pairs, int max_tiles, int tile, int always, RouteRule rule) {
+    constexpr int kWaves = 1024 / kWave;
     const int routed = experts - always;               // experts the router chooses among; the others every row takes
     __shared__ int count[1024];
     __shared__ int first_tile[1024];
-    for (int row = threadIdx.x / kWave; row < rows; row += 1024 / kWave) {
-        const int lane = threadIdx.x % kWave;
-        if (total <= kWave) route_row<1>(row, lane, logits, correction, chosen, weight, total, top, group_count, group_keep, rule, routed, always);
-        else if (total <= 2 * kWave) route_row<2>(row, lane, logits, correction, chosen, weight, total, top, group_count, group_keep, rule, routed, always);
-        else route_row<kRouteSlots>(row, lane, logits, correction, chosen, weight, total, top, group_count, group_keep, rule, routed, always);
-    }
+    __shared__ int here[kPlanPairs];
+    const int pairs = rows * (top + always), room = kSlots < kRouteSlots && pairs <= kPlanPairs ? pairs : 0;
+    const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    for (int row = wave; row < rows; row += kWaves)
+        route_row<kSlots>(row, lane, logits, correction, chosen, weight, total, top, group_count, group_keep, rule, routed, always, here, room);
+    if (rows >= kWaves) clear_tiles(experts, tile_expert, tile_pairs, max_tiles, tile, count);
+    else if (wave >= rows) clear_tiles(experts, tile_expert, tile_pairs, max_tiles, tile, count, rows * kWave);
     __syncthreads();                                   // the choices are written; the same workgroup reads them
-    plan_tiles(chosen, rows * (top + always), experts, tile_expert, tile_pairs, max_tiles, tile, count, first_tile);
+    if (room > 0) plan_tiles(here, pairs, experts, tile_expert, tile_pairs, max_tiles, tile, count, first_tile);
+    else plan_tiles(chosen, pairs, experts, tile_expert, tile_pairs, max_tiles, tile, count, first_tile);
 }
 
 template <typename T>
@@ -975,8 +1004,10 @@ extern "C" int leone_route_topk(const float* logits, const void* correction, int
     LEONE_REQUIRE(!correction || correction_dtype == kF32 || correction_dtype == kBF16, "route_topk: unknown type of the correction");
     LEONE_REQUIRE(group_count >= 1 && total % group_count == 0 && group_keep >= 1 && group_keep <= group_count,
                   "route_topk: %d groups (dividing %d outputs), %d kept", group_count, total, group_keep);
-    route_topk_kernel<<<rows, kWave, 0, stream>>>(logits, AnyVec{correction, correction_dtype}, chosen, weight, total, top,
-                                                  group_count, group_keep, RouteRule{score, group_best, renorm, weight_scale});
+    const auto kernel = total <= kWave ? route_topk_kernel<1> : total <= 2 * kWave ? route_topk_kernel<2>
+                        : total <= 4 * kWave ? route_topk_kernel<4> : route_topk_kernel<kRouteSlots>;
+    kernel<<<rows, kWave, 0, stream>>>(logits, AnyVec{correction, correction_dtype}, chosen, weight, total, top, group_count, group_keep,
+                                       RouteRule{score, group_best, renorm, weight_scale});
     LEONE_LAUNCH_CHECK("route_topk");
     return 0;
 }
@@ -1005,9 +1036,10 @@ extern "C" int leone_route_plan(const float* logits, const void* correction, int
     const long needed = pairs / tile + experts;
     LEONE_REQUIRE(max_tiles >= (needed < pairs ? needed : pairs), "route_plan: %d tiles cannot hold %ld pairs of %d experts", max_tiles,
                   pairs, experts);
-    route_plan_kernel<<<1, 1024, 0, stream>>>(logits, AnyVec{correction, correction_dtype}, chosen, weight, rows, total, top,
-                                              group_count, group_keep, experts, tile_expert, tile_pairs, max_tiles, tile, always,
-                                              RouteRule{score, group_best, renorm, weight_scale});
+    const auto kernel = total <= kWave ? route_plan_kernel<1> : total <= 2 * kWave ? route_plan_kernel<2>
+                        : total <= 4 * kWave ? route_plan_kernel<4> : route_plan_kernel<kRouteSlots>;
+    kernel<<<1, 1024, 0, stream>>>(logits, AnyVec{correction, correction_dtype}, chosen, weight, rows, total, top, group_count, group_keep,
+                                   experts, tile_expert, tile_pairs, max_tiles, tile, always, RouteRule{score, group_best, renorm, weight_scale});
     LEONE_LAUNCH_CHECK("route_plan");
     return 0;
 }

@@ -171,3 +171,34 @@ def test_products_with_one_chunk_ahead():
     from leone_amd.ops.library import library
     assert library().leone_moe_one_chunk_ahead(16, 1, 1024, 2048)
     _check_pairs([3, 64, 1, 65, 0, 130] + [20] * 10, 2048, 1024, True, 64)
+
+
+@pytest.mark.parametrize("rows,total,top,always", [(1, 1, 1, 0), (8, 35, 4, 1), (17, 64, 12, 0), (64, 100, 9, 2), (256, 64, 8, 0), (256, 64, 9, 0),
+                                                   (30, 300, 70, 1)])
+@pytest.mark.parametrize("corrected", [None, torch.float32, torch.bfloat16])
+def test_choice_and_tiles_in_one_launch(rows, total, top, always, corrected):
+    """The choices and weights of route_topk and every pair once, in a tile of its expert, on both sides of what is handed on through
+    shared memory (2,048 pairs) and of the launch's 16 rows at a time; outputs that stand for no matrix are numbered behind all."""
+    from leone_amd import ops
+    gen = torch.Generator().manual_seed(rows + total)
+    logits = torch.randn(rows, total, generator=gen).to(DEV)
+    correction = None if corrected is None else torch.randn(total, generator=gen).to(DEV).to(corrected)
+    routed = max(1, total - 3)                             # three outputs stand for no matrix
+    experts, places, tile = routed + always, top + always, ops.library().leone_moe_tile_pairs()
+    want, want_weight = ops.route_topk(logits, correction, top)
+    pairs = rows * places
+    tiles = min(pairs // tile + experts, pairs)
+    chosen = torch.empty(rows, places, dtype=torch.int32, device=DEV)
+    weight = torch.empty(rows, places, device=DEV)
+    tile_expert, tile_pairs = torch.empty(tiles, dtype=torch.int32, device=DEV), torch.empty(tiles, tile, dtype=torch.int32, device=DEV)
+    ops.call("leone_route_plan", logits.data_ptr(), 0 if correction is None else correction.data_ptr(),
+                     ops.BF16 if corrected == torch.bfloat16 else ops.F32, chosen.data_ptr(), weight.data_ptr(), rows, total, top,
+                     1, 1, experts, tile_expert.data_ptr(), tile_pairs.data_ptr(), tiles, tile, always, *ops._DEFAULT_RULE.args(), ops._stream())
+    torch.cuda.synchronize()
+    assert torch.equal(chosen[:, :top], torch.where(want >= routed, want + always, want)) and torch.equal(weight[:, :top], want_weight)
+    assert chosen[:, top:].tolist() == [list(range(routed, experts))] * rows and bool((weight[:, top:] == 1).all())
+    of = chosen.flatten().tolist()
+    found = [(pair, e) for e, held in zip(tile_expert.tolist(), tile_pairs.tolist()) for pair in held if pair >= 0]
+    assert sorted(found) == [(pair, e) for pair, e in enumerate(of) if e < experts]
+    held = [e for e in tile_expert.tolist() if e >= 0]
+    assert len(held) == sum(math.ceil(of.count(e) / tile) for e in set(of) if e < experts)
