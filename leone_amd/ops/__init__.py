@@ -514,18 +514,6 @@ def choose_splits(rows: int, kv_heads: int, group: int, max_context: int, units:
     return best[1]
 
 
-def whole_rounds(splits: int, blocks: int, max_context: int) -> int:
-    """``splits`` of few blocks (up to eight kv heads of rows in all, so that the parts never share a unit), raised to where a part
-    is one round less of the workgroup's four waves: a fifth tile a part is a second round for one wave.  One row of eight
-    kv heads at 2,052 keys 12.0 us in 13 parts, 10.5 in 17."""
-    tiles = (max_context + 31) // 32
-    rounds = -(-tiles // (4 * splits))
-    if splits == 1 or blocks > 8 or rounds < 2:          # (a part that is the whole needs no merge)
-        return splits
-    more = -(-tiles // (4 * (rounds - 1)))
-    return more if more <= 32 else splits
-
-
 def attention_decode(q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor, positions: torch.Tensor,
                      row_entry: torch.Tensor, block_table: torch.Tensor, q_heads: int, scale: float,
                      window: int = 0, max_context: int = 1, splits: Optional[int] = None,
@@ -591,7 +579,6 @@ def attention_decode_projected(qkv: torch.Tensor, q_heads: int, kv_heads: int, h
         raise KernelError("attention_decode_projected: q and k gains must come together in one type")
     if splits is None:
         splits = choose_splits(rows, kv_heads, q_heads // kv_heads, max_context, compute_units(qkv.device))
-        splits = whole_rounds(splits, rows * kv_heads * ((q_heads // kv_heads + 15) // 16), max_context)
     out = torch.empty((rows, q_heads * head_dim), dtype=torch.bfloat16, device=qkv.device)
     part_acc = part_ml = None
     if splits > 1:

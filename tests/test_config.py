@@ -126,16 +126,3 @@ def test_decode_attention_cuts_keys_to_fill_the_compute_units():
     assert ops.choose_splits(40, 8, 4, 8192) in (2, 4)
     assert ops.choose_splits(8, 8, 4, 100) == 1                     # four tiles in all: nothing to cut
     assert ops.choose_splits(1, 64, 1, 8192, units=304) >= 4        # other head counts, another chip
-
-
-def test_parts_of_few_rows_are_whole_rounds_of_a_workgroups_waves():
-    from leone_amd import ops
-
-    for blocks in (1, 8, 9):
-        for context in (1, 100, 512, 1000, 2052, 4096, 5000, 100_000):
-            tiles, splits = -(-context // 32), ops.choose_splits(1, blocks, 4, context)
-            more = ops.whole_rounds(splits, blocks, context)
-            assert splits <= more <= 32 and (blocks <= 8 or more == splits)
-            if more > splits:       # a round less, and no part without keys
-                assert -(-tiles // (4 * more)) == -(-tiles // (4 * splits)) - 1 and (more - 1) * -(-tiles // more) < tiles
-    assert ops.whole_rounds(1, 4, 192) == 1 and ops.whole_rounds(13, 8, 2052) == 17 and ops.whole_rounds(4, 8, 512) == 4 and ops.whole_rounds(32, 8, 8192) == 32

@@ -72,6 +72,24 @@ def test_rows_that_bring_their_own_key_do_not_depend_on_the_pages(size, group, k
                     assert torch.equal(out, found[0][0]) and torch.equal(new, found[0][1])
 
 
+def test_rows_that_bring_their_own_key_are_cut_by_the_rule():
+    """How many parts a row's keys are cut into decides in which order their results are added: the projected call's own number is
+    ``choose_splits``'s, as it is for ``attention_decode``."""
+    from leone_amd import ops
+    heads, size, context = 8, 128, 2052
+    gen = torch.Generator().manual_seed(5)
+    k, v = (torch.randn(1, context, heads, size, generator=gen) for _ in range(2))
+    qkv = torch.randn(1, 6 * heads * size, generator=gen).bfloat16().to(DEV)
+    found = []
+    for splits in (None, ops.choose_splits(1, heads, 4, context, ops.compute_units(torch.device(DEV)))):
+        k_pool, v_pool, table = pools(k, v, 64, 2)
+        found.append(ops.attention_decode_projected(qkv, 4 * heads, heads, size, None, None, 1e-6, None, None, bits(k_pool), bits(v_pool),
+                                                    torch.tensor([context - 1], dtype=torch.int32, device=DEV),
+                                                    torch.zeros(1, dtype=torch.int32, device=DEV), table, size ** -0.5,
+                                                    max_context=context, splits=splits))
+    assert torch.equal(*found)
+
+
 def test_a_key_without_a_page_spoils_the_rows_that_see_it():
     from leone_amd import ops
     k, v = made(2, 128, 3)
