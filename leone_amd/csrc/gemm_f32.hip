@@ -100,18 +100,53 @@ __device__ inline f32x4 add_term(int term, const Operand& a, const Operand& b, c
 }
 // An infinity has no parts (what is left of it is not a number), and neither have numbers that round to one; the parts of a number
 // below 2^-108 can lie below what the instruction takes for zero, which is off by at most 2^-126 of the other factor.  A segment's
-// sum that comes out infinite, NaN or that small is therefore made again, one product after the other.
+// sum that comes out infinite, NaN or that small is therefore made again on the float instructions.
 constexpr unsigned kLeastBits = 0x1f800000u, kMostBits = 0x7f7fffffu;      // 2^-64 and the largest number
 __device__ inline bool in_doubt(float v) {
     const unsigned size = __float_as_uint(v) & 0x7fffffffu;
     return size != 0 && size - kLeastBits > kMostBits - kLeastBits;
 }
-__device__ float plain_segment(const float* __restrict__ a, const float* __restrict__ b, int first, int end) {
-    float sum = 0.f;
-    for (int at = first; at < end; at += 16) {
-        float chain = 0.f;
-        for (int e = at; e < at + 16 && e < end; ++e) chain = fmaf(a[e], b[e], chain);
-        sum += chain;
+// Register j of quarter g becomes register g of quarter j.
+__device__ inline f32x4 transpose_quarters(const f32x4 v) {
+    const auto bits = [](float f) { return __float_as_uint(f); };
+    const u32x2 p = __builtin_amdgcn_permlane32_swap(bits(v[0]), bits(v[2]), false, false);
+    const u32x2 q = __builtin_amdgcn_permlane32_swap(bits(v[1]), bits(v[3]), false, false);
+    const u32x2 r = __builtin_amdgcn_permlane16_swap(p[0], q[0], false, false);
+    const u32x2 s = __builtin_amdgcn_permlane16_swap(p[1], q[1], false, false);
+    return f32x4{__uint_as_float(r[0]), __uint_as_float(r[1]), __uint_as_float(s[0]), __uint_as_float(s[1])};
+}
+// The segment's sums of a square of 16 x 16 outputs on the float instructions: 16 products a chain, k ascending, and the chains' sums
+// added in order.  This lane's row of A and row of B are those of number lane % 16 of the square; what comes out lies as the bfloat16
+// instruction's results do, and depends on an output's own two rows alone.  The 16 x 16 x 4 instruction adds its four products in the
+// order of the lanes' quarters, so the four quarters' registers are transposed by lane swaps: instruction j takes elements 4 j .. 4 j + 3
+// in turn; the next run is on its way meanwhile.  (By a loop over K for every output in doubt, a row that is not a number held up whoever
+// shared its launch.  us, all sums ordinary, one row NaN by a loop and so, all rows by a loop and so: one row against 2048 x 2048 10, 100,
+// 12, 248, 16; 200 rows against 3072 x 2048 30, 79, 41, 2842, 108; 777 against 12288 x 2048 256, 287, 252, 38668, 1379.)
+constexpr int kPlainRun = 16;                          // elements of K on their way at a time
+template <bool kVec>
+__device__ inline f32x4 plain_square(const float* __restrict__ arow, const float* __restrict__ brow, int first, int end, int g) {
+    f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+    constexpr int kLoads = kPlainRun / 16;
+    f32x4 x[kLoads], y[kLoads];
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) x[i] = load_four<kVec>(arow, first + i * 16 + 4 * g, end), y[i] = load_four<kVec>(brow, first + i * 16 + 4 * g, end);
+#pragma unroll 1
+    for (int at = first; at < end; at += kPlainRun) {
+        f32x4 next_x[kLoads], next_y[kLoads];
+#pragma unroll
+        for (int i = 0; i < kLoads; ++i) {
+            next_x[i] = load_four<kVec>(arow, at + kPlainRun + i * 16 + 4 * g, end);
+            next_y[i] = load_four<kVec>(brow, at + kPlainRun + i * 16 + 4 * g, end);
+        }
+#pragma unroll
+        for (int i = 0; i < kLoads; ++i) {
+            const f32x4 xt = transpose_quarters(x[i]), yt = transpose_quarters(y[i]);
+            f32x4 chain = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int j = 0; j < 4; ++j) chain = __builtin_amdgcn_mfma_f32_16x16x4f32(xt[j], yt[j], chain, 0, 0, 0);
+            sum += chain;
+            x[i] = next_x[i], y[i] = next_y[i];
+        }
     }
     return sum;
 }
@@ -206,13 +241,15 @@ gemm_f32_stream_kernel(const float* __restrict__ a, const float* __restrict__ b,
         left % 2 ? multiply(0, true) : multiply(0, false);
     }
 #pragma unroll
-    for (int t = 0; t < kTilesM; ++t)
+    for (int t = 0; t < kTilesM; ++t) {
+        if (__any(in_doubt(sum[t][0]) || in_doubt(sum[t][1]) || in_doubt(sum[t][2]) || in_doubt(sum[t][3]))) {
+            const f32x4 plain = plain_square<kVec>(arow[t], brow, first, end, lane / 16);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int row = t * 16 + h + i;
-            if (in_doubt(sum[t][i])) sum[t][i] = plain_segment(a + static_cast<long>(row < m ? row : m - 1) * k, brow, first, end);
-            sums[wave][t][(h + i) * kStreamTile + r] = sum[t][i];
+            for (int i = 0; i < 4; ++i) sum[t][i] = in_doubt(sum[t][i]) ? plain[i] : sum[t][i];
         }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sums[wave][t][(h + i) * kStreamTile + r] = sum[t][i];
+    }
     __syncthreads();
     if (then.gated) {                                  // the tile's 16 rows of B are eight gates and their ups
         for (int e = threadIdx.x; e < kTilesM * 128; e += kWaves * kWave) {
@@ -366,28 +403,31 @@ gemm_f32_tile_kernel(const float* __restrict__ a, const float* __restrict__ b, f
         fetch_a(k0 + 2 * kSlab);
         sign = -sign;
         if (k0 + kSlab >= k_end || k0 + kSlab == segment_first + segment) {
-            unsigned furthest = 0;                       // from the sums that are not in doubt; a sum of 0 is looked at below
+            unsigned furthest = 0;                       // from the sums that are not in doubt (0 is one of them)
 #pragma unroll
             for (int i = 0; i < kFragA; ++i)
 #pragma unroll
                 for (int j = 0; j < kFragB; ++j)
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) furthest = max(furthest, (__float_as_uint(sum[i][j][e]) & 0x7fffffffu) - kLeastBits);
+                    for (int e = 0; e < 4; ++e) {
+                        const unsigned size = __float_as_uint(sum[i][j][e]) & 0x7fffffffu;
+                        furthest = max(furthest, (size ? size : kMostBits) - kLeastBits);
+                    }
             if (__any(furthest > kMostBits - kLeastBits)) {
                 const int end = segment_first + segment < k_end ? segment_first + segment : k_end;
 #pragma unroll 1
-                for (int x = 0; x < kFragA * kFragB * 4; ++x) {
-                    const int i = x / (kFragB * 4), j = x / 4 % kFragB, e = x % 4;
-                    float v = 0.f;
+                for (int x = 0; x < kFragA * kFragB; ++x) {
+                    f32x4 v = sum[0][0];
 #pragma unroll
-                    for (int y = 0; y < kFragA * kFragB * 4; ++y) v = x == y ? sum[y / (kFragB * 4)][y / 4 % kFragB][y % 4] : v;
-                    if (in_doubt(v) && row_of(i, e) < m && col + j * 16 < n)
-                        v = plain_segment(a + static_cast<long>(row_of(i, e)) * k, b + static_cast<long>(col + j * 16) * k, segment_first, end);
+                    for (int y = 1; y < kFragA * kFragB; ++y) v = x == y ? sum[y / kFragB][y % kFragB] : v;
+                    if (!__any(in_doubt(v[0]) || in_doubt(v[1]) || in_doubt(v[2]) || in_doubt(v[3]))) continue;
+                    const int row = m0 + x / kFragB * 16 + r, of = col + x % kFragB * 16;
+                    const f32x4 plain = plain_square<kVec>(a + static_cast<long>(row < m ? row : m - 1) * k,
+                                                           b + static_cast<long>(of < n ? of : n - 1) * k, segment_first, end, g);
 #pragma unroll
-                    for (int y = 0; y < kFragA * kFragB * 4; ++y) {
-                        float& to = reinterpret_cast<float*>(&sum[y / (kFragB * 4)][y / 4 % kFragB])[y % 4];
-                        to = x == y ? v : to;
-                    }
+                    for (int e = 0; e < 4; ++e) v[e] = in_doubt(v[e]) ? plain[e] : v[e];
+#pragma unroll
+                    for (int y = 0; y < kFragA * kFragB; ++y) sum[y / kFragB][y % kFragB] = x == y ? v : sum[y / kFragB][y % kFragB];
                 }
             }
             segment_first += segment;
