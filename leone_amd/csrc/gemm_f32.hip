@@ -98,13 +98,24 @@ constexpr int kTerms = 6, kTermA[kTerms] = {2, 0, 1, 1, 0, 0}, kTermB[kTerms] = 
 __device__ inline f32x4 add_term(int term, const Operand& a, const Operand& b, const f32x4& sum) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.part[kTermA[term]], b.part[kTermB[term]], sum, 0, 0, 0);
 }
-// An infinity has no parts (what is left of it is not a number), and neither have numbers that round to one; the parts of a number
-// below 2^-108 can lie below what the instruction takes for zero, which is off by at most 2^-126 of the other factor.  A segment's
-// sum that comes out infinite, NaN or that small is therefore made again on the float instructions.
-constexpr unsigned kLeastBits = 0x1f800000u, kMostBits = 0x7f7fffffu;      // 2^-64 and the largest number
-__device__ inline bool in_doubt(float v) {
-    const unsigned size = __float_as_uint(v) & 0x7fffffffu;
-    return size != 0 && size - kLeastBits > kMostBits - kLeastBits;
+// An infinity has no parts (what is left of it is not a number), and neither have numbers that round to one; and what lies below
+// bfloat16's least number, 2^-133, is lost from the parts of a number below 2^-110, and from the products of parts what lies below a
+// float's, which counts where the other factor is large.  A segment's sum that comes out infinite or NaN, or so small beside the largest
+// numbers of its row of A and its row of B that what is lost could count, is therefore made again on the float instructions.  For
+// largest numbers a and b less than 2^-132 max(a, 1) max(b, 1) is lost a product (half of 2^-133 of either factor times the other, and eight
+// products' 2^-149); a sum is in doubt below 2^-90 max(a, 1) max(b, 1), so that others lose less than half of a float's last bit up to
+// segments of 2^17.  Rows of zeros are not in doubt.
+// A row's share of the limit below which a sum is in doubt (0: never); the sum's own: their product.
+__device__ inline float least_of(float largest) { return largest > 0.f ? fmaxf(largest, 1.0f) * 0x1p-45f : 0.f; }
+__device__ inline bool in_doubt(float v, float least_a, float least_b) {
+    return fmaf(-least_a, least_b, fabsf(v)) < 0.f || !(fabsf(v) <= 3.402823466e38f);
+}
+// The largest absolute value so far (of NaN any: it spoils its sum).  Two instructions for four numbers; from fmaxf and fabsf the
+// compiler makes more, to quiet NaN first.
+__device__ inline float largest_of(float so_far, const f32x4& v) {
+    asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(so_far) : "v"(v[0]), "v"(v[1]));
+    asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(so_far) : "v"(v[2]), "v"(v[3]));
+    return so_far;
 }
 // Register j of quarter g becomes register g of quarter j.
 __device__ inline f32x4 transpose_quarters(const f32x4 v) {
@@ -180,6 +191,7 @@ gemm_f32_stream_kernel(const float* __restrict__ a, const float* __restrict__ b,
 #pragma unroll
     for (int t = 0; t < kTilesM; ++t) arow[t] = a + static_cast<long>(t * 16 + r < m ? t * 16 + r : m - 1) * k;
     f32x4 sum[kTilesM] = {};
+    float largest_b = 0.f, largest_a[kTilesM] = {};
     f32x4 w[kDepth][kStreamLoads], x[kDepth][kTilesM][kStreamLoads];
     const int first = wave * segment, end = first + segment < k ? first + segment : k;
     const auto fetch = [&](int at, int into) {         // a run that lies whole before the segment's end
@@ -194,13 +206,16 @@ gemm_f32_stream_kernel(const float* __restrict__ a, const float* __restrict__ b,
 #pragma unroll
         for (int i = 0; i < kStreamLoads; i += 2) {
             const Operand wp = operand_of(w[from][i], w[from][i + 1]);
+            largest_b = largest_of(largest_of(largest_b, w[from][i]), w[from][i + 1]);
 #pragma unroll
             for (int t = 0; t < kTilesM; ++t) {
+                largest_a[t] = largest_of(largest_of(largest_a[t], x[from][t][i]), x[from][t][i + 1]);
                 const Operand xp = odd ? operand_of(-x[from][t][i], -x[from][t][i + 1]) : operand_of(x[from][t][i], x[from][t][i + 1]);
                 f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int e = 0; e < kTerms; ++e) acc = add_term(e, xp, wp, acc);
                 sum[t] = odd ? sum[t] - acc : sum[t] + acc;
+                __builtin_amdgcn_sched_barrier(0);     // (interleaved with the next ones' products the waves' number would not fit the registers)
             }
         }
     };
@@ -240,12 +255,21 @@ gemm_f32_stream_kernel(const float* __restrict__ a, const float* __restrict__ b,
             for (int i = 0; i < kStreamLoads; ++i) x[0][t][i] = load_four<kVec>(arow[t], at + i * 16 + h, end);
         left % 2 ? multiply(0, true) : multiply(0, false);
     }
+    const float least_b = least_of(max_lanes<16>(max_lanes<32>(largest_b)));
 #pragma unroll
     for (int t = 0; t < kTilesM; ++t) {
-        if (__any(in_doubt(sum[t][0]) || in_doubt(sum[t][1]) || in_doubt(sum[t][2]) || in_doubt(sum[t][3]))) {
+        const float least_a = least_of(max_lanes<16>(max_lanes<32>(largest_a[t])));
+        float least[4];
+        bool any = false;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            least[i] = __shfl(least_a, h + i, kWave);
+            any |= in_doubt(sum[t][i], least[i], least_b);
+        }
+        if (__any(any)) {
             const f32x4 plain = plain_square<kVec>(arow[t], brow, first, end, lane / 16);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) sum[t][i] = in_doubt(sum[t][i]) ? plain[i] : sum[t][i];
+            for (int i = 0; i < 4; ++i) sum[t][i] = in_doubt(sum[t][i], least[i], least_b) ? plain[i] : sum[t][i];
         }
 #pragma unroll
         for (int i = 0; i < 4; ++i) sums[wave][t][(h + i) * kStreamTile + r] = sum[t][i];
@@ -295,21 +319,35 @@ gemm_f32_tile_kernel(const float* __restrict__ a, const float* __restrict__ b, f
                      int segment, int each, Epilogue then) {
     constexpr int kFragA = kTileRows / 16, kFragB = kCols / 64;                      // 16 x 16 squares of a wave
     constexpr int kLoadsA = kTileRows / 32;                                          // 16-byte loads a thread and slab
+    constexpr int kSquares = kFragA * kFragB;
+    constexpr int kHeld = kFragB > 1 ? 2 : kSquares;                                 // squares whose totals are in registers,
+    constexpr int kAway = kCut ? 0 : kSquares - kHeld;                               // and in shared memory (with all of them a wave would spill)
     __shared__ u32x2 slabs[2][3][kTileRows][8];
-    const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+    __shared__ f32x4 away[kAway ? kAway : 1][kAway ? 256 : 1];
+    __shared__ __align__(16) float least_a[2][kTileRows];       // (see least_of) of this segment's rows of A and, by turns, the next one's
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;       // (a scalar register)
     const int m0 = blockIdx.y * kTileRows, n0 = blockIdx.x * kCols + wave * (kCols / 4);
     const int r = lane % 16, g = lane / 16;
     const long part = static_cast<long>(segment) * each;
     const int k_first = static_cast<int>(blockIdx.z * part), k_end = k - k_first > part ? static_cast<int>(k_first + part) : k;
     const int four = threadIdx.x % 8, from_row = threadIdx.x / 8;                // this thread's four elements of every 32nd row of A
-    const float *arow[kLoadsA], *brow[kFragB];
-#pragma unroll
-    for (int i = 0; i < kLoadsA; ++i) arow[i] = a + static_cast<long>(m0 + from_row + i * 32 < m ? m0 + from_row + i * 32 : m - 1) * k;
-#pragma unroll
-    for (int j = 0; j < kFragB; ++j) brow[j] = b + static_cast<long>(n0 + j * 16 + r < n ? n0 + j * 16 + r : n - 1) * k;
+    // A number whose uses are computed where they stand: held in registers throughout, they would leave the sums none.
+    const auto here = [](int v) {
+        asm volatile("" : "+v"(v));
+        return v;
+    };
+    const auto arow = [&](int i) {
+        const int row = m0 + i * 32 + here(from_row);
+        return a + static_cast<long>(row < m ? row : m - 1) * k;
+    };
+    const auto brow = [&](int j) {
+        const int row = n0 + j * 16 + here(r);
+        return b + static_cast<long>(row < n ? row : n - 1) * k;
+    };
     f32x4 sum[kFragA][kFragB] = {};
-    [[maybe_unused]] f32x4 total[kFragA][kFragB] = {};
+    [[maybe_unused]] f32x4 total[kHeld] = {};
     f32x4 ra[kLoadsA], rb[kFragB][2];
+    float largest_a[kLoadsA] = {}, largest_b[kFragB] = {};
     // (past the last element of a row: its last ones, and not used)
     const auto load_at = [&](const float* row, int at) {
         if (kVec) return *reinterpret_cast<const f32x4*>(row + (at < k ? at : k - 4));
@@ -320,13 +358,13 @@ gemm_f32_tile_kernel(const float* __restrict__ a, const float* __restrict__ b, f
     };
     const auto fetch_a = [&](int k0) {
 #pragma unroll
-        for (int i = 0; i < kLoadsA; ++i) ra[i] = load_at(arow[i], k0 + four * 4);
+        for (int i = 0; i < kLoadsA; ++i) ra[i] = load_at(arow(i), k0 + four * 4);
     };
     const auto fetch_b = [&](int k0) {
 #pragma unroll
         for (int j = 0; j < kFragB; ++j)
 #pragma unroll
-            for (int half = 0; half < 2; ++half) rb[j][half] = load_at(brow[j], k0 + half * 16 + g * 4);
+            for (int half = 0; half < 2; ++half) rb[j][half] = load_at(brow(j), k0 + half * 16 + g * 4);
     };
     const auto cut_off = [&](int k0) {                  // what lies past K in a slab of A counts as zero
         if (k0 + kSlab <= k) return;
@@ -351,6 +389,7 @@ gemm_f32_tile_kernel(const float* __restrict__ a, const float* __restrict__ b, f
     const auto place = [](int row, int of) { return of ^ (row / 2 % 4); };       // of lane group `of`'s sixteen bytes
     const int kept_at = place(from_row, four % 4) * 2 + four / 4;                // (32 rows further it is the same)
     const auto keep = [&](int into, int i, float sign) {
+        largest_a[i] = largest_of(largest_a[i], ra[i]);
         const FourParts v = parts_of(ra[i] * sign);
 #pragma unroll
         for (int p = 0; p < 3; ++p) slabs[into][p][from_row + i * 32][kept_at] = v.part[p];
@@ -358,29 +397,52 @@ gemm_f32_tile_kernel(const float* __restrict__ a, const float* __restrict__ b, f
     const int col = n0 + r;                                                      // of the first square; rows 4 g .. + 3
     const auto row_of = [&](int i, int e) { return m0 + i * 16 + 4 * g + e; };
     const auto store = [&](const f32x4 (&of)[kFragA][kFragB], float* to) {
+        const int left_m = m - m0, left_n = n - n0, row0 = here(4 * g), column = here(r);
 #pragma unroll
         for (int i = 0; i < kFragA; ++i)
 #pragma unroll
             for (int e = 0; e < 4; ++e)
 #pragma unroll
                 for (int j = 0; j < kFragB; ++j)
-                    if (row_of(i, e) < m && col + j * 16 < n) to[static_cast<long>(row_of(i, e)) * n + col + j * 16] = of[i][j][e];
+                    if (row0 + i * 16 + e < left_m && column + j * 16 < left_n)
+                        to[static_cast<long>(m0 + row0 + i * 16 + e) * n + n0 + column + j * 16] = of[i][j][e];
     };
+    // the slab of A that was kept ends its segment: the segment's rows are known (eight threads have one)
+    int kept_turn = 0, kept_end = k_first + segment;
+    const auto kept = [&](int k0) {
+        if (k0 + kSlab < kept_end && k0 + kSlab < k_end) return;
+#pragma unroll
+        for (int i = 0; i < kLoadsA; ++i) {
+            const float least = least_of(join_span<8>(largest_a[i], [](float x, float y) { return fmaxf(x, y); }));
+            const int thread = here(threadIdx.x);
+            if (thread % 8 == 0) least_a[kept_turn][thread / 8 + i * 32] = least;
+            largest_a[i] = 0.f;
+        }
+        kept_turn ^= 1, kept_end += segment;
+    };
+    if constexpr (kAway > 0) {
+#pragma unroll
+        for (int i = 0; i < kAway; ++i) away[i][threadIdx.x] = f32x4{0.f, 0.f, 0.f, 0.f};       // (a thread's own)
+    }
     fetch_a(k_first);
     fetch_b(k_first);
     cut_off(k_first);
 #pragma unroll
     for (int i = 0; i < kLoadsA; ++i) keep(0, i, 1.0f);
+    kept(k_first);
     fetch_a(k_first + kSlab);
     float sign = 1.0f;                                 // of the slab that is multiplied (see kTerms)
-    int at = 0, segment_first = k_first;               // segments are an even number of slabs
+    int at = 0, turn = 0, segment_first = k_first;     // segments are an even number of slabs
     float* plane = c + static_cast<long>(blockIdx.z) * each * m * n;
     const int mine = place(r, g) * 2;
     for (int k0 = k_first; k0 < k_end; k0 += kSlab, at ^= 1) {
         cut_off_b(k0);
         Operand bp[kFragB];
 #pragma unroll
-        for (int j = 0; j < kFragB; ++j) bp[j] = operand_of(rb[j][0], rb[j][1]);
+        for (int j = 0; j < kFragB; ++j) {
+            bp[j] = operand_of(rb[j][0], rb[j][1]);
+            largest_b[j] = largest_of(largest_of(largest_b[j], rb[j][0]), rb[j][1]);
+        }
         fetch_b(k0 + kSlab);
         __syncthreads();               // this slab is there, and nobody reads the one before it any more
         cut_off(k0 + kSlab);
@@ -390,46 +452,63 @@ gemm_f32_tile_kernel(const float* __restrict__ a, const float* __restrict__ b, f
 #pragma unroll
             for (int p = 0; p < 3; ++p)
                 ap.part[p] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(&slabs[at][p][i * 16 + r][mine]));
+#pragma unroll
+            for (int l = i * kLoadsA / kFragA; l < (i + 1) * kLoadsA / kFragA; ++l) keep(at ^ 1, l, -sign);
             f32x4 acc[kFragB] = {};
 #pragma unroll
             for (int e = 0; e < kTerms; ++e)
 #pragma unroll
                 for (int j = 0; j < kFragB; ++j) acc[j] = add_term(e, ap, bp[j], acc[j]);
 #pragma unroll
-            for (int l = i * kLoadsA / kFragA; l < (i + 1) * kLoadsA / kFragA; ++l) keep(at ^ 1, l, -sign);
-#pragma unroll
             for (int j = 0; j < kFragB; ++j) sum[i][j] = acc[j] * sign + sum[i][j];        // (one instruction, and exact)
+            __builtin_amdgcn_sched_barrier(0);             // (the next one's operands ahead of these sums would not fit the registers)
         }
+        if (k0 + kSlab < k_end) kept(k0 + kSlab);
         fetch_a(k0 + 2 * kSlab);
         sign = -sign;
         if (k0 + kSlab >= k_end || k0 + kSlab == segment_first + segment) {
-            unsigned furthest = 0;                       // from the sums that are not in doubt (0 is one of them)
+            // (that segment's rows of A were written before the slab's barrier, and are written again behind the next one at the earliest)
+            const int row0 = here(4 * g), column0 = here(r);
+            float least_b[kFragB], least = 0.f, odd = 0.f;       // least: below 0 if a sum is in doubt; odd: NaN if one is no finite number
 #pragma unroll
-            for (int i = 0; i < kFragA; ++i)
+            for (int j = 0; j < kFragB; ++j) {
+                least_b[j] = least_of(max_lanes<16>(max_lanes<32>(largest_b[j])));
+                largest_b[j] = 0.f;
+            }
+#pragma unroll
+            for (int i = 0; i < kFragA; ++i) {
+                const f32x4 of = *reinterpret_cast<const f32x4*>(&least_a[turn][i * 16 + row0]);
 #pragma unroll
                 for (int j = 0; j < kFragB; ++j)
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
-                        const unsigned size = __float_as_uint(sum[i][j][e]) & 0x7fffffffu;
-                        furthest = max(furthest, (size ? size : kMostBits) - kLeastBits);
+                        least = fminf(least, fmaf(-of[e], least_b[j], fabsf(sum[i][j][e])));
+                        odd = fmaf(sum[i][j][e], 0.f, odd);
                     }
-            if (__any(furthest > kMostBits - kLeastBits)) {
+            }
+            if (__any(least < 0.f || odd != 0.f)) {
                 const int end = segment_first + segment < k_end ? segment_first + segment : k_end;
 #pragma unroll 1
                 for (int x = 0; x < kFragA * kFragB; ++x) {
                     f32x4 v = sum[0][0];
+                    float of_b = least_b[0];
 #pragma unroll
                     for (int y = 1; y < kFragA * kFragB; ++y) v = x == y ? sum[y / kFragB][y % kFragB] : v;
-                    if (!__any(in_doubt(v[0]) || in_doubt(v[1]) || in_doubt(v[2]) || in_doubt(v[3]))) continue;
-                    const int row = m0 + x / kFragB * 16 + r, of = col + x % kFragB * 16;
-                    const f32x4 plain = plain_square<kVec>(a + static_cast<long>(row < m ? row : m - 1) * k,
-                                                           b + static_cast<long>(of < n ? of : n - 1) * k, segment_first, end, g);
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) v[e] = in_doubt(v[e]) ? plain[e] : v[e];
+                    for (int j = 1; j < kFragB; ++j) of_b = x % kFragB == j ? least_b[j] : of_b;
+                    const f32x4 of = *reinterpret_cast<const f32x4*>(&least_a[turn][x / kFragB * 16 + row0]);
+                    const auto doubt = [&](int e) { return in_doubt(v[e], of[e], of_b); };
+                    if (!__any(doubt(0) || doubt(1) || doubt(2) || doubt(3))) continue;
+                    const int row = m0 + x / kFragB * 16 + column0, column = n0 + x % kFragB * 16 + column0;
+                    const f32x4 plain = plain_square<kVec>(a + static_cast<long>(row < m ? row : m - 1) * k,
+                                                           b + static_cast<long>(column < n ? column : n - 1) * k, segment_first, end, row0 / 4);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[e] = doubt(e) ? plain[e] : v[e];
 #pragma unroll
                     for (int y = 0; y < kFragA * kFragB; ++y) sum[y / kFragB][y % kFragB] = x == y ? v : sum[y / kFragB][y % kFragB];
                 }
             }
+            turn ^= 1;
             segment_first += segment;
             if constexpr (kCut) {
                 store(sum, plane);
@@ -439,13 +518,23 @@ gemm_f32_tile_kernel(const float* __restrict__ a, const float* __restrict__ b, f
             for (int i = 0; i < kFragA; ++i)
 #pragma unroll
                 for (int j = 0; j < kFragB; ++j) {
-                    if constexpr (!kCut) total[i][j] += sum[i][j];
+                    if constexpr (!kCut) {
+                        constexpr int kRoom = kAway ? kAway : 1;
+                        const int x = i * kFragB + j;
+                        if (x < kHeld) total[x % kHeld] += sum[i][j];
+                        else away[(x - kHeld) % kRoom][threadIdx.x] += sum[i][j];
+                    }
                     sum[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
                 }
         }
     }
     if constexpr (!kCut) {
-        if (!then.gated) return store(total, c);
+        const auto total_of = [&](int x) { return x < kHeld ? total[x % kHeld] : away[(x - kHeld) % (kAway ? kAway : 1)][threadIdx.x]; };
+#pragma unroll
+        for (int i = 0; i < kFragA; ++i)
+#pragma unroll
+            for (int j = 0; j < kFragB; ++j) sum[i][j] = total_of(i * kFragB + j);
+        if (!then.gated) return store(sum, c);
         // lanes 0 .. 7 of a row of 16 hold gates, the lane eight further its up
 #pragma unroll
         for (int i = 0; i < kFragA; ++i)
@@ -453,10 +542,10 @@ gemm_f32_tile_kernel(const float* __restrict__ a, const float* __restrict__ b, f
             for (int e = 0; e < 4; ++e)
 #pragma unroll
                 for (int j = 0; j < kFragB; ++j) {
-                    const float up = lane_pair<8>(total[i][j][e]).b;
+                    const float up = lane_pair<8>(sum[i][j][e]).b;
                     if (r < 8 && row_of(i, e) < m && col + j * 16 < n)
                         c[static_cast<long>(row_of(i, e)) * (n / 2) + (n0 + j * 16) / 2 + r] =
-                            glu_value(total[i][j][e], up, then.act, then.limit);
+                            glu_value(sum[i][j][e], up, then.act, then.limit);
                 }
     }
 }
@@ -671,14 +760,14 @@ int launch_f32(const F32Plan& p, const float* a, const float* b, float* c, float
         // 18.7).  Two tiles of A fill the registers: 24 rows against 12288 x 2048 32.5 with two, 37.0 with three.
         const bool large = segments.length >= 256 && static_cast<long>(n) * k >= 8l << 20;
         if (segments.count <= 4) {
-            if (m <= kStreamTile) LEONE_STREAM(1, 4, 2, 4);
+            if (m <= kStreamTile) LEONE_STREAM(1, 4, 2, 6);
             else LEONE_STREAM(2, 4, 2, 2);
         } else if (m > kStreamTile) {
             LEONE_STREAM(2, 8, 2, 2);
         } else if (large) {
             LEONE_STREAM(1, 8, 4, 4);
         } else {
-            LEONE_STREAM(1, 8, 2, 4);
+            LEONE_STREAM(1, 8, 2, 6);
         }
 #undef LEONE_STREAM
         LEONE_LAUNCH_CHECK("gemm_f32");

@@ -83,7 +83,7 @@ def test_results_off_sixteen_bytes():
 @pytest.mark.parametrize("m,n,k", [(1, 17, 257), (16, 129, 511), (33, 128, 513), (65, 130, 609), (200, 127, 1100), (70, 300, 2048)])
 @pytest.mark.parametrize("scale", [1e-37, 1e-30, 1e-12, 1.0, 1e12])
 def test_numbers_of_every_size(m, n, k, scale):
-    """Numbers in three parts: none of their 24 bits is lost, whatever the numbers' size and wherever the row ends."""
+    """Numbers in three parts: none of their 24 bits is lost, whatever the size of A's numbers and wherever the row ends."""
     from leone_amd import ops
     gen = torch.Generator(device=DEV).manual_seed(n)
     a, b = torch.randn(m, k, generator=gen, device=DEV) * scale, torch.randn(n, k, generator=gen, device=DEV)
@@ -91,6 +91,39 @@ def test_numbers_of_every_size(m, n, k, scale):
     error = float((ops.gemm_f32(a, b).double() - want).norm() / want.norm())
     # a product that loses more than a float's last bit is off by 2^-24 of itself, at random; sums round as sums of floats do
     assert error < 2.0 ** -24 * (1.0 + math.sqrt(math.log2(k))), error
+
+
+# scales of A and B: below bfloat16's least number, 2^-133, a number's parts are lost, which counts where the other factor is large; the
+# last two bring numbers that are no normal floats, and sums of products that are none
+@pytest.mark.parametrize("m,n,k", [(1, 17, 257), (16, 129, 511), (33, 128, 513), (40, 130, 2048), (300, 127, 1100), (70, 300, 6144)])
+@pytest.mark.parametrize("sizes", [(-110, 80), (80, -110), (-124, 70), (-122, 62), (62, -122), (-126, 100), (-70, -20), (-140, 100), (100, -140), (-75, -50)])
+def test_small_numbers_against_large_ones(m, n, k, sizes):
+    from leone_amd import ops
+    gen = torch.Generator(device=DEV).manual_seed(n)
+    a, b = (torch.randn(rows, k, generator=gen, device=DEV) * 2.0 ** (size / 2) * 2.0 ** (size / 2) for rows, size in zip((m, n), sizes))
+    want = a.double() @ b.double().T
+    got = ops.gemm_f32(a, b)
+    # as in test_numbers_of_every_size; a product or a sum below the least normal float is off by half of 2^-149 at most
+    bound = 2.0 ** -24 * (1.0 + math.sqrt(math.log2(k))) * float(want.norm()) + 2.0 ** -150 * (2 * k) * math.sqrt(m * n)
+    assert float((got.double() - want).norm()) < bound
+    alone = torch.cat([ops.gemm_f32(a[i:i + 1].contiguous(), b) for i in (0, m - 1)])
+    assert torch.equal(got[[0, m - 1]], alone)             # whether a sum is made again is its own two rows' matter
+
+
+@pytest.mark.parametrize("m", [3, 40, 300])
+def test_a_lone_small_number_against_a_large_one(m):
+    """2^-140 x 2^100 is an ordinary number, and so is what a row holds of both kinds; rows of zeros give zeros."""
+    from leone_amd import ops
+    n, k = 140, 600
+    a, b = torch.zeros(m, k, device=DEV), torch.zeros(n, k, device=DEV)
+    a[0, 5], b[:, 5] = 2.0 ** -140, 2.0 ** 100
+    a[1, 7], b[:, 7] = 1.2345678 * 2.0 ** -126, 2.0 ** 100
+    a[2, 7], a[2, 590] = 2.0 ** -120 * (1 + 2.0 ** -14), -1.5 * 2.0 ** -60
+    b[:, 590] = 3.0 * 2.0 ** 40
+    got = ops.gemm_f32(a, b)
+    assert bool((got[0] == 2.0 ** -40).all()) and not bool(got[3:].any())
+    assert torch.equal(got[1], (a[1, 7] * 2.0 ** 100).expand(n))
+    assert torch.equal(got[2], (a[2, 7].double() * 2.0 ** 100 - 4.5 * 2.0 ** -20).float().expand(n))
 
 
 def test_numbers_that_are_no_sums_of_parts():
