@@ -1,6 +1,6 @@
-// Single-precision matrix product for the true 32-bit path:
-// C[M,N] = A[M,K] . B[N,K]^T on the float matrix instructions (products and sums in float, fused; no reduced-precision
-// mode).  The reference's scalar backend folds each output left to right in float (crates/leone/src/cpu.rs:1379-1405,
+// Single-precision matrix product for the true 32-bit path: C[M,N] = A[M,K] . B[N,K]^T, operands, products and sums with a float's 24
+// bits (no reduced-precision mode).  A K below 256 goes to the float matrix instructions; from there on to those of bfloat16, every
+// number taken apart into three.  The reference's scalar backend folds each output left to right in float (crates/leone/src/cpu.rs:1379-1405,
 // 1622-1640).
 //
 // An output's bits depend on its row of A, its row of B and K alone, never on the rows that share the launch (what a request gets
@@ -9,9 +9,11 @@
 // backend's fold.
 //
 // The matrix instructions take floats at a sixteenth of the rate of bfloat16.  From a K of 256 on, numbers are therefore taken apart
-// into three bfloat16 each, which hold all of their 24 bits, and a product is made of the six products of parts that reach a float's last
-// bit: 2.7 times the float rate, and the sums of 32 round less often than chains of float products do (error against 64 bits over the
-// result's norm, 1 to 1,024 rows: K 512 0.7e-7, 2048 0.9e-7, 6144 1.2e-7; chains of 16 float products 1.0e-7, 1.2e-7 and 1.6e-7).
+// into three bfloat16 each, which hold all of their 24 bits, and a product is made of eight of the nine products of parts (the method is
+// published: Henry, Tang, Heinecke, "Leveraging the bfloat16 artificial intelligence datatype for higher-precision computations", 2019):
+// twice the float rate.  The sums of 32 round less often than chains of float products do (error against 64 bits over the
+// result's norm, 1 to 1,024 rows: K 512 0.7e-7, 2048 0.9e-7, 6144 1.1e-7; chains of 16 float products 1.0e-7, 1.2e-7 and 1.6e-7), and a
+// row's only product is rounded as a float product is (at most 1.003 of 2^-24 off, 0.15 % not to the nearest).
 //
 // Few rows (decoding): a product reads every weight once for 2 M operations, so the weights' bytes are the
 // bound and what matters is how much of them is in flight: a workgroup owns 16 rows of B, its waves take a segment each, and a
@@ -50,8 +52,8 @@ __device__ inline f32x4 load_whole(const float* __restrict__ at) {
 
 // ---- three parts a number --------------------------------------------------------------------------------------------
 // The 16 x 16 x 32 instruction takes eight bfloat16 a lane and adds in float.  A float is the sum of three bfloat16 (8 bits each,
-// rounded to nearest, so that what is left is at most half of the last bit and of either sign); a product of two floats is six of
-// the nine products of their parts, the other three lie below a quarter of a float's last bit.
+// rounded to nearest, so that what is left is at most half of the last bit and of either sign).  Of the nine products of two floats' parts the
+// one of both last parts is left out: it is at most 2^-32 of the product.
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
 typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
@@ -91,12 +93,16 @@ __device__ inline Operand operand_of(const f32x4& first, const f32x4& second) {
     for (int p = 0; p < 3; ++p) r.part[p] = __builtin_bit_cast(bf16x8, u32x4{a.part[p][0], a.part[p][1], b.part[p][0], b.part[p][1]});
     return r;
 }
-// The sum of 32 products, the smallest parts first.  What the instruction loses when it brings its products to one exponent it takes
+// The sum of 32 products: those of lower parts, the smallest first, and those of both highest parts, which a float addition rounds (added to
+// the others by the instruction, a fifth of lone products came out one off).  What the instruction loses when it brings its products to one exponent it takes
 // off, whatever their sign (sums of 2,048 come out 5e-8 of their root mean square too low), so every other 32 elements of a segment
 // are multiplied with A's sign turned and their sum is subtracted.
-constexpr int kTerms = 6, kTermA[kTerms] = {2, 0, 1, 1, 0, 0}, kTermB[kTerms] = {0, 2, 1, 0, 1, 0};
+constexpr int kTerms = 7, kTermA[kTerms] = {2, 1, 2, 0, 1, 1, 0}, kTermB[kTerms] = {1, 2, 0, 2, 1, 0, 1};
 __device__ inline f32x4 add_term(int term, const Operand& a, const Operand& b, const f32x4& sum) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.part[kTermA[term]], b.part[kTermB[term]], sum, 0, 0, 0);
+}
+__device__ inline f32x4 highest_term(const Operand& a, const Operand& b) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.part[0], b.part[0], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
 }
 // An infinity has no parts (what is left of it is not a number), and neither have numbers that round to one; and what lies below
 // bfloat16's least number, 2^-133, is lost from the parts of a number below 2^-110, and from the products of parts what lies below a
@@ -214,6 +220,7 @@ gemm_f32_stream_kernel(const float* __restrict__ a, const float* __restrict__ b,
                 f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int e = 0; e < kTerms; ++e) acc = add_term(e, xp, wp, acc);
+                acc += highest_term(xp, wp);
                 sum[t] = odd ? sum[t] - acc : sum[t] + acc;
                 __builtin_amdgcn_sched_barrier(0);     // (interleaved with the next ones' products the waves' number would not fit the registers)
             }
@@ -304,10 +311,11 @@ gemm_f32_stream_kernel(const float* __restrict__ a, const float* __restrict__ b,
 // every bank once.  While a slab is multiplied, A's next one is taken apart between the instructions, and the one after that and B's
 // next one are on their way into registers.
 //
-// What bounds it is that the matrix instructions (six for what one product of floats needs), the taking apart (half of the vector
+// What bounds it is that the matrix instructions (eight for what one product of floats needs), the taking apart (half of the vector
 // instructions) and the trips through shared memory follow one another within a wave; three workgroups a unit make up for it to half of
-// the instructions' rate.  Columns of their own keep B out of shared memory: 777 rows against 12288 x 2048 take 243 us (161 TFLOP/s
-// in floats), with both operands in shared memory 303, on the float instructions 437; against 2048 x 6144 137, 150 and 219.
+// the instructions' rate.  Columns of their own keep B out of shared memory (777 rows against 12288 x 2048, with six products of parts:
+// 243 us, with both operands in shared memory 303).  With eight 777 rows against 12288 x 2048 take 315 us, 2048 x 6144 169, of which six would be
+// 266 and 148; on the float instructions 440 and 219.
 //
 // kCut: blockIdx.z takes `each` segments and leaves a plane of c for every one of them; else one workgroup walks them all.
 constexpr int kSlab = kChain;
@@ -459,6 +467,8 @@ gemm_f32_tile_kernel(const float* __restrict__ a, const float* __restrict__ b, f
             for (int e = 0; e < kTerms; ++e)
 #pragma unroll
                 for (int j = 0; j < kFragB; ++j) acc[j] = add_term(e, ap, bp[j], acc[j]);
+#pragma unroll
+            for (int j = 0; j < kFragB; ++j) acc[j] += highest_term(ap, bp[j]);
 #pragma unroll
             for (int j = 0; j < kFragB; ++j) sum[i][j] = acc[j] * sign + sum[i][j];        // (one instruction, and exact)
             __builtin_amdgcn_sched_barrier(0);             // (the next one's operands ahead of these sums would not fit the registers)

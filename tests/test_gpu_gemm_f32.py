@@ -93,6 +93,21 @@ def test_numbers_of_every_size(m, n, k, scale):
     assert error < 2.0 ** -24 * (1.0 + math.sqrt(math.log2(k))), error
 
 
+@pytest.mark.parametrize("m,n,k", [(1, 4096, 256), (16, 999, 513), (32, 2048, 2048), (200, 1001, 1001), (300, 512, 6144)])
+def test_a_lone_product_is_rounded_as_a_float_product_is(m, n, k):
+    """All that is left out of a product and lost on the way is below 2^-8 of a float's last bit: the product of both last parts (2^-32)
+    and what the sums of the lower ones round."""
+    from leone_amd import ops
+    gen = torch.Generator(device=DEV).manual_seed(n)
+    a, b = torch.zeros(m, k, device=DEV), torch.randn(n, k, generator=gen, device=DEV)
+    at, value = torch.randint(0, k, (m,), generator=gen, device=DEV), torch.randn(m, generator=gen, device=DEV)
+    a[torch.arange(m, device=DEV), at] = value
+    want = value.double()[:, None] * b[:, at].double().T
+    got = ops.gemm_f32(a, b)
+    assert float(((got.double() - want) / want).abs().max()) < 2.0 ** -24 * (1.0 + 2.0 ** -7)
+    assert float((got != want.float()).double().mean()) < 2.0 ** -7
+
+
 # scales of A and B: below bfloat16's least number, 2^-133, a number's parts are lost, which counts where the other factor is large; the
 # last two bring numbers that are no normal floats, and sums of products that are none
 @pytest.mark.parametrize("m,n,k", [(1, 17, 257), (16, 129, 511), (33, 128, 513), (40, 130, 2048), (300, 127, 1100), (70, 300, 6144)])
