@@ -116,6 +116,11 @@ __device__ inline float least_of(float largest) { return largest > 0.f ? fmaxf(l
 __device__ inline bool in_doubt(float v, float least_a, float least_b) {
     return fmaf(-least_a, least_b, fabsf(v)) < 0.f || !(fabsf(v) <= 3.402823466e38f);
 }
+// No sum is in doubt where no factor lies above the one bound and every sum is a number not below the other (seen without a word between
+// the lanes; the limit of factors of 2^30 is 2^-30).
+__device__ inline bool beyond_doubt(float largest, float least_sum, float no_number) {
+    return largest <= 0x1p30f && least_sum >= 0x1p-30f && no_number == 0.f;
+}
 // The largest absolute value so far (of NaN any: it spoils its sum).  Two instructions for four numbers; from fmaxf and fabsf the
 // compiler makes more, to quiet NaN first.
 __device__ inline float largest_of(float so_far, const f32x4& v) {
@@ -183,26 +188,54 @@ constexpr int kStreamRun = 32;                         // elements of K a wave t
 constexpr int kStreamLoads = kStreamRun / 16;
 constexpr int kChain = 32;                             // elements of K whose products are added up before they meet a sum
 
-template <int kTilesM, int kWaves, int kDepth, int kEach, bool kVec>
+// The waves' sums of the workgroup's tiles, added and stored.
+template <int kTilesM, int kTilesN, int kWaves>
+__device__ inline void add_segments(const float (&sums)[kWaves][kTilesM][kTilesN][kStreamTile * kStreamTile], float* __restrict__ c, int m, int n,
+                                    int n0, const Epilogue& then) {
+    if (then.gated) {                                  // a tile's 16 rows of B are eight gates and their ups (n is whole tiles)
+        for (int e = threadIdx.x; e < kTilesM * kTilesN * 128; e += kWaves * kWave) {
+            const int t = e / (kTilesN * 128), j = e / 128 % kTilesN, row = t * 16 + e % 128 / 8, at = e % 128 / 8 * kStreamTile + e % 8;
+            if (row >= m || n0 + j * kStreamTile >= n) continue;
+            float gate = sums[0][t][j][at], up = sums[0][t][j][at + 8];
+#pragma unroll
+            for (int v = 1; v < kWaves; ++v) gate += sums[v][t][j][at], up += sums[v][t][j][at + 8];
+            c[static_cast<long>(row) * (n / 2) + n0 / 2 + j * 8 + e % 8] = glu_value(gate, up, then.act, then.limit);
+        }
+        return;
+    }
+    for (int e = threadIdx.x; e < kTilesM * kTilesN * 256; e += kWaves * kWave) {
+        const int t = e / (kTilesN * 256), j = e / 256 % kTilesN, row = t * 16 + e % 256 / 16, col = n0 + j * kStreamTile + e % 16;
+        if (row >= m || col >= n) continue;
+        float total = sums[0][t][j][e % 256];
+#pragma unroll
+        for (int v = 1; v < kWaves; ++v) total += sums[v][t][j][e % 256];     // (segments past K's end are zeros)
+        c[static_cast<long>(row) * n + col] = total;
+    }
+}
+
+template <int kTilesM, int kTilesN, int kWaves, int kDepth, int kEach, bool kVec>
 __global__ void __launch_bounds__(kWaves * kWave, kEach)
 gemm_f32_stream_kernel(const float* __restrict__ a, const float* __restrict__ b, float* __restrict__ c, int m, int n, int k, int segment,
                        Epilogue then) {
-    __shared__ float sums[kWaves][kTilesM][kStreamTile * kStreamTile];
+    __shared__ float sums[kWaves][kTilesM][kTilesN][kStreamTile * kStreamTile];
     static_assert(kDepth % 2 == 0, "a register's runs are all even ones or all odd ones");
     const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-    const int n0 = blockIdx.x * kStreamTile;
+    const int n0 = blockIdx.x * kTilesN * kStreamTile;
     const int r = lane % 16, h = (lane / 16) * 4;
-    const float* brow = b + static_cast<long>(n0 + r < n ? n0 + r : n - 1) * k;
-    const float* arow[kTilesM];
+    const float *brow[kTilesN], *arow[kTilesM];
+#pragma unroll
+    for (int j = 0; j < kTilesN; ++j) brow[j] = b + static_cast<long>(n0 + j * 16 + r < n ? n0 + j * 16 + r : n - 1) * k;
 #pragma unroll
     for (int t = 0; t < kTilesM; ++t) arow[t] = a + static_cast<long>(t * 16 + r < m ? t * 16 + r : m - 1) * k;
-    f32x4 sum[kTilesM] = {};
-    float largest_b = 0.f, largest_a[kTilesM] = {};
-    f32x4 w[kDepth][kStreamLoads], x[kDepth][kTilesM][kStreamLoads];
+    f32x4 sum[kTilesM][kTilesN] = {};
+    float largest_b[kTilesN] = {}, largest_a[kTilesM] = {};
+    f32x4 w[kDepth][kTilesN][kStreamLoads], x[kDepth][kTilesM][kStreamLoads];
     const int first = wave * segment, end = first + segment < k ? first + segment : k;
     const auto fetch = [&](int at, int into) {         // a run that lies whole before the segment's end
 #pragma unroll
-        for (int i = 0; i < kStreamLoads; ++i) w[into][i] = load_whole<kVec>(brow + at + i * 16 + h);
+        for (int j = 0; j < kTilesN; ++j)
+#pragma unroll
+            for (int i = 0; i < kStreamLoads; ++i) w[into][j][i] = load_whole<kVec>(brow[j] + at + i * 16 + h);
 #pragma unroll
         for (int t = 0; t < kTilesM; ++t)
 #pragma unroll
@@ -211,17 +244,26 @@ gemm_f32_stream_kernel(const float* __restrict__ a, const float* __restrict__ b,
     const auto multiply = [&](int from, bool odd) {     // (see kTerms)
 #pragma unroll
         for (int i = 0; i < kStreamLoads; i += 2) {
-            const Operand wp = operand_of(w[from][i], w[from][i + 1]);
-            largest_b = largest_of(largest_of(largest_b, w[from][i]), w[from][i + 1]);
+            Operand wp[kTilesN];
+#pragma unroll
+            for (int j = 0; j < kTilesN; ++j) {
+                wp[j] = operand_of(w[from][j][i], w[from][j][i + 1]);
+                largest_b[j] = largest_of(largest_of(largest_b[j], w[from][j][i]), w[from][j][i + 1]);
+            }
 #pragma unroll
             for (int t = 0; t < kTilesM; ++t) {
                 largest_a[t] = largest_of(largest_of(largest_a[t], x[from][t][i]), x[from][t][i + 1]);
                 const Operand xp = odd ? operand_of(-x[from][t][i], -x[from][t][i + 1]) : operand_of(x[from][t][i], x[from][t][i + 1]);
-                f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+                f32x4 acc[kTilesN] = {};
 #pragma unroll
-                for (int e = 0; e < kTerms; ++e) acc = add_term(e, xp, wp, acc);
-                acc += highest_term(xp, wp);
-                sum[t] = odd ? sum[t] - acc : sum[t] + acc;
+                for (int e = 0; e < kTerms; ++e)
+#pragma unroll
+                    for (int j = 0; j < kTilesN; ++j) acc[j] = add_term(e, xp, wp[j], acc[j]);
+#pragma unroll
+                for (int j = 0; j < kTilesN; ++j) {
+                    acc[j] += highest_term(xp, wp[j]);
+                    sum[t][j] = odd ? sum[t][j] - acc[j] : sum[t][j] + acc[j];
+                }
                 __builtin_amdgcn_sched_barrier(0);     // (interleaved with the next ones' products the waves' number would not fit the registers)
             }
         }
@@ -255,52 +297,158 @@ gemm_f32_stream_kernel(const float* __restrict__ a, const float* __restrict__ b,
     at += left * kStreamRun;
     if (at < end) {                                    // the rest of the last segment, filled up with zeros
 #pragma unroll
-        for (int i = 0; i < kStreamLoads; ++i) w[0][i] = load_four<kVec>(brow, at + i * 16 + h, end);
+        for (int j = 0; j < kTilesN; ++j)
+#pragma unroll
+            for (int i = 0; i < kStreamLoads; ++i) w[0][j][i] = load_four<kVec>(brow[j], at + i * 16 + h, end);
 #pragma unroll
         for (int t = 0; t < kTilesM; ++t)
 #pragma unroll
             for (int i = 0; i < kStreamLoads; ++i) x[0][t][i] = load_four<kVec>(arow[t], at + i * 16 + h, end);
         left % 2 ? multiply(0, true) : multiply(0, false);
     }
-    const float least_b = least_of(max_lanes<16>(max_lanes<32>(largest_b)));
+    float largest = 0.f, least_sum = INFINITY, no_number = 0.f;
 #pragma unroll
     for (int t = 0; t < kTilesM; ++t) {
-        const float least_a = least_of(max_lanes<16>(max_lanes<32>(largest_a[t])));
+        largest = fmaxf(largest, largest_a[t]);
+#pragma unroll
+        for (int j = 0; j < kTilesN; ++j) {
+            largest = fmaxf(largest, largest_b[j]);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) least_sum = fminf(least_sum, fabsf(sum[t][j][i])), no_number = fmaf(sum[t][j][i], 0.f, no_number);
+        }
+    }
+    if (!__all(beyond_doubt(largest, least_sum, no_number))) {
+        float least_b[kTilesN];
+#pragma unroll
+        for (int j = 0; j < kTilesN; ++j) least_b[j] = least_of(max_lanes<16>(max_lanes<32>(largest_b[j])));
+#pragma unroll
+        for (int t = 0; t < kTilesM; ++t) {
+            const float least_a = least_of(max_lanes<16>(max_lanes<32>(largest_a[t])));
+            float least[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) least[i] = __shfl(least_a, h + i, kWave);
+#pragma unroll
+            for (int j = 0; j < kTilesN; ++j) {
+                const auto doubt = [&](int i) { return in_doubt(sum[t][j][i], least[i], least_b[j]); };
+                if (!__any(doubt(0) || doubt(1) || doubt(2) || doubt(3))) continue;
+                const f32x4 plain = plain_square<kVec>(arow[t], brow[j], first, end, lane / 16);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) sum[t][j][i] = doubt(i) ? plain[i] : sum[t][j][i];
+            }
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < kTilesM; ++t)
+#pragma unroll
+        for (int j = 0; j < kTilesN; ++j)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) sums[wave][t][j][(h + i) * kStreamTile + r] = sum[t][j][i];
+    __syncthreads();
+    add_segments<kTilesM, kTilesN, kWaves>(sums, c, m, n, n0, then);
+}
+
+// Up to eight rows: half of the instruction's 16 rows of A are taken for the run after, so that A is asked for and taken apart
+// once for two runs (a third of the taking apart, which is most of a wave's instructions).  Of the first run's products rows 0 .. 7 count, of
+// the second's (whose B has its sign turned, see kTerms) rows 8 .. 15, which the other half of the wave holds.
+constexpr int kFewRows = 8;
+constexpr long kManyTiles = 1024;
+
+template <int kWaves, int kAhead, int kEach, bool kVec>
+__global__ void __launch_bounds__(kWaves * kWave, kEach)
+gemm_f32_few_kernel(const float* __restrict__ a, const float* __restrict__ b, float* __restrict__ c, int m, int n, int k, int segment,
+                    Epilogue then) {
+    constexpr int kPair = 2 * kStreamRun;
+    __shared__ float sums[kWaves][1][1][kStreamTile * kStreamTile];
+    const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+    const int n0 = blockIdx.x * kStreamTile;
+    const int r = lane % 16, h = (lane / 16) * 4, later = r < kFewRows ? 0 : kStreamRun;
+    const float* brow = b + static_cast<long>(n0 + r < n ? n0 + r : n - 1) * k;
+    const float* arow = a + static_cast<long>(r % kFewRows < m ? r % kFewRows : m - 1) * k;
+    f32x4 sum = {0.f, 0.f, 0.f, 0.f};                  // (of the lower half of the wave)
+    float largest_a = 0.f, largest_b = 0.f;
+    f32x4 w[kAhead][2][kStreamLoads], x[kAhead][kStreamLoads];
+    const int first = wave * segment, end = first + segment < k ? first + segment : k;
+    const auto fetch_a = [&](int at, int into) {       // a pair of runs that lies whole before the segment's end
+#pragma unroll
+        for (int i = 0; i < kStreamLoads; ++i) x[into][i] = load_whole<kVec>(arow + at + later + i * 16 + h);
+    };
+    const auto fetch_b = [&](int at, int into, int run) {
+#pragma unroll
+        for (int i = 0; i < kStreamLoads; ++i) w[into][run][i] = load_whole<kVec>(brow + at + run * kStreamRun + i * 16 + h);
+    };
+    // the pair in the registers `of`; another one from `next` on is asked for as they become free
+    const auto multiply = [&](int of, bool more, int next) {
+        const Operand xp = operand_of(x[of][0], x[of][1]);
+        largest_a = largest_of(largest_of(largest_a, x[of][0]), x[of][1]);
+        if (more) fetch_a(next, of);
+        f32x4 acc[2];
+#pragma unroll
+        for (int run = 0; run < 2; ++run) {
+            const f32x4 w0 = w[of][run][0], w1 = w[of][run][1];
+            const Operand wp = run ? operand_of(-w0, -w1) : operand_of(w0, w1);
+            largest_b = largest_of(largest_of(largest_b, w0), w1);
+            if (more) fetch_b(next, of, run);
+            acc[run] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int e = 0; e < kTerms; ++e) acc[run] = add_term(e, xp, wp, acc[run]);
+            acc[run] += highest_term(xp, wp);
+            if (run == 0) sum += acc[0];
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e)                    // (the upper half's results to the lower one)
+            sum[e] -= __uint_as_float(__builtin_amdgcn_permlane32_swap(__float_as_uint(acc[1][e]), __float_as_uint(acc[0][e]), false, false)[1]);
+    };
+    int left = end > first ? (end - first) / kPair : 0, at = first;
+    if (left >= kAhead) {
+#pragma unroll
+        for (int d = 0; d < kAhead; ++d) fetch_a(at + d * kPair, d), fetch_b(at + d * kPair, d, 0), fetch_b(at + d * kPair, d, 1);
+        for (; left >= 2 * kAhead; left -= kAhead, at += kAhead * kPair)
+#pragma unroll
+            for (int d = 0; d < kAhead; ++d) multiply(d, true, at + (kAhead + d) * kPair);
+#pragma unroll
+        for (int d = 0; d < kAhead; ++d) multiply(d, kAhead + d < left, at + (kAhead + d) * kPair);
+        left -= kAhead, at += kAhead * kPair;
+    } else {
+#pragma unroll
+        for (int d = 0; d < kAhead - 1; ++d)
+            if (d < left) fetch_a(at + d * kPair, d), fetch_b(at + d * kPair, d, 0), fetch_b(at + d * kPair, d, 1);
+    }
+#pragma unroll
+    for (int d = 0; d < kAhead - 1; ++d)
+        if (d < left) multiply(d, false, 0);
+    at += left * kPair;
+    if (at < end) {                                    // the rest of the last segment, filled up with zeros
+#pragma unroll
+        for (int i = 0; i < kStreamLoads; ++i) {
+            x[0][i] = load_four<kVec>(arow, at + later + i * 16 + h, end);
+#pragma unroll
+            for (int run = 0; run < 2; ++run) w[0][run][i] = load_four<kVec>(brow, at + run * kStreamRun + i * 16 + h, end);
+        }
+        multiply(0, false, 0);
+    }
+    const bool mine = lane < kWave / 2;
+    float least_sum = INFINITY, no_number = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) least_sum = fminf(least_sum, fabsf(sum[i])), no_number = fmaf(sum[i], 0.f, no_number);
+    if (!__all(beyond_doubt(fmaxf(largest_a, largest_b), mine ? least_sum : 1.0f, mine ? no_number : 0.f))) {
+        const float least_b = least_of(max_lanes<16>(max_lanes<32>(largest_b)));
+        const float least_a = least_of(max_lanes<8>(max_lanes<16>(max_lanes<32>(largest_a))));
         float least[4];
-        bool any = false;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            least[i] = __shfl(least_a, h + i, kWave);
-            any |= in_doubt(sum[t][i], least[i], least_b);
+        for (int i = 0; i < 4; ++i) least[i] = __shfl(least_a, h + i, kWave);
+        const auto doubt = [&](int i) { return mine && in_doubt(sum[i], least[i], least_b); };
+        if (__any(doubt(0) || doubt(1) || doubt(2) || doubt(3))) {
+            const f32x4 plain = plain_square<kVec>(arow, brow, first, end, lane / 16);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) sum[i] = doubt(i) ? plain[i] : sum[i];
         }
-        if (__any(any)) {
-            const f32x4 plain = plain_square<kVec>(arow[t], brow, first, end, lane / 16);
+    }
+    if (mine) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) sum[t][i] = in_doubt(sum[t][i], least[i], least_b) ? plain[i] : sum[t][i];
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) sums[wave][t][(h + i) * kStreamTile + r] = sum[t][i];
+        for (int i = 0; i < 4; ++i) sums[wave][0][0][(h + i) * kStreamTile + r] = sum[i];
     }
     __syncthreads();
-    if (then.gated) {                                  // the tile's 16 rows of B are eight gates and their ups
-        for (int e = threadIdx.x; e < kTilesM * 128; e += kWaves * kWave) {
-            const int t = e / 128, row = t * 16 + e % 128 / 8, at = e % 128 / 8 * kStreamTile + e % 8;
-            if (row >= m) continue;
-            float gate = sums[0][t][at], up = sums[0][t][at + 8];
-#pragma unroll
-            for (int v = 1; v < kWaves; ++v) gate += sums[v][t][at], up += sums[v][t][at + 8];
-            c[static_cast<long>(row) * (n / 2) + n0 / 2 + e % 8] = glu_value(gate, up, then.act, then.limit);
-        }
-        return;
-    }
-    for (int e = threadIdx.x; e < kTilesM * 256; e += kWaves * kWave) {
-        const int t = e / 256, row = t * 16 + e % 256 / 16, col = n0 + e % 16;
-        if (row >= m || col >= n) continue;
-        float total = sums[0][t][e % 256];
-#pragma unroll
-        for (int v = 1; v < kWaves; ++v) total += sums[v][t][e % 256];        // (segments past K's end are zeros)
-        c[static_cast<long>(row) * n + col] = total;
-    }
+    add_segments<1, 1, kWaves>(sums, c, m, n, n0, then);
 }
 
 // ---- many rows -----------------------------------------------------------------------------------------------------
@@ -471,7 +619,7 @@ gemm_f32_tile_kernel(const float* __restrict__ a, const float* __restrict__ b, f
             for (int j = 0; j < kFragB; ++j) acc[j] += highest_term(ap, bp[j]);
 #pragma unroll
             for (int j = 0; j < kFragB; ++j) sum[i][j] = acc[j] * sign + sum[i][j];        // (one instruction, and exact)
-            __builtin_amdgcn_sched_barrier(0);             // (the next one's operands ahead of these sums would not fit the registers)
+            if constexpr (kFragB > 1) __builtin_amdgcn_sched_barrier(0);             // (the next one's operands ahead of these sums would not fit the registers)
         }
         if (k0 + kSlab < k_end) kept(k0 + kSlab);
         fetch_a(k0 + 2 * kSlab);
@@ -681,10 +829,11 @@ gemm_f32_sum_gated_kernel(const float* __restrict__ planes, float* __restrict__ 
     }
 }
 
-// Up to here a product is a stream of weights.  Measured (us, streamed : tiled) against 2048 x 2048 weights 11.4 : 12.1 at 17 rows,
-// 13.7 : 12.5 at 32, 3072 x 512 5.9 : 9.7 at 32, 6144 x 1024 13.9 : 14.4; beyond, the stream's reads of A, then four times the
-// weights', cost more.  A long K leaves the tiles' workgroups enough to do from the second tile of rows on: 1024 x 3072 15.1 : 14.6
-// and 18.9 : 15.0 at 17 and 32 rows, 2048 x 6144 27.9 : 26.4 and 35.5 : 26.8.
+// Up to here a product is a stream of weights.  Measured (us, streamed : tiled) against 2048 x 2048 weights 10.7 : 12.4 at 17 rows,
+// 13.1 : 13.1 at 32, 3072 x 512 5.5 : 10.1 at 32, 6144 x 1024 13.2 : 15.7, 12288 x 2048 36.0 : 35.2, 32768 x 2048 74.7 : 77.9 and 89.9 : 83.2 at 17
+// and 32; beyond, the stream's reads of A, then four times the weights', cost more.  A long K leaves the tiles' workgroups enough to do
+// from the second tile of rows on: with six products of parts 1024 x 3072 15.1 : 14.6 and 18.9 : 15.0 at 17 and 32 rows, 2048 x 6144 27.9 : 26.4
+// and 35.5 : 26.8.
 constexpr int kStreamRows = 32;
 constexpr int kStreamLongK = 3072;
 constexpr int kStreamK = 256;          // a shorter K is no work to share out over four waves: one chain, in tiles whatever the rows
@@ -723,8 +872,8 @@ F32Plan f32_chain_plan(int m, int n) {
 // The tile's width and the cut of K that take least time.  Up to four workgroups of a unit work side by side: a slab takes them the longer
 // of a workgroup's own way through it and of what they ask of the unit together.  A cut K costs a plane written and read for every
 // segment (mostly in the caches) and a second launch.  Constants (microseconds; bytes a microsecond) fitted to both tiles and every cut
-// timed at 17 to 2,048 rows against the matrices of layers of 512, 1,024 and 2,048 channels: the choice is 0.4 % off the best on
-// average and 10 % at worst.
+// timed at 17 to 2,048 rows against the matrices of layers of 512, 1,024, 2,048 and 4,096 channels: the choice is 0.5 % off the best on
+// average and 8 % at worst (512 rows against 4096 x 12288 408 us, 378 with every segment a workgroup).
 F32Plan f32_plan(int m, int n, int k) {
     F32Plan best;
     if (k < kStreamK) return f32_chain_plan(m, n);
@@ -760,25 +909,35 @@ int launch_f32(const F32Plan& p, const float* a, const float* b, float* c, float
     const auto aligned = [](const void* at) { return reinterpret_cast<uintptr_t>(at) % 16 == 0; };
     const bool vec = k % 4 == 0 && aligned(a) && aligned(b);
     if (p.rows == 0) {
-        const int blocks = ceil_div(n, kStreamTile);
-#define LEONE_STREAM(T, W, D, E)                                                                                                       \
-    (vec ? gemm_f32_stream_kernel<T, W, D, E, true><<<blocks, W * kWave, 0, stream>>>(a, b, c, m, n, k, segments.length, then)         \
-         : gemm_f32_stream_kernel<T, W, D, E, false><<<blocks, W * kWave, 0, stream>>>(a, b, c, m, n, k, segments.length, then))
-        // Runs on their way a wave: two leave room for more waves, whose loads count as well, and segments of few runs have no use for
-        // more; of a large matrix four (us, two and four runs: one row against 12288 x 2048 21.2 and 19.0, 32768 x 2048 48.1 and 44.0,
-        // 2048 x 6144 17.7 and 17.2; but 2048 x 2048 7.1 and 7.4, 1024 x 3072 10.9 and 11.5, five rows against 32768 x 512 16.4 and
-        // 18.7).  Two tiles of A fill the registers: 24 rows against 12288 x 2048 32.5 with two, 37.0 with three.
-        const bool large = segments.length >= 256 && static_cast<long>(n) * k >= 8l << 20;
+#define LEONE_FEW(W, D, E)                                                                                                             \
+    (vec ? gemm_f32_few_kernel<W, D, E, true><<<ceil_div(n, kStreamTile), W * kWave, 0, stream>>>(a, b, c, m, n, k, segments.length, then) \
+         : gemm_f32_few_kernel<W, D, E, false><<<ceil_div(n, kStreamTile), W * kWave, 0, stream>>>(a, b, c, m, n, k, segments.length, then))
+#define LEONE_STREAM(T, N, W, D, E)                                                                                                    \
+    (vec ? gemm_f32_stream_kernel<T, N, W, D, E, true><<<ceil_div(n, N * kStreamTile), W * kWave, 0, stream>>>(a, b, c, m, n, k, segments.length, then)  \
+         : gemm_f32_stream_kernel<T, N, W, D, E, false><<<ceil_div(n, N * kStreamTile), W * kWave, 0, stream>>>(a, b, c, m, n, k, segments.length, then))
+        // Up to eight rows one pair of runs on its way a wave; of a large matrix two, for two waves a SIMD (us, one and two pairs: one row
+        // against 12288 x 2048 19.6 and 18.8, five against 24576 x 4096 72.5 and 69.7, 32768 x 2048 49.5 and 47.7; but 4096 x 2048 7.6 and 7.8,
+        // 32768 x 1024 26.8 and 27.4).  Beyond, two runs; where there are many tiles and more than eight rows or short segments, two tiles
+        // of B share what A's parts cost (one and two tiles: 16 rows against 32768 x 2048 64.6 and 53.5, 24576 x 4096 96.3 and 76.8, one row against
+        // 32768 x 512 16.6 and 14.6; but 16 against 12288 x 2048 26.6 and 27.0, 4096 x 2048 9.8 and 13.6).
+        const bool large = segments.length >= 256 && static_cast<long>(n) * k >= 16l << 20;
+        const bool many = n >= kManyTiles * kStreamTile && (m > kFewRows || segments.length <= 64);
         if (segments.count <= 4) {
-            if (m <= kStreamTile) LEONE_STREAM(1, 4, 2, 6);
-            else LEONE_STREAM(2, 4, 2, 2);
+            if (m <= kFewRows) LEONE_FEW(4, 1, 4);
+            else if (m <= kStreamTile) LEONE_STREAM(1, 1, 4, 2, 4);
+            else LEONE_STREAM(2, 1, 4, 2, 2);
         } else if (m > kStreamTile) {
-            LEONE_STREAM(2, 8, 2, 2);
+            LEONE_STREAM(2, 1, 8, 2, 2);
+        } else if (many) {
+            LEONE_STREAM(1, 2, 8, 2, 4);
+        } else if (m > kFewRows) {
+            LEONE_STREAM(1, 1, 8, 2, 4);
         } else if (large) {
-            LEONE_STREAM(1, 8, 4, 4);
+            LEONE_FEW(8, 2, 2);
         } else {
-            LEONE_STREAM(1, 8, 2, 6);
+            LEONE_FEW(8, 1, 4);
         }
+#undef LEONE_FEW
 #undef LEONE_STREAM
         LEONE_LAUNCH_CHECK("gemm_f32");
         return 0;

@@ -66,6 +66,23 @@ def test_a_row_is_the_same_whatever_rows_are_beside_it(n, k):
         assert torch.equal(ops.gemm_f32(moved, b), together), m
 
 
+@pytest.mark.parametrize("n,k", [(33, 257), (40, 511), (40, 520), (40, 545), (96, 577), (16401, 512), (16400, 515), (16392, 2048), (8200, 2084)])
+def test_few_rows_give_the_bits_of_many(n, k):
+    """Two runs an instruction (up to eight rows) and two tiles a workgroup (many of them): ends of K off a pair of runs, a last tile
+    alone, and rows whose sums are made again beside others."""
+    from leone_amd import ops
+    gen = torch.Generator(device=DEV).manual_seed(k)
+    a, b = torch.randn(64, k, generator=gen, device=DEV), torch.randn(n, k, generator=gen, device=DEV)
+    a[1, k - 1], a[4] = math.nan, 0.0
+    a[5] *= 1e-36
+    b[n - 1, 0], b[n - 2] = math.inf, 0.0
+    many = ops.gemm_f32(a, b).nan_to_num(7.5, 8.5, 9.5)
+    for m in (1, 2, 7, 8, 9, 16, 17):
+        for shift in (0, 1):
+            rows = torch.empty(m * k + shift, device=DEV)[shift:].view(m, k).copy_(a[:m])
+            assert torch.equal(ops.gemm_f32(rows, b).nan_to_num(7.5, 8.5, 9.5), many[:m]), (m, shift)
+
+
 def test_results_off_sixteen_bytes():
     """Where K is cut, the sum over its parts writes a result that lies anywhere."""
     from leone_amd import ops
