@@ -96,12 +96,13 @@ __device__ inline void route_row(int row, int lane, const float* __restrict__ lo
     // `always` experts that every row takes with weight 1 stand behind the routed ones in the matrices (indices
     // shift_from .. shift_from + always - 1): a row's places are its `top` choices and then these; a chosen router
     // output from shift_from on (one that hands the row on) is numbered behind them.
-    // here: a second copy of the first `room` choices of all rows, for the workgroup's own use.
+    // here: a second copy of the first `room` choices of all rows, for the workgroup's own use (not with kRouteSlots outputs a lane).
     const int places = top + always;
     const auto choose = [&](int place, int e) {
         const long at = static_cast<long>(row) * places + place;
         chosen[at] = e;
-        if (at < room) here[at] = e;
+        if constexpr (kSlots < kRouteSlots)
+            if (at < room) here[at] = e;
     };
     const float* z = logits + static_cast<long>(row) * total;
     float s[kSlots], choice[kSlots];
@@ -340,7 +341,8 @@ moe_plan_kernel(const int* __restrict__ chosen, int pairs, int experts, int* __r
 // its logits), and the choices are handed to the plan through shared memory (kPlanPairs of them; more are read back from where
 // they were written).  kSlots: outputs a lane; each number is a kernel of its own, without the others' registers.  One behind the
 // other in a recording: 8 rows over 64 outputs 7.5 -> 6.1 us, 64 rows over 64 in 8 groups 28.4 -> 26.0, 64 over 256 (4 outputs a lane,
-// not 8) 47.7 -> 36.5; over 512, where the copy in shared memory gave nothing and is not made, 49.8 -> 50.7.
+// not 8) 47.7 -> 36.5.  With 8 outputs a lane the copy in shared memory gave nothing and is not made, and of 16 and more rows the tiles are
+// cleared behind a barrier of their own (64 over 512 as before 50.2, without the barrier 50.6, with the copy 51.1).
 constexpr int kPlanPairs = 2048;
 
 template <int kSlots>
@@ -357,6 +359,7 @@ route_plan_kernel(const float* __restrict__ logits, AnyVec correction, int* __re
     const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     for (int row = wave; row < rows; row += kWaves)
         route_row<kSlots>(row, lane, logits, correction, chosen, weight, total, top, group_count, group_keep, rule, routed, always, here, room);
+    if (kSlots == kRouteSlots && rows >= kWaves) __syncthreads();
     if (rows >= kWaves) clear_tiles(experts, tile_expert, tile_pairs, max_tiles, tile, count);
     else if (wave >= rows) clear_tiles(experts, tile_expert, tile_pairs, max_tiles, tile, count, rows * kWave);
     __syncthreads();                                   // the choices are written; the same workgroup reads them
