@@ -33,8 +33,9 @@
 // another order there).  Head sizes that are multiples of 64 only: there a lane holds both halves of its pairs.
 //
 // With few keys a call is a chain of trips to memory, and their order is what it costs: what norms and rotation
-// start from is asked for first, before the row's position is known; then the angles; then the block table; then every
-// wave's first tile, whose way from memory covers the arithmetic on the heads.  Two rows of 100 keys, 8 heads over 2:
+// start from is asked for first, before the row's position is known; then the angles, and by the last wave, which has no heads to make,
+// the page ids; then the waves without heads of queries or keys ask for their first tile, the other two once their heads are made (what
+// the heads start from would stand in the queue with the tile).  Two rows of 100 keys, 8 heads over 2:
 // 9.1 us with the launch (11.1 when every wave made the queries for itself and all waited for the new key to come
 // back from the cache).
 //
@@ -384,7 +385,7 @@ attention_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__
     // wave waits for a write to come back.
     const bool writes = kFused && from.k_out != nullptr && my_begin < my_end && my_end == n_tiles;
     [[maybe_unused]] const int page = writes ? table[pos >> page_shift] : -1;   // the host reserves the page before the launch
-    // The wave's first tile is asked for before the queries are made: neither waits for the other.
+    // Waves that make no heads ask for their first tile before the queries are there: neither waits for the other.
     Tile one, two;
     if ((!kFused || wave >= 2) && my_begin + wave < my_end) issue(my_begin + wave, true, one, true);
     if constexpr (!kFused) __syncthreads();            // the page ids are there (else where the queries are)

@@ -25,7 +25,7 @@ def pools(k, v, page_tokens, seed):
 
 
 def both(rows, group, kv_heads, size, tokens=150, spoil=None, unmapped=None, **options):
-    """``rows``: (request, position) of every row.  Results of the two kernels, pages of 16 and 64 the second."""
+    """``rows``: (request, position) of every row.  Results of the two kernels, pages of 16, 64 and 48 (no power of two) the second."""
     from leone_amd import ops
     gen = torch.Generator().manual_seed(17)
     requests = 1 + max(r for r, _ in rows)
@@ -36,7 +36,7 @@ def both(rows, group, kv_heads, size, tokens=150, spoil=None, unmapped=None, **o
     entry = torch.tensor([r for r, _ in rows], dtype=torch.int32, device=DEV)
     positions = torch.tensor([p for _, p in rows], dtype=torch.int32, device=DEV)
     results = []
-    for page_tokens in (8, 16, 64):
+    for page_tokens in (8, 16, 64, *(() if unmapped else (48,))):          # (64 positions that are gone are no whole pages of 48)
         k_pool, v_pool, table = pools(k, v, page_tokens, page_tokens)
         for request, position in unmapped or []:        # 64 positions are gone, whatever the pages' size
             table[request, position // page_tokens:(position + 64) // page_tokens] = -1

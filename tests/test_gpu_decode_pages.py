@@ -104,20 +104,22 @@ def test_a_key_without_a_page_spoils_the_rows_that_see_it():
 
 
 @pytest.mark.parametrize("size", [16, 64, 80, 112, 128, 144, 256])
-@pytest.mark.parametrize("splits", [2, 7, 8, 9, 63, 64, 65])
+@pytest.mark.parametrize("splits", [2, 7, 8, 9, 17, 32, 63, 64, 65])
 def test_ranges_are_merged_whatever_their_number(size, splits):
-    """Up to 64 ranges by lanes, more through shared memory; more ranges than tiles leave empty ones."""
+    """Up to 64 ranges by lanes, more through shared memory, all of them with keys (66 tiles); the shorter rows leave empty ones."""
     from leone_amd import ops
-    places = [0, 40, 329]
-    k, v = made(2, size, 3)
+    places = [0, 40, 329, 65 * 32 + 19]
+    tokens = places[-1] + 1
+    gen = torch.Generator().manual_seed(3)
+    k, v = [torch.randn(len(places), tokens, 2, size, generator=gen).bfloat16().float() for _ in range(2)]
     k_pool, v_pool, table = pools(k, v, 64, 1)
-    q = torch.randn(3, 6 * size, generator=torch.Generator().manual_seed(1)).bfloat16().to(DEV)
-    args = (q, bits(k_pool), bits(v_pool), torch.tensor(places, dtype=torch.int32, device=DEV), torch.arange(3, dtype=torch.int32, device=DEV),
-            table, 6, size ** -0.5)
-    whole = ops.attention_decode(*args, max_context=TOKENS, splits=1).float()
-    cut = ops.attention_decode(*args, max_context=TOKENS, splits=splits).float()
-    # the weights are the same numbers however the keys are cut; sums in another order round once more to bfloat16
-    assert float((whole - cut).abs().max()) <= 2.0 ** -7 * float(whole.abs().max())
+    q = torch.randn(len(places), 6 * size, generator=torch.Generator().manual_seed(1)).bfloat16().to(DEV)
+    args = (q, bits(k_pool), bits(v_pool), torch.tensor(places, dtype=torch.int32, device=DEV),
+            torch.arange(len(places), dtype=torch.int32, device=DEV), table, 6, size ** -0.5)
+    whole = ops.attention_decode(*args, max_context=tokens, splits=1).float()
+    cut = ops.attention_decode(*args, max_context=tokens, splits=splits).float()
+    # the weights are the same numbers however the keys are cut; sums in another order round once more to bfloat16, row by row
+    assert bool(((whole - cut).abs().amax(1) <= 2.0 ** -7 * whole.abs().amax(1)).all())
 
 
 @pytest.mark.parametrize("hidden", [4, 6, 64, 1000, 1023, 4096])
