@@ -142,8 +142,8 @@ __device__ inline f32x4 transpose_quarters(const f32x4 v) {
 // instruction's results do, and depends on an output's own two rows alone.  The 16 x 16 x 4 instruction adds its four products in the
 // order of the lanes' quarters, so the four quarters' registers are transposed by lane swaps: instruction j takes elements 4 j .. 4 j + 3
 // in turn; the next run is on its way meanwhile.  (By a loop over K for every output in doubt, a row that is not a number held up whoever
-// shared its launch.  us, all sums ordinary, one row NaN by a loop and so, all rows by a loop and so: one row against 2048 x 2048 10, 100,
-// 12, 248, 16; 200 rows against 3072 x 2048 30, 79, 41, 2842, 108; 777 against 12288 x 2048 256, 287, 252, 38668, 1379.)
+// shared its launch.  us, all sums ordinary, one row NaN, all rows: one row against 2048 x 2048 6.5, 14, 14 (by a loop 100); five against 32768 x
+// 2048 44, 94, 90; 200 against 3072 x 2048 36, 48, 113 (79 and 2842); 777 against 12288 x 2048 298, 344, 1408 (287 and 38668).)
 constexpr int kPlainRun = 16;                          // elements of K on their way at a time
 template <bool kVec>
 __device__ inline f32x4 plain_square(const float* __restrict__ arow, const float* __restrict__ brow, int first, int end, int g) {
@@ -462,8 +462,8 @@ gemm_f32_few_kernel(const float* __restrict__ a, const float* __restrict__ b, fl
 // What bounds it is that the matrix instructions (eight for what one product of floats needs), the taking apart (half of the vector
 // instructions) and the trips through shared memory follow one another within a wave; three workgroups a unit make up for it to half of
 // the instructions' rate.  Columns of their own keep B out of shared memory (777 rows against 12288 x 2048, with six products of parts:
-// 243 us, with both operands in shared memory 303).  With eight 777 rows against 12288 x 2048 take 315 us, 2048 x 6144 169, of which six would be
-// 266 and 148; on the float instructions 440 and 219.
+// 243 us, with both operands in shared memory 303).  With eight 777 rows take 300 to 320 us there and 170 against 2048 x 6144 (with six on the
+// same card 266 and 148; on the float instructions 440 and 219).
 //
 // kCut: blockIdx.z takes `each` segments and leaves a plane of c for every one of them; else one workgroup walks them all.
 constexpr int kSlab = kChain;
