@@ -87,6 +87,15 @@ def test_gated_products_of_many_rows(kernels):
     assert len(gated) == 3 and all(k[".vgpr_count"] <= 168 for k in gated)
 
 
+def test_float_products(kernels):
+    """Nothing in scratch; where the weights are streamed, four waves a SIMD (their loads are what counts), in tiles three."""
+    streams = [k for name, k in kernels.items() if "gemm_f32_few_kernel" in name or "gemm_f32_stream_kernel" in name]
+    tiles = [k for name, k in kernels.items() if "gemm_f32_tile_kernel" in name]
+    assert len(streams) == 16 and len(tiles) == 8
+    for k, most in [(k, 128) for k in streams] + [(k, 168) for k in tiles]:
+        assert k[".vgpr_count"] <= most and k[".private_segment_fixed_size"] == 0, k[".name"]
+
+
 def test_attention_with_mixed_scores(kernels):
     """What 32 heads of 128 leave to scratch, with keys of their own and with keys that four share, and no more; smaller ones less or nothing."""
     found = {name.split("attention_talk_prefill_kernel")[1][:24]: k[".private_segment_fixed_size"] for name, k in kernels.items()
