@@ -137,6 +137,11 @@ __device__ inline f32x4 transpose_quarters(const f32x4 v) {
     const u32x2 s = __builtin_amdgcn_permlane16_swap(p[1], q[1], false, false);
     return f32x4{__uint_as_float(r[0]), __uint_as_float(r[1]), __uint_as_float(s[0]), __uint_as_float(s[1])};
 }
+// Elements of a normed row, rounded as the norm's own kernel rounds them (not taken into a subtraction of what follows).
+__device__ inline f32x4 normed(const f32x4& v, const f32x4& gain, float inv) {
+#pragma clang fp contract(off)
+    return v * gain * inv;
+}
 // The segment's sums of a square of 16 x 16 outputs on the float instructions: 16 products a chain, k ascending, and the chains' sums
 // added in order.  This lane's row of A and row of B are those of number lane % 16 of the square; what comes out lies as the bfloat16
 // instruction's results do, and depends on an output's own two rows alone.  The 16 x 16 x 4 instruction adds its four products in the
@@ -145,19 +150,26 @@ __device__ inline f32x4 transpose_quarters(const f32x4 v) {
 // shared its launch.  us, all sums ordinary, one row NaN, all rows: one row against 2048 x 2048 6.5, 14, 14 (by a loop 100); five against 32768 x
 // 2048 44, 94, 90; 200 against 3072 x 2048 36, 48, 113 (79 and 2842); 777 against 12288 x 2048 298, 344, 1408 (287 and 38668).)
 constexpr int kPlainRun = 16;                          // elements of K on their way at a time
-template <bool kVec>
-__device__ inline f32x4 plain_square(const float* __restrict__ arow, const float* __restrict__ brow, int first, int end, int g) {
+// kNormed: A's elements are (a * gain) * inv.
+template <bool kVec, bool kNormed = false>
+__device__ inline f32x4 plain_square(const float* __restrict__ arow, const float* __restrict__ brow, int first, int end, int g,
+                                     const float* __restrict__ gain = nullptr, float inv = 1.0f) {
+    const auto of_a = [&](int at) {
+        f32x4 v = load_four<kVec>(arow, at, end);
+        if constexpr (kNormed) v = normed(v, load_four<kVec>(gain, at, end), inv);
+        return v;
+    };
     f32x4 sum = {0.f, 0.f, 0.f, 0.f};
     constexpr int kLoads = kPlainRun / 16;
     f32x4 x[kLoads], y[kLoads];
 #pragma unroll
-    for (int i = 0; i < kLoads; ++i) x[i] = load_four<kVec>(arow, first + i * 16 + 4 * g, end), y[i] = load_four<kVec>(brow, first + i * 16 + 4 * g, end);
+    for (int i = 0; i < kLoads; ++i) x[i] = of_a(first + i * 16 + 4 * g), y[i] = load_four<kVec>(brow, first + i * 16 + 4 * g, end);
 #pragma unroll 1
     for (int at = first; at < end; at += kPlainRun) {
         f32x4 next_x[kLoads], next_y[kLoads];
 #pragma unroll
         for (int i = 0; i < kLoads; ++i) {
-            next_x[i] = load_four<kVec>(arow, at + kPlainRun + i * 16 + 4 * g, end);
+            next_x[i] = of_a(at + kPlainRun + i * 16 + 4 * g);
             next_y[i] = load_four<kVec>(brow, at + kPlainRun + i * 16 + 4 * g, end);
         }
 #pragma unroll
@@ -189,9 +201,11 @@ constexpr int kStreamLoads = kStreamRun / 16;
 constexpr int kChain = 32;                             // elements of K whose products are added up before they meet a sum
 
 // The waves' sums of the workgroup's tiles, added and stored.
-template <int kTilesM, int kTilesN, int kWaves>
+// kAdds (one tile): what lay in c before, of the thread's one element, is added.
+template <int kTilesM, int kTilesN, int kWaves, bool kAdds = false>
 __device__ inline void add_segments(const float (&sums)[kWaves][kTilesM][kTilesN][kStreamTile * kStreamTile], float* __restrict__ c, int m, int n,
-                                    int n0, const Epilogue& then) {
+                                    int n0, const Epilogue& then, float before = 0.f) {
+    static_assert(!kAdds || (kTilesM == 1 && kTilesN == 1 && kWaves * kWave >= 256), "an element a thread");
     if (then.gated) {                                  // a tile's 16 rows of B are eight gates and their ups (n is whole tiles)
         for (int e = threadIdx.x; e < kTilesM * kTilesN * 128; e += kWaves * kWave) {
             const int t = e / (kTilesN * 128), j = e / 128 % kTilesN, row = t * 16 + e % 128 / 8, at = e % 128 / 8 * kStreamTile + e % 8;
@@ -209,7 +223,7 @@ __device__ inline void add_segments(const float (&sums)[kWaves][kTilesM][kTilesN
         float total = sums[0][t][j][e % 256];
 #pragma unroll
         for (int v = 1; v < kWaves; ++v) total += sums[v][t][j][e % 256];     // (segments past K's end are zeros)
-        c[static_cast<long>(row) * n + col] = total;
+        c[static_cast<long>(row) * n + col] = kAdds ? before + total : total;
     }
 }
 
@@ -353,11 +367,18 @@ gemm_f32_stream_kernel(const float* __restrict__ a, const float* __restrict__ b,
 constexpr int kFewRows = 8;
 constexpr long kManyTiles = 1024;
 
-template <int kWaves, int kAhead, int kEach, bool kVec>
-__global__ void __launch_bounds__(kWaves * kWave, kEach)
-gemm_f32_few_kernel(const float* __restrict__ a, const float* __restrict__ b, float* __restrict__ c, int m, int n, int k, int segment,
-                    Epilogue then) {
+// kFold, what else the launch does: 0 nothing; kFoldAdds: the product is added to what lies in C; from 2 on: A's rows are normed first, every
+// element (a * gain) / sqrt(mean(a^2) + eps), rows of up to 256 kFold elements.  A workgroup needs the sums of squares of all rows: a wave
+// asks for a whole row ahead of its first weights and adds up while those are on their way, in the order of the norm's own kernel
+// (add_rmsnorm_vec_kernel), so that results are the same bits as of two launches.
+constexpr int kFoldAdds = 1;
+
+template <int kWaves, int kAhead, bool kVec, int kFold>
+__device__ inline void few_rows(const float* __restrict__ a, const float* __restrict__ b, float* __restrict__ c, int m, int n, int k, int segment,
+                                const Epilogue& then, const float* __restrict__ gain, float eps) {
     constexpr int kPair = 2 * kStreamRun;
+    constexpr bool kNorm = kFold >= 2;
+    static_assert(kVec || kFold == 0, "what is folded goes with aligned rows");
     __shared__ float sums[kWaves][1][1][kStreamTile * kStreamTile];
     const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
     const int n0 = blockIdx.x * kStreamTile;
@@ -367,10 +388,59 @@ gemm_f32_few_kernel(const float* __restrict__ a, const float* __restrict__ b, fl
     f32x4 sum = {0.f, 0.f, 0.f, 0.f};                  // (of the lower half of the wave)
     float largest_a = 0.f, largest_b = 0.f;
     f32x4 w[kAhead][2][kStreamLoads], x[kAhead][kStreamLoads];
+    [[maybe_unused]] f32x4 gains[kNorm ? kAhead : 1][kStreamLoads];
+    [[maybe_unused]] float inv = 1.0f, before = 0.f;
+    // the whole rows of this wave: the norm's threads 64 v + lane take four elements of every 4 kThreads
+    constexpr int kThreads = kFold == 2 ? 64 : 256, kTurns = kThreads / 64, kChunks = kNorm ? kFold / kTurns : 1, kRowsEach = kFewRows / kWaves;
+    [[maybe_unused]] __shared__ float inverses[kFewRows];
+    [[maybe_unused]] f32x4 whole[kNorm ? kRowsEach : 1][kNorm ? kFold : 1];
+    const auto place = [&](int q) { return 4 * ((q / kChunks) * 64 + lane + (q % kChunks) * kThreads); };
+    if constexpr (kNorm) {
+#pragma unroll
+        for (int e = 0; e < kRowsEach; ++e) {
+            const int row = wave + e * kWaves;
+            const float* from = a + static_cast<long>(row < m ? row : m - 1) * k;
+#pragma unroll
+            for (int q = 0; q < kFold; ++q) whole[e][q] = *reinterpret_cast<const f32x4*>(from + (place(q) < k ? place(q) : 0));
+        }
+    }
+    if constexpr (kFold == kFoldAdds) {                // the one element that this thread writes (see add_segments)
+        const int row = threadIdx.x / 16, col = n0 + threadIdx.x % 16;
+        before = c[static_cast<long>(row < m ? row : m - 1) * n + (col < n ? col : n - 1)];
+    }
+    const auto settle = [&] {                          // the rows' factors, once the first weights are on their way
+        if constexpr (kNorm) {
+#pragma unroll
+            for (int e = 0; e < kRowsEach; ++e) {
+                float total = 0.f;
+#pragma unroll
+                for (int v = 0; v < kTurns; ++v) {
+                    float ss = 0.f;
+#pragma unroll
+                    for (int i = 0; i < kChunks; ++i) {
+                        const int q = v * kChunks + i;
+                        float with = ss;
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) with = fmaf(whole[e][q][j], whole[e][q][j], with);
+                        ss = place(q) < k ? with : ss;
+                    }
+                    total += wave_sum(ss);
+                }
+                if (lane == 0) inverses[wave + e * kWaves] = 1.0f / sqrtf(total / static_cast<float>(k) + eps);
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");        // (__syncthreads waits for the weights)
+            __builtin_amdgcn_s_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+            inv = inverses[r % kFewRows < m ? r % kFewRows : m - 1];
+        }
+    };
     const int first = wave * segment, end = first + segment < k ? first + segment : k;
     const auto fetch_a = [&](int at, int into) {       // a pair of runs that lies whole before the segment's end
 #pragma unroll
-        for (int i = 0; i < kStreamLoads; ++i) x[into][i] = load_whole<kVec>(arow + at + later + i * 16 + h);
+        for (int i = 0; i < kStreamLoads; ++i) {
+            x[into][i] = load_whole<kVec>(arow + at + later + i * 16 + h);
+            if constexpr (kNorm) gains[into][i] = load_whole<kVec>(gain + at + later + i * 16 + h);
+        }
     };
     const auto fetch_b = [&](int at, int into, int run) {
 #pragma unroll
@@ -378,8 +448,10 @@ gemm_f32_few_kernel(const float* __restrict__ a, const float* __restrict__ b, fl
     };
     // the pair in the registers `of`; another one from `next` on is asked for as they become free
     const auto multiply = [&](int of, bool more, int next) {
-        const Operand xp = operand_of(x[of][0], x[of][1]);
-        largest_a = largest_of(largest_of(largest_a, x[of][0]), x[of][1]);
+        f32x4 x0 = x[of][0], x1 = x[of][1];
+        if constexpr (kNorm) x0 = normed(x0, gains[of][0], inv), x1 = normed(x1, gains[of][1], inv);
+        const Operand xp = operand_of(x0, x1);
+        largest_a = largest_of(largest_of(largest_a, x0), x1);
         if (more) fetch_a(next, of);
         f32x4 acc[2];
 #pragma unroll
@@ -402,6 +474,7 @@ gemm_f32_few_kernel(const float* __restrict__ a, const float* __restrict__ b, fl
     if (left >= kAhead) {
 #pragma unroll
         for (int d = 0; d < kAhead; ++d) fetch_a(at + d * kPair, d), fetch_b(at + d * kPair, d, 0), fetch_b(at + d * kPair, d, 1);
+        settle();
         for (; left >= 2 * kAhead; left -= kAhead, at += kAhead * kPair)
 #pragma unroll
             for (int d = 0; d < kAhead; ++d) multiply(d, true, at + (kAhead + d) * kPair);
@@ -412,6 +485,7 @@ gemm_f32_few_kernel(const float* __restrict__ a, const float* __restrict__ b, fl
 #pragma unroll
         for (int d = 0; d < kAhead - 1; ++d)
             if (d < left) fetch_a(at + d * kPair, d), fetch_b(at + d * kPair, d, 0), fetch_b(at + d * kPair, d, 1);
+        settle();
     }
 #pragma unroll
     for (int d = 0; d < kAhead - 1; ++d)
@@ -421,6 +495,7 @@ gemm_f32_few_kernel(const float* __restrict__ a, const float* __restrict__ b, fl
 #pragma unroll
         for (int i = 0; i < kStreamLoads; ++i) {
             x[0][i] = load_four<kVec>(arow, at + later + i * 16 + h, end);
+            if constexpr (kNorm) gains[0][i] = load_four<kVec>(gain, at + later + i * 16 + h, end);
 #pragma unroll
             for (int run = 0; run < 2; ++run) w[0][run][i] = load_four<kVec>(brow, at + run * kStreamRun + i * 16 + h, end);
         }
@@ -438,7 +513,7 @@ gemm_f32_few_kernel(const float* __restrict__ a, const float* __restrict__ b, fl
         for (int i = 0; i < 4; ++i) least[i] = __shfl(least_a, h + i, kWave);
         const auto doubt = [&](int i) { return mine && in_doubt(sum[i], least[i], least_b); };
         if (__any(doubt(0) || doubt(1) || doubt(2) || doubt(3))) {
-            const f32x4 plain = plain_square<kVec>(arow, brow, first, end, lane / 16);
+            const f32x4 plain = plain_square<kVec, kNorm>(arow, brow, first, end, lane / 16, gain, inv);
 #pragma unroll
             for (int i = 0; i < 4; ++i) sum[i] = doubt(i) ? plain[i] : sum[i];
         }
@@ -448,7 +523,22 @@ gemm_f32_few_kernel(const float* __restrict__ a, const float* __restrict__ b, fl
         for (int i = 0; i < 4; ++i) sums[wave][0][0][(h + i) * kStreamTile + r] = sum[i];
     }
     __syncthreads();
-    add_segments<1, 1, kWaves>(sums, c, m, n, n0, then);
+    add_segments<1, 1, kWaves, kFold == kFoldAdds>(sums, c, m, n, n0, then, before);
+}
+
+template <int kWaves, int kAhead, int kEach, bool kVec>
+__global__ void __launch_bounds__(kWaves * kWave, kEach)
+gemm_f32_few_kernel(const float* __restrict__ a, const float* __restrict__ b, float* __restrict__ c, int m, int n, int k, int segment,
+                    Epilogue then) {
+    few_rows<kWaves, kAhead, kVec, 0>(a, b, c, m, n, k, segment, then, nullptr, 0.f);
+}
+
+// The same with a neighbour folded in.
+template <int kWaves, int kAhead, int kEach, int kFold>
+__global__ void __launch_bounds__(kWaves * kWave, kEach)
+gemm_f32_folded_kernel(const float* __restrict__ a, const float* __restrict__ b, float* __restrict__ c, int m, int n, int k, int segment,
+                       Epilogue then, const float* __restrict__ gain, float eps) {
+    few_rows<kWaves, kAhead, true, kFold>(a, b, c, m, n, k, segment, then, gain, eps);
 }
 
 // ---- many rows -----------------------------------------------------------------------------------------------------
@@ -902,6 +992,34 @@ F32Plan f32_plan(int m, int n, int k) {
     return best;
 }
 
+// Up to eight rows one pair of runs on its way a wave; of a large matrix two, for two waves a SIMD (us, one and two pairs: one row
+// against 12288 x 2048 19.6 and 18.8, five against 24576 x 4096 72.5 and 69.7, 32768 x 2048 49.5 and 47.7; but 4096 x 2048 7.6 and 7.8,
+// 32768 x 1024 26.8 and 27.4).  Beyond, two runs; where there are many tiles and more than eight rows or short segments, two tiles
+// of B share what A's parts cost (one and two tiles: 16 rows against 32768 x 2048 64.6 and 53.5, 24576 x 4096 96.3 and 76.8, one row against
+// 32768 x 512 16.6 and 14.6; but 16 against 12288 x 2048 26.6 and 27.0, 4096 x 2048 9.8 and 13.6).
+bool large_matrix(const F32Segments& segments, int n, int k) { return segments.length >= 256 && static_cast<long>(n) * k >= 16l << 20; }
+bool many_tiles(const F32Segments& segments, int m, int n) { return n >= kManyTiles * kStreamTile && (m > kFewRows || segments.length <= 64); }
+
+// Products of at most eight rows with a neighbour folded in: which ones, and their launch.
+constexpr int kFoldedK = 4096;         // longest row that a product norms
+bool folds(int m, int n, int k, bool norm) {
+    return m > 0 && m <= kFewRows && n > 0 && k >= kStreamK && k % 4 == 0 && (!norm || k <= kFoldedK) && !many_tiles(f32_segments(k), m, n);
+}
+int launch_folded(const float* a, const float* b, float* c, int m, int n, int k, const Epilogue& then, const float* gain, float eps, hipStream_t stream) {
+    const F32Segments segments = f32_segments(k);
+    const bool large = large_matrix(segments, n, k);
+    const int fold = !gain ? kFoldAdds : k <= 512 ? 2 : k <= 2048 ? 8 : 16;
+#define LEONE_FOLDED(W, D, E, F)                                                                                                       \
+    gemm_f32_folded_kernel<W, D, E, F><<<ceil_div(n, kStreamTile), W * kWave, 0, stream>>>(a, b, c, m, n, k, segments.length, then, gain, eps)
+    if (segments.count <= 4) fold == kFoldAdds ? LEONE_FOLDED(4, 1, 4, kFoldAdds) : LEONE_FOLDED(4, 1, 4, 2);
+    else if (large) fold == kFoldAdds ? LEONE_FOLDED(8, 2, 2, kFoldAdds) : fold == 8 ? LEONE_FOLDED(8, 2, 2, 8) : LEONE_FOLDED(8, 2, 2, 16);
+    else if (fold <= 2) fold == kFoldAdds ? LEONE_FOLDED(8, 1, 4, kFoldAdds) : LEONE_FOLDED(8, 1, 4, 2);
+    else fold == 8 ? LEONE_FOLDED(8, 1, 4, 8) : LEONE_FOLDED(8, 1, 4, 16);
+#undef LEONE_FOLDED
+    LEONE_LAUNCH_CHECK("gemm_f32_folded");
+    return 0;
+}
+
 int launch_f32(const F32Plan& p, const float* a, const float* b, float* c, float* planes, int m, int n, int k, const Epilogue& then,
                hipStream_t stream) {
     const F32Segments segments = f32_segments(k);
@@ -915,13 +1033,7 @@ int launch_f32(const F32Plan& p, const float* a, const float* b, float* c, float
 #define LEONE_STREAM(T, N, W, D, E)                                                                                                    \
     (vec ? gemm_f32_stream_kernel<T, N, W, D, E, true><<<ceil_div(n, N * kStreamTile), W * kWave, 0, stream>>>(a, b, c, m, n, k, segments.length, then)  \
          : gemm_f32_stream_kernel<T, N, W, D, E, false><<<ceil_div(n, N * kStreamTile), W * kWave, 0, stream>>>(a, b, c, m, n, k, segments.length, then))
-        // Up to eight rows one pair of runs on its way a wave; of a large matrix two, for two waves a SIMD (us, one and two pairs: one row
-        // against 12288 x 2048 19.6 and 18.8, five against 24576 x 4096 72.5 and 69.7, 32768 x 2048 49.5 and 47.7; but 4096 x 2048 7.6 and 7.8,
-        // 32768 x 1024 26.8 and 27.4).  Beyond, two runs; where there are many tiles and more than eight rows or short segments, two tiles
-        // of B share what A's parts cost (one and two tiles: 16 rows against 32768 x 2048 64.6 and 53.5, 24576 x 4096 96.3 and 76.8, one row against
-        // 32768 x 512 16.6 and 14.6; but 16 against 12288 x 2048 26.6 and 27.0, 4096 x 2048 9.8 and 13.6).
-        const bool large = segments.length >= 256 && static_cast<long>(n) * k >= 16l << 20;
-        const bool many = n >= kManyTiles * kStreamTile && (m > kFewRows || segments.length <= 64);
+        const bool large = large_matrix(segments, n, k), many = many_tiles(segments, m, n);
         if (segments.count <= 4) {
             if (m <= kFewRows) LEONE_FEW(4, 1, 4);
             else if (m <= kStreamTile) LEONE_STREAM(1, 1, 4, 2, 4);
@@ -1009,4 +1121,22 @@ extern "C" int leone_gemm_f32_glu(const float* a, const float* b, float* c, floa
     LEONE_REQUIRE(act == kGateSilu || act == kGateGeluTanh || (act == kGateClampedSwish && limit > 0.f),
                   "gemm_f32_glu: unknown activation %d (limit %g)", act, limit);
     return launch_f32(f32_plan(m, n, k), a, b, c, planes, m, n, k, Epilogue{1, act, limit}, stream);
+}
+
+// What else a product of few rows can do in its launch, to the bit what the launches give one by one: 1: C += A . B^T; 2: A's rows are
+// normed first, (a * gain) / sqrt(mean(a^2) + eps) with float gains, and the product may be gated as leone_gemm_f32_glu's is (n whole tiles).
+extern "C" int leone_gemm_f32_folds(int m, int n, int k, int kind) { return (kind == 1 || kind == 2) && folds(m, n, k, kind == 2); }
+
+// gain: null for kind 1; act -1: the product is not gated.
+extern "C" int leone_gemm_f32_folded(const float* a, const float* b, float* c, int m, int n, int k, const float* gain, float eps, int act,
+                                     float limit, hipStream_t stream) {
+    LEONE_REQUIRE(a && b && c, "gemm_f32_folded: null pointer");
+    LEONE_REQUIRE(folds(m, n, k, gain != nullptr), "gemm_f32_folded: sizes %d x %d x %d", m, n, k);
+    for (const void* at : {static_cast<const void*>(a), static_cast<const void*>(b), static_cast<const void*>(gain)})
+        LEONE_REQUIRE(reinterpret_cast<uintptr_t>(at) % 16 == 0, "gemm_f32_folded: operands must be aligned to 16 bytes");
+    LEONE_REQUIRE(!gain || (eps > 0.f && eps == eps), "gemm_f32_folded: eps must be positive");
+    LEONE_REQUIRE(act < 0 || (gain && n % 16 == 0), "gemm_f32_folded: a gated product goes with a norm and %d columns", n);
+    LEONE_REQUIRE(act < 0 || act == kGateSilu || act == kGateGeluTanh || (act == kGateClampedSwish && limit > 0.f),
+                  "gemm_f32_folded: unknown activation %d (limit %g)", act, limit);
+    return launch_folded(a, b, c, m, n, k, act < 0 ? Epilogue{} : Epilogue{1, act, limit}, gain, eps, stream);
 }

@@ -101,6 +101,10 @@ int leone_gemm_f32(const float* a, const float* b, float* c, float* planes, int 
 int leone_gemm_f32_glu_fits(int n, int k);              // whether leone_gemm_f32_glu takes [n, k]
 int leone_gemm_f32_glu(const float* a, const float* b, float* c, float* planes, int m, int n, int k, int act, float limit,
                        hipStream_t stream);
+// Up to eight rows with a neighbour in the launch: C += A . B^T (kind 1, no gain), or A normed first (kind 2; act -1: not gated).
+int leone_gemm_f32_folds(int m, int n, int k, int kind);
+int leone_gemm_f32_folded(const float* a, const float* b, float* c, int m, int n, int k, const float* gain, float eps, int act,
+                          float limit, hipStream_t stream);
 
 // Tiled weights.  The two weight-streaming products below read W either row by row ([N,K]) or, with w_tiled, from
 // a copy laid out in the order in which their waves ask for it, for K a multiple of 64: rows in tiles of 16

@@ -728,6 +728,51 @@ def gemm_f32_glu(a: torch.Tensor, b: torch.Tensor, activation: str = "silu", lim
     return out
 
 
+FOLDED_F32_ROWS = 8          # most rows of a float32 product that carries out its neighbours
+# Every workgroup (16 weight rows) norms all rows for itself, which a launch of its own outweighs while there are few (us, norm and product
+# in two launches : in one, 1 row and 8: 768 x 512 5.9 : 3.9 and 6.3 : 4.2, 12288 x 512 10.0 : 8.2 and 10.5 : 8.8, 3072 x 2048 9.8 : 8.2 and 11.2 :
+# 9.2, 12288 x 1024 14.8 : 14.1 and 16.3 : 16.0, 6144 x 2048 16.5 : 14.3 and 19.0 : 16.8; but 8192 x 2048 17.2 : 17.2 and 18.7 : 19.8, 12288 x
+# 2048 22.7 : 24.5 and 24.5 : 28.8).
+FOLDED_F32_NORM_ELEMENTS = 12 << 20
+
+
+def _folds_f32(x, weight: torch.Tensor, residual: Optional[torch.Tensor], gated: bool) -> bool:
+    """Whether the float32 product of few rows does its neighbour in its own launch (``gemm_f32_folded``): the norm of ``x``
+    (``NormedRows`` of the whole stream under float gains), or the sum into ``residual``.  Everything else stays as it is."""
+    rows, k = x.shape
+    normed = isinstance(x, NormedRows)
+    if rows > FOLDED_F32_ROWS or not weight.is_cuda or not weight.is_contiguous() or weight.data_ptr() % 16 \
+            or (residual is not None and (normed or gated)):
+        return False
+    n = weight.shape[0]
+    if normed:
+        return (n * k <= FOLDED_F32_NORM_ELEMENTS and x.rows is None and x.gain.dtype == torch.float32 and x.x.dtype == torch.float32
+                and x.x.is_contiguous() and x.gain.is_contiguous() and x.x.data_ptr() % 16 == 0 and x.gain.data_ptr() % 16 == 0
+                and (not gated or n % 16 == 0) and bool(library().leone_gemm_f32_folds(rows, n, k, 2)))
+    return (residual is not None and residual.dtype == torch.float32 and tuple(residual.shape) == (rows, n) and residual.is_contiguous()
+            and x.is_contiguous() and x.data_ptr() % 16 == 0 and bool(library().leone_gemm_f32_folds(rows, n, k, 1)))
+
+
+def gemm_f32_folded(x, weight: torch.Tensor, residual: Optional[torch.Tensor] = None, gated: bool = False, activation: str = "silu",
+                    limit: Optional[float] = None) -> Optional[torch.Tensor]:
+    """The float32 product of at most FOLDED_F32_ROWS rows with its neighbour in the launch, to the bit what the launches give one by
+    one: ``x`` ``NormedRows`` (``gated``: act(gate) * up comes out), or the product added into ``residual`` (None returned)."""
+    rows, k = x.shape
+    n, k2 = weight.shape
+    if k != k2:
+        raise KernelError(f"gemm_f32_folded: inner sizes {k} and {k2} differ")
+    normed = isinstance(x, NormedRows)
+    if normed == (residual is not None) or (gated and not normed):
+        raise KernelError("gemm_f32_folded: either a norm goes ahead of the product or it is added into the stream")
+    out = residual if residual is not None else torch.empty((rows, n // 2 if gated else n), dtype=torch.float32, device=weight.device)
+    with profile.span("gemm f32", weight):
+        call("leone_gemm_f32_folded", _dev(x.x if normed else x, "gemm a", torch.float32, (rows, k)), _dev(weight, "gemm b", torch.float32),
+             _dev(out, "gemm out", torch.float32, (rows, n // 2 if gated else n)), rows, n, k,
+             _dev(x.gain, "gain", torch.float32, (k,)) if normed else 0, x.eps if normed else 0.0,
+             _glu_code(activation, limit) if gated else -1, float(limit or 0.0), _stream())
+    return None if residual is not None else out
+
+
 # Up to here norm, gate and residual are folded into the weight-streaming kernel for few rows; beyond, the
 # multi-row kernel runs with the row-wise kernels between.  Measured in whole decode steps at the 8B layer sizes
 # with the second copies of the weights (ms a step, folded : multi-row): 5.98 : 6.40 at 11 rows, 6.17 : 6.47 at
@@ -1169,6 +1214,12 @@ def linear(x, weight: torch.Tensor, out_dtype: Optional[torch.dtype] = None,
                                       or next_norm[2] != torch.bfloat16):
             next_norm = None
         return gemm_fused(x, weight, out_dtype, residual, gated, next_norm, activation=activation, limit=limit)
+    if dtype == torch.float32 and out_dtype == torch.float32:
+        if isinstance(x, NormedRows) and _folds_f32(x, weight, None, gated):
+            return gemm_f32_folded(x, weight, None, gated, activation, limit)
+        x = materialize(x)
+        if residual is not None and _folds_f32(x, weight, residual, gated):
+            return gemm_f32_folded(x, weight, residual)
     x = materialize(x)
     if dtype == torch.bfloat16 and weight.is_cuda and k % 8 == 0 and rows <= ROWS_MAX \
             and (not gated or weight.shape[0] % 16 == 0):

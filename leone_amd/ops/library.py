@@ -40,6 +40,7 @@ _PROTOTYPES = {
                                 c_int, P],
     "leone_gemm_f32": [P, P, P, P, c_int, c_int, c_int, P],
     "leone_gemm_f32_glu": [P, P, P, P, c_int, c_int, c_int, c_int, c_float, P],
+    "leone_gemm_f32_folded": [P, P, P, c_int, c_int, c_int, P, c_float, c_int, c_float, P],
     "leone_gemm_fused_bf16": [P, c_int, P, P, c_int, c_float, P, c_int, P, c_int, c_int, c_int, c_int, c_int, P, P, P, P,
                               c_int, c_float, P],
     "leone_gemm_planes_bf16": [P, c_int, c_int, P, c_int, P, c_int, c_int, c_int, c_int, P],
@@ -180,6 +181,8 @@ def library() -> ctypes.CDLL:
             lib.leone_state_slots_max.argtypes = []
             lib.leone_gemm_f32_planes.restype = c_int
             lib.leone_gemm_f32_planes.argtypes = [c_int, c_int, c_int]
+            lib.leone_gemm_f32_folds.restype = c_int
+            lib.leone_gemm_f32_folds.argtypes = [c_int, c_int, c_int, c_int]
             lib.leone_gemm_f32_glu_fits.restype = c_int
             lib.leone_gemm_f32_glu_fits.argtypes = [c_int, c_int]
             lib.leone_sample_truncated_stages.restype = c_int
