@@ -202,7 +202,8 @@ constexpr int kChain = 32;                             // elements of K whose pr
 
 // The waves' sums of the workgroup's tiles, added and stored.
 // kAdds (one tile): what lay in c before, of the thread's one element, is added.
-template <int kTilesM, int kTilesN, int kWaves, bool kAdds = false>
+// kCols: of the tile's 16 columns the first so many count.
+template <int kTilesM, int kTilesN, int kWaves, bool kAdds = false, int kCols = kStreamTile>
 __device__ inline void add_segments(const float (&sums)[kWaves][kTilesM][kTilesN][kStreamTile * kStreamTile], float* __restrict__ c, int m, int n,
                                     int n0, const Epilogue& then, float before = 0.f) {
     static_assert(!kAdds || (kTilesM == 1 && kTilesN == 1 && kWaves * kWave >= 256), "an element a thread");
@@ -219,7 +220,7 @@ __device__ inline void add_segments(const float (&sums)[kWaves][kTilesM][kTilesN
     }
     for (int e = threadIdx.x; e < kTilesM * kTilesN * 256; e += kWaves * kWave) {
         const int t = e / (kTilesN * 256), j = e / 256 % kTilesN, row = t * 16 + e % 256 / 16, col = n0 + j * kStreamTile + e % 16;
-        if (row >= m || col >= n) continue;
+        if (row >= m || col >= n || (kCols < kStreamTile && e % 16 >= kCols)) continue;
         float total = sums[0][t][j][e % 256];
 #pragma unroll
         for (int v = 1; v < kWaves; ++v) total += sums[v][t][j][e % 256];     // (segments past K's end are zeros)
@@ -373,7 +374,9 @@ constexpr long kManyTiles = 1024;
 // (add_rmsnorm_vec_kernel), so that results are the same bits as of two launches.
 constexpr int kFoldAdds = 1;
 
-template <int kWaves, int kAhead, bool kVec, int kFold>
+// kNarrow: the workgroup owns eight rows of B, not 16, and the instruction's 16 columns too are taken for two runs: twice as many
+// workgroups where 16 rows each would leave units idle.  Of the products the first run's lie in rows and columns 0 .. 7, the second's in 8 .. 15.
+template <int kWaves, int kAhead, bool kVec, int kFold, bool kNarrow = false>
 __device__ inline void few_rows(const float* __restrict__ a, const float* __restrict__ b, float* __restrict__ c, int m, int n, int k, int segment,
                                 const Epilogue& then, const float* __restrict__ gain, float eps) {
     constexpr int kPair = 2 * kStreamRun;
@@ -381,13 +384,14 @@ __device__ inline void few_rows(const float* __restrict__ a, const float* __rest
     static_assert(kVec || kFold == 0, "what is folded goes with aligned rows");
     __shared__ float sums[kWaves][1][1][kStreamTile * kStreamTile];
     const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-    const int n0 = blockIdx.x * kStreamTile;
+    constexpr int kCols = kNarrow ? kStreamTile / 2 : kStreamTile, kRuns = kNarrow ? 1 : 2;
+    const int n0 = blockIdx.x * kCols;
     const int r = lane % 16, h = (lane / 16) * 4, later = r < kFewRows ? 0 : kStreamRun;
-    const float* brow = b + static_cast<long>(n0 + r < n ? n0 + r : n - 1) * k;
+    const float* brow = b + static_cast<long>(n0 + r % kCols < n ? n0 + r % kCols : n - 1) * k + (kNarrow ? later : 0);
     const float* arow = a + static_cast<long>(r % kFewRows < m ? r % kFewRows : m - 1) * k;
     f32x4 sum = {0.f, 0.f, 0.f, 0.f};                  // (of the lower half of the wave)
     float largest_a = 0.f, largest_b = 0.f;
-    f32x4 w[kAhead][2][kStreamLoads], x[kAhead][kStreamLoads];
+    f32x4 w[kAhead][kRuns][kStreamLoads], x[kAhead][kStreamLoads];
     [[maybe_unused]] f32x4 gains[kNorm ? kAhead : 1][kStreamLoads];
     [[maybe_unused]] float inv = 1.0f, before = 0.f;
     // the whole rows of this wave: the norm's threads 64 v + lane take four elements of every 4 kThreads
@@ -405,7 +409,7 @@ __device__ inline void few_rows(const float* __restrict__ a, const float* __rest
         }
     }
     if constexpr (kFold == kFoldAdds) {                // the one element that this thread writes (see add_segments)
-        const int row = threadIdx.x / 16, col = n0 + threadIdx.x % 16;
+        const int row = threadIdx.x / 16, col = n0 + threadIdx.x % kCols;
         before = c[static_cast<long>(row < m ? row : m - 1) * n + (col < n ? col : n - 1)];
     }
     const auto settle = [&] {                          // the rows' factors, once the first weights are on their way
@@ -446,6 +450,17 @@ __device__ inline void few_rows(const float* __restrict__ a, const float* __rest
 #pragma unroll
         for (int i = 0; i < kStreamLoads; ++i) w[into][run][i] = load_whole<kVec>(brow + at + run * kStreamRun + i * 16 + h);
     };
+    const auto fetch_pair = [&](int at, int into) {
+#pragma unroll
+        for (int run = 0; run < kRuns; ++run) fetch_b(at, into, run);
+    };
+    [[maybe_unused]] const unsigned sign = kNarrow && later ? 0x80000000u : 0u;
+    [[maybe_unused]] const auto turned = [&](const f32x4& v) {
+        f32x4 t;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) t[e] = __uint_as_float(__float_as_uint(v[e]) ^ sign);
+        return t;
+    };
     // the pair in the registers `of`; another one from `next` on is asked for as they become free
     const auto multiply = [&](int of, bool more, int next) {
         f32x4 x0 = x[of][0], x1 = x[of][1];
@@ -453,11 +468,11 @@ __device__ inline void few_rows(const float* __restrict__ a, const float* __rest
         const Operand xp = operand_of(x0, x1);
         largest_a = largest_of(largest_of(largest_a, x0), x1);
         if (more) fetch_a(next, of);
-        f32x4 acc[2];
+        f32x4 acc[kRuns];
 #pragma unroll
-        for (int run = 0; run < 2; ++run) {
+        for (int run = 0; run < kRuns; ++run) {
             const f32x4 w0 = w[of][run][0], w1 = w[of][run][1];
-            const Operand wp = run ? operand_of(-w0, -w1) : operand_of(w0, w1);
+            const Operand wp = kNarrow ? operand_of(turned(w0), turned(w1)) : run ? operand_of(-w0, -w1) : operand_of(w0, w1);
             largest_b = largest_of(largest_of(largest_b, w0), w1);
             if (more) fetch_b(next, of, run);
             acc[run] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -467,13 +482,16 @@ __device__ inline void few_rows(const float* __restrict__ a, const float* __rest
             if (run == 0) sum += acc[0];
         }
 #pragma unroll
-        for (int e = 0; e < 4; ++e)                    // (the upper half's results to the lower one)
-            sum[e] -= __uint_as_float(__builtin_amdgcn_permlane32_swap(__float_as_uint(acc[1][e]), __float_as_uint(acc[0][e]), false, false)[1]);
+        for (int e = 0; e < 4; ++e) {                  // (the upper half's results to the lower one, of columns 8 .. 15 to 0 .. 7)
+            const unsigned first = __float_as_uint(acc[0][e]), second = __float_as_uint(acc[kRuns - 1][e]);
+            const unsigned upper = __builtin_amdgcn_permlane32_swap(second, first, false, false)[1];
+            sum[e] -= __uint_as_float(kNarrow ? of_lane<0x128>(upper) : upper);
+        }
     };
     int left = end > first ? (end - first) / kPair : 0, at = first;
     if (left >= kAhead) {
 #pragma unroll
-        for (int d = 0; d < kAhead; ++d) fetch_a(at + d * kPair, d), fetch_b(at + d * kPair, d, 0), fetch_b(at + d * kPair, d, 1);
+        for (int d = 0; d < kAhead; ++d) fetch_a(at + d * kPair, d), fetch_pair(at + d * kPair, d);
         settle();
         for (; left >= 2 * kAhead; left -= kAhead, at += kAhead * kPair)
 #pragma unroll
@@ -484,7 +502,7 @@ __device__ inline void few_rows(const float* __restrict__ a, const float* __rest
     } else {
 #pragma unroll
         for (int d = 0; d < kAhead - 1; ++d)
-            if (d < left) fetch_a(at + d * kPair, d), fetch_b(at + d * kPair, d, 0), fetch_b(at + d * kPair, d, 1);
+            if (d < left) fetch_a(at + d * kPair, d), fetch_pair(at + d * kPair, d);
         settle();
     }
 #pragma unroll
@@ -497,23 +515,25 @@ __device__ inline void few_rows(const float* __restrict__ a, const float* __rest
             x[0][i] = load_four<kVec>(arow, at + later + i * 16 + h, end);
             if constexpr (kNorm) gains[0][i] = load_four<kVec>(gain, at + later + i * 16 + h, end);
 #pragma unroll
-            for (int run = 0; run < 2; ++run) w[0][run][i] = load_four<kVec>(brow, at + run * kStreamRun + i * 16 + h, end);
+            for (int run = 0; run < kRuns; ++run) w[0][run][i] = load_four<kVec>(brow, at + run * kStreamRun + i * 16 + h, end - (kNarrow ? later : 0));
         }
         multiply(0, false, 0);
     }
-    const bool mine = lane < kWave / 2;
+    const bool mine = lane < kWave / 2 && r < kCols;
     float least_sum = INFINITY, no_number = 0.f;
 #pragma unroll
     for (int i = 0; i < 4; ++i) least_sum = fminf(least_sum, fabsf(sum[i])), no_number = fmaf(sum[i], 0.f, no_number);
     if (!__all(beyond_doubt(fmaxf(largest_a, largest_b), mine ? least_sum : 1.0f, mine ? no_number : 0.f))) {
-        const float least_b = least_of(max_lanes<16>(max_lanes<32>(largest_b)));
+        float largest_of_b = max_lanes<16>(max_lanes<32>(largest_b));
+        if constexpr (kNarrow) largest_of_b = max_lanes<8>(largest_of_b);
+        const float least_b = least_of(largest_of_b);
         const float least_a = least_of(max_lanes<8>(max_lanes<16>(max_lanes<32>(largest_a))));
         float least[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) least[i] = __shfl(least_a, h + i, kWave);
         const auto doubt = [&](int i) { return mine && in_doubt(sum[i], least[i], least_b); };
         if (__any(doubt(0) || doubt(1) || doubt(2) || doubt(3))) {
-            const f32x4 plain = plain_square<kVec, kNorm>(arow, brow, first, end, lane / 16, gain, inv);
+            const f32x4 plain = plain_square<kVec, kNorm>(arow, brow - (kNarrow ? later : 0), first, end, lane / 16, gain, inv);
 #pragma unroll
             for (int i = 0; i < 4; ++i) sum[i] = doubt(i) ? plain[i] : sum[i];
         }
@@ -523,7 +543,7 @@ __device__ inline void few_rows(const float* __restrict__ a, const float* __rest
         for (int i = 0; i < 4; ++i) sums[wave][0][0][(h + i) * kStreamTile + r] = sum[i];
     }
     __syncthreads();
-    add_segments<1, 1, kWaves, kFold == kFoldAdds>(sums, c, m, n, n0, then, before);
+    add_segments<1, 1, kWaves, kFold == kFoldAdds, kCols>(sums, c, m, n, n0, then, before);
 }
 
 template <int kWaves, int kAhead, int kEach, bool kVec>
@@ -539,6 +559,14 @@ __global__ void __launch_bounds__(kWaves * kWave, kEach)
 gemm_f32_folded_kernel(const float* __restrict__ a, const float* __restrict__ b, float* __restrict__ c, int m, int n, int k, int segment,
                        Epilogue then, const float* __restrict__ gain, float eps) {
     few_rows<kWaves, kAhead, true, kFold>(a, b, c, m, n, k, segment, then, gain, eps);
+}
+
+// Eight rows of B a workgroup.
+template <int kWaves, int kAhead, int kEach, int kFold>
+__global__ void __launch_bounds__(kWaves * kWave, kEach)
+gemm_f32_narrow_kernel(const float* __restrict__ a, const float* __restrict__ b, float* __restrict__ c, int m, int n, int k, int segment,
+                       Epilogue then, const float* __restrict__ gain, float eps) {
+    few_rows<kWaves, kAhead, true, kFold, true>(a, b, c, m, n, k, segment, then, gain, eps);
 }
 
 // ---- many rows -----------------------------------------------------------------------------------------------------
@@ -1002,13 +1030,31 @@ bool many_tiles(const F32Segments& segments, int m, int n) { return n >= kManyTi
 
 // Products of at most eight rows with a neighbour folded in: which ones, and their launch.
 constexpr int kFoldedK = 4096;         // longest row that a product norms
+// Up to here a workgroup owns eight rows of B, not 16, so that every unit has at most one: a unit without one asks for nothing (us, 16 and
+// eight, 1 row and 8: 512 x 512 3.7 and 3.3, 4.0 and 3.6; 1024 x 3072 8.7 and 6.8, 10.7 and 8.4; 2048 x 2048 6.8 and 5.7, 8.1 and 6.7; 2048 x 6144
+// 16.1 and 12.4, 19.7 and 14.7; but 3072 x 2048 6.9 and 8.5, 8.1 and 10.2, 4096 x 4096 14.6 and 15.1, 15.1 and 18.3).
+constexpr int kNarrowColumns = 2048;
 bool folds(int m, int n, int k, bool norm) {
     return m > 0 && m <= kFewRows && n > 0 && k >= kStreamK && k % 4 == 0 && (!norm || k <= kFoldedK) && !many_tiles(f32_segments(k), m, n);
+}
+bool narrow(int n) { return n <= kNarrowColumns; }
+int launch_narrow(int fold, const float* a, const float* b, float* c, int m, int n, int k, const float* gain, float eps, hipStream_t stream) {
+    const F32Segments segments = f32_segments(k);
+#define LEONE_NARROW(W, D, E, F) \
+    gemm_f32_narrow_kernel<W, D, E, F><<<ceil_div(n, kStreamTile / 2), W * kWave, 0, stream>>>(a, b, c, m, n, k, segments.length, Epilogue{}, gain, eps)
+    if (segments.count <= 4) fold == 0 ? LEONE_NARROW(4, 1, 4, 0) : fold == kFoldAdds ? LEONE_NARROW(4, 1, 4, kFoldAdds) : LEONE_NARROW(4, 1, 4, 2);
+    else if (fold < 2) fold == 0 ? LEONE_NARROW(8, 2, 4, 0) : LEONE_NARROW(8, 2, 4, kFoldAdds);
+    else if (fold == 2) LEONE_NARROW(8, 1, 4, 2);
+    else fold == 8 ? LEONE_NARROW(8, 2, 4, 8) : LEONE_NARROW(8, 1, 4, 16);
+#undef LEONE_NARROW
+    LEONE_LAUNCH_CHECK("gemm_f32_narrow");
+    return 0;
 }
 int launch_folded(const float* a, const float* b, float* c, int m, int n, int k, const Epilogue& then, const float* gain, float eps, hipStream_t stream) {
     const F32Segments segments = f32_segments(k);
     const bool large = large_matrix(segments, n, k);
     const int fold = !gain ? kFoldAdds : k <= 512 ? 2 : k <= 2048 ? 8 : 16;
+    if (!then.gated && narrow(n)) return launch_narrow(fold, a, b, c, m, n, k, gain, eps, stream);
 #define LEONE_FOLDED(W, D, E, F)                                                                                                       \
     gemm_f32_folded_kernel<W, D, E, F><<<ceil_div(n, kStreamTile), W * kWave, 0, stream>>>(a, b, c, m, n, k, segments.length, then, gain, eps)
     if (segments.count <= 4) fold == kFoldAdds ? LEONE_FOLDED(4, 1, 4, kFoldAdds) : LEONE_FOLDED(4, 1, 4, 2);
@@ -1034,6 +1080,7 @@ int launch_f32(const F32Plan& p, const float* a, const float* b, float* c, float
     (vec ? gemm_f32_stream_kernel<T, N, W, D, E, true><<<ceil_div(n, N * kStreamTile), W * kWave, 0, stream>>>(a, b, c, m, n, k, segments.length, then)  \
          : gemm_f32_stream_kernel<T, N, W, D, E, false><<<ceil_div(n, N * kStreamTile), W * kWave, 0, stream>>>(a, b, c, m, n, k, segments.length, then))
         const bool large = large_matrix(segments, n, k), many = many_tiles(segments, m, n);
+        if (vec && m <= kFewRows && !then.gated && narrow(n)) return launch_narrow(0, a, b, c, m, n, k, nullptr, 0.f, stream);
         if (segments.count <= 4) {
             if (m <= kFewRows) LEONE_FEW(4, 1, 4);
             else if (m <= kStreamTile) LEONE_STREAM(1, 1, 4, 2, 4);

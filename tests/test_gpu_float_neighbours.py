@@ -16,7 +16,7 @@ def drawn(m, n, k, seed):
 
 # inner sizes at both ends of every variant (four waves up to 511; whole rows of 512, 2,048 and 4,096; large matrices), ends of K off a
 # pair of runs and off a segment; a last tile of a few columns, many workgroups
-SIZES = [(16, 256), (40, 260), (96, 508), (512, 512), (48, 516), (1536, 1024), (530, 2044), (12288, 2048), (96, 2052), (33, 4092), (4096, 4096)]
+SIZES = [(4, 256), (13, 644), (2048, 576), (2049, 512), (16, 256), (40, 260), (96, 508), (512, 512), (48, 516), (1536, 1024), (530, 2044), (12288, 2048), (96, 2052), (33, 4092), (4096, 4096)]
 
 
 @pytest.mark.parametrize("m", [1, 2, 5, 8])
@@ -70,3 +70,19 @@ def test_what_is_left_to_launches_of_their_own():
         assert not ops._folds_f32(ops.NormedRows(x, gain, 1e-5, torch.float32), w, None, False)
     with pytest.raises(ops.KernelError):
         ops.gemm_f32_folded(x, w)
+
+
+@pytest.mark.parametrize("n,k", [(1, 256), (7, 260), (9, 516), (40, 1000), (100, 2052), (2047, 640), (2048, 4100), (24, 6144)])
+def test_eight_columns_a_workgroup_give_the_bits_of_many_rows(n, k):
+    """Up to 2,048 columns and eight rows the instruction's columns are shared by two runs; ends of K off a pair of runs, columns off
+    eight, columns and rows that are made again on the float instructions."""
+    from leone_amd import ops
+    gen = torch.Generator(device=DEV).manual_seed(n + k)
+    a, b = torch.randn(64, k, generator=gen, device=DEV), torch.randn(n, k, generator=gen, device=DEV)
+    a[1, k - 1], a[4] = math.nan, 0.0
+    a[5] *= 1e-36
+    b[n // 2] *= 1e30
+    b[n - 1, k - 1] = math.inf
+    many = ops.gemm_f32(a, b).nan_to_num(7.5, 8.5, 9.5)
+    for m in (1, 3, 8):
+        assert torch.equal(ops.gemm_f32(a[:m].contiguous(), b).nan_to_num(7.5, 8.5, 9.5), many[:m]), m
