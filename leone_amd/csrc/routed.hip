@@ -519,15 +519,19 @@ __device__ inline moe_bf16x8 moe_zero8() {
 // leaves the caches to others (a decoding step of a model with 32 experts of 2,048 x 768: 6.96 ms, unmarked 7.09, its first products alone unmarked
 // 7.14); with longer rows some lines came twice (32 experts of 4,096 x 1,024, both products, 16 rows 172 us, the first one
 // unmarked 158; 8 of 1,024 x 4,096, eight rows 58, the second one unmarked 46 to 56).
+//
+// kTiled: the matrices come as a copy laid out as the waves ask for them (16 rows at a time, steps of 32 elements one after the other, a
+// step lane by lane), so that a load is one kilobyte in one piece; same numbers in the same places, same bits.
 constexpr int kStreamedInner = 2048;
 
-template <int kMode, bool kStreamed>
+enum MoeLayout : int { kMoeKept = 0, kMoeStreamed = 1, kMoeTiled = 2 };
+template <int kMode, int kLayout>
 __global__ void __launch_bounds__(kMoeThreads, 4)
 moe_product_stream_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, void* __restrict__ y,
                           const float* __restrict__ pair_weight, const int* __restrict__ tile_expert,
                           const int* __restrict__ tile_pairs, int top, int n, int k, int act, float limit) {
-    constexpr bool kGated = kMode == kMoeGated;
-    constexpr int kDepth = 8;
+    constexpr bool kGated = kMode == kMoeGated, kTiled = kLayout == kMoeTiled;
+    constexpr int kDepth = 8, kStep = kTiled ? 512 : 32;         // elements from a step of the matrix to the next
     __shared__ moe_floatx4 sums[kGated ? 2 : 1][kMoeWaves][kWave];
     const int tile = blockIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
@@ -540,14 +544,15 @@ moe_product_stream_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict
     const long matrix = static_cast<long>(n) * k;
     // Lanes past the last row take that one again, lanes without a pair the tile's first: their results are not written.  Nothing
     // stands between the loads: behind one that may not have been asked for the compiler cannot count those in flight and waits for all.
-    const bf16_t* wa = w + static_cast<long>(e) * (kGated ? 2 : 1) * matrix + static_cast<long>(row0 + c < n ? row0 + c : n - 1) * k;
+    const bf16_t* wa = w + static_cast<long>(e) * (kGated ? 2 : 1) * matrix +
+                       (kTiled ? static_cast<long>(row0) * k + 8 * lane : static_cast<long>(row0 + c < n ? row0 + c : n - 1) * k + 8 * g);
     const int pair = own < 0 ? first_pair : own;
     const bf16_t* xrow = x + static_cast<long>(kMode != kMoeDown ? pair / top : pair) * k;
     const int steps = (k + 31) / 32, share = (steps + kMoeWaves - 1) / kMoeWaves;
     const int first = wave * share, last = first + share < steps ? first + share : steps;
     moe_floatx4 acc = {0.f, 0.f, 0.f, 0.f}, acc2 = {0.f, 0.f, 0.f, 0.f};
     moe_bf16x8 a[kDepth], a2[kGated ? kDepth : 1], xb[kDepth];
-    const auto weights = [](const bf16_t* p) { return kStreamed ? __builtin_bit_cast(moe_bf16x8, load_streamed16(p)) : moe_load8(p); };
+    const auto weights = [](const bf16_t* p) { return kLayout != kMoeKept ? __builtin_bit_cast(moe_bf16x8, load_streamed16(p)) : moe_load8(p); };
     const auto ask = [&](int d, const bf16_t* of_w, const bf16_t* of_x) {
         a[d] = weights(of_w);
         if constexpr (kGated) a2[d] = weights(of_w + matrix);
@@ -558,26 +563,26 @@ moe_product_stream_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict
         if constexpr (kGated) acc2 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2[d], xb[d], acc2, 0, 0, 0);
     };
     const int whole = last * 32 <= k ? last : last - 1;          // steps without the inner size's end
-    const bf16_t *from_w = wa + 32 * first + 8 * g, *from_x = xrow + 32 * first + 8 * g;
+    const bf16_t *from_w = wa + static_cast<long>(kStep) * first, *from_x = xrow + 32 * first + 8 * g;
     int left = whole > first ? whole - first : 0;
     if (left >= kDepth) {
 #pragma unroll
-        for (int d = 0; d < kDepth; ++d) ask(d, from_w + 32 * d, from_x + 32 * d);
+        for (int d = 0; d < kDepth; ++d) ask(d, from_w + kStep * d, from_x + 32 * d);
         for (; left >= 2 * kDepth; left -= kDepth) {
-            from_w += 32 * kDepth, from_x += 32 * kDepth;
+            from_w += kStep * kDepth, from_x += 32 * kDepth;
 #pragma unroll
             for (int d = 0; d < kDepth; ++d) {
                 multiply(d);
-                ask(d, from_w + 32 * d, from_x + 32 * d);
+                ask(d, from_w + kStep * d, from_x + 32 * d);
             }
         }
 #pragma unroll
         for (int d = 0; d < kDepth; ++d) multiply(d);
-        from_w += 32 * kDepth, from_x += 32 * kDepth, left -= kDepth;
+        from_w += kStep * kDepth, from_x += 32 * kDepth, left -= kDepth;
     }
     const auto rest = [&](auto count) {
 #pragma unroll
-        for (int d = 0; d < decltype(count)::value; ++d) ask(d, from_w + 32 * d, from_x + 32 * d);
+        for (int d = 0; d < decltype(count)::value; ++d) ask(d, from_w + kStep * d, from_x + 32 * d);
 #pragma unroll
         for (int d = 0; d < decltype(count)::value; ++d) multiply(d);
     };
@@ -591,9 +596,9 @@ moe_product_stream_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict
         case 1: rest(std::integral_constant<int, 1>{}); break;
         default: break;
     }
-    if (first < last && whole < last) {                            // the step that holds the inner size's end; zeros beyond it
+    if (!kTiled && first < last && whole < last) {                 // the step that holds the inner size's end; zeros beyond it
         const int wanted = 32 * whole + 8 * g, at = wanted < k ? wanted : k - 8;
-        ask(0, wa + at, xrow + at);
+        ask(0, wa + at - 8 * g, xrow + at);
         if (wanted >= k) {
             a[0] = xb[0] = moe_zero8();
             if constexpr (kGated) a2[0] = moe_zero8();
@@ -1070,9 +1075,10 @@ extern "C" int leone_moe_plan(const int* chosen, int pairs, int experts, int* ti
 // experts: how many there are, for the rule that looks at how many workgroups their matrices give (see one_chunk_ahead).
 // tile: pairs a tile holds, as leone_moe_plan was told: leone_moe_tile_pairs() for the kernel that takes any type and
 // size; 16, 64 or 128 for the matrix-core kernels (bfloat16, n and k multiples of 8).
-extern "C" int leone_moe_product(const void* x, const void* w, void* y, const float* pair_weight, int dtype, int gated,
-                                 const int* tile_expert, const int* tile_pairs, int max_tiles, int tile, int experts, int top, int n,
-                                 int k, int act, float limit, hipStream_t stream) {
+static int run_moe_product(const void* x, const void* w, int w_tiled, void* y, const float* pair_weight, int dtype, int gated,
+                           const int* tile_expert, const int* tile_pairs, int max_tiles, int tile, int experts, int top, int n, int k,
+                           int act, float limit, hipStream_t stream) {
+    LEONE_REQUIRE(!w_tiled || (tile == 16 && n % 16 == 0 && k % 32 == 0), "moe_product: matrices in tiles go with 16 pairs and sizes %d x %d", n, k);
     LEONE_REQUIRE(gated >= kMoeDown && gated <= kMoePlain, "moe_product: unknown kind of product %d", gated);
     LEONE_REQUIRE(act == kGateSilu || act == kGateGeluTanh || (act == kGateClampedSwish && limit > 0.f && gated != kMoePlain) ||
                       (act == kActReluSquared && gated != kMoeGated),
@@ -1087,15 +1093,16 @@ extern "C" int leone_moe_product(const void* x, const void* w, void* y, const fl
             const dim3 grid(max_tiles, ceil_div(n, 16));
             LEONE_REQUIRE(grid.y <= 65535, "moe_product: %d rows of a matrix are too many", n);
             const bool streamed = k <= kStreamedInner;
+#define LEONE_MOE_LAID(MODE, LAYOUT)                                                                                           \
+    moe_product_stream_kernel<MODE, LAYOUT><<<grid, kMoeThreads, 0, stream>>>(                                                 \
+        static_cast<const bf16_t*>(x), static_cast<const bf16_t*>(w), y, pair_weight, tile_expert, tile_pairs, top, n, k, act, limit)
 #define LEONE_MOE_STREAM(MODE)                                                                                                 \
-    (streamed ? moe_product_stream_kernel<MODE, true><<<grid, kMoeThreads, 0, stream>>>(                                      \
-                    static_cast<const bf16_t*>(x), static_cast<const bf16_t*>(w), y, pair_weight, tile_expert, tile_pairs, top, n, k, act, limit) \
-              : moe_product_stream_kernel<MODE, false><<<grid, kMoeThreads, 0, stream>>>(                                     \
-                    static_cast<const bf16_t*>(x), static_cast<const bf16_t*>(w), y, pair_weight, tile_expert, tile_pairs, top, n, k, act, limit))
+    (w_tiled ? LEONE_MOE_LAID(MODE, kMoeTiled) : streamed ? LEONE_MOE_LAID(MODE, kMoeStreamed) : LEONE_MOE_LAID(MODE, kMoeKept))
             if (gated == kMoeGated) LEONE_MOE_STREAM(kMoeGated);
             else if (gated == kMoePlain) LEONE_MOE_STREAM(kMoePlain);
             else LEONE_MOE_STREAM(kMoeDown);
 #undef LEONE_MOE_STREAM
+#undef LEONE_MOE_LAID
         } else {
             const int blocks = ceil_div(n, tile == kWidePairs ? kWideRows : gated == kMoeGated ? kBigRows / 2 : kBigRows);
             const long places = static_cast<long>(max_tiles) * blocks;
@@ -1137,6 +1144,20 @@ extern "C" int leone_moe_product(const void* x, const void* w, void* y, const fl
 #undef LEONE_MOE
     LEONE_LAUNCH_CHECK("moe_product");
     return 0;
+}
+
+extern "C" int leone_moe_product(const void* x, const void* w, void* y, const float* pair_weight, int dtype, int gated,
+                                 const int* tile_expert, const int* tile_pairs, int max_tiles, int tile, int experts, int top, int n,
+                                 int k, int act, float limit, hipStream_t stream) {
+    return run_moe_product(x, w, 0, y, pair_weight, dtype, gated, tile_expert, tile_pairs, max_tiles, tile, experts, top, n, k, act, limit, stream);
+}
+
+// The same for tiles of 16 pairs with w as the copy [experts (, 2)][n / 16][k / 32][4][16][8]: element e of lane 16 g + c of step s of tile
+// t is row 16 t + c's element 32 s + 8 g + e.  n a multiple of 16, k of 32.
+extern "C" int leone_moe_product_tiles(const void* x, const void* w, void* y, const float* pair_weight, int gated, const int* tile_expert,
+                                       const int* tile_pairs, int max_tiles, int experts, int top, int n, int k, int act, float limit,
+                                       hipStream_t stream) {
+    return run_moe_product(x, w, 1, y, pair_weight, kBF16, gated, tile_expert, tile_pairs, max_tiles, 16, experts, top, n, k, act, limit, stream);
 }
 
 extern "C" int leone_moe_combine(const float* pair_out, const int* chosen, const float* weight, const void* x, int dtype,

@@ -2048,6 +2048,17 @@ def _expert_tiles(x: torch.Tensor, rows: int, top: int, experts: int, hidden: in
             torch.empty((max_tiles, tile), dtype=torch.int32, device=x.device))
 
 
+def tile_experts(weight: torch.Tensor) -> Optional[torch.Tensor]:
+    """The copy of experts' matrices ``[experts (, 2), rows, K]`` (bfloat16) that the products of few pairs read fastest: rows in tiles
+    of 16, K in steps of 32; element e of lane 16 g + c of step s of a tile is row c's element 32 s + 8 g + e, so that each load of a
+    wave is 1 KB in one piece.  None where the sizes have no such form (rows off 16, K off 32)."""
+    rows, k = weight.shape[-2:]
+    if weight.dtype != torch.bfloat16 or rows % 16 or k % 32:
+        return None
+    tiles = weight.reshape(-1, 16, k // 32, 4, 8).permute(0, 2, 3, 1, 4).contiguous()
+    return tiles.view(*weight.shape[:-2], rows // 16, k // 32, 4, 16, 8)
+
+
 def _check_experts(x: torch.Tensor, w_up: torch.Tensor, w_down: torch.Tensor):
     """(rows, hidden, experts, ff, whether the experts have a gate)."""
     rows, hidden = x.shape
@@ -2060,7 +2071,19 @@ def _check_experts(x: torch.Tensor, w_up: torch.Tensor, w_down: torch.Tensor):
     return rows, hidden, experts, ff, gated
 
 
-def _expert_products(x, chosen, weight, tiles, w_up, w_down, activation, extra, limit=None, weigh_input=False, paired=False):
+def _expert_copy(tiles: Optional[torch.Tensor], w: torch.Tensor, pairs_a_tile: int) -> Optional[torch.Tensor]:
+    """``tiles`` if the product of such tiles of pairs reads the experts' copy (of ``w``, or of more experts that begin with them)."""
+    if tiles is None or pairs_a_tile != 16:
+        return None
+    rows, k = w.shape[-2:]
+    if tiles.dtype != torch.bfloat16 or tiles.device != w.device or not tiles.is_contiguous() or tiles.shape[0] < w.shape[0] \
+            or tuple(tiles.shape[1:]) != (*w.shape[1:-2], rows // 16, k // 32, 4, 16, 8):
+        raise KernelError(f"routed experts: a copy {tuple(tiles.shape)} of {tiles.dtype} does not belong to {tuple(w.shape)}")
+    return tiles
+
+
+def _expert_products(x, chosen, weight, tiles, w_up, w_down, activation, extra, limit=None, weigh_input=False, paired=False,
+                     copies=(None, None)):
     rows, hidden, experts, ff, gated = _check_experts(x, w_up, w_down)
     if weigh_input and gated:
         raise KernelError("routed experts: a weight on what an expert reads goes with experts without a gate")
@@ -2072,51 +2095,58 @@ def _expert_products(x, chosen, weight, tiles, w_up, w_down, activation, extra, 
     weights = _dev(weight, "weights", torch.float32, (rows, top))
     hidden_act = torch.empty((pairs, ff), dtype=x.dtype, device=device)
     # the weight stands on the input's side (a product of weight * x is weight times the product) or on the result's
-    call("leone_moe_product", _dev(x, "routed rows"), _dev(w_up, "expert up"), _dev(hidden_act, "expert hidden"),
-         weights if weigh_input else 0, _code(x, "routed rows"), 1 if gated else 2, _dev(tile_expert, "tiles"),
-         _dev(tile_pairs, "tile pairs"), max_tiles, tile, experts, top, ff, hidden, act, limit, _stream())
     pair_out = torch.empty((pairs, hidden), dtype=torch.float32, device=device)
-    call("leone_moe_product", _dev(hidden_act, "expert hidden"), _dev(w_down, "expert down"), _dev(pair_out, "pair results"),
-         0 if weigh_input else weights, _code(x, "routed rows"), 0, _dev(tile_expert, "tiles"),
-         _dev(tile_pairs, "tile pairs"), max_tiles, tile, experts, top, hidden, ff, 0, 0.0, _stream())
+
+    def product(rows_in, w, copy, out, pair_weight, kind, n, k, code, held):
+        copy = _expert_copy(copy, w, tile)
+        if copy is not None:
+            call("leone_moe_product_tiles", _dev(rows_in, "routed rows", torch.bfloat16), _dev(copy, "experts' tiles"), _dev(out, "experts' results"),
+                 pair_weight, kind, _dev(tile_expert, "tiles"), _dev(tile_pairs, "tile pairs"), max_tiles, experts, top, n, k, code, held, _stream())
+            return
+        call("leone_moe_product", _dev(rows_in, "routed rows"), _dev(w, "experts"), _dev(out, "experts' results"), pair_weight,
+             _code(rows_in, "routed rows"), kind, _dev(tile_expert, "tiles"), _dev(tile_pairs, "tile pairs"), max_tiles, tile, experts, top, n, k,
+             code, held, _stream())
+
+    product(x, w_up, copies[0], hidden_act, weights if weigh_input else 0, 1 if gated else 2, ff, hidden, act, limit)
+    product(hidden_act, w_down, copies[1], pair_out, 0 if weigh_input else weights, 0, hidden, ff, 0, 0.0)
     out = PairedRows(pair_out, chosen, weight, x, extra, experts)
     return out if paired else out.sum()
 
 
 def routed_experts(x: torch.Tensor, chosen: torch.Tensor, weight: torch.Tensor, w_gate_up: torch.Tensor,
                    w_down: torch.Tensor, activation: str = "silu", extra: Optional[torch.Tensor] = None,
-                   limit: Optional[float] = None, weigh_input: bool = False, paired: bool = False):
+                   limit: Optional[float] = None, weigh_input: bool = False, paired: bool = False, copies: tuple = (None, None)):
     """Every row through the experts chosen for it: float32 ``[rows, hidden]`` = sum over a row's places of
     weight * W_down[e] (act(W_gate[e] x) * (W_up[e] x)), in the places' order; a chosen index from the number of
     experts on stands for an expert that hands the row on as it is; ``extra`` (float32 ``[rows, hidden]``) is added.
     ``w_gate_up`` is ``[experts, 2, ff, hidden]`` (gate rows, then up rows), ``w_down`` ``[experts, hidden, ff]``, both
     of ``x``'s type; experts without a gate come as ``[experts, ff, hidden]`` and compute W_down[e] act(W_up[e] x)
     (``PLAIN_ACTIVATIONS``).  ``weigh_input`` (experts without a gate): the weight multiplies what the expert reads
-    instead of what it gives.  ``paired``: the sum is left to the consumer (``PairedRows``).  Nothing here depends on the choice
-    except through device arrays."""
+    instead of what it gives.  ``paired``: the sum is left to the consumer (``PairedRows``).  ``copies``: ``tile_experts`` of both
+    matrices (None: none), which products of few pairs read instead.  Nothing here depends on the choice except through device arrays."""
     rows, hidden, experts, ff, _ = _check_experts(x, w_gate_up, w_down)
     top = chosen.shape[1]
     tiles = _expert_tiles(x, rows, top, experts, hidden, ff)
     call("leone_moe_plan", _dev(chosen, "chosen", torch.int32, (rows, top)), rows * top, experts, _dev(tiles[2], "tiles"),
          _dev(tiles[3], "tile pairs"), tiles[1], tiles[0], _stream())
-    return _expert_products(x, chosen, weight, tiles, w_gate_up, w_down, activation, extra, limit, weigh_input, paired)
+    return _expert_products(x, chosen, weight, tiles, w_gate_up, w_down, activation, extra, limit, weigh_input, paired, copies)
 
 
 def routed_feed_forward(x: torch.Tensor, logits: torch.Tensor, correction: Optional[torch.Tensor], top: int, group_count: int,
                         group_keep: int, w_gate_up: torch.Tensor, w_down: torch.Tensor, activation: str = "silu",
                         extra: Optional[torch.Tensor] = None, always: int = 0, rule: Optional[RouterRule] = None,
-                        limit: Optional[float] = None, weigh_input: bool = False, paired: bool = False):
+                        limit: Optional[float] = None, weigh_input: bool = False, paired: bool = False, copies: tuple = (None, None)):
     """``route_topk`` on the router's float32 ``logits`` and ``routed_experts`` with its choice; for steps of few rows
     (up to ``ROUTE_PLAN_ROWS``) the choice and the tiles are made in one launch.  ``always`` (such steps only): the
     last so many experts of the matrices are no choice of the router's but taken by every row with weight 1 (a
-    shared expert cut to the experts' size rides along in the experts' launches).  ``paired`` as for ``routed_experts``."""
+    shared expert cut to the experts' size rides along in the experts' launches).  ``paired`` and ``copies`` as for ``routed_experts``."""
     rows, hidden, experts, ff, _ = _check_experts(x, w_gate_up, w_down)
     total = logits.shape[1]
     if rows > ROUTE_PLAN_ROWS:
         if always:
             raise KernelError(f"routed_feed_forward: experts for every row ride along in steps of up to {ROUTE_PLAN_ROWS} rows only")
         chosen, weight = route_topk(logits, correction, top, group_count, group_keep, rule)
-        return routed_experts(x, chosen, weight, w_gate_up, w_down, activation, extra, limit, weigh_input, paired)
+        return routed_experts(x, chosen, weight, w_gate_up, w_down, activation, extra, limit, weigh_input, paired, copies)
     if total > library().leone_route_max_outputs():
         raise KernelError(f"route_topk: {total} router outputs, the kernel takes {library().leone_route_max_outputs()}")
     if not 0 <= always < experts:
@@ -2130,7 +2160,7 @@ def routed_feed_forward(x: torch.Tensor, logits: torch.Tensor, correction: Optio
          _dev(chosen, "chosen"), _dev(weight, "weights"), rows, total, int(top), int(group_count), int(group_keep), experts,
          _dev(tiles[2], "tiles"), _dev(tiles[3], "tile pairs"), tiles[1], tiles[0], int(always),
          *(rule or _DEFAULT_RULE).args(), _stream())
-    return _expert_products(x, chosen, weight, tiles, w_gate_up, w_down, activation, extra, limit, weigh_input, paired)
+    return _expert_products(x, chosen, weight, tiles, w_gate_up, w_down, activation, extra, limit, weigh_input, paired, copies)
 
 
 # ---- a forget gate per key channel, attention through a shared latent, the stream as a sum over depth -----------

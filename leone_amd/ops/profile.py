@@ -75,6 +75,7 @@ OPERATIONS = {
     "leone_moe_plan": "router",
     "leone_route_plan": "router",
     "leone_moe_product": "experts",
+    "leone_moe_product_tiles": "experts",
     "leone_moe_combine": "experts",
     "leone_gated_scan": "gated scan",
     "leone_gated_chain": "gated scan",

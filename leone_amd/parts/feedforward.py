@@ -156,6 +156,7 @@ class RoutedGluMlp(Part):
     """
 
     graph_safe = True
+    copies = (None, None)        # the experts' second copies, if the model keeps them
 
     def __init__(self, spec: PartSpec, **context):
         p = spec.params
@@ -217,6 +218,7 @@ class RoutedGluMlp(Part):
             down = torch.cat([down, cols.to(down.dtype)])
             self.always = pieces
         self.w_gate_up_all, self.w_down_all = gate_up.contiguous(), down.contiguous()
+        self.copies = (None, None)
         self.w_gate_up, self.w_down = self.w_gate_up_all[:self.experts], self.w_down_all[:self.experts]
         if self.shared is not None:
             self.shared.bind(tensors)
@@ -224,13 +226,22 @@ class RoutedGluMlp(Part):
     def streamed_weights(self) -> List[torch.Tensor]:
         return self.shared.streamed_weights() if self.shared is not None else []
 
+    def expert_copy_bytes(self) -> int:
+        """Bytes of the experts' second copies (``ops.tile_experts``), 0 if their sizes have no such form."""
+        both = (self.w_gate_up_all, self.w_down_all)
+        fits = all(w is not None and w.is_cuda and w.dtype == torch.bfloat16 and w.shape[-2] % 16 == 0 and w.shape[-1] % 32 == 0 for w in both)
+        return 2 * sum(w.numel() for w in both) if fits else 0
+
+    def keep_expert_copies(self) -> None:
+        self.copies = (ops.tile_experts(self.w_gate_up_all), ops.tile_experts(self.w_down_all))
+
     def forward(self, y: torch.Tensor, step: StepContext, paired: bool = False):
         y = ops.materialize(y)
         logits = ops.linear(y, self.w_router, out_dtype=torch.float32)
         if self.always and y.shape[0] <= ops.ROUTE_PLAN_ROWS:
             return ops.routed_feed_forward(y, logits, self.correction, self.top, self.group_count, self.group_keep,
                                            self.w_gate_up_all, self.w_down_all, self.activation, always=self.always,
-                                           rule=self.rule, limit=self.limit, paired=paired)
+                                           rule=self.rule, limit=self.limit, paired=paired, copies=self.copies)
         extra = None
         if self.shared is not None:
             extra = self.shared.forward(y, step)
@@ -240,6 +251,6 @@ class RoutedGluMlp(Part):
                 extra = extra.float()
         return ops.routed_feed_forward(y, logits, self.correction, self.top, self.group_count, self.group_keep,
                                        self.w_gate_up, self.w_down, self.activation, extra=extra, rule=self.rule,
-                                       limit=self.limit, weigh_input=self.weigh_input, paired=paired)
+                                       limit=self.limit, weigh_input=self.weigh_input, paired=paired, copies=self.copies)
 
     forward.gives_pairs = True       # ``paired``: the sum over a row's places is left to the norm behind (``ops.PairedRows``)

@@ -163,8 +163,8 @@ class DecoderModel:
         library's products of prompt portions and for the token table).  The results are the same bit for
         bit; a decode step of few rows takes a sixth less time; the weights take twice the memory.
         ``wanted`` None decides by room: yes if the copies take at most a quarter of the device's memory
-        and half of what is free.  Returns the bytes the copies take (0: none kept).  Asked again, it
-        answers what it did the first time."""
+        and half of what is free.  Routed experts get theirs (``ops.tile_experts``) behind these, all or none, if there is room for
+        both.  Returns the bytes the copies take (0: none kept).  Asked again, it answers what it did the first time."""
         if self.streamed_copy_bytes is not None:
             return self.streamed_copy_bytes
         self.streamed_copy_bytes = 0
@@ -172,12 +172,19 @@ class DecoderModel:
         weights = [w for w in weights if w.is_cuda and w.dtype == torch.bfloat16 and w.dim() == 2 and w.shape[1] % 64 == 0]
         if not weights:
             return 0
-        if wanted is None:
-            needed = sum(-(-w.shape[0] // 16) * 16 * w.shape[1] * 2 for w in weights)
-            free, total = torch.cuda.mem_get_info(weights[0].device)
-            if needed > self.STREAMED_SHARE_OF_DEVICE * total or needed > self.STREAMED_SHARE_OF_FREE * free:
-                return 0
+        needed = sum(-(-w.shape[0] // 16) * 16 * w.shape[1] * 2 for w in weights)
+        free, total = torch.cuda.mem_get_info(weights[0].device)
+        room = min(self.STREAMED_SHARE_OF_DEVICE * total, self.STREAMED_SHARE_OF_FREE * free)
+        if wanted is None and needed > room:
+            return 0
+        experts = [part for layer in self.layers for part in (layer.parts() if hasattr(layer, "parts") else ())
+                   if hasattr(part, "expert_copy_bytes") and part.expert_copy_bytes()]
+        of_experts = sum(part.expert_copy_bytes() for part in experts)
         self.streamed_copy_bytes = sum(ops.keep_streamed_copy(w) for w in weights)
+        if experts and needed + of_experts <= room:
+            for part in experts:
+                part.keep_expert_copies()
+            self.streamed_copy_bytes += of_experts
         return self.streamed_copy_bytes
 
     def row_tilings(self) -> list:

@@ -1,0 +1,66 @@
+"""Experts' products of few pairs from the matrices' second copies: the bits of the products from the matrices themselves."""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+# inner sizes of fewer steps than waves, of one, of eight and more a wave, off whole shares; rows of one tile and of many
+@pytest.mark.parametrize("gated", [True, False])
+@pytest.mark.parametrize("experts,rows,top,hidden,ff", [(4, 1, 1, 32, 16), (6, 3, 2, 96, 32), (5, 20, 2, 288, 160), (34, 8, 6, 1056, 768),
+                                                        (33, 8, 4, 2048, 768), (16, 9, 3, 4096, 1024)])
+def test_the_same_bits(gated, experts, rows, top, hidden, ff):
+    from leone_amd import ops
+    gen = torch.Generator().manual_seed(experts + hidden)
+    chosen = torch.stack([torch.randperm(experts + 1, generator=gen)[:top] for _ in range(rows)]).to(torch.int32).to(DEV)
+    weight = torch.rand(rows, top, generator=gen).to(DEV)
+    x = torch.randn(rows, hidden, generator=gen).bfloat16().to(DEV)
+    up = (torch.randn(experts, *((2,) if gated else ()), ff, hidden, generator=gen) / math.sqrt(hidden)).bfloat16().to(DEV)
+    down = (torch.randn(experts, hidden, ff, generator=gen) / math.sqrt(ff)).bfloat16().to(DEV)
+    copies = (ops.tile_experts(up), ops.tile_experts(down))
+    for options in (({}, {"activation": "gelu_tanh"}) if gated else ({"activation": "relu2"}, {"activation": "relu2", "weigh_input": True})):
+        want = ops.routed_experts(x, chosen, weight, up, down, **options)
+        assert torch.equal(ops.routed_experts(x, chosen, weight, up, down, copies=copies, **options), want)
+        # a copy of more experts than take part
+        fewer = ops.routed_experts(x, chosen, weight, up[:experts - 1], down[:experts - 1], **options)
+        assert torch.equal(ops.routed_experts(x, chosen, weight, up[:experts - 1], down[:experts - 1], copies=copies, **options), fewer)
+
+
+def test_where_there_is_no_copy():
+    from leone_amd import ops
+    assert ops.tile_experts(torch.zeros(2, 24, 32, dtype=torch.bfloat16)) is None
+    assert ops.tile_experts(torch.zeros(2, 32, 48, dtype=torch.bfloat16)) is None
+    assert ops.tile_experts(torch.zeros(2, 32, 32)) is None
+    x = torch.randn(2, 64, device=DEV).bfloat16()
+    up, down = torch.randn(3, 2, 32, 64, device=DEV).bfloat16(), torch.randn(3, 64, 32, device=DEV).bfloat16()
+    chosen, weight = torch.zeros(2, 1, dtype=torch.int32, device=DEV), torch.ones(2, 1, device=DEV)
+    with pytest.raises(ops.KernelError, match="does not belong"):
+        ops.routed_experts(x, chosen, weight, up, down, copies=(ops.tile_experts(up)[:2], None))
+    want = ops.routed_experts(x, chosen, weight, up, down)
+    assert torch.equal(ops.routed_experts(x, chosen, weight, up, down, copies=(None, ops.tile_experts(down))), want)
+
+
+@pytest.mark.parametrize("wanted,free,kept", [(None, 1 << 40, True), (False, 1 << 40, False), (True, 1 << 40, True), (None, 1 << 15, False), (True, 1 << 15, False)])
+def test_a_model_keeps_the_copies_if_there_is_room(monkeypatch, wanted, free, kept):
+    from leone_amd import ops
+    from leone_amd.parts.base import FEED_FORWARDS, PartSpec
+    from leone_amd.parts.model import DecoderModel
+    part = FEED_FORWARDS.build(PartSpec("routed_glu", {"hidden": 64, "experts": 2, "top": 1, "intermediate": 32, "router": "r", "expert": "e{e}"}))
+    made = {"r": torch.zeros(2, 64), **{f"e{e}.{n}": torch.randn(*shape) for e in range(2)
+                                        for n, shape in (("gate", (32, 64)), ("up", (32, 64)), ("down", (64, 32)))}}
+    part.bind({name: t.bfloat16().to(DEV) for name, t in made.items()})
+    dense = torch.randn(64, 64, device=DEV).bfloat16()
+
+    class Layer:
+        parts = staticmethod(lambda: (part,))
+        streamed_weights = staticmethod(lambda: [dense])
+    model = DecoderModel.__new__(DecoderModel)
+    model.layers, model.dtype, model.streamed_copy_bytes, model.head, model.embedding = [Layer], torch.bfloat16, None, None, None
+    monkeypatch.setattr(DecoderModel, "streamed_weights", lambda self: [dense])
+    monkeypatch.setattr(torch.cuda, "mem_get_info", lambda *a: (free, 1 << 40))
+    assert model.keep_streamed_copies(wanted) == (0 if wanted is False else 64 * 64 * 2 + (part.expert_copy_bytes() if kept else 0))
+    assert (part.copies[0] is not None) == kept
+    ops.drop_streamed_copies()
