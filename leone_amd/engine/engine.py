@@ -154,6 +154,15 @@ class _DecodeGraph:
         self.rows = rows
         self._pieces, self._tables = pieces, {g: pieces[5 + len(tilings) + g].view(rows, widths[g]) for g in range(groups)}
         self._engine_type = (engine.dtype, engine.device)
+        # what the layout routine is given for ``rows`` single tokens and gives back; requests and tokens are filled in step by step
+        ones, nothing = (c_int * rows)(*[1] * rows), (c_int * rows)()
+        self._requests, self._given = (c_int64 * rows)(), (ctypes.c_int32 * rows)()
+        flat = [v for t in tilings for v in (t.tile_rows, t.min_rows, t.group_tiles)]
+        self._sections, self._summary = (c_long * (len(sizes) + 1))(), (c_int * (4 + 2 * len(tilings)))()
+        self._placed = (c_int * (5 * rows))()
+        self._pack_args = (ones, nothing, self._given, (ctypes.c_int32 * 1)(),
+                           (c_int * (3 + len(flat)))(engine.vocab_size, 1, len(tilings), *flat),
+                           ctypes.cast(self.host.data_ptr(), hostlib.PI32), total, self._sections, self._summary, self._placed)
         self.recordings: Dict[int, tuple] = {}        # context range -> (graph, its logits)
         self.copied = torch.cuda.Event()
 
@@ -165,15 +174,38 @@ class _DecodeGraph:
             row_entry=pieces[2], entries=[], entry_slots=pieces[3], want_rows=pieces[4],
             block_tables=self._tables, max_position=bucket - 1, decode_only=True)
 
-    def fill(self, engine: "Engine", entries: Sequence[StepEntry]) -> PackedStep:
+    def _pack_single(self, engine: "Engine", entries: Sequence[StepEntry]) -> Optional[int]:
+        """The layout of ``rows`` single tokens, written in one native call from arrays that are there already; the largest position, or
+        None for anything out of the ordinary (``PackedStep`` then takes it, or says what is wrong with it)."""
+        key_of, vocab = engine.cache.keys.key, engine.vocab_size
+        if len(entries) != self.rows:
+            return None
+        for i, e in enumerate(entries):
+            if len(e.tokens) != 1 or len(e.want) > 1 or (len(e.want) == 1 and e.want[0] != 0):
+                return None
+            token = e.tokens[0]
+            if type(token) is not int or not 0 <= token < vocab:
+                return None
+            key = key_of(e.request)
+            if key is None:
+                return None
+            self._requests[i], self._given[i] = key, token
+        total = hostlib.library().leone_step_pack(engine.cache.handle, self.rows, self._requests, *self._pack_args)
+        return self._summary[1] if total == self.offsets[-1] and self._sections[:] == self.offsets else None
+
+    def fill(self, engine: "Engine", entries: Sequence[StepEntry]) -> int:
+        """The step's metadata on its way to the device; the largest position of its rows."""
         self.copied.synchronize()                     # the last upload has left the pinned buffer
-        packed = PackedStep(engine.cache, engine.vocab_size, entries, all_rows_wanted=True, host=self.host,
-                            tilings=engine.tilings)
-        if packed.offsets != self.offsets:
-            raise StepError("the step does not fit the recorded layout")
+        position = self._pack_single(engine, entries)
+        if position is None:
+            packed = PackedStep(engine.cache, engine.vocab_size, entries, all_rows_wanted=True, host=self.host,
+                                tilings=engine.tilings)
+            if packed.offsets != self.offsets:
+                raise StepError("the step does not fit the recorded layout")
+            position = packed.max_position
         self.dev.copy_(self.host, non_blocking=True)
         self.copied.record()
-        return packed
+        return position
 
 
 class Engine:
@@ -386,10 +418,10 @@ class Engine:
         # replayed from a recording it already has cannot fail half way (it is refused before the replay or not at
         # all), so the copy of the state, a launch and all its bytes, is left out there.
         replayed = self.graphs and not profile.recording() and all(len(e.tokens) == 1 for e in entries)
-        saved_state = None if (replayed and self._has_recording(entries)) else \
+        saved_state = None if not self.pools.state or (replayed and self._has_recording(entries)) else \
             self.pools.snapshot_state([self.cache.slot(e.request) for e in entries])
         try:
-            for e in entries:
+            for e in entries if self.pools.state else ():
                 if self.cache.length(e.request) == 0:
                     self.pools.zero_state(self.cache.slot(e.request))   # a request's state starts from zero
             # A step that is being profiled runs call by call: a replayed recording has no calls to time.
@@ -427,10 +459,10 @@ class Engine:
         state = self._decode_graphs.get(len(entries))
         if state is None:
             state = self._decode_graphs[len(entries)] = _DecodeGraph(self, len(entries))
-        packed = state.fill(self, entries)
+        position = state.fill(self, entries)
         if device_tokens is not None:                 # after the upload, on the same stream
             torch.clamp(device_tokens, 0, self.vocab_size - 1, out=state.tokens)
-        bucket = context_bucket(packed.max_position + 1, self.max_context)
+        bucket = context_bucket(position + 1, self.max_context)
         recording = state.recordings.get(bucket)
         if recording is None:
             # First step of this size and context range: run it for real on the static buffers, then record

@@ -85,36 +85,32 @@ class DeviceChoice:
         count = len(rows)
         draws = [rng.uniform(p.seed, e.sample_position) if kind in ("temperature", "truncated") else 0.0
                  for p, e, kind in zip(policies, rows, kinds)]
-        pieces = []
-        if "temperature" in kinds:
-            pieces.append(np.array([[p.temperature if kind == "temperature" else 1.0 for p, kind in zip(policies, kinds)],
-                                    draws], dtype=np.float64).reshape(-1))
-        if "truncated" in kinds:
-            pieces.append(ops.truncated_rows([(p.temperature, u, p.truncations) if kind == "truncated" else None
-                                              for p, u, kind in zip(policies, draws, kinds)]).reshape(-1))
         # which rows are of which kind (a batch of one kind needs no list)
         self.names = [name for name in ops.CHOICE_KINDS if name in kinds]
-        if len(self.names) > 1:
-            pieces.append(np.array([ops.CHOICE_KINDS.get(kind, 0) for kind in kinds], dtype=np.float64))
+        mixed, tempered, cut = len(self.names) > 1, "temperature" in kinds, "truncated" in kinds
         self.scaled = self.truncated = self.codes = None
-        if pieces:
-            flat = np.concatenate(pieces)
-            if staging is not None:
-                host = staging(flat.size)
-                host.numpy()[:] = flat
-                on_device = host.to(device, non_blocking=True)
-            else:
-                on_device = torch.from_numpy(flat).to(device)
-            at = 0
-            if "temperature" in kinds:
-                self.scaled = on_device[:2 * count].view(2, count)
-                at = 2 * count
-            if "truncated" in kinds:
-                width = 3 + 2 * ops.TRUNCATED_STAGES
-                self.truncated = on_device[at:at + count * width].view(count, width)
-                at += count * width
-            if len(self.names) > 1:
-                self.codes = on_device[at:at + count]
+        if not tempered and not cut:
+            return
+        width = 3 + 2 * ops.TRUNCATED_STAGES
+        size = count * (2 * tempered + width * cut + mixed)
+        host = staging(size) if staging is not None else torch.empty(size, dtype=torch.float64)
+        flat, at = host.numpy(), 0
+        if tempered:
+            flat[:2 * count] = [p.temperature if kind == "temperature" else 1.0 for p, kind in zip(policies, kinds)] + draws
+            at = 2 * count
+        if cut:
+            flat[at:at + count * width] = ops.truncated_rows([(p.temperature, u, p.truncations) if kind == "truncated" else None
+                                                              for p, u, kind in zip(policies, draws, kinds)]).reshape(-1)
+            at += count * width
+        if mixed:
+            flat[at:] = [ops.CHOICE_KINDS.get(kind, 0) for kind in kinds]
+        on_device = host.to(device, non_blocking=staging is not None)
+        if tempered:
+            self.scaled = on_device[:2 * count].view(2, count)
+        if cut:
+            self.truncated = on_device[at - count * width:at].view(count, width)
+        if mixed:
+            self.codes = on_device[at:]
 
     def choose(self, logits: torch.Tensor) -> torch.Tensor:
         """int32 [rows] on the device: the token each row's kernel chose, -1 for a row without a finite logit; None if no row is
