@@ -385,9 +385,9 @@ int leone_moe_plan(const int* chosen, int pairs, int experts, int* tile_expert, 
 int leone_moe_product(const void* x, const void* w, void* y, const float* pair_weight, int dtype, int gated,
                       const int* tile_expert, const int* tile_pairs, int max_tiles, int tile, int experts, int top, int n, int k,
                       int act, float limit, hipStream_t stream);
-// The same for tiles of 16 pairs, bfloat16, with w as a copy in tiles (layout at the kernel's entry in routed.hip).
+// The same for tiles of 16, 64 and 128 pairs, bfloat16, with w as a copy in tiles (layout at the kernel's entry in routed.hip).
 int leone_moe_product_tiles(const void* x, const void* w, void* y, const float* pair_weight, int gated, const int* tile_expert,
-                            const int* tile_pairs, int max_tiles, int experts, int top, int n, int k, int act, float limit,
+                            const int* tile_pairs, int max_tiles, int tile, int experts, int top, int n, int k, int act, float limit,
                             hipStream_t stream);
 // Whether tiles of 64 pairs keep one chunk of such experts' matrices on its way, not two.
 int leone_moe_one_chunk_ahead(int experts, int gated, int n, int k);

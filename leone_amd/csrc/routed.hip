@@ -969,6 +969,202 @@ moe_product_wide_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__
     }
 }
 
+// Tiles of 64 and 128 pairs from the matrices' second copies (kMoeTiled), inner sizes that are multiples of 64: a workgroup takes a tile of
+// pairs and 128 kNT rows of its expert's matrix (gated: half as many gate rows and their up rows), a wave a quarter of them in parts of 32, whose
+// elements it takes from memory as its instruction (32 x 32 x 16) wants them, one or two stages of 64 ahead: they pass neither through shared memory
+// nor a barrier.  The pairs' rows, which all four waves read, go through shared memory, a stage's 128 bytes of a row turned about by the row's
+// number so that the same piece of 16 rows lies in 16 places; a stage is written while the one before it is worked on.
+//
+// What bounds it is the power of the chip (matrix instructions alone, on all units, run at two thirds of the clock) and what goes through
+// shared memory: hence 256 rows a workgroup, which read a piece of the pairs' rows half as often, wherever that leaves work for the units (see
+// many_rows), and results turned in shared memory so that stores are whole lines (as 16 bytes of 32 rows they took a third of the
+// second product).  With the matrices row by row the same kernel takes 1.4 times as long (half a line of 32 rows a load).
+// Both products, us, best tiles of moe_product_tiled_kernel and moe_product_wide_kernel and now: 32 experts of 2,048 x 768, 40 pairs each 79 and 63, 100
+// pairs 109 and 75, 240 pairs 176 and 132, 400 pairs 256 and 181, 700 pairs 358 and 277; 32 of 4,096 x 1,024, 240 pairs 413 and 306; 64 of 2,048 x 1,408,
+// 100 pairs 322 and 250; 32 of 1,024 x 384, 100 pairs 37 and 26; 8 of 1,024 x 4,096, 300 pairs 138 and 125.
+typedef float moe_floatx16 __attribute__((ext_vector_type(16)));
+constexpr int kTogether = 2;
+template <int kMode, int kMT, int kNT>
+__global__ void __launch_bounds__(kMoeThreads, kNT == 1 ? 3 : 2)
+moe_product_many_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, void* __restrict__ y, const float* __restrict__ pair_weight,
+                        const int* __restrict__ tile_expert, const int* __restrict__ tile_pairs, int top, int n, int k, int act, float limit,
+                        int n_tiles, int n_blocks) {
+    constexpr bool kGated = kMode == kMoeGated;
+    constexpr int kPairs = 32 * kMT, kOwnRows = (kGated ? 64 : 128) * kNT, kWAhead = kNT == 1 ? 2 : 1, kCopies = kPairs * 8 / kMoeThreads;
+    __shared__ uint4 sx[2][kPairs * 8];
+    __shared__ int s_pairs[kPairs];
+    __shared__ float s_scale[kPairs];
+    // Workgroups go to the eight dies in turn: a die gets every eighth run of kTogether tiles, with all blocks of their matrices' rows, the
+    // tiles of a run fastest.  The pairs' rows are then read from the die's own cache by all blocks but the first, and a block of rows by the tiles
+    // of one expert at about the same time.
+    const int place = static_cast<int>(blockIdx.x / 8), run = place / (kTogether * n_blocks), within = place % (kTogether * n_blocks);
+    const int tile = (run * 8 + static_cast<int>(blockIdx.x % 8)) * kTogether + within % kTogether, row_block = within / kTogether;
+    if (tile >= n_tiles) return;
+    const int e = tile_expert[tile];
+    if (e < 0) return;
+    const int tid = threadIdx.x, lane = tid % kWave, wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int c = lane & 31, hi = lane >> 5;
+    const long matrix = static_cast<long>(n) * k;
+    const int* my_pairs = tile_pairs + static_cast<long>(tile) * kPairs;
+    const int stages = k / 64;
+
+    // this lane's row of the matrix: of 32, the first 16 and the others are a tile each (gated: gate rows and their up rows)
+    const bf16_t* wp[kNT];
+#pragma unroll
+    for (int u = 0; u < kNT; ++u) {
+        const int wanted = kGated ? (row_block * 4 + wave) * kNT + u : ((row_block * 4 + wave) * kNT + u) * 2 + (c >> 4);
+        const int tile16 = wanted < n / 16 ? wanted : n / 16 - 1;
+        wp[u] = w + static_cast<long>(e) * (kGated ? 2 : 1) * matrix + (kGated ? (c >> 4) * matrix : 0) +
+                static_cast<long>(tile16) * 16 * k + hi * 128 + (c & 15) * 8;
+    }
+    const bf16_t* x_from[kCopies];
+    int x_to[kCopies];
+#pragma unroll
+    for (int i = 0; i < kCopies; ++i) {                  // (in place of no pair the tile's first one: not written)
+        const int q = i * kMoeThreads + tid, row = q >> 3, part = q & 7;
+        const int own = my_pairs[row], pair = own < 0 ? my_pairs[0] : own;
+        x_from[i] = x + static_cast<long>(kMode != kMoeDown ? pair / top : pair) * k + 8 * part;
+        x_to[i] = row * 8 + (part ^ ((row >> 1) & 7));
+    }
+    if (tid < kPairs) {                                  // the pairs again, for the end
+        const int own = my_pairs[tid];
+        s_pairs[tid] = own;
+        if (!kGated && pair_weight) s_scale[tid] = pair_weight[own < 0 ? my_pairs[0] : own];
+    }
+    const auto inside = [&](int s) { return s < stages ? s : stages - 1; };              // (past the end the last stage again, unused)
+    const auto load_x = [&](int s, int i) { return *reinterpret_cast<const uint4*>(x_from[i] + static_cast<long>(inside(s)) * 64); };
+    const auto load_w = [&](int s, int j, int u) {
+        return *reinterpret_cast<const uint4*>(wp[u] + static_cast<long>(inside(s)) * 1024 + j * 256);
+    };
+    moe_floatx16 acc[kMT][kNT];
+#pragma unroll
+    for (int t = 0; t < kMT; ++t)
+#pragma unroll
+        for (int u = 0; u < kNT; ++u)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) acc[t][u][i] = 0.f;
+    constexpr int kAhead = kMT <= 2 ? 2 : 1;             // stages of the pairs' rows on their way in registers
+    uint4 held[kAhead][kCopies], weights[kWAhead][4][kNT];
+    moe_bf16x8 xb[2][kMT];
+    const auto read_x = [&](const uint4* from, int j, int t) {
+        const int row = 32 * t + c;
+        return __builtin_bit_cast(moe_bf16x8, from[row * 8 + ((2 * j + hi) ^ ((row >> 1) & 7))]);
+    };
+    // The i-th copy belongs to this place among a stage's 4 kMT pairs of a read and an instruction: within the first three quarters, behind
+    // which the stage's barrier stands.  The loads ahead of the loop are asked for in the loop's order, or the compiler, which counts the
+    // loads in flight, would wait for younger ones.
+    const auto place_of = [&](int i) { return i * 3 * kMT / kCopies; };
+    {
+        uint4 first[kCopies];
+#pragma unroll
+        for (int i = 0; i < kCopies; ++i) first[i] = load_x(0, i);
+#pragma unroll
+        for (int v = 0; v < 2; ++v)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+#pragma unroll
+                for (int i = 0; i < kCopies; ++i)
+                    if (place_of(i) / kMT == j && v >= 2 - kAhead) held[(v + 1 + kAhead) % kAhead][i] = load_x(v - 1 + kAhead, i);
+                if (v >= 2 - kWAhead)
+#pragma unroll
+                    for (int u = 0; u < kNT; ++u) weights[v % kWAhead][j][u] = load_w(v - 2 + kWAhead, j, u);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+        for (int i = 0; i < kCopies; ++i) sx[0][x_to[i]] = first[i];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < kMT; ++t) xb[0][t] = read_x(sx[0], 0, t);
+    const auto stage = [&](int s, auto parity) {
+        constexpr int p = decltype(parity)::value;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            if (j == 3) {                                // the next stage lies in shared memory, and everyone has read this one
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+                __builtin_amdgcn_s_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+            }
+#pragma unroll
+            for (int t = 0; t < kMT; ++t) {
+                xb[(j + 1) & 1][t] = j < 3 ? read_x(sx[p], j + 1, t) : read_x(sx[p ^ 1], 0, t);
+#pragma unroll
+                for (int i = 0; i < kCopies; ++i)
+                    if (place_of(i) == j * kMT + t) {
+                        sx[p ^ 1][x_to[i]] = held[(p + 1) % kAhead][i];
+                        held[(p + 1) % kAhead][i] = load_x(s + 1 + kAhead, i);
+                    }
+#pragma unroll
+                for (int u = 0; u < kNT; ++u)
+                    acc[t][u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(moe_bf16x8, weights[p % kWAhead][j][u]), xb[j & 1][t], acc[t][u], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int u = 0; u < kNT; ++u) weights[p % kWAhead][j][u] = load_w(s + kWAhead, j, u);
+        }
+    };
+    int s = 0;
+    for (; s + 1 < stages; s += 2) {
+        stage(s, std::integral_constant<int, 0>{});
+        stage(s + 1, std::integral_constant<int, 1>{});
+    }
+    if (s < stages) stage(s, std::integral_constant<int, 0>{});
+    // Lane (c, hi) holds, of pair c of every t, rows 8 q + 4 hi .. + 3 of each of the wave's 32.  They are turned in shared memory, a wave's
+    // own part of it, so that a store covers whole runs of a pair's rows (straight from the registers it would be 16 bytes of 32 rows).
+    __syncthreads();                                     // the last stage has been read
+    constexpr int kBytes = kMode == kMoeDown ? 4 : 2, kWaveRows = kOwnRows / 4;
+    constexpr int kAtOnce = kMode == kMoeDown ? 1 : kNT;             // of the wave's parts of 32 (gated: 16) rows
+    constexpr int kRun = kWaveRows / kNT * kAtOnce * kBytes / 16;    // 16-byte pieces of a pair's rows at once
+    static_assert(kRun * 32 * 16 <= sizeof(sx) / 4 && (kRun == 2 || kRun == 4 || kRun == 8), "a wave's part of the stages' memory");
+    uint4* mine = &sx[0][0] + wave * (kRun * 32);
+    const auto turn = [](int pair) { return (kRun == 8 ? pair >> 1 : kRun == 4 ? pair >> 2 : pair >> 3) & (kRun - 1); };
+    const int row0 = row_block * kOwnRows + wave * kWaveRows;
+#pragma unroll
+    for (int t = 0; t < kMT; ++t) {
+        const float scale = kGated || !pair_weight ? 1.f : s_scale[32 * t + c];
+#pragma unroll
+        for (int u0 = 0; u0 < kNT; u0 += kAtOnce) {
+#pragma unroll
+            for (int u = u0; u < u0 + kAtOnce; ++u)
+#pragma unroll
+                for (int q = 0; q < (kGated ? 2 : 4); ++q) {
+                    float v[4];
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const float value = acc[t][u][4 * q + j];
+                        v[j] = kGated ? glu_value(value, acc[t][u][(4 * q + j + 8) & 15], act, limit)
+                                      : kMode == kMoePlain ? plain_act(value * scale, act) : value * scale;
+                    }
+                    const int at = (u - u0) * (kWaveRows / kNT) + 8 * q + 4 * hi;        // the first of the four rows
+                    const int piece = (at * kBytes / 16) ^ turn(c);
+                    if constexpr (kBytes == 4) {
+                        mine[c * kRun + piece] = __builtin_bit_cast(uint4, float4{v[0], v[1], v[2], v[3]});
+                    } else {
+                        uint2 packed;
+                        packed.x = bf16_bits_from_float(v[0]) | (static_cast<uint32_t>(bf16_bits_from_float(v[1])) << 16);
+                        packed.y = bf16_bits_from_float(v[2]) | (static_cast<uint32_t>(bf16_bits_from_float(v[3])) << 16);
+                        reinterpret_cast<uint2*>(mine)[2 * (c * kRun + piece) + hi] = packed;
+                    }
+                }
+            __builtin_amdgcn_wave_barrier();             // (the wave's own writes, read by its other lanes: in order in shared memory)
+#pragma unroll
+            for (int i = 0; i < kRun / 2; ++i) {
+                const int pair = i * (kWave / kRun) + lane / kRun, piece = lane % kRun;
+                const uint4 whole = mine[pair * kRun + (piece ^ turn(pair))];
+                const int to = s_pairs[32 * t + pair], r = row0 + u0 * (kWaveRows / kNT) + piece * (16 / kBytes);
+                if (to >= 0 && r < n) *reinterpret_cast<uint4*>(static_cast<char*>(y) + (static_cast<long>(to) * n + r) * kBytes) = whole;
+            }
+            __builtin_amdgcn_wave_barrier();
+        }
+    }
+}
+
+// 256 rows of the matrix a workgroup (gated: 128 and their up rows) where tiles are of 128 pairs and that leaves some 200 workgroups, by the tiles
+// that are likely to be used: us, 256 and 128 rows: 32 experts of 2,048 x 768, first product, 100 pairs each (246 workgroups) 52 and 55, 240 pairs (456) 79 and 85; second, 240
+// pairs 52 and 50, 400 pairs 70 and 80; 8 of 4,096 x 2,048, 150 pairs (208) 75 and 83; but 32 of 1,024 x 384, 100 pairs (198) 18.0 and 16.2; 16 of
+// 2,048 x 1,024, 16 pairs (96) 31 and 26; second product of 8 of 1,024 x 4,096, 300 pairs (88) 43 and 35.
+static bool many_rows(int tiles, int n, bool gated) { return static_cast<long>(tiles) * ceil_div(n, gated ? 128 : 256) >= 200; }
+
 // A workgroup takes 256 columns of a row; a thread one column.
 template <typename T>
 __global__ void __launch_bounds__(256)
@@ -1078,7 +1274,8 @@ extern "C" int leone_moe_plan(const int* chosen, int pairs, int experts, int* ti
 static int run_moe_product(const void* x, const void* w, int w_tiled, void* y, const float* pair_weight, int dtype, int gated,
                            const int* tile_expert, const int* tile_pairs, int max_tiles, int tile, int experts, int top, int n, int k,
                            int act, float limit, hipStream_t stream) {
-    LEONE_REQUIRE(!w_tiled || (tile == 16 && n % 16 == 0 && k % 32 == 0), "moe_product: matrices in tiles go with 16 pairs and sizes %d x %d", n, k);
+    LEONE_REQUIRE(!w_tiled || (n % 16 == 0 && (tile == 16 ? k % 32 == 0 : (tile == kBigPairs || tile == kWidePairs) && k % 64 == 0)),
+                  "moe_product: matrices in tiles do not go with tiles of %d pairs and sizes %d x %d", tile, n, k);
     LEONE_REQUIRE(gated >= kMoeDown && gated <= kMoePlain, "moe_product: unknown kind of product %d", gated);
     LEONE_REQUIRE(act == kGateSilu || act == kGateGeluTanh || (act == kGateClampedSwish && limit > 0.f && gated != kMoePlain) ||
                       (act == kActReluSquared && gated != kMoeGated),
@@ -1103,6 +1300,22 @@ static int run_moe_product(const void* x, const void* w, int w_tiled, void* y, c
             else LEONE_MOE_STREAM(kMoeDown);
 #undef LEONE_MOE_STREAM
 #undef LEONE_MOE_LAID
+        } else if (w_tiled) {
+            const bool many = tile == kWidePairs && many_rows(max_tiles - experts / 2, n, gated == kMoeGated);
+            const int blocks = ceil_div(n, (gated == kMoeGated ? 64 : 128) * (many ? 2 : 1));
+            const long places = static_cast<long>(ceil_div(max_tiles, 8 * kTogether)) * 8 * kTogether * blocks;
+            LEONE_REQUIRE(places <= 0x7fffffffL, "moe_product: too many tiles");
+            const int grid = static_cast<int>(places);
+#define LEONE_MOE_MANY(MODE, MT, NT)                                                                                          \
+    moe_product_many_kernel<MODE, MT, NT><<<grid, kMoeThreads, 0, stream>>>(                                                   \
+        static_cast<const bf16_t*>(x), static_cast<const bf16_t*>(w), y, pair_weight, tile_expert, tile_pairs, top, n, k, act, limit, max_tiles, blocks)
+#define LEONE_MOE_PAIRS(MODE)                                                                                                  \
+    (tile == kBigPairs ? LEONE_MOE_MANY(MODE, 2, 1) : many ? LEONE_MOE_MANY(MODE, 4, 2) : LEONE_MOE_MANY(MODE, 4, 1))
+            if (gated == kMoeGated) LEONE_MOE_PAIRS(kMoeGated);
+            else if (gated == kMoePlain) LEONE_MOE_PAIRS(kMoePlain);
+            else LEONE_MOE_PAIRS(kMoeDown);
+#undef LEONE_MOE_PAIRS
+#undef LEONE_MOE_MANY
         } else {
             const int blocks = ceil_div(n, tile == kWidePairs ? kWideRows : gated == kMoeGated ? kBigRows / 2 : kBigRows);
             const long places = static_cast<long>(max_tiles) * blocks;
@@ -1152,12 +1365,13 @@ extern "C" int leone_moe_product(const void* x, const void* w, void* y, const fl
     return run_moe_product(x, w, 0, y, pair_weight, dtype, gated, tile_expert, tile_pairs, max_tiles, tile, experts, top, n, k, act, limit, stream);
 }
 
-// The same for tiles of 16 pairs with w as the copy [experts (, 2)][n / 16][k / 32][4][16][8]: element e of lane 16 g + c of step s of tile
-// t is row 16 t + c's element 32 s + 8 g + e.  n a multiple of 16, k of 32.
+// The same for tiles of 16, 64 and 128 pairs with w as the copy [experts (, 2)][n / 16][k / 32][4][16][8]: element e of lane 16 g + c of step s of tile
+// t is row 16 t + c's element 32 s + 8 g + e.  n a multiple of 16, k of 32 (of 64 beyond 16 pairs).
 extern "C" int leone_moe_product_tiles(const void* x, const void* w, void* y, const float* pair_weight, int gated, const int* tile_expert,
-                                       const int* tile_pairs, int max_tiles, int experts, int top, int n, int k, int act, float limit,
-                                       hipStream_t stream) {
-    return run_moe_product(x, w, 1, y, pair_weight, kBF16, gated, tile_expert, tile_pairs, max_tiles, 16, experts, top, n, k, act, limit, stream);
+                                       const int* tile_pairs, int max_tiles, int tile, int experts, int top, int n, int k, int act,
+                                       float limit, hipStream_t stream) {
+    LEONE_REQUIRE(tile != kTilePairs, "moe_product: matrices in tiles do not go with tiles of %d pairs", tile);
+    return run_moe_product(x, w, 1, y, pair_weight, kBF16, gated, tile_expert, tile_pairs, max_tiles, tile, experts, top, n, k, act, limit, stream);
 }
 
 extern "C" int leone_moe_combine(const float* pair_out, const int* chosen, const float* weight, const void* x, int dtype,

@@ -2024,8 +2024,8 @@ def route_topk(logits: torch.Tensor, correction: Optional[torch.Tensor], top: in
 ROUTE_PLAN_ROWS = 64          # up to here the router's choice and the tiles are made in one launch
 
 
-def _expert_tiles(x: torch.Tensor, rows: int, top: int, experts: int, hidden: int, ff: int):
-    """(pairs a tile, tiles at most, tile_expert, tile_pairs) for a step of ``rows`` rows."""
+def _expert_tiles(x: torch.Tensor, rows: int, top: int, experts: int, hidden: int, ff: int, copied: bool = False):
+    """(pairs a tile, tiles at most, tile_expert, tile_pairs) for a step of ``rows`` rows.  ``copied``: both matrices have a copy."""
     pairs = rows * top
     # bfloat16 with inner sizes in runs of 8 goes to the matrix cores: the more pairs an expert gets on average, the larger the
     # tiles (its matrices are read once a tile); anything else in tiles of the plain kernel's size.  Both products, matrices from
@@ -2039,8 +2039,17 @@ def _expert_tiles(x: torch.Tensor, rows: int, top: int, experts: int, hidden: in
     if x.dtype == torch.bfloat16 and hidden % 8 == 0 and ff % 8 == 0:
         each = pairs / experts
         fills = experts * -(-hidden // 128) >= compute_units(x.device)
-        few = 14 if not fills else 12 if hidden <= 1024 else 8
-        tile = 128 if each >= 160 and pairs * hidden * ff >= 20e9 else 64 if each >= few else 16
+        if copied and hidden % 64 == 0 and ff % 64 == 0:
+            # From the second copies, us: tiles of 16 and 64: 32 experts of 2,048 x 768, 8 pairs an expert 56 and 59, 11 pairs 59 and 59, 14 pairs 74
+            # and 60; 64 of 2,048 x 1,408, 8 pairs 185 and 203, 11 pairs 206 and 206; 8 of 4,096 x 2,048, 11 pairs 81 and 100, 14 pairs 99 and 101.
+            # Tiles of 64 and 128: 34 of 2,048 x 768, 115 pairs 104 and 108, 130 pairs 127 and 120; 32 of 1,024 x 384, 130 pairs 36 and 39, 160 pairs
+            # 39 and 37; 64 of 2,048 x 1,408, 40 pairs 220 and 228, 60 pairs 249 and 235, 100 pairs 285 and 250; 32 of 4,096 x 1,024, 40 pairs 160 and 161, 50
+            # pairs 189 and 162; 8 of 4,096 x 2,048, 115 pairs 107 and 140, 130 pairs 189 and 142
+            few, many = 10 if fills else 14, 48 if fills and hidden * ff >= 2500000 else 125
+            tile = 128 if each >= many else 64 if each >= few else 16
+        else:
+            few = 14 if not fills else 12 if hidden <= 1024 else 8
+            tile = 128 if each >= 160 and pairs * hidden * ff >= 20e9 else 64 if each >= few else 16
     else:
         tile = library().leone_moe_tile_pairs()
     max_tiles = min(pairs, pairs // tile + experts)
@@ -2049,7 +2058,7 @@ def _expert_tiles(x: torch.Tensor, rows: int, top: int, experts: int, hidden: in
 
 
 def tile_experts(weight: torch.Tensor) -> Optional[torch.Tensor]:
-    """The copy of experts' matrices ``[experts (, 2), rows, K]`` (bfloat16) that the products of few pairs read fastest: rows in tiles
+    """The copy of experts' matrices ``[experts (, 2), rows, K]`` (bfloat16) that their products read fastest: rows in tiles
     of 16, K in steps of 32; element e of lane 16 g + c of step s of a tile is row c's element 32 s + 8 g + e, so that each load of a
     wave is 1 KB in one piece.  None where the sizes have no such form (rows off 16, K off 32)."""
     rows, k = weight.shape[-2:]
@@ -2071,11 +2080,15 @@ def _check_experts(x: torch.Tensor, w_up: torch.Tensor, w_down: torch.Tensor):
     return rows, hidden, experts, ff, gated
 
 
+def _whole(copies: tuple) -> tuple:
+    return (True,) if copies[0] is not None and copies[1] is not None else ()
+
+
 def _expert_copy(tiles: Optional[torch.Tensor], w: torch.Tensor, pairs_a_tile: int) -> Optional[torch.Tensor]:
     """``tiles`` if the product of such tiles of pairs reads the experts' copy (of ``w``, or of more experts that begin with them)."""
-    if tiles is None or pairs_a_tile != 16:
-        return None
     rows, k = w.shape[-2:]
+    if tiles is None or not (pairs_a_tile == 16 or (pairs_a_tile in (64, 128) and k % 64 == 0)):
+        return None
     if tiles.dtype != torch.bfloat16 or tiles.device != w.device or not tiles.is_contiguous() or tiles.shape[0] < w.shape[0] \
             or tuple(tiles.shape[1:]) != (*w.shape[1:-2], rows // 16, k // 32, 4, 16, 8):
         raise KernelError(f"routed experts: a copy {tuple(tiles.shape)} of {tiles.dtype} does not belong to {tuple(w.shape)}")
@@ -2101,7 +2114,7 @@ def _expert_products(x, chosen, weight, tiles, w_up, w_down, activation, extra, 
         copy = _expert_copy(copy, w, tile)
         if copy is not None:
             call("leone_moe_product_tiles", _dev(rows_in, "routed rows", torch.bfloat16), _dev(copy, "experts' tiles"), _dev(out, "experts' results"),
-                 pair_weight, kind, _dev(tile_expert, "tiles"), _dev(tile_pairs, "tile pairs"), max_tiles, experts, top, n, k, code, held, _stream())
+                 pair_weight, kind, _dev(tile_expert, "tiles"), _dev(tile_pairs, "tile pairs"), max_tiles, tile, experts, top, n, k, code, held, _stream())
             return
         call("leone_moe_product", _dev(rows_in, "routed rows"), _dev(w, "experts"), _dev(out, "experts' results"), pair_weight,
              _code(rows_in, "routed rows"), kind, _dev(tile_expert, "tiles"), _dev(tile_pairs, "tile pairs"), max_tiles, tile, experts, top, n, k,
@@ -2123,10 +2136,10 @@ def routed_experts(x: torch.Tensor, chosen: torch.Tensor, weight: torch.Tensor, 
     of ``x``'s type; experts without a gate come as ``[experts, ff, hidden]`` and compute W_down[e] act(W_up[e] x)
     (``PLAIN_ACTIVATIONS``).  ``weigh_input`` (experts without a gate): the weight multiplies what the expert reads
     instead of what it gives.  ``paired``: the sum is left to the consumer (``PairedRows``).  ``copies``: ``tile_experts`` of both
-    matrices (None: none), which products of few pairs read instead.  Nothing here depends on the choice except through device arrays."""
+    matrices (None: none), which the products read instead.  Nothing here depends on the choice except through device arrays."""
     rows, hidden, experts, ff, _ = _check_experts(x, w_gate_up, w_down)
     top = chosen.shape[1]
-    tiles = _expert_tiles(x, rows, top, experts, hidden, ff)
+    tiles = _expert_tiles(x, rows, top, experts, hidden, ff, *_whole(copies))
     call("leone_moe_plan", _dev(chosen, "chosen", torch.int32, (rows, top)), rows * top, experts, _dev(tiles[2], "tiles"),
          _dev(tiles[3], "tile pairs"), tiles[1], tiles[0], _stream())
     return _expert_products(x, chosen, weight, tiles, w_gate_up, w_down, activation, extra, limit, weigh_input, paired, copies)
@@ -2152,7 +2165,7 @@ def routed_feed_forward(x: torch.Tensor, logits: torch.Tensor, correction: Optio
     if not 0 <= always < experts:
         raise KernelError(f"routed_feed_forward: {always} of {experts} experts for every row")
     places = top + always
-    tiles = _expert_tiles(x, rows, places, experts, hidden, ff)
+    tiles = _expert_tiles(x, rows, places, experts, hidden, ff, *_whole(copies))
     chosen = torch.empty((rows, places), dtype=torch.int32, device=x.device)
     weight = torch.empty((rows, places), dtype=torch.float32, device=x.device)
     call("leone_route_plan", _dev(logits, "router logits", torch.float32, (rows, total)),

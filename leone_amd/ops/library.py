@@ -110,7 +110,7 @@ _PROTOTYPES = {
     "leone_route_plan": [P, P, c_int, P, P, c_int, c_int, c_int, c_int, c_int, c_int, P, P, c_int, c_int, c_int, c_int, c_int, c_int,
                          c_float, P],
     "leone_moe_plan": [P, c_int, c_int, P, P, c_int, c_int, P],
-    "leone_moe_product_tiles": [P, P, P, P, c_int, P, P, c_int, c_int, c_int, c_int, c_int, c_int, c_float, P],
+    "leone_moe_product_tiles": [P, P, P, P, c_int, P, P, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, P],
     "leone_moe_product": [P, P, P, P, c_int, c_int, P, P, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, P],
     "leone_moe_one_chunk_ahead": [c_int, c_int, c_int, c_int],
     "leone_moe_combine": [P, P, P, P, c_int, P, P, c_int, c_int, c_int, c_int, P],

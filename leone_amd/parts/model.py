@@ -160,11 +160,11 @@ class DecoderModel:
     def keep_streamed_copies(self, wanted: Optional[bool] = None) -> int:
         """Keeps, beside every matrix that decode steps stream through, a second copy in the order in which
         the weight-streaming kernels read it fastest (``ops.tile_weight``; the row-major one stays for the
-        library's products of prompt portions and for the token table).  The results are the same bit for
+        library's products of prompt portions and for the token table).  The results of these products are the same bit for
         bit; a decode step of few rows takes a sixth less time; the weights take twice the memory.
         ``wanted`` None decides by room: yes if the copies take at most a quarter of the device's memory
         and half of what is free.  Routed experts get theirs (``ops.tile_experts``) behind these, all or none, if there is room for
-        both.  Returns the bytes the copies take (0: none kept).  Asked again, it answers what it did the first time."""
+        both; their products of many pairs then run on a kernel of their own, with sums in its order.  Returns the bytes the copies take (0: none kept).  Asked again, it answers what it did the first time."""
         if self.streamed_copy_bytes is not None:
             return self.streamed_copy_bytes
         self.streamed_copy_bytes = 0

@@ -1,4 +1,5 @@
-"""Experts' products of few pairs from the matrices' second copies: the bits of the products from the matrices themselves."""
+"""Experts' products from the matrices' second copies: of few pairs the bits of the products from the matrices themselves; of many pairs
+against the same sums in 64 bits."""
 import math
 
 import pytest
@@ -21,6 +22,7 @@ def test_the_same_bits(gated, experts, rows, top, hidden, ff):
     up = (torch.randn(experts, *((2,) if gated else ()), ff, hidden, generator=gen) / math.sqrt(hidden)).bfloat16().to(DEV)
     down = (torch.randn(experts, hidden, ff, generator=gen) / math.sqrt(ff)).bfloat16().to(DEV)
     copies = (ops.tile_experts(up), ops.tile_experts(down))
+    assert rows * top < 8 * experts or experts < 8                    # (tiles of 16 pairs whatever the matrices are read from)
     for options in (({}, {"activation": "gelu_tanh"}) if gated else ({"activation": "relu2"}, {"activation": "relu2", "weigh_input": True})):
         want = ops.routed_experts(x, chosen, weight, up, down, **options)
         assert torch.equal(ops.routed_experts(x, chosen, weight, up, down, copies=copies, **options), want)
@@ -64,3 +66,53 @@ def test_a_model_keeps_the_copies_if_there_is_room(monkeypatch, wanted, free, ke
     assert model.keep_streamed_copies(wanted) == (0 if wanted is False else 64 * 64 * 2 + (part.expert_copy_bytes() if kept else 0))
     assert (part.copies[0] is not None) == kept
     ops.drop_streamed_copies()
+
+
+# tiles of 64 and 128 pairs, the last of an expert nearly empty or full, experts without pairs; one stage of the inner size, two, an odd number;
+# rows of a matrix below, at and off what a workgroup takes, few and many workgroups
+@pytest.mark.parametrize("mode", ["gated", "clamped", "plain", "weighed"])
+@pytest.mark.parametrize("experts,rows,top,hidden,ff", [(2, 64, 1, 64, 64), (3, 129, 2, 128, 64), (4, 200, 2, 192, 448), (5, 333, 3, 320, 192),
+                                                        (40, 1300, 4, 704, 1344), (3, 700, 2, 2048, 832)])
+def test_many_pairs(mode, experts, rows, top, hidden, ff):
+    from leone_amd import ops
+    gen = torch.Generator(device=DEV).manual_seed(rows + ff)
+    gated = mode in ("gated", "clamped")
+    # the last expert gets nothing, the one before it hands rows on; the first is everybody's favourite
+    liked = torch.rand(rows, experts, generator=gen, device=DEV)
+    liked[:, 0] += 0.5
+    liked[:, experts - 1] = -1.0
+    chosen = liked.topk(min(top, experts - 1), dim=1).indices.to(torch.int32).contiguous()
+    weight = torch.rand(rows, chosen.shape[1], generator=gen, device=DEV) + 0.1
+    x = torch.randn(rows, hidden, generator=gen, device=DEV).bfloat16()
+    up = (torch.randn(experts, *((2,) if gated else ()), ff, hidden, generator=gen, device=DEV) / math.sqrt(hidden)).bfloat16()
+    down = (torch.randn(experts, hidden, ff, generator=gen, device=DEV) / math.sqrt(ff)).bfloat16()
+    options = {"gated": {}, "clamped": {"activation": "clamped_swish", "limit": 0.8}, "plain": {"activation": "relu2"},
+               "weighed": {"activation": "gelu_tanh", "weigh_input": True}}[mode]
+    copies = (ops.tile_experts(up), ops.tile_experts(down))
+    got = ops.routed_experts(x, chosen, weight, up, down, copies=copies, **options)
+    want = torch.zeros(rows, hidden, dtype=torch.float64, device=DEV)
+    for e in range(experts):
+        row, place = (chosen == e).nonzero(as_tuple=True)
+        if not len(row):
+            continue
+        a, t = weight[row, place].double()[:, None], x[row].double()
+        if gated:
+            g, u = t @ up[e, 0].double().T, t @ up[e, 1].double().T
+            if mode == "clamped":
+                g, u = g.clamp(max=0.8), u.clamp(-0.8, 0.8)
+                h = g * torch.sigmoid(1.702 * g) * (u + 1)
+            else:
+                h = torch.nn.functional.silu(g) * u
+        else:
+            h = t @ up[e].double().T * (a if mode == "weighed" else 1.0)
+            h = torch.relu(h).square() if mode == "plain" else torch.nn.functional.gelu(h, approximate="tanh")
+        out = h.bfloat16().double() @ down[e].double().T
+        want.index_add_(0, row, out if mode == "weighed" else a * out)
+    # the middle is rounded to 8 bits on both sides, now and then to neighbours: 2^-8 of some elements
+    assert float((got - want).norm() / want.norm()) < 2e-3
+    assert torch.equal(ops.routed_experts(x, chosen, weight, up, down, copies=copies, **options), got)
+    # a pair's result does not depend on the pairs beside it (tiles of the same size)
+    some = torch.randperm(rows, generator=torch.Generator().manual_seed(1))[:rows - 3].to(DEV)
+    if ops._expert_tiles(x, rows, chosen.shape[1], experts, hidden, ff, True)[0] == ops._expert_tiles(x, rows - 3, chosen.shape[1], experts, hidden, ff, True)[0]:
+        assert torch.equal(ops.routed_experts(x[some].contiguous(), chosen[some].contiguous(), weight[some].contiguous(), up, down, copies=copies, **options),
+                           got[some])
