@@ -1038,6 +1038,83 @@ def gemm_rows(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype = to
     return None if (residual is not None and splits == 1) else out
 
 
+MANY_TILES = ((64, 128, 2.1, 0.277), (96, 128, 2.6, 0.332), (128, 128, 2.8, 0.40), (96, 256, 3.2, 0.533))
+MANY_LEAST = 1024            # fewest rows and columns of a weight ``gemm_many`` is asked for
+MANY_MOST = 10 << 30         # most products of two elements it is asked for
+
+
+@functools.lru_cache(maxsize=4096)
+def many_plan(m: int, n: int, k: int, may_split: bool, units: int = 256) -> tuple[int, int, int]:
+    """(rows, columns, ranges of K) of a workgroup of ``gemm_many``.  Its time is a start and then, a stage of 64 elements of K, so
+    much for every tile that falls to one compute unit (``MANY_TILES``: rows, columns, us to start, us a stage; fitted to 700 measured
+    products a tile, 129 to 2,048 rows of 1,024 to 4,096 wide layers, standing off by 12 %); planes cost half a microsecond a megabyte,
+    written and read.  What is chosen so is within 1 % of the best of the four tiles and 1 to 4 ranges on average, 22 % at worst; tiles of
+    64 x 256 and 128 x 256 as well would gain less than half a percent."""
+    stages = k // 64
+    best = None
+    for rows, columns, start, stage in MANY_TILES:
+        tiles = -(-m // rows) * -(-n // columns)
+        for splits in range(1, (min(stages, 4) if may_split else 1) + 1):
+            per = -(-stages // splits)
+            if per * (splits - 1) >= stages:            # a range would be empty
+                continue
+            cost = start + stage * per * -(-tiles * splits // units) + (0.48e-6 * 4 * m * n * splits if may_split else 0.0)
+            if best is None or cost < best[0]:
+                best = (cost, rows, columns, splits)
+    return best[1:]
+
+
+def _takes_many(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype, residual: Optional[torch.Tensor],
+                gated: bool, tiles: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
+    """The weight's tiled copy (``tiles`` where it is not kept under the weight itself) if ``gemm_many`` is the faster for this product of many rows; None leaves it to the library.
+
+    The line lies where both were measured, us, library and ``gemm_many``: into the stream 2,048 x 6,144 for 129, 513 and 1,300 rows
+    26 and 15, 30 and 22, 47 and 43; 4,096 x 4,096 for 160, 384, 800 and 1,300 rows 26 and 15, 26 and 23, 46 and 44, 57 and 60; 1,024 x 3,072 for
+    300 and 1,700 rows 14 and 9, 28 and 23; gated 6,144 x 1,024 for 256, 640 and 1,300 rows 18 and 10, 20 and 15, 29 and 25 and 12,288 x 2,048 for 300, 640 and
+    800 rows 27 and 24, 40 and 40, 45 and 53; 3,072 x 2,048 for 192, 640 and 1,700 rows 15 and 9, 19 and 15, 29 and 27; 6,144 x 4,096 for 256, 640 and
+    1,300 rows 30 and 22, 46 and 43, 71 and 88.  Taken together a third faster up to 4 G products of two elements, a seventh at 7 G, a
+    fourteenth at 11 G, level at 16 G, behind beyond.  Products that were tuned, or are being noted for it, stay with the library."""
+    m, (n, k) = x.shape[0], weight.shape
+    if not _streamed or k % 64 or n % 16 or n < MANY_LEAST or k < MANY_LEAST or m * n * k > MANY_MOST or _recorded_products is not None:
+        return None
+    if not x.is_contiguous() or x.data_ptr() % 16 or out_dtype not in _CODES or (gated and (out_dtype != torch.bfloat16 or residual is not None)):
+        return None
+    if residual is not None and (residual.dtype != torch.float32 or residual.shape != (m, n) or not residual.is_contiguous() or residual.data_ptr() % 16):
+        return None
+    if _tuned_products and _library_problem(x, weight, torch.float32 if residual is not None else out_dtype, residual is not None) in _tuned_products:
+        return None
+    return streamed_copy(weight) if tiles is None else tiles
+
+
+def gemm_many(x: torch.Tensor, tiles: torch.Tensor, n: int, out_dtype: torch.dtype = torch.bfloat16, residual: Optional[torch.Tensor] = None,
+              gated: bool = False, plan: Optional[tuple] = None, activation: str = "silu", limit: Optional[float] = None) -> Optional[torch.Tensor]:
+    """x[R,K] . weight[N,K]^T for any number of rows from the weight's tiled copy (``tile_weight``), K a multiple of 64 and N of 16.  With
+    ``residual`` and one range of K the product is added into that float32 tensor (None returned), with more ranges float32 planes come
+    back whose sum, in order, the caller adds; with ``gated`` the weight is an interleaved gate/up weight and act(gate) * up comes out,
+    both rounded to bfloat16 first.  ``plan``: (rows, columns, ranges of K) of a workgroup, by default ``many_plan``'s."""
+    m, k = x.shape
+    if gated and residual is not None:
+        raise KernelError("gemm_many: a gated product cannot also be added into the stream")
+    if tiles.shape != (-(-n // 16), k // 64, 2, 4, 16, 8):
+        raise KernelError(f"gemm_many: a tiled copy of shape {tuple(tiles.shape)} is not one of {n} x {k}")
+    rows, columns, splits = plan or many_plan(m, n, k, residual is not None, compute_units(x.device))
+    mode, code, kind = 0, 0, out_dtype
+    if gated:
+        mode, code, kind = 2, _glu_code(activation, limit), torch.bfloat16
+    elif splits > 1:
+        mode, kind = 3, torch.float32
+    elif residual is not None:
+        mode, kind = 1, torch.float32
+    if mode == 1:
+        out = residual
+        _dev(out, "gemm_many stream", torch.float32, (m, n))
+    else:
+        out = torch.empty((splits, m, n) if mode == 3 else (m, n // 2 if gated else n), dtype=kind, device=x.device)
+    call("leone_gemm_many_bf16", _dev(x, "gemm x", torch.bfloat16, (m, k)), _dev(tiles, "gemm weight", torch.bfloat16), _dev(out, "gemm out", kind),
+         mode, _CODES[kind], m, n, k, splits, m * n, rows, columns, code, float(limit or 0.0), _stream())
+    return None if mode == 1 else out
+
+
 def inner_parts(rows: int, n: int, k: int) -> int:
     """Into how many parts the inner dimension of x[rows, k] . w[n, k]^T is cut when the result goes into the
     float32 stream.  The library's product does badly with a few hundred rows, few columns and a long inner
@@ -1195,7 +1272,8 @@ def linear(x, weight: torch.Tensor, out_dtype: Optional[torch.dtype] = None,
 
     float32 runs the single-precision kernel.  bfloat16 accumulates in float: up to FUSED_ROWS rows on the
     weight-streaming kernel with everything folded in, up to ROWS_MAX rows (a decode step of many requests)
-    on the multi-row weight-streaming kernel, more rows (prompt portions) through the library's matrix
+    on the multi-row weight-streaming kernel, more rows (prompt portions) on the kernel for many rows where the weight has a
+    tiled copy and that kernel is the faster (``_takes_many``), else through the library's matrix
     product, with float32 output for logits and for what goes into the stream.
     """
     dtype = x.dtype if isinstance(x, NormedRows) else x.dtype
@@ -1225,6 +1303,11 @@ def linear(x, weight: torch.Tensor, out_dtype: Optional[torch.dtype] = None,
             and (not gated or weight.shape[0] % 16 == 0):
         return gemm_rows(x, weight, out_dtype, residual, gated, may_split=planes_ok or residual is not None,
                          activation=activation, limit=limit)
+    if dtype == torch.bfloat16 and x.is_cuda and weight.is_cuda and rows > ROWS_MAX:
+        tiles = _takes_many(x, weight, out_dtype, residual, gated)
+        if tiles is not None:
+            with profile.span("gemm many", weight):
+                return gemm_many(x, tiles, weight.shape[0], out_dtype, residual, gated, activation=activation, limit=limit)
     if dtype == torch.float32:
         if out_dtype != torch.float32:
             raise KernelError("linear: the float32 path produces float32")
@@ -1279,6 +1362,13 @@ def linear_planes(x: torch.Tensor, weight: torch.Tensor, rows_of) -> list:
         if x.dtype == torch.bfloat16 and FUSED_ROWS < rows <= ROWS_MAX and k % 8 == 0 and tiles is not None and at % 16 == 0:
             # the whole matrix's second copy is tiles of 16 rows: a part that begins at one has its own piece of it
             results.append(gemm_rows(x[p], part, torch.float32, may_split=False, tiles=tiles[at // 16:-(-(at + r) // 16)]))
+            continue
+        many = None
+        if x.dtype == torch.bfloat16 and rows > ROWS_MAX and tiles is not None and at % 16 == 0:
+            many = _takes_many(x[p], part, torch.float32, None, False, tiles[at // 16:-(-(at + r) // 16)])
+        if many is not None:
+            with profile.span("gemm many", part):
+                results.append(gemm_many(x[p], many, r, torch.float32))
         else:
             results.append(linear(x[p], part, out_dtype=torch.float32))
     return results

@@ -31,6 +31,7 @@ OPERATIONS = {
     "leone_gemm_fused_bf16": "gemv fused",
     "leone_gemm_planes_bf16": "gemv fused",
     "leone_gemm_rows_bf16": "gemm rows",
+    "leone_gemm_many_bf16": "gemm many",
     "leone_gemm_f32": "gemm f32",
     "leone_swiglu": "swiglu",
     "leone_argmax": "argmax",
@@ -97,7 +98,7 @@ OPERATIONS = {
     "leone_add_bias": "bias",
 }
 LIBRARY_PRODUCT = "gemm library"
-ORDER = ["embed", "norm", "gemv fused", "gemm rows", LIBRARY_PRODUCT, "gemm f32", "qknorm rope kv", "attention", "swiglu",
+ORDER = ["embed", "norm", "gemv fused", "gemm rows", "gemm many", LIBRARY_PRODUCT, "gemm f32", "qknorm rope kv", "attention", "swiglu",
          "argmax", "sample"]
 
 
