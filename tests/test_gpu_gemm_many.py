@@ -1,0 +1,84 @@
+"""Products of more rows than the weight-streaming kernels take, from the weight's tiled copy (``gemm_many``): every tile and output at the edges
+of tiles, stages and ranges of K, against 64 bits; and the rule that hands products to it."""
+import pytest
+import torch
+
+from leone_amd import ops
+
+pytestmark = pytest.mark.gpu
+TILES = [plan[:2] for plan in ops.MANY_TILES]
+
+
+def _operands(m, n, k):
+    gen = torch.Generator().manual_seed(m * 7 + n * 3 + k)
+    x = torch.randn((m, k), generator=gen).bfloat16().cuda()
+    weight = (torch.randn((n, k), generator=gen) / k ** 0.5).bfloat16().cuda()
+    want = x.double() @ weight.double().t()
+    # a float sum of k products is off by at most (k + 1) units of 2^-24 of the sum of their sizes (its planes' sum by a few more)
+    bound = (k + 8) * 2.0 ** -24 * (x.double().abs() @ weight.double().abs().t())
+    return x, weight, ops.tile_weight(weight), want, bound
+
+
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("m, n, k, splits", [
+    (1, 16, 64, 1),             # the smallest: one row, half a part, one stage
+    (129, 272, 192, 3),         # one over tiles; one stage a range
+    (191, 1040, 320, 2),        # odd stages, a last range that is shorter
+    (256, 512, 448, 1),         # whole tiles of rows and columns
+    (1153, 2064, 128, 1),       # more than eight rows of tiles
+])
+def test_every_tile_and_output(tile, m, n, k, splits):
+    x, weight, tiles, want, bound = _operands(m, n, k)
+    planes = ops.gemm_many(x, tiles, n, torch.float32, plan=(*tile, splits))
+    assert planes.dtype == torch.float32 and tuple(planes.shape) == ((splits, m, n) if splits > 1 else (m, n))
+    got = (planes.sum(dim=0) if splits > 1 else planes).double()
+    assert ((got - want).abs() <= bound).all()
+    whole = ops.gemm_many(x, tiles, n, torch.float32, plan=(*tile, 1))
+    assert torch.equal(ops.gemm_many(x, tiles, n, plan=(*tile, 1)), whole.bfloat16())
+    stream = torch.randn((m, n), generator=torch.Generator().manual_seed(5)).cuda()
+    added = stream.clone()
+    assert ops.gemm_many(x, tiles, n, residual=added, plan=(*tile, 1)) is None
+    assert torch.equal(added, stream + whole)
+    for activation, limit in (("silu", None), ("gelu_tanh", None), ("clamped_swish", 0.5)):
+        both = ops.gemm_many(x, tiles, n, gated=True, plan=(*tile, 1), activation=activation, limit=limit)
+        assert torch.equal(both, ops.swiglu(whole.bfloat16(), activation=activation, limit=limit))
+
+
+def test_rows_beyond_the_matrices_are_not_written():
+    m, n, k = 130, 144, 128
+    x, weight, tiles, want, bound = _operands(m, n, k)
+    for tile in TILES:
+        held = torch.full((m + 2, n), 7.0, device="cuda")
+        ops.gemm_many(x, tiles, n, residual=held[1:-1], plan=(*tile, 1))
+        assert (held[0] == 7).all() and (held[-1] == 7).all()
+        assert ((held[1:-1].double() - 7 - want).abs() <= bound + 2.0 ** -23 * (want.abs() + 7)).all()
+
+
+@pytest.mark.parametrize("m, n, k", [(129, 1024, 1024), (300, 1040, 4096), (640, 3072, 1088)])
+def test_products_with_a_copy_take_it_and_agree_with_those_without(m, n, k):
+    x, weight, tiles, want, bound = _operands(m, n, k)
+    plain = ops.linear(x, weight, out_dtype=torch.float32)
+    gated = ops.linear(x, weight, gated=True)
+    try:
+        ops.keep_streamed_copy(weight)
+        assert ops._takes_many(x, weight, torch.float32, None, False) is not None
+        assert ((ops.linear(x, weight, out_dtype=torch.float32).double() - want).abs() <= bound).all()
+        assert ((plain.double() - want).abs() <= bound).all()
+        stream = torch.zeros((m, n), device="cuda")
+        left = ops.linear(x, weight, residual=stream)
+        if left is not None:                             # planes for the caller to add
+            assert left.dim() == 3 and left.shape[0] == ops.many_plan(m, n, k, True)[2]
+            stream = left.sum(dim=0)
+        assert ((stream.double() - want).abs() <= bound).all()
+        # gate and up may round to another neighbour where the two sums differ: a unit of bfloat16 of either, and of the result
+        half = ops.linear(x, weight, gated=True).double()
+        assert ((half - gated.double()).abs() <= 2.0 ** -7 * (half.abs() + want.abs().amax() ** 2 * 2 + 1e-6)).all()
+        # what it does not take stays with the library: other layouts, other types, products being noted
+        assert ops._takes_many(x[:, ::2], weight[:, :k // 2], torch.float32, None, False) is None
+        assert ops._takes_many(x, weight, torch.float16, None, False) is None
+        assert ops._takes_many(x, weight, torch.float32, torch.zeros((n, m), device="cuda").t(), False) is None
+        with ops.record_library_products() as seen:
+            ops.linear(x, weight, out_dtype=torch.float32)
+        assert len(seen.problems) == 1
+    finally:
+        ops.drop_streamed_copies()
