@@ -1,15 +1,20 @@
-// Matrix products of more rows than the weight-streaming kernels take: a step's prompt portions, the prompts of a few requests, decode
-// steps of more than 128 requests.  Y[M,N] = X[M,K] . W[N,K]^T for bfloat16 X and the tiled copy of bfloat16 W (see leone_hip.h).
+// Matrix products of many rows: a step's prompt portions, the prompts of a few requests, decode steps of 17 requests and more.  Y[M,N] = X[M,K] . W[N,K]^T for bfloat16 X and the tiled copy of bfloat16 W (see leone_hip.h).
 //
-// A workgroup of four waves takes 32 kMT rows and 128 kNT columns, a wave a quarter of the columns in parts of 32.  The wave's own elements
-// of W come from memory as its instruction (32 x 32 x 16) wants them, one or two stages of 64 elements of K ahead, and pass neither through
-// shared memory nor a barrier.  X, which all four waves read, goes through shared memory, a stage's 128 bytes of a row turned about by the row's
+// A workgroup of four waves (or two) takes 32 kMT rows and 32 kNT columns a wave, in parts of 32.  The wave's own elements
+// of W come from memory as its instruction (32 x 32 x 16) wants them, one to four stages of 64 elements of K ahead, and pass neither through
+// shared memory nor a barrier.  X, which all waves read, goes through shared memory, a stage's 128 bytes of a row turned about by the row's
 // number so that the same piece of 16 rows lies in 16 places; a stage is written while the one before it is worked on.
 //
 // What bounds it: with few tiles the time one takes (0.28 us a stage for 64 x 128, 0.33 for 96 x 128, 0.40 for 128 x 128, 0.53 for 96 x 256,
 // which a second tile on the same unit doubles), so a product with fewer tiles than units is cut along K, into planes, where its caller
 // takes them; with many, the chip's power, where the vendor library with its 256 x 256 tiles is as good or better (6,144 x 4,096 for 2,048 rows: 81
 // us here, 67 there).  ops.many_plan chooses; its comment has both sides' figures.
+//
+// kDeep, for up to 128 rows, which have one row of tiles: the weight is read once, so what bounds it is memory, that is, the bytes that a unit has
+// asked for and not yet got.  Four stages of W are on their way (64 KB of 128 columns, where the kernel of gemm_rows.hip has 32 KB), asked for with
+// the hint that they are read once, and the last four stages ask for nothing; workgroups of two waves take 64 columns where 128 would leave
+// units without work.  4,096 x 12,288 for 64 rows 24.1 us in gemm_rows.hip, 21.8 here two stages ahead, 20.0 four ahead (5.0 TB/s); 4,096 x
+// 4,096 12.3, 10.0 and 9.3; 2,048 x 2,048 6.6, 5.8 and 5.0.  ops.deep_plan chooses.
 #include "common.h"
 
 #include <type_traits>
@@ -20,7 +25,6 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 
 enum ManyOut : int { kManyStore = 0, kManyResidual = 1, kManyGated = 2, kManyPlanes = 3 };
-constexpr int kManyThreads = 256;
 
 struct ManyArgs {
     const bf16_t* x;
@@ -31,12 +35,14 @@ struct ManyArgs {
     float limit;
 };
 
-template <int kMT, int kNT, int kOut, typename TOut>
-__global__ void __launch_bounds__(kManyThreads, kNT == 1 ? 3 : 2)
+template <int kMT, int kNT, int kWaves, bool kDeep, int kOut, typename TOut>
+__global__ void __launch_bounds__(kWaves * kWave, kDeep ? (kMT == 1 || (kMT == 2 && kWaves == 4) ? 3 : 2) : kNT == 1 ? 3 : 2)
 gemm_many_kernel(ManyArgs a) {
-    constexpr int kRows = 32 * kMT, kCopies = kRows * 8 / kManyThreads;
-    constexpr int kWAhead = kNT == 1 ? 2 : 1, kAhead = kMT <= 2 ? 2 : 1;                 // stages of W and of X on their way in registers
-    __shared__ uint4 sx[2][kRows * 8];
+    constexpr int kThreads = kWaves * kWave, kRows = 32 * kMT, kPieces = kRows * 8, kCopies = kPieces / kThreads;
+    static_assert(kPieces % kThreads == 0, "every thread copies as many pieces of X");
+    // stages of W and of X on their way in registers; stages that the loop takes at a time
+    constexpr int kWAhead = kDeep ? 4 : kNT == 1 ? 2 : 1, kAhead = kMT <= 2 ? 2 : 1, kTurns = kDeep ? 4 : 2;
+    __shared__ uint4 sx[2][kPieces > kWaves * 128 ? kPieces : kWaves * 128];
     const int tid = threadIdx.x, lane = tid % kWave, wave = __builtin_amdgcn_readfirstlane(tid / kWave);
     const int c = lane & 31, hi = lane >> 5;
     const int tiles = a.tiles_m * a.tiles_n, total = tiles * a.splits;
@@ -55,14 +61,14 @@ gemm_many_kernel(ManyArgs a) {
 #pragma unroll
     for (int u = 0; u < kNT; ++u) {
         // the lane's row of W (gated: gate and up rows take turns by eights); past the last the last again, not written
-        const int want = ((tn * 4 + wave) * kNT + u) * 2 + (c >> 4), t16 = want < a.n / 16 ? want : a.n / 16 - 1;
+        const int want = ((tn * kWaves + wave) * kNT + u) * 2 + (c >> 4), t16 = want < a.n / 16 ? want : a.n / 16 - 1;
         wp[u] = a.w + (static_cast<long>(t16) * all + s0) * 1024 + hi * 128 + (c & 15) * 8;
     }
     const bf16_t* x_from[kCopies];
     int x_to[kCopies];
 #pragma unroll
     for (int i = 0; i < kCopies; ++i) {
-        const int q = i * kManyThreads + tid, row = q >> 3, part = q & 7;
+        const int q = i * kThreads + tid, row = q >> 3, part = q & 7;
         const int wanted = tm * kRows + row, gr = wanted < a.m ? wanted : a.m - 1;
         x_from[i] = a.x + static_cast<long>(gr) * a.k + s0 * 64 + part * 8;
         x_to[i] = row * 8 + (part ^ ((row >> 1) & 7));
@@ -70,7 +76,9 @@ gemm_many_kernel(ManyArgs a) {
     const auto inside = [&](int s) { return s < count ? s : count - 1; };                // (past the end the last stage again, unused)
     const auto load_x = [&](int s, int i) { return *reinterpret_cast<const uint4*>(x_from[i] + static_cast<long>(inside(s)) * 64); };
     const auto load_w = [&](int s, int j, int u) {
-        return *reinterpret_cast<const uint4*>(wp[u] + static_cast<long>(inside(s)) * 1024 + (j >> 1) * 512 + (j & 1) * 256);
+        const bf16_t* from = wp[u] + static_cast<long>(inside(s)) * 1024 + (j >> 1) * 512 + (j & 1) * 256;
+        if constexpr (kDeep) return load_streamed16(from);
+        else return *reinterpret_cast<const uint4*>(from);
     };
     floatx16 acc[kMT][kNT];
 #pragma unroll
@@ -94,15 +102,15 @@ gemm_many_kernel(ManyArgs a) {
 #pragma unroll
         for (int i = 0; i < kCopies; ++i) first[i] = load_x(0, i);
 #pragma unroll
-        for (int v = 0; v < 2; ++v)
+        for (int v = 0; v < kTurns; ++v)
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
 #pragma unroll
                 for (int i = 0; i < kCopies; ++i)
-                    if (place_of(i) / kMT == j && v >= 2 - kAhead) held[(v + 1 + kAhead) % kAhead][i] = load_x(v - 1 + kAhead, i);
-                if (v >= 2 - kWAhead)
+                    if (place_of(i) / kMT == j && v >= kTurns - kAhead) held[(v + 1 + kAhead) % kAhead][i] = load_x(v + 1 - kTurns + kAhead, i);
+                if (v >= kTurns - kWAhead)
 #pragma unroll
-                    for (int u = 0; u < kNT; ++u) wr[v % kWAhead][j][u] = load_w(v - 2 + kWAhead, j, u);
+                    for (int u = 0; u < kNT; ++u) wr[v % kWAhead][j][u] = load_w(v - kTurns + kWAhead, j, u);
                 __builtin_amdgcn_sched_barrier(0);
             }
 #pragma unroll
@@ -111,8 +119,8 @@ gemm_many_kernel(ManyArgs a) {
     __syncthreads();
 #pragma unroll
     for (int t = 0; t < kMT; ++t) xb[0][t] = read_x(sx[0], 0, t);
-    const auto stage = [&](int s, auto parity) {
-        constexpr int p = decltype(parity)::value;
+    const auto stage = [&](int s, auto number, auto last) {
+        constexpr int at_turn = decltype(number)::value, p = at_turn & 1;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             if (j == 3) {                                // the next stage lies in shared memory, and everyone has read this one
@@ -131,19 +139,40 @@ gemm_many_kernel(ManyArgs a) {
                     }
 #pragma unroll
                 for (int u = 0; u < kNT; ++u)
-                    acc[t][u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, wr[p % kWAhead][j][u]), xb[j & 1][t], acc[t][u], 0, 0, 0);
+                    acc[t][u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, wr[at_turn % kWAhead][j][u]), xb[j & 1][t], acc[t][u], 0, 0, 0);
                 __builtin_amdgcn_sched_barrier(0);
             }
+            if constexpr (!decltype(last)::value)
 #pragma unroll
-            for (int u = 0; u < kNT; ++u) wr[p % kWAhead][j][u] = load_w(s + kWAhead, j, u);
+                for (int u = 0; u < kNT; ++u) wr[at_turn % kWAhead][j][u] = load_w(s + kWAhead, j, u);
         }
     };
     int s = 0;
-    for (; s + 1 < count; s += 2) {
-        stage(s, std::integral_constant<int, 0>{});
-        stage(s + 1, std::integral_constant<int, 1>{});
+    if constexpr (kDeep) {
+        const std::false_type more;
+        const std::true_type last;                       // (of W nothing is asked for any more)
+        for (; s + kTurns < count; s += kTurns) {
+            stage(s, std::integral_constant<int, 0>{}, more);
+            stage(s + 1, std::integral_constant<int, 1>{}, more);
+            stage(s + 2, std::integral_constant<int, 2>{}, more);
+            stage(s + 3, std::integral_constant<int, 3>{}, more);
+        }
+        stage(s, std::integral_constant<int, 0>{}, last);
+        if (s + 1 < count) {
+            stage(s + 1, std::integral_constant<int, 1>{}, last);
+            if (s + 2 < count) {
+                stage(s + 2, std::integral_constant<int, 2>{}, last);
+                if (s + 3 < count) stage(s + 3, std::integral_constant<int, 3>{}, last);
+            }
+        }
+    } else {
+        const std::false_type more;
+        for (; s + 1 < count; s += 2) {
+            stage(s, std::integral_constant<int, 0>{}, more);
+            stage(s + 1, std::integral_constant<int, 1>{}, more);
+        }
+        if (s < count) stage(s, std::integral_constant<int, 0>{}, more);
     }
-    if (s < count) stage(s, std::integral_constant<int, 0>{});
     // Lane (c, hi) holds, of row c of every t, columns 8 q + 4 hi .. + 3 of each of the wave's 32.  They are turned in shared memory, a wave's
     // own part of it, so that a store covers whole runs of a row (straight from the registers it would be 16 bytes of 32 rows).
     __syncthreads();                                     // the last stage has been read
@@ -152,11 +181,11 @@ gemm_many_kernel(ManyArgs a) {
     constexpr int kPart = kGate ? 16 : 32;                           // results of one of the wave's parts
     constexpr int kAtOnce = kBytes == 4 ? 1 : kNT;                   // of these parts
     constexpr int kRun = kPart * kAtOnce * kBytes / 16;              // 16-byte pieces of a row at once
-    static_assert(kRun * 32 * 16 <= sizeof(sx) / 4 && (kRun == 2 || kRun == 4 || kRun == 8), "a wave's part of the stages' memory");
+    static_assert(kRun * 32 * 16 <= sizeof(sx) / kWaves && (kRun == 2 || kRun == 4 || kRun == 8), "a wave's part of the stages' memory");
     uint4* mine = &sx[0][0] + wave * (kRun * 32);
     const auto turn = [](int r) { return (kRun == 8 ? r >> 1 : kRun == 4 ? r >> 2 : r >> 3) & (kRun - 1); };
     const int width = kGate ? a.n / 2 : a.n;
-    const int col0 = (tn * 4 + wave) * kNT * kPart;
+    const int col0 = (tn * kWaves + wave) * kNT * kPart;
     char* out = static_cast<char*>(a.y) + (kOut == kManyPlanes ? split * a.plane * 4 : 0);
 #pragma unroll
     for (int t = 0; t < kMT; ++t)
@@ -179,8 +208,14 @@ gemm_many_kernel(ManyArgs a) {
 #pragma unroll
                     for (int j = 0; j < 4; ++j) {
                         v[j] = acc[t][u][4 * q + j];
-                        if constexpr (kGate)                         // both rounded first, as they are where a kernel of its own does this
-                            v[j] = glu_value(to_float(from_float<bf16_t>(v[j])), to_float(from_float<bf16_t>(acc[t][u][(4 * q + 4 + j) & 15])), a.act, a.limit);
+                        if constexpr (kGate) {
+                            float gate = v[j], up = acc[t][u][(4 * q + 4 + j) & 15];
+                            if constexpr (!kDeep) {                  // both rounded first, as they are where a kernel of its own does this
+                                gate = to_float(from_float<bf16_t>(gate));
+                                up = to_float(from_float<bf16_t>(up));
+                            }
+                            v[j] = glu_value(gate, up, a.act, a.limit);
+                        }
                     }
                     const int first = (u - u0) * kPart + (kGate ? 4 * q : 8 * q) + 4 * hi, piece = (first * kBytes / 16) ^ turn(c);
                     if constexpr (kBytes == 4) {
@@ -212,16 +247,16 @@ gemm_many_kernel(ManyArgs a) {
         }
 }
 
-template <int kMT, int kNT>
+template <int kMT, int kNT, int kWaves, bool kDeep>
 void launch_many(ManyArgs a, int out_mode, int out_dtype, hipStream_t stream) {
     a.tiles_m = ceil_div(a.m, 32 * kMT);
-    a.tiles_n = ceil_div(a.n, 128 * kNT);
-    const int groups = a.tiles_m * a.tiles_n * a.splits;
-    if (out_mode == kManyResidual) gemm_many_kernel<kMT, kNT, kManyResidual, float><<<groups, kManyThreads, 0, stream>>>(a);
-    else if (out_mode == kManyGated) gemm_many_kernel<kMT, kNT, kManyGated, bf16_t><<<groups, kManyThreads, 0, stream>>>(a);
-    else if (out_mode == kManyPlanes) gemm_many_kernel<kMT, kNT, kManyPlanes, float><<<groups, kManyThreads, 0, stream>>>(a);
-    else if (out_dtype == kF32) gemm_many_kernel<kMT, kNT, kManyStore, float><<<groups, kManyThreads, 0, stream>>>(a);
-    else gemm_many_kernel<kMT, kNT, kManyStore, bf16_t><<<groups, kManyThreads, 0, stream>>>(a);
+    a.tiles_n = ceil_div(a.n, 32 * kWaves * kNT);
+    const int groups = a.tiles_m * a.tiles_n * a.splits, threads = kWaves * kWave;
+    if (out_mode == kManyResidual) gemm_many_kernel<kMT, kNT, kWaves, kDeep, kManyResidual, float><<<groups, threads, 0, stream>>>(a);
+    else if (out_mode == kManyGated) gemm_many_kernel<kMT, kNT, kWaves, kDeep, kManyGated, bf16_t><<<groups, threads, 0, stream>>>(a);
+    else if (out_mode == kManyPlanes) gemm_many_kernel<kMT, kNT, kWaves, kDeep, kManyPlanes, float><<<groups, threads, 0, stream>>>(a);
+    else if (out_dtype == kF32) gemm_many_kernel<kMT, kNT, kWaves, kDeep, kManyStore, float><<<groups, threads, 0, stream>>>(a);
+    else gemm_many_kernel<kMT, kNT, kWaves, kDeep, kManyStore, bf16_t><<<groups, threads, 0, stream>>>(a);
 }
 
 }  // namespace leone
@@ -229,7 +264,7 @@ void launch_many(ManyArgs a, int out_mode, int out_dtype, hipStream_t stream) {
 using namespace leone;
 
 extern "C" int leone_gemm_many_bf16(const void* x, const void* w, void* y, int out_mode, int out_dtype, int m, int n, int k, int splits,
-                                    long plane, int tile_rows, int tile_columns, int act, float limit, hipStream_t stream) {
+                                    long plane, int tile_rows, int tile_columns, int deep, int act, float limit, hipStream_t stream) {
     LEONE_REQUIRE(x && w && y, "gemm_many: null pointer");
     LEONE_REQUIRE(m > 0 && n > 0 && k > 0 && n % 16 == 0 && k % 64 == 0, "gemm_many: bad sizes %d x %d x %d", m, n, k);
     LEONE_REQUIRE((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(y)) % 16 == 0,
@@ -243,12 +278,21 @@ extern "C" int leone_gemm_many_bf16(const void* x, const void* w, void* y, int o
     const int per = ceil_div(stages, splits);
     LEONE_REQUIRE(per * (splits - 1) < stages, "gemm_many: %d ranges of K would leave one empty (%d stages)", splits, stages);
     LEONE_REQUIRE(out_mode != kManyPlanes || (plane >= static_cast<long>(m) * n && plane % 4 == 0), "gemm_many: planes overlap");
-    LEONE_REQUIRE(static_cast<long>(ceil_div(m, 64)) * ceil_div(n, 128) * splits < (1l << 30), "gemm_many: %d x %d is too large", m, n);
+    LEONE_REQUIRE(static_cast<long>(ceil_div(m, 32)) * ceil_div(n, 64) * splits < (1l << 30), "gemm_many: %d x %d is too large", m, n);
     const ManyArgs a{static_cast<const bf16_t*>(x), static_cast<const bf16_t*>(w), y, plane, m, n, k, 0, 0, splits, per, act, limit};
-    if (tile_rows == 64 && tile_columns == 128) launch_many<2, 1>(a, out_mode, out_dtype, stream);
-    else if (tile_rows == 96 && tile_columns == 128) launch_many<3, 1>(a, out_mode, out_dtype, stream);
-    else if (tile_rows == 128 && tile_columns == 128) launch_many<4, 1>(a, out_mode, out_dtype, stream);
-    else if (tile_rows == 96 && tile_columns == 256) launch_many<3, 2>(a, out_mode, out_dtype, stream);
+    if (deep) {
+        switch (tile_rows * 1000 + tile_columns) {
+            case 32064: launch_many<1, 1, 2, true>(a, out_mode, out_dtype, stream); break;
+            case 64064: launch_many<2, 1, 2, true>(a, out_mode, out_dtype, stream); break;
+            case 64128: launch_many<2, 1, 4, true>(a, out_mode, out_dtype, stream); break;
+            case 96128: launch_many<3, 1, 4, true>(a, out_mode, out_dtype, stream); break;
+            case 128128: launch_many<4, 1, 4, true>(a, out_mode, out_dtype, stream); break;
+            default: set_error("gemm_many: tiles of %d x %d are not built", tile_rows, tile_columns); return 1;
+        }
+    } else if (tile_rows == 64 && tile_columns == 128) launch_many<2, 1, 4, false>(a, out_mode, out_dtype, stream);
+    else if (tile_rows == 96 && tile_columns == 128) launch_many<3, 1, 4, false>(a, out_mode, out_dtype, stream);
+    else if (tile_rows == 128 && tile_columns == 128) launch_many<4, 1, 4, false>(a, out_mode, out_dtype, stream);
+    else if (tile_rows == 96 && tile_columns == 256) launch_many<3, 2, 4, false>(a, out_mode, out_dtype, stream);
     else {
         set_error("gemm_many: tiles of %d x %d are not built", tile_rows, tile_columns);
         return 1;

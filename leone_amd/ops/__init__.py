@@ -1064,6 +1064,17 @@ def many_plan(m: int, n: int, k: int, may_split: bool, units: int = 256) -> tupl
     return best[1:]
 
 
+def _many_fits(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype, residual: Optional[torch.Tensor], gated: bool) -> bool:
+    """Whether ``gemm_many`` takes these operands, some weight with a tiled copy given."""
+    m, (n, k) = x.shape[0], weight.shape
+    if not _streamed or k % 64 or n % 16 or n < MANY_LEAST or k < MANY_LEAST:
+        return False
+    if not x.is_contiguous() or x.data_ptr() % 16 or out_dtype not in _CODES or (gated and (out_dtype != torch.bfloat16 or residual is not None)):
+        return False
+    return residual is None or (residual.dtype == torch.float32 and residual.shape == (m, n) and residual.is_contiguous()
+                                and residual.data_ptr() % 16 == 0)
+
+
 def _takes_many(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype, residual: Optional[torch.Tensor],
                 gated: bool, tiles: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
     """The weight's tiled copy (``tiles`` where it is not kept under the weight itself) if ``gemm_many`` is the faster for this product of many rows; None leaves it to the library.
@@ -1074,14 +1085,58 @@ def _takes_many(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype, r
     800 rows 27 and 24, 40 and 40, 45 and 53; 3,072 x 2,048 for 192, 640 and 1,700 rows 15 and 9, 19 and 15, 29 and 27; 6,144 x 4,096 for 256, 640 and
     1,300 rows 30 and 22, 46 and 43, 71 and 88.  Taken together a third faster up to 4 G products of two elements, a seventh at 7 G, a
     fourteenth at 11 G, level at 16 G, behind beyond.  Products that were tuned, or are being noted for it, stay with the library."""
-    m, (n, k) = x.shape[0], weight.shape
-    if not _streamed or k % 64 or n % 16 or n < MANY_LEAST or k < MANY_LEAST or m * n * k > MANY_MOST or _recorded_products is not None:
-        return None
-    if not x.is_contiguous() or x.data_ptr() % 16 or out_dtype not in _CODES or (gated and (out_dtype != torch.bfloat16 or residual is not None)):
-        return None
-    if residual is not None and (residual.dtype != torch.float32 or residual.shape != (m, n) or not residual.is_contiguous() or residual.data_ptr() % 16):
+    if x.shape[0] * weight.numel() > MANY_MOST or _recorded_products is not None or not _many_fits(x, weight, out_dtype, residual, gated):
         return None
     if _tuned_products and _library_problem(x, weight, torch.float32 if residual is not None else out_dtype, residual is not None) in _tuned_products:
+        return None
+    return streamed_copy(weight) if tiles is None else tiles
+
+
+# Tiles of ``gemm_many`` that read the weight once, four stages ahead, for up to ROWS_MAX rows: (rows, columns): us to start, us a stage of 64
+# elements of K, TB/s of the weight with every unit at work, us a megabyte of results, what a further workgroup on a unit costs of the first,
+# and how much of a last round's idle units is lost.
+DEEP_TILES = {(32, 64): (2.411, 0.197, 6.777, 0.331, 0.827, 0.637), (64, 64): (2.678, 0.252, 6.785, 0.245, 1.268, 0.545),
+              (64, 128): (2.762, 0.376, 6.775, 0.244, 1.567, 0.411), (96, 128): (3.225, 0.418, 6.516, 0.209, 1.395, 0.673),
+              (128, 128): (3.654, 0.456, 6.025, 0.186, 1.508, 0.666)}
+DEEP_GATED_MOST = 25 << 20   # most elements of a gated weight that they are asked for
+
+
+@functools.lru_cache(maxsize=4096)
+def deep_plan(m: int, n: int, k: int, may_split: bool, gated: bool, units: int = 256) -> tuple[int, int, int, bool]:
+    """(rows, columns, ranges of K, True) of a workgroup of ``gemm_many`` for up to ROWS_MAX rows.  A workgroup's stages and the weight's
+    way from memory overlap: their times are joined as by a fourth power, which was fitted to 6,000 measured products (34 shapes, 17 to 128
+    rows; off by 4 to 8 %).  A plane costs its reader 0.3 us a megabyte.  What is chosen is within 1 % of the best of these tiles on
+    average, 18 % at worst."""
+    stages, best = k // 64, None
+    for (rows, columns), (start, stage, rate, result, further, idle) in DEEP_TILES.items():
+        if rows - m >= 32:
+            continue
+        tiles = -(-m // rows) * -(-n // columns)
+        for splits in range(1, (max(1, min(stages // 3, 16)) if may_split else 1) + 1):
+            per = -(-stages // splits)
+            if per * (splits - 1) >= stages:            # a range would be empty
+                continue
+            groups = tiles * splits
+            rounds = -(-groups // units)
+            work = stage * per * (1 + further * (rounds - 1))
+            memory = 2e-6 * n * k / rate * (units * rounds / groups) ** idle
+            cost = start + (work ** 4 + memory ** 4) ** 0.25 + (result * (1 if gated else 4) + (1.2 if may_split else 0.0)) * 1e-6 * m * n * splits
+            if best is None or cost < best[0]:
+                best = (cost, rows, columns, splits)
+    return (*best[1:], True)
+
+
+def _takes_deep(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype, residual: Optional[torch.Tensor],
+                gated: bool, tiles: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
+    """The weight's tiled copy (``tiles`` where it is not kept under the weight itself) if ``gemm_many`` is the faster for this product of
+    more than FUSED_ROWS and up to ROWS_MAX rows; None leaves it to ``gemm_rows``.
+
+    us, ``gemm_rows`` and ``gemm_many`` with ``deep_plan``, weights from memory, 17, 64 and 128 rows: planes of 6,144 x 4,096 12.4 and 10.7, 16.3 and
+    12.1, 21.5 and 17.4; of 4,096 x 12,288 21.2 and 19.3, 24.4 and 21.3, 32.2 and 24.5; of 2,048 x 2,048 4.9 and 4.2, 6.6 and 5.0, 9.8 and 6.8; logits
+    of 32,768 x 4,096 58 and 46, 54 and 49, 65 and 63; of 32,768 x 1,024 20 and 14, 24 and 15, 27 and 20; gated 12,288 x 2,048 15.1 and 13.6, 17.6 and
+    14.8, 22.7 and 19.0, 6,144 x 1,024 7.8 and 7.2, 10.4 and 9.1, 15.3 and 9.1.  Over the shapes measured planes are 1.28 times as fast (0.94 at the least), logits
+    1.27 (0.99); larger gated weights, whose units are all at work either way, are behind (18,432 x 3,072 25.3 and 27.9, 27.8 and 29.7, 35 and 39)."""
+    if not FUSED_ROWS < x.shape[0] <= ROWS_MAX or (gated and weight.numel() > DEEP_GATED_MOST) or not _many_fits(x, weight, out_dtype, residual, gated):
         return None
     return streamed_copy(weight) if tiles is None else tiles
 
@@ -1091,13 +1146,14 @@ def gemm_many(x: torch.Tensor, tiles: torch.Tensor, n: int, out_dtype: torch.dty
     """x[R,K] . weight[N,K]^T for any number of rows from the weight's tiled copy (``tile_weight``), K a multiple of 64 and N of 16.  With
     ``residual`` and one range of K the product is added into that float32 tensor (None returned), with more ranges float32 planes come
     back whose sum, in order, the caller adds; with ``gated`` the weight is an interleaved gate/up weight and act(gate) * up comes out,
-    both rounded to bfloat16 first.  ``plan``: (rows, columns, ranges of K) of a workgroup, by default ``many_plan``'s."""
+    both rounded to bfloat16 first (not with the deep tiles).  ``plan``: (rows, columns, ranges of K) of a workgroup, by default ``many_plan``'s; with a fourth, True, for
+    the tiles that read the weight once and further ahead (``DEEP_TILES``)."""
     m, k = x.shape
     if gated and residual is not None:
         raise KernelError("gemm_many: a gated product cannot also be added into the stream")
     if tiles.shape != (-(-n // 16), k // 64, 2, 4, 16, 8):
         raise KernelError(f"gemm_many: a tiled copy of shape {tuple(tiles.shape)} is not one of {n} x {k}")
-    rows, columns, splits = plan or many_plan(m, n, k, residual is not None, compute_units(x.device))
+    rows, columns, splits, *deep = plan or many_plan(m, n, k, residual is not None, compute_units(x.device))
     mode, code, kind = 0, 0, out_dtype
     if gated:
         mode, code, kind = 2, _glu_code(activation, limit), torch.bfloat16
@@ -1111,7 +1167,8 @@ def gemm_many(x: torch.Tensor, tiles: torch.Tensor, n: int, out_dtype: torch.dty
     else:
         out = torch.empty((splits, m, n) if mode == 3 else (m, n // 2 if gated else n), dtype=kind, device=x.device)
     call("leone_gemm_many_bf16", _dev(x, "gemm x", torch.bfloat16, (m, k)), _dev(tiles, "gemm weight", torch.bfloat16), _dev(out, "gemm out", kind),
-         mode, _CODES[kind], m, n, k, splits, m * n, rows, columns, code, float(limit or 0.0), _stream())
+         mode, _CODES[kind], m, n, k, splits, m * n, rows, columns, bool(deep and deep[0]), code,
+         float(limit or 0.0), _stream())
     return None if mode == 1 else out
 
 
@@ -1272,7 +1329,7 @@ def linear(x, weight: torch.Tensor, out_dtype: Optional[torch.dtype] = None,
 
     float32 runs the single-precision kernel.  bfloat16 accumulates in float: up to FUSED_ROWS rows on the
     weight-streaming kernel with everything folded in, up to ROWS_MAX rows (a decode step of many requests)
-    on the multi-row weight-streaming kernel, more rows (prompt portions) on the kernel for many rows where the weight has a
+    on the multi-row weight-streaming kernel or from the weight's tiled copy (``_takes_deep``), more rows (prompt portions) on the kernel for many rows where the weight has a
     tiled copy and that kernel is the faster (``_takes_many``), else through the library's matrix
     product, with float32 output for logits and for what goes into the stream.
     """
@@ -1301,8 +1358,13 @@ def linear(x, weight: torch.Tensor, out_dtype: Optional[torch.dtype] = None,
     x = materialize(x)
     if dtype == torch.bfloat16 and weight.is_cuda and k % 8 == 0 and rows <= ROWS_MAX \
             and (not gated or weight.shape[0] % 16 == 0):
-        return gemm_rows(x, weight, out_dtype, residual, gated, may_split=planes_ok or residual is not None,
-                         activation=activation, limit=limit)
+        may_split = planes_ok or residual is not None
+        tiles = _takes_deep(x, weight, out_dtype, residual, gated)
+        if tiles is not None:
+            plan = deep_plan(rows, *weight.shape, may_split and not gated, gated, compute_units(x.device))
+            with profile.span("gemm rows", weight):
+                return gemm_many(x, tiles, weight.shape[0], out_dtype, residual, gated, plan, activation=activation, limit=limit)
+        return gemm_rows(x, weight, out_dtype, residual, gated, may_split=may_split, activation=activation, limit=limit)
     if dtype == torch.bfloat16 and x.is_cuda and weight.is_cuda and rows > ROWS_MAX:
         tiles = _takes_many(x, weight, out_dtype, residual, gated)
         if tiles is not None:
@@ -1361,7 +1423,12 @@ def linear_planes(x: torch.Tensor, weight: torch.Tensor, rows_of) -> list:
         part = weight[at:at + r]
         if x.dtype == torch.bfloat16 and FUSED_ROWS < rows <= ROWS_MAX and k % 8 == 0 and tiles is not None and at % 16 == 0:
             # the whole matrix's second copy is tiles of 16 rows: a part that begins at one has its own piece of it
-            results.append(gemm_rows(x[p], part, torch.float32, may_split=False, tiles=tiles[at // 16:-(-(at + r) // 16)]))
+            own = tiles[at // 16:-(-(at + r) // 16)]
+            if _takes_deep(x[p], part, torch.float32, None, False, own) is not None:
+                with profile.span("gemm rows", part):
+                    results.append(gemm_many(x[p], own, r, torch.float32, plan=deep_plan(rows, r, k, False, False, compute_units(x.device))))
+            else:
+                results.append(gemm_rows(x[p], part, torch.float32, may_split=False, tiles=own))
             continue
         many = None
         if x.dtype == torch.bfloat16 and rows > ROWS_MAX and tiles is not None and at % 16 == 0:

@@ -160,8 +160,8 @@ class DecoderModel:
     def keep_streamed_copies(self, wanted: Optional[bool] = None) -> int:
         """Keeps, beside every matrix that decode steps stream through, a second copy in the order in which
         the weight-streaming kernels read it fastest (``ops.tile_weight``; the row-major one stays for the
-        library's products of prompt portions and for the token table).  The results of these products are the same bit for
-        bit; a decode step of few rows takes a sixth less time; the weights take twice the memory.
+        library's products of prompt portions and for the token table).  The results of products of up to 16 rows
+        are the same bit for bit (of more, sums may be in another order); a decode step of few rows takes a sixth less time; the weights take twice the memory.
         ``wanted`` None decides by room: yes if the copies take at most a quarter of the device's memory
         and half of what is free.  Routed experts get theirs (``ops.tile_experts``) behind these, all or none, if there is room for
         both; their products of many pairs then run on a kernel of their own, with sums in its order.  Returns the bytes the copies take (0: none kept).  Asked again, it answers what it did the first time."""

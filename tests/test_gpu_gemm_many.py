@@ -82,3 +82,58 @@ def test_products_with_a_copy_take_it_and_agree_with_those_without(m, n, k):
         assert len(seen.problems) == 1
     finally:
         ops.drop_streamed_copies()
+
+
+@pytest.mark.parametrize("tile", list(ops.DEEP_TILES))
+@pytest.mark.parametrize("m, n, k, splits", [
+    (1, 16, 64, 1),             # the smallest: one row, half a part, one stage of the four that are asked for ahead
+    (17, 80, 256, 1),           # one turn of four stages, and no second
+    (32, 144, 320, 1),          # a turn and one stage
+    (33, 1040, 704, 2),         # ranges of six stages and five
+    (64, 512, 960, 3),          # ranges of five stages
+    (65, 272, 1984, 4),         # ranges of eight stages, the last of seven; a second row of the smaller tiles
+    (128, 256, 512, 1),         # whole tiles, whole turns
+])
+def test_every_deep_tile_and_output(tile, m, n, k, splits):
+    x, weight, tiles, want, bound = _operands(m, n, k)
+    planes = ops.gemm_many(x, tiles, n, torch.float32, plan=(*tile, splits, True))
+    got = (planes.sum(dim=0) if splits > 1 else planes).double()
+    assert ((got - want).abs() <= bound).all()
+    whole = ops.gemm_many(x, tiles, n, torch.float32, plan=(*tile, 1, True))
+    assert torch.equal(whole, ops.gemm_many(x, tiles, n, torch.float32, plan=(64, 128, 1)))       # the same sums as the other tiles
+    assert torch.equal(ops.gemm_many(x, tiles, n, plan=(*tile, 1, True)), whole.bfloat16())
+    stream = torch.randn((m, n), generator=torch.Generator().manual_seed(5)).cuda()
+    added = stream.clone()
+    assert ops.gemm_many(x, tiles, n, residual=added, plan=(*tile, 1, True)) is None
+    assert torch.equal(added, stream + whole)
+    gate, up = (p.reshape(m, n // 2).double() for p in whole.view(m, n // 16, 2, 8).unbind(2))
+    both = ops.gemm_many(x, tiles, n, gated=True, plan=(*tile, 1, True)).double()
+    exact = torch.nn.functional.silu(gate) * up              # of the float sums: rounded once, at the end
+    assert ((both - exact).abs() <= 2.0 ** -8 * exact.abs() * 1.01 + 1e-30).all()
+
+
+@pytest.mark.parametrize("m, n, k", [(17, 1024, 1024), (64, 1040, 3072), (100, 3072, 1088), (128, 1024, 2048)])
+def test_products_of_up_to_128_rows_take_the_copy(m, n, k):
+    x, weight, tiles, want, bound = _operands(m, n, k)
+    plain, gated = ops.linear(x, weight, out_dtype=torch.float32), ops.linear(x, weight, gated=True).double()
+    assert ops._takes_deep(x, weight, torch.float32, None, False) is None                  # there is none yet
+    try:
+        ops.keep_streamed_copy(weight)
+        assert ops._takes_deep(x, weight, torch.float32, None, False) is not None
+        for got in (plain, ops.linear(x, weight, out_dtype=torch.float32)):
+            assert ((got.double() - want).abs() <= bound).all()
+        for stream in (torch.zeros((m, n), device="cuda"), None):
+            left = ops.linear(x, weight, torch.float32, residual=stream, planes_ok=True)
+            got = stream if left is None else left.sum(dim=0) if left.dim() == 3 else left
+            assert left is None or left.dim() == 2 or left.shape[0] == ops.deep_plan(m, n, k, True, False)[2]
+            assert ((got.double() - want).abs() <= bound).all()
+        # the results of both round once, from sums that differ by their bounds at the most
+        both = ops.linear(x, weight, gated=True).double()
+        assert ((both - gated).abs() <= 2.0 ** -7 * both.abs() + 4 * bound.amax() * (1 + want.abs().amax())).all()
+        assert ops._takes_deep(x[:, ::2], weight[:, :k // 2], torch.float32, None, False) is None
+        assert ops._takes_deep(x[:16], weight, torch.float32, None, False) is None
+        assert ops._takes_deep(x, weight, torch.float32, torch.zeros((n, m), device="cuda").t(), False) is None
+        pieces = ops.linear_planes(torch.stack([x, x]), weight, [512, n - 512])
+        assert ((torch.cat(pieces, 1).double() - want).abs() <= bound).all()
+    finally:
+        ops.drop_streamed_copies()
