@@ -1,6 +1,6 @@
 // Matrix products of many rows: a step's prompt portions, the prompts of a few requests, decode steps of 17 requests and more.  Y[M,N] = X[M,K] . W[N,K]^T for bfloat16 X and the tiled copy of bfloat16 W (see leone_hip.h).
 //
-// A workgroup of four waves (or two) takes 32 kMT rows and 32 kNT columns a wave, in parts of 32.  The wave's own elements
+// A workgroup of four waves (or two, or three) takes 32 kMT rows and 32 kNT columns a wave, in parts of 32.  The wave's own elements
 // of W come from memory as its instruction (32 x 32 x 16) wants them, one to four stages of 64 elements of K ahead, and pass neither through
 // shared memory nor a barrier.  X, which all waves read, goes through shared memory, a stage's 128 bytes of a row turned about by the row's
 // number so that the same piece of 16 rows lies in 16 places; a stage is written while the one before it is worked on.
@@ -12,8 +12,8 @@
 //
 // kDeep, for up to 128 rows, which have one row of tiles: the weight is read once, so what bounds it is memory, that is, the bytes that a unit has
 // asked for and not yet got.  Four stages of W are on their way (64 KB of 128 columns, where the kernel of gemm_rows.hip has 32 KB), asked for with
-// the hint that they are read once, and the last four stages ask for nothing; workgroups of two waves take 64 columns where 128 would leave
-// units without work.  4,096 x 12,288 for 64 rows 24.1 us in gemm_rows.hip, 21.8 here two stages ahead, 20.0 four ahead (5.0 TB/s); 4,096 x
+// the hint that they are read once, and the last four stages ask for nothing; workgroups of two or three waves take 64 or 96 columns where 128
+// would leave units without work (gated 24,576 x 4,096 for 64 rows, 256 groups of 96: 37.3 us, 39.1 with 192 of 128, 40.3 in gemm_rows.hip).  4,096 x 12,288 for 64 rows 24.1 us in gemm_rows.hip, 21.8 here two stages ahead, 20.0 four ahead (5.0 TB/s); 4,096 x
 // 4,096 12.3, 10.0 and 9.3; 2,048 x 2,048 6.6, 5.8 and 5.0.  ops.deep_plan chooses.
 #include "common.h"
 
@@ -38,8 +38,7 @@ struct ManyArgs {
 template <int kMT, int kNT, int kWaves, bool kDeep, int kOut, typename TOut>
 __global__ void __launch_bounds__(kWaves * kWave, kDeep ? (kMT == 1 || (kMT == 2 && kWaves == 4) ? 3 : 2) : kNT == 1 ? 3 : 2)
 gemm_many_kernel(ManyArgs a) {
-    constexpr int kThreads = kWaves * kWave, kRows = 32 * kMT, kPieces = kRows * 8, kCopies = kPieces / kThreads;
-    static_assert(kPieces % kThreads == 0, "every thread copies as many pieces of X");
+    constexpr int kThreads = kWaves * kWave, kRows = 32 * kMT, kPieces = kRows * 8, kCopies = (kPieces + kThreads - 1) / kThreads;
     // stages of W and of X on their way in registers; stages that the loop takes at a time
     constexpr int kWAhead = kDeep ? 4 : kNT == 1 ? 2 : 1, kAhead = kMT <= 2 ? 2 : 1, kTurns = kDeep ? 4 : 2;
     __shared__ uint4 sx[2][kPieces > kWaves * 128 ? kPieces : kWaves * 128];
@@ -68,7 +67,7 @@ gemm_many_kernel(ManyArgs a) {
     int x_to[kCopies];
 #pragma unroll
     for (int i = 0; i < kCopies; ++i) {
-        const int q = i * kThreads + tid, row = q >> 3, part = q & 7;
+        const int q = (i * kThreads + tid) % kPieces, row = q >> 3, part = q & 7;         // (past the last piece one again: the same bytes)
         const int wanted = tm * kRows + row, gr = wanted < a.m ? wanted : a.m - 1;
         x_from[i] = a.x + static_cast<long>(gr) * a.k + s0 * 64 + part * 8;
         x_to[i] = row * 8 + (part ^ ((row >> 1) & 7));
@@ -284,6 +283,8 @@ extern "C" int leone_gemm_many_bf16(const void* x, const void* w, void* y, int o
         switch (tile_rows * 1000 + tile_columns) {
             case 32064: launch_many<1, 1, 2, true>(a, out_mode, out_dtype, stream); break;
             case 64064: launch_many<2, 1, 2, true>(a, out_mode, out_dtype, stream); break;
+            case 32096: launch_many<1, 1, 3, true>(a, out_mode, out_dtype, stream); break;
+            case 64096: launch_many<2, 1, 3, true>(a, out_mode, out_dtype, stream); break;
             case 64128: launch_many<2, 1, 4, true>(a, out_mode, out_dtype, stream); break;
             case 96128: launch_many<3, 1, 4, true>(a, out_mode, out_dtype, stream); break;
             case 128128: launch_many<4, 1, 4, true>(a, out_mode, out_dtype, stream); break;

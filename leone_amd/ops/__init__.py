@@ -1095,10 +1095,11 @@ def _takes_many(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype, r
 # Tiles of ``gemm_many`` that read the weight once, four stages ahead, for up to ROWS_MAX rows: (rows, columns): us to start, us a stage of 64
 # elements of K, TB/s of the weight with every unit at work, us a megabyte of results, what a further workgroup on a unit costs of the first,
 # and how much of a last round's idle units is lost.
-DEEP_TILES = {(32, 64): (2.411, 0.197, 6.777, 0.331, 0.827, 0.637), (64, 64): (2.678, 0.252, 6.785, 0.245, 1.268, 0.545),
+DEEP_TILES = {(32, 64): (2.411, 0.197, 6.777, 0.331, 0.827, 0.637), (32, 96): (2.518, 0.233, 7.219, 0.295, 1.699, 0.561),
+              (64, 64): (2.678, 0.252, 6.785, 0.245, 1.268, 0.545), (64, 96): (2.740, 0.276, 6.927, 0.288, 1.470, 0.620),
               (64, 128): (2.762, 0.376, 6.775, 0.244, 1.567, 0.411), (96, 128): (3.225, 0.418, 6.516, 0.209, 1.395, 0.673),
               (128, 128): (3.654, 0.456, 6.025, 0.186, 1.508, 0.666)}
-DEEP_GATED_MOST = 25 << 20   # most elements of a gated weight that they are asked for
+DEEP_GATED_MOST = 25 << 20   # most elements of a gated weight that they are asked for with more than 64 rows
 
 
 @functools.lru_cache(maxsize=4096)
@@ -1109,7 +1110,7 @@ def deep_plan(m: int, n: int, k: int, may_split: bool, gated: bool, units: int =
     average, 18 % at worst."""
     stages, best = k // 64, None
     for (rows, columns), (start, stage, rate, result, further, idle) in DEEP_TILES.items():
-        if rows - m >= 32:
+        if rows - m >= 32 or (rows < m and (rows, columns) not in ((64, 64), (64, 128))):      # (two rows of tiles: only these were measured)
             continue
         tiles = -(-m // rows) * -(-n // columns)
         for splits in range(1, (max(1, min(stages // 3, 16)) if may_split else 1) + 1):
@@ -1134,9 +1135,10 @@ def _takes_deep(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype, r
     us, ``gemm_rows`` and ``gemm_many`` with ``deep_plan``, weights from memory, 17, 64 and 128 rows: planes of 6,144 x 4,096 12.4 and 10.7, 16.3 and
     12.1, 21.5 and 17.4; of 4,096 x 12,288 21.2 and 19.3, 24.4 and 21.3, 32.2 and 24.5; of 2,048 x 2,048 4.9 and 4.2, 6.6 and 5.0, 9.8 and 6.8; logits
     of 32,768 x 4,096 58 and 46, 54 and 49, 65 and 63; of 32,768 x 1,024 20 and 14, 24 and 15, 27 and 20; gated 12,288 x 2,048 15.1 and 13.6, 17.6 and
-    14.8, 22.7 and 19.0, 6,144 x 1,024 7.8 and 7.2, 10.4 and 9.1, 15.3 and 9.1.  Over the shapes measured planes are 1.28 times as fast (0.94 at the least), logits
-    1.27 (0.99); larger gated weights, whose units are all at work either way, are behind (18,432 x 3,072 25.3 and 27.9, 27.8 and 29.7, 35 and 39)."""
-    if not FUSED_ROWS < x.shape[0] <= ROWS_MAX or (gated and weight.numel() > DEEP_GATED_MOST) or not _many_fits(x, weight, out_dtype, residual, gated):
+    14.8, 22.7 and 19.0, 6,144 x 1,024 7.8 and 7.2, 10.4 and 9.1, 15.3 and 9.1, 24,576 x 4,096 39.3 and 36.6, 40.3 and 37.3.  Over the shapes measured planes are
+    1.28 times as fast (0.94 at the least), logits 1.27 (0.99), gated products of up to 64 rows 1.06 (0.97); of more rows the larger gated weights,
+    whose units are all at work either way, are behind (24,576 x 4,096 for 96 and 128 rows 44 and 45, 48 and 49, 18,432 x 3,072 30 and 34, 35 and 39)."""
+    if not FUSED_ROWS < x.shape[0] <= ROWS_MAX or (gated and x.shape[0] > 64 and weight.numel() > DEEP_GATED_MOST) or not _many_fits(x, weight, out_dtype, residual, gated):
         return None
     return streamed_copy(weight) if tiles is None else tiles
 
