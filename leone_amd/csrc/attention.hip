@@ -265,14 +265,16 @@ extern "C" int leone_attention_rows_biased(const void* q, void* out, const void*
 
 // The same with what score_shape.h describes: cap (0: none), sinks, and the tables that turn results back (null: none);
 // chunk > 0 (no window, no kept first keys): a row sees the keys of its own chunk of so many positions only.
-extern "C" int leone_attention_rows_shaped(const void* q, void* out, const void* k_pool, const void* v_pool, int dtype,
-                                           const int* positions, const int* row_entry, const int* block_table,
-                                           int max_blocks, int rows, int q_heads, int kv_heads, int head_dim, int v_dim,
-                                           int page_tokens, float scale, int window, const float* gate, long gate_stride,
-                                           int keep_first, int gate_each, const float* slopes, float temp_coef,
-                                           int temp_every, float cap, const float* sinks, const float* turn_cos,
-                                           const float* turn_sin, int turn_positions, int turn_pairing, int chunk,
-                                           hipStream_t stream) {
+// part_acc, part_ml (may be null; see attention_f32.h): room for the shares' results where few rows of float32 heads of 64 or 128 elements are cut
+// into shares; everything else ignores it.
+extern "C" int leone_attention_rows_parts(const void* q, void* out, const void* k_pool, const void* v_pool, int dtype,
+                                          const int* positions, const int* row_entry, const int* block_table,
+                                          int max_blocks, int rows, int q_heads, int kv_heads, int head_dim, int v_dim,
+                                          int page_tokens, float scale, int window, const float* gate, long gate_stride,
+                                          int keep_first, int gate_each, const float* slopes, float temp_coef,
+                                          int temp_every, float cap, const float* sinks, const float* turn_cos,
+                                          const float* turn_sin, int turn_positions, int turn_pairing, int chunk,
+                                          float* part_acc, float* part_ml, hipStream_t stream) {
     if (check_mask("attention_rows", window, chunk, keep_first)) return 1;
     const ScoreShape shape{cap, sinks, turn_cos, turn_sin, turn_positions, turn_pairing};
     if (check_score_shape("attention_rows", shape, v_dim)) return 1;
@@ -295,7 +297,7 @@ extern "C" int leone_attention_rows_shaped(const void* q, void* out, const void*
         launch_attention_f32(static_cast<const float*>(q), static_cast<float*>(out), static_cast<const float*>(k_pool),
                              static_cast<const float*>(v_pool), positions, row_entry, block_table, max_blocks, rows, q_heads, kv_heads,
                              head_dim, page_tokens, scale, window, gate, gate_stride, keep_first, gate_each, slopes, temp_coef,
-                             temp_every, shape, chunk, stream);
+                             temp_every, shape, chunk, part_acc, part_ml, stream);
         LEONE_LAUNCH_CHECK("attention_rows");
         return 0;
     }
@@ -315,6 +317,20 @@ extern "C" int leone_attention_rows_shaped(const void* q, void* out, const void*
 }
 
 // talk [q_heads, q_heads] of talk_dtype: the heads' scores are mixed by it before the softmax.
+extern "C" int leone_attention_rows_shaped(const void* q, void* out, const void* k_pool, const void* v_pool, int dtype,
+                                           const int* positions, const int* row_entry, const int* block_table,
+                                           int max_blocks, int rows, int q_heads, int kv_heads, int head_dim, int v_dim,
+                                           int page_tokens, float scale, int window, const float* gate, long gate_stride,
+                                           int keep_first, int gate_each, const float* slopes, float temp_coef,
+                                           int temp_every, float cap, const float* sinks, const float* turn_cos,
+                                           const float* turn_sin, int turn_positions, int turn_pairing, int chunk,
+                                           hipStream_t stream) {
+    return leone_attention_rows_parts(q, out, k_pool, v_pool, dtype, positions, row_entry, block_table, max_blocks, rows,
+                                      q_heads, kv_heads, head_dim, v_dim, page_tokens, scale, window, gate, gate_stride,
+                                      keep_first, gate_each, slopes, temp_coef, temp_every, cap, sinks, turn_cos, turn_sin, turn_positions,
+                                      turn_pairing, chunk, nullptr, nullptr, stream);
+}
+
 extern "C" int leone_attention_rows_talk(const void* q, void* out, const void* k_pool, const void* v_pool, int dtype,
                                          const void* talk, int talk_dtype, const int* positions, const int* row_entry,
                                          const int* block_table, int max_blocks, int rows, int q_heads, int kv_heads,

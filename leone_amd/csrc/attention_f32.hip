@@ -20,7 +20,8 @@
 // needs neither masks nor a look for values that are no numbers: of the instructions between the products, which the other wave of a
 // SIMD has to cover, that is a third.
 //
-// Measured (us; with those, the row kernel of attention.hip): 16 heads over 4 of 128 elements, one row at 780 keys 23.5 (24.9, 314), a prompt
+// Measured (us; with those, the row kernel of attention.hip): 16 heads over 4 of 128 elements, one row at 780 keys 23.5 (24.9, 314; 15.1 with a
+// workgroup a share, below), a prompt
 // of 777 rows 64 (71, 1375), of 2,048 rows 260 (292, 8589).
 #include "common.h"
 #include "leone_hip.h"
@@ -58,6 +59,43 @@ struct AttentionF32Args {
     ScoreShape shape;
     int chunk;
 };
+
+// The end of a row: its query's sums over the denominator, turned back, behind their gate.  Lane l of a wave has elements h .. h + 3, h = 4 (l /
+// 16), of the kCount runs of 16 from `first` on, kStep runs apart (a run's partner for turning is kCount / 2 further).
+template <int kDim, int kCount, int kStep>
+__device__ inline void finish_row(const AttentionF32Args& g, f32x4 (&result)[kCount], int first, float denom, int row, int head, int pos,
+                                  int lane, bool real) {
+    static_assert(kCount * kStep * 16 == kDim, "the runs are every kStep-th of the head's");
+    const int h = (lane / 16) * 4;
+#pragma unroll
+    for (int i = 0; i < kCount; ++i) result[i] /= denom;
+    if (g.shape.turn_cos) {
+        f32x4 turned[kCount];
+#pragma unroll
+        for (int i = 0; i < kCount; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float partner = g.shape.turn_pairing ? result[i][r ^ 1] : result[(i + kCount / 2) % kCount][r];
+                turned[i][r] = turned_back(result[i][r], partner, (first + i * kStep) * 16 + h + r, kDim, pos, g.shape);
+            }
+#pragma unroll
+        for (int i = 0; i < kCount; ++i) result[i] = turned[i];
+    }
+    if (!real) return;
+    float* orow = g.out + (static_cast<long>(row) * g.q_heads + head) * kDim;
+    const float* gate_row = g.gate ? g.gate + static_cast<long>(row) * g.gate_stride + (g.gate_each ? static_cast<long>(head) * kDim : head) : nullptr;
+    const float open_head = (g.gate && !g.gate_each) ? 1.0f / (1.0f + expf(-gate_row[0])) : 1.0f;
+#pragma unroll
+    for (int i = 0; i < kCount; ++i) {
+        const int at = (first + i * kStep) * 16 + h;
+        f32x4 open = {open_head, open_head, open_head, open_head};
+        if (g.gate && g.gate_each) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) open[r] = 1.0f / (1.0f + expf(-gate_row[at + r]));
+        }
+        *reinterpret_cast<f32x4*>(orow + at) = result[i] * open;
+    }
+}
 
 // kWaves waves with kShares / kWaves shares each.
 template <int kDim, int kWaves>
@@ -299,34 +337,274 @@ __global__ void __launch_bounds__(kWaves * kWave, kDim == 64 ? 3 : 2) attention_
         }
     }
     if (wave != 0) return;
-    // lane l: its query's elements 16 i + h .. + 3
+    finish_row<kDim, kRuns, 1>(g, result, 0, denom, row, head, pos, lane, real);
+}
+
+// ---- few rows: a workgroup a share -----------------------------------------------------------------------------------------
+//
+// With a workgroup a row and kv head a step of one request uses as many units as there are kv heads.  Here every share of a row's keys has a
+// workgroup of its own, and what bounds it are the instructions of its waves, each alone on its SIMD (some five cycles apiece): so its four
+// waves take four tiles at a time, make the scores of one each, tell each other the tiles' highest scores, weigh their own tile, and then add up
+// the values of all four, a quarter of the runs each.  (All four waves on one tile, a quarter of each product apiece, repeated the softmax in
+// every wave: 18.7 us where this takes 15.1.)  16 heads over 4 of 128 elements, one row at 300, 780 and 4,000 keys, both launches: 10.5, 15.1 and
+// 42 us; with a workgroup a row and kv head 13.2, 23.5 and 88.  Sums, shares and the order in which they are merged are attention_f32_kernel's: the results are the same bits.
+constexpr int kPartWaves = 4;
+
+// Waits for what this wave has put into shared memory and read from it, not for its loads from memory.
+__device__ inline void shares_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+template <int kDim>
+__global__ void __launch_bounds__(kPartWaves * kWave) attention_f32_share_kernel(const AttentionF32Args g, float* part_acc, float* part_ml) {
+    constexpr int kRuns = kDim / 16, kOwnRuns = kRuns / kPartWaves;
+    __shared__ float sm_top[kPartWaves][kQueries], sm_alpha[kPartWaves][kQueries], sm_sum[kPartWaves][kQueries];
+    __shared__ f32x4 sm_s[kPartWaves][kWave];
+    const int own = blockIdx.x, row = blockIdx.y, kvh = blockIdx.z, group = g.group;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
+    const int mine = lane % 16, h = (lane / 16) * 4;
+    const int entry = g.row_entry[row], pos = g.positions[row];
+    const int head = kvh * group + (mine < group ? mine : group - 1);
+    f32x4 q[kRuns];
+    {
+        const float* qr = g.q + (static_cast<long>(row) * g.q_heads + head) * kDim + h;
 #pragma unroll
-    for (int i = 0; i < kRuns; ++i) result[i] /= denom;
-    if (g.shape.turn_cos) {
-        f32x4 turned[kRuns];
+        for (int i = 0; i < kRuns; ++i) q[i] = *reinterpret_cast<const f32x4*>(qr + i * 16);
+    }
+    float scale = g.scale;
+    if (g.temp_every > 0) scale *= 1.0f + g.temp_coef * logf(static_cast<float>((pos + 1) / g.temp_every + 1));
+    const float slope = g.slopes ? g.slopes[head] : 0.f;
+    const int first = first_key(pos, g.window, g.chunk);
+    const int low_tile = first / kKeys, kept_tiles = min((g.keep_first + kKeys - 1) / kKeys, low_tile), tiles = pos / kKeys + 1;
+    // the share's tiles, numbered: first those of the kept keys, then those from the first that the row sees
+    const int kept = own < kept_tiles ? (kept_tiles - own + kShares - 1) / kShares : 0;
+    const int base = own >= low_tile ? own : own + (low_tile - own + kShares - 1) / kShares * kShares;
+    const int count = kept + (base < tiles ? (tiles - base + kShares - 1) / kShares : 0);
+    const auto start_of = [&](int n) { return (n < kept ? own + kShares * n : base + kShares * (n - kept)) * kKeys; };
+
+    f32x4 acc[kOwnRuns] = {};
+    float m = -INFINITY, l = 0.f;
+    if (count > 0) {
+        const int* table = g.block_table + static_cast<long>(entry) * g.max_blocks;
+        const long page_floats = static_cast<long>(g.page_tokens) * kDim, run_step = 2l * g.page_tokens * 8;
+        const auto page_of = [&](int key) { return g.page_shift >= 0 ? key >> g.page_shift : key / g.page_tokens; };
+        const int key_lane = (h / 8) * g.page_tokens * 8 + mine * 8 + h % 8, value_lane = ((h / 8) * kDim + mine) * 8 + h % 8 + wave * kOwnRuns * 128;
+        f32x4 kf[kRuns], vf[kPartWaves][kOwnRuns];
+        // four tiles: their starts, their pages' places, whether they have one (past the last tile that one again, unused)
+        struct Four {
+            int start[kPartWaves], in_page[kPartWaves];
+            long block[kPartWaves];
+            bool mapped[kPartWaves];
+        };
+        int pages = 0;                                        // of 64 tiles, a lane each
+        const auto four_from = [&](int n0) {
+            if (n0 % kWave == 0) {
+                pages = table[page_of(start_of(min(n0 + lane, count - 1)))];
+                asm volatile("" : "+v"(pages));               // waited for here: behind a join, every load in flight would be waited for
+            }
+            Four f;
 #pragma unroll
-        for (int i = 0; i < kRuns; ++i)
+            for (int t = 0; t < kPartWaves; ++t) {
+                const int n = min(n0 + t, count - 1), page = __builtin_amdgcn_readlane(pages, n % kWave);
+                f.start[t] = start_of(n);
+                f.in_page[t] = f.start[t] - page_of(f.start[t]) * g.page_tokens;
+                f.mapped[t] = page >= 0;
+                f.block[t] = (static_cast<long>(page >= 0 ? page : 0) * g.kv_heads + kvh) * page_floats;
+            }
+            return f;
+        };
+        const auto pick = [&](const auto& of) { return wave == 0 ? of[0] : wave == 1 ? of[1] : wave == 2 ? of[2] : of[3]; };
+        const auto fetch_keys = [&](const Four& f) {
+            const float* at = g.k_pool + pick(f.block) + pick(f.in_page) * 8 + key_lane;
+#pragma unroll
+            for (int i = 0; i < kRuns; ++i) kf[i] = *reinterpret_cast<const f32x4*>(at + i * run_step);
+        };
+        const auto fetch_values = [&](const Four& f) {
+#pragma unroll
+            for (int t = 0; t < kPartWaves; ++t) {
+                const float* at = g.v_pool + f.block[t] + static_cast<long>(f.in_page[t]) * kDim + value_lane;
+#pragma unroll
+                for (int i = 0; i < kOwnRuns; ++i) vf[t][i] = *reinterpret_cast<const f32x4*>(at + i * 128);
+            }
+        };
+        Four four = four_from(0);
+        fetch_keys(four);
+        fetch_values(four);
+        for (int n0 = 0; n0 < count; n0 += kPartWaves) {
+            const int here = min(count - n0, kPartWaves);
+            f32x4 dots[4] = {};
+#pragma unroll
+            for (int i = 0; i < kRuns; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) dots[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[i][j], q[i][j], dots[j], 0, 0, 0);
+            f32x4 s = (dots[0] + dots[1]) + (dots[2] + dots[3]);
+            const bool more = n0 + kPartWaves < count;
+            Four next = four;
+            if (more) {
+                next = four_from(n0 + kPartWaves);
+                fetch_keys(next);
+            }
+            const int start = pick(four.start);
+            const bool there = pick(four.mapped);
+            const auto whole_at = [&](int at, bool is) { return is && at + kKeys - 1 <= pos && (at >= first || at + kKeys <= g.keep_first); };
+            const bool whole = whole_at(start, there);
+            float top = -INFINITY;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const float partner = g.shape.turn_pairing ? result[i][r ^ 1] : result[(i + kRuns / 2) % kRuns][r];
-                turned[i][r] = turned_back(result[i][r], partner, i * 16 + h + r, kDim, pos, g.shape);
+                float v = s[r] * scale;
+                if (g.shape.cap > 0.f) v = g.shape.cap * tanhf(v / g.shape.cap);
+                if (g.slopes) v -= slope * static_cast<float>(pos - (start + h + r));
+                s[r] = v;
+            }
+            if (!whole) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int key = start + h + r;
+                    const bool seen = key <= pos && (key >= first || key < g.keep_first);
+                    s[r] = seen ? (there ? s[r] : __builtin_nanf("")) : -INFINITY;
+                }
             }
 #pragma unroll
-        for (int i = 0; i < kRuns; ++i) result[i] = turned[i];
-    }
-    if (!real) return;
-    float* orow = g.out + (static_cast<long>(row) * g.q_heads + head) * kDim;
-    const float* gate_row = g.gate ? g.gate + static_cast<long>(row) * g.gate_stride + (g.gate_each ? static_cast<long>(head) * kDim : head) : nullptr;
-    const float open_head = (g.gate && !g.gate_each) ? 1.0f / (1.0f + expf(-gate_row[0])) : 1.0f;
+            for (int r = 0; r < 4; ++r) top = fmaxf(top, s[r]);
+            top = max_lanes<16>(top);
+            top = max_lanes<32>(top);
+            if (lane < kQueries) sm_top[wave][lane] = top;
+            shares_barrier();
+            // the running maximum through the four tiles; this wave's tile is weighed by what it has come to there
+            float m_before = m, m_own = m;
 #pragma unroll
-    for (int i = 0; i < kRuns; ++i) {
-        f32x4 open = {open_head, open_head, open_head, open_head};
-        if (g.gate && g.gate_each) {
+            for (int t = 0; t < kPartWaves; ++t) {
+                if (t == wave) m_before = m;
+                if (t < here) m = fmaxf(m, sm_top[t][mine]);
+                if (t == wave) m_own = m;
+            }
+            const float reference = m_own == -INFINITY ? 0.f : m_own;      // nothing seen yet: every weight is 0
+            const float alpha = expf(m_before - reference);
+            float sum = 0.f;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) open[r] = 1.0f / (1.0f + expf(-gate_row[i * 16 + h + r]));
+            for (int r = 0; r < 4; ++r) {
+                s[r] = expf(s[r] - reference);
+                sum += s[r];
+            }
+            sum = add_lanes<16>(sum);
+            sum = add_lanes<32>(sum);
+            sm_s[wave][lane] = s;
+            if (lane < kQueries) {
+                sm_alpha[wave][lane] = alpha;
+                sm_sum[wave][lane] = sum;
+            }
+            shares_barrier();
+#pragma unroll
+            for (int t = 0; t < kPartWaves; ++t) {
+                if (t >= here) break;
+                const float alpha_t = sm_alpha[t][mine];
+                const f32x4 s_t = sm_s[t][lane];
+                l = l * alpha_t + sm_sum[t][mine];
+                f32x4 (&v)[kOwnRuns] = vf[t];
+                const int at = four.start[t];
+                const bool whole_t = whole_at(at, four.mapped[t]);
+                bool odd_value = false;
+                if (!whole_t) {
+                    if (!four.mapped[t] || at + kKeys > pos + 1) {         // places nobody has written
+#pragma unroll
+                        for (int i = 0; i < kOwnRuns; ++i)
+#pragma unroll
+                            for (int r = 0; r < 4; ++r)
+                                if (!four.mapped[t] || at + h + r > pos) v[i][r] = 0.f;
+                    }
+                    f32x4 odd = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int i = 0; i < kOwnRuns; ++i) odd += v[i] * 0.f;
+                    odd_value = __any(!(odd[0] + odd[1] + odd[2] + odd[3] == 0.f));
+                }
+#pragma unroll
+                for (int i = 0; i < kOwnRuns; ++i) acc[i] *= alpha_t;
+                if (odd_value) {                              // not a number where the row does not see it: see above
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+#pragma unroll 1
+                        for (int from = 0; from < 4; ++from) {
+                            const int key = at + 4 * from + j;
+                            const bool seen = key <= pos && (key >= first || key < g.keep_first);
+                            const float p = __shfl(s_t[j], from * 16 + mine, kWave);
+#pragma unroll
+                            for (int i = 0; i < kOwnRuns; ++i)
+#pragma unroll
+                                for (int r = 0; r < 4; ++r) {
+                                    const float each = __shfl(v[i][j], from * 16 + h + r, kWave);
+                                    if (seen) acc[i][r] = fmaf(p, each, acc[i][r]);
+                                }
+                        }
+                } else {
+#pragma unroll
+                    for (int i = 0; i < kOwnRuns; ++i)
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[i][j], s_t[j], acc[i], 0, 0, 0);
+                }
+            }
+            if (more) fetch_values(next);
+            four = next;
         }
-        *reinterpret_cast<f32x4*>(orow + i * 16 + h) = result[i] * open;
     }
+    const long place = (static_cast<long>(row) * g.kv_heads + kvh) * kShares + own;
+    if (wave == 0 && lane < kQueries) {
+        part_ml[(place * 2) * kQueries + lane] = m;
+        part_ml[(place * 2 + 1) * kQueries + lane] = l;
+    }
+#pragma unroll
+    for (int i = 0; i < kOwnRuns; ++i)
+        reinterpret_cast<f32x4*>(part_acc)[(place * kRuns + wave * kOwnRuns + i) * kWave + lane] = acc[i];
+}
+
+// The shares' results of a row and kv head, merged as attention_f32_kernel merges them; wave w takes runs w and w + half of them.
+template <int kDim>
+__global__ void __launch_bounds__(kDim / 32 * kWave) attention_f32_join_kernel(const AttentionF32Args g, const float* part_acc, const float* part_ml) {
+    constexpr int kRuns = kDim / 16;
+    const int row = blockIdx.x, kvh = blockIdx.y, group = g.group;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave, mine = lane % 16;
+    const int head = kvh * group + (mine < group ? mine : group - 1);
+    const long place = (static_cast<long>(row) * g.kv_heads + kvh) * kShares;
+    f32x4 acc[kShares][2];
+    float ms[kShares], ls[kShares];
+#pragma unroll
+    for (int w = 0; w < kShares; ++w) {
+        ms[w] = part_ml[((place + w) * 2) * kQueries + mine];
+        ls[w] = part_ml[((place + w) * 2 + 1) * kQueries + mine];
+    }
+#pragma unroll
+    for (int w = 0; w < kShares; ++w)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+            acc[w][i] = reinterpret_cast<const f32x4*>(part_acc)[((place + w) * kRuns + wave + i * (kRuns / 2)) * kWave + lane];
+    const int pos = g.positions[row];
+    float top = ms[0];
+#pragma unroll
+    for (int w = 1; w < kShares; ++w) top = fmaxf(top, ms[w]);
+    const float sink = g.shape.sinks ? g.shape.sinks[head] : -INFINITY;
+    top = fmaxf(top, sink);
+    const auto weight = [&](float of) { return of == -INFINITY ? 0.f : expf(of - top); };
+    float denom = g.shape.sinks ? expf(sink - top) : 0.f;
+    float weights[kShares];
+#pragma unroll
+    for (int w = 0; w < kShares; ++w) {
+        weights[w] = weight(ms[w]);
+        denom += ls[w] * weights[w];
+    }
+    {
+#pragma clang fp contract(off)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+#pragma unroll
+            for (int w = 0; w < kShares; ++w) acc[w][i] = acc[w][i] * weights[w];
+#pragma unroll
+            for (int half = kShares / 2; half > 0; half /= 2)
+#pragma unroll
+                for (int w = 0; w < half; ++w) acc[w][i] = acc[w][i] + acc[w + half][i];
+        }
+    }
+    finish_row<kDim, 2, kRuns / 2>(g, acc[0], wave, denom, row, head, pos, lane, mine < group);
 }
 
 // Whether the kernel takes this shape: 16-byte rows of q and of the results follow from the head's size, tiles of 16 keys lie
@@ -341,7 +619,8 @@ bool attention_f32_takes(const void* q, const void* out, const void* k_pool, con
 void launch_attention_f32(const float* q, float* out, const float* k_pool, const float* v_pool, const int* positions, const int* row_entry,
                           const int* block_table, int max_blocks, int rows, int q_heads, int kv_heads, int head_dim, int page_tokens,
                           float scale, int window, const float* gate, long gate_stride, int keep_first, int gate_each,
-                          const float* slopes, float temp_coef, int temp_every, const ScoreShape& shape, int chunk, hipStream_t stream) {
+                          const float* slopes, float temp_coef, int temp_every, const ScoreShape& shape, int chunk, float* part_acc,
+                          float* part_ml, hipStream_t stream) {
     const int group = q_heads / kv_heads, most = kQueries / group;
     const long multiples = ceil_div(rows, most);
     const int page_shift = (page_tokens & (page_tokens - 1)) == 0 ? __builtin_ctz(page_tokens) : -1;
@@ -349,6 +628,17 @@ void launch_attention_f32(const float* q, float* out, const float* k_pool, const
                                 group, most, multiples > 1 && multiples * (rows + kQueries) < 1l << 32 ? static_cast<unsigned>(((1ull << 32) + multiples - 1) / multiples) : 0u,
                                 page_tokens, page_shift, scale, window, gate, gate_stride, keep_first, gate_each, slopes, temp_coef, temp_every,
                                 shape, chunk};
+    if (part_acc && part_ml && rows <= 65535) {
+        const dim3 shares(kShares, rows, kv_heads), joined(rows, kv_heads);
+        if (head_dim == 128) {
+            attention_f32_share_kernel<128><<<shares, kPartWaves * kWave, 0, stream>>>(args, part_acc, part_ml);
+            attention_f32_join_kernel<128><<<joined, 4 * kWave, 0, stream>>>(args, part_acc, part_ml);
+        } else {
+            attention_f32_share_kernel<64><<<shares, kPartWaves * kWave, 0, stream>>>(args, part_acc, part_ml);
+            attention_f32_join_kernel<64><<<joined, 2 * kWave, 0, stream>>>(args, part_acc, part_ml);
+        }
+        return;
+    }
     const dim3 grid(ceil_div(rows, most) * most, kv_heads);
     // Eight waves, a share each, where the launch is small or heads are of 128 elements; four waves with two shares each for many
     // rows of 64, whose workgroups are short (us, eight waves and four: 8 heads over 2, 1,500 rows 66 and 58, 300 decoded rows at 500

@@ -448,6 +448,13 @@ int leone_attention_rows_shaped(const void* q, void* out, const void* k_pool, co
                                 long gate_stride, int keep_first, int gate_each, const float* slopes, float temp_coef,
                                 int temp_every, float cap, const float* sinks, const float* turn_cos, const float* turn_sin,
                                 int turn_positions, int turn_pairing, int chunk, hipStream_t stream);
+// leone_attention_rows_shaped with room for the results of shares of the keys (attention_f32.h says how much; may be null).
+int leone_attention_rows_parts(const void* q, void* out, const void* k_pool, const void* v_pool, int dtype, const int* positions,
+                                const int* row_entry, const int* block_table, int max_blocks, int rows, int q_heads, int kv_heads,
+                                int head_dim, int v_dim, int page_tokens, float scale, int window, const float* gate,
+                                long gate_stride, int keep_first, int gate_each, const float* slopes, float temp_coef,
+                                int temp_every, float cap, const float* sinks, const float* turn_cos, const float* turn_sin,
+                                int turn_positions, int turn_pairing, int chunk, float* part_acc, float* part_ml, hipStream_t stream);
 int leone_attention_decode_shaped(const void* q, void* out, const void* k_pool, const void* v_pool, const int* positions,
                                   const int* row_entry, const int* block_table, int max_blocks, float* part_acc, float* part_ml,
                                   int rows, int q_heads, int kv_heads, int head_dim, int page_tokens, float scale, int window,

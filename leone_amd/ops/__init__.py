@@ -347,11 +347,27 @@ def _strided_rows(t: Optional[torch.Tensor], what: str, rows: int, columns: int,
     return t.data_ptr(), t.stride(0)
 
 
+def f32_attention_shares(rows: int, kv_heads: int, head_dim: int, keys: int) -> bool:
+    """Whether float32 attention of few rows gets a workgroup for every share of a row's keys and a second launch that merges them.
+
+    Two launches cost two microseconds more, so the row's walk along its keys has to be long; and with as many workgroups as the chip
+    holds anyway there is nothing to gain.  us, in one launch and in two, heads of 128: 4 rows times kv heads at 128, 200, 780 and 1,500 keys 9.1 and 9.6, 12.1 and
+    10.1, 23.8 and 14.9, 38.4 and 20.5; 16 at the same 9.2 and 10.3, 12.4 and 11.1, 24.4 and 16.3, 39.6 and 21.6; 32 at 200, 300 and 780 keys 12.5 and 12.3, 13.8 and
+    13.1, 24.8 and 19.0; 64 at 780 and 1,500 keys 28 and 28, 46 and 39; 128 at 4,000 keys 121 and 158.  Heads of 64: 8 at 300, 500 and 780 keys 8.8 and 9.1, 11.4 and
+    9.7, 15.0 and 12.7; 32 at 500 and 780 keys 11.8 and 11.7, 15.2 and 14.7.  ``keys`` may be up to twice what the rows see (a recorded
+    step's range)."""
+    units = rows * kv_heads
+    if head_dim == 128:
+        return units <= 64 and keys > (128 if units <= 16 else 256 if units <= 32 else 1024)
+    return units <= 32 and keys > (256 if units <= 8 else 512)
+
+
 def attention_rows(q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor, positions: torch.Tensor,
                    row_entry: torch.Tensor, block_table: torch.Tensor, q_heads: int, scale: float,
                    window: int = 0, out: Optional[torch.Tensor] = None, gate: Optional[torch.Tensor] = None,
                    keep_first: int = 0, gate_each: bool = False, slopes: Optional[torch.Tensor] = None,
-                   query_factor: Optional[tuple] = None, shape: Optional[ScoreShape] = None, chunk: int = 0) -> torch.Tensor:
+                   query_factor: Optional[tuple] = None, shape: Optional[ScoreShape] = None, chunk: int = 0,
+                   max_context: int = 0, shares: Optional[bool] = None) -> torch.Tensor:
     """Each query row attends its request's cached keys up to its own position (the last ``window`` of them,
     and, whatever the window, those at positions below ``keep_first``).  The result has the values'
     size a head.  ``slopes`` float32 ``[q_heads]``: head h's score for the key at distance d is lowered by
@@ -360,7 +376,8 @@ def attention_rows(q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor, 
     heads): head h of row r is multiplied by sigmoid(gate[r, h]); with ``gate_each`` the gate holds a value for
     every element of the result, ``[rows, >= q_heads * value_dim]``.  ``shape``: capped scores, sinks, results turned
     back (``ScoreShape``; results are turned back before the gate).  ``chunk`` (without a window): a row sees the keys of its
-    own chunk of so many positions, counted from 0, only."""
+    own chunk of so many positions, counted from 0, only.  ``max_context`` (0: not known) is about how many keys the rows see; it, or
+    ``shares``, decides whether few float32 rows get a workgroup for every share of their keys; the results are the same bits."""
     rows = q.shape[0]
     pages, kv_heads, page_tokens, head_dim, value_dim = cache_dims_kv(k_pool, v_pool)
     if q.shape[1] != q_heads * head_dim:
@@ -369,13 +386,18 @@ def attention_rows(q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor, 
         out = torch.empty((rows, q_heads * value_dim), dtype=q.dtype, device=q.device)
     gate_at, gate_stride = _strided_rows(gate, "attention gate", rows, q_heads * value_dim if gate_each else q_heads)
     coef, every = query_factor if query_factor is not None else (0.0, 0)
-    call("leone_attention_rows_shaped", _dev(q, "attention q"), _dev(out, "attention out", q.dtype, (rows, q_heads * value_dim)),
+    part_acc = part_ml = None
+    if q.dtype == torch.float32 and head_dim == value_dim and head_dim in (64, 128) \
+            and (f32_attention_shares(rows, kv_heads, head_dim, min(max_context, window or max_context, chunk or max_context)) if shares is None else shares):
+        part_acc = torch.empty((rows * kv_heads * 8 * 16 * head_dim,), dtype=torch.float32, device=q.device)
+        part_ml = torch.empty((rows * kv_heads * 8 * 2 * 16,), dtype=torch.float32, device=q.device)
+    call("leone_attention_rows_parts", _dev(q, "attention q"), _dev(out, "attention out", q.dtype, (rows, q_heads * value_dim)),
          _dev(k_pool, "k pool", q.dtype), _dev(v_pool, "v pool", q.dtype), _code(q, "attention q"),
          _dev(positions, "positions", torch.int32, (rows,)), _dev(row_entry, "row map", torch.int32, (rows,)),
          _dev(block_table, "block table", torch.int32), block_table.shape[1], rows, q_heads, kv_heads, head_dim,
          value_dim, page_tokens, float(scale), int(window), gate_at, gate_stride, int(keep_first),
          1 if (gate_each and gate is not None) else 0, _dev(slopes, "slopes", torch.float32, (q_heads,)), float(coef),
-         int(every), *(shape or _PLAIN_SCORES).args(q_heads, value_dim), int(chunk), _stream())
+         int(every), *(shape or _PLAIN_SCORES).args(q_heads, value_dim), int(chunk), _dev(part_acc, "shares"), _dev(part_ml, "shares' sums"), _stream())
     return out
 
 

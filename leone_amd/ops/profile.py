@@ -58,7 +58,7 @@ OPERATIONS = {
     "leone_attention_rows_kept": "attention",
     "leone_attention_decode_kept": "attention",
     "leone_attention_prefill_kept": "attention",
-    "leone_attention_rows_shaped": "attention",
+    "leone_attention_rows_parts": "attention",
     "leone_attention_decode_shaped": "attention",
     "leone_attention_prefill_shaped": "attention",
     "leone_attention_rows_talk": "attention",

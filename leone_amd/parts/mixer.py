@@ -344,7 +344,7 @@ class GqaAttention(Part):
             return ops.attention_rows(q, cache.k_pool, cache.v_pool, step.positions, step.row_entry,
                                       cache.block_table, self.q_heads, self.scale, window, gate=gate,
                                       keep_first=self.keep_first, gate_each=self.gate_each, slopes=self.slopes,
-                                      query_factor=self.query_factor, shape=shape, chunk=self.chunk)
+                                      query_factor=self.query_factor, shape=shape, chunk=self.chunk, max_context=step.max_position + 1)
         first = 0
         out = torch.empty_like(q)
         tiled = step.tiled.get(self.row_tiling())
