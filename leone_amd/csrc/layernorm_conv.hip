@@ -692,11 +692,23 @@ __global__ void causal_conv_state_kernel(const TIn* __restrict__ in, long in_str
     for (int j = 0; j < taps - 1; ++j) mine[static_cast<long>(j) * channels] = keep[j];
 }
 
+// Where the new running maximum of exponential gates made in a step of single rows (outer_step) goes: row r's is top's, in the state of the
+// slot that the r-th span writes.
+struct KeepTop {
+    float* state;                // the first slot's first maximum; null: nowhere
+    long slot_stride, head_stride;
+    const int* spans;            // [rows, 4]
+};
+__device__ inline void keep_top(const KeepTop& keep, int row, int head, float value) {
+    const int slot = keep.spans[4 * row + 3];
+    if (slot >= 0) keep.state[slot * keep.slot_stride + head * keep.head_stride] = value;
+}
+
 // One wave per (row, head).
 template <typename TOut, int kKept>
 __global__ void head_norm_gate_kernel(const float* __restrict__ o, const float* __restrict__ dot, const float* __restrict__ top,
                                       AnyVec gain, int gain_per_head, const float* __restrict__ gate, long gate_stride,
-                                      int act, float eps, TOut* __restrict__ out, int heads, int vdim, int gate_first) {
+                                      int act, float eps, TOut* __restrict__ out, int heads, int vdim, int gate_first, KeepTop keep) {
     const int row = blockIdx.x;
     const int head = blockIdx.y * (blockDim.x / kWave) + threadIdx.x / kWave;
     const int lane = threadIdx.x % kWave;
@@ -729,6 +741,7 @@ __global__ void head_norm_gate_kernel(const float* __restrict__ o, const float* 
     }
     float under = 1.f;
     if (dot) under = fmaxf(fabsf(read), expf(-highest)) + 1e-6f;
+    if (keep.state && lane == 0) keep_top(keep, row, head, highest);
     // with gate_first the gate multiplies ahead of the norm, and the root mean square is that of the gated values
     auto opened = [&](float v, float g) {
         v /= under;
@@ -768,10 +781,11 @@ template <typename TOut, int kThreads>
 __global__ void __launch_bounds__(kThreads)
 head_norm_gate_wide_kernel(const float* __restrict__ o, const float* __restrict__ dot, const float* __restrict__ top, AnyVec gain,
                            int gain_per_head, const float* __restrict__ gate, long gate_stride, int act, float eps,
-                           TOut* __restrict__ out, int heads, int vdim, int gate_first) {
+                           TOut* __restrict__ out, int heads, int vdim, int gate_first, KeepTop keep) {
     __shared__ float scratch[kThreads / kWave];
     const int row = blockIdx.x, head = blockIdx.y;
     const long at = static_cast<long>(row) * heads + head;
+    if (keep.state && threadIdx.x == 0) keep_top(keep, row, head, top[at]);
     const float* src = o + at * vdim;
     const float under = dot ? fmaxf(fabsf(dot[at]), expf(-top[at])) + 1e-6f : 1.f;
     const float* gate_row = gate ? gate + static_cast<long>(row) * gate_stride + static_cast<long>(head) * vdim : nullptr;
@@ -1059,11 +1073,15 @@ extern "C" int leone_head_norm_gate(const float* o, const float* dot, const floa
                                         out_dtype, rows, heads, vdim, stream);
 }
 
+// keep_state (may be null): see KeepTop.
 // gate_first: the gate multiplies ahead of the norm (the root mean square is taken of the gated values) instead of behind it.
-extern "C" int leone_head_norm_gate_ordered(const float* o, const float* dot, const float* top, const void* gain, int gain_dtype,
-                                            int gain_per_head, const float* gate, long gate_stride, int act, int gate_first,
-                                            float eps, void* out, int out_dtype, int rows, int heads, int vdim,
-                                            hipStream_t stream) {
+extern "C" int leone_head_norm_gate_kept(const float* o, const float* dot, const float* top, const void* gain, int gain_dtype,
+                                         int gain_per_head, const float* gate, long gate_stride, int act, int gate_first,
+                                         float eps, void* out, int out_dtype, int rows, int heads, int vdim,
+                                         float* keep_state, long keep_slot_stride, long keep_head_stride,
+                                         const int* keep_spans, hipStream_t stream) {
+    LEONE_REQUIRE(!keep_state || (top && keep_spans), "head_norm_gate: a maximum that is kept needs its value and the rows' slots");
+    const KeepTop keep{keep_state, keep_slot_stride, keep_head_stride, keep_spans};
     LEONE_REQUIRE(o && out && rows > 0 && heads > 0 && vdim > 0, "head_norm_gate: needs read-outs and positive sizes");
     LEONE_REQUIRE(known(out_dtype) && (!gain || known(gain_dtype)), "head_norm_gate: unknown element type");
     LEONE_REQUIRE((dot == nullptr) == (top == nullptr), "head_norm_gate: the denominator's two parts come together");
@@ -1074,7 +1092,7 @@ extern "C" int leone_head_norm_gate_ordered(const float* o, const float* dot, co
         LEONE_REQUIRE(heads <= 65535, "head_norm_gate: too many heads");
 #define LEONE_WIDE_HEAD(T, THREADS)                                                                                           \
     head_norm_gate_wide_kernel<T, THREADS><<<dim3(rows, heads), THREADS, 0, stream>>>(o, dot, top, vg, gain_per_head, gate, gate_stride, \
-                                                                                    act, eps, static_cast<T*>(out), heads, vdim, gate_first)
+                                                                                    act, eps, static_cast<T*>(out), heads, vdim, gate_first, keep)
         // few rows: a row in as few trips to memory as threads allow; many rows: more rows in flight a compute unit
         if (out_dtype == kF32) {
             if (rows >= kNormManyRows) LEONE_WIDE_HEAD(float, kNormThreadsMany);
@@ -1092,7 +1110,7 @@ extern "C" int leone_head_norm_gate_ordered(const float* o, const float* dot, co
     // 64, eight and one: 26.8 and 19.6; 16 of 128, eight and two: 17.9 and 14.1).
 #define LEONE_HEAD(T, KEPT)                                                                                                    \
     head_norm_gate_kernel<T, KEPT><<<grid, 4 * kWave, 0, stream>>>(o, dot, top, vg, gain_per_head, gate, gate_stride, act, eps, \
-                                                                   static_cast<T*>(out), heads, vdim, gate_first)
+                                                                   static_cast<T*>(out), heads, vdim, gate_first, keep)
 #define LEONE_HEAD_KEPT(T) (vdim <= kWave ? LEONE_HEAD(T, 1) : vdim <= 2 * kWave ? LEONE_HEAD(T, 2) : LEONE_HEAD(T, 8))
     if (out_dtype == kF32) LEONE_HEAD_KEPT(float);
     else LEONE_HEAD_KEPT(bf16_t);
@@ -1100,6 +1118,14 @@ extern "C" int leone_head_norm_gate_ordered(const float* o, const float* dot, co
 #undef LEONE_HEAD
     LEONE_LAUNCH_CHECK("head_norm_gate");
     return 0;
+}
+
+extern "C" int leone_head_norm_gate_ordered(const float* o, const float* dot, const float* top, const void* gain, int gain_dtype,
+                                            int gain_per_head, const float* gate, long gate_stride, int act, int gate_first,
+                                            float eps, void* out, int out_dtype, int rows, int heads, int vdim,
+                                            hipStream_t stream) {
+    return leone_head_norm_gate_kept(o, dot, top, gain, gain_dtype, gain_per_head, gate, gate_stride, act, gate_first, eps, out, out_dtype,
+                                     rows, heads, vdim, nullptr, 0, 0, nullptr, stream);
 }
 
 extern "C" int leone_rms_mix(const float* const* branch_rows, const void* const* gains, int gain_dtype, int branches,

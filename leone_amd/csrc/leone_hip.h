@@ -266,6 +266,11 @@ int leone_causal_conv_biased(const void* in, int in_dtype, long in_stride, void*
 int leone_head_norm_gate_ordered(const float* o, const float* dot, const float* top, const void* gain, int gain_dtype,
                                  int gain_per_head, const float* gate, long gate_stride, int act, int gate_first, float eps,
                                  void* out, int out_dtype, int rows, int heads, int vdim, hipStream_t stream);
+// The same; with keep_state row r's top goes into the state of the slot in the fourth place of keep_spans[r].
+int leone_head_norm_gate_kept(const float* o, const float* dot, const float* top, const void* gain, int gain_dtype,
+                                 int gain_per_head, const float* gate, long gate_stride, int act, int gate_first, float eps,
+                                 void* out, int out_dtype, int rows, int heads, int vdim, float* keep_state, long keep_slot_stride,
+                             long keep_head_stride, const int* keep_spans, hipStream_t stream);
 // out = sum over branches of weights[b] * branch (host floats; n elements each), nothing normed.
 int leone_weighted_mix(const float* const* branch_rows, const float* weights, int branches, float* out, long n,
                        hipStream_t stream);
@@ -298,6 +303,12 @@ int leone_outer_step(const float* proj, long stride, int q_off, int k_off, int v
                      const int* segments, int n_segments, const float* state_in, long in_stride, float* state_out,
                      long out_stride, long head_stride, float* out, float* dot, int heads, int dim, int vdim,
                      hipStream_t stream);
+// The same with a normaliser and exponential gates made in the launch: top gets the rows' maxima, the state keeps its own.
+int leone_outer_step_gated(const float* proj, long stride, int q_off, int k_off, int v_off, int i_off, int f_off, const void* i_bias,
+                           const void* f_bias, int bias_dtype, float cap, long top_at, float* top, float q_scale, float k_scale, int silu,
+                           const float* cos_table, const float* sin_table, int rotary_dim, int table_positions, const int* positions,
+                           const int* segments, int n_segments, const float* state_in, long in_stride, float* state_out, long out_stride,
+                           long head_stride, float* out, float* dot, int heads, int dim, int vdim, hipStream_t stream);
 int leone_delta_scan(const float* qkv, long stride, int q_off, int k_off, int v_off, const float* beta,
                      long beta_stride, const float* step, long step_stride, int per_head, const void* rate_log,
                      const void* step_bias, int vec_dtype, float q_scale, float unit_eps, int no_input, int accumulate,

@@ -66,6 +66,12 @@ struct OuterScanArgs {
     float* out;                 // [rows, heads, vdim]
     float* dot;                 // [rows, heads]
     int heads, dim, vdim;
+    // outer_step alone, instead of coef: the gates are made where they are used (null: they are not)
+    AnyVec i_bias, f_bias;      // [heads]
+    int i_off, f_off;           // the first columns of their pre-activations in a row of proj
+    float cap;
+    long top_at;                // the running maximum's place in a head's state, which is read; the new one goes to top
+    float* top;                 // [rows, heads]
 };
 
 __device__ inline float silu_if(float x, int silu) { return silu ? x / (1.0f + expf(-x)) : x; }
@@ -277,7 +283,9 @@ __global__ void __launch_bounds__(kScanThreads) outer_scan_kernel(OuterScanArgs 
 // 256 bytes (the other kernel's are pieces of 32), and its waves take 32 key channels each; a row's q and k are made by
 // the lanes of the wave that needs them.  A segment's row, gates, values and state are
 // all asked for before the first is used.  The waves' sums meet in shared memory in the order in which the other kernel's
-// lanes meet.  Eight rows of four heads of 256 x 512 with a normaliser: 9.6 us (18.3 walked).
+// lanes meet.  Eight rows of four heads of 256 x 512 with a normaliser: 9.6 us (18.3 walked).  Exponential gates are made here as well
+// (GATEFIGURES): every workgroup of a head reads the running maximum, so none of them may write the new one into
+// the state; head_norm_gate, the next launch, does.
 // The float at a wave's own row (in bytes from a base that all waves share) and a lane's own column: one base and one offset of 32
 // bits a load, so that no row needs an address of its own.
 __device__ inline const float& float_at(const float* base, unsigned row_bytes, unsigned col_bytes) {
@@ -328,8 +336,14 @@ __global__ void __launch_bounds__(kGroups * kWave) outer_step_kernel(OuterScanAr
     const int other = ch < half ? ch + half : ch < 2 * half ? ch - half : ch;
     const int turned = ch < half ? ch : ch < 2 * half ? ch - half : 0;
     const float* from = seg.in < 0 ? nullptr : p.state_in + seg.in * p.in_stride + head * p.head_stride;
-    const float fixed = p.coef ? 0.f : p.decay[head];
+    const float fixed = p.coef || p.top ? 0.f : p.decay[head];
     float S[kLaneRows], N = 0.f;
+    float m = 0.f, bi = 0.f, bf = 0.f;
+    if (p.top) {
+        m = from ? from[p.top_at] : 0.f;
+        bi = load_any(p.i_bias, head);
+        bf = load_any(p.f_bias, head);
+    }
 #pragma unroll
     for (int i = 0; i < kLaneRows; ++i) S[i] = 0.f;
 
@@ -348,6 +362,11 @@ __global__ void __launch_bounds__(kGroups * kWave) outer_step_kernel(OuterScanAr
             a = p.coef[2 * at];
             b = p.coef[2 * at + 1];
         }
+        float raw_i = 0.f, raw_f = 0.f;
+        if (p.top) {
+            raw_i = base[p.i_off + head];
+            raw_f = base[p.f_off + head];
+        }
         if (p.cos_table) {
             const long angle = static_cast<long>(min(pos, p.table_positions - 1)) * half + turned;
             q.c = k.c = p.cos_table[angle];
@@ -357,6 +376,15 @@ __global__ void __launch_bounds__(kGroups * kWave) outer_step_kernel(OuterScanAr
 #pragma unroll
             for (int i = 0; i < kLaneRows; ++i) S[i] = float_at(from, (ch0 + i) * row_bytes, 4u * ccol);
             if (norm) N = from[static_cast<long>(p.dim) * p.vdim + ch];
+        }
+        if (p.top) {                                           // as exp_gates_kernel makes them, to the bit: no product joins a sum
+#pragma clang fp contract(off)
+            const float li = soft_cap_f(raw_i + bi, p.cap), lf = log_sigmoid_f(soft_cap_f(raw_f + bf, p.cap));
+            const float next = fmaxf(lf + m, li);
+            a = expf(lf + m - next);
+            b = expf(li - next);
+            m = next;
+            if (blockIdx.z == 0 && tid == 0) p.top[at] = m;
         }
         const float qv = turn(q, ch, p.silu, half) * p.q_scale;
         const float kv = turn(k, ch, p.silu, half) * p.k_scale;
@@ -724,12 +752,12 @@ static int run_outer_scan(bool single, const float* proj, long stride, int q_off
                                 const float* cos_table, const float* sin_table, int rotary_dim, int table_positions,
                                 const int* positions, const int* segments, int n_segments, const float* state_in,
                                 long in_stride, float* state_out, long out_stride, long head_stride, float* out, float* dot,
-                                int heads, int dim, int vdim, hipStream_t stream) {
+                                int heads, int dim, int vdim, hipStream_t stream, const OuterScanArgs* gates = nullptr) {
     LEONE_REQUIRE(proj && positions && segments && out, "outer_scan: null pointer");
     LEONE_REQUIRE(n_segments > 0 && heads > 0 && heads <= 65535 && dim > 0 && vdim > 0, "outer_scan: %d segments, %d heads of %d x %d",
                   n_segments, heads, dim, vdim);
     LEONE_REQUIRE(dim <= leone_scan_max_dim(), "outer_scan: heads of %d key channels, the kernel takes up to %d", dim, leone_scan_max_dim());
-    LEONE_REQUIRE(coef || decay, "outer_scan: neither per-row coefficients nor a fixed decay");
+    LEONE_REQUIRE(coef || decay || gates, "outer_scan: neither per-row coefficients nor a fixed decay");
     LEONE_REQUIRE(!norm_column || dot, "outer_scan: the normaliser's read-out needs a place");
     LEONE_REQUIRE((cos_table == nullptr) == (sin_table == nullptr), "outer_scan: cos and sin tables come together");
     LEONE_REQUIRE(!cos_table || (rotary_dim > 0 && rotary_dim % 2 == 0 && rotary_dim <= dim && table_positions > 0),
@@ -742,7 +770,11 @@ static int run_outer_scan(bool single, const float* proj, long stride, int q_off
     OuterScanArgs a{proj, stride, q_off, k_off, v_off, coef, decay, norm_column, q_scale, k_scale,
                     silu, cos_table, sin_table, cos_table ? rotary_dim / 2 : 0, cos_table ? table_positions : 1, positions,
                     reinterpret_cast<const Segment*>(segments), state_in, in_stride, state_out, out_stride, head_stride,
-                    out, dot, heads, dim, vdim};
+                    out, dot, heads, dim, vdim, AnyVec{nullptr, kF32}, AnyVec{nullptr, kF32}, 0, 0, 0.f, 0, nullptr};
+    if (gates) {
+        a.i_bias = gates->i_bias, a.f_bias = gates->f_bias, a.i_off = gates->i_off, a.f_off = gates->f_off;
+        a.cap = gates->cap, a.top_at = gates->top_at, a.top = gates->top;
+    }
     const int groups = lane_groups(dim);
     const int per_block = (kScanThreads / kWave) * (kWave / groups) * kLaneCols;          // columns a workgroup
     const dim3 grid(n_segments, heads, ceil_div(vdim + (norm_column ? 1 : 0), per_block));
@@ -783,6 +815,26 @@ extern "C" int leone_outer_step(const float* proj, long stride, int q_off, int k
     return run_outer_scan(true, proj, stride, q_off, k_off, v_off, coef, decay, norm_column, q_scale, k_scale, silu, cos_table,
         sin_table, rotary_dim, table_positions, positions, segments, n_segments, state_in, in_stride, state_out, out_stride,
         head_stride, out, dot, heads, dim, vdim, stream);
+}
+
+// leone_outer_step with a normaliser and exponential gates made in the launch (what leone_exp_gates writes to coef and top, but the state's
+// maximum stays as it is: leone_head_norm_gate_kept writes it).
+extern "C" int leone_outer_step_gated(const float* proj, long stride, int q_off, int k_off, int v_off, int i_off, int f_off,
+                                      const void* i_bias, const void* f_bias, int bias_dtype, float cap, long top_at, float* top,
+                                      float q_scale, float k_scale, int silu, const float* cos_table, const float* sin_table, int rotary_dim,
+                                      int table_positions, const int* positions, const int* segments, int n_segments, const float* state_in,
+                                      long in_stride, float* state_out, long out_stride, long head_stride, float* out, float* dot, int heads,
+                                      int dim, int vdim, hipStream_t stream) {
+    LEONE_REQUIRE(i_bias && f_bias && top && state_in, "outer_step: the gates' operands are missing");
+    LEONE_REQUIRE(known_vec(bias_dtype) && cap > 0.f, "outer_step: unknown bias type or cap %g", cap);
+    LEONE_REQUIRE(i_off >= 0 && f_off >= 0 && stride >= i_off + heads && stride >= f_off + heads, "outer_step: rows of %ld do not hold the gates", stride);
+    LEONE_REQUIRE(top_at >= 0 && top_at < head_stride, "outer_step: the maximum's place %ld", top_at);
+    OuterScanArgs gates{};
+    gates.i_bias = AnyVec{i_bias, bias_dtype}, gates.f_bias = AnyVec{f_bias, bias_dtype};
+    gates.i_off = i_off, gates.f_off = f_off, gates.cap = cap, gates.top_at = top_at, gates.top = top;
+    return run_outer_scan(true, proj, stride, q_off, k_off, v_off, nullptr, nullptr, 1, q_scale, k_scale, silu, cos_table,
+        sin_table, rotary_dim, table_positions, positions, segments, n_segments, state_in, in_stride, state_out, out_stride,
+        head_stride, out, dot, heads, dim, vdim, stream, &gates);
 }
 
 static int run_delta_scan(bool single, const float* qkv, long stride, int q_off, int k_off, int v_off, const float* beta,

@@ -867,12 +867,13 @@ def tile_weight(weight: torch.Tensor) -> torch.Tensor:
     return weight.view(tiles, 16, k // 64, 4, 2, 8).permute(0, 2, 4, 3, 1, 5).contiguous()
 
 
-_streamed: dict = {}         # (address, shape) of a weight -> (weak reference to the weight, its tiled copy)
+_streamed: dict = {}         # (address, shape) of a weight -> (weak reference to the weight, its tiled copy, whether sums may be in another order)
 
 
-def keep_streamed_copy(weight: torch.Tensor) -> int:
+def keep_streamed_copy(weight: torch.Tensor, any_order: bool = True) -> int:
     """Makes and keeps the tiled copy of a weight; the products take it from then on whenever they are given
-    this weight, and it is dropped when the weight is.  Returns the copy's bytes (0 if the weight's shape or
+    this weight, and it is dropped when the weight is.  Without ``any_order`` only those take it that add in the order they have
+    without it, to the bit.  Returns the copy's bytes (0 if the weight's shape or
     type has no tiled form)."""
     if weight.dtype != torch.bfloat16 or weight.dim() != 2 or weight.shape[1] % 64 or not weight.is_cuda:
         return 0
@@ -881,13 +882,19 @@ def keep_streamed_copy(weight: torch.Tensor) -> int:
     if held is None or held[0]() is not weight:
         def forget(_, key=key):
             _streamed.pop(key, None)
-        _streamed[key] = (weakref.ref(weight, forget), tile_weight(weight))
+        _streamed[key] = (weakref.ref(weight, forget), tile_weight(weight), bool(any_order))
     return _streamed[key][1].numel() * 2
 
 
 def streamed_copy(weight: torch.Tensor) -> Optional[torch.Tensor]:
     held = _streamed.get((weight.data_ptr(), tuple(weight.shape)))
     return None if held is None or held[0]() is not weight else held[1]
+
+
+def _any_order(weight: torch.Tensor) -> bool:
+    """Whether the weight has a copy that its products may take in any order of their sums."""
+    held = _streamed.get((weight.data_ptr(), tuple(weight.shape)))
+    return held is not None and held[0]() is weight and held[2]
 
 
 def drop_streamed_copies() -> None:
@@ -1111,7 +1118,9 @@ def _takes_many(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype, r
         return None
     if _tuned_products and _library_problem(x, weight, torch.float32 if residual is not None else out_dtype, residual is not None) in _tuned_products:
         return None
-    return streamed_copy(weight) if tiles is None else tiles
+    if tiles is not None:
+        return tiles
+    return streamed_copy(weight) if _any_order(weight) else None
 
 
 # Tiles of ``gemm_many`` that read the weight once, four stages ahead, for up to ROWS_MAX rows: (rows, columns): us to start, us a stage of 64
@@ -1162,7 +1171,9 @@ def _takes_deep(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype, r
     whose units are all at work either way, are behind (24,576 x 4,096 for 96 and 128 rows 44 and 45, 48 and 49, 18,432 x 3,072 30 and 34, 35 and 39)."""
     if not FUSED_ROWS < x.shape[0] <= ROWS_MAX or (gated and x.shape[0] > 64 and weight.numel() > DEEP_GATED_MOST) or not _many_fits(x, weight, out_dtype, residual, gated):
         return None
-    return streamed_copy(weight) if tiles is None else tiles
+    if tiles is not None:
+        return tiles
+    return streamed_copy(weight) if _any_order(weight) else None
 
 
 def gemm_many(x: torch.Tensor, tiles: torch.Tensor, n: int, out_dtype: torch.dtype = torch.bfloat16, residual: Optional[torch.Tensor] = None,
@@ -1434,6 +1445,7 @@ def linear_planes(x: torch.Tensor, weight: torch.Tensor, rows_of) -> list:
         raise KernelError(f"linear_planes: inputs {tuple(x.shape)} of {x.dtype} against {tuple(weight.shape)} of {weight.dtype} in {rows_of} rows")
     starts = [sum(rows_of[:p]) for p in range(planes)]
     tiles = streamed_copy(weight) if _streamed else None
+    any_order = _any_order(weight)
     if x.dtype == torch.bfloat16 and rows <= FUSED_ROWS and k % 8 == 0 and rows_of[0] % 16 == 0 \
             and all(r == rows_of[0] for r in rows_of[:-1]) and rows_of[-1] <= rows_of[0]:
         out = torch.empty((rows, weight.shape[0]), dtype=torch.float32, device=x.device)
@@ -1448,14 +1460,14 @@ def linear_planes(x: torch.Tensor, weight: torch.Tensor, rows_of) -> list:
         if x.dtype == torch.bfloat16 and FUSED_ROWS < rows <= ROWS_MAX and k % 8 == 0 and tiles is not None and at % 16 == 0:
             # the whole matrix's second copy is tiles of 16 rows: a part that begins at one has its own piece of it
             own = tiles[at // 16:-(-(at + r) // 16)]
-            if _takes_deep(x[p], part, torch.float32, None, False, own) is not None:
+            if any_order and _takes_deep(x[p], part, torch.float32, None, False, own) is not None:
                 with profile.span("gemm rows", part):
                     results.append(gemm_many(x[p], own, r, torch.float32, plan=deep_plan(rows, r, k, False, False, compute_units(x.device))))
             else:
                 results.append(gemm_rows(x[p], part, torch.float32, may_split=False, tiles=own))
             continue
         many = None
-        if x.dtype == torch.bfloat16 and rows > ROWS_MAX and tiles is not None and at % 16 == 0:
+        if x.dtype == torch.bfloat16 and rows > ROWS_MAX and any_order and at % 16 == 0:
             many = _takes_many(x[p], part, torch.float32, None, False, tiles[at // 16:-(-(at + r) // 16)])
         if many is not None:
             with profile.span("gemm many", part):
@@ -1807,7 +1819,7 @@ def head_norm_gate(o: torch.Tensor, heads: int, vdim: int, eps: float, out_dtype
                    activation: Optional[str] = None, denominator: Optional[tuple] = None,
                    gate_first: bool = False) -> torch.Tensor:
     """Head by head: o (float32 ``[rows, heads * vdim]``), divided by max(|dot|, exp(-top)) + 1e-6 if
-    ``denominator`` = (dot, top) (float32 ``[rows, heads]``) comes, over its root mean square, times ``gain``
+    ``denominator`` = (dot, top) (float32 ``[rows, heads]``; perhaps a third, ``outer_scan``'s) comes, over its root mean square, times ``gain``
     (``[heads * vdim]``, or ``[vdim]`` shared by the heads), times activation(gate) (float32 rows of heads * vdim,
     possibly a slice of wider rows).  ``gate_first``: the gate multiplies ahead of the norm, so the root mean square
     is that of the gated values.  A "head" is whatever run of ``vdim`` columns is normed by itself."""
@@ -1820,11 +1832,15 @@ def head_norm_gate(o: torch.Tensor, heads: int, vdim: int, eps: float, out_dtype
         elif gain.numel() != vdim:
             raise KernelError(f"head_norm_gate: a gain of {gain.numel()} for {heads} heads of {vdim}")
     gate_at, gate_stride = _strided_rows(gate, "head_norm_gate gate", rows, heads * vdim)
-    dot, top = denominator if denominator is not None else (None, None)
-    call("leone_head_norm_gate_ordered", _dev(o, "read-outs", torch.float32, (rows, heads * vdim)),
+    dot, top, *keep = denominator if denominator is not None else (None, None)
+    kept = (0, 0, 0, 0)
+    if keep:                                              # the running maxima go into their state (``outer_scan``)
+        state, top_at, per_head_state, spans = keep[0]
+        kept = (_dev(state, "state", torch.float32) + 4 * top_at, state.stride(0), per_head_state, _dev(spans, "spans", torch.int32, (rows, 4)))
+    call("leone_head_norm_gate_kept", _dev(o, "read-outs", torch.float32, (rows, heads * vdim)),
          _dev(dot, "dot", torch.float32, (rows, heads)), _dev(top, "top", torch.float32, (rows, heads)),
          _dev(gain, "gain"), _code(gain, "gain") if gain is not None else F32, per_head, gate_at, gate_stride,
-         ACTIVATIONS[activation], 1 if gate_first else 0, float(eps), _dev(out, "out"), _CODES[out_dtype], rows, heads, vdim, _stream())
+         ACTIVATIONS[activation], 1 if gate_first else 0, float(eps), _dev(out, "out"), _CODES[out_dtype], rows, heads, vdim, *kept, _stream())
     return out
 
 
@@ -1970,7 +1986,7 @@ def chunked_memory(rows: torch.Tensor, columns: dict, plan: dict, state: torch.T
 def outer_scan(proj: torch.Tensor, columns: dict, state: torch.Tensor, step, heads: int, dim: int, vdim: int, *,
                gates: Optional[dict] = None, decay: Optional[torch.Tensor] = None, q_scale: float = 1.0,
                k_scale: float = 1.0, cos: Optional[torch.Tensor] = None, sin: Optional[torch.Tensor] = None,
-               activation: Optional[str] = None, write_state: bool = True):
+               activation: Optional[str] = None, write_state: bool = True, keep_later: bool = False):
     """The matrix-memory recurrence S_t = a_t S_(t-1) + b_t k_t v_t^T, o_t = S_t^T q_t over every entry's rows,
     from and into ``state`` (float32 ``[slots, heads, dim * vdim]``, with ``gates`` ``dim * vdim + dim + 1``: the
     normaliser and the running maximum ride along).  ``proj`` is float32 ``[rows, width]``; ``columns`` names the
@@ -1978,7 +1994,9 @@ def outer_scan(proj: torch.Tensor, columns: dict, state: torch.Tensor, step, hea
     ``gates`` = {"i_bias", "f_bias", "cap"}: exponential gates with a running maximum that starts at 0; else
     ``decay`` (float32 ``[heads]``) with b = 1.  ``cos``/``sin``: rotary tables for q and k.  ``activation`` "silu": q, k and v
     pass through it first.
-    Returns o float32 ``[rows, heads * vdim]`` and, with gates, (dot, top) for ``head_norm_gate``.
+    Returns o float32 ``[rows, heads * vdim]`` and, with gates, (dot, top) for ``head_norm_gate``; with ``keep_later`` and one row an
+    entry the gates are made in the step's own launch and (dot, top, where the state's running maximum is kept) comes back, which
+    ``head_norm_gate`` writes: it has to be called with it, whatever the rows are for.
 
     Single tokens and short portions are walked row by row, a long portion goes through as ``chunked_memory``."""
     rows, width = proj.shape
@@ -1994,9 +2012,20 @@ def outer_scan(proj: torch.Tensor, columns: dict, state: torch.Tensor, step, hea
     if gates:
         dot = torch.empty((rows, heads), dtype=torch.float32, device=device)
         top = torch.empty((rows, heads), dtype=torch.float32, device=device)
-        coef = torch.empty((rows, heads, 2), dtype=torch.float32, device=device)
         if gates["i_bias"].dtype != gates["f_bias"].dtype:
             raise KernelError("outer_scan: the gates' biases must share one type")
+    if gates and keep_later and spans.shape[0] == rows and longest_entry(step) == 1 and library().leone_step_fits(dim, vdim):
+        call("leone_outer_step_gated", _dev(proj, "projection", torch.float32), width, columns["q"], columns["k"], columns["v"],
+             columns["i"], columns["f"], _dev(gates["i_bias"], "i bias", None, (heads,)), _dev(gates["f_bias"], "f bias", None, (heads,)),
+             _code(gates["i_bias"], "i bias"), float(gates["cap"]), dim * vdim + dim, _dev(top, "top"), float(q_scale), float(k_scale),
+             1 if activation == "silu" else 0, _dev(cos, "rope cos", torch.float32), _dev(sin, "rope sin", torch.float32),
+             2 * cos.shape[1] if cos is not None else 0, cos.shape[0] if cos is not None else 0,
+             _dev(step.positions, "positions", torch.int32, (rows,)), _dev(spans, "spans", torch.int32), rows, _dev(state, "state read"),
+             state.stride(0), _dev(state if write_state else None, "state written"), state.stride(0) if write_state else 0, per_head,
+             _dev(out, "out"), _dev(dot, "dot"), heads, dim, vdim, _stream())
+        return out, (dot, top, (state, dim * vdim + dim, per_head, spans)) if write_state else (dot, top)
+    if gates:
+        coef = torch.empty((rows, heads, 2), dtype=torch.float32, device=device)
         call("leone_exp_gates", _dev(proj, "projection", torch.float32), width, columns["i"], columns["f"],
              _dev(gates["i_bias"], "i bias", None, (heads,)), _dev(gates["f_bias"], "f bias", None, (heads,)),
              _code(gates["i_bias"], "i bias"), float(gates["cap"]), _dev(spans, "spans"), spans.shape[0],

@@ -65,6 +65,7 @@ _PROTOTYPES = {
                           c_int, c_int, c_int, c_int, c_int, P],
     "leone_head_norm_gate": [P, P, P, P, c_int, c_int, P, ctypes.c_long, c_int, c_float, P, c_int, c_int, c_int, c_int, P],
     "leone_head_norm_gate_ordered": [P, P, P, P, c_int, c_int, P, ctypes.c_long, c_int, c_int, c_float, P, c_int, c_int, c_int, c_int, P],
+    "leone_head_norm_gate_kept": [P, P, P, P, c_int, c_int, P, ctypes.c_long, c_int, c_int, c_float, P, c_int, c_int, c_int, c_int, P, ctypes.c_long, ctypes.c_long, P, P],
     "leone_weighted_mix": [P, P, c_int, P, ctypes.c_long, P],
     "leone_causal_conv_biased": [P, c_int, ctypes.c_long, P, c_int, ctypes.c_long, P, P, c_int, P, c_int, P, c_int, P, P, P, c_int,
                                  c_int, c_int, c_int, c_int, c_int, P],
@@ -88,6 +89,8 @@ _PROTOTYPES = {
     "leone_step_fits": [c_int, c_int],
     "leone_outer_step": [P, ctypes.c_long, c_int, c_int, c_int, P, P, c_int, c_float, c_float, c_int, P, P, c_int, c_int,
                          P, P, c_int, P, ctypes.c_long, P, ctypes.c_long, ctypes.c_long, P, P, c_int, c_int, c_int, P],
+    "leone_outer_step_gated": [P, ctypes.c_long, c_int, c_int, c_int, c_int, c_int, P, P, c_int, c_float, ctypes.c_long, P, c_float, c_float, c_int,
+                               P, P, c_int, c_int, P, P, c_int, P, ctypes.c_long, P, ctypes.c_long, ctypes.c_long, P, P, c_int, c_int, c_int, P],
     "leone_delta_scan": [P, ctypes.c_long, c_int, c_int, c_int, P, ctypes.c_long, P, ctypes.c_long, c_int, P, P, c_int, c_float,
                          c_float, c_int, c_int, P, c_int, P, ctypes.c_long, P, ctypes.c_long, P, P, c_int, c_int, c_int, c_int, P],
     "leone_delta_step": [P, ctypes.c_long, c_int, c_int, c_int, P, ctypes.c_long, P, ctypes.c_long, c_int, P, P, c_int, c_float,

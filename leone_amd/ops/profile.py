@@ -47,6 +47,7 @@ OPERATIONS = {
     "leone_head_gate": "head gate",
     "leone_outer_scan": "outer scan",
     "leone_outer_step": "outer scan",
+    "leone_outer_step_gated": "outer scan",
     "leone_exp_gates": "exp gates",
     "leone_delta_scan": "delta scan",
     "leone_delta_step": "delta scan",
@@ -90,7 +91,7 @@ OPERATIONS = {
     "leone_attention_decode_biased": "attention",
     "leone_attention_prefill_biased": "attention",
     "leone_causal_conv_biased": "causal conv",
-    "leone_head_norm_gate_ordered": "head norm gate",
+    "leone_head_norm_gate_kept": "head norm gate",
     "leone_weighted_mix": "branch mix",
     "leone_state_space_scan": "state space scan",
     "leone_bias_span_norm": "bias span norm",

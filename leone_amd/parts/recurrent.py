@@ -78,7 +78,7 @@ class MlstmMixer(Part):
         proj = ops.linear(h, self.w_in, out_dtype=torch.float32)
         o, under = ops.outer_scan(proj, self.columns, cache.state, step, self.heads, self.dim, self.vdim,
                                   gates={"i_bias": self.i_bias, "f_bias": self.f_bias, "cap": self.cap},
-                                  q_scale=1.0 / math.sqrt(self.dim), write_state=cache.writes)
+                                  q_scale=1.0 / math.sqrt(self.dim), write_state=cache.writes, keep_later=True)
         gate = proj[:, self.columns["g"]:self.columns["i"]]
         y = ops.head_norm_gate(o, self.heads, self.vdim, self.eps, step.dtype, gain=self.norm, gate=gate,
                                activation="sigmoid", denominator=under)

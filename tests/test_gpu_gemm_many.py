@@ -137,3 +137,15 @@ def test_products_of_up_to_128_rows_take_the_copy(m, n, k):
         assert ((torch.cat(pieces, 1).double() - want).abs() <= bound).all()
     finally:
         ops.drop_streamed_copies()
+
+
+@pytest.mark.parametrize("m", [64, 300])
+def test_a_copy_for_sums_in_their_old_order_is_left_alone_by_others(m):
+    x, weight, tiles, want, bound = _operands(m, 1040, 1024)
+    plain, parts = ops.linear(x, weight, out_dtype=torch.float32), ops.linear_planes(torch.stack([x, x]), weight, [16, 1024])
+    try:
+        ops.keep_streamed_copy(weight, any_order=False)
+        assert torch.equal(ops.linear(x, weight, out_dtype=torch.float32), plain)
+        assert all(torch.equal(a, b) for a, b in zip(ops.linear_planes(torch.stack([x, x]), weight, [16, 1024]), parts))
+    finally:
+        ops.drop_streamed_copies()
