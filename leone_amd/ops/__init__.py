@@ -867,7 +867,7 @@ def tile_weight(weight: torch.Tensor) -> torch.Tensor:
     return weight.view(tiles, 16, k // 64, 4, 2, 8).permute(0, 2, 4, 3, 1, 5).contiguous()
 
 
-_streamed: dict = {}         # (address, shape) of a weight -> (weak reference to the weight, its tiled copy, whether sums may be in another order)
+_streamed: dict = {}         # (address, shape) of a weight -> (weak reference to the weight, its tiled copy, whether sums may be in another order, plans)
 
 
 def keep_streamed_copy(weight: torch.Tensor, any_order: bool = True) -> int:
@@ -882,7 +882,7 @@ def keep_streamed_copy(weight: torch.Tensor, any_order: bool = True) -> int:
     if held is None or held[0]() is not weight:
         def forget(_, key=key):
             _streamed.pop(key, None)
-        _streamed[key] = (weakref.ref(weight, forget), tile_weight(weight), bool(any_order))
+        _streamed[key] = (weakref.ref(weight, forget), tile_weight(weight), bool(any_order), {})
     return _streamed[key][1].numel() * 2
 
 
@@ -960,7 +960,7 @@ _UNITS = {}
 
 
 def compute_units(device) -> int:
-    index = torch.device(device).index or 0
+    index = (device if isinstance(device, torch.device) else torch.device(device)).index or 0
     if index not in _UNITS:
         _UNITS[index] = torch.cuda.get_device_properties(index).multi_processor_count if torch.cuda.is_available() else 256
     return _UNITS[index]
@@ -1169,11 +1169,38 @@ def _takes_deep(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype, r
     14.8, 22.7 and 19.0, 6,144 x 1,024 7.8 and 7.2, 10.4 and 9.1, 15.3 and 9.1, 24,576 x 4,096 39.3 and 36.6, 40.3 and 37.3.  Over the shapes measured planes are
     1.28 times as fast (0.94 at the least), logits 1.27 (0.99), gated products of up to 64 rows 1.06 (0.97); of more rows the larger gated weights,
     whose units are all at work either way, are behind (24,576 x 4,096 for 96 and 128 rows 44 and 45, 48 and 49, 18,432 x 3,072 30 and 34, 35 and 39)."""
-    if not FUSED_ROWS < x.shape[0] <= ROWS_MAX or (gated and x.shape[0] > 64 and weight.numel() > DEEP_GATED_MOST) or not _many_fits(x, weight, out_dtype, residual, gated):
+    found = _deep_choice(x, weight, out_dtype, residual, gated, False, tiles)
+    return None if found is None else found[0]
+
+
+def _deep_choice(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype, residual: Optional[torch.Tensor], gated: bool,
+                 may_split: bool, tiles: Optional[torch.Tensor] = None) -> Optional[tuple]:
+    """(tiled copy, plan) if ``_takes_deep``; what sizes and types say is kept beside the copy, since steps that are not recorded wait
+    for the host (a microsecond a product)."""
+    m, n = x.shape[0], weight.shape[0]
+    if tiles is None:
+        held = _streamed.get((weight.data_ptr(), weight.shape))
+        if held is None or not held[2] or held[0]() is not weight:
+            return None
+        tiles, plans, key = held[1], held[3], (m, may_split, gated, out_dtype)
+        plan = plans.get(key, 0)
+        if plan == 0:
+            plan = plans[key] = _deep_sizes(m, n, x.shape[1], may_split, gated, out_dtype, compute_units(weight.device))
+    else:
+        plan = _deep_sizes(m, n, x.shape[1], may_split, gated, out_dtype, compute_units(weight.device))
+    if plan is None or not x.is_contiguous() or x.data_ptr() % 16 or x.shape[1] != weight.shape[1]:
         return None
-    if tiles is not None:
-        return tiles
-    return streamed_copy(weight) if _any_order(weight) else None
+    if residual is not None and (gated or residual.dtype != torch.float32 or residual.shape != (m, n) or not residual.is_contiguous()
+                                 or residual.data_ptr() % 16):
+        return None
+    return tiles, plan
+
+
+def _deep_sizes(m: int, n: int, k: int, may_split: bool, gated: bool, out_dtype: torch.dtype, units: int) -> Optional[tuple]:
+    if not FUSED_ROWS < m <= ROWS_MAX or k % 64 or n % 16 or n < MANY_LEAST or k < MANY_LEAST or out_dtype not in _CODES \
+            or (gated and (out_dtype != torch.bfloat16 or (m > 64 and n * k > DEEP_GATED_MOST))):
+        return None
+    return deep_plan(m, n, k, may_split and not gated, gated, units)
 
 
 def gemm_many(x: torch.Tensor, tiles: torch.Tensor, n: int, out_dtype: torch.dtype = torch.bfloat16, residual: Optional[torch.Tensor] = None,
@@ -1186,7 +1213,7 @@ def gemm_many(x: torch.Tensor, tiles: torch.Tensor, n: int, out_dtype: torch.dty
     m, k = x.shape
     if gated and residual is not None:
         raise KernelError("gemm_many: a gated product cannot also be added into the stream")
-    if tiles.shape != (-(-n // 16), k // 64, 2, 4, 16, 8):
+    if tiles.numel() != (n + 15) // 16 * 16 * k or tiles.dim() != 6 or tiles.shape[1] * 64 != k:
         raise KernelError(f"gemm_many: a tiled copy of shape {tuple(tiles.shape)} is not one of {n} x {k}")
     rows, columns, splits, *deep = plan or many_plan(m, n, k, residual is not None, compute_units(x.device))
     mode, code, kind = 0, 0, out_dtype
@@ -1394,11 +1421,10 @@ def linear(x, weight: torch.Tensor, out_dtype: Optional[torch.dtype] = None,
     if dtype == torch.bfloat16 and weight.is_cuda and k % 8 == 0 and rows <= ROWS_MAX \
             and (not gated or weight.shape[0] % 16 == 0):
         may_split = planes_ok or residual is not None
-        tiles = _takes_deep(x, weight, out_dtype, residual, gated)
-        if tiles is not None:
-            plan = deep_plan(rows, *weight.shape, may_split and not gated, gated, compute_units(x.device))
+        deep = _deep_choice(x, weight, out_dtype, residual, gated, may_split) if _streamed else None
+        if deep is not None:
             with profile.span("gemm rows", weight):
-                return gemm_many(x, tiles, weight.shape[0], out_dtype, residual, gated, plan, activation=activation, limit=limit)
+                return gemm_many(x, deep[0], weight.shape[0], out_dtype, residual, gated, deep[1], activation, limit)
         return gemm_rows(x, weight, out_dtype, residual, gated, may_split=may_split, activation=activation, limit=limit)
     if dtype == torch.bfloat16 and x.is_cuda and weight.is_cuda and rows > ROWS_MAX:
         tiles = _takes_many(x, weight, out_dtype, residual, gated)
@@ -1460,9 +1486,10 @@ def linear_planes(x: torch.Tensor, weight: torch.Tensor, rows_of) -> list:
         if x.dtype == torch.bfloat16 and FUSED_ROWS < rows <= ROWS_MAX and k % 8 == 0 and tiles is not None and at % 16 == 0:
             # the whole matrix's second copy is tiles of 16 rows: a part that begins at one has its own piece of it
             own = tiles[at // 16:-(-(at + r) // 16)]
-            if any_order and _takes_deep(x[p], part, torch.float32, None, False, own) is not None:
+            deep = _deep_choice(x[p], part, torch.float32, None, False, False, own) if any_order else None
+            if deep is not None:
                 with profile.span("gemm rows", part):
-                    results.append(gemm_many(x[p], own, r, torch.float32, plan=deep_plan(rows, r, k, False, False, compute_units(x.device))))
+                    results.append(gemm_many(x[p], own, r, torch.float32, plan=deep[1]))
             else:
                 results.append(gemm_rows(x[p], part, torch.float32, may_split=False, tiles=own))
             continue
