@@ -39,8 +39,8 @@ namespace leone {
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
 
-enum FusedIn : int { kInPlain = 0, kInNorm = 1, kInPrepared = 2 };
-enum FusedOut : int { kOutStore = 0, kOutResidual = 1, kOutGated = 2, kOutPrepare = 3 };
+enum FusedIn : int { kInPlain = 0, kInNorm = 1, kInPrepared = 2, kInFloats = 3 };
+enum FusedOut : int { kOutStore = 0, kOutResidual = 1, kOutGated = 2, kOutPrepare = 3, kOutSquared = 6 };
 
 struct FusedArgs {
     const void* x;       // plain: bfloat16 [M,K]; norm: float [*, K]
@@ -60,6 +60,7 @@ struct FusedArgs {
     float limit = 0.f;         // gated: what that activation holds gate and up to
     int plane_rows = 0;        // plain: rows of W that read one plane of X, a multiple of 16 (0: there is one plane)
     int planes = 1;
+    long x_row = 0, x_plane = 0;   // floats: from row to row of X and from plane to plane, in elements
 };
 
 __device__ inline bf16x8 fz8() {
@@ -114,12 +115,12 @@ gemm_fused_kernel(FusedArgs a) {
     extern __shared__ float4 sums_of_squares[];      // [m * k / 64]
     const int quads = kIn == kInPrepared ? m * (k / 64) : 0;
     long plane = 0;
-    if (kIn == kInPlain && a.plane_rows > 0) {
+    if ((kIn == kInPlain || kIn == kInFloats) && a.plane_rows > 0) {
         plane = n0 / a.plane_rows;
         plane = plane < a.planes ? plane : a.planes - 1;
     }
     const bf16_t* xb = static_cast<const bf16_t*>(a.x) + (plane * m + xrow_index) * k + 16 * g;   // plain
-    const float* xf = static_cast<const float*>(a.x) + xrow_index * k + 16 * g;     // norm
+    const float* xf = static_cast<const float*>(a.x) + (kIn == kInFloats ? plane * a.x_plane + xrow_index * a.x_row : xrow_index * k) + 16 * g;   // norm, floats
     floatx4 acc = {0.f, 0.f, 0.f, 0.f};
 
     // One step: 64 elements of K; this lane's run is elements at + 16g .. + 15, `left` of which exist.
@@ -130,8 +131,14 @@ gemm_fused_kernel(FusedArgs a) {
         for (int h = 0; h < 2; ++h) {
             if (left < 8 * (h + 1)) {
                 b[h] = fz8();
-            } else if (kIn != kInNorm) {
+            } else if (kIn == kInPlain || kIn == kInPrepared) {
                 b[h] = fld8(xb + at + 8 * h);
+            } else if (kIn == kInFloats) {
+                const float4 lo = *reinterpret_cast<const float4*>(xf + at + 8 * h);
+                const float4 hi = *reinterpret_cast<const float4*>(xf + at + 8 * h + 4);
+                const float v[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+#pragma unroll
+                for (int i = 0; i < 8; ++i) b[h][i] = static_cast<__bf16>(v[i]);
             } else {
                 const float4 lo = *reinterpret_cast<const float4*>(xf + at + 8 * h);
                 const float4 hi = *reinterpret_cast<const float4*>(xf + at + 8 * h + 4);
@@ -259,7 +266,7 @@ gemm_fused_kernel(FusedArgs a) {
     for (int v = 0; v < kWaves; ++v)
 #pragma unroll
         for (int r = 0; r < 4; ++r) sum[r] += partial[v][lane][r];
-    if (kIn != kInPlain) {
+    if (kIn == kInNorm || kIn == kInPrepared) {
         float total = 0.f;
         if (kIn == kInPrepared) {
             // lane (c, g) adds the g-th quarter of row c's partial sums, then the four quarters meet
@@ -341,8 +348,14 @@ gemm_fused_kernel(FusedArgs a) {
     } else {
         TOut* out = static_cast<TOut*>(a.y) + static_cast<long>(row) * n + col;
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-            if (col + r < n) out[r] = from_float<TOut>(sum[r]);
+        for (int r = 0; r < 4; ++r) {
+            float v = sum[r];
+            if constexpr (kOut == kOutSquared) {         // (not by an argument: its load, at the end, cost every other store 0.2 us)
+                v = fmaxf(to_float(from_float<TOut>(v)), 0.f);
+                v *= v;
+            }
+            if (col + r < n) out[r] = from_float<TOut>(v);
+        }
     }
 }
 
@@ -393,6 +406,8 @@ using namespace leone;
 // [m,k] and squares_in float32 [m, ceil(k / 16)] as an earlier call's out_mode 3 wrote them, eps).
 // out_mode: 0 store (y of out_dtype [m,n]), 1 residual (y float32 [m,n] += product), 2 gated (y bfloat16 [m,n/2]),
 // 4 gated with the tanh form of gelu on the gate instead of silu, 5 gated with gate and up held to `limit` (GateAct 2),
+// 6 plain bfloat16 rows alone: store of the result, rounded, below zero zero, squared (what a launch of relu_squared behind a store gives, to the bit; eight rows of
+// 2,048 x 4,096: that launch was 4.9 us),
 // 3 prepare (as 1, and operand_out bfloat16 [m,n] = bf16(y * next_gain), squares_out float32 [m, ceil(n / 16)]).
 extern "C" int leone_gemm_fused_bf16(const void* x, int in_mode, const int* rows, const void* gain, int gain_dtype,
                                      float eps, const void* w, int w_tiled, void* y, int out_mode, int out_dtype, int m, int n,
@@ -412,9 +427,10 @@ extern "C" int leone_gemm_fused_bf16(const void* x, int in_mode, const int* rows
     LEONE_REQUIRE(in_mode != kInPrepared || (k % 64 == 0 && static_cast<long>(m) * (k / 64) <= 8 * 256 &&
                                              reinterpret_cast<uintptr_t>(squares_in) % 16 == 0),
                   "gemm_fused: the prepared input takes K %d a multiple of 64 with rows x K / 64 up to 2048", k);
-    LEONE_REQUIRE(out_mode >= kOutStore && out_mode <= kOutPrepare + 2, "gemm_fused: unknown output mode %d", out_mode);
+    LEONE_REQUIRE(out_mode >= kOutStore && out_mode <= kOutSquared, "gemm_fused: unknown output mode %d", out_mode);
+    LEONE_REQUIRE(out_mode != kOutSquared || (in_mode == kInPlain && out_dtype == kBF16), "gemm_fused: the square goes with plain bfloat16 rows");
     const int act = out_mode == kOutPrepare + 1 ? kGateGeluTanh : out_mode == kOutPrepare + 2 ? kGateClampedSwish : kGateSilu;
-    if (out_mode > kOutPrepare) out_mode = kOutGated;
+    if (out_mode > kOutPrepare && out_mode != kOutSquared) out_mode = kOutGated;
     LEONE_REQUIRE(act != kGateClampedSwish || limit > 0.f, "gemm_fused: the clamped activation needs a positive limit, found %g", limit);
     LEONE_REQUIRE(out_mode != kOutGated || n % 16 == 0, "gemm_fused: gated output needs N %d to be a multiple of 16", n);
     LEONE_REQUIRE(out_mode != kOutStore || out_dtype == kF32 || out_dtype == kBF16, "gemm_fused: unknown output type");
@@ -433,7 +449,9 @@ extern "C" int leone_gemm_fused_bf16(const void* x, int in_mode, const int* rows
         case kOutPrepare: launch_fused<IN, kOutPrepare, float>(a, w_tiled != 0, stream); break;            \
         default: launch_fused<IN, kOutGated, bf16_t>(a, w_tiled != 0, stream); break;                      \
     }
-    if (in_mode == kInPlain) {
+    if (out_mode == kOutSquared) {
+        launch_fused<kInPlain, kOutSquared, bf16_t>(a, w_tiled != 0, stream);
+    } else if (in_mode == kInPlain) {
         LEONE_FUSED_OUT(kInPlain)
     } else if (in_mode == kInNorm) {
         LEONE_FUSED_OUT(kInNorm)
@@ -459,6 +477,25 @@ extern "C" int leone_gemm_planes_bf16(const void* x, int planes, int plane_rows,
     a.x = x, a.w = static_cast<const bf16_t*>(w), a.y = y, a.m = m, a.n = n, a.k = k, a.plane_rows = plane_rows, a.planes = planes;
     if (out_dtype == kF32) launch_fused<kInPlain, kOutStore, float>(a, w_tiled != 0, stream);
     else launch_fused<kInPlain, kOutStore, bf16_t>(a, w_tiled != 0, stream);
+    LEONE_LAUNCH_CHECK("gemm_planes");
+    return 0;
+}
+
+// The same from float rows, rounded to bfloat16 as they are read: row r of plane p at x + p * x_plane + r * x_row, 16-byte runs.  (Rounded by a launch of
+// its own that was 4.9 us a layer of eight rows.)
+extern "C" int leone_gemm_float_planes_bf16(const float* x, long x_row, long x_plane, int planes, int plane_rows, const void* w, int w_tiled, float* y,
+                                            int m, int n, int k, hipStream_t stream) {
+    LEONE_REQUIRE(x && w && y, "gemm_planes: null pointer");
+    LEONE_REQUIRE(!w_tiled || (k % 64 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0),
+                  "gemm_planes: tiled weights need K %d to be a multiple of 64", k);
+    LEONE_REQUIRE(m > 0 && m <= 16 && n > 0 && k > 0 && k % 8 == 0, "gemm_planes: %d rows (1..16), sizes %d x %d, K a multiple of 8", m, n, k);
+    LEONE_REQUIRE(planes >= 1 && plane_rows > 0 && plane_rows % 16 == 0, "gemm_planes: %d planes, %d rows each (a multiple of 16)", planes, plane_rows);
+    LEONE_REQUIRE(reinterpret_cast<uintptr_t>(x) % 16 == 0 && x_row % 4 == 0 && x_plane % 4 == 0 && x_row >= 0 && x_plane >= 0,
+                  "gemm_planes: float rows %ld apart, planes %ld, are not 16-byte runs", x_row, x_plane);
+    FusedArgs a{};
+    a.x = x, a.w = static_cast<const bf16_t*>(w), a.y = y, a.m = m, a.n = n, a.k = k, a.plane_rows = plane_rows, a.planes = planes;
+    a.x_row = x_row, a.x_plane = x_plane;
+    launch_fused<kInFloats, kOutStore, float>(a, w_tiled != 0, stream);
     LEONE_LAUNCH_CHECK("gemm_planes");
     return 0;
 }

@@ -549,6 +549,9 @@ int leone_heads_in_pairs(int rows, int heads, int write_cache);
 // The weight-streaming product of several inputs against matrices that lie together (see gemm_fused.hip).
 int leone_gemm_planes_bf16(const void* x, int planes, int plane_rows, const void* w, int w_tiled, void* y, int out_dtype, int m,
                            int n, int k, hipStream_t stream);
+// The same from float rows, rounded to bfloat16 as they are read: row r of plane p at x + p * x_plane + r * x_row, 16-byte runs; y float32.
+int leone_gemm_float_planes_bf16(const float* x, long x_row, long x_plane, int planes, int plane_rows, const void* w, int w_tiled, float* y, int m,
+                                 int n, int k, hipStream_t stream);
 // Request slots of many state tensors cleared, copied, saved and put back in one launch (see state_slots.hip).
 int leone_state_chunk();
 int leone_state_slots_max();

@@ -903,14 +903,17 @@ def drop_streamed_copies() -> None:
 
 def gemm_fused(x, weight: torch.Tensor, out_dtype: torch.dtype = torch.bfloat16,
                residual: Optional[torch.Tensor] = None, gated: bool = False, next_norm=None, activation: str = "silu",
-               limit: Optional[float] = None):
+               limit: Optional[float] = None, squared: bool = False):
     """The product for at most 16 rows with its neighbours folded in: ``x`` may be ``NormedRows`` or
     ``PreparedRows``; with ``residual`` the product is added into that float32 tensor and None is returned;
     with ``gated`` the weight is an interleaved gate/up weight and silu(gate) * up comes out.  With
     ``residual`` and ``next_norm = (gain, eps, dtype)`` the kernel also leaves the operand of that norm
-    behind and ``PreparedRows`` is returned (the residual has been added)."""
+    behind and ``PreparedRows`` is returned (the residual has been added).  ``squared`` (a plain product): what ``relu_squared``
+    makes of the result comes out."""
     m, k = x.shape
     n, k2 = weight.shape
+    if squared and (residual is not None or gated):
+        raise KernelError("gemm_fused: the square goes with a plain product")
     if k != k2:
         raise KernelError(f"gemm_fused: inner sizes {k} and {k2} differ")
     prepared = isinstance(x, PreparedRows)
@@ -931,7 +934,7 @@ def gemm_fused(x, weight: torch.Tensor, out_dtype: torch.dtype = torch.bfloat16,
         out, mode, out_dtype = (torch.empty((m, n // 2), dtype=torch.bfloat16, device=weight.device),
                                 (2, 4, 5)[_glu_code(activation, limit)], torch.bfloat16)
     else:
-        out, mode = torch.empty((m, n), dtype=out_dtype, device=weight.device), 0
+        out, mode = torch.empty((m, n), dtype=out_dtype, device=weight.device), 6 if squared else 0
     if prepared:
         source, in_mode = _dev(x.operand, "prepared operand", torch.bfloat16, (m, k)), 2
         _dev(x.squares, "prepared sums", torch.float32, (m, -(-k // 16)))
@@ -1460,6 +1463,31 @@ def linear(x, weight: torch.Tensor, out_dtype: Optional[torch.dtype] = None,
     return swiglu(y, activation=activation, limit=limit) if gated else y
 
 
+def linear_planes_of_floats(x: torch.Tensor, weight: torch.Tensor, rows_of) -> list:
+    """``linear_planes`` of float32 ``x[planes, R, K]`` (a view with any strides, rows in one piece) rounded to the weight's bfloat16; few rows are
+    rounded as the product reads them."""
+    planes, rows, k = x.shape
+    rows_of = [int(r) for r in rows_of]
+    if x.dtype != torch.float32 or weight.dtype != torch.bfloat16 or rows > FUSED_ROWS or not weight.is_cuda or k % 8 or weight.shape[1] != k \
+            or len(rows_of) != planes or sum(rows_of) != weight.shape[0] or not _even_planes(rows_of) \
+            or x.stride(2) != 1 or x.stride(1) % 4 or x.stride(0) % 4 or x.data_ptr() % 16:
+        narrow = torch.empty((planes, rows, k), dtype=weight.dtype, device=x.device)
+        narrow.copy_(x)
+        return linear_planes(narrow, weight, rows_of)
+    tiles = streamed_copy(weight) if _streamed else None
+    out = torch.empty((rows, weight.shape[0]), dtype=torch.float32, device=x.device)
+    with profile.span("gemv fused", weight):
+        call("leone_gemm_float_planes_bf16", x.data_ptr(), x.stride(1), x.stride(0), planes, rows_of[0],
+             _dev(weight if tiles is None else tiles, "gemm weight", torch.bfloat16), 0 if tiles is None else 1, _dev(out, "gemm out"), rows,
+             weight.shape[0], k, _stream())
+    return [out[:, sum(rows_of[:p]):sum(rows_of[:p + 1])] for p in range(planes)]
+
+
+def _even_planes(rows_of) -> bool:
+    """Whether matrices of so many rows, one behind the other, are one launch: equal multiples of 16 rows, the last perhaps smaller."""
+    return rows_of[0] % 16 == 0 and all(r == rows_of[0] for r in rows_of[:-1]) and rows_of[-1] <= rows_of[0]
+
+
 def linear_planes(x: torch.Tensor, weight: torch.Tensor, rows_of) -> list:
     """Products of several inputs ``x[planes, R, K]`` against matrices that lie one behind the other in ``weight[N, K]``
     (``rows_of`` says how many rows each has): a list of float32 ``[R, rows_of[p]]`` = x[p] . weight_p^T, which may be slices
@@ -1472,8 +1500,7 @@ def linear_planes(x: torch.Tensor, weight: torch.Tensor, rows_of) -> list:
     starts = [sum(rows_of[:p]) for p in range(planes)]
     tiles = streamed_copy(weight) if _streamed else None
     any_order = _any_order(weight)
-    if x.dtype == torch.bfloat16 and rows <= FUSED_ROWS and k % 8 == 0 and rows_of[0] % 16 == 0 \
-            and all(r == rows_of[0] for r in rows_of[:-1]) and rows_of[-1] <= rows_of[0]:
+    if x.dtype == torch.bfloat16 and rows <= FUSED_ROWS and k % 8 == 0 and _even_planes(rows_of):
         out = torch.empty((rows, weight.shape[0]), dtype=torch.float32, device=x.device)
         with profile.span("gemv fused", weight):
             call("leone_gemm_planes_bf16", _dev(x, "gemm x", torch.bfloat16), planes, rows_of[0],
@@ -1940,6 +1967,15 @@ def add_bias(x: torch.Tensor, bias: torch.Tensor) -> torch.Tensor:
     n, width = x.shape
     call("leone_add_bias", _dev(x, "rows", torch.float32), _dev(bias, "bias", None, (width,)), _code(bias, "bias"), n, width, _stream())
     return x
+
+
+def linear_relu_squared(x, weight: torch.Tensor) -> torch.Tensor:
+    """``relu_squared(linear(x, weight))``, for few bfloat16 rows in the product's own launch, to the bit."""
+    rows, k = x.shape
+    if x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and weight.is_cuda and k % 8 == 0 and rows <= FUSED_ROWS \
+            and not isinstance(x, NormedRows):
+        return gemm_fused(x, weight, torch.bfloat16, squared=True)
+    return relu_squared(linear(x, weight))
 
 
 def relu_squared(x: torch.Tensor) -> torch.Tensor:

@@ -44,6 +44,7 @@ _PROTOTYPES = {
     "leone_gemm_fused_bf16": [P, c_int, P, P, c_int, c_float, P, c_int, P, c_int, c_int, c_int, c_int, c_int, P, P, P, P,
                               c_int, c_float, P],
     "leone_gemm_planes_bf16": [P, c_int, c_int, P, c_int, P, c_int, c_int, c_int, c_int, P],
+    "leone_gemm_float_planes_bf16": [P, ctypes.c_long, ctypes.c_long, c_int, c_int, P, c_int, P, c_int, c_int, c_int, P],
     "leone_gemm_rows_bf16": [P, P, c_int, P, c_int, c_int, c_int, c_int, c_int, c_int, ctypes.c_long, c_int, c_int, c_float, P],
     "leone_gemm_many_bf16": [P, P, P, c_int, c_int, c_int, c_int, c_int, c_int, ctypes.c_long, c_int, c_int, c_int, c_int, c_float, P],
     "leone_gemm_rows_shape_built": [c_int, c_int, c_int],

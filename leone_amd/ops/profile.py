@@ -30,6 +30,7 @@ OPERATIONS = {
     "leone_attention_prefill": "attention",
     "leone_gemm_fused_bf16": "gemv fused",
     "leone_gemm_planes_bf16": "gemv fused",
+    "leone_gemm_float_planes_bf16": "gemv fused",
     "leone_gemm_rows_bf16": "gemm rows",
     "leone_gemm_many_bf16": "gemm many",
     "leone_gemm_f32": "gemm f32",

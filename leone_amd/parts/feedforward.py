@@ -124,7 +124,7 @@ class ReluSquaredMlp(Part):
         return [self.w_up, self.w_down]
 
     def forward(self, y: torch.Tensor, step: StepContext) -> torch.Tensor:
-        return ops.linear(ops.relu_squared(ops.linear(y, self.w_up)), self.w_down, out_dtype=torch.float32)
+        return ops.linear(ops.linear_relu_squared(y, self.w_up), self.w_down, out_dtype=torch.float32)
 
 
 @FEED_FORWARDS.register("routed_glu")

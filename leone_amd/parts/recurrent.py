@@ -238,9 +238,8 @@ class ChannelDeltaMixer(Part):
         qkv = self.conv.forward(proj[:, :self.conv_width], step, cache["conv"], torch.float32)
         # the two low-rank pairs: their narrow halves came out of the fused product
         if self.w_low is not None and step.dtype == torch.bfloat16:
-            narrow = torch.empty((2, proj.shape[0], self.a_rank), dtype=step.dtype, device=proj.device)
-            narrow.copy_(proj[:, c["a1"]:].unflatten(1, (2, self.a_rank)).transpose(0, 1))
-            step_size, gate = ops.linear_planes(narrow, self.w_low, [self.w_a2.shape[0], self.w_g2.shape[0]])
+            narrow = proj[:, c["a1"]:].unflatten(1, (2, self.a_rank)).transpose(0, 1)
+            step_size, gate = ops.linear_planes_of_floats(narrow, self.w_low, [self.w_a2.shape[0], self.w_g2.shape[0]])
         else:
             step_size = ops.linear(proj[:, c["a1"]:c["g1"]].to(step.dtype).contiguous(), self.w_a2, out_dtype=torch.float32)
             gate = ops.linear(proj[:, c["g1"]:].to(step.dtype).contiguous(), self.w_g2, out_dtype=torch.float32)
