@@ -1117,13 +1117,13 @@ def _takes_many(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype, r
     800 rows 27 and 24, 40 and 40, 45 and 53; 3,072 x 2,048 for 192, 640 and 1,700 rows 15 and 9, 19 and 15, 29 and 27; 6,144 x 4,096 for 256, 640 and
     1,300 rows 30 and 22, 46 and 43, 71 and 88.  Taken together a third faster up to 4 G products of two elements, a seventh at 7 G, a
     fourteenth at 11 G, level at 16 G, behind beyond.  Products that were tuned, or are being noted for it, stay with the library."""
+    if not _streamed or (tiles is None and not _any_order(weight)):
+        return None
     if x.shape[0] * weight.numel() > MANY_MOST or _recorded_products is not None or not _many_fits(x, weight, out_dtype, residual, gated):
         return None
     if _tuned_products and _library_problem(x, weight, torch.float32 if residual is not None else out_dtype, residual is not None) in _tuned_products:
         return None
-    if tiles is not None:
-        return tiles
-    return streamed_copy(weight) if _any_order(weight) else None
+    return streamed_copy(weight) if tiles is None else tiles
 
 
 # Tiles of ``gemm_many`` that read the weight once, four stages ahead, for up to ROWS_MAX rows: (rows, columns): us to start, us a stage of 64
@@ -2354,13 +2354,13 @@ def _check_experts(x: torch.Tensor, w_up: torch.Tensor, w_down: torch.Tensor):
 
 
 def _whole(copies: tuple) -> tuple:
-    return (True,) if copies[0] is not None and copies[1] is not None else ()
+    return (True,) if copies[0] is not None and copies[1] is not None and all(copies[2:]) else ()
 
 
-def _expert_copy(tiles: Optional[torch.Tensor], w: torch.Tensor, pairs_a_tile: int) -> Optional[torch.Tensor]:
+def _expert_copy(tiles: Optional[torch.Tensor], w: torch.Tensor, pairs_a_tile: int, any_order: bool = True) -> Optional[torch.Tensor]:
     """``tiles`` if the product of such tiles of pairs reads the experts' copy (of ``w``, or of more experts that begin with them)."""
     rows, k = w.shape[-2:]
-    if tiles is None or not (pairs_a_tile == 16 or (pairs_a_tile in (64, 128) and k % 64 == 0)):
+    if tiles is None or not (pairs_a_tile == 16 or (any_order and pairs_a_tile in (64, 128) and k % 64 == 0)):
         return None
     if tiles.dtype != torch.bfloat16 or tiles.device != w.device or not tiles.is_contiguous() or tiles.shape[0] < w.shape[0] \
             or tuple(tiles.shape[1:]) != (*w.shape[1:-2], rows // 16, k // 32, 4, 16, 8):
@@ -2384,7 +2384,7 @@ def _expert_products(x, chosen, weight, tiles, w_up, w_down, activation, extra, 
     pair_out = torch.empty((pairs, hidden), dtype=torch.float32, device=device)
 
     def product(rows_in, w, copy, out, pair_weight, kind, n, k, code, held):
-        copy = _expert_copy(copy, w, tile)
+        copy = _expert_copy(copy, w, tile, all(copies[2:]))
         if copy is not None:
             call("leone_moe_product_tiles", _dev(rows_in, "routed rows", torch.bfloat16), _dev(copy, "experts' tiles"), _dev(out, "experts' results"),
                  pair_weight, kind, _dev(tile_expert, "tiles"), _dev(tile_pairs, "tile pairs"), max_tiles, tile, experts, top, n, k, code, held, _stream())
@@ -2409,7 +2409,7 @@ def routed_experts(x: torch.Tensor, chosen: torch.Tensor, weight: torch.Tensor, 
     of ``x``'s type; experts without a gate come as ``[experts, ff, hidden]`` and compute W_down[e] act(W_up[e] x)
     (``PLAIN_ACTIVATIONS``).  ``weigh_input`` (experts without a gate): the weight multiplies what the expert reads
     instead of what it gives.  ``paired``: the sum is left to the consumer (``PairedRows``).  ``copies``: ``tile_experts`` of both
-    matrices (None: none), which the products read instead.  Nothing here depends on the choice except through device arrays."""
+    matrices (None: none), which the products read instead; with a third, False, those products alone whose sums keep their order.  Nothing here depends on the choice except through device arrays."""
     rows, hidden, experts, ff, _ = _check_experts(x, w_gate_up, w_down)
     top = chosen.shape[1]
     tiles = _expert_tiles(x, rows, top, experts, hidden, ff, *_whole(copies))

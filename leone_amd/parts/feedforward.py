@@ -232,8 +232,8 @@ class RoutedGluMlp(Part):
         fits = all(w is not None and w.is_cuda and w.dtype == torch.bfloat16 and w.shape[-2] % 16 == 0 and w.shape[-1] % 32 == 0 for w in both)
         return 2 * sum(w.numel() for w in both) if fits else 0
 
-    def keep_expert_copies(self) -> None:
-        self.copies = (ops.tile_experts(self.w_gate_up_all), ops.tile_experts(self.w_down_all))
+    def keep_expert_copies(self, any_order: bool = True) -> None:
+        self.copies = (ops.tile_experts(self.w_gate_up_all), ops.tile_experts(self.w_down_all), any_order)
 
     def forward(self, y: torch.Tensor, step: StepContext, paired: bool = False):
         y = ops.materialize(y)

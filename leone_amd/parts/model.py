@@ -171,7 +171,8 @@ class DecoderModel:
         are the same bit for bit (of more, sums may be in another order, but not in a model that carries memories); a decode step of few rows takes a sixth less time; the weights take twice the memory.
         ``wanted`` None decides by room: yes if the copies take at most a quarter of the device's memory
         and half of what is free.  Routed experts get theirs (``ops.tile_experts``) behind these, all or none, if there is room for
-        both; their products of many pairs then run on a kernel of their own, with sums in its order.  Returns the bytes the copies take (0: none kept).  Asked again, it answers what it did the first time."""
+        both; their products of many pairs then run on a kernel of their own, with sums in its order (not in a model that carries
+        memories).  Returns the bytes the copies take (0: none kept).  Asked again, it answers what it did the first time."""
         if self.streamed_copy_bytes is not None:
             return self.streamed_copy_bytes
         self.streamed_copy_bytes = 0
@@ -191,7 +192,7 @@ class DecoderModel:
         self.streamed_copy_bytes = sum(ops.keep_streamed_copy(w, any_order) for w in weights)
         if experts and needed + of_experts <= room:
             for part in experts:
-                part.keep_expert_copies()
+                part.keep_expert_copies(any_order)
             self.streamed_copy_bytes += of_experts
         return self.streamed_copy_bytes
 

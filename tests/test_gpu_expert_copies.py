@@ -116,3 +116,17 @@ def test_many_pairs(mode, experts, rows, top, hidden, ff):
     if ops._expert_tiles(x, rows, chosen.shape[1], experts, hidden, ff, True)[0] == ops._expert_tiles(x, rows - 3, chosen.shape[1], experts, hidden, ff, True)[0]:
         assert torch.equal(ops.routed_experts(x[some].contiguous(), chosen[some].contiguous(), weight[some].contiguous(), up, down, copies=copies, **options),
                            got[some])
+
+
+@pytest.mark.parametrize("experts,rows,top,hidden,ff", [(4, 3, 1, 64, 64), (4, 45, 2, 128, 64), (3, 700, 2, 2048, 832)])
+def test_copies_for_sums_in_their_old_order(experts, rows, top, hidden, ff):
+    """Few pairs, tiles of 64 and of 128: the bits of the products from the matrices themselves, whatever reads the copies."""
+    from leone_amd import ops
+    gen = torch.Generator(device=DEV).manual_seed(rows)
+    chosen = torch.rand(rows, experts, generator=gen, device=DEV).topk(top, dim=1).indices.to(torch.int32).contiguous()
+    weight = torch.rand(rows, top, generator=gen, device=DEV) + 0.1
+    x = torch.randn(rows, hidden, generator=gen, device=DEV).bfloat16()
+    up = (torch.randn(experts, 2, ff, hidden, generator=gen, device=DEV) / math.sqrt(hidden)).bfloat16()
+    down = (torch.randn(experts, hidden, ff, generator=gen, device=DEV) / math.sqrt(ff)).bfloat16()
+    copies = (ops.tile_experts(up), ops.tile_experts(down), False)
+    assert torch.equal(ops.routed_experts(x, chosen, weight, up, down, copies=copies), ops.routed_experts(x, chosen, weight, up, down))
