@@ -1470,7 +1470,7 @@ def linear_planes_of_floats(x: torch.Tensor, weight: torch.Tensor, rows_of) -> l
     rows_of = [int(r) for r in rows_of]
     if x.dtype != torch.float32 or weight.dtype != torch.bfloat16 or rows > FUSED_ROWS or not weight.is_cuda or k % 8 or weight.shape[1] != k \
             or len(rows_of) != planes or sum(rows_of) != weight.shape[0] or not _even_planes(rows_of) \
-            or x.stride(2) != 1 or x.stride(1) % 4 or x.stride(0) % 4 or x.data_ptr() % 16:
+            or x.device != weight.device or x.stride(2) != 1 or x.stride(1) % 4 or x.stride(0) % 4 or x.data_ptr() % 16:
         narrow = torch.empty((planes, rows, k), dtype=weight.dtype, device=x.device)
         narrow.copy_(x)
         return linear_planes(narrow, weight, rows_of)

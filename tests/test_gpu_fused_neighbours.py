@@ -40,3 +40,10 @@ def test_rounding_ahead_of_products_side_by_side(rows, parts, k):
         want = ops.linear_planes(x.bfloat16().contiguous(), w, parts)
         got = ops.linear_planes_of_floats(x, w, parts)
         assert len(got) == len(want) and all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+def test_floats_that_lie_elsewhere_are_refused():
+    """The kernel gets no address that the device does not have: what is on the host is refused, as by ``linear_planes``."""
+    w = some(64, 32, seed=7).bfloat16()
+    with pytest.raises(ops.KernelError, match="on cpu"):
+        ops.linear_planes_of_floats(some(2, 3, 32, seed=8).cpu(), w, [32, 32])
