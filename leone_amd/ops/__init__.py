@@ -758,9 +758,15 @@ FOLDED_F32_ROWS = 8          # most rows of a float32 product that carries out i
 FOLDED_F32_NORM_ELEMENTS = 12 << 20
 
 
+def _apart(a: torch.Tensor, b: torch.Tensor) -> bool:
+    """Whether two tensors in one piece share no memory."""
+    return a.data_ptr() + a.numel() * a.element_size() <= b.data_ptr() or b.data_ptr() + b.numel() * b.element_size() <= a.data_ptr()
+
+
 def _folds_f32(x, weight: torch.Tensor, residual: Optional[torch.Tensor], gated: bool) -> bool:
     """Whether the float32 product of few rows does its neighbour in its own launch (``gemm_f32_folded``): the norm of ``x``
-    (``NormedRows`` of the whole stream under float gains), or the sum into ``residual``.  Everything else stays as it is."""
+    (``NormedRows`` of the whole stream under float gains), or the sum into ``residual``, unless that is what the product reads, which
+    workgroups that are done would change under the others.  Everything else stays as it is."""
     rows, k = x.shape
     normed = isinstance(x, NormedRows)
     if rows > FOLDED_F32_ROWS or not weight.is_cuda or not weight.is_contiguous() or weight.data_ptr() % 16 \
@@ -772,7 +778,8 @@ def _folds_f32(x, weight: torch.Tensor, residual: Optional[torch.Tensor], gated:
                 and x.x.is_contiguous() and x.gain.is_contiguous() and x.x.data_ptr() % 16 == 0 and x.gain.data_ptr() % 16 == 0
                 and (not gated or n % 16 == 0) and bool(library().leone_gemm_f32_folds(rows, n, k, 2)))
     return (residual is not None and residual.dtype == torch.float32 and tuple(residual.shape) == (rows, n) and residual.is_contiguous()
-            and x.is_contiguous() and x.data_ptr() % 16 == 0 and bool(library().leone_gemm_f32_folds(rows, n, k, 1)))
+            and x.is_contiguous() and x.data_ptr() % 16 == 0 and residual.device == weight.device and _apart(residual, x)
+            and _apart(residual, weight) and bool(library().leone_gemm_f32_folds(rows, n, k, 1)))
 
 
 def gemm_f32_folded(x, weight: torch.Tensor, residual: Optional[torch.Tensor] = None, gated: bool = False, activation: str = "silu",
@@ -786,6 +793,8 @@ def gemm_f32_folded(x, weight: torch.Tensor, residual: Optional[torch.Tensor] = 
     normed = isinstance(x, NormedRows)
     if normed == (residual is not None) or (gated and not normed):
         raise KernelError("gemm_f32_folded: either a norm goes ahead of the product or it is added into the stream")
+    if residual is not None and not (_apart(residual, x) and _apart(residual, weight)):
+        raise KernelError("gemm_f32_folded: the product cannot be added into what it is made of")
     out = residual if residual is not None else torch.empty((rows, n // 2 if gated else n), dtype=torch.float32, device=weight.device)
     with profile.span("gemm f32", weight):
         call("leone_gemm_f32_folded", _dev(x.x if normed else x, "gemm a", torch.float32, (rows, k)), _dev(weight, "gemm b", torch.float32),

@@ -86,3 +86,19 @@ def test_eight_columns_a_workgroup_give_the_bits_of_many_rows(n, k):
     many = ops.gemm_f32(a, b).nan_to_num(7.5, 8.5, 9.5)
     for m in (1, 3, 8):
         assert torch.equal(ops.gemm_f32(a[:m].contiguous(), b).nan_to_num(7.5, 8.5, 9.5), many[:m]), m
+
+
+def test_a_product_is_not_added_into_what_it_reads():
+    """The stream is the product's own operand, or overlaps it: the product comes back and the stream is as it was."""
+    from leone_amd import ops
+    x, w, _, _ = drawn(12, 512, 512, 6)
+    kept = x.clone()
+    for rows, stream in ((x[:8], x[:8]), (x[:8], x[2:10]), (x[3:8], x[:5])):
+        want = ops.gemm_f32(rows, w)
+        assert torch.equal(ops.linear(rows, w, residual=stream), want) and torch.equal(x, kept)
+        with pytest.raises(ops.KernelError, match="made of"):
+            ops.gemm_f32_folded(rows, w, stream)
+    assert ops.linear(x[:4], w, residual=x[4:8]) is None and torch.equal(x[4:8], kept[4:8] + ops.gemm_f32(kept[:4], w))
+    few = w[:8]                                            # the matrix itself
+    assert torch.equal(ops.linear(kept[:8], w, residual=few), ops.gemm_f32(kept[:8], w))
+    assert isinstance(ops.linear(kept[:8], w, residual=torch.zeros(8, 512)), torch.Tensor)          # a stream that lies elsewhere
