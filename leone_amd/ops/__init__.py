@@ -1082,15 +1082,18 @@ def gemm_rows(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype = to
 MANY_TILES = ((64, 128, 2.1, 0.277), (96, 128, 2.6, 0.332), (128, 128, 2.8, 0.40), (96, 256, 3.2, 0.533))
 MANY_LEAST = 1024            # fewest rows and columns of a weight ``gemm_many`` is asked for
 MANY_MOST = 10 << 30         # most products of two elements it is asked for
+STREAM_MOST = 8192           # widest stream it leaves planes for: widths the norms behind it were measured at
 
 
 @functools.lru_cache(maxsize=4096)
 def many_plan(m: int, n: int, k: int, may_split: bool, units: int = 256) -> tuple[int, int, int]:
-    """(rows, columns, ranges of K) of a workgroup of ``gemm_many``.  Its time is a start and then, a stage of 64 elements of K, so
-    much for every tile that falls to one compute unit (``MANY_TILES``: rows, columns, us to start, us a stage; fitted to 700 measured
-    products a tile, 129 to 2,048 rows of 1,024 to 4,096 wide layers, standing off by 12 %); planes cost half a microsecond a megabyte,
-    written and read.  What is chosen so is within 1 % of the best of the four tiles and 1 to 4 ranges on average, 22 % at worst; tiles of
-    64 x 256 and 128 x 256 as well would gain less than half a percent."""
+    """(rows, columns, ranges of K) of a workgroup of ``gemm_many``.  Its time is taken for a start and then, a stage of 64 elements of K, so
+    much for every tile that falls to one compute unit (``MANY_TILES``: rows, columns, us to start, us a stage; fitted to 700 products
+    whose weights lay in the caches); planes for 0.6 us a megabyte, written and read.  It ranks tiles and ranges and is no estimate of the time: from
+    memory, and with all units multiplying, products take up to twice as long (over estimate, on average: 1.1 into the stream, 1.6 gated
+    or stored).  With the norm behind it, weights from memory, what is chosen into the stream is within 1 % of the best of the four tiles and 1 to 4
+    ranges on average, 9 % at worst (121 products, 144 to 1,500 rows; at 0.48 us a megabyte 1 % and 15 %, 8 of them behind the
+    library, now 4)."""
     stages = k // 64
     best = None
     for rows, columns, start, stage in MANY_TILES:
@@ -1099,10 +1102,37 @@ def many_plan(m: int, n: int, k: int, may_split: bool, units: int = 256) -> tupl
             per = -(-stages // splits)
             if per * (splits - 1) >= stages:            # a range would be empty
                 continue
-            cost = start + stage * per * -(-tiles * splits // units) + (0.48e-6 * 4 * m * n * splits if may_split else 0.0)
+            cost = start + stage * per * -(-tiles * splits // units) + (0.6e-6 * 4 * m * n * splits if may_split else 0.0)
             if best is None or cost < best[0]:
                 best = (cost, rows, columns, splits)
     return best[1:]
+
+
+@functools.lru_cache(maxsize=4096)
+def many_pays(m: int, n: int, k: int, into_stream: bool, gated: bool, units: int = 256) -> bool:
+    """Whether a product of more than ROWS_MAX rows is faster with ``gemm_many`` than in the library.
+
+    Into the stream (its planes fill the units) up to MANY_MOST, see ``_takes_many``.  Otherwise K is in one range, and a workgroup's chain of
+    stages takes its time however few workgroups there are, where the library cuts K: from a K of 1,024 on there have to be more of them
+    the longer K is.  us, library and ``gemm_many``, weights from memory: stored, 1,024 x 4,096 for 256 rows (32 workgroups) 11.6 and 21.2, 1,216 x
+    6,912 for 174 (30) 17.8 and 40.6, 2,304 x 1,536 for 160 and 512 (54 and 144) 9.1 and 10.1, 14.5 and 10.9, 4,608 x 3,072 for 320 (180) 20.0 and 22.8,
+    2,048 x 1,024 for 129 (48) 10.1 and 7.1; gated, which saves a launch, 1,408 x 4,352 for 273 (55) 19.1 and 27.7, 2,816 x 2,048 for 129 (66)
+    14.4 and 13.9.  Stored products of more workgroups than units are level, and where small tiles give many rounds behind (6,144 x 1,152 for
+    1,024 rows, 768 of 64 x 128, 20.0 and 24.4; 4,096 x 1,536 for 1,700, 448 of 128 x 128, 1.01 times as fast).  And tiles of 96 x 256 have to fill their
+    last round: gated 8,192 x 2,048 for 576 rows (192) 32.3 and 35.3, 13,824 x 2,304 for 288 (162) 35.8 and 39.7, 12,288 x 2,048 for 420
+    (240) 36.6 and 35.1.  Of 1,623 stored products measured 718 are on this side of the line, 11 of them 3 to 7 % behind the library; of 536 gated ones
+    418, one (6 %)."""
+    if m * n * k > MANY_MOST:
+        return False
+    if into_stream:
+        return n <= STREAM_MOST
+    rows, columns, _ = many_plan(m, n, k, False, units)
+    groups = -(-m // rows) * -(-n // columns)
+    if columns > 128 and 16 * groups < 15 * units * -(-groups // units):
+        return False
+    if not gated and groups > units:
+        return False
+    return k <= 1024 or groups >= (max(units // 4, k // 24) if gated else max(units // 2, k // 16))
 
 
 def _many_fits(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype, residual: Optional[torch.Tensor], gated: bool) -> bool:
@@ -1120,15 +1150,15 @@ def _takes_many(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype, r
                 gated: bool, tiles: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
     """The weight's tiled copy (``tiles`` where it is not kept under the weight itself) if ``gemm_many`` is the faster for this product of many rows; None leaves it to the library.
 
-    The line lies where both were measured, us, library and ``gemm_many``: into the stream 2,048 x 6,144 for 129, 513 and 1,300 rows
-    26 and 15, 30 and 22, 47 and 43; 4,096 x 4,096 for 160, 384, 800 and 1,300 rows 26 and 15, 26 and 23, 46 and 44, 57 and 60; 1,024 x 3,072 for
-    300 and 1,700 rows 14 and 9, 28 and 23; gated 6,144 x 1,024 for 256, 640 and 1,300 rows 18 and 10, 20 and 15, 29 and 25 and 12,288 x 2,048 for 300, 640 and
-    800 rows 27 and 24, 40 and 40, 45 and 53; 3,072 x 2,048 for 192, 640 and 1,700 rows 15 and 9, 19 and 15, 29 and 27; 6,144 x 4,096 for 256, 640 and
-    1,300 rows 30 and 22, 46 and 43, 71 and 88.  Taken together a third faster up to 4 G products of two elements, a seventh at 7 G, a
-    fourteenth at 11 G, level at 16 G, behind beyond.  Products that were tuned, or are being noted for it, stay with the library."""
+    us, library and ``gemm_many``, weights from memory, with the norm behind them: into the stream 2,048 x 6,144 for 129, 512 and 800 rows
+    23.6 and 15.8, 33.8 and 26.3, 42.8 and 35.3; 4,096 x 4,096 for 160, 384 and 640 rows 31 and 20, 31 and 29, 42.3 and 41.2; 1,024 x 3,072 for
+    320 and 1,700 rows 17.1 and 13.1, 26.3 and 24.0.  A fifth faster on average over 451 products of up to 10 G of two elements (19 %
+    up to 2 G, 15 % from 7 G on), 4 to 6 % behind in 6 of them (2,048 x 2,048 for 720 rows 19.1 and 20.1).  Others: ``many_pays``.  Products that were
+    tuned, or are being noted for it, stay with the library."""
     if not _streamed or (tiles is None and not _any_order(weight)):
         return None
-    if x.shape[0] * weight.numel() > MANY_MOST or _recorded_products is not None or not _many_fits(x, weight, out_dtype, residual, gated):
+    if _recorded_products is not None or not _many_fits(x, weight, out_dtype, residual, gated) \
+            or not many_pays(x.shape[0], *weight.shape, residual is not None, gated, compute_units(weight.device)):
         return None
     if _tuned_products and _library_problem(x, weight, torch.float32 if residual is not None else out_dtype, residual is not None) in _tuned_products:
         return None

@@ -54,14 +54,14 @@ def test_rows_beyond_the_matrices_are_not_written():
         assert ((held[1:-1].double() - 7 - want).abs() <= bound + 2.0 ** -23 * (want.abs() + 7)).all()
 
 
-@pytest.mark.parametrize("m, n, k", [(129, 1024, 1024), (300, 1040, 4096), (640, 3072, 1088)])
+@pytest.mark.parametrize("m, n, k", [(129, 1024, 1024), (300, 1040, 4096), (640, 3072, 1088), (300, 3600, 2112)])
 def test_products_with_a_copy_take_it_and_agree_with_those_without(m, n, k):
     x, weight, tiles, want, bound = _operands(m, n, k)
     plain = ops.linear(x, weight, out_dtype=torch.float32)
     gated = ops.linear(x, weight, gated=True)
     try:
         ops.keep_streamed_copy(weight)
-        assert ops._takes_many(x, weight, torch.float32, None, False) is not None
+        assert (ops._takes_many(x, weight, torch.float32, None, False) is not None) == ops.many_pays(m, n, k, False, False) == (n != 1040)
         assert ((ops.linear(x, weight, out_dtype=torch.float32).double() - want).abs() <= bound).all()
         assert ((plain.double() - want).abs() <= bound).all()
         stream = torch.zeros((m, n), device="cuda")
@@ -75,11 +75,32 @@ def test_products_with_a_copy_take_it_and_agree_with_those_without(m, n, k):
         assert ((half - gated.double()).abs() <= 2.0 ** -7 * (half.abs() + want.abs().amax() ** 2 * 2 + 1e-6)).all()
         # what it does not take stays with the library: other layouts, other types, products being noted
         assert ops._takes_many(x[:, ::2], weight[:, :k // 2], torch.float32, None, False) is None
-        assert ops._takes_many(x, weight, torch.float16, None, False) is None
+        assert ops._takes_many(x, weight, torch.float16, torch.zeros((m, n), device="cuda"), False) is None
         assert ops._takes_many(x, weight, torch.float32, torch.zeros((n, m), device="cuda").t(), False) is None
         with ops.record_library_products() as seen:
             ops.linear(x, weight, out_dtype=torch.float32)
         assert len(seen.problems) == 1
+    finally:
+        ops.drop_streamed_copies()
+
+
+@pytest.mark.parametrize("m, n, k, gated, takes", [
+    (256, 1024, 4096, False, False), (174, 1216, 6912, False, False), (160, 2304, 1536, False, False), (512, 2304, 1536, False, True),
+    (320, 4608, 3072, False, False), (129, 2048, 1024, False, True), (640, 8192, 2048, False, False), (1024, 6144, 1024, False, False),
+    (273, 1408, 4352, True, False), (129, 2816, 2048, True, True), (576, 8192, 2048, True, False), (420, 12288, 2048, True, True),
+])
+def test_products_in_one_range_whose_workgroups_are_few_stay_with_the_library(m, n, k, gated, takes):
+    """A workgroup walks all of K: where there are few, or the widest tiles leave a round of units half empty, the library is ahead.  Into the
+    stream, where planes fill the units, the copy is taken."""
+    x, weight = torch.randn((m, k), device="cuda").bfloat16(), (torch.randn((n, k), device="cuda") / k ** 0.5).bfloat16()
+    kind = torch.bfloat16 if gated else torch.float32
+    plain = ops.linear(x, weight, out_dtype=kind, gated=gated)
+    try:
+        ops.keep_streamed_copy(weight)
+        assert (ops._takes_many(x, weight, kind, None, gated) is not None) == takes
+        if not takes:
+            assert torch.equal(ops.linear(x, weight, out_dtype=kind, gated=gated), plain)
+        assert gated or m * n * k > ops.MANY_MOST or ops._takes_many(x, weight, kind, torch.zeros((m, n), device="cuda"), False) is not None
     finally:
         ops.drop_streamed_copies()
 
