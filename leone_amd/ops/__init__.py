@@ -1116,8 +1116,8 @@ def many_pays(m: int, n: int, k: int, into_stream: bool, gated: bool, units: int
     stages takes its time however few workgroups there are, where the library cuts K: from a K of 1,024 on there have to be more of them
     the longer K is.  us, library and ``gemm_many``, weights from memory: stored, 1,024 x 4,096 for 256 rows (32 workgroups) 11.6 and 21.2, 1,216 x
     6,912 for 174 (30) 17.8 and 40.6, 2,304 x 1,536 for 160 and 512 (54 and 144) 9.1 and 10.1, 14.5 and 10.9, 4,608 x 3,072 for 320 (180) 20.0 and 22.8,
-    2,048 x 1,024 for 129 (48) 10.1 and 7.1; gated, which saves a launch, 1,408 x 4,352 for 273 (55) 19.1 and 27.7, 2,816 x 2,048 for 129 (66)
-    14.4 and 13.9.  Stored products of more workgroups than units are level, and where small tiles give many rounds behind (6,144 x 1,152 for
+    2,048 x 1,024 for 129 (48) 10.1 and 7.1; gated, which saves a launch, 1,408 x 4,352 for 273 (55) 19.1 and 27.7, 2,816 x 2,048 for 200 (88)
+    15.4 and 14.1.  Stored products of more workgroups than units are level, and where small tiles give many rounds behind (6,144 x 1,152 for
     1,024 rows, 768 of 64 x 128, 20.0 and 24.4; 4,096 x 1,536 for 1,700, 448 of 128 x 128, 1.01 times as fast).  And tiles of 96 x 256 have to fill their
     last round: gated 8,192 x 2,048 for 576 rows (192) 32.3 and 35.3, 13,824 x 2,304 for 288 (162) 35.8 and 39.7, 12,288 x 2,048 for 420
     (240) 36.6 and 35.1.  Of 1,623 stored products measured 718 are on this side of the line, 11 of them 3 to 7 % behind the library; of 536 gated ones
