@@ -1172,7 +1172,7 @@ DEEP_TILES = {(32, 64): (2.411, 0.197, 6.777, 0.331, 0.827, 0.637), (32, 96): (2
               (64, 64): (2.678, 0.252, 6.785, 0.245, 1.268, 0.545), (64, 96): (2.740, 0.276, 6.927, 0.288, 1.470, 0.620),
               (64, 128): (2.762, 0.376, 6.775, 0.244, 1.567, 0.411), (96, 128): (3.225, 0.418, 6.516, 0.209, 1.395, 0.673),
               (128, 128): (3.654, 0.456, 6.025, 0.186, 1.508, 0.666)}
-DEEP_GATED_MOST = 25 << 20   # most elements of a gated weight that they are asked for with more than 64 rows
+DEEP_WHOLE_MOST = 25 << 20   # most elements of a weight that they are asked for with more than 64 rows and one range of K whatever else its sizes say
 
 
 @functools.lru_cache(maxsize=4096)
@@ -1200,25 +1200,11 @@ def deep_plan(m: int, n: int, k: int, may_split: bool, gated: bool, units: int =
     return (*best[1:], True)
 
 
-def _takes_deep(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype, residual: Optional[torch.Tensor],
-                gated: bool, tiles: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
-    """The weight's tiled copy (``tiles`` where it is not kept under the weight itself) if ``gemm_many`` is the faster for this product of
-    more than FUSED_ROWS and up to ROWS_MAX rows; None leaves it to ``gemm_rows``.
-
-    us, ``gemm_rows`` and ``gemm_many`` with ``deep_plan``, weights from memory, 17, 64 and 128 rows: planes of 6,144 x 4,096 12.4 and 10.7, 16.3 and
-    12.1, 21.5 and 17.4; of 4,096 x 12,288 21.2 and 19.3, 24.4 and 21.3, 32.2 and 24.5; of 2,048 x 2,048 4.9 and 4.2, 6.6 and 5.0, 9.8 and 6.8; logits
-    of 32,768 x 4,096 58 and 46, 54 and 49, 65 and 63; of 32,768 x 1,024 20 and 14, 24 and 15, 27 and 20; gated 12,288 x 2,048 15.1 and 13.6, 17.6 and
-    14.8, 22.7 and 19.0, 6,144 x 1,024 7.8 and 7.2, 10.4 and 9.1, 15.3 and 9.1, 24,576 x 4,096 39.3 and 36.6, 40.3 and 37.3.  Over the shapes measured planes are
-    1.28 times as fast (0.94 at the least), logits 1.27 (0.99), gated products of up to 64 rows 1.06 (0.97); of more rows the larger gated weights,
-    whose units are all at work either way, are behind (24,576 x 4,096 for 96 and 128 rows 44 and 45, 48 and 49, 18,432 x 3,072 30 and 34, 35 and 39)."""
-    found = _deep_choice(x, weight, out_dtype, residual, gated, False, tiles)
-    return None if found is None else found[0]
-
-
 def _deep_choice(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype, residual: Optional[torch.Tensor], gated: bool,
                  may_split: bool, tiles: Optional[torch.Tensor] = None) -> Optional[tuple]:
-    """(tiled copy, plan) if ``_takes_deep``; what sizes and types say is kept beside the copy, since steps that are not recorded wait
-    for the host (a microsecond a product)."""
+    """The weight's tiled copy (``tiles`` where it is not kept under the weight itself) and the plan if ``gemm_many`` is the faster for this
+    product of more than FUSED_ROWS and up to ROWS_MAX rows; None leaves it to ``gemm_rows``.  What sizes and types say (``_deep_sizes``)
+    is kept beside the copy, since steps that are not recorded wait for the host (a microsecond a product)."""
     m, n = x.shape[0], weight.shape[0]
     if tiles is None:
         held = _streamed.get((weight.data_ptr(), weight.shape))
@@ -1239,10 +1225,33 @@ def _deep_choice(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype, 
 
 
 def _deep_sizes(m: int, n: int, k: int, may_split: bool, gated: bool, out_dtype: torch.dtype, units: int) -> Optional[tuple]:
+    """The plan of a product of FUSED_ROWS to ROWS_MAX rows if ``gemm_many`` takes such sizes and is faster than ``gemm_rows``, whose waves share
+    K out.
+
+    Planes: always, up to the widest stream that was measured (us, ``gemm_rows`` and ``gemm_many`` with ``deep_plan``, weights from memory, 17, 64 and 128 rows:
+    6,144 x 4,096 14.0 and 11.8, 17.5 and 14.0, 23.8 and 19.5; 2,048 x 2,048 5.6 and 4.5, 8.1 and 6.1, 12.5 and 7.0; 4,096 x 1,024
+    5.5 and 4.5, 8.1 and 6.0, 12.5 and 7.4; 1.03 times as fast at the least; but with the norm behind it 9,024 x 3,264 for 46 rows 38 and 56).
+    In one range of K a workgroup's chain of stages bounds few workgroups: up to 48 rows it takes longer than in ``gemm_rows`` unless K is
+    short or the units are at work (stored, 17 and 33 rows: 1,024 x 8,192 26.5 and 30.3, 29.3 and 33.6, 4,096 x 4,096 16.5 and 17.4, 17.8 and 19.0; 4,096 x 2,048 9.7
+    and 9.5, 10.7 and 10.5, 16,384 x 2,048 17.4 and 13.5, 18.1 and 13.8, 1,024 x 1,024 5.8 and 5.5, 6.9 and 6.4; gated, whose gate and up share a tile, 4,096 x
+    4,096 17.6 and 18.6, 19.1 and 21.2, 2,048 x 2,048 10.3 and 10.3, 11.6 and 12.3, 8,192 x 2,048 12.9 and 11.4, 14.4 and 13.4, 24,576 x 4,096 39 and 37 for 17).
+    Beyond 64 rows the larger matrices are behind where the weight is asked for twice or units are idle (14,912 x 5,760 for 66 rows 37 and 51, 19,264 x 5,120 for 95 43 and
+    49; 32,768 x 4,096 for 65 and 128 1.23 and 1.28 times as fast, 6,528 x 5,120 for 92 1.19), and gated ones altogether (24,576 x 4,096 for 96 and 128 rows 44 and 45, 48 and
+    49).  Of 889 products in one range measured 645 are on this side of the line, 1.22 times as fast on average, 0.95 at the least (without it 156 were more than 3 % behind)."""
     if not FUSED_ROWS < m <= ROWS_MAX or k % 64 or n % 16 or n < MANY_LEAST or k < MANY_LEAST or out_dtype not in _CODES \
-            or (gated and (out_dtype != torch.bfloat16 or (m > 64 and n * k > DEEP_GATED_MOST))):
+            or (gated and out_dtype != torch.bfloat16) or (may_split and not gated and n > STREAM_MOST):
         return None
-    return deep_plan(m, n, k, may_split and not gated, gated, units)
+    plan = deep_plan(m, n, k, may_split and not gated, gated, units)
+    if may_split and not gated:
+        return plan
+    rows, columns = plan[:2]
+    groups = -(-m // rows) * -(-n // columns)
+    full = 8 * groups >= 7 * units
+    if m <= 48:
+        pays = k <= 1024 or full or (k <= 2048 and (not gated or 8 * groups >= 3 * units))
+    else:
+        pays = m <= 64 or n * k <= DEEP_WHOLE_MOST or (not gated and (k <= 2048 or columns == 64 or (full and rows >= m)))
+    return plan if pays else None
 
 
 def gemm_many(x: torch.Tensor, tiles: torch.Tensor, n: int, out_dtype: torch.dtype = torch.bfloat16, residual: Optional[torch.Tensor] = None,
@@ -1433,7 +1442,7 @@ def linear(x, weight: torch.Tensor, out_dtype: Optional[torch.dtype] = None,
 
     float32 runs the single-precision kernel.  bfloat16 accumulates in float: up to FUSED_ROWS rows on the
     weight-streaming kernel with everything folded in, up to ROWS_MAX rows (a decode step of many requests)
-    on the multi-row weight-streaming kernel or from the weight's tiled copy (``_takes_deep``), more rows (prompt portions) on the kernel for many rows where the weight has a
+    on the multi-row weight-streaming kernel or from the weight's tiled copy (``_deep_choice``), more rows (prompt portions) on the kernel for many rows where the weight has a
     tiled copy and that kernel is the faster (``_takes_many``), else through the library's matrix
     product, with float32 output for logits and for what goes into the stream.
     """

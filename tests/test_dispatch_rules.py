@@ -33,3 +33,19 @@ def test_gates_in_runs(lib, kind, each, n, runs):
                                                    (8, 1, 2049, 4096, 0), (32, 1, 768, 2048, 0), (8, 1, 2048, 5120, 0), (4, 1, 2048, 4096, 0), (32, 1, 512, 4096, 0)])
 def test_chunks_of_experts_matrices_on_their_way(lib, experts, gated, n, k, one):
     assert lib.leone_moe_one_chunk_ahead(experts, gated, n, k) == one
+
+
+@pytest.mark.parametrize("m, n, k, kind, takes", [
+    (17, 1024, 8192, "store", False), (48, 4096, 4096, "store", False), (49, 4096, 4096, "store", True), (33, 4096, 2048, "store", True),
+    (33, 1024, 1024, "gated", True), (33, 2048, 2048, "gated", False), (33, 6144, 2048, "gated", True), (17, 24576, 4096, "gated", True), (33, 4096, 4096, "gated", False),
+    (66, 14912, 5760, "store", False), (95, 19264, 5120, "store", False), (65, 32768, 4096, "store", True), (92, 6528, 5120, "store", True), (96, 24576, 4096, "gated", False),
+    (17, 1024, 8192, "planes", True), (46, 9024, 3264, "planes", False), (128, 8192, 1024, "planes", True),
+])
+def test_which_products_of_up_to_128_rows_take_the_copy(m, n, k, kind, takes):
+    """In one range of K few workgroups walk all of it, which the waves of ``gemm_rows`` share; large matrices are not read twice."""
+    import torch
+
+    from leone_amd import ops
+    kind_of = torch.bfloat16 if kind == "gated" else torch.float32
+    plan = ops._deep_sizes(m, n, k, kind == "planes", kind == "gated", kind_of, 256)
+    assert (plan is not None) == takes and (plan is None or plan == ops.deep_plan(m, n, k, kind == "planes", kind == "gated"))

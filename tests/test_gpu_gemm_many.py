@@ -137,10 +137,10 @@ def test_every_deep_tile_and_output(tile, m, n, k, splits):
 def test_products_of_up_to_128_rows_take_the_copy(m, n, k):
     x, weight, tiles, want, bound = _operands(m, n, k)
     plain, gated = ops.linear(x, weight, out_dtype=torch.float32), ops.linear(x, weight, gated=True).double()
-    assert ops._takes_deep(x, weight, torch.float32, None, False) is None                  # there is none yet
+    assert ops._deep_choice(x, weight, torch.float32, None, False, False) is None                  # there is none yet
     try:
         ops.keep_streamed_copy(weight)
-        assert ops._takes_deep(x, weight, torch.float32, None, False) is not None
+        assert ops._deep_choice(x, weight, torch.float32, None, False, False) is not None
         for got in (plain, ops.linear(x, weight, out_dtype=torch.float32)):
             assert ((got.double() - want).abs() <= bound).all()
         for stream in (torch.zeros((m, n), device="cuda"), None):
@@ -151,9 +151,9 @@ def test_products_of_up_to_128_rows_take_the_copy(m, n, k):
         # the results of both round once, from sums that differ by their bounds at the most
         both = ops.linear(x, weight, gated=True).double()
         assert ((both - gated).abs() <= 2.0 ** -7 * both.abs() + 4 * bound.amax() * (1 + want.abs().amax())).all()
-        assert ops._takes_deep(x[:, ::2], weight[:, :k // 2], torch.float32, None, False) is None
-        assert ops._takes_deep(x[:16], weight, torch.float32, None, False) is None
-        assert ops._takes_deep(x, weight, torch.float32, torch.zeros((n, m), device="cuda").t(), False) is None
+        assert ops._deep_choice(x[:, ::2], weight[:, :k // 2], torch.float32, None, False, False) is None
+        assert ops._deep_choice(x[:16], weight, torch.float32, None, False, False) is None
+        assert ops._deep_choice(x, weight, torch.float32, torch.zeros((n, m), device="cuda").t(), False, True) is None
         pieces = ops.linear_planes(torch.stack([x, x]), weight, [512, n - 512])
         assert ((torch.cat(pieces, 1).double() - want).abs() <= bound).all()
     finally:
