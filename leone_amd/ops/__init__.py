@@ -2345,8 +2345,39 @@ def route_topk(logits: torch.Tensor, correction: Optional[torch.Tensor], top: in
 ROUTE_PLAN_ROWS = 64          # up to here the router's choice and the tiles are made in one launch
 
 
-def _expert_tiles(x: torch.Tensor, rows: int, top: int, experts: int, hidden: int, ff: int, copied: bool = False):
-    """(pairs a tile, tiles at most, tile_expert, tile_pairs) for a step of ``rows`` rows.  ``copied``: both matrices have a copy."""
+@functools.lru_cache(maxsize=4096)
+def _copied_tile(pairs: int, experts: int, hidden: int, ff: int, gated: bool, units: int) -> int:
+    """Pairs a tile of experts' products that read the second copies; 0: more than 16, but from the matrices themselves they are faster.
+
+    Both products, matrices from memory, us: tiles of 16 and 64: 32 experts of 2,048 x 768, 8 pairs an expert 56 and 59, 11 pairs 59 and 59, 14
+    pairs 74 and 60; 64 of 2,048 x 1,408, 8 pairs 185 and 203, 11 pairs 206 and 206; 8 of 4,096 x 2,048, 11 pairs 81 and 100, 14 pairs 99 and
+    101.  Tiles of 64 and 128: 34 of 2,048 x 768, 115 pairs 104 and 108, 130 pairs 127 and 120; 32 of 1,024 x 384, 130 pairs 36 and 39, 160
+    pairs 39 and 37; 64 of 2,048 x 1,408, 40 pairs 220 and 228, 60 pairs 249 and 235, 100 pairs 285 and 250; 32 of 4,096 x 1,024, 40 pairs 160 and
+    161, 50 pairs 189 and 162; 8 of 4,096 x 2,048, 115 pairs 107 and 140, 130 pairs 189 and 142; with tiles of 128 for less than half of
+    the units 4 of 3,456 x 1,216, 128 pairs 82 and 110.
+
+    From the copies a workgroup walks a whole inner size, a stage of 64 at a time, which takes its time however few workgroups there are; the kernels
+    that read the matrices have more waves on a unit.  So each product needs a workgroup for every twelve elements of its inner size, or a
+    short one (us, from the matrices and from the copies: 2 of 3,520 x 3,968, 31 pairs 81 and 158, 8 of 2,688 x 5,696, 34 pairs 161 and 238,
+    8 of 5,248 x 3,136, 13 pairs 170 and 246, 4 of 2,944 x 1,216, 31 pairs 53 and 70; 32 of 2,048 x 768, 40 pairs 79 and 63).  Of 331 pairs of products
+    measured, 2 to 64 experts of 512 to 6,144 wide layers, 57 were slower from the copies, up to twice; of those on this side of the line one, by 4 %."""
+    each = pairs / experts
+    fills = experts * -(-hidden // 128) >= units
+    few, many = 10 if fills else 14, 48 if fills and hidden * ff >= 2500000 else 125
+    if each < few:
+        return 16
+
+    def workgroups(tile):
+        used = experts * math.ceil(each / tile)
+        return used * -(-ff // (64 if gated else 128)), used * -(-hidden // 128)
+    tile = 128 if each >= many and 2 * min(workgroups(128)) >= units else 64
+    first, second = workgroups(tile)
+    return tile if (hidden <= 1024 or 12 * first >= hidden) and (ff <= 1024 or 12 * second >= ff) else 0
+
+
+def _expert_tiles(x: torch.Tensor, rows: int, top: int, experts: int, hidden: int, ff: int, copied: bool = False, gated: bool = True):
+    """(pairs a tile, tiles at most, tile_expert, tile_pairs) for a step of ``rows`` rows.  ``copied``: the products read copies of both
+    matrices where that is the faster (``_copied_tile``)."""
     pairs = rows * top
     # bfloat16 with inner sizes in runs of 8 goes to the matrix cores: the more pairs an expert gets on average, the larger the
     # tiles (its matrices are read once a tile); anything else in tiles of the plain kernel's size.  Both products, matrices from
@@ -2358,18 +2389,10 @@ def _expert_tiles(x: torch.Tensor, rows: int, top: int, experts: int, hidden: in
     #   348; 8 of 4,096 x 2,048, 200 pairs (13e9) 231 and 239, 300 pairs (21e9) 282 and 247; 64 of 2,048 x 1,408, 160 pairs (30e9) 476 and 473,
     #   200 pairs (37e9) 570 and 517; 8 of 1,024 x 4,096, 500 pairs (17e9) 229 and 234, 700 pairs (23e9) 290 and 259
     if x.dtype == torch.bfloat16 and hidden % 8 == 0 and ff % 8 == 0:
-        each = pairs / experts
-        fills = experts * -(-hidden // 128) >= compute_units(x.device)
-        if copied and hidden % 64 == 0 and ff % 64 == 0:
-            # From the second copies, us: tiles of 16 and 64: 32 experts of 2,048 x 768, 8 pairs an expert 56 and 59, 11 pairs 59 and 59, 14 pairs 74
-            # and 60; 64 of 2,048 x 1,408, 8 pairs 185 and 203, 11 pairs 206 and 206; 8 of 4,096 x 2,048, 11 pairs 81 and 100, 14 pairs 99 and 101.
-            # Tiles of 64 and 128: 34 of 2,048 x 768, 115 pairs 104 and 108, 130 pairs 127 and 120; 32 of 1,024 x 384, 130 pairs 36 and 39, 160 pairs
-            # 39 and 37; 64 of 2,048 x 1,408, 40 pairs 220 and 228, 60 pairs 249 and 235, 100 pairs 285 and 250; 32 of 4,096 x 1,024, 40 pairs 160 and 161, 50
-            # pairs 189 and 162; 8 of 4,096 x 2,048, 115 pairs 107 and 140, 130 pairs 189 and 142
-            few, many = 10 if fills else 14, 48 if fills and hidden * ff >= 2500000 else 125
-            tile = 128 if each >= many else 64 if each >= few else 16
-        else:
-            few = 14 if not fills else 12 if hidden <= 1024 else 8
+        tile = _copied_tile(pairs, experts, hidden, ff, gated, compute_units(x.device)) if copied and hidden % 64 == 0 and ff % 64 == 0 else 0
+        if not tile:
+            each = pairs / experts
+            few = 14 if experts * -(-hidden // 128) < compute_units(x.device) else 12 if hidden <= 1024 else 8
             tile = 128 if each >= 160 and pairs * hidden * ff >= 20e9 else 64 if each >= few else 16
     else:
         tile = library().leone_moe_tile_pairs()
@@ -2401,8 +2424,15 @@ def _check_experts(x: torch.Tensor, w_up: torch.Tensor, w_down: torch.Tensor):
     return rows, hidden, experts, ff, gated
 
 
-def _whole(copies: tuple) -> tuple:
-    return (True,) if copies[0] is not None and copies[1] is not None and all(copies[2:]) else ()
+def _whole(copies: tuple) -> bool:
+    return copies[0] is not None and copies[1] is not None and all(copies[2:])
+
+
+def _paying_copies(copies: tuple, pairs: int, experts: int, hidden: int, ff: int, gated: bool, device) -> tuple:
+    """``copies``, for tiles of 16 pairs alone where those of more pairs are faster from the matrices themselves."""
+    if _whole(copies) and hidden % 64 == 0 and ff % 64 == 0 and not _copied_tile(pairs, experts, hidden, ff, gated, compute_units(device)):
+        return (*copies[:2], False)
+    return copies
 
 
 def _expert_copy(tiles: Optional[torch.Tensor], w: torch.Tensor, pairs_a_tile: int, any_order: bool = True) -> Optional[torch.Tensor]:
@@ -2457,10 +2487,12 @@ def routed_experts(x: torch.Tensor, chosen: torch.Tensor, weight: torch.Tensor, 
     of ``x``'s type; experts without a gate come as ``[experts, ff, hidden]`` and compute W_down[e] act(W_up[e] x)
     (``PLAIN_ACTIVATIONS``).  ``weigh_input`` (experts without a gate): the weight multiplies what the expert reads
     instead of what it gives.  ``paired``: the sum is left to the consumer (``PairedRows``).  ``copies``: ``tile_experts`` of both
-    matrices (None: none), which the products read instead; with a third, False, those products alone whose sums keep their order.  Nothing here depends on the choice except through device arrays."""
-    rows, hidden, experts, ff, _ = _check_experts(x, w_gate_up, w_down)
+    matrices (None: none), which the products read instead where that is the faster; with a third, False, those products alone whose sums keep
+    their order.  Nothing here depends on the choice except through device arrays."""
+    rows, hidden, experts, ff, gated = _check_experts(x, w_gate_up, w_down)
     top = chosen.shape[1]
-    tiles = _expert_tiles(x, rows, top, experts, hidden, ff, *_whole(copies))
+    copies = _paying_copies(copies, rows * top, experts, hidden, ff, gated, x.device)
+    tiles = _expert_tiles(x, rows, top, experts, hidden, ff, *((True, gated) if _whole(copies) else ()))
     call("leone_moe_plan", _dev(chosen, "chosen", torch.int32, (rows, top)), rows * top, experts, _dev(tiles[2], "tiles"),
          _dev(tiles[3], "tile pairs"), tiles[1], tiles[0], _stream())
     return _expert_products(x, chosen, weight, tiles, w_gate_up, w_down, activation, extra, limit, weigh_input, paired, copies)
@@ -2474,7 +2506,7 @@ def routed_feed_forward(x: torch.Tensor, logits: torch.Tensor, correction: Optio
     (up to ``ROUTE_PLAN_ROWS``) the choice and the tiles are made in one launch.  ``always`` (such steps only): the
     last so many experts of the matrices are no choice of the router's but taken by every row with weight 1 (a
     shared expert cut to the experts' size rides along in the experts' launches).  ``paired`` and ``copies`` as for ``routed_experts``."""
-    rows, hidden, experts, ff, _ = _check_experts(x, w_gate_up, w_down)
+    rows, hidden, experts, ff, gated = _check_experts(x, w_gate_up, w_down)
     total = logits.shape[1]
     if rows > ROUTE_PLAN_ROWS:
         if always:
@@ -2486,7 +2518,8 @@ def routed_feed_forward(x: torch.Tensor, logits: torch.Tensor, correction: Optio
     if not 0 <= always < experts:
         raise KernelError(f"routed_feed_forward: {always} of {experts} experts for every row")
     places = top + always
-    tiles = _expert_tiles(x, rows, places, experts, hidden, ff, *_whole(copies))
+    copies = _paying_copies(copies, rows * places, experts, hidden, ff, gated, x.device)
+    tiles = _expert_tiles(x, rows, places, experts, hidden, ff, *((True, gated) if _whole(copies) else ()))
     chosen = torch.empty((rows, places), dtype=torch.int32, device=x.device)
     weight = torch.empty((rows, places), dtype=torch.float32, device=x.device)
     call("leone_route_plan", _dev(logits, "router logits", torch.float32, (rows, total)),

@@ -74,6 +74,23 @@ def test_a_model_keeps_the_copies_if_there_is_room(monkeypatch, wanted, free, ke
 @pytest.mark.parametrize("experts,rows,top,hidden,ff", [(2, 64, 1, 64, 64), (3, 129, 2, 128, 64), (4, 200, 2, 192, 448), (5, 333, 3, 320, 192),
                                                         (40, 1300, 4, 704, 1344), (3, 700, 2, 2048, 832)])
 def test_many_pairs(mode, experts, rows, top, hidden, ff):
+    of_many_pairs(mode, experts, rows, top, hidden, ff)
+
+
+# every kind of tile whatever the rule takes for such sizes
+@pytest.mark.parametrize("tile", [64, 128])
+@pytest.mark.parametrize("mode", ["gated", "clamped", "plain", "weighed"])
+@pytest.mark.parametrize("experts,rows,top,hidden,ff", [(2, 64, 1, 64, 64), (3, 129, 2, 128, 64), (4, 200, 2, 192, 448), (5, 333, 3, 320, 192), (3, 700, 2, 2048, 832)])
+def test_every_tile_of_many_pairs(monkeypatch, tile, mode, experts, rows, top, hidden, ff):
+    from leone_amd import ops
+    monkeypatch.setattr(ops, "_copied_tile", lambda *sizes: tile)
+    read = []
+    monkeypatch.setattr(ops, "call", lambda name, *args, real=ops.call: (read.append(name), real(name, *args))[1])
+    of_many_pairs(mode, experts, rows, top, hidden, ff)
+    assert "leone_moe_product_tiles" in read and "leone_moe_product" not in read
+
+
+def of_many_pairs(mode, experts, rows, top, hidden, ff):
     from leone_amd import ops
     gen = torch.Generator(device=DEV).manual_seed(rows + ff)
     gated = mode in ("gated", "clamped")
