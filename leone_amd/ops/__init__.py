@@ -350,15 +350,18 @@ def _strided_rows(t: Optional[torch.Tensor], what: str, rows: int, columns: int,
 def f32_attention_shares(rows: int, kv_heads: int, head_dim: int, keys: int) -> bool:
     """Whether float32 attention of few rows gets a workgroup for every share of a row's keys and a second launch that merges them.
 
-    Two launches cost two microseconds more, so the row's walk along its keys has to be long; and with as many workgroups as the chip
-    holds anyway there is nothing to gain.  us, in one launch and in two, heads of 128: 4 rows times kv heads at 128, 200, 780 and 1,500 keys 9.1 and 9.6, 12.1 and
-    10.1, 23.8 and 14.9, 38.4 and 20.5; 16 at the same 9.2 and 10.3, 12.4 and 11.1, 24.4 and 16.3, 39.6 and 21.6; 32 at 200, 300 and 780 keys 12.5 and 12.3, 13.8 and
-    13.1, 24.8 and 19.0; 64 at 780 and 1,500 keys 28 and 28, 46 and 39; 128 at 4,000 keys 121 and 158.  Heads of 64: 8 at 300, 500 and 780 keys 8.8 and 9.1, 11.4 and
-    9.7, 15.0 and 12.7; 32 at 500 and 780 keys 11.8 and 11.7, 15.2 and 14.7.  ``keys`` may be up to twice what the rows see (a recorded
-    step's range)."""
+    Two launches cost one to two microseconds more, so the row's walk along its keys has to be long; and with as many workgroups as the chip
+    holds anyway there is nothing to gain.  us, in one launch and in two, heads of 128, at 20, 128, 200, 300 and 700 keys: 4 rows times kv heads 7.8
+    and 9.4, 8.7 and 9.2, 11.9 and 9.8, 12.9 and 10.3, 21 and 14; 16 7.8 and 9.8, 8.8 and 9.9, 12.0 and 10.7, 13.2 and 11.4, 22 and 16; 32
+    8.0 and 10.8, 9.1 and 11.2, 12.2 and 11.8, 13.6 and 12.9, 22 and 18; 64 at 700, 1,024 and 1,300 keys 26 and 28, 34 and 31, 41 and 38; 128 at
+    4,000 keys 121 and 158.  Heads of 64: 8 at 300, 400 and 700 keys 8.5 and 8.8, 9.7 and 9.0, 13.2 and 11.9; 32 at 512 and 700 11.5 and 11.2, 13.6
+    and 14.1, at 1,024 17.7 and 14.9.
+
+    ``keys`` is the longest row's count or, in a recorded step, the end of its range (``engine.context_bucket``): rows see any number from half of it on, but
+    in the first range, of 256, any from one on.  That range as a whole is level (16 at 20 to 200 keys, above), so it keeps the one launch."""
     units = rows * kv_heads
     if head_dim == 128:
-        return units <= 64 and keys > (128 if units <= 16 else 256 if units <= 32 else 1024)
+        return units <= 64 and keys > (256 if units <= 32 else 1024)
     return units <= 32 and keys > (256 if units <= 8 else 512)
 
 

@@ -4,6 +4,7 @@ import pytest
 import torch
 
 from leone_amd import ops
+from leone_amd.engine.engine import DECODE_BUCKET_MIN
 from tests.test_gpu_attention_f32 import DEV, pools
 
 pytestmark = pytest.mark.gpu
@@ -75,3 +76,6 @@ def test_the_rule():
         taken = [[ops.f32_attention_shares(units, 1, size, keys) for keys in (16, 128, 256, 512, 1024, 4096, 1 << 20)] for units in (1, 8, 16, 32, 64, 128, 4096)]
         assert all(line == sorted(line) for line in taken) and not any(taken[-1])          # more keys: rather; more rows: rather not
         assert all(column == sorted(column, reverse=True) for column in map(list, zip(*taken)))
+    # steps of a few tokens' context are recorded for the first range, whose end says nothing of theirs
+    assert not any(ops.f32_attention_shares(units, 1, size, DECODE_BUCKET_MIN) for units in (1, 4, 16, 64) for size in (64, 128))
+    assert ops.f32_attention_shares(16, 1, 128, 2 * DECODE_BUCKET_MIN)
