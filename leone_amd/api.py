@@ -71,7 +71,7 @@ class Runtime:
         ``prefill_chunk_tokens``) run with the fastest of the library's algorithms, measured now (a few
         seconds; ``Engine.tune_products``)."""
         self.model = model
-        model.keep_streamed_copies(streamed_weights)       # before the cache is sized by what is free
+        model.keep_streamed_copies(streamed_weights, experts=None)       # before the cache is sized by what is free
         self.config = getattr(model, "config", None)
         context = min(max_context or model.spec.max_positions, model.spec.max_positions)
         if num_pages is None and max_tokens is None:

@@ -217,8 +217,8 @@ class Engine:
         if not torch.cuda.is_available() or model.device.type != "cuda":
             raise RuntimeError("the engine runs on a GPU only; there is no CPU path")
         # A second copy of the matrices in the order the decode kernels read fastest: by default if there is
-        # ample room (``DecoderModel.keep_streamed_copies``); before the pools take their memory.
-        model.keep_streamed_copies(streamed_weights)
+        # ample room (``DecoderModel.keep_streamed_copies``); before the pools take their memory, of routed experts behind them.
+        model.keep_streamed_copies(streamed_weights, experts=None)
         self.model = model
         self.device = model.device
         self.dtype = model.dtype
@@ -229,6 +229,7 @@ class Engine:
                 raise ValueError("give num_pages or max_tokens")
             num_pages = (max_tokens + page_tokens - 1) // page_tokens
         self.pools = DevicePools(model.cache_needs(), self.dtype, self.device, num_pages, page_tokens, max_requests)
+        model.keep_expert_copies()
         self.cache = CacheManager(self.pools.group_specs, max_requests, self.max_context)
         # With poison_freed every page is filled with NaN when its last holder lets go of it, whoever frees it
         # (this engine, a scheduler on the same cache manager, a window that has passed): the manager notes

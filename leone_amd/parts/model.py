@@ -164,15 +164,17 @@ class DecoderModel:
         return any(isinstance(need, StateNeed) for layer in self.layers if hasattr(layer, "cache_need")
                    for _, need in flatten_needs(layer.cache_need()))
 
-    def keep_streamed_copies(self, wanted: Optional[bool] = None) -> int:
+    _experts_decided = False                              # ``keep_expert_copies``
+
+    def keep_streamed_copies(self, wanted: Optional[bool] = None, experts: Optional[bool] = True) -> int:
         """Keeps, beside every matrix that decode steps stream through, a second copy in the order in which
         the weight-streaming kernels read it fastest (``ops.tile_weight``; the row-major one stays for the
         library's products of prompt portions and for the token table).  The results of products of up to 16 rows
         are the same bit for bit (of more, sums may be in another order, but not in a model that carries memories); a decode step of few rows takes a sixth less time; the weights take twice the memory.
         ``wanted`` None decides by room: yes if the copies take at most a quarter of the device's memory
-        and half of what is free.  Routed experts get theirs (``ops.tile_experts``) behind these, all or none, if there is room for
-        both; their products of many pairs then run on a kernel of their own, with sums in its order (not in a model that carries
-        memories).  Returns the bytes the copies take (0: none kept).  Asked again, it answers what it did the first time."""
+        and half of what is free.  ``experts``: routed experts get theirs behind these (``keep_expert_copies``) at once, later,
+        when whoever asks for them has taken the memory it needs (None), or never (False).
+        Returns the bytes the copies take (0: none kept).  Asked again, it answers what it did the first time."""
         if self.streamed_copy_bytes is not None:
             return self.streamed_copy_bytes
         self.streamed_copy_bytes = 0
@@ -180,20 +182,37 @@ class DecoderModel:
         weights = [w for w in weights if w.is_cuda and w.dtype == torch.bfloat16 and w.dim() == 2 and w.shape[1] % 64 == 0]
         if not weights:
             return 0
-        needed = sum(-(-w.shape[0] // 16) * 16 * w.shape[1] * 2 for w in weights)
-        free, total = torch.cuda.mem_get_info(weights[0].device)
-        room = min(self.STREAMED_SHARE_OF_DEVICE * total, self.STREAMED_SHARE_OF_FREE * free)
-        if wanted is None and needed > room:
-            return 0
-        experts = [part for layer in self.layers for part in (layer.parts() if hasattr(layer, "parts") else ())
-                   if hasattr(part, "expert_copy_bytes") and part.expert_copy_bytes()]
-        of_experts = sum(part.expert_copy_bytes() for part in experts)
+        if wanted is None:
+            needed = sum(-(-w.shape[0] // 16) * 16 * w.shape[1] * 2 for w in weights)
+            free, total = torch.cuda.mem_get_info(weights[0].device)
+            if needed > self.STREAMED_SHARE_OF_DEVICE * total or needed > self.STREAMED_SHARE_OF_FREE * free:
+                return 0
         any_order = not self.carries_memories()
         self.streamed_copy_bytes = sum(ops.keep_streamed_copy(w, any_order) for w in weights)
-        if experts and needed + of_experts <= room:
-            for part in experts:
-                part.keep_expert_copies(any_order)
-            self.streamed_copy_bytes += of_experts
+        if experts:
+            self.keep_expert_copies()
+        elif experts is not None:
+            self._experts_decided = True
+        return self.streamed_copy_bytes
+
+    def keep_expert_copies(self) -> int:
+        """Second copies of the routed experts' matrices (``ops.tile_experts``), all or none, where ``keep_streamed_copies`` kept the
+        others: if all copies together take at most a quarter of the device's memory and these at most half of what is free.  An
+        engine asks behind its cache, so that no cache is smaller for them.  Their products of many pairs then run on a kernel of their own, with sums in
+        its order (not in a model that carries memories).  Returns the bytes of all copies; decided once."""
+        if self._experts_decided or not self.streamed_copy_bytes:
+            return self.streamed_copy_bytes or 0
+        self._experts_decided = True
+        experts = [part for layer in self.layers for part in (layer.parts() if hasattr(layer, "parts") else ())
+                   if hasattr(part, "expert_copy_bytes") and part.expert_copy_bytes()]
+        needed = sum(part.expert_copy_bytes() for part in experts)
+        if experts:
+            free, total = torch.cuda.mem_get_info(experts[0].w_gate_up_all.device)
+            if self.streamed_copy_bytes + needed <= self.STREAMED_SHARE_OF_DEVICE * total and needed <= self.STREAMED_SHARE_OF_FREE * free:
+                any_order = not self.carries_memories()
+                for part in experts:
+                    part.keep_expert_copies(any_order)
+                self.streamed_copy_bytes += needed
         return self.streamed_copy_bytes
 
     def row_tilings(self) -> list:

@@ -68,6 +68,43 @@ def test_a_model_keeps_the_copies_if_there_is_room(monkeypatch, wanted, free, ke
     ops.drop_streamed_copies()
 
 
+@pytest.mark.parametrize("given", [False, True])
+@pytest.mark.parametrize("room", [False, True])
+def test_a_cache_is_no_smaller_for_the_copies(monkeypatch, room, given):
+    """Memory that would hold the cache or the experts' copies holds the cache, of a size that is given or found; the copies come where there is
+    room beside it."""
+    from leone_amd import ops
+    from leone_amd.api import Runtime, cache_bytes_per_token
+    from leone_amd.benchmark import zukinex_shape
+    from leone_amd.runtime import random_model
+    model = random_model(zukinex_shape(512, 2, 512, 512), 3, "bfloat16")
+    experts = sum(part.expert_copy_bytes() for layer in model.layers for part in layer.parts() if hasattr(part, "expert_copy_bytes"))
+    dense = sum(-(-w.shape[0] // 16) * 16 * w.shape[1] * 2 for w in model.streamed_weights())
+    free = 2 * (dense + experts) + (1 << 20)                 # of which all copies are no more than half
+    page = 16 * cache_bytes_per_token(model)
+    requests = int(0.7 * (free - dense) / page) // 64        # a cache for them: 64 pages each, most of what is left by the other copies
+    limit = torch.cuda.memory_allocated() + free + (3 * experts if room else 0)
+    monkeypatch.setattr(torch.cuda, "mem_get_info", lambda *a: (limit - torch.cuda.memory_allocated(), 1 << 40))
+    runtime = Runtime(model, num_pages=64 * requests if given else None, page_tokens=16, max_requests=requests, max_context=1024)
+    assert runtime.engine.cache.free_pages(0) == 64 * requests and torch.cuda.memory_allocated() < limit
+    assert model.streamed_copy_bytes == dense + (experts if room else 0)
+    assert model.keep_expert_copies() == model.keep_streamed_copies() == model.streamed_copy_bytes        # decided once
+    ops.drop_streamed_copies()
+
+
+def test_copies_without_those_of_the_experts():
+    from leone_amd import ops
+    from leone_amd.api import Runtime
+    from leone_amd.benchmark import zukinex_shape
+    from leone_amd.runtime import random_model
+    model = random_model(zukinex_shape(512, 2, 512, 512), 3, "bfloat16")
+    dense = model.keep_streamed_copies(experts=False)
+    Runtime(model, num_pages=8, page_tokens=16, max_requests=1)
+    assert dense > 0 and model.streamed_copy_bytes == dense
+    assert all(part.copies == (None, None) for layer in model.layers for part in layer.parts() if hasattr(part, "copies"))
+    ops.drop_streamed_copies()
+
+
 # tiles of 64 and 128 pairs, the last of an expert nearly empty or full, experts without pairs; one stage of the inner size, two, an odd number;
 # rows of a matrix below, at and off what a workgroup takes, few and many workgroups
 @pytest.mark.parametrize("mode", ["gated", "clamped", "plain", "weighed"])
