@@ -895,6 +895,8 @@ def keep_streamed_copy(weight: torch.Tensor, any_order: bool = True) -> int:
         def forget(_, key=key):
             _streamed.pop(key, None)
         _streamed[key] = (weakref.ref(weight, forget), tile_weight(weight), bool(any_order), {})
+    elif held[2] and not any_order:                      # a matrix of two models: the stricter one's rule
+        _streamed[key] = (*held[:2], False, {})
     return _streamed[key][1].numel() * 2
 
 

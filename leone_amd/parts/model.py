@@ -8,7 +8,7 @@ import torch
 
 from .. import ops
 from ..weights.loader import MATRIX, VECTOR, TensorSpec
-from .base import BLOCKS, NORMS, POSITIONS, PartSpec, StateNeed, flatten_needs, nest_views
+from .base import BLOCKS, NORMS, POSITIONS, PartSpec, flatten_needs, nest_views
 from .context import CacheView, StepContext
 
 
@@ -161,8 +161,9 @@ class DecoderModel:
         """Whether requests carry state beside keys and values.  Memories hand every rounding on from token to token and are read over their own
         root mean square: decoded logits of mLSTM, retention and delta-rule layers are 1.5 to 6 % from 64 bits, and another order of a
         prompt's sums, no worse by itself, moved them by up to 4 %.  Their products keep the order they have without second copies."""
-        return any(isinstance(need, StateNeed) for layer in self.layers if hasattr(layer, "cache_need")
-                   for _, need in flatten_needs(layer.cache_need()))
+        def state(layer):
+            return not hasattr(layer, "cache_need") or any(not need.paged for _, need in flatten_needs(layer.cache_need()))
+        return any(state(layer) for layer in self.layers)          # (a layer that does not say what it keeps may keep some)
 
     _experts_decided = False                              # ``keep_expert_copies``
 

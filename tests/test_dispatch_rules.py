@@ -59,3 +59,19 @@ def test_tiles_of_experts_products_from_their_copies(experts, each, hidden, ff, 
     """Few workgroups that each walk a long inner size are slower than the kernels that read the matrices themselves (0)."""
     from leone_amd import ops
     assert ops._copied_tile(experts * each, experts, hidden, ff, gated, 256) == tile
+
+
+@pytest.mark.parametrize("shape,carries", [("qwen3", False), ("zukinex", False), ("pamevik", True), ("fosulix", True), ("nogidra", True), ("reverax", True),
+                                           ("sonulorn", True)])
+def test_which_models_carry_memories(shape, carries):
+    import torch
+
+    from leone_amd import benchmark
+    from leone_amd.architectures import config_from_dict, model_spec_for
+    from leone_amd.parts.model import DecoderModel
+    raw = dict(benchmark.QWEN3_8B, num_hidden_layers=2) if shape == "qwen3" else getattr(benchmark, shape + "_shape")(512, 4, 256, 256)
+    model = DecoderModel(model_spec_for(config_from_dict(raw)), torch.bfloat16, torch.device("cpu"))
+    assert model.carries_memories() == carries
+    silent = DecoderModel.__new__(DecoderModel)
+    silent.layers = [*model.layers, object()]              # a layer that does not say what it keeps
+    assert silent.carries_memories()

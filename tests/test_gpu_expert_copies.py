@@ -92,6 +92,20 @@ def test_a_cache_is_no_smaller_for_the_copies(monkeypatch, room, given):
     ops.drop_streamed_copies()
 
 
+@pytest.mark.parametrize("design", ["zukinex", "fosulix", "pamevik"])
+def test_models_with_memories_keep_the_order_of_their_sums(design):
+    """What a model says of its memories reaches every matrix and every expert's copy."""
+    from leone_amd import benchmark, ops
+    from leone_amd.runtime import random_model
+    model = random_model(getattr(benchmark, design + "_shape")(512, 4, 512, 512), 3, "bfloat16")
+    assert model.keep_streamed_copies(True) > 0
+    copied = [w for w in model.streamed_weights() if ops.streamed_copy(w) is not None]
+    assert copied and all(ops._any_order(w) == (not model.carries_memories()) == (design == "zukinex") for w in copied)
+    routed = [part.copies for layer in model.layers for part in layer.parts() if hasattr(part, "expert_copy_bytes")]
+    assert bool(routed) == (design != "pamevik") and all(copies[0] is not None and copies[2] == (design == "zukinex") for copies in routed)
+    ops.drop_streamed_copies()
+
+
 def test_copies_without_those_of_the_experts():
     from leone_amd import ops
     from leone_amd.api import Runtime

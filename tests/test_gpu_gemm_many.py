@@ -165,7 +165,11 @@ def test_a_copy_for_sums_in_their_old_order_is_left_alone_by_others(m):
     x, weight, tiles, want, bound = _operands(m, 1040, 1024)
     plain, parts = ops.linear(x, weight, out_dtype=torch.float32), ops.linear_planes(torch.stack([x, x]), weight, [16, 1024])
     try:
-        ops.keep_streamed_copy(weight, any_order=False)
+        ops.keep_streamed_copy(weight)
+        held = ops.streamed_copy(weight)
+        ops.keep_streamed_copy(weight, any_order=False)      # of a matrix that is kept in any order already: the stricter rule, the same copy
+        ops.keep_streamed_copy(weight)
+        assert ops.streamed_copy(weight) is held
         assert torch.equal(ops.linear(x, weight, out_dtype=torch.float32), plain)
         assert all(torch.equal(a, b) for a, b in zip(ops.linear_planes(torch.stack([x, x]), weight, [16, 1024]), parts))
     finally:
