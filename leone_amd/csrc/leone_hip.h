@@ -410,6 +410,8 @@ int leone_moe_product_tiles(const void* x, const void* w, void* y, const float* 
                             hipStream_t stream);
 // Whether tiles of 64 pairs keep one chunk of such experts' matrices on its way, not two.
 int leone_moe_one_chunk_ahead(int experts, int gated, int n, int k);
+// Whether tiles of 128 pairs take 256 rows of the matrices' copies a workgroup, not 128 (gated: gate and up rows).
+int leone_moe_many_rows(int max_tiles, int experts, int n, int gated);
 int leone_moe_combine(const float* pair_out, const int* chosen, const float* weight, const void* x, int dtype,
                       const float* extra, float* out, int rows, int top, int experts, int hidden, hipStream_t stream);
 // A matrix memory whose forget gate per head and key channel also says what is written (see gated_scan.hip).

@@ -1248,6 +1248,9 @@ extern "C" int leone_route_plan(const float* logits, const void* correction, int
     return 0;
 }
 
+// Whether tiles of 128 pairs that read the matrices' copies take 256 rows of a matrix a workgroup, not 128 (see many_rows).
+extern "C" int leone_moe_many_rows(int max_tiles, int experts, int n, int gated) { return many_rows(max_tiles - experts / 2, n, gated == kMoeGated); }
+
 extern "C" int leone_moe_one_chunk_ahead(int experts, int gated, int n, int k) {
     return one_chunk_ahead(experts, ceil_div(n, gated == kMoeGated ? kBigRows / 2 : kBigRows), n, k);
 }
@@ -1301,7 +1304,7 @@ static int run_moe_product(const void* x, const void* w, int w_tiled, void* y, c
 #undef LEONE_MOE_STREAM
 #undef LEONE_MOE_LAID
         } else if (w_tiled) {
-            const bool many = tile == kWidePairs && many_rows(max_tiles - experts / 2, n, gated == kMoeGated);
+            const bool many = tile == kWidePairs && leone_moe_many_rows(max_tiles, experts, n, gated);
             const int blocks = ceil_div(n, (gated == kMoeGated ? 64 : 128) * (many ? 2 : 1));
             const long places = static_cast<long>(ceil_div(max_tiles, 8 * kTogether)) * 8 * kTogether * blocks;
             LEONE_REQUIRE(places <= 0x7fffffffL, "moe_product: too many tiles");

@@ -118,6 +118,7 @@ _PROTOTYPES = {
     "leone_moe_product_tiles": [P, P, P, P, c_int, P, P, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, P],
     "leone_moe_product": [P, P, P, P, c_int, c_int, P, P, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, P],
     "leone_moe_one_chunk_ahead": [c_int, c_int, c_int, c_int],
+    "leone_moe_many_rows": [c_int, c_int, c_int, c_int],
     "leone_moe_combine": [P, P, P, P, c_int, P, P, c_int, c_int, c_int, c_int, P],
     "leone_gated_scan": [P, ctypes.c_long, c_int, c_int, c_int, P, P, c_int, c_int, c_int, c_int, P, c_int, P, ctypes.c_long, P,
                          ctypes.c_long, P, P, c_int, c_int, c_int, P],

@@ -141,6 +141,19 @@ def test_every_tile_of_many_pairs(monkeypatch, tile, mode, experts, rows, top, h
     assert "leone_moe_product_tiles" in read and "leone_moe_product" not in read
 
 
+# 256 rows of both matrices a workgroup, the second's end within one, below and above its half
+@pytest.mark.parametrize("mode", ["gated", "plain", "weighed"])
+@pytest.mark.parametrize("experts,rows,top,hidden,ff", [(40, 1300, 4, 832, 1344), (40, 1300, 4, 960, 1088), (12, 3100, 2, 1920, 1600)])
+def test_twice_the_rows_a_workgroup_in_both_products(mode, experts, rows, top, hidden, ff):
+    from leone_amd import ops
+    assert hidden % 256 and ff % 128
+    pairs, gated = rows * top, mode == "gated"
+    assert ops._copied_tile(pairs, experts, hidden, ff, gated, 256) == 128
+    tiles = min(pairs, pairs // 128 + experts)
+    assert ops.library().leone_moe_many_rows(tiles, experts, ff, 1 if gated else 2) and ops.library().leone_moe_many_rows(tiles, experts, hidden, 0)
+    of_many_pairs(mode, experts, rows, top, hidden, ff)
+
+
 def of_many_pairs(mode, experts, rows, top, hidden, ff):
     from leone_amd import ops
     gen = torch.Generator(device=DEV).manual_seed(rows + ff)
