@@ -16,6 +16,8 @@
 
 #include <math.h>
 
+#include <type_traits>
+
 namespace leone {
 
 // Threads a row.  Few rows (decode steps): 1,024, so that a thread has few elements and a row is a handful of trips to
@@ -693,9 +695,9 @@ __global__ void causal_conv_state_kernel(const TIn* __restrict__ in, long in_str
 }
 
 // Where the new running maximum of exponential gates made in a step of single rows (outer_step) goes: row r's is top's, in the state of the
-// slot that the r-th span writes.
+// slot that the r-th span writes.  Kernels that keep none have no such argument (asked for at run time it cost them up to 6 %).
 struct KeepTop {
-    float* state;                // the first slot's first maximum; null: nowhere
+    float* state;                // the first slot's first maximum
     long slot_stride, head_stride;
     const int* spans;            // [rows, 4]
 };
@@ -705,10 +707,10 @@ __device__ inline void keep_top(const KeepTop& keep, int row, int head, float va
 }
 
 // One wave per (row, head).
-template <typename TOut, int kKept>
+template <typename TOut, int kKept, typename... Keep>
 __global__ void head_norm_gate_kernel(const float* __restrict__ o, const float* __restrict__ dot, const float* __restrict__ top,
                                       AnyVec gain, int gain_per_head, const float* __restrict__ gate, long gate_stride,
-                                      int act, float eps, TOut* __restrict__ out, int heads, int vdim, int gate_first, KeepTop keep) {
+                                      int act, float eps, TOut* __restrict__ out, int heads, int vdim, int gate_first, Keep... keep) {
     const int row = blockIdx.x;
     const int head = blockIdx.y * (blockDim.x / kWave) + threadIdx.x / kWave;
     const int lane = threadIdx.x % kWave;
@@ -741,7 +743,8 @@ __global__ void head_norm_gate_kernel(const float* __restrict__ o, const float* 
     }
     float under = 1.f;
     if (dot) under = fmaxf(fabsf(read), expf(-highest)) + 1e-6f;
-    if (keep.state && lane == 0) keep_top(keep, row, head, highest);
+    if constexpr (sizeof...(Keep) > 0)
+        if (lane == 0) (keep_top(keep, row, head, highest), ...);
     // with gate_first the gate multiplies ahead of the norm, and the root mean square is that of the gated values
     auto opened = [&](float v, float g) {
         v /= under;
@@ -777,15 +780,16 @@ __global__ void head_norm_gate_kernel(const float* __restrict__ o, const float* 
 // The same for runs too long for a wave: a workgroup a (row, head), the values kept in registers between the passes where they
 // fit, sums added in a fixed order.
 constexpr int kWideHeadFrom = 1024;                            // runs of more columns go here
-template <typename TOut, int kThreads>
+template <typename TOut, int kThreads, typename... Keep>
 __global__ void __launch_bounds__(kThreads)
 head_norm_gate_wide_kernel(const float* __restrict__ o, const float* __restrict__ dot, const float* __restrict__ top, AnyVec gain,
                            int gain_per_head, const float* __restrict__ gate, long gate_stride, int act, float eps,
-                           TOut* __restrict__ out, int heads, int vdim, int gate_first, KeepTop keep) {
+                           TOut* __restrict__ out, int heads, int vdim, int gate_first, Keep... keep) {
     __shared__ float scratch[kThreads / kWave];
     const int row = blockIdx.x, head = blockIdx.y;
     const long at = static_cast<long>(row) * heads + head;
-    if (keep.state && threadIdx.x == 0) keep_top(keep, row, head, top[at]);
+    if constexpr (sizeof...(Keep) > 0)
+        if (threadIdx.x == 0) (keep_top(keep, row, head, top[at]), ...);
     const float* src = o + at * vdim;
     const float under = dot ? fmaxf(fabsf(dot[at]), expf(-top[at])) + 1e-6f : 1.f;
     const float* gate_row = gate ? gate + static_cast<long>(row) * gate_stride + static_cast<long>(head) * vdim : nullptr;
@@ -1090,32 +1094,36 @@ extern "C" int leone_head_norm_gate_kept(const float* o, const float* dot, const
     const AnyVec vg{gain, gain_dtype};
     if (vdim > kWideHeadFrom) {
         LEONE_REQUIRE(heads <= 65535, "head_norm_gate: too many heads");
-#define LEONE_WIDE_HEAD(T, THREADS)                                                                                           \
-    head_norm_gate_wide_kernel<T, THREADS><<<dim3(rows, heads), THREADS, 0, stream>>>(o, dot, top, vg, gain_per_head, gate, gate_stride, \
-                                                                                    act, eps, static_cast<T*>(out), heads, vdim, gate_first, keep)
         // few rows: a row in as few trips to memory as threads allow; many rows: more rows in flight a compute unit
-        if (out_dtype == kF32) {
-            if (rows >= kNormManyRows) LEONE_WIDE_HEAD(float, kNormThreadsMany);
-            else LEONE_WIDE_HEAD(float, kNormThreadsFew);
-        } else {
-            if (rows >= kNormManyRows) LEONE_WIDE_HEAD(bf16_t, kNormThreadsMany);
-            else LEONE_WIDE_HEAD(bf16_t, kNormThreadsFew);
-        }
-#undef LEONE_WIDE_HEAD
+        const auto launch = [&](auto* to, auto... kept) {
+            using T = std::remove_pointer_t<decltype(to)>;
+            if (rows >= kNormManyRows)
+                head_norm_gate_wide_kernel<T, kNormThreadsMany><<<dim3(rows, heads), kNormThreadsMany, 0, stream>>>(
+                    o, dot, top, vg, gain_per_head, gate, gate_stride, act, eps, to, heads, vdim, gate_first, kept...);
+            else
+                head_norm_gate_wide_kernel<T, kNormThreadsFew><<<dim3(rows, heads), kNormThreadsFew, 0, stream>>>(
+                    o, dot, top, vg, gain_per_head, gate, gate_stride, act, eps, to, heads, vdim, gate_first, kept...);
+        };
+        if (out_dtype == kF32) keep_state ? launch(static_cast<float*>(out), keep) : launch(static_cast<float*>(out));
+        else keep_state ? launch(static_cast<bf16_t*>(out), keep) : launch(static_cast<bf16_t*>(out));
         LEONE_LAUNCH_CHECK("head_norm_gate");
         return 0;
     }
     const dim3 grid(rows, ceil_div(heads, 4));
     // Heads of 64 and 128 hold one and two values a lane: asking for eight reads the same ones again (us, 2,048 rows of 32 heads of
     // 64, eight and one: 26.8 and 19.6; 16 of 128, eight and two: 17.9 and 14.1).
-#define LEONE_HEAD(T, KEPT)                                                                                                    \
-    head_norm_gate_kernel<T, KEPT><<<grid, 4 * kWave, 0, stream>>>(o, dot, top, vg, gain_per_head, gate, gate_stride, act, eps, \
-                                                                   static_cast<T*>(out), heads, vdim, gate_first, keep)
-#define LEONE_HEAD_KEPT(T) (vdim <= kWave ? LEONE_HEAD(T, 1) : vdim <= 2 * kWave ? LEONE_HEAD(T, 2) : LEONE_HEAD(T, 8))
-    if (out_dtype == kF32) LEONE_HEAD_KEPT(float);
-    else LEONE_HEAD_KEPT(bf16_t);
-#undef LEONE_HEAD_KEPT
-#undef LEONE_HEAD
+    const auto launch = [&](auto* to, auto... kept) {
+        using T = std::remove_pointer_t<decltype(to)>;
+        const auto of = [&](auto values) {
+            head_norm_gate_kernel<T, decltype(values)::value><<<grid, 4 * kWave, 0, stream>>>(o, dot, top, vg, gain_per_head, gate, gate_stride, act, eps,
+                                                                                              to, heads, vdim, gate_first, kept...);
+        };
+        if (vdim <= kWave) of(std::integral_constant<int, 1>{});
+        else if (vdim <= 2 * kWave) of(std::integral_constant<int, 2>{});
+        else of(std::integral_constant<int, 8>{});
+    };
+    if (out_dtype == kF32) keep_state ? launch(static_cast<float*>(out), keep) : launch(static_cast<float*>(out));
+    else keep_state ? launch(static_cast<bf16_t*>(out), keep) : launch(static_cast<bf16_t*>(out));
     LEONE_LAUNCH_CHECK("head_norm_gate");
     return 0;
 }

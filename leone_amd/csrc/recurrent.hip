@@ -22,6 +22,8 @@
 
 #include <math.h>
 
+#include <type_traits>
+
 namespace leone {
 
 constexpr int kScanTokens = 16;
@@ -66,7 +68,11 @@ struct OuterScanArgs {
     float* out;                 // [rows, heads, vdim]
     float* dot;                 // [rows, heads]
     int heads, dim, vdim;
-    // outer_step alone, instead of coef: the gates are made where they are used (null: they are not)
+};
+
+// outer_step with exponential gates, made where they are used, in place of coef and decay.  (Arguments and kernels of their own: as a run-time
+// question they cost a step without them up to 6 %.)
+struct GatedStepArgs : OuterScanArgs {
     AnyVec i_bias, f_bias;      // [heads]
     int i_off, f_off;           // the first columns of their pre-activations in a row of proj
     float cap;
@@ -317,8 +323,8 @@ __device__ inline float turn(const Turned& t, int i, int silu, int rot_half) {
     return i < rot_half ? x * t.c - silu_if(t.other, silu) * t.s : x * t.c + silu_if(t.other, silu) * t.s;
 }
 
-template <int kGroups>
-__global__ void __launch_bounds__(kGroups * kWave) outer_step_kernel(OuterScanArgs p) {
+template <int kGroups, bool kGated>
+__global__ void __launch_bounds__(kGroups * kWave) outer_step_kernel(std::conditional_t<kGated, GatedStepArgs, OuterScanArgs> p) {
     __shared__ float sums[2][kGroups][kWave + 1];             // the columns' shares; one more for the normaliser's
     __shared__ __align__(16) float2 skq[kGroups][kLaneRows];  // a wave's own k and q
     __shared__ float snorm[kGroups][kLaneRows];
@@ -336,10 +342,11 @@ __global__ void __launch_bounds__(kGroups * kWave) outer_step_kernel(OuterScanAr
     const int other = ch < half ? ch + half : ch < 2 * half ? ch - half : ch;
     const int turned = ch < half ? ch : ch < 2 * half ? ch - half : 0;
     const float* from = seg.in < 0 ? nullptr : p.state_in + seg.in * p.in_stride + head * p.head_stride;
-    const float fixed = p.coef || p.top ? 0.f : p.decay[head];
     float S[kLaneRows], N = 0.f;
-    float m = 0.f, bi = 0.f, bf = 0.f;
-    if (p.top) {
+    [[maybe_unused]] float fixed = 0.f, m = 0.f, bi = 0.f, bf = 0.f;
+    if constexpr (!kGated) {
+        fixed = p.coef ? 0.f : p.decay[head];
+    } else {
         m = from ? from[p.top_at] : 0.f;
         bi = load_any(p.i_bias, head);
         bf = load_any(p.f_bias, head);
@@ -358,12 +365,13 @@ __global__ void __launch_bounds__(kGroups * kWave) outer_step_kernel(OuterScanAr
         const float v_raw = base[p.v_off + head * p.vdim + ccol];
         const long at = row * p.heads + head;
         float a = fixed, b = 1.f;
-        if (p.coef) {
-            a = p.coef[2 * at];
-            b = p.coef[2 * at + 1];
-        }
-        float raw_i = 0.f, raw_f = 0.f;
-        if (p.top) {
+        [[maybe_unused]] float raw_i = 0.f, raw_f = 0.f;
+        if constexpr (!kGated) {
+            if (p.coef) {
+                a = p.coef[2 * at];
+                b = p.coef[2 * at + 1];
+            }
+        } else {
             raw_i = base[p.i_off + head];
             raw_f = base[p.f_off + head];
         }
@@ -377,7 +385,7 @@ __global__ void __launch_bounds__(kGroups * kWave) outer_step_kernel(OuterScanAr
             for (int i = 0; i < kLaneRows; ++i) S[i] = float_at(from, (ch0 + i) * row_bytes, 4u * ccol);
             if (norm) N = from[static_cast<long>(p.dim) * p.vdim + ch];
         }
-        if (p.top) {                                           // as exp_gates_kernel makes them, to the bit: no product joins a sum
+        if constexpr (kGated) {                                // as exp_gates_kernel makes them, to the bit: no product joins a sum
 #pragma clang fp contract(off)
             const float li = soft_cap_f(raw_i + bi, p.cap), lf = log_sigmoid_f(soft_cap_f(raw_f + bf, p.cap));
             const float next = fmaxf(lf + m, li);
@@ -752,7 +760,7 @@ static int run_outer_scan(bool single, const float* proj, long stride, int q_off
                                 const float* cos_table, const float* sin_table, int rotary_dim, int table_positions,
                                 const int* positions, const int* segments, int n_segments, const float* state_in,
                                 long in_stride, float* state_out, long out_stride, long head_stride, float* out, float* dot,
-                                int heads, int dim, int vdim, hipStream_t stream, const OuterScanArgs* gates = nullptr) {
+                                int heads, int dim, int vdim, hipStream_t stream, const GatedStepArgs* gates = nullptr) {
     LEONE_REQUIRE(proj && positions && segments && out, "outer_scan: null pointer");
     LEONE_REQUIRE(n_segments > 0 && heads > 0 && heads <= 65535 && dim > 0 && vdim > 0, "outer_scan: %d segments, %d heads of %d x %d",
                   n_segments, heads, dim, vdim);
@@ -770,11 +778,7 @@ static int run_outer_scan(bool single, const float* proj, long stride, int q_off
     OuterScanArgs a{proj, stride, q_off, k_off, v_off, coef, decay, norm_column, q_scale, k_scale,
                     silu, cos_table, sin_table, cos_table ? rotary_dim / 2 : 0, cos_table ? table_positions : 1, positions,
                     reinterpret_cast<const Segment*>(segments), state_in, in_stride, state_out, out_stride, head_stride,
-                    out, dot, heads, dim, vdim, AnyVec{nullptr, kF32}, AnyVec{nullptr, kF32}, 0, 0, 0.f, 0, nullptr};
-    if (gates) {
-        a.i_bias = gates->i_bias, a.f_bias = gates->f_bias, a.i_off = gates->i_off, a.f_off = gates->f_off;
-        a.cap = gates->cap, a.top_at = gates->top_at, a.top = gates->top;
-    }
+                    out, dot, heads, dim, vdim};
     const int groups = lane_groups(dim);
     const int per_block = (kScanThreads / kWave) * (kWave / groups) * kLaneCols;          // columns a workgroup
     const dim3 grid(n_segments, heads, ceil_div(vdim + (norm_column ? 1 : 0), per_block));
@@ -782,10 +786,20 @@ static int run_outer_scan(bool single, const float* proj, long stride, int q_off
     if (single) {
         LEONE_REQUIRE(leone_step_fits(dim, vdim), "outer_step: heads have 32, 64, 128 or 256 key channels (not %d x %d)", dim, vdim);
         const dim3 columns(n_segments, heads, ceil_div(vdim, kWave));
-        if (groups == 1) outer_step_kernel<1><<<columns, kWave, 0, stream>>>(a);
-        else if (groups == 2) outer_step_kernel<2><<<columns, 2 * kWave, 0, stream>>>(a);
-        else if (groups == 4) outer_step_kernel<4><<<columns, 4 * kWave, 0, stream>>>(a);
-        else outer_step_kernel<8><<<columns, 8 * kWave, 0, stream>>>(a);
+        const auto launch = [&](auto gated, const auto& args) {
+            constexpr bool kGated = decltype(gated)::value;
+            if (groups == 1) outer_step_kernel<1, kGated><<<columns, kWave, 0, stream>>>(args);
+            else if (groups == 2) outer_step_kernel<2, kGated><<<columns, 2 * kWave, 0, stream>>>(args);
+            else if (groups == 4) outer_step_kernel<4, kGated><<<columns, 4 * kWave, 0, stream>>>(args);
+            else outer_step_kernel<8, kGated><<<columns, 8 * kWave, 0, stream>>>(args);
+        };
+        if (gates) {
+            GatedStepArgs with = *gates;
+            static_cast<OuterScanArgs&>(with) = a;
+            launch(std::true_type{}, with);
+        } else {
+            launch(std::false_type{}, a);
+        }
         LEONE_LAUNCH_CHECK("outer_step");
         return 0;
     }
@@ -829,7 +843,7 @@ extern "C" int leone_outer_step_gated(const float* proj, long stride, int q_off,
     LEONE_REQUIRE(known_vec(bias_dtype) && cap > 0.f, "outer_step: unknown bias type or cap %g", cap);
     LEONE_REQUIRE(i_off >= 0 && f_off >= 0 && stride >= i_off + heads && stride >= f_off + heads, "outer_step: rows of %ld do not hold the gates", stride);
     LEONE_REQUIRE(top_at >= 0 && top_at < head_stride, "outer_step: the maximum's place %ld", top_at);
-    OuterScanArgs gates{};
+    GatedStepArgs gates{};
     gates.i_bias = AnyVec{i_bias, bias_dtype}, gates.f_bias = AnyVec{f_bias, bias_dtype};
     gates.i_off = i_off, gates.f_off = f_off, gates.cap = cap, gates.top_at = top_at, gates.top = top;
     return run_outer_scan(true, proj, stride, q_off, k_off, v_off, nullptr, nullptr, 1, q_scale, k_scale, silu, cos_table,
