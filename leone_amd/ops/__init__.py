@@ -761,9 +761,9 @@ FOLDED_F32_ROWS = 8          # most rows of a float32 product that carries out i
 FOLDED_F32_NORM_ELEMENTS = 12 << 20
 
 
-def _apart(a: torch.Tensor, b: torch.Tensor) -> bool:
-    """Whether two tensors in one piece share no memory."""
-    return a.data_ptr() + a.numel() * a.element_size() <= b.data_ptr() or b.data_ptr() + b.numel() * b.element_size() <= a.data_ptr()
+def _shares_memory(at: int, of: int, other: int, of_other: int) -> bool:
+    """Whether ``of`` floats from address ``at`` on and ``of_other`` from ``other`` on have any in common."""
+    return at < other + 4 * of_other and other < at + 4 * of
 
 
 def _folds_f32(x, weight: torch.Tensor, residual: Optional[torch.Tensor], gated: bool) -> bool:
@@ -780,9 +780,12 @@ def _folds_f32(x, weight: torch.Tensor, residual: Optional[torch.Tensor], gated:
         return (n * k <= FOLDED_F32_NORM_ELEMENTS and x.rows is None and x.gain.dtype == torch.float32 and x.x.dtype == torch.float32
                 and x.x.is_contiguous() and x.gain.is_contiguous() and x.x.data_ptr() % 16 == 0 and x.gain.data_ptr() % 16 == 0
                 and (not gated or n % 16 == 0) and bool(library().leone_gemm_f32_folds(rows, n, k, 2)))
-    return (residual is not None and residual.dtype == torch.float32 and tuple(residual.shape) == (rows, n) and residual.is_contiguous()
-            and x.is_contiguous() and x.data_ptr() % 16 == 0 and residual.device == weight.device and _apart(residual, x)
-            and _apart(residual, weight) and bool(library().leone_gemm_f32_folds(rows, n, k, 1)))
+    if residual is None or residual.dtype != torch.float32 or residual.shape != (rows, n) or not residual.is_contiguous() \
+            or residual.get_device() != weight.get_device() or not x.is_contiguous():
+        return False
+    at, to = x.data_ptr(), residual.data_ptr()
+    return (at % 16 == 0 and not _shares_memory(to, rows * n, at, rows * k) and not _shares_memory(to, rows * n, weight.data_ptr(), n * k)
+            and bool(library().leone_gemm_f32_folds(rows, n, k, 1)))
 
 
 def gemm_f32_folded(x, weight: torch.Tensor, residual: Optional[torch.Tensor] = None, gated: bool = False, activation: str = "silu",
@@ -796,14 +799,14 @@ def gemm_f32_folded(x, weight: torch.Tensor, residual: Optional[torch.Tensor] = 
     normed = isinstance(x, NormedRows)
     if normed == (residual is not None) or (gated and not normed):
         raise KernelError("gemm_f32_folded: either a norm goes ahead of the product or it is added into the stream")
-    if residual is not None and not (_apart(residual, x) and _apart(residual, weight)):
-        raise KernelError("gemm_f32_folded: the product cannot be added into what it is made of")
     out = residual if residual is not None else torch.empty((rows, n // 2 if gated else n), dtype=torch.float32, device=weight.device)
+    of_x, of_w, to = (_dev(x.x if normed else x, "gemm a", torch.float32, (rows, k)), _dev(weight, "gemm b", torch.float32),
+                      _dev(out, "gemm out", torch.float32, (rows, n // 2 if gated else n)))
+    if residual is not None and (_shares_memory(to, rows * n, of_x, rows * k) or _shares_memory(to, rows * n, of_w, n * k)):
+        raise KernelError("gemm_f32_folded: the product cannot be added into what it is made of")
     with profile.span("gemm f32", weight):
-        call("leone_gemm_f32_folded", _dev(x.x if normed else x, "gemm a", torch.float32, (rows, k)), _dev(weight, "gemm b", torch.float32),
-             _dev(out, "gemm out", torch.float32, (rows, n // 2 if gated else n)), rows, n, k,
-             _dev(x.gain, "gain", torch.float32, (k,)) if normed else 0, x.eps if normed else 0.0,
-             _glu_code(activation, limit) if gated else -1, float(limit or 0.0), _stream())
+        call("leone_gemm_f32_folded", of_x, of_w, to, rows, n, k, _dev(x.gain, "gain", torch.float32, (k,)) if normed else 0,
+             x.eps if normed else 0.0, _glu_code(activation, limit) if gated else -1, float(limit or 0.0), _stream())
     return None if residual is not None else out
 
 
@@ -1940,14 +1943,15 @@ def head_norm_gate(o: torch.Tensor, heads: int, vdim: int, eps: float, out_dtype
             raise KernelError(f"head_norm_gate: a gain of {gain.numel()} for {heads} heads of {vdim}")
     gate_at, gate_stride = _strided_rows(gate, "head_norm_gate gate", rows, heads * vdim)
     dot, top, *keep = denominator if denominator is not None else (None, None)
-    kept = (0, 0, 0, 0)
+    given = (_dev(o, "read-outs", torch.float32, (rows, heads * vdim)), _dev(dot, "dot", torch.float32, (rows, heads)),
+             _dev(top, "top", torch.float32, (rows, heads)), _dev(gain, "gain"), _code(gain, "gain") if gain is not None else F32, per_head, gate_at,
+             gate_stride, ACTIVATIONS[activation], 1 if gate_first else 0, float(eps), _dev(out, "out"), _CODES[out_dtype], rows, heads, vdim)
     if keep:                                              # the running maxima go into their state (``outer_scan``)
         state, top_at, per_head_state, spans = keep[0]
-        kept = (_dev(state, "state", torch.float32) + 4 * top_at, state.stride(0), per_head_state, _dev(spans, "spans", torch.int32, (rows, 4)))
-    call("leone_head_norm_gate_kept", _dev(o, "read-outs", torch.float32, (rows, heads * vdim)),
-         _dev(dot, "dot", torch.float32, (rows, heads)), _dev(top, "top", torch.float32, (rows, heads)),
-         _dev(gain, "gain"), _code(gain, "gain") if gain is not None else F32, per_head, gate_at, gate_stride,
-         ACTIVATIONS[activation], 1 if gate_first else 0, float(eps), _dev(out, "out"), _CODES[out_dtype], rows, heads, vdim, *kept, _stream())
+        call("leone_head_norm_gate_kept", *given, _dev(state, "state", torch.float32) + 4 * top_at, state.stride(0), per_head_state,
+             _dev(spans, "spans", torch.int32, (rows, 4)), _stream())
+    else:
+        call("leone_head_norm_gate_ordered", *given, _stream())
     return out
 
 
@@ -2429,24 +2433,22 @@ def _check_experts(x: torch.Tensor, w_up: torch.Tensor, w_down: torch.Tensor):
     return rows, hidden, experts, ff, gated
 
 
-def _whole(copies: tuple) -> bool:
-    return copies[0] is not None and copies[1] is not None and all(copies[2:])
-
-
 def _paying_copies(copies: tuple, pairs: int, experts: int, hidden: int, ff: int, gated: bool, device) -> tuple:
-    """``copies``, for tiles of 16 pairs alone where those of more pairs are faster from the matrices themselves."""
-    if _whole(copies) and hidden % 64 == 0 and ff % 64 == 0 and not _copied_tile(pairs, experts, hidden, ff, gated, compute_units(device)):
-        return (*copies[:2], False)
-    return copies
+    """(``copies``, for tiles of 16 pairs alone where those of more are faster from the matrices themselves; what ``_expert_tiles`` is told)."""
+    if copies[0] is None or copies[1] is None or not all(copies[2:]):
+        return copies, ()
+    if hidden % 64 == 0 and ff % 64 == 0 and not _copied_tile(pairs, experts, hidden, ff, gated, compute_units(device)):
+        return (*copies[:2], False), ()
+    return copies, (True, gated)
 
 
-def _expert_copy(tiles: Optional[torch.Tensor], w: torch.Tensor, pairs_a_tile: int, any_order: bool = True) -> Optional[torch.Tensor]:
+def _expert_copy(tiles: torch.Tensor, w: torch.Tensor, pairs_a_tile: int, any_order: bool = True) -> Optional[torch.Tensor]:
     """``tiles`` if the product of such tiles of pairs reads the experts' copy (of ``w``, or of more experts that begin with them)."""
     rows, k = w.shape[-2:]
-    if tiles is None or not (pairs_a_tile == 16 or (any_order and pairs_a_tile in (64, 128) and k % 64 == 0)):
+    if not (pairs_a_tile == 16 or (any_order and pairs_a_tile in (64, 128) and k % 64 == 0)):
         return None
     if tiles.dtype != torch.bfloat16 or tiles.device != w.device or not tiles.is_contiguous() or tiles.shape[0] < w.shape[0] \
-            or tuple(tiles.shape[1:]) != (*w.shape[1:-2], rows // 16, k // 32, 4, 16, 8):
+            or tiles.shape[1:] != (*w.shape[1:-2], rows // 16, k // 32, 4, 16, 8):
         raise KernelError(f"routed experts: a copy {tuple(tiles.shape)} of {tiles.dtype} does not belong to {tuple(w.shape)}")
     return tiles
 
@@ -2466,18 +2468,18 @@ def _expert_products(x, chosen, weight, tiles, w_up, w_down, activation, extra, 
     # the weight stands on the input's side (a product of weight * x is weight times the product) or on the result's
     pair_out = torch.empty((pairs, hidden), dtype=torch.float32, device=device)
 
-    def product(rows_in, w, copy, out, pair_weight, kind, n, k, code, held):
-        copy = _expert_copy(copy, w, tile, all(copies[2:]))
+    common = (_dev(tile_expert, "tiles"), _dev(tile_pairs, "tile pairs"), max_tiles, tile, experts, top)
+    for rows_in, w, copy, results, pair_weight, kind, n, k, code, held in (
+            (x, w_up, copies[0], hidden_act, weights if weigh_input else 0, 1 if gated else 2, ff, hidden, act, limit),
+            (hidden_act, w_down, copies[1], pair_out, 0 if weigh_input else weights, 0, hidden, ff, 0, 0.0)):
         if copy is not None:
-            call("leone_moe_product_tiles", _dev(rows_in, "routed rows", torch.bfloat16), _dev(copy, "experts' tiles"), _dev(out, "experts' results"),
-                 pair_weight, kind, _dev(tile_expert, "tiles"), _dev(tile_pairs, "tile pairs"), max_tiles, tile, experts, top, n, k, code, held, _stream())
-            return
-        call("leone_moe_product", _dev(rows_in, "routed rows"), _dev(w, "experts"), _dev(out, "experts' results"), pair_weight,
-             _code(rows_in, "routed rows"), kind, _dev(tile_expert, "tiles"), _dev(tile_pairs, "tile pairs"), max_tiles, tile, experts, top, n, k,
-             code, held, _stream())
-
-    product(x, w_up, copies[0], hidden_act, weights if weigh_input else 0, 1 if gated else 2, ff, hidden, act, limit)
-    product(hidden_act, w_down, copies[1], pair_out, 0 if weigh_input else weights, 0, hidden, ff, 0, 0.0)
+            copy = _expert_copy(copy, w, tile, all(copies[2:]))
+        if copy is not None:
+            call("leone_moe_product_tiles", _dev(rows_in, "routed rows", torch.bfloat16), _dev(copy, "experts' tiles"), _dev(results, "experts' results"),
+                 pair_weight, kind, *common, n, k, code, held, _stream())
+        else:
+            call("leone_moe_product", _dev(rows_in, "routed rows"), _dev(w, "experts"), _dev(results, "experts' results"), pair_weight,
+                 _code(rows_in, "routed rows"), kind, *common, n, k, code, held, _stream())
     out = PairedRows(pair_out, chosen, weight, x, extra, experts)
     return out if paired else out.sum()
 
@@ -2496,8 +2498,8 @@ def routed_experts(x: torch.Tensor, chosen: torch.Tensor, weight: torch.Tensor, 
     their order.  Nothing here depends on the choice except through device arrays."""
     rows, hidden, experts, ff, gated = _check_experts(x, w_gate_up, w_down)
     top = chosen.shape[1]
-    copies = _paying_copies(copies, rows * top, experts, hidden, ff, gated, x.device)
-    tiles = _expert_tiles(x, rows, top, experts, hidden, ff, *((True, gated) if _whole(copies) else ()))
+    copies, copied = _paying_copies(copies, rows * top, experts, hidden, ff, gated, x.device)
+    tiles = _expert_tiles(x, rows, top, experts, hidden, ff, *copied)
     call("leone_moe_plan", _dev(chosen, "chosen", torch.int32, (rows, top)), rows * top, experts, _dev(tiles[2], "tiles"),
          _dev(tiles[3], "tile pairs"), tiles[1], tiles[0], _stream())
     return _expert_products(x, chosen, weight, tiles, w_gate_up, w_down, activation, extra, limit, weigh_input, paired, copies)
@@ -2523,8 +2525,8 @@ def routed_feed_forward(x: torch.Tensor, logits: torch.Tensor, correction: Optio
     if not 0 <= always < experts:
         raise KernelError(f"routed_feed_forward: {always} of {experts} experts for every row")
     places = top + always
-    copies = _paying_copies(copies, rows * places, experts, hidden, ff, gated, x.device)
-    tiles = _expert_tiles(x, rows, places, experts, hidden, ff, *((True, gated) if _whole(copies) else ()))
+    copies, copied = _paying_copies(copies, rows * places, experts, hidden, ff, gated, x.device)
+    tiles = _expert_tiles(x, rows, places, experts, hidden, ff, *copied)
     chosen = torch.empty((rows, places), dtype=torch.int32, device=x.device)
     weight = torch.empty((rows, places), dtype=torch.float32, device=x.device)
     call("leone_route_plan", _dev(logits, "router logits", torch.float32, (rows, total)),

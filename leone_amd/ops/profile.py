@@ -92,6 +92,7 @@ OPERATIONS = {
     "leone_attention_decode_biased": "attention",
     "leone_attention_prefill_biased": "attention",
     "leone_causal_conv_biased": "causal conv",
+    "leone_head_norm_gate_ordered": "head norm gate",
     "leone_head_norm_gate_kept": "head norm gate",
     "leone_weighted_mix": "branch mix",
     "leone_state_space_scan": "state space scan",
