@@ -1097,12 +1097,12 @@ STREAM_MOST = 8192           # widest stream it leaves planes for: widths the no
 def many_plan(m: int, n: int, k: int, may_split: bool, units: int = 256) -> tuple[int, int, int]:
     """(rows, columns, ranges of K) of a workgroup of ``gemm_many``.  Its time is taken for a start and then, a stage of 64 elements of K, so
     much for every tile that falls to one compute unit (``MANY_TILES``: rows, columns, us to start, us a stage; fitted to 700 products
-    whose weights lay in the caches); planes for 0.6 us a megabyte, written and read.  It ranks tiles and ranges and is no estimate of the time: from
+    whose weights lay in the caches); planes for 0.5 to 0.6 us a megabyte, written and read (of short chains, which the caches flatter less, the more).  It ranks tiles and ranges and is no estimate of the time: from
     memory, and with all units multiplying, products take up to twice as long (over estimate, on average: 1.1 into the stream, 1.6 gated
     or stored).  With the norm behind it, weights from memory, what is chosen into the stream is within 1 % of the best of the four tiles and 1 to 4
-    ranges on average, 9 % at worst (121 products, 144 to 1,500 rows; at 0.48 us a megabyte 1 % and 15 %, 8 of them behind the
+    ranges on average, 9 % at worst (122 products, 144 to 1,500 rows; at 0.48 us a megabyte for all 15 %, 8 of them behind the
     library, now 4)."""
-    stages = k // 64
+    stages, plane = k // 64, (0.6e-6 if k <= 2048 else 0.48e-6) * 4 * m * n if may_split else 0.0
     best = None
     for rows, columns, start, stage in MANY_TILES:
         tiles = -(-m // rows) * -(-n // columns)
@@ -1110,7 +1110,7 @@ def many_plan(m: int, n: int, k: int, may_split: bool, units: int = 256) -> tupl
             per = -(-stages // splits)
             if per * (splits - 1) >= stages:            # a range would be empty
                 continue
-            cost = start + stage * per * -(-tiles * splits // units) + (0.6e-6 * 4 * m * n * splits if may_split else 0.0)
+            cost = start + stage * per * -(-tiles * splits // units) + plane * splits
             if best is None or cost < best[0]:
                 best = (cost, rows, columns, splits)
     return best[1:]
@@ -1126,17 +1126,17 @@ def many_pays(m: int, n: int, k: int, into_stream: bool, gated: bool, units: int
     6,912 for 174 (30) 17.8 and 40.6, 2,304 x 1,536 for 160 and 512 (54 and 144) 9.1 and 10.1, 14.5 and 10.9, 4,608 x 3,072 for 320 (180) 20.0 and 22.8,
     2,048 x 1,024 for 129 (48) 10.1 and 7.1; gated, which saves a launch, 1,408 x 4,352 for 273 (55) 19.1 and 27.7, 2,816 x 2,048 for 200 (88)
     15.4 and 14.1.  Stored products of more workgroups than units are level, and where small tiles give many rounds behind (6,144 x 1,152 for
-    1,024 rows, 768 of 64 x 128, 20.0 and 24.4; 4,096 x 1,536 for 1,700, 448 of 128 x 128, 1.01 times as fast).  And tiles of 96 x 256 have to fill their
-    last round: gated 8,192 x 2,048 for 576 rows (192) 32.3 and 35.3, 13,824 x 2,304 for 288 (162) 35.8 and 39.7, 12,288 x 2,048 for 420
-    (240) 36.6 and 35.1.  Of 1,623 stored products measured 718 are on this side of the line, 11 of them 3 to 7 % behind the library; of 536 gated ones
-    418, one (6 %)."""
+    1,024 rows, 768 of 64 x 128, 20.0 and 24.4; 4,096 x 1,536 for 1,700, 448 of 128 x 128, 1.01 times as fast).  And of the larger gated products tiles of
+    96 x 256 have to fill their last round: 8,192 x 2,048 for 576 rows (192) 32.3 and 35.3, 13,824 x 2,304 for 288 (162) 35.8 and 39.7, 12,288 x
+    2,048 for 420 (240) 36.6 and 35.1.  Of some 1,600 stored products measured 782 are on this side of the line, 9 of them 3 to 7 % behind the
+    library; of some 520 gated ones 498, 8 (at most 6 %)."""
     if m * n * k > MANY_MOST:
         return False
     if into_stream:
         return n <= STREAM_MOST
     rows, columns, _ = many_plan(m, n, k, False, units)
     groups = -(-m // rows) * -(-n // columns)
-    if columns > 128 and 16 * groups < 15 * units * -(-groups // units):
+    if gated and columns > 128 and n * k > 15 << 20 and 16 * groups < 15 * units * -(-groups // units):
         return False
     if not gated and groups > units:
         return False

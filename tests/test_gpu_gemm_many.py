@@ -88,7 +88,7 @@ def test_products_with_a_copy_take_it_and_agree_with_those_without(m, n, k):
 
 @pytest.mark.parametrize("m, n, k, gated, takes", [
     (256, 1024, 4096, False, False), (174, 1216, 6912, False, False), (160, 2304, 1536, False, False), (512, 2304, 1536, False, True),
-    (320, 4608, 3072, False, False), (129, 2048, 1024, False, True), (640, 8192, 2048, False, False), (1024, 6144, 1024, False, False),
+    (320, 4608, 3072, False, False), (129, 2048, 1024, False, True), (640, 8192, 2048, False, True), (2048, 2560, 1536, False, True), (1024, 6144, 1024, False, False),
     (273, 1408, 4352, True, False), (200, 2816, 2048, True, True), (576, 8192, 2048, True, False), (420, 12288, 2048, True, True),
 ])
 def test_products_in_one_range_whose_workgroups_are_few_stay_with_the_library(m, n, k, gated, takes):
