@@ -316,7 +316,7 @@ extern "C" int leone_attention_rows_parts(const void* q, void* out, const void* 
     return 0;
 }
 
-// talk [q_heads, q_heads] of talk_dtype: the heads' scores are mixed by it before the softmax.
+// The same without such room.
 extern "C" int leone_attention_rows_shaped(const void* q, void* out, const void* k_pool, const void* v_pool, int dtype,
                                            const int* positions, const int* row_entry, const int* block_table,
                                            int max_blocks, int rows, int q_heads, int kv_heads, int head_dim, int v_dim,
@@ -331,6 +331,7 @@ extern "C" int leone_attention_rows_shaped(const void* q, void* out, const void*
                                       turn_pairing, chunk, nullptr, nullptr, stream);
 }
 
+// talk [q_heads, q_heads] of talk_dtype: the heads' scores are mixed by it before the softmax.
 extern "C" int leone_attention_rows_talk(const void* q, void* out, const void* k_pool, const void* v_pool, int dtype,
                                          const void* talk, int talk_dtype, const int* positions, const int* row_entry,
                                          const int* block_table, int max_blocks, int rows, int q_heads, int kv_heads,

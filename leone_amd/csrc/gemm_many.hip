@@ -10,11 +10,14 @@
 // takes them; with many, the chip's power, where the vendor library with its 256 x 256 tiles is as good or better (6,144 x 4,096 for 2,048 rows: 81
 // us here, 67 there).  ops.many_plan chooses; its comment has both sides' figures.
 //
-// kDeep, for up to 128 rows, which have one row of tiles: the weight is read once, so what bounds it is memory, that is, the bytes that a unit has
-// asked for and not yet got.  Four stages of W are on their way (64 KB of 128 columns, where the kernel of gemm_rows.hip has 32 KB), asked for with
-// the hint that they are read once, and the last four stages ask for nothing; workgroups of two or three waves take 64 or 96 columns where 128
-// would leave units without work (gated 24,576 x 4,096 for 64 rows, 256 groups of 96: 37.3 us, 39.1 with 192 of 128, 40.3 in gemm_rows.hip).  4,096 x 12,288 for 64 rows 24.1 us in gemm_rows.hip, 21.8 here two stages ahead, 20.0 four ahead (5.0 TB/s); 4,096 x
-// 4,096 12.3, 10.0 and 9.3; 2,048 x 2,048 6.6, 5.8 and 5.0.  ops.deep_plan chooses.
+// kDeep, for up to 128 rows: what bounds it is memory, that is, the bytes that a unit has asked for and not yet got.  Four stages of W are on their way (64
+// KB of 128 columns, where the kernel of gemm_rows.hip has 32 KB), asked for with the hint that they are read once, and the last four stages ask for
+// nothing; workgroups of two or three waves take 64 or 96 columns where 128 would leave units without work.  us, 64 rows, gemm_rows.hip and here: 4,096 x
+// 12,288 24.3 and 21.3 (4.7 TB/s), 6,144 x 4,096 16.5 and 11.7, 4,096 x 4,096 12.4 and 10.1, 2,048 x 2,048 6.7 and 5.4, gated 24,576 x 4,096 41.9 and 37.2.
+// Beyond 64 rows there are one or two rows of tiles, whatever is faster; with two, W is asked for twice, by workgroups that work side by side.  The hint
+// is worth its while there too (128 rows in two rows of tiles, with it and without: 6,144 x 4,096 17.5 and 18.8, 4,096 x 4,096 13.1 and 13.9, 4,096 x 12,288
+// 31.5 and 32.6, gated 12,288 x 2,048 20.6 and 21.6), but not for the smallest matrices (1,024 x 3,072 5.6 and 5.0; 64 rows 5.2 and 4.6).
+// ops.deep_plan chooses.
 #include "common.h"
 
 #include <type_traits>

@@ -145,7 +145,7 @@ int leone_gemm_rows_bf16(const void* x, const void* w, int w_tiled, void* y, int
 // The same product for any number of rows from W's tiled copy, N a multiple of 16, K of 64, x, w and y at multiples of 16 bytes (out_mode
 // 0 to 3 as above; gated: gate and up are rounded to bfloat16 (not where `deep`), then act(gate) * up).  splits > 1 only with out_mode 3; ranges of K are whole
 // stages of 64, ceil(stages / splits) each, none empty.  tile_rows x tile_columns: 64 x 128, 96 x 128, 128 x 128 or 96 x 256 results a
-// workgroup, with `deep` 32 x 64, 32 x 96, 64 x 64, 64 x 96, 64 x 128, 96 x 128 or 128 x 128, the weight read once and four stages ahead; that
+// workgroup, with `deep` 32 x 64, 32 x 96, 64 x 64, 64 x 96, 64 x 128, 96 x 128 or 128 x 128, with the weight asked for four stages ahead; that
 // choice changes no sum.
 int leone_gemm_many_bf16(const void* x, const void* w, void* y, int out_mode, int out_dtype, int m, int n, int k, int splits, long plane,
                          int tile_rows, int tile_columns, int deep, int act, float limit, hipStream_t stream);

@@ -979,9 +979,10 @@ moe_product_wide_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__
 // shared memory: hence 256 rows a workgroup, which read a piece of the pairs' rows half as often, wherever that leaves work for the units (see
 // many_rows), and results turned in shared memory so that stores are whole lines (as 16 bytes of 32 rows they took a third of the
 // second product).  With the matrices row by row the same kernel takes 1.4 times as long (half a line of 32 rows a load).
+// And a workgroup walks a whole inner size: with few of them that is what takes the time, and ops._copied_tile leaves such products to the kernels above.
 // Both products, us, best tiles of moe_product_tiled_kernel and moe_product_wide_kernel and now: 32 experts of 2,048 x 768, 40 pairs each 79 and 63, 100
 // pairs 109 and 75, 240 pairs 176 and 132, 400 pairs 256 and 181, 700 pairs 358 and 277; 32 of 4,096 x 1,024, 240 pairs 413 and 306; 64 of 2,048 x 1,408,
-// 100 pairs 322 and 250; 32 of 1,024 x 384, 100 pairs 37 and 26; 8 of 1,024 x 4,096, 300 pairs 138 and 125.
+// 100 pairs 322 and 250; 32 of 1,024 x 384, 100 pairs 37 and 26.
 typedef float moe_floatx16 __attribute__((ext_vector_type(16)));
 constexpr int kTogether = 2;
 template <int kMode, int kMT, int kNT>

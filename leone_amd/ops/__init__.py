@@ -1173,7 +1173,7 @@ def _takes_many(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype, r
     return streamed_copy(weight) if tiles is None else tiles
 
 
-# Tiles of ``gemm_many`` that read the weight once, four stages ahead, for up to ROWS_MAX rows: (rows, columns): us to start, us a stage of 64
+# Tiles of ``gemm_many`` that ask for the weight four stages ahead, for up to ROWS_MAX rows: (rows, columns): us to start, us a stage of 64
 # elements of K, TB/s of the weight with every unit at work, us a megabyte of results, what a further workgroup on a unit costs of the first,
 # and how much of a last round's idle units is lost.
 DEEP_TILES = {(32, 64): (2.411, 0.197, 6.777, 0.331, 0.827, 0.637), (32, 96): (2.518, 0.233, 7.219, 0.295, 1.699, 0.561),
@@ -1236,7 +1236,8 @@ def _deep_sizes(m: int, n: int, k: int, may_split: bool, gated: bool, out_dtype:
     """The plan of a product of FUSED_ROWS to ROWS_MAX rows if ``gemm_many`` takes such sizes and is faster than ``gemm_rows``, whose waves share
     K out.
 
-    Planes: always, up to the widest stream that was measured (us, ``gemm_rows`` and ``gemm_many`` with ``deep_plan``, weights from memory, 17, 64 and 128 rows:
+    Planes: always, up to the widest stream that was measured (us, ``gemm_rows`` and ``gemm_many`` with ``deep_plan``, weights from memory, planes' readers
+    at 0.3 us a megabyte, 17, 64 and 128 rows:
     6,144 x 4,096 14.0 and 11.8, 17.5 and 14.0, 23.8 and 19.5; 2,048 x 2,048 5.6 and 4.5, 8.1 and 6.1, 12.5 and 7.0; 4,096 x 1,024
     5.5 and 4.5, 8.1 and 6.0, 12.5 and 7.4; 1.03 times as fast at the least; but with the norm behind it 9,024 x 3,264 for 46 rows 38 and 56).
     In one range of K a workgroup's chain of stages bounds few workgroups: up to 48 rows it takes longer than in ``gemm_rows`` unless K is
@@ -1268,7 +1269,7 @@ def gemm_many(x: torch.Tensor, tiles: torch.Tensor, n: int, out_dtype: torch.dty
     ``residual`` and one range of K the product is added into that float32 tensor (None returned), with more ranges float32 planes come
     back whose sum, in order, the caller adds; with ``gated`` the weight is an interleaved gate/up weight and act(gate) * up comes out,
     both rounded to bfloat16 first (not with the deep tiles).  ``plan``: (rows, columns, ranges of K) of a workgroup, by default ``many_plan``'s; with a fourth, True, for
-    the tiles that read the weight once and further ahead (``DEEP_TILES``)."""
+    the tiles that ask for the weight further ahead (``DEEP_TILES``)."""
     m, k = x.shape
     if gated and residual is not None:
         raise KernelError("gemm_many: a gated product cannot also be added into the stream")
