@@ -2367,10 +2367,11 @@ def _copied_tile(pairs: int, experts: int, hidden: int, ff: int, gated: bool, un
     the units 4 of 3,456 x 1,216, 128 pairs 82 and 110.
 
     From the copies a workgroup walks a whole inner size, a stage of 64 at a time, which takes its time however few workgroups there are; the kernels
-    that read the matrices have more waves on a unit.  So each product needs a workgroup for every twelve elements of its inner size, or a
+    that read the matrices have more waves on a unit.  So each product needs a workgroup for every eight elements of its inner size, or a
     short one (us, from the matrices and from the copies: 2 of 3,520 x 3,968, 31 pairs 81 and 158, 8 of 2,688 x 5,696, 34 pairs 161 and 238,
-    8 of 5,248 x 3,136, 13 pairs 170 and 246, 4 of 2,944 x 1,216, 31 pairs 53 and 70; 32 of 2,048 x 768, 40 pairs 79 and 63).  Of 331 pairs of products
-    measured, 2 to 64 experts of 512 to 6,144 wide layers, 57 were slower from the copies, up to twice; of those on this side of the line one, by 4 %."""
+    8 of 2,176 x 1,536, 26 pairs 53 and 72, 4 of 2,944 x 1,216, 31 pairs 53 and 70; 32 of 2,048 x 768, 40 pairs 79 and 63).  Of 893 pairs of products
+    of more than 16 pairs a tile, 2 to 64 experts of 512 to 6,144 wide layers, 336 are on this side of the line, two of them slower from the copies, by
+    4 and 6 %; of 332 others in engines' shapes 124, six, by at most 4 %."""
     each = pairs / experts
     fills = experts * -(-hidden // 128) >= units
     few, many = 10 if fills else 14, 48 if fills and hidden * ff >= 2500000 else 125
@@ -2382,7 +2383,7 @@ def _copied_tile(pairs: int, experts: int, hidden: int, ff: int, gated: bool, un
         return used * -(-ff // (64 if gated else 128)), used * -(-hidden // 128)
     tile = 128 if each >= many and 2 * min(workgroups(128)) >= units else 64
     first, second = workgroups(tile)
-    return tile if (hidden <= 1024 or 12 * first >= hidden) and (ff <= 1024 or 12 * second >= ff) else 0
+    return tile if (hidden <= 1024 or 8 * first >= hidden) and (ff <= 1024 or 8 * second >= ff) else 0
 
 
 def _expert_tiles(x: torch.Tensor, rows: int, top: int, experts: int, hidden: int, ff: int, copied: bool = False, gated: bool = True):
