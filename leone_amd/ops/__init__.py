@@ -904,13 +904,13 @@ def keep_streamed_copy(weight: torch.Tensor, any_order: bool = True) -> int:
 
 
 def streamed_copy(weight: torch.Tensor) -> Optional[torch.Tensor]:
-    held = _streamed.get((weight.data_ptr(), tuple(weight.shape)))
+    held = _streamed.get((weight.data_ptr(), weight.shape))
     return None if held is None or held[0]() is not weight else held[1]
 
 
 def _any_order(weight: torch.Tensor) -> bool:
     """Whether the weight has a copy that its products may take in any order of their sums."""
-    held = _streamed.get((weight.data_ptr(), tuple(weight.shape)))
+    held = _streamed.get((weight.data_ptr(), weight.shape))
     return held is not None and held[0]() is weight and held[2]
 
 
@@ -1161,16 +1161,21 @@ def _takes_many(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype, r
     us, library and ``gemm_many``, weights from memory, with the norm behind them: into the stream 2,048 x 6,144 for 129, 512 and 800 rows
     23.6 and 15.8, 33.8 and 26.3, 42.8 and 35.3; 4,096 x 4,096 for 160, 384 and 640 rows 31 and 20, 31 and 29, 42.3 and 41.2; 1,024 x 3,072 for
     320 and 1,700 rows 17.1 and 13.1, 26.3 and 24.0.  A fifth faster on average over 451 products of up to 10 G of two elements (19 %
-    up to 2 G, 15 % from 7 G on), 4 to 6 % behind in 6 of them (2,048 x 2,048 for 720 rows 19.1 and 20.1).  Others: ``many_pays``.  Products that were
-    tuned, or are being noted for it, stay with the library."""
-    if not _streamed or (tiles is None and not _any_order(weight)):
+    up to 2 G, 15 % from 7 G on); of 122 with tiles and ranges as ``many_plan`` has them 4 are 2 to 5 % behind (1,024 x 2,048 for 1,024 rows 16.3 and 17.2).
+    Others: ``many_pays``.  Products that were tuned, or are being noted for it, stay with the library."""
+    if not _streamed:
         return None
+    if tiles is None:
+        held = _streamed.get((weight.data_ptr(), weight.shape))
+        if held is None or not held[2] or held[0]() is not weight:
+            return None
+        tiles = held[1]
     if _recorded_products is not None or not _many_fits(x, weight, out_dtype, residual, gated) \
             or not many_pays(x.shape[0], *weight.shape, residual is not None, gated, compute_units(weight.device)):
         return None
     if _tuned_products and _library_problem(x, weight, torch.float32 if residual is not None else out_dtype, residual is not None) in _tuned_products:
         return None
-    return streamed_copy(weight) if tiles is None else tiles
+    return tiles
 
 
 # Tiles of ``gemm_many`` that ask for the weight four stages ahead, for up to ROWS_MAX rows: (rows, columns): us to start, us a stage of 64
@@ -1486,7 +1491,7 @@ def linear(x, weight: torch.Tensor, out_dtype: Optional[torch.dtype] = None,
             with profile.span("gemm rows", weight):
                 return gemm_many(x, deep[0], weight.shape[0], out_dtype, residual, gated, deep[1], activation, limit)
         return gemm_rows(x, weight, out_dtype, residual, gated, may_split=may_split, activation=activation, limit=limit)
-    if dtype == torch.bfloat16 and x.is_cuda and weight.is_cuda and rows > ROWS_MAX:
+    if _streamed and dtype == torch.bfloat16 and rows > ROWS_MAX and x.is_cuda and weight.is_cuda:
         tiles = _takes_many(x, weight, out_dtype, residual, gated)
         if tiles is not None:
             with profile.span("gemm many", weight):
