@@ -1121,26 +1121,22 @@ def many_pays(m: int, n: int, k: int, into_stream: bool, gated: bool, units: int
     """Whether a product of more than ROWS_MAX rows is faster with ``gemm_many`` than in the library.
 
     Into the stream (its planes fill the units) up to MANY_MOST, see ``_takes_many``.  Otherwise K is in one range, and a workgroup's chain of
-    stages takes its time however few workgroups there are, where the library cuts K: from a K of 1,024 on there have to be more of them
-    the longer K is.  us, library and ``gemm_many``, weights from memory: stored, 1,024 x 4,096 for 256 rows (32 workgroups) 11.6 and 21.2, 1,216 x
-    6,912 for 174 (30) 17.8 and 40.6, 2,304 x 1,536 for 160 and 512 (54 and 144) 9.1 and 10.1, 14.5 and 10.9, 4,608 x 3,072 for 320 (180) 20.0 and 22.8,
-    2,048 x 1,024 for 129 (48) 10.1 and 7.1; gated, which saves a launch, 1,408 x 4,352 for 273 (55) 19.1 and 27.7, 2,816 x 2,048 for 200 (88)
-    15.4 and 14.1.  Stored products of more workgroups than units are level, and where small tiles give many rounds behind (6,144 x 1,152 for
-    1,024 rows, 768 of 64 x 128, 20.0 and 24.4; 4,096 x 1,536 for 1,700, 448 of 128 x 128, 1.01 times as fast).  And of the larger gated products tiles of
-    96 x 256 have to fill their last round: 8,192 x 2,048 for 576 rows (192) 32.3 and 35.3, 13,824 x 2,304 for 288 (162) 35.8 and 39.7, 12,288 x
-    2,048 for 420 (240) 36.6 and 35.1.  Of some 1,600 stored products measured 782 are on this side of the line, 9 of them 3 to 7 % behind the
-    library; of some 520 gated ones 498, 8 (at most 6 %)."""
+    stages takes its time however few workgroups there are, where the library cuts K; but the host is 20 us sooner done with ``gemm_many`` than with
+    a library product (30 with an activation behind it), and it sets the pace of prompts of up to a few hundred rows.  Whole prompts of eight
+    layers, us with the library's and with these products: q/k/v of 1,280 to 2,560 wide layers, 130 to 450 rows, 1,240 to 1,470 and 1,070 to 1,410; of
+    4,096 wide ones 1,570 to 2,150 and 1,520 to 2,130; 6,144 x 1,024 and x 2,048 for 1,024 rows (768 and 384 workgroups, the product itself
+    slower) 1,317 and 1,178, 1,909 and 1,903; gated 1,408 x 2,048 for 200 rows (44) 1,365 and 1,183; 8,192 x 2,048 for 576 (192 of 96 x 256,
+    32.3 and 35.3 by themselves) 1,276 and 1,097; none behind by more than 0.4 %.
+    So the line is where the product itself loses more than about 3 us: us, library and ``gemm_many``, weights from memory, stored 1,024 x 2,048 for 256
+    rows (32 workgroups) 9.7 and 11.9, 2,304 x 1,536 for 512 (144) 14.5 and 10.9, 4,608 x 3,072 for 256 and 320 (144 and 180) 30.6 and 20.0, 20.1 and 22.8,
+    1,024 x 4,096 for 256 (32) 11.5 and 20.9, 1,216 x 6,912 for 174 (30) 17.8 and 40.6; gated 1,024 x 2,048 for 256 (32) 12.7 and
+    14.5, 1,408 x 4,352 for 273 (55) 19.1 and 27.7: up to a K of 2,048 always, beyond at a workgroup for 32 elements of K."""
     if m * n * k > MANY_MOST:
         return False
     if into_stream:
         return n <= STREAM_MOST
     rows, columns, _ = many_plan(m, n, k, False, units)
-    groups = -(-m // rows) * -(-n // columns)
-    if gated and columns > 128 and n * k > 15 << 20 and 16 * groups < 15 * units * -(-groups // units):
-        return False
-    if not gated and groups > units:
-        return False
-    return k <= 1024 or groups >= (max(units // 4, k // 24) if gated else max(units // 2, k // 16))
+    return k <= 2048 or 32 * -(-m // rows) * -(-n // columns) >= k
 
 
 def _many_fits(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype, residual: Optional[torch.Tensor], gated: bool) -> bool:
