@@ -1245,9 +1245,13 @@ def _deep_sizes(m: int, n: int, k: int, may_split: bool, gated: bool, out_dtype:
     short or the units are at work (stored, 17 and 33 rows: 1,024 x 8,192 26.5 and 30.3, 29.3 and 33.6, 4,096 x 4,096 16.5 and 17.4, 17.8 and 19.0; 4,096 x 2,048 9.7
     and 9.5, 10.7 and 10.5, 16,384 x 2,048 17.4 and 13.5, 18.1 and 13.8, 1,024 x 1,024 5.8 and 5.5, 6.9 and 6.4; gated, whose gate and up share a tile, 4,096 x
     4,096 17.6 and 18.6, 19.1 and 21.2, 2,048 x 2,048 10.3 and 10.3, 11.6 and 12.3, 8,192 x 2,048 12.9 and 11.4, 14.4 and 13.4, 24,576 x 4,096 39 and 37 for 17).
-    Beyond 64 rows the larger matrices are behind where the weight is asked for twice or units are idle (14,912 x 5,760 for 66 rows 37 and 51, 19,264 x 5,120 for 95 43 and
-    49; 32,768 x 4,096 for 65 and 128 1.23 and 1.28 times as fast, 6,528 x 5,120 for 92 1.19), and gated ones altogether (24,576 x 4,096 for 96 and 128 rows 44 and 45, 48 and
-    49).  Of 889 products in one range measured 645 are on this side of the line, 1.22 times as fast on average, 0.95 at the least (without it 156 were more than 3 % behind)."""
+    The widest matrices, with 96 columns a workgroup, are ahead from three quarters of the units on (18,432 x 3,072, 192 of them, for 22 rows 23.3 and 20.8; of 110
+    such products 6 % on average, 0.94 at the least), the others from seven eighths (192 and 208 of 64 columns 0.995 to 1.036 times as fast on average).
+    Beyond 64 rows the larger matrices are behind where units are idle or a second row of tiles of 128 columns has few rows (14,912 x 5,760 for 66 rows 37
+    and 51, 15,360 x 2,560 for 65 and 112 22 and 28, 27 and 24, 19,264 x 5,120 for 95 43 and 49; 32,768 x 4,096 for 65 and 128 1.23 and 1.28 times as fast, 6,528
+    x 5,120 for 92, tiles of 64 columns, 1.19), and gated ones with one row of tiles altogether (24,576 x 4,096 for 96 and 128 rows 44 and 51, 49 and
+    49, 28,672 x 5,120 59 and 62; but 6,144 x 6,144 for 96, 64 columns, 40 and 32, 16,384 x 4,096 for 65 and 128, two rows, 37 and 41, 44 and 41).  Of 1,453
+    products in one range measured 988 are on this side of the line, 1.16 times as fast on average, 18 of them 3 to 7 % behind."""
     if not FUSED_ROWS < m <= ROWS_MAX or k % 64 or n % 16 or n < MANY_LEAST or k < MANY_LEAST or out_dtype not in _CODES \
             or (gated and out_dtype != torch.bfloat16) or (may_split and not gated and n > STREAM_MOST):
         return None
@@ -1256,11 +1260,12 @@ def _deep_sizes(m: int, n: int, k: int, may_split: bool, gated: bool, out_dtype:
         return plan
     rows, columns = plan[:2]
     groups = -(-m // rows) * -(-n // columns)
-    full = 8 * groups >= 7 * units
+    full = 8 * groups >= (6 if columns == 96 else 7) * units
     if m <= 48:
         pays = k <= 1024 or full or (k <= 2048 and (not gated or 8 * groups >= 3 * units))
     else:
-        pays = m <= 64 or n * k <= DEEP_WHOLE_MOST or (not gated and (k <= 2048 or columns == 64 or (full and rows >= m)))
+        pays = m <= 64 or n * k <= DEEP_WHOLE_MOST or columns == 64 or (rows == 64 and m > 100) \
+            or (not gated and (k <= 2048 or (full and rows >= m)))
     return plan if pays else None
 
 

@@ -39,6 +39,8 @@ def test_chunks_of_experts_matrices_on_their_way(lib, experts, gated, n, k, one)
     (17, 1024, 8192, "store", False), (48, 4096, 4096, "store", False), (49, 4096, 4096, "store", True), (33, 4096, 2048, "store", True),
     (33, 1024, 1024, "gated", True), (33, 2048, 2048, "gated", False), (33, 6144, 2048, "gated", True), (17, 24576, 4096, "gated", True), (33, 4096, 4096, "gated", False),
     (66, 14912, 5760, "store", False), (95, 19264, 5120, "store", False), (65, 32768, 4096, "store", True), (92, 6528, 5120, "store", True), (96, 24576, 4096, "gated", False),
+    (96, 6144, 6144, "gated", True), (65, 16384, 4096, "gated", False), (128, 16384, 4096, "gated", True), (65, 15360, 2560, "store", False), (112, 15360, 2560, "store", True),
+    (22, 18432, 3072, "gated", True), (17, 12288, 3072, "gated", False),                 # 192 workgroups of 96 and of 64 columns
     (17, 1024, 8192, "planes", True), (46, 9024, 3264, "planes", False), (128, 8192, 1024, "planes", True),
 ])
 def test_which_products_of_up_to_128_rows_take_the_copy(m, n, k, kind, takes):
