@@ -18,6 +18,8 @@
 // is worth its while there too (128 rows in two rows of tiles, with it and without: 6,144 x 4,096 17.5 and 18.8, 4,096 x 4,096 13.1 and 13.9, 4,096 x 12,288
 // 31.5 and 32.6, gated 12,288 x 2,048 20.6 and 21.6), but not for the smallest matrices (1,024 x 3,072 5.6 and 5.0; 64 rows 5.2 and 4.6).
 // ops.deep_plan chooses.
+//
+// The walk along the stages and the turned stores stand in moe_product_many_kernel (routed.hip) as well: what is mended in one is mended in both.
 #include "common.h"
 
 #include <type_traits>

@@ -973,7 +973,8 @@ moe_product_wide_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__
 // pairs and 128 kNT rows of its expert's matrix (gated: half as many gate rows and their up rows), a wave a quarter of them in parts of 32, whose
 // elements it takes from memory as its instruction (32 x 32 x 16) wants them, one or two stages of 64 ahead: they pass neither through shared memory
 // nor a barrier.  The pairs' rows, which all four waves read, go through shared memory, a stage's 128 bytes of a row turned about by the row's
-// number so that the same piece of 16 rows lies in 16 places; a stage is written while the one before it is worked on.
+// number so that the same piece of 16 rows lies in 16 places; a stage is written while the one before it is worked on.  (The walk along the stages and the
+// turned stores are gemm_many_kernel's: what is mended in one is mended in both.)
 //
 // What bounds it is the power of the chip (matrix instructions alone, on all units, run at two thirds of the clock) and what goes through
 // shared memory: hence 256 rows a workgroup, which read a piece of the pairs' rows half as often, wherever that leaves work for the units (see

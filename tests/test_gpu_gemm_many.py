@@ -77,6 +77,7 @@ def test_products_with_a_copy_take_it_and_agree_with_those_without(m, n, k):
         assert torch.equal(half, ops.swiglu(ops.gemm_many(x, tiles, n, plan=ops.many_plan(m, n, k, False))) if taken else gated)
         # what it does not take stays with the library: other layouts, other types, products being noted
         assert ops._takes_many(x[:, ::2], weight[:, :k // 2], torch.float32, None, False) is None
+        assert ops._takes_many(x, weight, torch.float16, None, False) is None
         assert ops._takes_many(x, weight, torch.float16, torch.zeros((m, n), device="cuda"), False) is None
         assert ops._takes_many(x, weight, torch.float32, torch.zeros((n, m), device="cuda").t(), False) is None
         with ops.record_library_products() as seen:
